@@ -6,7 +6,9 @@ truncation of what a caller gets are here.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
+import gc
 from typing import Any, Callable, Dict, List, Optional, Sequence, Union
 
 import torch
@@ -18,6 +20,20 @@ BF16 = torch.bfloat16
 DEFAULT_MAX_TOKENS = 768
 DEFAULT_TEMPERATURE = 0.5
 DEFAULT_TOP_P = 0.3
+
+
+@contextlib.contextmanager
+def no_collection():
+    """Keeps Python's cyclic collector out of a graph capture.  A captured graph that is part of a cycle (a model whose graphs refer back to it)
+    is freed by the collector, at whatever allocation that happens to run; freeing a graph synchronises the device, which a capture
+    forbids: the graph's destructor then ends the process."""
+    was = gc.isenabled()
+    gc.disable()
+    try:
+        yield
+    finally:
+        if was:
+            gc.enable()
 
 
 class DeviceEngine:
@@ -109,11 +125,12 @@ class DeviceEngine:
     # ------------------------------------------------------------ decode loop
     def _lockstep_loop(self, first: torch.Tensor, pos: Sequence[int], max_tokens: int, make_step: Callable, graph_key: tuple,
                        eos_id: Optional[int], check_every: int = 16, uniforms: Optional[torch.Tensor] = None,
-                       graphs: Optional[bool] = None) -> torch.Tensor:
+                       graphs: Optional[bool] = None, keep: Sequence[torch.Tensor] = ()) -> torch.Tensor:
         """Device-resident lockstep decode: int32 [steps + 1, B], row 0 = ``first``.  ``make_step(pos_buf)`` binds a position buffer
         (device int32 [B], advanced by the step itself) and returns ``step(tok_in, tok_out, uniform_row)``, which queues one decode
         step.  ``uniforms`` [max_tokens, B]: one draw per (step, sequence) of a sampled decode.  With ``compile()`` the steps are
-        replayed from a hipGraph in chunks; ``graph_key`` names everything the captured launches depend on."""
+        replayed from a hipGraph in chunks; ``graph_key`` names everything the captured launches depend on, ``keep`` holds the tensors
+        they read that nothing else keeps (a kept graph must not refer to the model: see no_collection)."""
         b = first.shape[0]
         hist = torch.zeros(max_tokens + 1, b, dtype=torch.int32, device=self._device)
         hist[0] = first
@@ -158,11 +175,11 @@ class DeviceEngine:
                 hist[steps + 1 : steps + n + 1] = buf[1:]
                 torch.cuda.synchronize(self._device)
                 g = torch.cuda.CUDAGraph()
-                with torch.cuda.graph(g):
+                with no_collection(), torch.cuda.graph(g):
                     for i in range(n):
                         step(buf[i], buf[i + 1], u_buf[i])
                 # the capture did not execute; nothing to undo
-                self._graphs[key] = (g, buf, pos_buf, u_buf, step)
+                self._graphs[key] = (g, buf, pos_buf, u_buf, keep)
             else:
                 g, buf, pos_buf, u_buf, _ = entry
                 buf[0] = hist[steps]

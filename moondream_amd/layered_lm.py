@@ -194,7 +194,7 @@ class LayeredLM(DeviceEngine):
             return one_step
 
         key = (tuple(slots), ctx, suppress_id, ws.data_ptr(), logits.data_ptr(), float(temperature), float(top_p), self.dtype)
-        hist = self._lockstep_loop(first, pos, max_tokens, make_step, key, eos_id, check_every, uniforms)
+        hist = self._lockstep_loop(first, pos, max_tokens, make_step, key, eos_id, check_every, uniforms, keep=(rows, ws, logits))
         for s in slots:
             self.state.pool.length[s] += hist.shape[0] - 1
         return hist

@@ -924,7 +924,7 @@ class MoondreamModel(DeviceEngine):
 
         key = (slot0, suppress_id, ws.data_ptr(), self._kv_k.data_ptr(), logits.data_ptr(), b1, float(temperature), float(top_p))
         return self._lockstep_loop(first, pos_list, max_tokens, make_step, key, eos_id, check_every, uniforms,
-                                   graphs=self.use_graphs and lora is None)
+                                   graphs=self.use_graphs and lora is None, keep=(ws, logits))
 
     def _check_b1_barriers(self):
         """Call after the tokens of a single-sequence decode have reached the host: the persistent kernel's grid barriers
