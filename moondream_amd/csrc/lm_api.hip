@@ -28,7 +28,7 @@ struct LmWs {
   char *h, *proj, *q, *att, *y, *gu, *act;
   float *part, *qf, *kf, *of, *chunk_state, *attn_part;
   char *c_rows, *kv, *q_lat, *conv_out;
-  float *latent_part, *dt, *seg, *seg_decay, *route_weight;
+  float *latent_part, *dt, *seg, *seg_decay, *route_weight, *sumsq;
   int32_t *chosen, *slot_of, *row_of, *offsets;
   void* splitk;
   size_t splitk_bytes;
@@ -37,6 +37,14 @@ struct LmWs {
 };
 
 inline bool decode_regime(const md_lm_model* m, int rows) { return m->dtype == MD_DTYPE_BF16 && rows <= DECODE_ROWS; }
+
+// Most rows for which a product of gemm_step.hip is the faster one where nothing is saved behind it: rows that were normed in a launch of
+// their own (10304 columns, 16 rows: 15.2 us, the tile product 14.4), and the head (51200 columns; 1 row: 41-47 us against 55 with its norm, 16
+// rows: 59 against 56, 32 rows: 85).
+constexpr int STEP_PLAIN_ROWS = 8;
+
+// products that go on with the row-wise step behind them (gemm_step.hip)
+inline bool step_regime(const md_lm_model* m, int rows) { return m->dtype == MD_DTYPE_BF16 && rows <= LM_STEP_ROWS; }
 
 inline bool own_row_steps(const md_lm_model* m) { return m->streams > 0 || m->pos || m->embed_norm.w; }
 inline int n_streams(const md_lm_model* m) { return m->streams > 0 ? m->streams : 1; }
@@ -146,6 +154,7 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
   w.slot_of = (int32_t*)a.take(slots * 4);
   w.row_of = (int32_t*)a.take(slots * 4);
   w.offsets = (int32_t*)a.take(slots ? (experts + 1) * 4 : 0);
+  w.sumsq = (float*)a.take(step_regime(m, rows) ? M * (m->width_pad / 8) * 4 : 0);
   w.total = a.off;
   return w;
 }
@@ -221,6 +230,27 @@ struct Step {
   bool dec;
   LmAddend add = {};           // pending addend of the residual stream(s)
   const float* mix = nullptr;  // streams: the weights around the sublayer that made it
+  bool few = false;            // a step of few rows
+  bool ready = false;          // w.h holds the next sublayer's input already ...
+  const float* sumsq = nullptr;  // ... but for the factor that these give its rows, in the order of the matrix operand
+
+  // ordered: the rows of `a` lie as another of these products left them
+  LmStepGemm step_gemm(const void* a, int64_t lda, const md_linear& lin, bool ordered) const {
+    LmStepGemm g = {};
+    g.a = (const bf16_t*)a;
+    g.lda = ordered ? 8 : lda;
+    g.chunk = ordered ? 8 * b->n_rows : 8;
+    g.out_chunk = 8 * b->n_rows;
+    g.w = (const bf16_t*)lin.w;
+    g.k = lin.k_pad;
+    g.rows = b->n_rows;
+    g.sumsq = sumsq;
+    g.sumsq_n = m->width_pad / 8;
+    g.eps = m->eps;
+    g.width = m->width;
+    g.bias = (const bf16_t*)lin.b;
+    return g;
+  }
 
   md_status linear(const void* a, int64_t lda, const md_linear& lin, void* c, int64_t ldc, int rows, bool split = true) {
     if (m->dtype == MD_DTYPE_F32) return md_gemm_f32(a, lda, &lin, c, ldc, rows, s);
@@ -241,6 +271,12 @@ struct Step {
 
   // a mixer's projection -> w.proj.  Decode regime: K-slice partials and their sum in two launches, unless one slice fills the chip
   md_status project(const md_linear& lin) {
+    if (few && (sumsq || b->n_rows <= STEP_PLAIN_ROWS)) {
+      LmStepGemm g = step_gemm(w.h, m->width_pad, lin, sumsq != nullptr);
+      g.out = (bf16_t*)w.proj;
+      g.ldo = lin.n_pad;
+      return lm_step_rows(g, lin.n_pad, s);
+    }
     const int sl = dec ? md_gemm_partial_slices(&lin) : 1;
     if (sl == 1) return linear(w.h, m->width_pad, lin, w.proj, lin.n_pad, b->n_rows, !dec);
     const int64_t stride = (int64_t)b->n_rows * lin.n_pad;
@@ -260,6 +296,36 @@ struct Step {
     }
     add.src = w.y;
     return linear(a, lda, lin, w.y, m->width_pad, b->n_rows);
+  }
+
+  // a sublayer's last projection.  Few rows: the residual stream(s) and the input of the next sublayer (nw == nullptr: it needs whole
+  // normed rows) in the same launch
+  md_status finish(const void* a, int64_t lda, const md_linear& lin, bool ordered, const float* prev, const md_rms_weight* nw, const float* next) {
+    mix = prev;
+    if (!few || !nw) return to_residual(a, lda, lin);
+    LmStepGemm g = step_gemm(a, lda, lin, ordered);
+    g.out = (bf16_t*)w.h;
+    g.x = w.x;
+    g.stride = (int64_t)b->n_rows * m->width_pad;
+    g.streams = n_streams(m);
+    g.width_pad = m->width_pad;
+    g.prev = prev;
+    g.next = next;
+    g.norm = *nw;
+    g.sumsq_out = w.sumsq;
+    sumsq = w.sumsq;
+    ready = true;
+    return lm_step_resid(g, s);
+  }
+
+  // a sublayer's input -> w.h
+  md_status input(const md_rms_weight& nw, const float* next) {
+    if (ready) {
+      ready = false;
+      return MD_OK;
+    }
+    sumsq = nullptr;
+    return add_norm(nw, w.h, next, nullptr, true, b->n_rows);
   }
 
   // x += pending;  y = norm(x).  Streams: mixed with the weights around the pending sublayer, then u = their sum weighted for the next one
@@ -417,9 +483,17 @@ struct Step {
     }
   }
 
-  md_status feed_forward(const md_lm_layer& l) {
-    if (l.experts > 0) return expert_forward(l);
-    if (dec) {
+  md_status feed_forward(const md_lm_layer& l, const md_rms_weight* nw, const float* next) {
+    if (l.experts > 0) {
+      mix = l.mix2;
+      return expert_forward(l);
+    }
+    if (few) {
+      LmStepGemm g = step_gemm(w.h, m->width_pad, l.gate_up, sumsq != nullptr);
+      g.out = (bf16_t*)w.act;
+      g.ff_pad = l.ff_pad;
+      MD_TRY(lm_step_silu(g, s));
+    } else if (dec) {
       const int sl = md_gemm_partial_slices(&l.gate_up);
       const int64_t ld = l.gate_up.n_pad, stride = (int64_t)b->n_rows * ld;
       MD_TRY(md_gemm_partial_f32(w.h, m->width_pad, &l.gate_up, b->n_rows, w.part, ld, stride, s));
@@ -428,7 +502,7 @@ struct Step {
       MD_TRY(linear(w.h, m->width_pad, l.gate_up, w.gu, l.gate_up.n_pad, b->n_rows));
       MD_TRY(lm_silu_mul(m->dtype, w.gu, l.gate_up.n_pad, w.act, l.down.k_pad, b->n_rows, l.ff_pad, s));
     }
-    return to_residual(w.act, l.down.k_pad, l.down);
+    return finish(w.act, l.down.k_pad, l.down, few, l.mix2, nw, next);
   }
 
   md_status expert_forward(const md_lm_layer& l) {
@@ -474,24 +548,40 @@ struct Step {
     const int64_t row_floats = (int64_t)b->n_rows * m->width_pad;
     if (own_row_steps(m)) MD_TRY(lm_embed_streams(m, b->tokens, b->row_pos, w.x, row_floats, b->n_rows, s));
     else MD_TRY(lm_embed(m->dtype, m->embed, m->width_pad, b->tokens, w.x, b->n_rows, m->vocab, s));
+    const bool few_logits = n_logits > 0 && n_logits <= STEP_PLAIN_ROWS;
     for (int i = 0; i < m->n_layers; ++i) {
       const md_lm_layer& l = m->layers[i];
-      MD_TRY(add_norm(l.norm1, w.h, l.mix1, nullptr, true, b->n_rows));
+      // what follows this layer: the next one's mixer, or the head
+      const md_lm_layer* after = i + 1 < m->n_layers ? &m->layers[i + 1] : nullptr;
+      const md_rms_weight* nw = after ? &after->norm1 : &m->final_norm;
+      const float* next = after ? after->mix1 : nullptr;
+      MD_TRY(input(l.norm1, l.mix1));
       MD_TRY(project(l.in_proj));
       if (l.out_proj.k_pad != l.heads * l.vdim_pad) MD_TRY(zero_fill(w.att, (size_t)b->n_rows * l.out_proj.k_pad * esize(m), s));
       MD_TRY(mixer(i));
-      MD_TRY(to_residual(w.att, l.out_proj.k_pad, l.out_proj));
-      mix = l.mix1;
       if (l.ff > 0) {
-        MD_TRY(add_norm(l.norm2, w.h, l.mix2, nullptr, true, b->n_rows));
-        MD_TRY(feed_forward(l));
-        mix = l.mix2;
+        // (the router of an expert layer takes whole normed rows)
+        MD_TRY(finish(w.att, l.out_proj.k_pad, l.out_proj, false, l.mix1, l.experts > 0 ? nullptr : &l.norm2, l.mix2));
+        MD_TRY(input(l.norm2, l.mix2));
+        MD_TRY(feed_forward(l, nw, next));
+      } else {
+        MD_TRY(finish(w.att, l.out_proj.k_pad, l.out_proj, false, l.mix1, nw, next));
       }
       if (layer_out) MD_TRY(tap(layer_out + i * row_floats));
     }
     if (n_logits == 0) return MD_OK;
-    MD_TRY(add_norm(m->final_norm, w.h, nullptr, logit_rows, false, n_logits));
-    return linear(w.h, m->width_pad, m->head, logits, ld_logits, n_logits);
+    ready = ready && few_logits;
+    if (!ready) {
+      sumsq = nullptr;
+      MD_TRY(add_norm(m->final_norm, w.h, nullptr, logit_rows, false, n_logits));
+    }
+    if (!few || !few_logits) return linear(w.h, m->width_pad, m->head, logits, ld_logits, n_logits);
+    LmStepGemm g = step_gemm(w.h, m->width_pad, m->head, ready);
+    g.rows = n_logits;
+    g.rows_idx = ready ? logit_rows : nullptr;  // (otherwise w.h holds the wanted rows only)
+    g.out = (bf16_t*)logits;
+    g.ldo = ld_logits;
+    return lm_step_rows(g, m->head.n_pad, s);
   }
 };
 
@@ -518,6 +608,7 @@ extern "C" md_status md_lm_forward(const md_lm_model* m, const md_lm_batch* b, c
   const LmWs w = layout(m, b, n_logits, workspace);
   if (workspace_bytes < w.total) return MD_ERR_WORKSPACE;
   Step step{m, b, st, w, (hipStream_t)stream, decode_regime(m, b->n_rows)};
+  step.few = step_regime(m, b->n_rows);
   return step.run(logit_rows, n_logits, logits, ld_logits, layer_out);
 }
 

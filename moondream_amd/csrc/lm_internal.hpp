@@ -194,6 +194,37 @@ struct LmRoute {
   int32_t *offsets, *row_of, *slot_of;  // [experts + 1], [rows * top], [rows][top]
 };
 
+// A product of a step of few rows and what follows it (gemm_step.hip).  Rows that a residual epilogue wrote carry no norm factor: it
+// comes from their sums of squares (sumsq; nullptr: the rows are complete).
+constexpr int LM_STEP_ROWS = 28;  // (32 rows: 1792 us a step against 1778 of the tile products on gafapel-dense, 23 rows: 1651 against 1752)
+struct LmStepGemm {
+  const bf16_t* a;       // row m's columns 8 c .. 8 c + 7 at m * lda + c * chunk (plain rows: chunk 8)
+  int64_t lda;
+  int chunk;
+  const bf16_t* w;       // [.][k]
+  int k, rows;
+  const int32_t* rows_idx;  // which rows of a (nullptr: 0, 1, ..); not for the residual epilogue
+  const float* sumsq;    // [.][sumsq_n] partial sums of squares of the rows of a before their norm
+  int sumsq_n;
+  float eps;
+  int width;             // that the mean of squares is over
+  bf16_t* out;           // rows: [rows][ldo]; otherwise [columns / 8][rows][8], residual: the next sublayer's input times its norm weight
+  int64_t ldo;
+  int out_chunk;         // = 8 * rows
+  const bf16_t* bias;
+  int ff_pad;            // SiLU gate: rows 0 .. of w are the gates, ff_pad .. the inputs
+  // residual epilogue: streams, weights around this sublayer and of the next one (nullptr: plain sum), as in LmStreams
+  float* x;
+  int64_t stride;
+  int streams, width_pad;
+  const float *prev, *next;
+  md_rms_weight norm;
+  float* sumsq_out;      // [rows][width_pad / 8]
+};
+md_status lm_step_rows(const LmStepGemm& a, int n, hipStream_t s);   // out = a w^T + bias
+md_status lm_step_silu(const LmStepGemm& a, hipStream_t s);          // out = silu(gate) * input
+md_status lm_step_resid(const LmStepGemm& a, hipStream_t s);         // streams += a w^T; out and sumsq_out for the next product
+
 // dtype: MD_DTYPE_*
 md_status lm_embed_streams(const md_lm_model* m, const int32_t* tokens, const int32_t* row_pos, float* x, int64_t stride, int rows, hipStream_t s);
 md_status lm_stream_step(int dtype, const LmStreams& a, int rows, hipStream_t s);

@@ -1,0 +1,70 @@
+"""Decode steps of few rows: products that own whole columns and go on with the row-wise step (gemm_step.hip), at the edges of their row
+tiles, for every count of streams that has a kernel of its own, beside the products that take more rows."""
+import pytest
+import torch
+
+import lm_util as U
+from oracle import layered_lm_oracle as O
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+def build(name, **kw):
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    cfg = U.CONFIGS[name] if isinstance(name, str) else name
+    return LayeredLM(LayeredLMConfig.from_dict(cfg), U.weights(cfg, 3, 1.5), dtype=BF16, max_batch=80, max_context=64, **kw)
+
+
+ONE, TWO, FOUR = (U.stream_config([(U.ssm(4, 32, 32), U.dense(320)), (U.latent(4, 32, 32, 64), U.dense(96))], width=w, vocab=200, streams=n)
+                  for n, w in ((1, 320), (2, 136), (4, 64)))
+
+
+@pytest.mark.parametrize("name", ["odd", "shared", ONE, TWO, "streams", FOUR, "five_streams"],
+                         ids=["odd", "shared", "one_stream", "two_streams", "streams", "four_streams", "five_streams"])
+def test_rows_of_a_step(name):
+    """Two tokens of 1 .. 64 sequences against the oracle (every row alone), and the logits of rows chosen among them in any order."""
+    cfg = U.CONFIGS[name] if isinstance(name, str) else name
+    m, w = build(name), U.weights(cfg, 3, 1.5)
+    ts = [U.tokens(2, cfg["vocab"], i) for i in range(64)]
+    want = torch.stack([O.forward(cfg, w, t) for t in ts])  # [64, 2, vocab]
+    scale = (want - want.mean(-1, keepdim=True)).pow(2).mean().sqrt()
+    for n in (1, 2, 8, 9, 16, 17, 28, 29, 64):
+        slots = [m.open_sequence() for _ in range(n)]
+        for k in range(2):
+            got = m.step([(s, [t[k]], [0]) for s, t in zip(slots, ts)]).double().cpu()
+            d = got - want[:n, k]
+            e = ((d - d.mean(-1, keepdim=True)).pow(2).mean(-1).sqrt() / scale).sort().values
+            # bf16 rounding through the layers, as in the other tests of whole models: 7e-2; routers enlarge it at single rows
+            assert float(e[int(0.9 * (n - 1))]) < 7e-2 and float(e[-1]) < 1.0, (n, k, e[-4:])
+        for s in slots:
+            m.close_sequence(s)
+    # both tokens of 14 sequences at once (28 rows), logits of some of them
+    slots = [m.open_sequence() for _ in range(14)]
+    places = [[1] if i % 3 == 0 else [1, 0] if i % 3 == 1 else [] for i in range(14)]
+    got = m.step([(s, t, p) for s, t, p in zip(slots, ts, places)])
+    ref = torch.cat([want[i][p] for i, p in enumerate(places) if p])
+    e = U.logit_errors(got, ref).sort().values
+    assert float(e[int(0.9 * (len(e) - 1))]) < 7e-2 and float(e[-1]) < 1.0
+    # more logits than rows
+    t = U.tokens(9, cfg["vocab"], 5)
+    got = m.step([(m.open_sequence(), t, [8, 0, 4] * 12)])
+    e = U.logit_errors(got, O.forward(cfg, w, t)[[8, 0, 4] * 12]).sort().values
+    assert float(e[len(e) // 2]) < 7e-2 and float(e[-1]) < 1.0
+    # no logits at all, then the state it left
+    a, b = m.open_sequence(), m.open_sequence()
+    assert m.step([(a, ts[0][:1], []), (b, ts[1][:1], [])]).shape[0] == 0
+    got = m.step([(a, ts[0][1:], [0]), (b, ts[1][1:], [0])])
+    assert float(U.logit_errors(got, want[:2, 1]).max()) < 0.3
+
+
+@pytest.mark.parametrize("rows", [5, 28])
+def test_residual_stream_behind_every_layer(rows):
+    for cfg in (U.CONFIGS["shared"], TWO):
+        m, t, ref, got = build(cfg), U.tokens(rows, cfg["vocab"], 0), [], []
+        O.forward(cfg, U.weights(cfg, 3, 1.5), t, layers_out=ref)
+        m.step([(m.open_sequence(), t, [])], layer_out=got)
+        for a, b in zip(got[0].double().cpu(), ref):
+            assert float((a - b).norm() / b.norm()) < 2e-2
