@@ -4,6 +4,7 @@
 //
 //   attn_prep_kernel     one workgroup per (row, q | k | v): convolution from the step's rows and the slot's last projections, norm,
 //                        query row / cache row written
+//   attn_prep_step_kernel   the same for a decode step (one row per sequence), up to 8192 columns, in registers
 //   attn_prep_block_kernel  the same for 8 positions per workgroup (prefill, up to 4096 columns)
 //   conv_state_kernel    the last projections of every sequence of the step -> its slot (row p % taps of the slot's ring)
 //   attn_plain_kernel    one workgroup per query row, fp32 on the vector ALUs: any dtype, any head size
@@ -71,11 +72,11 @@ __device__ __forceinline__ void norm_row(const LmAttn& a, int nh, float ss, cons
   for (int c = threadIdx.x * 4; c < nh * a.dp; c += 1024) put(c, *(const f32x4*)(conv_out + c) * r * *(const f32x4*)(w + c));
 }
 
-// the row's values in conv_out (complete and visible), normed per head -> cache
-template <typename T>
+// the row's values in conv_out (complete and visible), normed per head -> cache; NW waves
+template <typename T, int NW = 4>
 __device__ __forceinline__ void store_values(const LmAttn& a, int slot, int pos, const float* conv_out) {
   const int lane = threadIdx.x & 63, nh = a.kv_heads, hp = a.vp;
-  for (int g = threadIdx.x >> 6; g < nh; g += 4) {
+  for (int g = threadIdx.x >> 6; g < nh; g += NW) {
     float r = 1.0f;
     if (a.value_norm) {
       float s = 0.f;
@@ -107,6 +108,65 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(const LmAttn a) {
   } else {
     __syncthreads();
     store_values<T>(a, slot, pos, conv_out);
+  }
+}
+
+// A decode step: grid (sequences, q | k | v), 4 NI columns per thread.  What bounds it is the chain of dependent loads, so the row is its
+// sequence, everything the row needs is requested at once, and the convolved columns stay in registers (2048 columns, one row: 5.5 us
+// against 8.9; 16 rows: 7.5 against 11.4).
+template <int NI>
+__global__ __launch_bounds__(512) void attn_prep_step_kernel(const LmAttn a) {
+  extern __shared__ __attribute__((aligned(16))) float conv_out[];
+  __shared__ float red[8];
+  const int row = blockIdx.x, part = blockIdx.y, tid = threadIdx.x;  // 0 q, 1 k, 2 v
+  const int pos = a.r.row_pos[row], slot = a.r.seq_slot[row];
+  const int col0 = part == 0 ? a.col_q : part == 1 ? a.col_k : a.col_v;
+  const int ncol = part == 0 ? a.heads * a.dp : a.kv_heads * (part == 1 ? a.dp : a.vp);
+  const bf16_t* proj = (const bf16_t*)a.proj + (int64_t)row * a.ldp + col0;
+  bf16_t* ring = (bf16_t*)a.conv_state + (int64_t)slot * a.taps * a.conv_ld + col0;
+  const float *cw = a.conv + col0, *norm = part == 0 ? a.q_norm : a.k_norm;
+  f32x4 y[NI], nw[NI];
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int c = (tid + 512 * i) * 4;
+    y[i] = nw[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (c >= ncol) continue;
+    constexpr int AT_ONCE = 4;  // the newest taps
+    f32x4 u[AT_ONCE], w[AT_ONCE];
+    u[0] = ld4(proj + c);
+    w[0] = *(const f32x4*)(cw + (int64_t)(a.taps - 1) * a.conv_ld + c);
+#pragma unroll
+    for (int k = 1; k < AT_ONCE; ++k) {
+      u[k] = w[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (k < a.taps && pos - k >= 0) {
+        u[k] = ld4(ring + (int64_t)((pos - k) % a.taps) * a.conv_ld + c);
+        w[k] = *(const f32x4*)(cw + (int64_t)(a.taps - 1 - k) * a.conv_ld + c);
+      }
+    }
+    if (part < 2) nw[i] = *(const f32x4*)(norm + c);
+    for (int k = AT_ONCE; k < a.taps && pos - k >= 0; ++k)
+      y[i] += *(const f32x4*)(cw + (int64_t)(a.taps - 1 - k) * a.conv_ld + c) * ld4(ring + (int64_t)((pos - k) % a.taps) * a.conv_ld + c);
+#pragma unroll
+    for (int k = AT_ONCE - 1; k >= 0; --k) y[i] += w[k] * u[k];
+    if (a.taps > 1) st4(ring + (int64_t)(pos % a.taps) * a.conv_ld + c, u[0]);
+    ss += y[i][0] * y[i][0] + y[i][1] * y[i][1] + y[i][2] * y[i][2] + y[i][3] * y[i][3];
+    if (part == 2) *(f32x4*)(conv_out + c) = y[i];
+  }
+  if (part == 2) {
+    __syncthreads();
+    store_values<bf16_t, 8>(a, slot, pos, conv_out);
+    return;
+  }
+  ss = block_sum<8>(ss, red);
+  const float r = 1.0f / sqrtf(ss / (float)((part == 0 ? a.heads : a.kv_heads) * a.dim) + a.eps);
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int c = (tid + 512 * i) * 4;
+    if (c >= ncol) continue;
+    const f32x4 v = y[i] * r * nw[i];
+    if (part == 0) st4((bf16_t*)a.q + (int64_t)row * a.heads * a.dp + c, v);
+    else store_key4<bf16_t>(a, slot, pos, c, v);
   }
 }
 
@@ -355,7 +415,10 @@ md_status prep(const LmAttn& a, hipStream_t s) {
   const bool step = a.r.max_len == 1;
   auto fn = step ? attn_prep_kernel<T, true> : attn_prep_kernel<T, false>;
   const int mc = mx > a.kv_heads * a.dp ? mx : a.kv_heads * a.dp;
-  if (!step && mc <= 4096) {
+  if (step && sizeof(T) == 2 && mc <= 8192) {
+    auto sf = mc <= 2048 ? attn_prep_step_kernel<1> : mc <= 4096 ? attn_prep_step_kernel<2> : attn_prep_step_kernel<4>;
+    hipLaunchKernelGGL(sf, dim3(a.r.n_rows, a.own_kv ? 3 : 1), dim3(512), a.own_kv ? a.kv_heads * a.vp * 4 : 0, s, a);
+  } else if (!step && mc <= 4096) {
     auto bf = mc <= 1024 ? prep_block_pick<T, 1>(a.taps) : mc <= 2048 ? prep_block_pick<T, 2>(a.taps) : prep_block_pick<T, 4>(a.taps);
     const int ni = mc <= 1024 ? 1 : mc <= 2048 ? 2 : 4;
     const int kvc = a.kv_heads * (a.dp > a.vp ? a.dp : a.vp);
@@ -764,6 +827,7 @@ md_status lm_attn_mfma(const LmAttn& a, hipStream_t s) {
 namespace {
 
 constexpr int DTK = 64;  // keys per tile of a decode workgroup: one per lane in the mixture and the softmax
+constexpr int NWD = 8;   // its waves
 
 struct DecodeLds {
   int q, raw, p, mix, stat, total;
@@ -784,8 +848,11 @@ __host__ __device__ inline DecodeLds decode_lds(int H, int dp) {
 // queries and the row's own key and value are attn_prep_kernel's.  HPW: output heads per wave, D: dp / 32, C: vp / 32.
 // Waves read many blocks before they use the first (no branch between loads): keys of a whole tile row by groups of heads, values of one
 // head at a time; blocks past the last key are read (finite spare positions) and masked.
+// Few keys: what counts is the chain of dependent loads, a batch of key heads and a value head after the other.  Eight waves (two share the
+// heads of 16 keys) halve it: 32 heads of 64, one sequence at 50 keys 13.3 us against 19.4 with four waves; many keys are the same either
+// way (64 sequences at 1500: 4.11 ms a step of the 24-layer model against 4.08).
 template <int HPW, int D, int C>
-__global__ __launch_bounds__(256, 2) void attn_decode_kernel(const LmAttn a) {
+__global__ __launch_bounds__(64 * NWD, 2) void attn_decode_kernel(const LmAttn a) {
   extern __shared__ __attribute__((aligned(16))) char dsm[];
   const int H = a.heads, G = a.kv_heads, rep = H / G, dp = 32 * D, vp = 32 * C, hs = (H + 3) / 4 * 4;
   const DecodeLds L = decode_lds(H, dp);
@@ -798,18 +865,18 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const LmAttn a) {
   const int k0 = (first & ~31) + split * a.split_keys, k1 = min(k0 + a.split_keys - 1, i);
   float* part = a.part + ((int64_t)seq * a.n_split + split) * (H * vp + 2 * H);
   if (k0 > i) {  // nothing to see for this split
-    for (int h = tid; h < H; h += 256) {
+    for (int h = tid; h < H; h += 64 * NWD) {
       part[H * vp + 2 * h] = -INFINITY;
       part[H * vp + 2 * h + 1] = 0.f;
     }
     return;
   }
-  for (int c = tid * 8; c < H * dp; c += 2048) *(u32x4*)(qs + c) = *(const u32x4*)((const bf16_t*)a.q + (int64_t)row * H * dp + c);
-  for (int e = tid; e < H * hs; e += 256) {  // transposed, heads padded to a multiple of four
+  for (int c = tid * 8; c < H * dp; c += 512 * NWD) *(u32x4*)(qs + c) = *(const u32x4*)((const bf16_t*)a.q + (int64_t)row * H * dp + c);
+  for (int e = tid; e < H * hs; e += 64 * NWD) {  // transposed, heads padded to a multiple of four
     const int h = e % hs, g = e / hs;
     mixT[e] = h < H ? a.mix[h * H + g] : 0.f;
   }
-  for (int h = tid; h < hs; h += 256) {
+  for (int h = tid; h < hs; h += 64 * NWD) {
     ms[h] = -INFINITY;
     ls[h] = 0.f;
     sl[h] = h < H ? a.slope[h] : 0.f;
@@ -818,30 +885,31 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const LmAttn a) {
 
   const bf16_t* Kb = (const bf16_t*)a.k + (int64_t)slot * G * a.ctx * dp;
   const bf16_t* Vb = (const bf16_t*)a.v + (int64_t)slot * G * a.ctx * vp;
-  float acc[HPW][2 * C];  // heads wave, wave + 4, ..: coordinate 16 t + n16, the keys of this lane row
+  float acc[HPW][2 * C];  // heads wave, wave + NWD, ..: coordinate 16 t + n16, the keys of this lane row
 #pragma unroll
   for (int u = 0; u < HPW; ++u)
 #pragma unroll
     for (int t = 0; t < 2 * C; ++t) acc[u][t] = 0.f;
 
+  const int kwave = wave & 3, g_lo = (wave >> 2) * ((G + 1) / 2), g_hi = min(G, g_lo + (G + 1) / 2);
   for (int j0 = k0; j0 <= k1; j0 += DTK) {
     const int n = min(DTK, k1 + 1 - j0);
-    // wave w: scores of keys 16 w .. 16 w + 15, 16 query heads of one key head per matrix product
-    if (16 * wave < n) {
+    // waves w and w + 4: scores of keys 16 w .. 16 w + 15, half the key heads each, 16 query heads of one key head per matrix product
+    if (16 * kwave < n && g_lo < g_hi) {
       constexpr int UG = D >= 3 ? 2 : 4;
-      const bf16_t* kw = Kb + key_block(j0 + 16 * wave, 0, G, dp) + (wave & 1) * (D * 512) + 8 * lane;
-      const float dist = (float)(i - (j0 + 16 * wave + 4 * q4));
+      const bf16_t* kw = Kb + key_block(j0 + 16 * kwave, 0, G, dp) + (kwave & 1) * (D * 512) + 8 * lane;
+      const float dist = (float)(i - (j0 + 16 * kwave + 4 * q4));
       bf16x8 kf[2][UG][D];
       auto load = [&](int buf, int g0) {
 #pragma unroll
         for (int u = 0; u < UG; ++u)
 #pragma unroll
-          for (int d = 0; d < D; ++d) kf[buf][u][d] = *(const bf16x8*)(kw + min(g0 + u, G - 1) * (32 * dp) + 512 * d);
+          for (int d = 0; d < D; ++d) kf[buf][u][d] = *(const bf16x8*)(kw + min(g0 + u, g_hi - 1) * (32 * dp) + 512 * d);
       };
       auto scores = [&](int buf, int g0) {
 #pragma unroll
         for (int u = 0; u < UG; ++u) {
-          const int g = min(g0 + u, G - 1);
+          const int g = min(g0 + u, g_hi - 1);
           for (int r0 = 0; r0 < rep; r0 += 16) {
             const int h = g * rep + min(r0 + n16, rep - 1);
             f32x4 s = {0.f, 0.f, 0.f, 0.f};
@@ -853,13 +921,13 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const LmAttn a) {
               f32x4 o;
 #pragma unroll
               for (int e = 0; e < 4; ++e) o[e] = s[e] * a.scale - sl[h] * (dist - (float)e);
-              *(f32x4*)(raw + h * DTK + 16 * wave + 4 * q4) = o;
+              *(f32x4*)(raw + h * DTK + 16 * kwave + 4 * q4) = o;
             }
           }
         }
       };
-      load(0, 0);
-      for (int g0 = 0; g0 < G; g0 += 2 * UG) {
+      load(0, g_lo);
+      for (int g0 = g_lo; g0 < g_hi; g0 += 2 * UG) {
         load(1, g0 + UG);
         scores(0, g0);
         load(0, g0 + 2 * UG);  // (past the last head: clamped, unused)
@@ -869,7 +937,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const LmAttn a) {
     constexpr int NB = DTK / 32;
     u32x4 vf[2][NB][2 * C];
     auto load_v = [&](int u) {
-      const bf16_t* vh = Vb + key_block(j0, min(wave + 4 * u, H - 1) / rep, G, vp) + 8 * lane;
+      const bf16_t* vh = Vb + key_block(j0, min(wave + NWD * u, H - 1) / rep, G, vp) + 8 * lane;
 #pragma unroll
       for (int b = 0; b < NB; ++b)
 #pragma unroll
@@ -877,7 +945,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const LmAttn a) {
     };
     load_v(0);  // under the mixture and the softmax
     __syncthreads();
-    for (int h0 = 4 * wave; h0 < H; h0 += 16) {
+    for (int h0 = 4 * wave; h0 < H; h0 += 4 * NWD) {
       f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 8
       for (int g = 0; g < H; ++g) s += *(const f32x4*)(mixT + g * hs + h0) * raw[g * DTK + lane];
@@ -911,7 +979,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const LmAttn a) {
 #pragma unroll
     for (int u = 0; u < HPW; ++u) {
       if (u + 1 < HPW) load_v(u + 1);
-      const int h = min(wave + 4 * u, H - 1);
+      const int h = min(wave + NWD * u, H - 1);
       const float f = al[h];
 #pragma unroll
       for (int t = 0; t < 2 * C; ++t) acc[u][t] *= f;
@@ -930,7 +998,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const LmAttn a) {
   }
 #pragma unroll
   for (int u = 0; u < HPW; ++u) {
-    const int h = wave + 4 * u;
+    const int h = wave + NWD * u;
     if (h >= H) continue;
     const float inv = 1.0f / ls[h];
 #pragma unroll
@@ -944,7 +1012,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const LmAttn a) {
     }
   }
   if (a.n_split > 1)
-    for (int h = tid; h < H; h += 256) {
+    for (int h = tid; h < H; h += 64 * NWD) {
       part[H * vp + 2 * h] = ms[h];
       part[H * vp + 2 * h + 1] = ls[h];
     }
@@ -997,8 +1065,8 @@ size_t lm_attn_decode_part_floats(int n_seq, int n_split, int heads, int vp) { r
 namespace {
 template <int D, int C>
 TalkKernel decode_by_heads(int heads) {
-  return heads <= 4 ? attn_decode_kernel<1, D, C> : heads <= 8 ? attn_decode_kernel<2, D, C> : heads <= 16 ? attn_decode_kernel<4, D, C>
-         : heads <= 32 ? attn_decode_kernel<8, D, C> : heads <= 64 && D * C <= 4 ? attn_decode_kernel<16, D, C> : nullptr;
+  return heads <= 8 ? attn_decode_kernel<1, D, C> : heads <= 16 ? attn_decode_kernel<2, D, C> : heads <= 32 ? attn_decode_kernel<4, D, C>
+         : heads <= 64 && D * C <= 4 ? attn_decode_kernel<8, D, C> : nullptr;
 }
 template <int D>
 TalkKernel decode_by_width(const LmAttn& a) {
@@ -1028,7 +1096,7 @@ md_status lm_attn_decode(const LmAttn& a, hipStream_t s) {
   if (!fn) return MD_ERR_UNSUPPORTED;
   MD_TRY(md_ensure_dynamic_lds((const void*)fn, 160 * 1024));
   MD_TRY(lm_attn_prep(MD_DTYPE_BF16, a, s));
-  hipLaunchKernelGGL(fn, dim3(a.n_split, a.r.n_seq), dim3(256), decode_lds(a.heads, a.dp).total, s, a);
+  hipLaunchKernelGGL(fn, dim3(a.n_split, a.r.n_seq), dim3(64 * NWD), decode_lds(a.heads, a.dp).total, s, a);
   MD_TRY(md_launch_status());
   if (a.n_split == 1) return MD_OK;
   hipLaunchKernelGGL(attn_combine_kernel, dim3(a.heads, a.r.n_seq), dim3(256), 0, s, a);

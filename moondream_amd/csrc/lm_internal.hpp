@@ -42,14 +42,19 @@ __device__ __forceinline__ float silu_for(float z) {
   return std::is_same<T, float>::value ? silu_f32(z) : silu_fast(z);
 }
 
-// sum over a 256-thread workgroup; every thread gets it.  red: 4 floats of LDS.
-__device__ __forceinline__ float block_sum_256(float v, float* red) {
+// sum over a workgroup of N waves; every thread gets it.  red: N floats of LDS.
+template <int N>
+__device__ __forceinline__ float block_sum(float v, float* red) {
   v = wave_sum(v);
   __syncthreads();  // red may still be read from the previous call
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
-  return red[0] + red[1] + red[2] + red[3];
+  v = red[0];
+#pragma unroll
+  for (int i = 1; i < N; ++i) v += red[i];
+  return v;
 }
+__device__ __forceinline__ float block_sum_256(float v, float* red) { return block_sum<4>(v, red); }
 
 typedef __bf16 md_bf16x8v __attribute__((ext_vector_type(8)));  // what the gfx950 MFMA builtins take
 
