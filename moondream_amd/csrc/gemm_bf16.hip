@@ -691,7 +691,7 @@ template <int EPI>
 md_status launch_epi(const GemmK& k, int tile, hipStream_t stream) {
   switch (tile) {
     case 20: return md_gemm_w4_launch(k, EPI, stream);                              // 256x256, four waves (gemm_w4.hip)
-    case 1: return launch_cfg<256, 128, 4, 2, EPI>(k, stream);
+    case 1: return launch_cfg<256, 128, 4, 2, EPI, false, 3>(k, stream);
     case 3: return k.slices > 1 ? launch_cfg<64, 128, 1, 2, EPI, true, DEC_STAGES>(k, stream)
                                 : launch_cfg<64, 128, 1, 2, EPI, false, DEC_STAGES>(k, stream);
     // decode regime, 64x64 tiles: twice the tiles of 64x128 -> the wide fused layer needs no
@@ -726,7 +726,10 @@ md_status launch_epi(const GemmK& k, int tile, hipStream_t stream) {
     // weight panel per 128 rows instead of one per 64.  Same K order per output element as 16.
     case 21: return k.slices > 1 ? launch_cfg<128, 64, 4, 1, EPI, true, 4, 64, 0, 2>(k, stream)
                                  : launch_cfg<128, 64, 4, 1, EPI, false, 4, 64, 0, 2>(k, stream);
-    default: return launch_cfg<128, 128, 2, 2, EPI>(k, stream);
+    // up to one tile per CU: a ring of four instead of a second resident workgroup (216 tiles, K 2048: 32.8 -> 19.5 us)
+    default:
+      return (long)((k.M + 127) / 128) * ((k.n_store + 127) / 128) <= 256 ? launch_cfg<128, 128, 2, 2, EPI, false, 4>(k, stream)
+                                                                        : launch_cfg<128, 128, 2, 2, EPI>(k, stream);
   }
 }
 
@@ -789,6 +792,10 @@ int pick_tile(int M, int n_store, int K, int policy) {
     if (K >= 1024 && t128 <= 128) return 16;
     // ("small_m_rule": 0 = round 2's rule, 1 = the default below, n > 1 = that many tiles instead of 512 -- A/B)
     const int rule = knobs().small_m_rule;
+    //  * of these, where 256 x 128 tiles are one round of the CUs: a workgroup's loads through its CU bound all these configs (about
+    //    50 GB/s each), and 384 rows and columns per slice are fewer than two resident tiles' 512 (510 tiles, K 2048: 39.9 -> 33.0 us)
+    const long t256 = (long)((M + 255) / 256) * ((n_store + 127) / 128);
+    if (rule == 1 && t128 > 256 && t128 <= 512 && t256 <= 256) return 1;
     if (rule != 0 && t128 <= (rule > 1 ? rule : 512)) return 2;
   }
   const int bm[3] = {256, 256, 128}, bn[3] = {256, 128, 128};
@@ -966,7 +973,7 @@ extern "C" int32_t md_gemm_partial_slices(const md_linear* lin) {
 namespace {
 md_status fill_partial(GemmK& k, const void* a, int64_t lda, const md_linear* lin, int32_t m, float* partial,
                        int64_t ld_partial, int64_t slice_stride) {
-  MD_CHECK_ARG(a && lin && lin->w && partial && m > 0 && m <= 128);  // (65 .. 128 rows: the 128 x 64 tile, round 6)
+  MD_CHECK_ARG(a && lin && lin->w && partial && m > 0);
   MD_CHECK_ARG(lin->k_pad % BK == 0 && lin->k_pad >= lin->k && lin->n % 8 == 0 && lin->n_pad % 64 == 0);
   MD_CHECK_ARG(lda >= lin->k_pad && lda % 8 == 0 && ((uintptr_t)a & 15) == 0 && ((uintptr_t)lin->w & 15) == 0);
   MD_CHECK_ARG(ld_partial >= lin->n && ld_partial % 4 == 0 && ((uintptr_t)partial & 15) == 0);
@@ -1025,14 +1032,28 @@ struct ProfScope {  // HIP-event bracket of one launch for md_profile_gemm (kind
 extern "C" md_status md_gemm_partial_f32(const void* a, int64_t lda, const md_linear* lin, int32_t m,
                                          float* partial, int64_t ld_partial, int64_t slice_stride,
                                          void* stream) {
+  MD_CHECK_ARG(lin && m <= 128);  // (65 .. 128 rows: the 128 x 64 tile, round 6)
+  return md_gemm_partial_rows(a, lda, *lin, m, md_gemm_partial_slices(lin), partial, ld_partial, slice_stride, (hipStream_t)stream);
+}
+
+// More than 128 rows: where 128 x 128 tiles leave half of the CUs without one, as many slices as there are CUs.  (700 rows, 2048 columns, K 2048
+// and 5440 on average: 32.1 us as 64 x 64 tiles, 20.4 us as 2 x 96 tiles with a ring of four; the row-wise step behind reads 8 MB more, 0.7 us.)
+int md_gemm_partial_count(const md_linear& lin, int rows) {
+  if (rows <= 128) return md_gemm_partial_slices(&lin);
+  const int tiles = (rows + 127) / 128 * ((lin.n + 127) / 128);
+  return tiles > 128 || lin.k_pad < 1024 ? 0 : std::min(256 / tiles, std::min(8, lin.k_pad / BK / 4));
+}
+md_status md_gemm_partial_rows(const void* a, int64_t lda, const md_linear& lin, int m, int slices, float* partial, int64_t ld_partial,
+                               int64_t slice_stride, hipStream_t s) {
   GemmK k;
-  const md_status chk = fill_partial(k, a, lda, lin, m, partial, ld_partial, slice_stride);
-  if (chk != MD_OK) return chk;
-  hipStream_t s = (hipStream_t)stream;
+  MD_CHECK_ARG(slices > 0);
+  MD_TRY(fill_partial(k, a, lda, &lin, m, partial, ld_partial, slice_stride));
+  k.slices = slices;
   ProfScope prof;
-  if (prof.begin(2.0 * (double)lin->n * (double)lin->k, s) != MD_OK) return MD_ERR_LAUNCH;
+  if (prof.begin(2.0 * (double)lin.n * (double)lin.k, s) != MD_OK) return MD_ERR_LAUNCH;
   const int cfg = decode_cfg();
-  const md_status st = m > 64 ? launch_cfg<128, 64, 4, 1, MD_EPI_BIAS, true, 4, 64, 0, 2>(k, s)
+  const md_status st = m > 128 ? launch_cfg<128, 128, 2, 2, MD_EPI_BIAS, true, 4>(k, s)
+                       : m > 64 ? launch_cfg<128, 64, 4, 1, MD_EPI_BIAS, true, 4, 64, 0, 2>(k, s)
                        : (cfg == 17 || cfg == 18) ? launch_cfg<64, 64, 2, 2, MD_EPI_BIAS, true, 4, 64, 0, 2>(k, s)
                        : (cfg == 16 || cfg == 19) ? launch_cfg<64, 64, 2, 1, MD_EPI_BIAS, true, 4, 64, 0, 2>(k, s)
                                                   : launch_cfg<64, 64, 2, 1, MD_EPI_BIAS, true, 4>(k, s);

@@ -79,6 +79,10 @@ md_status md_gemm_grouped_bf16(const void* a, int64_t lda, const int32_t* row_of
 int md_gemm_grouped_slices(const md_linear& lin, int groups, int slots);
 md_status md_gemm_grouped_partial(const void* a, int64_t lda, const int32_t* row_of, const md_linear& lin, int groups, const int32_t* offsets, float* partial,
                                   int64_t ld, int64_t slice_stride, int slots, hipStream_t stream);
+// K-slice partial products of any number of rows: how many slices pay (0: a whole product is faster), and the launch
+int md_gemm_partial_count(const md_linear& lin, int rows);
+md_status md_gemm_partial_rows(const void* a, int64_t lda, const md_linear& lin, int rows, int slices, float* partial, int64_t ld_partial,
+                               int64_t slice_stride, hipStream_t stream);
 constexpr int MD_EPI_QKV_ROPE = 3;     // internal to the library (md_gemm_qkv_rope)
 
 // The fused layer of a decoder block at prefill with RoPE + KV write in its epilogue, when the four-wave kernel takes the

@@ -4,8 +4,9 @@
 // Prefill (more than 128 rows):  residual add + norm | input projection | mixer kernels | output projection | residual add + norm |
 //   gate/up GEMM | silu(gate) * up | down GEMM, the adds deferred into the next norm so that the fp32 residual is read and written
 //   once per half layer.
-// Decode regime (up to 128 rows, bf16):  the projections that feed a row-wise step leave fp32 K-slice partials
-//   (md_gemm_partial_f32) which that step sums: out / down -> residual add + norm, gate_up -> silu(gate) * up.
+// Where the tiles of a projection leave CUs idle (bf16), it leaves fp32 K-slice partials (md_gemm_partial_rows) which the row-wise step
+//   behind it sums: out / down -> residual add + norm; up to 128 rows also gate_up -> silu(gate) * up.
+// Few rows (LM_STEP_ROWS, bf16):  gemm_step.hip's products, which go on with the row-wise step themselves.
 // Experts:  router + choice | rows grouped by expert | grouped gate/up product | silu(gate) * up | grouped down product; the weighted sum
 //   of a row's experts is taken by the row-wise step that follows, as the sums of K-slice partials are.
 // Residual streams:  the row-wise step between two sublayers mixes them (streams.hip); x is then [streams][rows][width_pad].
@@ -59,15 +60,15 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
   auto splitk = [&](const md_linear& l, int n) {
     if (m->dtype == MD_DTYPE_BF16 && l.w && n > 0) sk = std::max(sk, md_gemm_workspace_bytes(&l, n, 1));
   };
-  auto partial = [&](const md_linear& l) {
-    if (dec && l.w) part = std::max(part, (size_t)md_gemm_partial_slices(&l) * M * l.n_pad);
+  auto partial = [&](const md_linear& l, bool residual) {
+    if (m->dtype == MD_DTYPE_BF16 && l.w && (dec || residual)) part = std::max(part, (size_t)md_gemm_partial_count(l, rows) * M * l.n_pad);
   };
   for (int i = 0; i < m->n_layers; ++i) {
     const md_lm_layer& l = m->layers[i];
     in = std::max(in, (size_t)l.in_proj.n_pad);
     att = std::max(att, (size_t)l.out_proj.k_pad);
-    partial(l.in_proj);
-    partial(l.out_proj);
+    partial(l.in_proj, true);
+    partial(l.out_proj, true);
     if (l.experts > 0) {
       const size_t T = M * l.top;
       slots = std::max(slots, T);
@@ -81,8 +82,8 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
     } else if (l.ff > 0) {
       gu = std::max(gu, M * l.gate_up.n_pad);
       act = std::max(act, M * l.down.k_pad);
-      partial(l.gate_up);
-      partial(l.down);
+      partial(l.gate_up, false);
+      partial(l.down, true);
     }
     if (l.mixer == MD_MIXER_ATTENTION) {
       q = std::max(q, (size_t)l.heads * l.dim_pad);
@@ -269,7 +270,7 @@ struct Step {
     return md_gemm_bf16(&g, s);
   }
 
-  // a mixer's projection -> w.proj.  Decode regime: K-slice partials and their sum in two launches, unless one slice fills the chip
+  // a mixer's projection -> w.proj.  Few rows: K-slice partials and their sum in two launches, unless one slice fills the chip
   md_status project(const md_linear& lin) {
     if (few && (sumsq || b->n_rows <= STEP_PLAIN_ROWS)) {
       LmStepGemm g = step_gemm(w.h, m->width_pad, lin, sumsq != nullptr);
@@ -277,10 +278,11 @@ struct Step {
       g.ldo = lin.n_pad;
       return lm_step_rows(g, lin.n_pad, s);
     }
-    const int sl = dec ? md_gemm_partial_slices(&lin) : 1;
+    int sl = m->dtype == MD_DTYPE_BF16 ? md_gemm_partial_count(lin, b->n_rows) : 0;
+    if (!dec && sl < 3) sl = 1;  // (two slices save about what the second launch takes)
     if (sl == 1) return linear(w.h, m->width_pad, lin, w.proj, lin.n_pad, b->n_rows, !dec);
     const int64_t stride = (int64_t)b->n_rows * lin.n_pad;
-    MD_TRY(md_gemm_partial_f32(w.h, m->width_pad, &lin, b->n_rows, w.part, lin.n_pad, stride, s));
+    MD_TRY(md_gemm_partial_rows(w.h, m->width_pad, lin, b->n_rows, sl, w.part, lin.n_pad, stride, s));
     return lm_reduce_rows(w.part, sl, lin.n_pad, stride, lin.b, w.proj, lin.n_pad, b->n_rows, lin.n_pad, s);
   }
 
@@ -288,11 +290,12 @@ struct Step {
   md_status to_residual(const void* a, int64_t lda, const md_linear& lin) {
     add = {};
     add.ld = m->width_pad;
-    if (dec) {
-      add.slices = md_gemm_partial_slices(&lin);
+    const int sl = m->dtype == MD_DTYPE_BF16 ? md_gemm_partial_count(lin, b->n_rows) : 0;
+    if (sl > 0) {
+      add.slices = sl;
       add.slice_stride = (int64_t)b->n_rows * lin.n_pad;
       add.src = w.part;
-      return md_gemm_partial_f32(a, lda, &lin, b->n_rows, w.part, lin.n_pad, add.slice_stride, s);
+      return md_gemm_partial_rows(a, lda, lin, b->n_rows, sl, w.part, lin.n_pad, add.slice_stride, s);
     }
     add.src = w.y;
     return linear(a, lda, lin, w.y, m->width_pad, b->n_rows);
@@ -494,9 +497,9 @@ struct Step {
       g.ff_pad = l.ff_pad;
       MD_TRY(lm_step_silu(g, s));
     } else if (dec) {
-      const int sl = md_gemm_partial_slices(&l.gate_up);
+      const int sl = md_gemm_partial_count(l.gate_up, b->n_rows);
       const int64_t ld = l.gate_up.n_pad, stride = (int64_t)b->n_rows * ld;
-      MD_TRY(md_gemm_partial_f32(w.h, m->width_pad, &l.gate_up, b->n_rows, w.part, ld, stride, s));
+      MD_TRY(md_gemm_partial_rows(w.h, m->width_pad, l.gate_up, b->n_rows, sl, w.part, ld, stride, s));
       MD_TRY(lm_reduce_silu_mul(w.part, sl, ld, stride, w.act, l.down.k_pad, b->n_rows, l.ff_pad, s));
     } else {
       MD_TRY(linear(w.h, m->width_pad, l.gate_up, w.gu, l.gate_up.n_pad, b->n_rows));

@@ -68,3 +68,20 @@ def test_residual_stream_behind_every_layer(rows):
         m.step([(m.open_sequence(), t, [])], layer_out=got)
         for a, b in zip(got[0].double().cpu(), ref):
             assert float((a - b).norm() / b.norm()) < 2e-2
+
+
+@pytest.mark.parametrize("rows", [129, 256, 300, 700])
+def test_prompts_whose_projections_leave_slices(rows):
+    """Prompts of a few hundred tokens on layers wide enough for K slices and for segments of the state space, whole and in two portions."""
+    cfg = U.stream_config([(U.ssm(8, 32, 32), U.dense(1100)), (U.latent(8, 32, 32, 64), U.dense(1030))], width=1032, vocab=200, streams=2, positions=900)
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    w = U.weights(cfg, 3, 1.5)
+    t = U.tokens(rows, cfg["vocab"], rows)
+    want = O.forward(cfg, w, t)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=BF16, max_batch=2, max_context=1024)
+    assert U.logit_error(m.step([(m.open_sequence(), t, range(rows))]), want) < 7e-2
+    s, k = m.open_sequence(), rows - 130 if rows > 400 else 1
+    got = torch.cat([m.step([(s, t[:k], range(k))]), m.step([(s, t[k:], range(rows - k))])])
+    assert U.logit_error(got, want) < 7e-2
