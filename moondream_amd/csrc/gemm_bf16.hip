@@ -205,7 +205,11 @@ __device__ __forceinline__ void gemm_body(const GemmK& p) {
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
       const int slot = j * NT + dtid, r = slot >> CH_SHIFT, c = (slot & (CH - 1)) ^ ((r >> (4 - CH_SHIFT)) & (CH - 1));
-      const int64_t row = min(n0 + r, p.n_pad - 1);
+      int64_t row = min(n0 + r, p.n_pad - 1);
+      if constexpr (EPI == MD_EPI_SILU) {  // 32 gates, then the inputs of the same 32 columns: a wave's two column blocks
+        const int v = n0 + r, half = p.n_pad >> 1;
+        row = min((v >> 6) * 32 + (v & 31), half - 1) + ((v & 32) ? half : 0);
+      }
       b_src[j] = (const char*)(W + row * p.ldw + c * 8);
     }
   };
@@ -521,6 +525,32 @@ __device__ __forceinline__ void gemm_body(const GemmK& p) {
   const uint32_t tile_lds = lds_base + (PERSIST ? STAGES * STAGE : 0) + wave * 4096;
   const int wn0 = n0c + wn * TN;
 
+  if constexpr (EPI == MD_EPI_SILU) {
+    static_assert(NI == 2 && !PERSIST && !SPLITK, "a wave's column blocks are 32 gates and their inputs");
+    // 32 rows x 32 columns at a time through the wave's LDS tile (64-byte rows, chunks swizzled)
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        float y[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float z = acc[i][0][4 * g + e], u = acc[i][1][4 * g + e];
+          if (p.round_first) z = bf2f(f2bf(z)), u = bf2f(f2bf(u));  // (uniform)
+          y[e] = silu_fast(z) * u;
+        }
+        *(u32x2*)(tile + l31 * 64 + ((g ^ ((l31 >> 1) & 3)) * 16) + hi * 8) = u32x2{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
+      }
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int idx = q * 64 + lane, row = idx >> 2, ch = idx & 3;
+        const u32x4 v = *(const u32x4*)(tile + row * 64 + ((ch ^ ((row >> 1) & 3)) * 16));
+        const int m = m0c + wm * TM + 32 * i + row, n = (wn0 >> 1) + ch * 8;
+        if (m < m_end && n < (p.n_store >> 1)) *(u32x4*)(p.C + (int64_t)m * p.ldc + n) = v;
+      }
+    }
+    return;
+  }
   float bias_v[NI][4][4];
 #pragma unroll
   for (int j = 0; j < NI; ++j)
@@ -652,14 +682,14 @@ __global__ __launch_bounds__((WM * WN + XW) * 64) void gemm_pair_kernel(const Ge
   gemm_body<BM, BN, WM, WN, EPI, SPLITK, STAGES, BKT, PP, XW>(pair.g[blockIdx.z]);
 }
 
-template <int BM, int BN, int WM, int WN, bool SPLITK, int STAGES, int BKT, int PP, int XW>
+template <int BM, int BN, int WM, int WN, int EPI, bool SPLITK, int STAGES, int BKT, int PP, int XW>
 __global__ __launch_bounds__((WM * WN + XW) * 64) void gemm_grouped_kernel(const GemmK p) {
-  gemm_body<BM, BN, WM, WN, MD_EPI_BIAS, SPLITK, STAGES, BKT, PP, XW, true>(p);
+  gemm_body<BM, BN, WM, WN, EPI, SPLITK, STAGES, BKT, PP, XW, true>(p);
 }
-template <int BM, int BN, int WM, int WN, bool SPLITK, int STAGES, int BKT = 64, int PP = 0, int XW = 0>
+template <int BM, int BN, int WM, int WN, int EPI, bool SPLITK, int STAGES, int BKT = 64, int PP = 0, int XW = 0>
 md_status launch_grouped(GemmK k, hipStream_t stream) {
   constexpr int ring = STAGES * (BM + BN) * BKT * 2, epi = WM * WN * 4096, lds = ring > epi ? ring : epi;
-  auto fn = gemm_grouped_kernel<BM, BN, WM, WN, SPLITK, STAGES, BKT, PP, XW>;
+  auto fn = gemm_grouped_kernel<BM, BN, WM, WN, EPI, SPLITK, STAGES, BKT, PP, XW>;
   MD_TRY(md_ensure_dynamic_lds((const void*)fn, lds));
   k.tiles_m = grouped_tiles(k.M, k.groups, BM);
   k.tiles_n = (k.n_store + BN - 1) / BN;
@@ -1091,20 +1121,56 @@ md_status fill_grouped(GemmK& k, const void* a, int64_t lda, const int32_t* row_
 }
 }  // namespace
 
+namespace {
+// per_group: the expected rows of a group.  The four-wave tile from 64 on: it moves the fewest bytes per product, which bounds all of them,
+// though most of its rows are padding at first (a whole prefill through 32 experts of 2 x 1360 columns, 24 layers: 87 rows a group 8.29 -> 7.78 ms
+// against the 64 x 64 tile, 212 rows 11.8 -> 10.8 against 128 x 128, 612 rows 24.4 -> 21.5 and 1000 rows 35.3 -> 30.9 against an eight-wave
+// 256 x 256 tile; 50 rows: 7.15 either way).
+template <int EPI>
+md_status grouped_by_height(GemmK k, int per_group, hipStream_t stream) {
+  if (per_group >= 64 && k.n_pad >= 256 && md_gemm_w4_takes(k, EPI) && (uint64_t)k.groups * k.n_pad * k.ldw * 2 < (1ull << 32)) {
+    k.group_m = 4;
+    return md_gemm_w4_launch_grouped(k, EPI, stream);
+  }
+  if (per_group >= 96) return launch_grouped<128, 128, 2, 2, EPI, false, 2>(k, stream);
+  return launch_grouped<64, 64, 2, 1, EPI, false, 4, 64, 0, 2>(k, stream);
+}
+}  // namespace
 md_status md_gemm_grouped_bf16(const void* a, int64_t lda, const int32_t* row_of, const md_linear& lin, int groups, const int32_t* offsets, void* c,
-                               int64_t ldc, int slots, hipStream_t stream) {
+                               int64_t ldc, int slots, bool silu, bool round_first, hipStream_t stream) {
   GemmK k;
   MD_TRY(fill_grouped(k, a, lda, row_of, lin, groups, offsets, slots));
-  MD_CHECK_ARG(c && ldc >= lin.n_pad && ldc % 8 == 0 && ((uintptr_t)c & 15) == 0);
+  MD_CHECK_ARG(c && ldc >= (silu ? lin.n_pad / 2 : lin.n_pad) && ldc % 8 == 0 && ((uintptr_t)c & 15) == 0 && (!silu || lin.n_pad % 128 == 0));
   k.C = (bf16_t*)c;
   k.ldc = ldc;
+  k.round_first = round_first;
   const int per_group = slots / groups;  // the expected height of a group
-  if (per_group >= 512 && lin.n_pad >= 256) {
-    k.group_m = 4;
-    return launch_grouped<256, 256, 2, 4, false, 4, 32, 2>(k, stream);
+  return silu ? grouped_by_height<MD_EPI_SILU>(k, per_group, stream) : grouped_by_height<MD_EPI_BIAS>(k, per_group, stream);
+}
+
+// What a separate launch for the gate cost: 5.6 us at 700 rows of 5440 columns, 104 us at 16384, 4.6 us behind the K slices of a decode step.
+md_status md_gemm_silu_bf16(const void* a, int64_t lda, const md_linear& lin, void* c, int64_t ldc, int rows, hipStream_t s) {
+  GemmK k;
+  MD_CHECK_ARG(lin.n == lin.n_pad && lin.n_pad % 128 == 0 && !lin.b && c && ldc >= lin.n_pad / 2 && ldc % 8 == 0 && ((uintptr_t)c & 15) == 0);
+  MD_TRY(fill_partial(k, a, lda, &lin, rows, (float*)c, lin.n, (int64_t)rows * lin.n));  // (checks; the rest as a whole product)
+  k.partial = nullptr;
+  k.slices = 1;
+  k.C = (bf16_t*)c;
+  k.ldc = ldc;
+  k.group_m = md_gemm_auto_group_m_w4(k.n_store, k.K);
+  k.round_first = rows > 128;
+  int tile = rows <= 64 ? 16 : rows <= 128 ? 21 : pick_tile(rows, k.n_store, k.K, MD_TILE_BY_SHAPE);
+  if (tile == 20 && !md_gemm_w4_takes(k, MD_EPI_SILU)) tile = 11;
+  switch (tile) {
+    case 20: return md_gemm_w4_launch(k, MD_EPI_SILU, s);
+    case 11: return launch_cfg<256, 256, 2, 4, MD_EPI_SILU, false, 4, 32, 2>(k, s);
+    case 21: return launch_cfg<128, 64, 4, 1, MD_EPI_SILU, false, 4, 64, 0, 2>(k, s);
+    case 16: return launch_cfg<64, 64, 2, 1, MD_EPI_SILU, false, 4, 64, 0, 2>(k, s);
+    case 1: return launch_cfg<256, 128, 4, 2, MD_EPI_SILU, false, 3>(k, s);
+    default:
+      return (long)((rows + 127) / 128) * ((k.n_store + 127) / 128) <= 256 ? launch_cfg<128, 128, 2, 2, MD_EPI_SILU, false, 4>(k, s)
+                                                                         : launch_cfg<128, 128, 2, 2, MD_EPI_SILU>(k, s);
   }
-  if (per_group >= 96) return launch_grouped<128, 128, 2, 2, false, 2>(k, stream);
-  return launch_grouped<64, 64, 2, 1, false, 4, 64, 0, 2>(k, stream);
 }
 
 int md_gemm_grouped_slices(const md_linear& lin, int groups, int slots) {
@@ -1120,7 +1186,7 @@ md_status md_gemm_grouped_partial(const void* a, int64_t lda, const int32_t* row
   k.partial_ld = ld;
   k.partial_slice_stride = slice_stride;
   k.slices = md_gemm_grouped_slices(lin, groups, slots);
-  return launch_grouped<64, 64, 2, 1, true, 4, 64, 0, 2>(k, stream);
+  return launch_grouped<64, 64, 2, 1, MD_EPI_BIAS, true, 4, 64, 0, 2>(k, stream);
 }
 
 // Both partial-product GEMMs of a decode block (proj over the attention output, fc2 over

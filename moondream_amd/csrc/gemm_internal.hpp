@@ -39,6 +39,7 @@ struct GemmK {
   const int32_t* row_of = nullptr;
   int groups = 0;
   int64_t group_stride = 0;
+  int round_first = 0;  // MD_EPI_SILU: gate and input are rounded to bf16 before they are multiplied (more than 128 rows), or not
 };
 
 // Row tiles of a grouped product: every group has its own ceil(rows / bm) tiles.  How many a launch needs at most, and which group and rows
@@ -72,9 +73,22 @@ __device__ __forceinline__ bool grouped_tile(const int32_t* offsets, int groups,
   return false;
 }
 
-// C[s] = A[row_of[s]] . W_g^T for the slots s of every group g (bf16; lin: one group's matrix, n == n_pad, all follow one another)
+// row tiles that the groups have
+__device__ __forceinline__ int grouped_total(const int32_t* offsets, int groups, int bm) {
+  const int lane = threadIdx.x & 63;
+  int n = 0;
+  for (int g = lane; g < groups; g += 64) n += (offsets[g + 1] - offsets[g] + bm - 1) / bm;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
+  return __builtin_amdgcn_readfirstlane(n);
+}
+
+// C[s] = A[row_of[s]] . W_g^T for the slots s of every group g (bf16; lin: one group's matrix, n == n_pad, all follow one another).
+// silu: the matrix is [gate | input], C[s] = silu(gate) * input
 md_status md_gemm_grouped_bf16(const void* a, int64_t lda, const int32_t* row_of, const md_linear& lin, int groups, const int32_t* offsets, void* c,
-                               int64_t ldc, int slots, hipStream_t stream);
+                               int64_t ldc, int slots, bool silu, bool round_first, hipStream_t stream);
+// C = silu(gate) * input of A . [gate | input]^T in one launch (bf16; n == n_pad, no bias)
+md_status md_gemm_silu_bf16(const void* a, int64_t lda, const md_linear& lin, void* c, int64_t ldc, int rows, hipStream_t stream);
 // the same as fp32 K-slice partial products [slice][slot][ld] (few rows per group)
 int md_gemm_grouped_slices(const md_linear& lin, int groups, int slots);
 md_status md_gemm_grouped_partial(const void* a, int64_t lda, const int32_t* row_of, const md_linear& lin, int groups, const int32_t* offsets, float* partial,
@@ -84,6 +98,7 @@ int md_gemm_partial_count(const md_linear& lin, int rows);
 md_status md_gemm_partial_rows(const void* a, int64_t lda, const md_linear& lin, int rows, int slices, float* partial, int64_t ld_partial,
                                int64_t slice_stride, hipStream_t stream);
 constexpr int MD_EPI_QKV_ROPE = 3;     // internal to the library (md_gemm_qkv_rope)
+constexpr int MD_EPI_SILU = 4;         // internal: columns are [gate | input], C = silu(gate) * input, half as wide
 
 // The fused layer of a decoder block at prefill with RoPE + KV write in its epilogue, when the four-wave kernel takes the
 // shape (MD_ERR_UNSUPPORTED otherwise: the caller runs md_gemm_bf16 + md_rope_kv_write).  MHA, head_dim 64, rot_dim 32.
@@ -110,6 +125,7 @@ md_status md_gemm_f8_qkv_rope(const md_gemm_f8_args* a, const md_rope_fuse* rf, 
 // gemm_w4.hip: the 256x256 tile kernel with one wave per SIMD (4 waves x 128x128), persistent.
 // epi = MD_EPI_*.  Fills tiles_m / tiles_n itself.
 md_status md_gemm_w4_launch(const GemmK& k, int epi, hipStream_t stream);
+md_status md_gemm_w4_launch_grouped(const GemmK& k, int epi, hipStream_t stream);  // k.offsets: bias-free rows or MD_EPI_SILU
 bool md_gemm_w4_takes(const GemmK& k, int epi);  // shape limits of the four-wave kernel for this launch
 void md_gemm_w4_set_grid(int v);     // persistent workgroups per launch of the four-wave kernel (0 = one per CU)
 void md_gemm_w4_set_debug(int half, uint32_t v);  // measurement builds: device buffer for in-kernel stamps

@@ -177,7 +177,8 @@ constexpr int frag_wait(int m) {
 
 // ABL: measurement builds (bit 1: no operand DMA, 2: no barrier, 3: no fragment reads, 4: no epilogue stores, 5: no
 // epilogue, 6: shader-clock stamps around the waits of gap 64 and the epilogue, 8: every operand load from one L2-resident MiB); results are garbage with bits 1-5 set.
-template <int EPI, int ABL = 0, int MODE = 1>
+// GRP: a grouped product (GemmK.offsets): a tile's rows are slots of one group, gathered through row_of, its matrix is that group's.
+template <int EPI, int ABL = 0, int MODE = 1, bool GRP = false>
 __global__ __launch_bounds__(256) void gemm_w4_kernel(const GemmK p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x;
@@ -187,7 +188,9 @@ __global__ __launch_bounds__(256) void gemm_w4_kernel(const GemmK p) {
   const int g4 = lane >> 4, l15 = lane & 15;
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
 
-  const int nwg = p.tiles_m * p.tiles_n;
+  const int tiles_m = GRP ? grouped_total(p.offsets, p.groups, BM) : p.tiles_m;  // (a grouped launch knows an upper bound)
+  const int nwg = tiles_m * p.tiles_n;
+  if (GRP && (int)blockIdx.x >= nwg) return;
   const int npair = p.K / 64;  // pairs of 32-wide K steps per tile
   int grid_x = gridDim.x;      // pinned in a scalar register: re-read from the dispatch packet inside the stream it is an
   asm volatile("" : "+s"(grid_x));  // s_load + lgkmcnt(0) in the middle of a pair
@@ -195,12 +198,17 @@ __global__ __launch_bounds__(256) void gemm_w4_kernel(const GemmK p) {
   // workgroup sequence number -> tile: XCD-contiguous remap, then grouped (group_m row panels x all
   // column panels) order, so the 32 workgroups of an XCD that run together cover a compact block
   const int per_group = p.group_m * p.tiles_n;
-  auto tile_origin = [&](int vv, int& m0, int& n0) {
+  // m_end: rows from there on belong to another group, or to nobody
+  auto tile_origin = [&](int vv, int& m0, int& n0, int& m_end, int& group) {
     const int L = xcd_remap(vv, nwg);
     const int first_m = (L / per_group) * p.group_m;
-    const int gsz = min(p.tiles_m - first_m, p.group_m);
-    m0 = (first_m + (L % per_group) % gsz) * BM;
+    const int gsz = min(tiles_m - first_m, p.group_m);
+    const int tm = first_m + (L % per_group) % gsz;
     n0 = ((L % per_group) / gsz) * BN;
+    m0 = tm * BM;
+    m_end = p.M;
+    group = 0;
+    if constexpr (GRP) grouped_tile(p.offsets, p.groups, BM, tm, group, m0, m_end);
   };
 
   // ---- load cursor: one pair (64 K elements) at a time, across tile boundaries --------------------------------
@@ -214,15 +222,29 @@ __global__ __launch_bounds__(256) void gemm_w4_kernel(const GemmK p) {
   int ld_tile = blockIdx.x, ld_pair = 0;
   uint32_t ld_soff = 0;
   auto set_load_tile = [&](int vv) {
-    int m0, n0;
-    tile_origin(vv, m0, n0);
+    int m0, n0, m_end, group;
+    tile_origin(vv, m0, n0, m_end, group);
     const int r8 = lane >> 3;
+    int a_row[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) a_row[j] = min(m0 + 64 * wave + 8 * j + r8, m_end - 1);
+    if constexpr (GRP)
+      if (p.row_of) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) a_row[j] = p.row_of[a_row[j]];
+      }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int row = 64 * wave + 8 * j + r8, c8 = (lane & 7) ^ ((row >> 1) & 7);
       const uint32_t fix = 4096u - (uint32_t)(j & 3) * 1024u + c8 * 16;
-      voff[j] = (uint32_t)min(m0 + row, p.M - 1) * (uint32_t)(p.lda * 2) + fix;
-      voff[8 + j] = (uint32_t)min(n0 + row, p.n_pad - 1) * (uint32_t)(p.ldw * 2) + fix;
+      int w_row = min(n0 + row, p.n_pad - 1);
+      if constexpr (EPI == MD_EPI_SILU) {  // 16 gates, then the inputs of the same 16 columns: neighbouring accumulator blocks
+        const int v = n0 + row, half = p.n_pad >> 1;
+        w_row = min((v >> 5) * 16 + (v & 15), half - 1) + ((v & 16) ? half : 0);
+      }
+      if constexpr (GRP) w_row += group * p.n_pad;
+      voff[j] = (uint32_t)a_row[j] * (uint32_t)(p.lda * 2) + fix;
+      voff[8 + j] = (uint32_t)w_row * (uint32_t)(p.ldw * 2) + fix;
     }
   };
   set_load_tile(ld_tile);
@@ -387,8 +409,8 @@ __global__ __launch_bounds__(256) void gemm_w4_kernel(const GemmK p) {
 
   // ---- tile loop ------------------------------------------------------------------------------
   for (int vtile = blockIdx.x; vtile < nwg; vtile += grid_x) {
-    int m0c, n0c;
-    tile_origin(vtile, m0c, n0c);
+    int m0c, n0c, m_end, group;
+    tile_origin(vtile, m0c, n0c, m_end, group);
     const int wm0 = m0c + wm * 128, wn0 = n0c + wn * 128;
     bias_soff = (uint32_t)wn0 * 2u;
     // the accumulators are (re)defined by the first K step of every tile: nothing is carried from
@@ -420,7 +442,7 @@ __global__ __launch_bounds__(256) void gemm_w4_kernel(const GemmK p) {
     }
     // C (and a residual R, and the KV slabs) are addressed through buffer resources: rows past M read as zero / are dropped by
     // the range check (no exec masking, no branch); an address is one 32-bit offset.
-    const __amdgpu_buffer_rsrc_t rsrc_c = __builtin_amdgcn_make_buffer_rsrc((void*)p.C, 0, (int)min((uint64_t)p.M * (uint64_t)p.ldc * 2, (uint64_t)0xffffffffu), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_c = __builtin_amdgcn_make_buffer_rsrc((void*)p.C, 0, (int)min((uint64_t)(GRP ? m_end : p.M) * (uint64_t)p.ldc * 2, (uint64_t)0xffffffffu), 0x00020000);
     // Eight passes of 32 rows x 64 columns (row pair ip = i / 2, column half jp) through the wave's LDS tile.
     // write side, on the accumulator layout: bias add + ONE bf16 rounding (F.linear's rounding point); a lane's quad of 4 columns
     // = 8 bytes at row 16 (i & 1) + l15, chunk 2 jj + (g4 >> 1), half g4 & 1 (chunks swizzled by row & 7).  Read side: piece q
@@ -576,7 +598,61 @@ __global__ __launch_bounds__(256) void gemm_w4_kernel(const GemmK p) {
         MD_PIN();
       });
     };
-    if constexpr (EPI == MD_EPI_QKV_ROPE) {
+    // MD_EPI_SILU: accumulator blocks 2 j and 2 j + 1 are gates and inputs of 16 columns, so a pass of 32 rows x 64 columns is a row pair of
+    // the wave's quarter; gates and inputs are rounded to bf16 before they meet (k.round_first is always set here)
+    auto silu_epilogue = [&]() {
+      const int lane_row = lane >> 3, lane_col = (lane & 7) * 8;
+      const int c0 = (wn0 >> 1) + lane_col;
+      const bool col_ok = c0 < (p.n_store >> 1);
+      const uint32_t c_base = (uint32_t)(wm0 + lane_row) * (uint32_t)(p.ldc * 2) + (uint32_t)c0 * 2u, c_step = (uint32_t)p.ldc * 16u;
+      auto convert_write = [&](auto pc) {
+        constexpr int ip = decltype(pc)::value;
+        static_for<0, 2>([&](auto iic) {
+          constexpr int ii = decltype(iic)::value, i = 2 * ip + ii;
+          const uint32_t row = 16 * ii + l15, row_lds = tile_lds + row * 128;
+          static_for<0, 4>([&](auto jjc) {
+            constexpr int jj = decltype(jjc)::value, base = 4 * (8 * i + 2 * jj);
+            u32x2 o;
+            static_for<0, 2>([&](auto hc) {
+              constexpr int at = base + 2 * decltype(hc)::value;
+              const uint32_t z = pack_bf16x2(acc_read<at>(), acc_read<at + 1>()), u = pack_bf16x2(acc_read<at + 4>(), acc_read<at + 5>());
+              o[decltype(hc)::value] = pack_bf16x2(silu_fast(lo_bf(z)) * lo_bf(u), silu_fast(hi_bf(z)) * hi_bf(u));
+            });
+            ds_write_b64_asm(row_lds + (((2 * jj + (g4 >> 1)) ^ (row & 7)) * 16) + (g4 & 1) * 8, o);
+          });
+        });
+      };
+      u32x4 tv[2][4];
+      auto read_pieces = [&](u32x4 (&t)[4]) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int idx = q * 64 + lane, row = idx >> 3, ch = idx & 7;
+          ds_read_b128_u32(t[q], tile_lds + row * 128 + ((ch ^ (row & 7)) * 16));
+        }
+      };
+      convert_write(I0{});
+      read_pieces(tv[0]);
+      MD_PIN();
+      static_for<0, 4>([&](auto pc) {
+        constexpr int ip = decltype(pc)::value;
+        if constexpr (ip + 1 < 4) {
+          convert_write(std::integral_constant<int, ip + 1>{});
+          wait_lgkm<8>();  // this pass's four reads are back; the next pass's eight writes may still be on their way
+        } else {
+          wait_lgkm<0>();
+        }
+        MD_PIN();
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          __builtin_amdgcn_raw_buffer_store_b128(tv[ip & 1][q], rsrc_c, col_ok ? c_base + (uint32_t)(4 * ip + q) * c_step : 0xfffff000u, 0, 0);
+        MD_PIN();
+        if constexpr (ip + 1 < 4) read_pieces(tv[(ip + 1) & 1]);
+        MD_PIN();
+      });
+    };
+    if constexpr (EPI == MD_EPI_SILU) {
+      silu_epilogue();
+    } else if constexpr (EPI == MD_EPI_QKV_ROPE) {
       const int sec = wn0 / p.rope_d;  // 0 q, 1 k, 2 v, >= 3: the fc1 columns   (wave-uniform)
       if (sec == 0) lds_epilogue(std::integral_constant<int, 1>{});
       else if (sec == 1) lds_epilogue(std::integral_constant<int, 2>{});
@@ -607,13 +683,13 @@ int g_w4_variant = [] { const char* e = getenv("MD_W4_VARIANT"); return (e && *e
 uint64_t g_w4_debug = 0;  // measurement builds: device buffer for the in-kernel stamps (md_gemm_set_tuning "w4_dbg_lo" / "w4_dbg_hi")
 constexpr int kDefaultMode = 2;
 
-template <int EPI, int ABL = 0, int MODE = kDefaultMode>
+template <int EPI, int ABL = 0, int MODE = kDefaultMode, bool GRP = false>
 md_status launch(const GemmK& k, hipStream_t stream) {
-  auto fn = gemm_w4_kernel<EPI, ABL, MODE>;
+  auto fn = gemm_w4_kernel<EPI, ABL, MODE, GRP>;
   MD_TRY(md_ensure_dynamic_lds((const void*)fn, LDS_BYTES));
   GemmK kk = k;
   if constexpr (ABL & 64) kk.slabs = (float*)(uintptr_t)g_w4_debug;
-  kk.tiles_m = (k.M + BM - 1) / BM;
+  kk.tiles_m = GRP ? grouped_tiles(k.M, k.groups, BM) : (k.M + BM - 1) / BM;
   kk.tiles_n = (k.n_store + BN - 1) / BN;
   const int nwg = kk.tiles_m * kk.tiles_n;
   static const int n_cu = [] {
@@ -687,6 +763,16 @@ md_status md_gemm_w4_launch(const GemmK& k, int epi, hipStream_t stream) {
     case MD_EPI_GELU: return launch<MD_EPI_GELU>(k, stream);
     case MD_EPI_RESIDUAL: return launch<MD_EPI_RESIDUAL>(k, stream);
     case MD_EPI_QKV_ROPE: return launch<MD_EPI_QKV_ROPE>(k, stream);
+    case MD_EPI_SILU: return launch<MD_EPI_SILU>(k, stream);
     default: return MD_ERR_INVALID_ARG;
   }
+}
+
+md_status md_gemm_w4_launch_grouped(const GemmK& k, int epi, hipStream_t stream) {
+  if (k.K % 64 != 0 || k.M <= 0 || !k.offsets || k.groups <= 0 || k.bias) return MD_ERR_INVALID_ARG;
+  // 32-bit byte offsets over all groups' matrices
+  if (!md_gemm_w4_takes(k, epi) || (uint64_t)k.groups * (uint64_t)k.n_pad * (uint64_t)k.ldw * 2 >= (1ull << 32)) return MD_ERR_UNSUPPORTED;
+  if (epi == MD_EPI_SILU) return launch<MD_EPI_SILU, 0, kDefaultMode, true>(k, stream);
+  if (epi == MD_EPI_BIAS) return launch<MD_EPI_BIAS, 0, kDefaultMode, true>(k, stream);
+  return MD_ERR_INVALID_ARG;
 }

@@ -2,12 +2,12 @@
 // of experts, as a sequence of this library's launches.  Nothing here allocates or synchronises.
 //
 // Prefill (more than 128 rows):  residual add + norm | input projection | mixer kernels | output projection | residual add + norm |
-//   gate/up GEMM | silu(gate) * up | down GEMM, the adds deferred into the next norm so that the fp32 residual is read and written
+//   gate/up GEMM with silu(gate) * up | down GEMM, the adds deferred into the next norm so that the fp32 residual is read and written
 //   once per half layer.
 // Where the tiles of a projection leave CUs idle (bf16), it leaves fp32 K-slice partials (md_gemm_partial_rows) which the row-wise step
-//   behind it sums: out / down -> residual add + norm; up to 128 rows also gate_up -> silu(gate) * up.
+//   behind it sums: out / down -> residual add + norm; up to 128 rows also gate_up -> silu(gate) * up (otherwise the product's epilogue).
 // Few rows (LM_STEP_ROWS, bf16):  gemm_step.hip's products, which go on with the row-wise step themselves.
-// Experts:  router + choice | rows grouped by expert | grouped gate/up product | silu(gate) * up | grouped down product; the weighted sum
+// Experts:  router + choice | rows grouped by expert | grouped gate/up product with silu(gate) * up | grouped down product; the weighted sum
 //   of a row's experts is taken by the row-wise step that follows, as the sums of K-slice partials are.
 // Residual streams:  the row-wise step between two sublayers mixes them (streams.hip); x is then [streams][rows][width_pad].
 #include "gemm_internal.hpp"
@@ -39,13 +39,18 @@ struct LmWs {
 
 inline bool decode_regime(const md_lm_model* m, int rows) { return m->dtype == MD_DTYPE_BF16 && rows <= DECODE_ROWS; }
 
-// Most rows for which a product of gemm_step.hip is the faster one where nothing is saved behind it: rows that were normed in a launch of
-// their own (10304 columns, 16 rows: 15.2 us, the tile product 14.4), and the head (51200 columns; 1 row: 41-47 us against 55 with its norm, 16
-// rows: 59 against 56, 32 rows: 85).
+// Most rows for which a product of gemm_step.hip is the faster one where nothing is saved behind it: the head (51200 columns; 1 row: 41-47 us
+// against 55 with its norm, 16 rows: 59 against 56, 32 rows: 85), and the first layer's projection.
 constexpr int STEP_PLAIN_ROWS = 8;
 
 // products that go on with the row-wise step behind them (gemm_step.hip)
-inline bool step_regime(const md_lm_model* m, int rows) { return m->dtype == MD_DTYPE_BF16 && rows <= LM_STEP_ROWS; }
+// (a router needs whole normed rows, which leaves nothing to go on with)
+inline bool step_regime(const md_lm_model* m, int rows) {
+  if (m->dtype != MD_DTYPE_BF16 || rows > LM_STEP_ROWS) return false;
+  for (int i = 0; i < m->n_layers; ++i)
+    if (m->layers[i].experts > 0) return false;
+  return true;
+}
 
 inline bool own_row_steps(const md_lm_model* m) { return m->streams > 0 || m->pos || m->embed_norm.w; }
 inline int n_streams(const md_lm_model* m) { return m->streams > 0 ? m->streams : 1; }
@@ -73,14 +78,14 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
       const size_t T = M * l.top;
       slots = std::max(slots, T);
       experts = std::max(experts, (size_t)l.experts);
-      gu = std::max(gu, T * l.gate_up.n_pad);
+      if (m->dtype == MD_DTYPE_F32) gu = std::max(gu, T * l.gate_up.n_pad);
       act = std::max(act, T * l.down.k_pad);
       y = std::max(y, T * m->width_pad);
       if (dec)
         part = std::max(part, std::max((size_t)md_gemm_grouped_slices(l.gate_up, l.experts, (int)T) * T * l.gate_up.n_pad,
                                        (size_t)md_gemm_grouped_slices(l.down, l.experts, (int)T) * T * l.down.n_pad));
     } else if (l.ff > 0) {
-      gu = std::max(gu, M * l.gate_up.n_pad);
+      if (m->dtype == MD_DTYPE_F32) gu = std::max(gu, M * l.gate_up.n_pad);
       act = std::max(act, M * l.down.k_pad);
       partial(l.gate_up, false);
       partial(l.down, true);
@@ -301,11 +306,10 @@ struct Step {
     return linear(a, lda, lin, w.y, m->width_pad, b->n_rows);
   }
 
-  // a sublayer's last projection.  Few rows: the residual stream(s) and the input of the next sublayer (nw == nullptr: it needs whole
-  // normed rows) in the same launch
-  md_status finish(const void* a, int64_t lda, const md_linear& lin, bool ordered, const float* prev, const md_rms_weight* nw, const float* next) {
+  // a sublayer's last projection.  Few rows: the residual stream(s) and the input of the next sublayer in the same launch
+  md_status finish(const void* a, int64_t lda, const md_linear& lin, bool ordered, const float* prev, const md_rms_weight& nw, const float* next) {
     mix = prev;
-    if (!few || !nw) return to_residual(a, lda, lin);
+    if (!few) return to_residual(a, lda, lin);
     LmStepGemm g = step_gemm(a, lda, lin, ordered);
     g.out = (bf16_t*)w.h;
     g.x = w.x;
@@ -314,7 +318,7 @@ struct Step {
     g.width_pad = m->width_pad;
     g.prev = prev;
     g.next = next;
-    g.norm = *nw;
+    g.norm = nw;
     g.sumsq_out = w.sumsq;
     sumsq = w.sumsq;
     ready = true;
@@ -486,7 +490,7 @@ struct Step {
     }
   }
 
-  md_status feed_forward(const md_lm_layer& l, const md_rms_weight* nw, const float* next) {
+  md_status feed_forward(const md_lm_layer& l, const md_rms_weight& nw, const float* next) {
     if (l.experts > 0) {
       mix = l.mix2;
       return expert_forward(l);
@@ -496,6 +500,8 @@ struct Step {
       g.out = (bf16_t*)w.act;
       g.ff_pad = l.ff_pad;
       MD_TRY(lm_step_silu(g, s));
+    } else if (m->dtype == MD_DTYPE_BF16 && (!dec || md_gemm_partial_count(l.gate_up, b->n_rows) == 1)) {
+      MD_TRY(md_gemm_silu_bf16(w.h, m->width_pad, l.gate_up, w.act, l.down.k_pad, b->n_rows, s));
     } else if (dec) {
       const int sl = md_gemm_partial_count(l.gate_up, b->n_rows);
       const int64_t ld = l.gate_up.n_pad, stride = (int64_t)b->n_rows * ld;
@@ -503,7 +509,7 @@ struct Step {
       MD_TRY(lm_reduce_silu_mul(w.part, sl, ld, stride, w.act, l.down.k_pad, b->n_rows, l.ff_pad, s));
     } else {
       MD_TRY(linear(w.h, m->width_pad, l.gate_up, w.gu, l.gate_up.n_pad, b->n_rows));
-      MD_TRY(lm_silu_mul(m->dtype, w.gu, l.gate_up.n_pad, w.act, l.down.k_pad, b->n_rows, l.ff_pad, s));
+      MD_TRY(lm_silu_mul_f32(w.gu, l.gate_up.n_pad, w.act, l.down.k_pad, b->n_rows, l.ff_pad, s));
     }
     return finish(w.act, l.down.k_pad, l.down, few, l.mix2, nw, next);
   }
@@ -520,8 +526,13 @@ struct Step {
     add.weight = w.route_weight;
     if (dec) {
       const int64_t stride = slots * ld;
-      MD_TRY(md_gemm_grouped_partial(w.h, m->width_pad, w.row_of, l.gate_up, l.experts, w.offsets, w.part, ld, stride, slots, s));
-      MD_TRY(lm_reduce_silu_mul(w.part, md_gemm_grouped_slices(l.gate_up, l.experts, slots), ld, stride, w.act, l.down.k_pad, slots, l.ff_pad, s));
+      const int sl = md_gemm_grouped_slices(l.gate_up, l.experts, slots);
+      if (sl == 1) {
+        MD_TRY(md_gemm_grouped_bf16(w.h, m->width_pad, w.row_of, l.gate_up, l.experts, w.offsets, w.act, l.down.k_pad, slots, true, false, s));
+      } else {
+        MD_TRY(md_gemm_grouped_partial(w.h, m->width_pad, w.row_of, l.gate_up, l.experts, w.offsets, w.part, ld, stride, slots, s));
+        MD_TRY(lm_reduce_silu_mul(w.part, sl, ld, stride, w.act, l.down.k_pad, slots, l.ff_pad, s));
+      }
       add.src = w.part;
       add.slices = md_gemm_grouped_slices(l.down, l.experts, slots);
       add.slice_stride = (int64_t)slots * l.down.n_pad;
@@ -530,12 +541,11 @@ struct Step {
     add.src = w.y;
     if (m->dtype == MD_DTYPE_F32) {
       MD_TRY(lm_grouped_gemm_f32(w.h, m->width_pad, w.row_of, l.gate_up, l.experts, w.offsets, w.gu, ld, slots, s));
-      MD_TRY(lm_silu_mul(m->dtype, w.gu, ld, w.act, l.down.k_pad, slots, l.ff_pad, s));
+      MD_TRY(lm_silu_mul_f32(w.gu, ld, w.act, l.down.k_pad, slots, l.ff_pad, s));
       return lm_grouped_gemm_f32(w.act, l.down.k_pad, nullptr, l.down, l.experts, w.offsets, w.y, m->width_pad, slots, s);
     }
-    MD_TRY(md_gemm_grouped_bf16(w.h, m->width_pad, w.row_of, l.gate_up, l.experts, w.offsets, w.gu, ld, slots, s));
-    MD_TRY(lm_silu_mul(m->dtype, w.gu, ld, w.act, l.down.k_pad, slots, l.ff_pad, s));
-    return md_gemm_grouped_bf16(w.act, l.down.k_pad, nullptr, l.down, l.experts, w.offsets, w.y, m->width_pad, slots, s);
+    MD_TRY(md_gemm_grouped_bf16(w.h, m->width_pad, w.row_of, l.gate_up, l.experts, w.offsets, w.act, l.down.k_pad, slots, true, true, s));
+    return md_gemm_grouped_bf16(w.act, l.down.k_pad, nullptr, l.down, l.experts, w.offsets, w.y, m->width_pad, slots, false, false, s);
   }
 
   // the residual stream behind everything so far -> out (fp32 [n_rows][width_pad]); streams: their sum
@@ -556,15 +566,14 @@ struct Step {
       const md_lm_layer& l = m->layers[i];
       // what follows this layer: the next one's mixer, or the head
       const md_lm_layer* after = i + 1 < m->n_layers ? &m->layers[i + 1] : nullptr;
-      const md_rms_weight* nw = after ? &after->norm1 : &m->final_norm;
+      const md_rms_weight& nw = after ? after->norm1 : m->final_norm;
       const float* next = after ? after->mix1 : nullptr;
       MD_TRY(input(l.norm1, l.mix1));
       MD_TRY(project(l.in_proj));
       if (l.out_proj.k_pad != l.heads * l.vdim_pad) MD_TRY(zero_fill(w.att, (size_t)b->n_rows * l.out_proj.k_pad * esize(m), s));
       MD_TRY(mixer(i));
       if (l.ff > 0) {
-        // (the router of an expert layer takes whole normed rows)
-        MD_TRY(finish(w.att, l.out_proj.k_pad, l.out_proj, false, l.mix1, l.experts > 0 ? nullptr : &l.norm2, l.mix2));
+        MD_TRY(finish(w.att, l.out_proj.k_pad, l.out_proj, false, l.mix1, l.norm2, l.mix2));
         MD_TRY(input(l.norm2, l.mix2));
         MD_TRY(feed_forward(l, nw, next));
       } else {

@@ -35,8 +35,6 @@ __device__ __forceinline__ void st8(float* p, f32x4 a, f32x4 b) {
 }
 
 __device__ __forceinline__ float silu_f32(float z) { return z / (1.0f + expf(-z)); }
-// fp32 with the hardware's exponential and reciprocal (an ulp or two each): for results that are stored as bf16
-__device__ __forceinline__ float silu_fast(float z) { return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z)); }
 template <typename T>
 __device__ __forceinline__ float silu_for(float z) {
   return std::is_same<T, float>::value ? silu_f32(z) : silu_fast(z);
@@ -267,7 +265,7 @@ md_status lm_reduce_resid_norm(float* x, int64_t ldx, const float* part, int sli
                                const md_rms_weight& w, float eps, int width, int width_pad, void* y, int64_t ldy, const int32_t* rows_idx,
                                bool write_x, int rows, hipStream_t s);
 // act = silu(gate) * up over [gate | up] rows
-md_status lm_silu_mul(int dtype, const void* gu, int64_t ldg, void* act, int64_t lda, int rows, int ff_pad, hipStream_t s);
+md_status lm_silu_mul_f32(const void* gu, int64_t ldg, void* act, int64_t lda, int rows, int ff_pad, hipStream_t s);
 md_status lm_reduce_silu_mul(const float* part, int slices, int64_t ldp, int64_t slice_stride, void* act, int64_t lda, int rows, int ff_pad,
                              hipStream_t s);
 

@@ -81,6 +81,9 @@ __device__ __forceinline__ void md_rope_pair(float re, float im, float cs, float
   o_im = c + d;
 }
 
+// fp32 with the hardware's exponential and reciprocal (an ulp or two each): for results that are stored as bf16
+__device__ __forceinline__ float silu_fast(float z) { return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z)); }
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

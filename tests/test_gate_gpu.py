@@ -1,0 +1,39 @@
+"""Gate products with SiLU in their epilogue, alone and grouped by expert, in every tile the row count picks: the four-wave tile, the smaller
+ones, remainders of rows, columns and groups, empty and single-row groups.  Against the layers' equations in float64."""
+import pytest
+import torch
+
+import lm_util as U
+from oracle import layered_lm_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def run(cfg, rows, gain=1.5):
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    w = U.weights(cfg, 3, gain)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=torch.bfloat16, max_batch=64, max_context=512)
+    n = -(-rows // 400)
+    ts = [U.tokens(min(400, rows - 400 * i), cfg["vocab"], i) for i in range(n)]
+    got = m.step([(m.open_sequence(), t, range(len(t))) for t in ts])
+    return got, torch.cat([O.forward(cfg, w, t) for t in ts])
+
+
+def mixer():
+    return U.latent(1, 32, 32, 64)
+
+
+@pytest.mark.parametrize("rows,ff", [(29, 100), (64, 330), (65, 330), (128, 70), (129, 330), (300, 2900), (700, 2900), (1100, 3000), (2300, 1300)])
+def test_dense(rows, ff):
+    got, want = run(U.stream_config([(mixer(), U.dense(ff))], width=320, vocab=120, streams=1, positions=400), rows)
+    assert U.logit_error(got, want) < 3e-2
+
+
+@pytest.mark.parametrize("rows,experts,top,ff", [(3, 5, 2, 40), (40, 6, 2, 300), (130, 7, 3, 300), (500, 9, 2, 200), (700, 4, 3, 200), (2100, 3, 2, 330), (1500, 40, 1, 70)])
+def test_experts(rows, experts, top, ff):
+    got, want = run(U.stream_config([(mixer(), U.moe(experts, top, ff))], width=320, vocab=120, streams=1, positions=400), rows)
+    e = U.logit_errors(got, want).sort().values
+    # a router between nearly equal logits may choose another expert at single rows
+    assert float(e[int(0.9 * (len(e) - 1))]) < 3e-2 and float(e.median()) < 1e-2
