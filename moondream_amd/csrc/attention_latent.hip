@@ -71,9 +71,10 @@ __global__ __launch_bounds__(256) void latent_plain_kernel(const LmLatent a) {
   __syncthreads();
   for (int r = tid; r < R; r += 256) {
     const T* w = (const T*)a.up_k_t + ((int64_t)h * R + r) * a.dp;
-    float s = 0.f;
-    for (int d = 0; d < a.dim; ++d) s += qs[d] * ldf(w + d);
-    ql[r] = s;
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+    for (int d = 0; d < a.dp; d += 4) s += *(const f32x4*)(qs + d) * ld4(w + d);  // (columns behind the head's are zeros)
+    ql[r] = (s[0] + s[1]) + (s[2] + s[3]);
     z[r] = 0.f;
   }
   float m = -INFINITY, l = 0.f;
@@ -82,12 +83,10 @@ __global__ __launch_bounds__(256) void latent_plain_kernel(const LmLatent a) {
     __syncthreads();
     float s = -INFINITY;
     if (tid < n) {
-      s = 0.f;
-      for (int r = 0; r < R; r += 4) {
-        const f32x4 v = ld4(c + (int64_t)(j0 + tid) * R + r), w = *(const f32x4*)(ql + r);
-        s += v[0] * w[0] + v[1] * w[1] + v[2] * w[2] + v[3] * w[3];
-      }
-      s *= a.scale;
+      f32x4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+      for (int r = 0; r < R; r += 4) d += ld4(c + (int64_t)(j0 + tid) * R + r) * *(const f32x4*)(ql + r);
+      s = ((d[0] + d[1]) + (d[2] + d[3])) * a.scale;
     }
     const float wm = wave_max(s);
     if (lane == 0) red[wave] = wm;
@@ -98,6 +97,7 @@ __global__ __launch_bounds__(256) void latent_plain_kernel(const LmLatent a) {
     m = mn;
     for (int r = tid; r < R; r += 256) {
       float o = z[r] * f;
+#pragma unroll 16
       for (int j = 0; j < n; ++j) o += ps[j] * ldf(c + (int64_t)(j0 + j) * R + r);
       z[r] = o;
     }
@@ -105,9 +105,10 @@ __global__ __launch_bounds__(256) void latent_plain_kernel(const LmLatent a) {
   __syncthreads();
   for (int e = tid; e < a.vp; e += 256) {
     const T* w = (const T*)a.up_kv.w + ((int64_t)a.heads * a.dp + h * a.vp + e) * R;
-    float o = 0.f;
-    for (int r = 0; r < R; ++r) o += z[r] * ldf(w + r);
-    o /= l;
+    f32x4 y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+    for (int r = 0; r < R; r += 4) y += *(const f32x4*)(z + r) * ld4(w + r);
+    float o = ((y[0] + y[1]) + (y[2] + y[3])) / l;
     if (a.col_g >= 0) o *= sigmoid_f32(ldf(proj + a.col_g + h * a.vp + e));
     stf((T*)a.out + (int64_t)row * a.ldo + h * a.vp + e, o);
   }

@@ -3,7 +3,7 @@
 //   route_row_kernel    one workgroup per row: logits on the vector ALUs (any dtype), choice and weights; a decode step, fp32 models
 //   route_tile_kernel   sixteen rows per workgroup: logits on the matrix cores (bf16 operands, fp32 sums), choice and weights
 //   group_kernel        one workgroup per expert: its slots in row order, deterministic, no atomics
-//   grouped_gemm_f32    C[slot] = A[row of slot] W_e^T in fp32 (the bf16 product is gemm_bf16.hip's, over the same slots)
+// The products over the slots are gemm_bf16.hip's and gemm_f32.hip's.
 //
 // Logits, softmax and weights are fp32.  A slot is one (row, chosen expert) pair; slots are numbered expert by expert.
 #include "gemm_internal.hpp"
@@ -194,55 +194,6 @@ __global__ __launch_bounds__(1024) void group_kernel(const LmRoute a) {
   });
 }
 
-// the tile gemm_f32_kernel of lm_ops.hip over the slots of one expert: grid (N / 64, tiles of 64 slots: see grouped_tile)
-__global__ __launch_bounds__(256) void grouped_gemm_f32_kernel(const float* __restrict__ A, int64_t lda, const int32_t* __restrict__ row_of,
-                                                               const float* __restrict__ W, int64_t ldw, int n_pad, const int32_t* __restrict__ offsets,
-                                                               int experts, float* __restrict__ C, int64_t ldc, int K) {
-  __shared__ __attribute__((aligned(16))) float As[64][20], Ws[64][20];
-  int e, m0, m1;
-  if (!grouped_tile(offsets, experts, 64, blockIdx.y, e, m0, m1)) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n0 = blockIdx.x * 64;
-  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32, lr = tid >> 2, lc = (tid & 3) * 4;
-  const int slot = min(m0 + lr, m1 - 1);
-  const float* ap = A + (int64_t)(row_of ? row_of[slot] : slot) * lda + lc;
-  const float* wp = W + ((int64_t)e * n_pad + n0 + lr) * ldw + lc;
-  f32x4 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int r = lane & 15, kq = lane >> 4;
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    const f32x4 av = *(const f32x4*)(ap + k0), wv = *(const f32x4*)(wp + k0);
-    __syncthreads();
-    *(f32x4*)&As[lr][lc] = av;
-    *(f32x4*)&Ws[lr][lc] = wv;
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 16; k += 4) {
-      float x[2], w[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        x[i] = As[wm + 16 * i + r][k + kq];
-        w[i] = Ws[wn + 16 * i + r][k + kq];
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], w[j], acc[i][j], 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int m = m0 + wm + 16 * i + 4 * kq + k;
-        if (m < m1) C[(int64_t)m * ldc + n0 + wn + 16 * j + r] = acc[i][j][k];
-      }
-}
-
 }  // namespace
 
 md_status lm_route(int dtype, const LmRoute& a, hipStream_t s) {
@@ -256,12 +207,5 @@ md_status lm_route(int dtype, const LmRoute& a, hipStream_t s) {
   }
   MD_TRY(md_launch_status());
   hipLaunchKernelGGL(group_kernel, dim3(a.experts), dim3(1024), 0, s, a);
-  return md_launch_status();
-}
-
-md_status lm_grouped_gemm_f32(const void* a, int64_t lda, const int32_t* row_of, const md_linear& lin, int experts, const int32_t* offsets, void* c,
-                              int64_t ldc, int slots, hipStream_t s) {
-  hipLaunchKernelGGL(grouped_gemm_f32_kernel, dim3(lin.n_pad / 64, grouped_tiles(slots, experts, 64)), dim3(256), 0, s, (const float*)a, lda, row_of,
-                     (const float*)lin.w, (int64_t)lin.k_pad, lin.n_pad, offsets, experts, (float*)c, ldc, lin.k_pad);
   return md_launch_status();
 }

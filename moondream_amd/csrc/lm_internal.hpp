@@ -40,6 +40,16 @@ __device__ __forceinline__ float silu_for(float z) {
   return std::is_same<T, float>::value ? silu_f32(z) : silu_fast(z);
 }
 
+// sum over the 16 lanes of a row; every lane gets it (vector instructions only)
+__device__ __forceinline__ float row_sum_16(float v) {
+  auto turned = [](float x, auto by) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x120 + decltype(by)::value, 0xf, 0xf, false)); };
+  v += turned(v, std::integral_constant<int, 8>{});
+  v += turned(v, std::integral_constant<int, 4>{});
+  v += turned(v, std::integral_constant<int, 2>{});
+  v += turned(v, std::integral_constant<int, 1>{});
+  return v;
+}
+
 // sum over a workgroup of N waves; every thread gets it.  red: N floats of LDS.
 template <int N>
 __device__ __forceinline__ float block_sum(float v, float* red) {

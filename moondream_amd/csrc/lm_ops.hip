@@ -1,4 +1,4 @@
-// Row-wise steps of the layered language models and their fp32 matrix product.
+// Row-wise steps of the layered language models.
 //
 // The residual stream is fp32 [rows][width_pad] whatever the model's dtype; columns width .. width_pad - 1 stay zero (the linears'
 // padded rows are zero), and the normed rows carry zeros there, so they feed a GEMM whose K is padded.
@@ -128,57 +128,6 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(const float* __restric
   st4(out + (int64_t)row * ldo + c, y);
 }
 
-// C[m][n] = sum_k A[m][k] W[n][k] + b[n] in fp32: 64 x 64 tile, four waves of 32 x 32 (2 x 2 v_mfma_f32_16x16x4_f32), K in steps
-// of 16 through LDS.  K % 64 == 0, N % 64 == 0; rows beyond M are read as the last row and not stored.
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ A, int64_t lda, const float* __restrict__ W, int64_t ldw,
-                                                       const float* __restrict__ bias, float* __restrict__ C, int64_t ldc, int M, int K) {
-  __shared__ __attribute__((aligned(16))) float As[64][20], Ws[64][20];  // row stride 20: 16-byte aligned, no bank conflicts
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
-  const int lr = tid >> 2, lc = (tid & 3) * 4;  // one f32x4 of each operand tile per thread
-  const float* ap = A + (int64_t)min(m0 + lr, M - 1) * lda + lc;
-  const float* wp = W + (int64_t)(n0 + lr) * ldw + lc;
-  f32x4 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int r = lane & 15, kq = lane >> 4;
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    const f32x4 av = *(const f32x4*)(ap + k0), wv = *(const f32x4*)(wp + k0);
-    __syncthreads();
-    *(f32x4*)&As[lr][lc] = av;
-    *(f32x4*)&Ws[lr][lc] = wv;
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 16; k += 4) {
-      float a[2], w[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        a[i] = As[wm + 16 * i + r][k + kq];
-        w[i] = Ws[wn + 16 * i + r][k + kq];
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], w[j], acc[i][j], 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int n = n0 + wn + 16 * j + r;
-      const float b = bias ? bias[n] : 0.f;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int m = m0 + wm + 16 * i + 4 * kq + e;
-        if (m < M) C[(int64_t)m * ldc + n] = acc[i][j][e] + b;
-      }
-    }
-}
-
 }  // namespace
 
 md_status lm_embed(int dtype, const void* table, int64_t ld, const int32_t* tokens, float* x, int rows, int vocab, hipStream_t s) {
@@ -222,13 +171,5 @@ md_status lm_reduce_rows(const float* part, int slices, int64_t ldp, int64_t sli
                          hipStream_t s) {
   hipLaunchKernelGGL(reduce_rows_kernel, dim3((rows * (n / 4) + 255) / 256), dim3(256), 0, s, part, slices, ldp, slice_stride, (const bf16_t*)bias,
                      (bf16_t*)out, ldo, rows, n);
-  return md_launch_status();
-}
-
-extern "C" md_status md_gemm_f32(const void* a, int64_t lda, const md_linear* lin, void* c, int64_t ldc, int32_t m, void* stream) {
-  MD_CHECK_ARG(a && lin && lin->w && c && m > 0 && lin->n_pad > 0 && lin->n_pad % 64 == 0 && lin->k_pad > 0 && lin->k_pad % 64 == 0);
-  MD_CHECK_ARG(lda >= lin->k_pad && lda % 4 == 0 && ldc >= lin->n_pad && ((uintptr_t)a & 15) == 0 && ((uintptr_t)lin->w & 15) == 0);
-  hipLaunchKernelGGL(gemm_f32_kernel, dim3(lin->n_pad / 64, (m + 63) / 64), dim3(256), 0, (hipStream_t)stream, (const float*)a, lda,
-                     (const float*)lin->w, (int64_t)lin->k_pad, (const float*)lin->b, (float*)c, ldc, m, lin->k_pad);
   return md_launch_status();
 }

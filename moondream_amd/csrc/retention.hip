@@ -39,52 +39,77 @@ __global__ __launch_bounds__(256) void ret_rotate_kernel(const LmRet a) {
   }
 }
 
-// grid (n_seq, heads, vp / 16): 16 columns of the state, 16 threads per column, each owning every 16th row of it
-constexpr int PLAIN_ROWS = 16;  // state rows per thread: dp <= 256
-template <typename T>
+// grid (n_seq, heads, vp / 16): 16 columns of the state, 16 neighbouring lanes per column, each owning rows 4 l .. + 3 of every 64.  Tokens are
+// staged 16 at a time and then run without a barrier: the recurrence is a chain, what counts is what lies on it (two sequences of 190 tokens,
+// 16 heads of 128: 57 us, 235 us with three barriers per token).
+// Q: quads of state rows per thread, dp <= 64 Q
+constexpr int PLAIN_TOKENS = 16;
+template <typename T, int Q>
 __global__ __launch_bounds__(256) void ret_scan_kernel(const LmRet a) {
-  __shared__ float qs[256], ks[256], red[16][17];
-  const int seq = blockIdx.x, h = blockIdx.y, e = blockIdx.z * 16 + (threadIdx.x & 15), dg = threadIdx.x >> 4;
+  __shared__ __attribute__((aligned(16))) float qs[PLAIN_TOKENS][64 * Q], ks[PLAIN_TOKENS][64 * Q];
+  __shared__ float vs[PLAIN_TOKENS][16], os[PLAIN_TOKENS][16];
+  const int seq = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, l = tid & 15, col = tid >> 4, e0 = blockIdx.z * 16, e = e0 + col;
   const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, pos0 = a.r.seq_pos0[seq];
   const int dp = a.dp, vp = a.vp, H = a.heads;
   float* st = a.state + (((int64_t)a.r.seq_slot[seq] * H + h) * vp + e) * dp;
   const float decay = a.decay[h];
-  float S[PLAIN_ROWS];
+  f32x4 S[Q];
 #pragma unroll
-  for (int i = 0; i < PLAIN_ROWS; ++i) {
-    const int d = dg + 16 * i;
-    S[i] = (pos0 > 0 && d < dp) ? st[d] : 0.f;
+  for (int i = 0; i < Q; ++i) {
+    const int d = 64 * i + 4 * l;
+    S[i] = (pos0 > 0 && d < dp) ? *(const f32x4*)(st + d) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  for (int t = 0; t < len; ++t) {
-    const int64_t row = row0 + t;
-    __syncthreads();
-    for (int d = threadIdx.x; d < dp; d += 256) {
-      qs[d] = a.qf[row * H * dp + h * dp + d];
-      ks[d] = a.kf[row * H * dp + h * dp + d];
-    }
-    __syncthreads();
-    const float v = ldf((const T*)a.proj + row * a.ldp + a.col_v + h * vp + e);
-    float o = 0.f;
+  f32x4 qn[Q], kn[Q];  // the next tokens', under way during these
+  float vn = 0.f;
+  const int quads = dp / 4;
+  auto load = [&](int t0) {
+    const int n = min(PLAIN_TOKENS, len - t0);
 #pragma unroll
-    for (int i = 0; i < PLAIN_ROWS; ++i) {
-      const int d = dg + 16 * i;
-      if (d < dp) {
-        S[i] = decay * S[i] + ks[d] * v;
-        o += S[i] * qs[d];
+    for (int j = 0; j < Q; ++j) {
+      const int i = tid + 256 * j, t = i / quads;
+      if (t >= n) continue;
+      const int64_t at = ((int64_t)(row0 + t0 + t) * H + h) * dp + (i - t * quads) * 4;
+      qn[j] = *(const f32x4*)(a.qf + at);
+      kn[j] = *(const f32x4*)(a.kf + at);
+    }
+    if (col < n) vn = ldf((const T*)a.proj + (int64_t)(row0 + t0 + col) * a.ldp + a.col_v + h * vp + e0 + l);
+  };
+  load(0);
+  for (int t0 = 0; t0 < len; t0 += PLAIN_TOKENS) {
+    const int n = min(PLAIN_TOKENS, len - t0);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < Q; ++j) {
+      const int i = tid + 256 * j, t = i / quads, d = (i - t * quads) * 4;
+      if (t >= n) continue;
+      *(f32x4*)(qs[t] + d) = qn[j];
+      *(f32x4*)(ks[t] + d) = kn[j];
+    }
+    if (col < n) vs[col][l] = vn;
+    __syncthreads();
+    if (t0 + PLAIN_TOKENS < len) load(t0 + PLAIN_TOKENS);
+#pragma unroll 4
+    for (int t = 0; t < n; ++t) {
+      const float v = vs[t][col];
+      f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < Q; ++i) {
+        const int d = 64 * i + 4 * l;
+        if (i + 1 < Q || d < dp) {
+          S[i] = decay * S[i] + *(const f32x4*)(ks[t] + d) * v;
+          o += S[i] * *(const f32x4*)(qs[t] + d);
+        }
       }
+      const float sum = row_sum_16((o[0] + o[1]) + (o[2] + o[3]));
+      if (l == 0) os[t][col] = sum;
     }
-    red[dg][threadIdx.x & 15] = o;
     __syncthreads();
-    if (dg == 0) {
-      float sum = 0.f;
-      for (int i = 0; i < 16; ++i) sum += red[i][threadIdx.x];
-      a.of[row * H * vp + h * vp + e] = sum;
-    }
+    if (col < n) a.of[((int64_t)(row0 + t0 + col) * H + h) * vp + e0 + l] = os[col][l];
   }
 #pragma unroll
-  for (int i = 0; i < PLAIN_ROWS; ++i) {
-    const int d = dg + 16 * i;
-    if (d < dp) st[d] = S[i];
+  for (int i = 0; i < Q; ++i) {
+    const int d = 64 * i + 4 * l;
+    if (d < dp) *(f32x4*)(st + d) = S[i];
   }
 }
 
@@ -104,10 +129,11 @@ __global__ __launch_bounds__(256) void ret_out_kernel(const LmRet a) {
 
 template <typename T>
 md_status plain(const LmRet& a, hipStream_t s) {
-  if (a.dp > 16 * PLAIN_ROWS) return MD_ERR_UNSUPPORTED;
+  if (a.dp > 256) return MD_ERR_UNSUPPORTED;
   hipLaunchKernelGGL(ret_rotate_kernel<T>, dim3(a.r.n_rows), dim3(256), 0, s, a);
   MD_TRY(md_launch_status());
-  hipLaunchKernelGGL(ret_scan_kernel<T>, dim3(a.r.n_seq, a.heads, a.vp / 16), dim3(256), 0, s, a);
+  auto scan = a.dp <= 64 ? ret_scan_kernel<T, 1> : a.dp <= 128 ? ret_scan_kernel<T, 2> : a.dp <= 192 ? ret_scan_kernel<T, 3> : ret_scan_kernel<T, 4>;
+  hipLaunchKernelGGL(scan, dim3(a.r.n_seq, a.heads, a.vp / 16), dim3(256), 0, s, a);
   MD_TRY(md_launch_status());
   hipLaunchKernelGGL(ret_out_kernel<T>, dim3(a.r.n_rows), dim3(256), 0, s, a);
   return md_launch_status();

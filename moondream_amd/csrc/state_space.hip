@@ -149,53 +149,90 @@ md_status conv(const LmSsm& a, hipStream_t s) {
   return md_launch_status();
 }
 
-// grid (n_seq, heads, vp / 16): 16 columns of the state, 16 threads per column, each owning every 16th row of it
-constexpr int SCAN_ROWS = 32;  // state rows per thread: dp <= 512
-template <typename T>
+// grid (n_seq, heads, vp / 16): 16 columns of the state, 16 neighbouring lanes per column, each owning rows 4 l .. + 3 of every 64.  Tokens are
+// staged 8 at a time and then run without a barrier: the recurrence is a chain, what counts is what lies on it (one sequence of 300 tokens, 32
+// heads of 64 x 64, fp32: 67 us, 342 us token by token).
+// Q: quads of state rows per thread, dp <= 64 Q (and for Q = 2 more than 64)
+template <typename T, int Q>
 __global__ __launch_bounds__(256) void ssm_scan_kernel(const LmSsm a) {
-  __shared__ float bs[16 * SCAN_ROWS], cs[16 * SCAN_ROWS], red[16][17];
-  const int seq = blockIdx.x, h = blockIdx.y, e = blockIdx.z * 16 + (threadIdx.x & 15), dg = threadIdx.x >> 4;
+  constexpr int SCAN_TOKENS = Q <= 4 ? 16 : 8;
+  __shared__ __attribute__((aligned(16))) float bs[SCAN_TOKENS][64 * Q], cs[SCAN_TOKENS][64 * Q];
+  __shared__ float xs[SCAN_TOKENS][16], zs[SCAN_TOKENS][16], os[SCAN_TOKENS][16], dts[SCAN_TOKENS], keeps[SCAN_TOKENS];
+  const int seq = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, l = tid & 15, col = tid >> 4, e0 = blockIdx.z * 16, e = e0 + col;
   const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, pos0 = a.r.seq_pos0[seq];
   const int dp = a.dp, vp = a.vp, H = a.heads, cw = a.cw(), g = h / (H / a.groups);
   float* st = a.state + (((int64_t)a.r.seq_slot[seq] * H + h) * vp + e) * dp;
   const float decay = a.decay[h], skip = a.skip[h];
-  float S[SCAN_ROWS];
+  f32x4 S[Q];
 #pragma unroll
-  for (int i = 0; i < SCAN_ROWS; ++i) {
-    const int d = dg + 16 * i;
-    S[i] = (pos0 > 0 && d < dp) ? st[d] : 0.f;
+  for (int i = 0; i < Q; ++i) {
+    const int d = 64 * i + 4 * l;
+    S[i] = (pos0 > 0 && d < dp) ? *(const f32x4*)(st + d) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  for (int t = 0; t < len; ++t) {
-    const int64_t row = row0 + t;
-    const T* u = (const T*)a.u + row * cw;
+  constexpr int QT = SCAN_TOKENS * 16 * Q / 256;  // quads of B (and C) per thread
+  f32x4 bn[QT], cn[QT];  // the next tokens', under way during these
+  float xn = 0.f, zn = 0.f, dtn = 0.f;
+  const int quads = dp / 4;
+  auto load = [&](int t0) {
+    const int n = min(SCAN_TOKENS, len - t0);
+#pragma unroll
+    for (int j = 0; j < QT; ++j) {
+      const int i = tid + 256 * j, t = i / quads;
+      if (t >= n) continue;
+      const T* u = (const T*)a.u + (int64_t)(row0 + t0 + t) * cw + H * vp + (i - t * quads) * 4;
+      bn[j] = ld4(u + g * dp);
+      cn[j] = ld4(u + (a.groups + g) * dp);
+    }
+    if (col < n) {
+      const int64_t row = row0 + t0 + col;
+      xn = ldf((const T*)a.u + row * cw + h * vp + e0 + l);
+      zn = ldf((const T*)a.proj + row * a.ldp + a.col_z + h * vp + e0 + l);
+    }
+    if (tid < n) dtn = a.dt[(int64_t)(row0 + t0 + tid) * H + h];
+  };
+  load(0);
+  for (int t0 = 0; t0 < len; t0 += SCAN_TOKENS) {
+    const int n = min(SCAN_TOKENS, len - t0);
     __syncthreads();
-    for (int d = threadIdx.x; d < dp; d += 256) {
-      bs[d] = ldf(u + H * vp + g * dp + d);
-      cs[d] = ldf(u + H * vp + (a.groups + g) * dp + d);
+#pragma unroll
+    for (int j = 0; j < QT; ++j) {
+      const int i = tid + 256 * j, t = i / quads, d = (i - t * quads) * 4;
+      if (t >= n) continue;
+      *(f32x4*)(bs[t] + d) = bn[j];
+      *(f32x4*)(cs[t] + d) = cn[j];
+    }
+    if (col < n) {
+      xs[col][l] = xn;
+      zs[col][l] = zn;
+    }
+    if (tid < n) {
+      dts[tid] = dtn;
+      keeps[tid] = expf(-decay * dtn);
     }
     __syncthreads();
-    const float dt = a.dt[row * H + h], keep = expf(-decay * dt), x = ldf(u + h * vp + e), in = dt * x;
-    float o = 0.f;
+    if (t0 + SCAN_TOKENS < len) load(t0 + SCAN_TOKENS);
+#pragma unroll 4
+    for (int t = 0; t < n; ++t) {
+      const float keep = keeps[t], x = xs[t][col], in = dts[t] * x;
+      f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < SCAN_ROWS; ++i) {
-      const int d = dg + 16 * i;
-      if (d < dp) {
-        S[i] = keep * S[i] + bs[d] * in;
-        o += S[i] * cs[d];
+      for (int i = 0; i < Q; ++i) {
+        const int d = 64 * i + 4 * l;
+        if ((Q <= 2 && i + 1 < Q) || d < dp) {
+          S[i] = keep * S[i] + *(const f32x4*)(bs[t] + d) * in;
+          o += S[i] * *(const f32x4*)(cs[t] + d);
+        }
       }
+      const float sum = row_sum_16((o[0] + o[1]) + (o[2] + o[3]));
+      if (l == 0) os[t][col] = sum + skip * x;
     }
-    red[dg][threadIdx.x & 15] = o;
     __syncthreads();
-    if (dg == 0) {
-      float sum = skip * x;
-      for (int i = 0; i < 16; ++i) sum += red[i][threadIdx.x];
-      stf((T*)a.out + row * a.ldo + h * vp + e, sum * silu_f32(ldf((const T*)a.proj + row * a.ldp + a.col_z + h * vp + e)));
-    }
+    if (col < n) stf((T*)a.out + (int64_t)(row0 + t0 + col) * a.ldo + h * vp + e0 + l, os[col][l] * silu_f32(zs[col][l]));
   }
 #pragma unroll
-  for (int i = 0; i < SCAN_ROWS; ++i) {
-    const int d = dg + 16 * i;
-    if (d < dp) st[d] = S[i];
+  for (int i = 0; i < Q; ++i) {
+    const int d = 64 * i + 4 * l;
+    if (d < dp) *(f32x4*)(st + d) = S[i];
   }
 }
 
@@ -244,9 +281,10 @@ md_status norm(const LmSsm& a, hipStream_t s) {
 
 template <typename T>
 md_status plain(const LmSsm& a, hipStream_t s) {
-  if (a.dp > 16 * SCAN_ROWS) return MD_ERR_UNSUPPORTED;
+  if (a.dp > 512) return MD_ERR_UNSUPPORTED;
   MD_TRY(conv<T>(a, s));
-  hipLaunchKernelGGL(ssm_scan_kernel<T>, dim3(a.r.n_seq, a.heads, a.vp / 16), dim3(256), 0, s, a);
+  auto scan = a.dp <= 64 ? ssm_scan_kernel<T, 1> : a.dp <= 128 ? ssm_scan_kernel<T, 2> : a.dp <= 256 ? ssm_scan_kernel<T, 4> : ssm_scan_kernel<T, 8>;
+  hipLaunchKernelGGL(scan, dim3(a.r.n_seq, a.heads, a.vp / 16), dim3(256), 0, s, a);
   MD_TRY(md_launch_status());
   return norm<T>(a, s);
 }
