@@ -483,6 +483,18 @@ md_status md_vision_project(const md_vit_model* m, const void* feats, int32_t n_
                             int32_t tiles_h, int32_t tiles_w, int32_t margin, void* out,
                             int64_t ld_out, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Crops of n images cut on the device (reference: image_crops.py:58-167): per image the whole picture at crop x crop, then
+ * tiles_y x tiles_x windows, `stride` apart, of the picture resized to tiles * stride + crop - stride; the bytes are those of
+ * PIL's LANCZOS resize.  images: host [n][4] = height, width, tiles_y, tiles_x; crop and stride even.
+ *   md_crops_staged_bytes     size of the staged buffer; offsets[n] (may be NULL): where in it image i's RGB pixels go (0: out of range)
+ *   md_crops_plan             writes the plan to the front of the staged buffer (host memory, 16-byte aligned)
+ *   md_cut_crops              staged: the buffer on the device; out: uint8 [sum of 1 + tiles_y * tiles_x][crop][crop][3] */
+size_t md_crops_staged_bytes(const int32_t* images, int32_t n, int32_t crop, int32_t stride, int64_t* offsets);
+size_t md_crops_workspace_bytes(const int32_t* images, int32_t n, int32_t crop, int32_t stride);
+md_status md_crops_plan(const int32_t* images, int32_t n, int32_t crop, int32_t stride, void* staged, size_t staged_bytes);
+md_status md_cut_crops(const int32_t* images, int32_t n, int32_t crop, int32_t stride, const void* staged, void* workspace,
+                       size_t workspace_bytes, void* out, void* stream);
+
 /* The seam form of the same stage: _vis_proj(g, r) with r the ALREADY stitched
  * [H][W][dim] grid, exactly what the reference passes (moondream.py:171-172,
  * vision.py:77-89).  global_feats: [g*g][dim]; out: [g*g][ld_out].  Workspace:

@@ -17,7 +17,7 @@ REPO = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB_PATH = os.path.join(HERE, "libmoondream_hip.so")
 SOURCES = ["gemm_bf16.hip", "gemm_w4.hip", "gemm_fp8w.hip", "gemm_f8.hip", "quant_f8.hip", "attention_f8kv.hip", "decode_b1.hip", "attention.hip",
-           "elementwise.hip", "sampling_region.hip", "api.hip", "abi.hip", "lm_ops.hip", "gemm_step.hip", "gemm_f32.hip", "attention_talk.hip", "retention.hip",
+           "elementwise.hip", "image_crops.hip", "sampling_region.hip", "api.hip", "abi.hip", "lm_ops.hip", "gemm_step.hip", "gemm_f32.hip", "attention_talk.hip", "retention.hip",
            "attention_latent.hip", "state_space.hip", "experts.hip", "streams.hip", "lm_api.hip"]
 # the part of the library that the layered language models use: a checkout that serves only such a model compiles no more
 LM_LIB_PATH = os.path.join(HERE, "libmoondream_lm.so")
@@ -250,6 +250,10 @@ SIGNATURES = {
                                     c_void_p, c_size_t, c_void_p]),
     "md_vision_project_grid": (C.c_int, [P(MdVitModel), c_void_p, c_void_p, c_int32, c_int32, c_void_p, c_int64,
                                          c_void_p, c_size_t, c_void_p]),
+    "md_crops_staged_bytes": (c_size_t, [c_void_p, c_int32, c_int32, c_int32, c_void_p]),
+    "md_crops_workspace_bytes": (c_size_t, [c_void_p, c_int32, c_int32, c_int32]),
+    "md_crops_plan": (C.c_int, [c_void_p, c_int32, c_int32, c_int32, c_void_p, c_size_t]),
+    "md_cut_crops": (C.c_int, [c_void_p, c_int32, c_int32, c_int32, c_void_p, c_void_p, c_size_t, c_void_p, c_void_p]),
     "md_text_workspace_bytes": (c_size_t, [P(MdTextModel), c_int32, c_int32]),
     "md_text_forward": (C.c_int, [P(MdTextModel), c_void_p, c_void_p, c_int32, c_int32, c_void_p, P(MdKvCache),
                                   c_void_p, c_size_t, c_void_p]),

@@ -21,6 +21,7 @@ import ctypes as C
 import os
 import math
 from dataclasses import dataclass
+from types import SimpleNamespace
 from typing import Any, Dict, Iterable, List, Literal, Optional, Sequence, Tuple, Union
 
 import numpy as np
@@ -30,7 +31,7 @@ from PIL import Image
 from . import _lib
 from .config import MoondreamConfig
 from .engine import DEFAULT_MAX_TOKENS, DEFAULT_TEMPERATURE, DEFAULT_TOP_P, DeviceEngine
-from .image_crops import crop_count, overlap_crop_image, reconstruct_from_crops
+from .image_crops import crop_count, overlap_crop_image, reconstruct_from_crops, resize_backend
 from .integration import MASK_CAUSAL, MASK_PREFIX_LM, classify_attn_mask
 from .lora import variant_state_dict
 from .weights import PackedLora, PackedModel
@@ -520,12 +521,12 @@ class MoondreamModel(DeviceEngine):
     def _run_vision_encoder_batch(self, images: Sequence[Image.Image], mark=None, staged=None) -> torch.Tensor:
         """images -> [B,729,D] projected embeddings (reference: moondream.py:206-228, per image).
 
-        Host tiling (PIL, reference image_crops.py:58-167) runs on a thread pool and is
-        pipelined against the GPU: the ViT of image chunk k is enqueued (async) while
-        the crops of chunk k+1 are still being cut.  The workers cut their crops STRAIGHT
-        INTO the pinned staging buffer the H2D copy reads (the tiling, hence every image's
-        crop count and offset, follows from its size alone): no concatenation pass over the
-        crop bytes on the host."""
+        The host's part runs on a thread pool and is pipelined against the GPU: the ViT of
+        image chunk k is enqueued (async) while chunk k+1 is still being staged.  The workers
+        write their pixels, or the crops they cut (reference image_crops.py:58-167; which of the
+        two: ``_cut_plan``), STRAIGHT INTO the pinned staging buffer the H2D copy reads (the
+        tiling, hence every image's crop count and offset, follows from its size alone): no
+        concatenation pass over the bytes on the host."""
         v = self.config.vision
         n_img = len(images)
         if staged is None:
@@ -538,17 +539,33 @@ class MoondreamModel(DeviceEngine):
                 self._drain_staged(staged)  # this call owns the staging it made / took over: nothing stays marked busy
                 raise
         chunks, staged = staged
-        cropped: List[Tuple[np.ndarray, Tuple[int, int]]] = []
+        cropped: List[Tuple[int, Tuple[int, int]]] = []  # (crops, tiling) per image
         feat_parts = []
         # OWNERSHIP of the pinned staging buffers: ``staged`` is consumed IN PLACE -- a chunk leaves the list at the moment its
         # buffer is handed back (uploaded or released), so whoever holds the list (the pipelined engine's drain, on an early
         # exit or an exception in here) releases exactly the chunks that are still in it and no token twice
         for ci in range(len(staged)):
-            host, token, futs = staged[0]
+            host, token, futs, plan = staged[0]
             part = [f.result() for f in futs]
             if mark is not None and ci == 0:
                 mark("host_tiling")  # phase timing: the GPU has nothing of this batch to run before the first crops exist
-            cropped.extend(part)
+            cropped.extend((1 + t[0] * t[1], t) for _, t in part)
+            if plan is not None:
+                pixels = self._upload_pinned(host, token)
+                staged.pop(0)
+                dev_crops = self._cut_crops(pixels, plan, part)
+                if self.dedup_identical_crops and any(t == (1, 1) for _, t in part):  # (a single window is the global crop, see below)
+                    uniq, expand, off = [], [], 0
+                    for n, tiling in cropped[-len(part) :]:
+                        own = 1 if tiling == (1, 1) else n
+                        expand += [len(uniq)] * 2 if own < n else range(len(uniq), len(uniq) + n)
+                        uniq += range(off, off + own)
+                        off += n
+                    uniq, expand = (torch.tensor(list(i), dtype=torch.int64, device=self._device) for i in (uniq, expand))
+                    feat_parts.append(self._vit_run(dev_crops[uniq], _lib.MD_CROPS_U8_HWC)[expand])
+                    continue
+                feat_parts.append(self._vit_run(dev_crops, _lib.MD_CROPS_U8_HWC))
+                continue
             if self.dedup_identical_crops:
                 # An image that is no larger than one crop has tiling (1, 1) and its single local crop holds the same
                 # pixels as the global crop (image_crops.py:124-167: both are the image resized to crop_size).  The
@@ -588,9 +605,9 @@ class MoondreamModel(DeviceEngine):
         out = torch.empty(n_img, v.n_patches, v.proj_out_dim, dtype=BF16, device=self._device)
         # images with the same tiling are projected together
         offsets, off = [], 0
-        for c, _ in cropped:
+        for n, _ in cropped:
             offsets.append(off)
-            off += c.shape[0]
+            off += n
         groups: Dict[Tuple[int, int], List[int]] = {}
         for i, (_, tiling) in enumerate(cropped):
             groups.setdefault(tiling, []).append(i)
@@ -616,8 +633,8 @@ class MoondreamModel(DeviceEngine):
         return out
 
     def _stage_crops(self, images: Sequence[Image.Image], pool=None):
-        """Queue the host tiling of a batch on the thread pool, chunk by chunk, each image cutting its crops into its
-        slice of a pinned staging buffer.  Returns (chunks, staged) for ``_run_vision_encoder_batch``."""
+        """Queue the host's part of a batch's tiling on the thread pool, chunk by chunk, each image writing its pixels or its
+        crops into its slice of a pinned staging buffer.  Returns (chunks, staged) for ``_run_vision_encoder_batch``."""
         v = self.config.vision
         n_img = len(images)
         pool = pool or self._crop_pool()
@@ -633,16 +650,66 @@ class MoondreamModel(DeviceEngine):
                 i1 += 1
             chunks.append((i0, i1, tot))
             i0 = i1
-        staged = []
+        staged, room = [], 1 << 30
         for (c0, c1, tot) in chunks:  # all host work is queued up front; the GPU side follows chunk by chunk
+            plan = self._cut_plan(images[c0:c1], [t for _, t in counts[c0:c1]], min(room, 8 * tot * v.crop_size * v.crop_size * 3))
+            if plan is not None:
+                room -= plan.staged_bytes
+                host, token = self._pinned_crops(1, (plan.staged_bytes,))
+                _lib.check(self.lib.md_crops_plan(plan.images, plan.n, v.crop_size, plan.stride, host.ctypes.data, plan.staged_bytes), "md_crops_plan")
+                futs = []
+                for i, at in zip(range(c0, c1), plan.offsets):
+                    w, h = images[i].size
+                    futs.append(pool.submit(self._pixels_into, images[i], host[0, at : at + h * w * 3].reshape(h, w, 3), counts[i]))
+                staged.append((host, token, futs, plan))
+                continue
             host, token = self._pinned_crops(tot, (v.crop_size, v.crop_size, 3))
             futs, off = [], 0
             for i in range(c0, c1):
                 n = counts[i][0]
                 futs.append(pool.submit(self._crop_into, images[i], host[off : off + n]))
                 off += n
-            staged.append((host, token, futs))
+            staged.append((host, token, futs, None))
         return chunks, staged
+
+    def _cut_plan(self, images: Sequence[Image.Image], tilings, most: int):
+        """How the device cuts these images' crops (``md_cut_crops``), or None: the host cuts them.  On the device wherever the
+        host would resize with PIL: 768 x 1024 takes a worker 21 ms per image, its pixels 0.8 ms; pictures of one crop's size
+        are only copied on the host, which is 0.3 ms sooner for a single one.  Not for pictures more than 64 times as high as wide (PIL shrinks some of those in another
+        order) and not where the sources are more than ``most`` bytes: pinned memory is for crops, eight times theirs (12
+        megapixels in 13 crops) is where it ends."""
+        v = self.config.vision
+        sizes = [im.size for im in images]
+        if resize_backend() != "pil" or all(s == (v.crop_size, v.crop_size) for s in sizes) or any(h > 64 * w for w, h in sizes):
+            return None
+        plan = SimpleNamespace(n=len(sizes), stride=v.crop_size - 2 * v.overlap_margin * v.enc_patch_size)
+        plan.images = (C.c_int32 * (4 * plan.n))(*[x for (w, h), t in zip(sizes, tilings) for x in (h, w, *t)])
+        offsets = (C.c_int64 * plan.n)()
+        plan.staged_bytes = int(self.lib.md_crops_staged_bytes(plan.images, plan.n, v.crop_size, plan.stride, offsets))
+        if not 0 < plan.staged_bytes <= most:
+            return None
+        plan.offsets = list(offsets)
+        return plan
+
+    def _pixels_into(self, image: Image.Image, out: np.ndarray, count):
+        arr = np.asarray(image if image.mode == "RGB" else image.convert("RGB"))
+        if arr.shape != out.shape:  # a file that names another size than it decodes to
+            v = self.config.vision
+            return self._crop_into(image, np.empty((count[0], v.crop_size, v.crop_size, 3), dtype=np.uint8))
+        np.copyto(out, arr)
+        return None, tuple(count[1])
+
+    def _cut_crops(self, pixels: torch.Tensor, plan, part) -> torch.Tensor:
+        size = self.config.vision.crop_size
+        counts = [1 + t[0] * t[1] for _, t in part]
+        out = torch.empty(sum(counts), size, size, 3, dtype=torch.uint8, device=self._device)
+        ws = torch.empty(int(self.lib.md_crops_workspace_bytes(plan.images, plan.n, size, plan.stride)), dtype=torch.uint8, device=self._device)
+        _lib.check(self.lib.md_cut_crops(plan.images, plan.n, size, plan.stride, pixels.data_ptr(), ws.data_ptr(), ws.numel(), out.data_ptr(),
+                                         self._stream()), "md_cut_crops")
+        for i, (crops, _) in enumerate(part):
+            if crops is not None:
+                out[sum(counts[:i]) : sum(counts[: i + 1])] = torch.from_numpy(crops).to(self._device)
+        return out
 
     def prefetch_crops(self, images: Sequence[Image.Image]) -> None:
         """Start the host tiling of a batch NOW (thread pool, pinned staging buffers) so that a later call that encodes
@@ -669,7 +736,7 @@ class MoondreamModel(DeviceEngine):
     def wait_prefetched_crops(self) -> None:
         """Block until every prefetched batch's crops are cut (tests, benchmarks: a steady-state serving loop never waits)."""
         for _, (_, staged) in getattr(self, "_prefetched_crops", {}).values():
-            for _, _, futs in staged:
+            for _, _, futs, _ in staged:
                 for f in futs:
                     f.result()
 
@@ -685,7 +752,7 @@ class MoondreamModel(DeviceEngine):
         from the list when it hands its buffer back, so what is left here is exactly what is still owned)."""
         lst = staged[1]
         while lst:
-            host, token, futs = lst.pop(0)
+            _, token, futs, _ = lst.pop(0)
             for f in futs:
                 try:
                     f.result()  # the worker must be done with the buffer before it is handed out again
