@@ -150,7 +150,9 @@ __device__ __forceinline__ float block_max(float v, float* red) {
 // lane l takes the 8 features [512 c + 8 l, +8) of every chunk c; DEPTH chunks (R x 16 B per lane each) stay in flight.
 // Branch-free around its loads (clamped addresses, zeroed operands) so that the compiler counts the in-order returns.
 // prime() issues the first DEPTH chunks (the weights do not depend on the activations: it is called before the phase's
-// prologue); run() returns the R dot products in every lane.
+// prologue); run() returns the R dot products in every lane.  With `more` the ring goes on with the first DEPTH chunks of `next`, the rows
+// of the wave's next run() (2B, a caption's 31 steps: 764 us per token; 818 us where a wave waits for the first chunk of every pair); without,
+// its last loads repeat the last chunk (no branch).
 template <int R, int DEPTH>
 struct Gemv {
   u32x4 w[DEPTH][R];
@@ -172,13 +174,18 @@ struct Gemv {
 #pragma unroll
     for (int u = 0; u < DEPTH; ++u) issue(rows, K, u, w[u]);
   }
-  __device__ __forceinline__ void run(const bf16_t* const (&rows)[R], int K, const char* act_lds, float (&d)[R]) {
+  __device__ __forceinline__ void run(const bf16_t* const (&rows)[R], int K, const char* act_lds, float (&d)[R]) { run(rows, K, act_lds, d, rows, false); }
+  __device__ __forceinline__ void run(const bf16_t* const (&rows)[R], int K, const char* act_lds, float (&d)[R], const bf16_t* const (&next)[R], bool more) {
     const int lane = threadIdx.x & 63, nchunk = (K + 511) / 512;
     const u32x4 zero4 = {0u, 0u, 0u, 0u};
     float a[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) a[r] = 0.f;
     for (int c0 = 0; c0 < nchunk; c0 += DEPTH) {
+      const bool on = more && c0 + DEPTH >= nchunk;
+      const bf16_t* src[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) src[r] = on ? next[r] : rows[r];
 #pragma unroll
       for (int u = 0; u < DEPTH; ++u) {
         const int c = c0 + u;
@@ -194,7 +201,7 @@ struct Gemv {
             a[r] = fmaf(hi_bf(av[e]), hi_bf(x[e]), a[r]);
           }
         }
-        issue(rows, K, c + DEPTH, w[u]);
+        issue(src, K, on ? u : c + DEPTH, w[u]);
       }
     }
 #pragma unroll
@@ -251,33 +258,37 @@ __global__ __launch_bounds__(64 * NWV) void decode_b1_kernel(const B1Args p) {
   const int np_d = p.vocab >> 1;
   const int npw_d = (p.lm_w && blockIdx.x < np_d) ? (np_d - 1 - blockIdx.x) / gridDim.x + 1 : 0;
 
-  const bf16_t* rows_a[2];
-  auto set_rows = [&](const bf16_t* wmat, int ld, int q) {
+  auto set_rows = [&](const bf16_t* (&rows)[2], const bf16_t* wmat, int ld, int q) {
     const int pp = blockIdx.x + gridDim.x * q;
-    rows_a[0] = wmat + (int64_t)(2 * pp) * ld;
-    rows_a[1] = rows_a[0] + ld;
+    rows[0] = wmat + (int64_t)(2 * pp) * ld;
+    rows[1] = rows[0] + ld;
   };
   Gemv<2, 4> ga;  // phases A and D; primed across the barrier that precedes the phase (the weights depend on nothing)
   auto prime_first = [&](int npw, const bf16_t* wmat, int ld) {
     if (wave < npw) {
-      set_rows(wmat, ld, wave);
-      ga.prime(rows_a, D);
+      const bf16_t* rows[2];
+      set_rows(rows, wmat, ld, wave);
+      ga.prime(rows, D);
     } else {
       ga.zero();
     }
   };
   // a workgroup's npw row pairs, round-robin over its waves (pair q = wave + NWV i: consecutive pairs land on the four
-  // SIMDs in turn); finish(pp, d0, d1) is called by every lane of the wave that holds the two dot products of row pair pp.
+  // SIMDs in turn); finish(pp, d0, d1, bias pair) is called by every lane of the wave that holds the two dot products of row pair pp.
   // (Sharing the last npw % NWV pairs between waves by K ranges evens the waves out on paper and measured slower.)
-  auto run_rows = [&](int npw, const bf16_t* wmat, int ld, auto finish) {
+  auto run_rows = [&](int npw, const bf16_t* wmat, int ld, const bf16_t* bias, auto finish) {
+    const bf16_t *rows[2], *next[2];
+    set_rows(next, wmat, ld, wave);
     for (int q = wave; q < npw; q += NWV) {
-      if (q != wave) {
-        set_rows(wmat, ld, q);
-        ga.prime(rows_a, D);
-      }
+      const bool more = q + NWV < npw;
+      rows[0] = next[0];
+      rows[1] = next[1];
+      set_rows(next, wmat, ld, more ? q + NWV : q);
+      const int pp = blockIdx.x + gridDim.x * q;
+      const uint32_t bw = *(const uint32_t*)(bias + 2 * pp);  // (before the next rows' loads: loads return in order)
       float d[2];
-      ga.run(rows_a, D, lds_row, d);
-      finish(blockIdx.x + gridDim.x * q, d[0], d[1]);
+      ga.run(rows, D, lds_row, d, next, more);
+      finish(pp, d[0], d[1], bw);
     }
   };
   prime_first(npw_a, p.layer[0].w1, p.ld1);
@@ -347,9 +358,8 @@ __global__ __launch_bounds__(64 * NWV) void decode_b1_kernel(const B1Args p) {
 
     // ================= phase A: layer norm + fused [qkv | fc1] rows ===================================================
     layer_norm_to_lds(xc, w.ln_w, w.ln_b);
-    run_rows(npw_a, w.w1, p.ld1, [&](int pp, float d0, float d1) {
+    run_rows(npw_a, w.w1, p.ld1, w.b1, [&](int pp, float d0, float d1, uint32_t bw) {
       if (lane == 0) {
-        const uint32_t bw = *(const uint32_t*)(w.b1 + 2 * pp);
         uint32_t o = pack_bf16x2(d0 + lo_bf(bw), d1 + hi_bf(bw));  // F.linear's rounding point
         if (2 * pp >= QW) {  // fc1 rows: gelu on the bf16 value, rounded again (layers.py:24-25,137)
           const md_f32x2 gl = gelu_tanh_f32x2(md_f32x2{lo_bf(o), hi_bf(o)});
@@ -636,8 +646,7 @@ __global__ __launch_bounds__(64 * NWV) void decode_b1_kernel(const B1Args p) {
     layer_norm_to_lds(xc, p.post_ln_w, p.post_ln_b);
     float best = -INFINITY;
     int bi = 0x7fffffff;
-    run_rows(npw_d, p.lm_w, p.ld_lm, [&](int pp, float d0, float d1) {
-      const uint32_t bw = *(const uint32_t*)(p.lm_b + 2 * pp);
+    run_rows(npw_d, p.lm_w, p.ld_lm, p.lm_b, [&](int pp, float d0, float d1, uint32_t bw) {
       const uint32_t o = pack_bf16x2(d0 + lo_bf(bw), d1 + hi_bf(bw));
       if (lane == 0) *(uint32_t*)(p.logits + 2 * pp) = o;
       // greedy choice on the bf16 logits, ties -> lowest index, the suppressed id never (argmax_kernel's rule)
