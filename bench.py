@@ -586,8 +586,8 @@ def detect13_leg(model, cfg, args, dev, fp8=False):
         "images_per_sec": B2 / dt, "ms_per_step": dt * 1e3, "images_per_sec_tiling_prefetched": B2 / dt_prefetch,
         "ms_per_step_tiling_prefetched": dt_prefetch * 1e3, "batch": B2, "crops_per_image": n_crops, "max_objects": max_objects,
         "phase_ms": phase, "host_tiling_ms_per_image_one_thread": host_ms_per_image,
-        "note": "steps run back to back on one stream: phase_ms.host_tiling (PIL LANCZOS resize + crop cutting on the thread pool, "
-                "reference image_crops.py:124-167) is NOT hidden behind GPU work in images_per_sec; *_tiling_prefetched: the next "
+        "note": "steps run back to back on one stream: phase_ms.host_tiling (the pictures' pixels into pinned memory; the resize and the cutting of "
+                "reference image_crops.py:124-167 run on the device) is NOT hidden behind GPU work in images_per_sec; *_tiling_prefetched: the next "
                 "step's tiling is started before the current step runs (MoondreamModel.batch_detect_pipelined), same objects",
     }
     if phase.get("vision"):

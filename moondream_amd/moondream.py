@@ -714,7 +714,7 @@ class MoondreamModel(DeviceEngine):
     def prefetch_crops(self, images: Sequence[Image.Image]) -> None:
         """Start the host tiling of a batch NOW (thread pool, pinned staging buffers) so that a later call that encodes
         exactly these image objects -- ``batch_detect``, ``batch_generate_ids``, ... -- finds its crops cut: a serving
-        loop calls this for batch k+1 before it runs batch k, which hides the PIL resize of large images behind the
+        loop calls this for batch k+1 before it runs batch k, which hides the host's part of large images behind the
         GPU (the pipelined caption engine does the same by construction).  Results are identical."""
         if not hasattr(self, "_prefetched_crops"):
             self._prefetched_crops = {}
@@ -725,7 +725,7 @@ class MoondreamModel(DeviceEngine):
         while len(self._prefetched_crops) >= 2:  # the batch about to run + one ahead
             self.discard_prefetched_crops(next(iter(self._prefetched_crops)))
         # a FEW background workers: the step that is running needs the host for its own launches, and the tiling of one
-        # batch (tens of ms of CPU per large image) has a whole step's GPU time to finish
+        # batch (a few ms of CPU per large image, tens where the host resizes it) has a whole step's GPU time to finish
         pool = getattr(self, "_prefetch_pool", None)
         if pool is None:
             from concurrent.futures import ThreadPoolExecutor
@@ -1838,7 +1838,7 @@ class MoondreamModel(DeviceEngine):
     def batch_detect_pipelined(self, batches, settings: Optional[dict] = None, kind: str = "detect"):
         """Generator over an iterable of (images, objects) batches; yields ``batch_detect`` / ``batch_point`` (``kind``) of
         each, in order.  The detect counterpart of ``batch_generate_ids_pipelined``: while batch k runs on the GPU, the host
-        tiling of batch k+1 (PIL LANCZOS resize + crop cutting of large images: ~19 ms of CPU per 768x1024 image, reference
+        part of batch k+1's tiling (the pictures' pixels, or PIL LANCZOS resize + crop cutting where ``_cut_plan`` says so; reference
         image_crops.py:124-167) is cut into pinned staging buffers by the background workers (``prefetch_crops``), so that
         only the first batch's tiling is exposed.  Results are identical to calling ``batch_detect`` per batch."""
         if kind not in ("detect", "point"):

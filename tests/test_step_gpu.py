@@ -85,3 +85,20 @@ def test_prompts_whose_projections_leave_slices(rows):
     s, k = m.open_sequence(), rows - 130 if rows > 400 else 1
     got = torch.cat([m.step([(s, t[:k], range(k))]), m.step([(s, t[k:], range(rows - k))])])
     assert U.logit_error(got, want) < 7e-2
+
+
+@pytest.mark.parametrize("lens", [[1], [1, 1, 1], [4, 1, 7], [28]], ids=str)
+def test_prompts_through_retention_layers_round_alike(lens):
+    """A first token's retention hangs on the sign of q . k: prompts of few rows get the bits that they get beside others."""
+    cfg = U.config([U.retention(4, 32, 32), U.attention(4, 4, 32, 32, 64), U.retention(2, 64, 64)], width=328)
+    m, prompts = build(cfg), [U.tokens(n, cfg["vocab"], i) for i, n in enumerate(lens)]
+
+    def logits(texts):
+        slots = [m.open_sequence() for _ in texts]
+        got = m.step([(s, t, range(len(t))) for s, t in zip(slots, texts)])
+        for s in slots:
+            m.close_sequence(s)
+        return got
+
+    alone, beside = logits(prompts), logits(prompts + [U.tokens(30, cfg["vocab"], 9)])
+    assert torch.equal(alone, beside[: sum(lens)])
