@@ -4,12 +4,12 @@
 // The state of a head is kept transposed, fp32 [vdim][dim].
 //
 //   ssm_conv_kernel        convolution + bias + silu of x | B | C, softplus of dt: whole rows, inputs before the step from the slot's ring
-//   ssm_ring_kernel        the last projections of every sequence of the step -> its slot (row p % taps of the ring)
 //   ssm_scan_kernel        plain recurrence, token by token, any dtype, fp32 on the vector ALUs
 //   ssm_chunk_kernel       bf16 prefill on the matrix cores, 64 tokens at a time (below)
 //   ssm_segments_kernel    states at the start of every segment
 //   ssm_decode_kernel      bf16 decode step, one workgroup per (sequence, head): convolution, state update, output and gate in one launch
-//   ssm_norm_kernel        grouped RMS norm of the gated outputs, in place
+//   ssm_norm_kernel        grouped RMS norm of the gated outputs, in place; and the last projections of every sequence of the step -> its slot
+//                          (row p % taps of the ring)
 //
 // ssm_chunk_kernel.  A workgroup walks the chunks of a segment of a sequence for one head with the state in registers:
 //   y_t = exp(c_t) S^T C_t + sum_{s<=t} exp(c_t - c_s) dt_s (C_t . B_s) x_s + skip x_t,   c: running sum of -decay dt in the chunk
@@ -24,11 +24,9 @@ namespace {
 
 __device__ __forceinline__ float softplus_f32(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
 
-constexpr int CONV_ROWS = 16;  // rows per thread
-
-// a thread: 8 columns of x | B | C of CONV_ROWS consecutive rows; behind those blocks, 8 heads' dt of one row.
+// a thread: 8 columns of x | B | C of ROWS consecutive rows; behind those blocks, 8 heads' dt of one row.
 // TAPS > 0: inputs slide through registers; 0: any number
-template <typename T, int TAPS>
+template <typename T, int TAPS, int ROWS>
 __global__ __launch_bounds__(256) void ssm_conv_kernel(const LmSsm a, unsigned conv_blocks) {
   const int cw = a.cw();
   if (blockIdx.x >= conv_blocks) {
@@ -43,7 +41,7 @@ __global__ __launch_bounds__(256) void ssm_conv_kernel(const LmSsm a, unsigned c
     return;
   }
   const unsigned idx = blockIdx.x * 256 + threadIdx.x, units = cw / 8, rb = idx / units;
-  const int unit = idx - rb * units, r0 = rb * CONV_ROWS, r1 = min(r0 + CONV_ROWS, a.r.n_rows);
+  const int unit = idx - rb * units, r0 = rb * ROWS, r1 = min(r0 + ROWS, a.r.n_rows);
   if (r0 >= r1) return;
   const int c = unit * 8;
   const T* proj = (const T*)a.proj + a.col_x + c;
@@ -80,11 +78,11 @@ __global__ __launch_bounds__(256) void ssm_conv_kernel(const LmSsm a, unsigned c
     st8((T*)a.u + (int64_t)row * cw + c, y[0], y[1]);
   };
   if constexpr (TAPS > 0) {
-    auto walk = [&](auto whole) {  // whole: CONV_ROWS rows of one sequence
-      constexpr int BATCH = 8;     // rows whose loads are in flight together
+    auto walk = [&](auto whole) {  // whole: ROWS rows of one sequence
+      constexpr int BATCH = ROWS < 8 ? ROWS : 8;  // rows whose loads are in flight together
       start(r0);
 #pragma unroll
-      for (int b = 0; b < CONV_ROWS; b += BATCH) {
+      for (int b = 0; b < ROWS; b += BATCH) {
         const int b0 = r0 + b;
         if (!whole && b0 >= r1) break;
         decltype(ld8(proj)) in[BATCH];
@@ -109,7 +107,7 @@ __global__ __launch_bounds__(256) void ssm_conv_kernel(const LmSsm a, unsigned c
         }
       }
     };
-    if (r1 - r0 == CONV_ROWS && a.r.row_seq[r0] == a.r.row_seq[r1 - 1]) walk(std::true_type{});
+    if (r1 - r0 == ROWS && a.r.row_seq[r0] == a.r.row_seq[r1 - 1]) walk(std::true_type{});
     else walk(std::false_type{});
   } else {
     for (int row = r0; row < r1; ++row) {
@@ -124,10 +122,10 @@ __global__ __launch_bounds__(256) void ssm_conv_kernel(const LmSsm a, unsigned c
   }
 }
 
-// grid (sequences, blocks of 1024 columns)
+// block of 1024 columns of a sequence's last projections -> its slot's ring (behind the convolution, which reads what was there)
 template <typename T>
-__global__ __launch_bounds__(256) void ssm_ring_kernel(const LmSsm a) {
-  const int seq = blockIdx.x, cw = a.cw(), c = (blockIdx.y * 256 + threadIdx.x) * 4;
+__device__ __forceinline__ void ssm_ring(const LmSsm& a, int seq, int block) {
+  const int cw = a.cw(), c = (block * 256 + threadIdx.x) * 4;
   const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, pos0 = a.r.seq_pos0[seq], slot = a.r.seq_slot[seq];
   T* ring = (T*)a.conv_state + (int64_t)slot * a.taps * cw;
   const int keep = min(len, a.taps - 1);
@@ -135,17 +133,21 @@ __global__ __launch_bounds__(256) void ssm_ring_kernel(const LmSsm a) {
   for (int t = len - keep; t < len; ++t) st4(ring + (int64_t)((pos0 + t) % a.taps) * cw + c, ld4((const T*)a.proj + (int64_t)(row0 + t) * a.ldp + a.col_x + c));
 }
 
+// 16 rows per thread, or 4 where that leaves most of the chip without a workgroup (700 rows, 2304 columns: 6.3 us, 16.6 with 16 rows;
+// 17 rows of 2176: 5.0 us, 8.3)
 template <typename T>
 md_status conv(const LmSsm& a, hipStream_t s) {
-  const int64_t n = (int64_t)((a.r.n_rows + CONV_ROWS - 1) / CONV_ROWS) * (a.cw() / 8), n_dt = (int64_t)a.r.n_rows * ((a.heads + 7) / 8);
-  if (n >= 1 << 30 || n_dt >= 1 << 30) return MD_ERR_UNSUPPORTED;
+  const int64_t units = a.cw() / 8, n_dt = (int64_t)a.r.n_rows * ((a.heads + 7) / 8);
+  if ((a.r.n_rows + 15) / 16 * units >= 1 << 30 || n_dt >= 1 << 30) return MD_ERR_UNSUPPORTED;
+  const bool few = a.taps <= 4 && (a.r.n_rows + 15) / 16 * units <= 256 * 256;
+  const int64_t n = (a.r.n_rows + (few ? 3 : 15)) / (few ? 4 : 16) * units;
   const unsigned conv_blocks = (unsigned)((n + 255) / 256), dt_blocks = (unsigned)((n_dt + 255) / 256);
-  auto fn = a.taps == 1 ? ssm_conv_kernel<T, 1> : a.taps == 2 ? ssm_conv_kernel<T, 2> : a.taps == 3 ? ssm_conv_kernel<T, 3>
-            : a.taps == 4 ? ssm_conv_kernel<T, 4> : ssm_conv_kernel<T, 0>;
+  auto pick = [&](auto rows) {
+    constexpr int R = decltype(rows)::value;
+    return a.taps == 1 ? ssm_conv_kernel<T, 1, R> : a.taps == 2 ? ssm_conv_kernel<T, 2, R> : a.taps == 3 ? ssm_conv_kernel<T, 3, R> : ssm_conv_kernel<T, 4, R>;
+  };
+  auto fn = a.taps > 4 ? ssm_conv_kernel<T, 0, 16> : few ? pick(std::integral_constant<int, 4>{}) : pick(std::integral_constant<int, 16>{});
   hipLaunchKernelGGL(fn, dim3(conv_blocks + dt_blocks), dim3(256), 0, s, a, conv_blocks);
-  MD_TRY(md_launch_status());
-  if (a.taps == 1) return MD_OK;
-  hipLaunchKernelGGL(ssm_ring_kernel<T>, dim3(a.r.n_seq, (a.cw() + 1023) / 1024), dim3(256), 0, s, a);
   return md_launch_status();
 }
 
@@ -238,10 +240,14 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(const LmSsm a) {
 
 // one row per workgroup.  Norm group k: elements k * gs .. of the heads' outputs without their padding; element f lies at column
 // f / vdim * vp + f % vdim.  BLOCK: all waves take the groups one after the other, else a wave takes every fourth group.
-// V: consecutive elements at a time (groups and heads are multiples of it).
+// V: consecutive elements at a time (groups and heads are multiples of it).  Workgroups behind the rows': the rings of the sequences.
 template <typename T, bool BLOCK, int V>
 __global__ __launch_bounds__(256) void ssm_norm_kernel(const LmSsm a) {
   __shared__ float red[4];
+  if ((int)blockIdx.x >= a.r.n_rows) {
+    const int i = blockIdx.x - a.r.n_rows, blocks = (a.cw() + 1023) / 1024;
+    return ssm_ring<T>(a, i / blocks, i % blocks);
+  }
   T* row = (T*)a.out + (int64_t)blockIdx.x * a.ldo;
   const int gs = a.heads * a.vdim / a.norm_groups, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int k = BLOCK ? 0 : wave; k < a.norm_groups; k += BLOCK ? 1 : 4) {
@@ -270,12 +276,13 @@ __global__ __launch_bounds__(256) void ssm_norm_kernel(const LmSsm a) {
   }
 }
 
+// ring: behind conv(), whose inputs the next step's go on from
 template <typename T>
-md_status norm(const LmSsm& a, hipStream_t s) {
+md_status norm(const LmSsm& a, bool ring, hipStream_t s) {
   const int gs = a.heads * a.vdim / a.norm_groups;
   const bool v4 = a.vdim % 4 == 0 && gs % 4 == 0, block = a.norm_groups < 4;
   auto fn = v4 ? (block ? ssm_norm_kernel<T, true, 4> : ssm_norm_kernel<T, false, 4>) : (block ? ssm_norm_kernel<T, true, 1> : ssm_norm_kernel<T, false, 1>);
-  hipLaunchKernelGGL(fn, dim3(a.r.n_rows), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(fn, dim3(a.r.n_rows + (ring && a.taps > 1 ? a.r.n_seq * ((a.cw() + 1023) / 1024) : 0)), dim3(256), 0, s, a);
   return md_launch_status();
 }
 
@@ -286,7 +293,7 @@ md_status plain(const LmSsm& a, hipStream_t s) {
   auto scan = a.dp <= 64 ? ssm_scan_kernel<T, 1> : a.dp <= 128 ? ssm_scan_kernel<T, 2> : a.dp <= 256 ? ssm_scan_kernel<T, 4> : ssm_scan_kernel<T, 8>;
   hipLaunchKernelGGL(scan, dim3(a.r.n_seq, a.heads, a.vp / 16), dim3(256), 0, s, a);
   MD_TRY(md_launch_status());
-  return norm<T>(a, s);
+  return norm<T>(a, true, s);
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
@@ -659,12 +666,12 @@ md_status lm_ssm_mfma(const LmSsm& a, hipStream_t s) {
   }
   hipLaunchKernelGGL(k.run, grid, dim3(256), k.lds, s, a);
   MD_TRY(md_launch_status());
-  return norm<bf16_t>(a, s);
+  return norm<bf16_t>(a, true, s);
 }
 
 bool lm_ssm_decode_takes(const LmSsm& a) { return decode_pick(a) != nullptr; }
 md_status lm_ssm_decode(const LmSsm& a, hipStream_t s) {
   hipLaunchKernelGGL(decode_pick(a), dim3(a.heads, a.r.n_seq), dim3(256), 0, s, a);
   MD_TRY(md_launch_status());
-  return norm<bf16_t>(a, s);
+  return norm<bf16_t>(a, false, s);
 }

@@ -102,3 +102,23 @@ def test_prompts_through_retention_layers_round_alike(lens):
 
     alone, beside = logits(prompts), logits(prompts + [U.tokens(30, cfg["vocab"], 9)])
     assert torch.equal(alone, beside[: sum(lens)])
+
+
+@pytest.mark.parametrize("lens", [[1100], [517, 3, 580]], ids=str)
+def test_state_space_prompts_that_fill_the_chip(lens):
+    """Rows and columns enough for the convolution's 16 rows per thread (8224 columns), and a token behind each prompt, whose window is what
+    the norm's launch left in the slots."""
+    cfg = U.stream_config([(U.ssm(64, 128, 16), None)], width=72, vocab=200, streams=1, positions=1200)
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    w = U.weights(cfg, 3, 1.5)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=BF16, max_batch=4, max_context=1200)
+    ts = [U.tokens(n + 1, cfg["vocab"], i) for i, n in enumerate(lens)]
+    want = [O.forward(cfg, w, t) for t in ts]
+    slots = [m.open_sequence() for _ in ts]
+    got = m.step([(s, t[:-1], range(len(t) - 1)) for s, t in zip(slots, ts)])
+    e = U.logit_errors(got, torch.cat([x[:-1] for x in want])).sort().values
+    assert float(e[int(0.9 * len(e))]) < 7e-2 and float(e[-1]) < 1.0
+    got = m.step([(s, t[-1:], [0]) for s, t in zip(slots, ts)])
+    assert float(U.logit_errors(got, torch.cat([x[-1:] for x in want])).max()) < 7e-2
