@@ -331,7 +331,7 @@ __global__ __launch_bounds__(256) void conv_state_kernel(const LmAttn a, int nco
 constexpr int PLAIN_TK = 64;
 
 // Its cost is the keys' and values' way through L2, once per row: eight elements of a key, or of eight keys, per load (380 rows of 190 keys, 16
-// heads of 128, fp32: 93 us, 560 us with one at a time).
+// heads of 128, fp32: 93 us, 560 us with one at a time).  Sums run over coordinates and keys in order, one chain each.
 template <typename T>
 __global__ __launch_bounds__(256) void attn_plain_kernel(const LmAttn a) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
@@ -355,26 +355,29 @@ __global__ __launch_bounds__(256) void attn_plain_kernel(const LmAttn a) {
   }
   __syncthreads();
   const int first = a.chunk > 0 ? i / a.chunk * a.chunk : 0;
-  for (int j0 = first & ~7; j0 <= i; j0 += PLAIN_TK) {  // (from a row of eight keys on: their values lie together)
+  for (int j0 = first; j0 <= i; j0 += PLAIN_TK) {
     const int n = min(PLAIN_TK, i + 1 - j0);
     for (int e = tid; e < H * PLAIN_TK; e += 256) {
       const int g = e / PLAIN_TK, jj = e - g * PLAIN_TK;
       if (jj >= n) continue;
-      f32x4 s = {0.f, 0.f, 0.f, 0.f};
+      float s = 0.f;
 #pragma unroll 4
       for (int d = 0; d < dp; d += 8) {  // (coordinates behind the head's are zeros)
         const auto k = ld8(kb + key_index(j0 + jj, g / rep, d, G, dp));
-        const float* q = qs + g * dp + d;
-        s += half8(k, 0) * *(const f32x4*)q;
-        s += half8(k, 1) * *(const f32x4*)(q + 4);
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+          const f32x4 kv = half8(k, hf), qv = *(const f32x4*)(qs + g * dp + d + 4 * hf);
+#pragma unroll
+          for (int t = 0; t < 4; ++t) s = __builtin_fmaf(qv[t], kv[t], s);
+        }
       }
-      raw[e] = ((s[0] + s[1]) + (s[2] + s[3])) * a.scale - a.slope[g] * (float)(i - (j0 + jj));
+      raw[e] = __builtin_fmaf(a.scale, s, -(a.slope[g] * (float)(i - (j0 + jj))));
     }
     __syncthreads();
     for (int e = tid; e < H * PLAIN_TK; e += 256) {
       const int h = e / PLAIN_TK, jj = e - h * PLAIN_TK;
       float s = -INFINITY;
-      if (jj < n && j0 + jj >= first) {
+      if (jj < n) {
         s = 0.f;
 #pragma unroll 4
         for (int g = 0; g < H; ++g) s += a.mix[h * H + g] * raw[g * PLAIN_TK + jj];
@@ -397,20 +400,19 @@ __global__ __launch_bounds__(256) void attn_plain_kernel(const LmAttn a) {
     __syncthreads();
     for (int c = tid; c < H * vp; c += 256) {
       const int h = c / vp, d = c - h * vp;
-      const int lo = max(first - j0, 0), lo8 = min((lo + 7) & ~7, n), hi8 = max(n & ~7, lo8);
       const float* p = mixed + h * PLAIN_TK;
-      f32x4 o = {0.f, 0.f, 0.f, 0.f};
-      float rest = 0.f;
-      auto one = [&](int jj) { rest += p[jj] * ldf(vb + value_index(j0 + jj, h / rep, d, G, vp)); };
-      for (int jj = lo; jj < lo8; ++jj) one(jj);
+      float o = acc[c] * al[h];
+      auto one = [&](int jj) { o = __builtin_fmaf(p[jj], ldf(vb + value_index(j0 + jj, h / rep, d, G, vp)), o); };
+      const int lo = min(-j0 & 7, n), hi = lo + ((n - lo) & ~7);  // the values of a row of eight keys lie together
+      for (int jj = 0; jj < lo; ++jj) one(jj);
 #pragma unroll 4
-      for (int jj = lo8; jj < hi8; jj += 8) {
+      for (int jj = lo; jj < hi; jj += 8) {
         const auto v = ld8(vb + value_index(j0 + jj, h / rep, d, G, vp));
-        o += half8(v, 0) * *(const f32x4*)(p + jj);
-        o += half8(v, 1) * *(const f32x4*)(p + jj + 4);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) o = __builtin_fmaf(p[jj + t], half8(v, t / 4)[t & 3], o);
       }
-      for (int jj = hi8; jj < n; ++jj) one(jj);
-      acc[c] = acc[c] * al[h] + (((o[0] + o[1]) + (o[2] + o[3])) + rest);
+      for (int jj = hi; jj < n; ++jj) one(jj);
+      acc[c] = o;
     }
     __syncthreads();
   }

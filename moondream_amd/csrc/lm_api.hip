@@ -240,6 +240,7 @@ struct Step {
   LmAddend add = {};           // pending addend of the residual stream(s)
   const float* mix = nullptr;  // streams: the weights around the sublayer that made it
   bool few = false;            // a step of few rows
+  bool chain = false;          // fp32: the products' order of sums (gemm_f32.hip)
   bool ready = false;          // w.h holds the next sublayer's input already ...
   const float* sumsq = nullptr;  // ... but for the factor that these give its rows, in the order of the matrix operand
 
@@ -262,7 +263,7 @@ struct Step {
   }
 
   md_status linear(const void* a, int64_t lda, const md_linear& lin, void* c, int64_t ldc, int rows, bool split = true) {
-    if (m->dtype == MD_DTYPE_F32) return md_gemm_f32(a, lda, &lin, c, ldc, rows, s);
+    if (m->dtype == MD_DTYPE_F32) return lm_gemm_f32(a, lda, lin, c, ldc, rows, chain, s);
     md_gemm_args g = {};
     g.a = a;
     g.lda = lda;
@@ -543,9 +544,9 @@ struct Step {
     }
     add.src = w.y;
     if (m->dtype == MD_DTYPE_F32) {
-      MD_TRY(lm_grouped_gemm_f32(w.h, m->width_pad, w.row_of, l.gate_up, l.experts, w.offsets, w.gu, ld, slots, s));
+      MD_TRY(lm_grouped_gemm_f32(w.h, m->width_pad, w.row_of, l.gate_up, l.experts, w.offsets, w.gu, ld, slots, chain, s));
       MD_TRY(lm_silu_mul_f32(w.gu, ld, w.act, l.down.k_pad, slots, l.ff_pad, s));
-      return lm_grouped_gemm_f32(w.act, l.down.k_pad, nullptr, l.down, l.experts, w.offsets, w.y, m->width_pad, slots, s);
+      return lm_grouped_gemm_f32(w.act, l.down.k_pad, nullptr, l.down, l.experts, w.offsets, w.y, m->width_pad, slots, chain, s);
     }
     MD_TRY(md_gemm_grouped_bf16(w.h, m->width_pad, w.row_of, l.gate_up, l.experts, w.offsets, w.act, l.down.k_pad, slots, true, true, s));
     return md_gemm_grouped_bf16(w.act, l.down.k_pad, nullptr, l.down, l.experts, w.offsets, w.y, m->width_pad, slots, false, false, s);
@@ -624,6 +625,7 @@ extern "C" md_status md_lm_forward(const md_lm_model* m, const md_lm_batch* b, c
   if (workspace_bytes < w.total) return MD_ERR_WORKSPACE;
   Step step{m, b, st, w, (hipStream_t)stream, decode_regime(m, b->n_rows)};
   step.few = step_regime(m, b);
+  for (int i = 0; i < m->n_layers; ++i) step.chain = step.chain || m->layers[i].mixer == MD_MIXER_RETENTION;
   return step.run(logit_rows, n_logits, logits, ld_logits, layer_out);
 }
 

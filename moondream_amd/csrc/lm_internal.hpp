@@ -262,7 +262,9 @@ md_status lm_ssm_decode(const LmSsm& a, hipStream_t s);                  // bf16
 md_status lm_route(int dtype, const LmRoute& a, hipStream_t s);          // router, choice, weights, rows by expert
 // C[slot] = A[row of slot] W_e^T for the slots of every expert e; lin: one expert's matrix, all follow one another
 md_status lm_grouped_gemm_f32(const void* a, int64_t lda, const int32_t* row_of, const md_linear& lin, int experts, const int32_t* offsets, void* c,
-                              int64_t ldc, int slots, hipStream_t s);
+                              int64_t ldc, int slots, bool chain, hipStream_t s);
+// md_gemm_f32, the order of sums chosen (gemm_f32.hip)
+md_status lm_gemm_f32(const void* a, int64_t lda, const md_linear& lin, void* c, int64_t ldc, int rows, bool chain, hipStream_t s);
 
 // dtype: MD_DTYPE_*
 md_status lm_embed(int dtype, const void* table, int64_t ld, const int32_t* tokens, float* x, int rows, int vocab, hipStream_t s);

@@ -39,26 +39,27 @@ __global__ __launch_bounds__(256) void ret_rotate_kernel(const LmRet a) {
   }
 }
 
-// grid (n_seq, heads, vp / 16): 16 columns of the state, 16 neighbouring lanes per column, each owning rows 4 l .. + 3 of every 64.  Tokens are
+// grid (n_seq, heads, vp / 16): 16 columns of the state, 16 neighbouring lanes per column, each owning every 16th row of it.  Tokens are
 // staged 16 at a time and then run without a barrier: the recurrence is a chain, what counts is what lies on it (two sequences of 190 tokens,
-// 16 heads of 128: 57 us, 235 us with three barriers per token).
-// Q: quads of state rows per thread, dp <= 64 Q
+// 16 heads of 128: 35 us; 235 us with three barriers per token).  An output is summed down a lane's rows, then over the lanes in turn: a first
+// token's result hangs on the order where q . k is small (gemm_f32.hip).
+// Q: quads of state rows per lane, dp <= 64 Q
 constexpr int PLAIN_TOKENS = 16;
 template <typename T, int Q>
 __global__ __launch_bounds__(256) void ret_scan_kernel(const LmRet a) {
-  __shared__ __attribute__((aligned(16))) float qs[PLAIN_TOKENS][64 * Q], ks[PLAIN_TOKENS][64 * Q];
-  __shared__ float vs[PLAIN_TOKENS][16], os[PLAIN_TOKENS][16];
+  constexpr int R = 4 * Q, LD = R + 4;  // rows per lane, their stride: [token][lane][row]
+  __shared__ __attribute__((aligned(16))) float qs[PLAIN_TOKENS][16 * LD], ks[PLAIN_TOKENS][16 * LD];
+  __shared__ float vs[PLAIN_TOKENS][16], os[PLAIN_TOKENS][16][17];
   const int seq = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, l = tid & 15, col = tid >> 4, e0 = blockIdx.z * 16, e = e0 + col;
   const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, pos0 = a.r.seq_pos0[seq];
   const int dp = a.dp, vp = a.vp, H = a.heads;
   float* st = a.state + (((int64_t)a.r.seq_slot[seq] * H + h) * vp + e) * dp;
   const float decay = a.decay[h];
-  f32x4 S[Q];
+  float S[R];
 #pragma unroll
-  for (int i = 0; i < Q; ++i) {
-    const int d = 64 * i + 4 * l;
-    S[i] = (pos0 > 0 && d < dp) ? *(const f32x4*)(st + d) : f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+  for (int i = 0; i < R; ++i) S[i] = (pos0 > 0 && 16 * i < dp) ? st[16 * i + l] : 0.f;
+  if (dp < 64 * Q)  // rows behind the head's: zeros, which add nothing
+    for (int i = tid; i < PLAIN_TOKENS * 16 * LD; i += 256) (&qs[0][0])[i] = (&ks[0][0])[i] = 0.f;
   f32x4 qn[Q], kn[Q];  // the next tokens', under way during these
   float vn = 0.f;
   const int quads = dp / 4;
@@ -82,8 +83,11 @@ __global__ __launch_bounds__(256) void ret_scan_kernel(const LmRet a) {
     for (int j = 0; j < Q; ++j) {
       const int i = tid + 256 * j, t = i / quads, d = (i - t * quads) * 4;
       if (t >= n) continue;
-      *(f32x4*)(qs[t] + d) = qn[j];
-      *(f32x4*)(ks[t] + d) = kn[j];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        qs[t][((d & 15) + k) * LD + (d >> 4)] = qn[j][k];
+        ks[t][((d & 15) + k) * LD + (d >> 4)] = kn[j][k];
+      }
     }
     if (col < n) vs[col][l] = vn;
     __syncthreads();
@@ -91,26 +95,29 @@ __global__ __launch_bounds__(256) void ret_scan_kernel(const LmRet a) {
 #pragma unroll 4
     for (int t = 0; t < n; ++t) {
       const float v = vs[t][col];
-      f32x4 o = {0.f, 0.f, 0.f, 0.f};
+      float o = 0.f;
 #pragma unroll
-      for (int i = 0; i < Q; ++i) {
-        const int d = 64 * i + 4 * l;
-        if (i + 1 < Q || d < dp) {
-          S[i] = decay * S[i] + *(const f32x4*)(ks[t] + d) * v;
-          o += S[i] * *(const f32x4*)(qs[t] + d);
+      for (int q = 0; q < Q; ++q) {
+        const f32x4 kq = *(const f32x4*)(ks[t] + l * LD + 4 * q), qq = *(const f32x4*)(qs[t] + l * LD + 4 * q);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          S[4 * q + k] = __builtin_fmaf(decay, S[4 * q + k], kq[k] * v);
+          o = __builtin_fmaf(S[4 * q + k], qq[k], o);
         }
       }
-      const float sum = row_sum_16((o[0] + o[1]) + (o[2] + o[3]));
-      if (l == 0) os[t][col] = sum;
+      os[t][col][l] = o;
     }
     __syncthreads();
-    if (col < n) a.of[((int64_t)(row0 + t0 + col) * H + h) * vp + e0 + l] = os[col][l];
+    if (col < n) {  // this thread's token col, column l
+      float sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sum += os[col][l][i];
+      a.of[((int64_t)(row0 + t0 + col) * H + h) * vp + e0 + l] = sum;
+    }
   }
 #pragma unroll
-  for (int i = 0; i < Q; ++i) {
-    const int d = 64 * i + 4 * l;
-    if (d < dp) *(f32x4*)(st + d) = S[i];
-  }
+  for (int i = 0; i < R; ++i)
+    if (16 * i < dp) st[16 * i + l] = S[i];
 }
 
 template <typename T>

@@ -1,8 +1,13 @@
-"""fp32 products at the edges of their tiles: few rows (K shared by the waves), tiles with remainders, every count of K steps, grouped rows."""
+"""fp32 products at the edges of their tiles: few rows, tiles with remainders, every count of K steps; one order of sums at every number of
+rows; prompts through retention layers, whose first tokens show any other order."""
 import ctypes as C
+import os
 
+import numpy as np
 import pytest
 import torch
+
+import lm_util as U
 
 from moondream_amd import _lib
 
@@ -25,3 +30,45 @@ def test_product(m, n, k, bias):
         # k products of rounding error 2^-24 each, added in fp32
         bound = (a[:, :k].abs().double() @ w.abs().double().t() + b.abs().double()) * (k + 1) * 2.0 ** -24
         assert bool(((c[:, :n].double() - want).abs() <= bound).all()) and bool((c[:, n:] == 7).all())
+
+
+@pytest.mark.parametrize("n,k", [(64, 64), (192, 320), (2048, 1472)])
+def test_a_row_has_the_same_sums_beside_any_others(n, k):
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    a, w = torch.randn(300, k, generator=g, device="cuda"), torch.randn(n, k, generator=g, device="cuda")
+    lin = _lib.MdLinear()
+    lin.w, lin.b, lin.n, lin.k, lin.n_pad, lin.k_pad = w.data_ptr(), None, n, k, n, k
+    got = []
+    for m in (1, 16, 17, 32, 33, 64, 65, 300):
+        c = torch.empty(m, n, device="cuda")
+        _lib.check(lib.md_gemm_f32(a.data_ptr(), k, C.byref(lin), c.data_ptr(), n, m, torch.cuda.current_stream().cuda_stream), "md_gemm_f32")
+        got.append(c)
+    assert all(torch.equal(c, got[-1][: c.shape[0]]) for c in got)
+
+
+RETENTION = U.config([U.retention(4, 32, 32), U.attention(4, 2, 32, 32, 50), U.retention(2, 96, 64), U.retention(1, 160, 32)], width=328, vocab=64, ff=600)
+LENS = [1, 1, 7, 3, 60, 33]
+
+
+def retention_logits(groups):
+    """Logits of LENS's prompts and of a token behind each, the prompts read in groups."""
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    m = LayeredLM(LayeredLMConfig.from_dict(RETENTION), U.weights(RETENTION, 3), dtype=torch.float32, max_batch=8, max_context=128)
+    ts, out = [U.tokens(n + 1, RETENTION["vocab"], i) for i, n in enumerate(LENS)], {}
+    for group in groups:
+        slots = {i: m.open_sequence() for i in group}
+        a = m.step([(slots[i], ts[i][:-1], range(LENS[i])) for i in group])
+        b = m.step([(slots[i], ts[i][-1:], [0]) for i in group])
+        out.update(zip(group, zip(a.split([LENS[i] for i in group]), b.split(1))))
+    return torch.cat([x for i in range(len(LENS)) for x in out[i]]).cpu()
+
+
+@pytest.mark.parametrize("groups", [[[0, 1, 2, 3, 4, 5]], [[0, 1, 2], [3], [4], [5]], [[0, 3], [1, 2], [4, 5]], [[5, 0], [4, 1, 2, 3]]], ids=str)
+def test_prompts_through_retention_layers_keep_their_results(groups):
+    """A first token's retention is its value times q . k, normed: where q . k is small another order of any sum before it changes the result beyond
+    fp32 rounding.  The results on record (made when every sum was one chain, token by token) stand, whatever else is in the step."""
+    want = np.load(os.path.join(os.path.dirname(__file__), "golden", "retention_f32.npz"))["logits"]
+    assert np.array_equal(retention_logits(groups).numpy(), want)
