@@ -1194,6 +1194,7 @@ md_status md_gemm_grouped_partial(const void* a, int64_t lda, const int32_t* row
 extern "C" md_status md_gemm_partial_f32_pair(const void* a0, int64_t lda0, const md_linear* lin0, float* partial0,
                                               const void* a1, int64_t lda1, const md_linear* lin1, float* partial1,
                                               int32_t m, int64_t ld_partial, int64_t slice_stride, void* stream) {
+  MD_CHECK_ARG(m <= 128);  // (one row tile)
   GemmPair pair;
   md_status chk = fill_partial(pair.g[0], a0, lda0, lin0, m, partial0, ld_partial, slice_stride);
   if (chk != MD_OK) return chk;

@@ -39,6 +39,14 @@ def test_argument_validation_needs_no_gpu():
     assert lib.md_vit_workspace_bytes(None, 4) == 0
 
 
+@pytest.mark.parametrize("m", [129, 200, 4096])
+def test_k_slice_products_refuse_more_rows_than_their_tile(m):
+    lib = _lib.load()
+    lin, at = ctypes.byref(_lib.MdLinear(4096, None, 64, 64, 64, 64)), 4096  # (refused before anything is read)
+    assert lib.md_gemm_partial_f32(at, 64, lin, m, at, 64, 64 * m, None) == 1
+    assert lib.md_gemm_partial_f32_pair(at, 64, lin, at, at, 64, lin, at, m, 64, 64 * m, None) == 1
+
+
 def test_fp8_entry_points_validate_on_the_host():
     lib = _lib.load()
     assert lib.md_gemm_f8(None, None) == 1
