@@ -790,6 +790,8 @@ typedef struct {
 
 typedef struct {
   int32_t n_seq, n_rows, max_len;  /* max_len: rows of the longest sequence of the step; 1 = a decode step */
+  int32_t n_going;                 /* how many of the sequences go on from earlier positions (0: not said).  With retention layers steps
+                                      of few rows are faster if all do: the first token of a sequence needs the rounding of long prompts */
   const int32_t* tokens;           /* device [n_rows] */
   const int32_t* row_seq;          /* device [n_rows] */
   const int32_t* row_pos;          /* device [n_rows] */
@@ -801,7 +803,7 @@ typedef struct {
   const int32_t* seq_ctx0;         /* device [n_seq + 1]: running sums of the same; not read when max_len == 1 */
 } md_lm_batch;
 
-/* Workspace of a step: reads the counts of b (n_seq, n_rows, max_len, max_ctx, ctx_rows), not its pointers. */
+/* Workspace of a step: reads the counts of b (n_seq, n_rows, max_len, n_going, max_ctx, ctx_rows), not its pointers. */
 size_t md_lm_workspace_bytes(const md_lm_model* m, const md_lm_batch* b, int32_t n_logits);
 
 /* One step: embedding, every layer, state update.  logit_rows (device int32 [n_logits], indices of rows of the step; NULL: rows

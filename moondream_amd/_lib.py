@@ -192,7 +192,7 @@ class MdLmState(C.Structure):
 
 
 class MdLmBatch(C.Structure):
-    _fields_ = [("n_seq", c_int32), ("n_rows", c_int32), ("max_len", c_int32), ("tokens", c_void_p), ("row_seq", c_void_p),
+    _fields_ = [("n_seq", c_int32), ("n_rows", c_int32), ("max_len", c_int32), ("n_going", c_int32), ("tokens", c_void_p), ("row_seq", c_void_p),
                 ("row_pos", c_void_p), ("seq_row0", c_void_p), ("seq_pos0", c_void_p), ("seq_slot", c_void_p), ("max_ctx", c_int32),
                 ("ctx_rows", c_int32), ("seq_ctx0", c_void_p)]
 

@@ -45,13 +45,12 @@ constexpr int STEP_PLAIN_ROWS = 8;
 
 // products that go on with the row-wise step behind them (gemm_step.hip)
 // (a router needs whole normed rows, which leaves nothing to go on with; and the first token's retention is its value times q . k, normed: only
-// the sign of q . k is left, so a rounding of the norm at another place turns it over where q . k is small.  Prompts through retention layers
-// keep the rounding of all other prompts: 12 tokens 1.78 ms, 1.29 this way.)
+// the sign of q . k is left, so a rounding of the norm at another place turns it over where q . k is small.  A step in which any sequence may
+// begin keeps the rounding of long prompts where a layer has retention: 12 tokens 1.78 ms, 1.29 this way.)
 inline bool step_regime(const md_lm_model* m, const md_lm_batch* b) {
   if (m->dtype != MD_DTYPE_BF16 || b->n_rows > LM_STEP_ROWS) return false;
-  const bool fresh = b->max_len > 1 ? b->ctx_rows == b->n_rows : b->max_ctx == 1;
   for (int i = 0; i < m->n_layers; ++i)
-    if (m->layers[i].experts > 0 || (fresh && m->layers[i].mixer == MD_MIXER_RETENTION)) return false;
+    if (m->layers[i].experts > 0 || (b->n_going != b->n_seq && m->layers[i].mixer == MD_MIXER_RETENTION)) return false;
   return true;
 }
 

@@ -135,7 +135,8 @@ class LayeredLM(DeviceEngine):
             for n in (n_rows, n_rows, n_rows, n_seq + 1, n_seq, n_seq, n_seq + 1, n_want):
                 at.append(at[-1] + n)
             ptr = [dev.data_ptr() + 4 * o for o in at]
-            batch = _lib.MdLmBatch(n_seq, n_rows, max(lens), ptr[0], ptr[1], ptr[2], ptr[3], ptr[4], ptr[5], max_ctx, ctx0[-1], ptr[6])
+            going = sum(p > 0 for p in pos0)
+            batch = _lib.MdLmBatch(n_seq, n_rows, max(lens), going, ptr[0], ptr[1], ptr[2], ptr[3], ptr[4], ptr[5], max_ctx, ctx0[-1], ptr[6])
             logits = torch.empty(max(n_want, 1), self.w.model.head.n_pad, dtype=self.dtype, device=self._device)
             taps = None
             if layer_out is not None:
@@ -172,14 +173,15 @@ class LayeredLM(DeviceEngine):
         self._reserve(max(pos) + max_tokens)
         logits = self._decode_logits(b)
         ctx = self.state.ctx
-        ws = self._workspace(self.lib.md_lm_workspace_bytes(C.byref(self.w.model), C.byref(_lib.MdLmBatch(b, b, 1, max_ctx=ctx)), b), 2)
+        going = sum(p > 0 for p in pos)
+        ws = self._workspace(self.lib.md_lm_workspace_bytes(C.byref(self.w.model), C.byref(_lib.MdLmBatch(b, b, 1, going, max_ctx=ctx)), b), 2)
         uniforms = torch.rand(max_tokens, b, device=self._device, dtype=torch.float32, generator=generator) if temperature != 0 else None
         rows = self._h2d(torch.tensor(list(range(b + 1)) + list(slots), dtype=torch.int32))
         st = self.state.struct()
 
         def make_step(pos_buf):
             def one_step(tok_in, tok_out, u_row):
-                batch = _lib.MdLmBatch(b, b, 1, tok_in.data_ptr(), rows.data_ptr(), pos_buf.data_ptr(), rows.data_ptr(), pos_buf.data_ptr(),
+                batch = _lib.MdLmBatch(b, b, 1, going, tok_in.data_ptr(), rows.data_ptr(), pos_buf.data_ptr(), rows.data_ptr(), pos_buf.data_ptr(),
                                        rows.data_ptr() + 4 * (b + 1), ctx, 0, None)
                 _lib.check(
                     self.lib.md_lm_decode_step(
@@ -193,7 +195,7 @@ class LayeredLM(DeviceEngine):
 
             return one_step
 
-        key = (tuple(slots), ctx, suppress_id, ws.data_ptr(), logits.data_ptr(), float(temperature), float(top_p), self.dtype)
+        key = (tuple(slots), ctx, going, suppress_id, ws.data_ptr(), logits.data_ptr(), float(temperature), float(top_p), self.dtype)
         hist = self._lockstep_loop(first, pos, max_tokens, make_step, key, eos_id, check_every, uniforms, keep=(rows, ws, logits))
         for s in slots:
             self.state.pool.length[s] += hist.shape[0] - 1

@@ -127,6 +127,14 @@ def test_entry_points_validate_on_the_host():
     assert lib.md_lm_workspace_bytes(ctypes.byref(p.model), ctypes.byref(_lib.MdLmBatch(2, 7, 5, max_ctx=64)), 2) > 0
 
 
+def test_steps_say_how_many_sequences_go_on():
+    """The count lies where the structure had padding: everything else is where it was."""
+    assert _lib.MdLmBatch.n_going.offset == 12 and _lib.MdLmBatch.tokens.offset == 16 and ctypes.sizeof(_lib.MdLmBatch) == 80
+    lib, (cfg, w, p) = _lib.load(), _packed("retention", torch.bfloat16)
+    size = lambda going: lib.md_lm_workspace_bytes(ctypes.byref(p.model), ctypes.byref(_lib.MdLmBatch(3, 9, 4, going, max_ctx=64, ctx_rows=40)), 3)  # noqa: E731
+    assert size(0) == size(2) < size(3)  # (the rows' sums of squares)
+
+
 def test_language_model_symbols_are_declared():
     assert set(_lib.LM_SYMBOLS) <= set(_lib.exported_symbols())
 

@@ -104,6 +104,22 @@ def test_prompts_through_retention_layers_round_alike(lens):
     assert torch.equal(alone, beside[: sum(lens)])
 
 
+@pytest.mark.parametrize("going", [1, 5])
+@pytest.mark.parametrize("lens", [[1], [1, 1], [7], [3, 1, 9], [20]], ids=str)
+def test_prompts_that_join_a_running_step_round_alike(lens, going):
+    """The same beside sequences that go on, in a step of few rows (continuous batching)."""
+    cfg = U.config([U.retention(4, 32, 32), U.attention(4, 4, 32, 32, 64), U.retention(2, 64, 64)], width=328)
+    m, prompts = build(cfg), [U.tokens(n, cfg["vocab"], i) for i, n in enumerate(lens)]
+    slots = [m.open_sequence() for _ in prompts]
+    alone = m.step([(s, t, range(len(t))) for s, t in zip(slots, prompts)])
+    for s in slots:
+        m.close_sequence(s)
+    running = [m.open_sequence() for _ in range(going)]
+    m.step([(s, U.tokens(4 + i, cfg["vocab"], 20 + i), []) for i, s in enumerate(running)])
+    entries = [(m.open_sequence(), t, range(len(t))) for t in prompts] + [(s, [i], [0]) for i, s in enumerate(running)]
+    assert torch.equal(m.step(entries)[: sum(lens)], alone)
+
+
 @pytest.mark.parametrize("lens", [[1100], [517, 3, 580]], ids=str)
 def test_state_space_prompts_that_fill_the_chip(lens):
     """Rows and columns enough for the convolution's 16 rows per thread (8224 columns), and a token behind each prompt, whose window is what
