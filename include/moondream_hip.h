@@ -803,7 +803,8 @@ typedef struct {
   const int32_t* seq_ctx0;         /* device [n_seq + 1]: running sums of the same; not read when max_len == 1 */
 } md_lm_batch;
 
-/* Workspace of a step: reads the counts of b (n_seq, n_rows, max_len, n_going, max_ctx, ctx_rows), not its pointers. */
+/* Workspace of a step: reads the counts of b (n_seq, n_rows, max_len, max_ctx, ctx_rows), not its pointers.  The workspace of the
+ * longest prompts (max_len > 1) serves shorter ones of as many sequences. */
 size_t md_lm_workspace_bytes(const md_lm_model* m, const md_lm_batch* b, int32_t n_logits);
 
 /* One step: embedding, every layer, state update.  logit_rows (device int32 [n_logits], indices of rows of the step; NULL: rows

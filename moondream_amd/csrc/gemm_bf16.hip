@@ -1073,6 +1073,14 @@ int md_gemm_partial_count(const md_linear& lin, int rows) {
   const int tiles = (rows + 127) / 128 * ((lin.n + 127) / 128);
   return tiles > 128 || lin.k_pad < 1024 ? 0 : std::min(256 / tiles, std::min(8, lin.k_pad / BK / 4));
 }
+size_t md_gemm_partial_most(const md_linear& lin, int rows) {
+  size_t most = (size_t)md_gemm_partial_slices(&lin) * std::min(rows, 128) * lin.n_pad;
+  for (int m = 256, n = 1; m < rows + 128 && n > 0; m += 128) {  // (the count falls from row tile to row tile)
+    n = md_gemm_partial_count(lin, m);
+    most = std::max(most, (size_t)n * std::min(rows, m) * lin.n_pad);
+  }
+  return most;
+}
 md_status md_gemm_partial_rows(const void* a, int64_t lda, const md_linear& lin, int m, int slices, float* partial, int64_t ld_partial,
                                int64_t slice_stride, hipStream_t s) {
   GemmK k;
@@ -1176,6 +1184,12 @@ md_status md_gemm_silu_bf16(const void* a, int64_t lda, const md_linear& lin, vo
 int md_gemm_grouped_slices(const md_linear& lin, int groups, int slots) {
   const int tiles = lin.n_pad / 64 * std::min(groups, slots), nk = lin.k_pad / BK;
   return std::max(1, std::min(512 / std::max(1, tiles), std::min(8, nk)));
+}
+// up to `groups` slots a tile each: at most 8 slices, or what 512 tiles of 64 columns hold; from there on the count stays
+size_t md_gemm_grouped_most(const md_linear& lin, int groups, int slots) {
+  const size_t few = std::min(groups, slots), held = 512 * 64;
+  const size_t most = std::min(8 * few * lin.n_pad, std::max(few * lin.n_pad, held));
+  return slots <= groups ? most : std::max(most, (size_t)md_gemm_grouped_slices(lin, groups, slots) * slots * lin.n_pad);
 }
 md_status md_gemm_grouped_partial(const void* a, int64_t lda, const int32_t* row_of, const md_linear& lin, int groups, const int32_t* offsets, float* partial,
                                   int64_t ld, int64_t slice_stride, int slots, hipStream_t stream) {

@@ -91,10 +91,12 @@ md_status md_gemm_grouped_bf16(const void* a, int64_t lda, const int32_t* row_of
 md_status md_gemm_silu_bf16(const void* a, int64_t lda, const md_linear& lin, void* c, int64_t ldc, int rows, hipStream_t stream);
 // the same as fp32 K-slice partial products [slice][slot][ld] (few rows per group)
 int md_gemm_grouped_slices(const md_linear& lin, int groups, int slots);
+size_t md_gemm_grouped_most(const md_linear& lin, int groups, int slots);  // floats that those of up to that many slots take at most
 md_status md_gemm_grouped_partial(const void* a, int64_t lda, const int32_t* row_of, const md_linear& lin, int groups, const int32_t* offsets, float* partial,
                                   int64_t ld, int64_t slice_stride, int slots, hipStream_t stream);
 // K-slice partial products of any number of rows: how many slices pay (0: a whole product is faster), and the launch
 int md_gemm_partial_count(const md_linear& lin, int rows);
+size_t md_gemm_partial_most(const md_linear& lin, int rows);  // floats that the partial products of up to that many rows take at most
 md_status md_gemm_partial_rows(const void* a, int64_t lda, const md_linear& lin, int rows, int slices, float* partial, int64_t ld_partial,
                                int64_t slice_stride, hipStream_t stream);
 constexpr int MD_EPI_QKV_ROPE = 3;     // internal to the library (md_gemm_qkv_rope)

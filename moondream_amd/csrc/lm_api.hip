@@ -58,17 +58,21 @@ inline bool own_row_steps(const md_lm_model* m) { return m->streams > 0 || m->po
 inline int n_streams(const md_lm_model* m) { return m->streams > 0 ? m->streams : 1; }
 inline int conv_columns(const md_lm_layer& l) { return l.heads * l.vdim_pad + 2 * l.groups * l.dim_pad; }
 
+// What splits its sums wants more memory at fewer rows: there is room for what any smaller step of the same kind (one token per sequence, or
+// prompts) would want, so that a workspace of the largest step serves all.
 LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base) {
   const int rows = b->n_rows, n_seq = b->n_seq, max_len = b->max_len, max_ctx = b->max_ctx;
   const size_t es = esize(m), M = rows;
   size_t in = 0, q = 0, att = 0, gu = 0, act = 0, qf = 0, of = 0, cs = 0, ap = 0, sk = 0, part = 0, y = M * m->width_pad;
   size_t c_rows = 0, kv = 0, q_lat = 0, lp = 0, conv = 0, dt = 0, seg = 0, segs = 0, slots = 0, experts = 0;
-  const bool dec = decode_regime(m, rows);
+  size_t sk_room = 0;
   auto splitk = [&](const md_linear& l, int n) {
-    if (m->dtype == MD_DTYPE_BF16 && l.w && n > 0) sk = std::max(sk, md_gemm_workspace_bytes(&l, n, 1));
+    if (m->dtype != MD_DTYPE_BF16 || !l.w || n <= 0) return;
+    sk = std::max(sk, md_gemm_workspace_bytes(&l, n, 1));
+    sk_room = std::max(sk_room, md_gemm_workspace_bytes(&l, std::min(n, DECODE_ROWS), 1));
   };
   auto partial = [&](const md_linear& l, bool residual) {
-    if (m->dtype == MD_DTYPE_BF16 && l.w && (dec || residual)) part = std::max(part, (size_t)md_gemm_partial_count(l, rows) * M * l.n_pad);
+    if (m->dtype == MD_DTYPE_BF16 && l.w) part = std::max(part, md_gemm_partial_most(l, residual ? rows : std::min(rows, DECODE_ROWS)));
   };
   for (int i = 0; i < m->n_layers; ++i) {
     const md_lm_layer& l = m->layers[i];
@@ -83,9 +87,9 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
       if (m->dtype == MD_DTYPE_F32) gu = std::max(gu, T * l.gate_up.n_pad);
       act = std::max(act, T * l.down.k_pad);
       y = std::max(y, T * m->width_pad);
-      if (dec)
-        part = std::max(part, std::max((size_t)md_gemm_grouped_slices(l.gate_up, l.experts, (int)T) * T * l.gate_up.n_pad,
-                                       (size_t)md_gemm_grouped_slices(l.down, l.experts, (int)T) * T * l.down.n_pad));
+      const int most = std::min(rows, DECODE_ROWS) * l.top;
+      if (m->dtype == MD_DTYPE_BF16)
+        part = std::max(part, std::max(md_gemm_grouped_most(l.gate_up, l.experts, most), md_gemm_grouped_most(l.down, l.experts, most)));
     } else if (l.ff > 0) {
       if (m->dtype == MD_DTYPE_F32) gu = std::max(gu, M * l.gate_up.n_pad);
       act = std::max(act, M * l.down.k_pad);
@@ -114,11 +118,10 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
     } else if (l.mixer == MD_MIXER_STATE_SPACE) {
       conv = std::max(conv, M * conv_columns(l));
       dt = std::max(dt, M * l.heads);
-      int chunks;
-      const size_t ns = lm_ssm_segments(n_seq, l.heads, max_len, &chunks);
-      if (m->dtype == MD_DTYPE_BF16 && ns > 1) {
-        segs = std::max(segs, n_seq * ns * l.heads);
-        seg = std::max(seg, n_seq * ns * l.heads * l.dim_pad * l.vdim_pad);
+      if (m->dtype == MD_DTYPE_BF16) {
+        const size_t ns = lm_ssm_most_segments(n_seq, l.heads, max_len);
+        segs = std::max(segs, ns * l.heads);
+        seg = std::max(seg, ns * l.heads * l.dim_pad * l.vdim_pad);
       }
     } else {
       qf = std::max(qf, (size_t)l.heads * l.dim_pad);
@@ -139,7 +142,7 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
   w.act = (char*)a.take(act * es);
   w.part = (float*)a.take(part * 4);
   w.part_floats = (int64_t)part;
-  w.splitk = a.take(sk);
+  w.splitk = a.take(sk_room);
   w.splitk_bytes = sk;
   w.attn_part = (float*)a.take(ap * 4);
   // the plain retention kernels' rotated rows and the matrix-core kernels' chunk states are never live together
@@ -162,7 +165,7 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
   w.slot_of = (int32_t*)a.take(slots * 4);
   w.row_of = (int32_t*)a.take(slots * 4);
   w.offsets = (int32_t*)a.take(slots ? (experts + 1) * 4 : 0);
-  w.sumsq = (float*)a.take(step_regime(m, b) ? M * (m->width_pad / 8) * 4 : 0);
+  w.sumsq = (float*)a.take(m->dtype == MD_DTYPE_BF16 ? (size_t)std::min(rows, LM_STEP_ROWS) * (m->width_pad / 8) * 4 : 0);
   w.total = a.off;
   return w;
 }

@@ -255,6 +255,7 @@ md_status lm_ssm_plain(int dtype, const LmSsm& a, hipStream_t s);
 bool lm_ssm_mfma_takes(const LmSsm& a);
 constexpr int LM_SSM_CHUNK = 64;
 int lm_ssm_segments(int n_seq, int heads, int max_len, int* chunks);     // segments per sequence that fill the chip, chunks of each
+int lm_ssm_most_segments(int n_seq, int heads, int max_len);  // segments that need memory, of all sequences, of steps up to that length
 md_status lm_ssm_mfma(const LmSsm& a, hipStream_t s);                    // bf16 prefill, chunked on the matrix cores
 bool lm_ssm_decode_takes(const LmSsm& a);
 md_status lm_ssm_decode(const LmSsm& a, hipStream_t s);                  // bf16 decode step

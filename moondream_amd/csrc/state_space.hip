@@ -650,6 +650,10 @@ int lm_ssm_segments(int n_seq, int heads, int max_len, int* chunks) {
   *chunks = 3 * per + 4 < 2 * n ? per : n;
   return (n + *chunks - 1) / *chunks;
 }
+int lm_ssm_most_segments(int n_seq, int heads, int max_len) {
+  const int64_t n = (max_len + L - 1) / L;
+  return n > 1 ? (int)std::min(n_seq * n, (int64_t)(512 / heads)) : 0;
+}
 bool lm_ssm_mfma_takes(const LmSsm& a) { return chunk_pick(a).run != nullptr; }
 md_status lm_ssm_mfma(const LmSsm& a, hipStream_t s) {
   const ChunkPick k = chunk_pick(a);

@@ -132,7 +132,24 @@ def test_steps_say_how_many_sequences_go_on():
     assert _lib.MdLmBatch.n_going.offset == 12 and _lib.MdLmBatch.tokens.offset == 16 and ctypes.sizeof(_lib.MdLmBatch) == 80
     lib, (cfg, w, p) = _lib.load(), _packed("retention", torch.bfloat16)
     size = lambda going: lib.md_lm_workspace_bytes(ctypes.byref(p.model), ctypes.byref(_lib.MdLmBatch(3, 9, 4, going, max_ctx=64, ctx_rows=40)), 3)  # noqa: E731
-    assert size(0) == size(2) < size(3)  # (the rows' sums of squares)
+    assert size(0) == size(2) == size(3) > 0
+
+
+@pytest.mark.parametrize("mixers", [[0, 1], [2, 3], [2]], ids=["attention_retention", "latent_state_space", "latent"])
+@pytest.mark.parametrize("experts", [0, 32])
+def test_a_workspace_of_the_largest_prompt_serves_all(mixers, experts):
+    lib, linear = _lib.load(), lambda n, k: _lib.MdLinear(4096, None, n, k, n, k)  # (sizes only: nothing is read through the pointers)
+    layers = (_lib.MdLmLayer * len(mixers))()
+    for i, (l, mixer) in enumerate(zip(layers, mixers)):
+        l.mixer, l.heads, l.kv_heads, l.kv_layer, l.taps, l.groups, l.norm_groups, l.rank, l.rank_pad = mixer, 32, 32, i, 4, 1, 1, 256, 256
+        l.dim = l.dim_pad = l.vdim = l.vdim_pad = 64
+        l.in_proj, l.out_proj, l.up_kv = linear(8192, 2048), linear(2048, 2048), linear(4096, 256)
+        l.ff, l.ff_pad, l.gate_up, l.down, l.experts, l.top = 5440, 5440, linear(10880, 2048), linear(2048, 5440), experts, 4 if experts else 0
+    m = _lib.MdLmModel(dtype=0, width=2048, width_pad=2048, vocab=51200, n_layers=len(mixers), layers=layers, head=linear(51200, 2048))
+    for n_seq in (1, 8):
+        batch = lambda n: _lib.MdLmBatch(n_seq, n * n_seq, n, 0, max_ctx=n, ctx_rows=n * n_seq)  # noqa: E731
+        sizes = [lib.md_lm_workspace_bytes(ctypes.byref(m), ctypes.byref(batch(n)), 1) for n in range(2, 2100)]
+        assert sizes == sorted(sizes) and sizes[0] > 0
 
 
 def test_language_model_symbols_are_declared():
