@@ -230,7 +230,10 @@ md_status rows(const LmStepGemm& a, int n, hipStream_t s) {
 }
 
 static_assert(LM_STEP_ROWS <= 32, "two row tiles");
-inline bool takes(const LmStepGemm& a) { return a.rows >= 1 && a.rows <= LM_STEP_ROWS && a.k >= 64 && a.k % 64 == 0 && a.lda % 8 == 0 && a.chunk % 8 == 0; }
+inline bool takes(const LmStepGemm& a) {
+  return a.rows >= 1 && a.rows <= LM_STEP_ROWS && a.k >= 64 && a.k % 64 == 0 && a.lda % 8 == 0 && a.chunk % 8 == 0 &&
+         (((uintptr_t)a.a | (uintptr_t)a.w | (uintptr_t)a.out) & 15) == 0;
+}
 
 }  // namespace
 

@@ -60,6 +60,21 @@ def test_rows_of_a_step(name):
     assert float(U.logit_errors(got, want[:2, 1]).max()) < 0.3
 
 
+@pytest.mark.parametrize("rows", [3, 40, 200])
+@pytest.mark.parametrize("which", ["in_proj", "out_proj", "gate_up", "down", "head"])
+def test_misaligned_weights_are_refused(rows, which):
+    """16-byte loads of the weights: at every number of rows."""
+    from moondream_amd._lib import MoondreamHipError
+
+    m = build(ONE)
+    lin = m.w.model.head if which == "head" else getattr(m.w.model.layers[0], which)
+    lin.w += 2
+    with pytest.raises(MoondreamHipError):
+        m.step([(m.open_sequence(), U.tokens(min(rows, 50), 200, i), [0]) for i in range(-(-rows // 50))])
+    lin.w -= 2
+    m.step([(m.open_sequence(), U.tokens(3, 200, 9), [0])])
+
+
 @pytest.mark.parametrize("rows", [5, 28])
 def test_residual_stream_behind_every_layer(rows):
     for cfg in (U.CONFIGS["shared"], TWO):
