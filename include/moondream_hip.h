@@ -709,7 +709,7 @@ typedef struct {
  *   S <- exp(-decay[h] dt) S + dt B x^T,  y = S^T C + skip[h] x  (fp32);  y * silu(z), RMS norm over each of norm_groups equal parts
  *   of the heads' concatenated outputs, times out_norm (fp32 [heads * vdim_pad]).
  * out_proj: columns in [heads][vdim_pad] order.  ff == 0: no feed-forward; else gate_up = [gate | up], ff_pad rows each.
- * experts > 0: gate_up and down describe ONE expert, the matrices of all follow one another; router logits (fp32) =
+ * experts > 0: gate_up and down describe ONE expert, the matrices of all follow one another (no biases); router logits (fp32) =
  *   router h + router_bias (fp32 [experts]); the `top` largest are chosen (ties: the lower index) and weighted by their softmax.
  * mix1 / mix2 (models with streams; around the mixer / the feed-forward): fp32 [in: S | out: S | mix: S x S, from x to]. */
 typedef struct {

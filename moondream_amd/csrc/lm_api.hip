@@ -46,11 +46,14 @@ constexpr int STEP_PLAIN_ROWS = 8;
 // products that go on with the row-wise step behind them (gemm_step.hip)
 // (a router needs whole normed rows, which leaves nothing to go on with; and the first token's retention is its value times q . k, normed: only
 // the sign of q . k is left, so a rounding of the norm at another place turns it over where q . k is small.  A step in which any sequence may
-// begin keeps the rounding of long prompts where a layer has retention: 12 tokens 1.78 ms, 1.29 this way.)
+// begin keeps the rounding of long prompts where a layer has retention: 12 tokens 1.78 ms, 1.29 this way.  Their sums and gates take no bias.)
 inline bool step_regime(const md_lm_model* m, const md_lm_batch* b) {
   if (m->dtype != MD_DTYPE_BF16 || b->n_rows > LM_STEP_ROWS) return false;
-  for (int i = 0; i < m->n_layers; ++i)
-    if (m->layers[i].experts > 0 || (b->n_going != b->n_seq && m->layers[i].mixer == MD_MIXER_RETENTION)) return false;
+  for (int i = 0; i < m->n_layers; ++i) {
+    const md_lm_layer& l = m->layers[i];
+    if (l.experts > 0 || l.out_proj.b || (l.ff > 0 && (l.gate_up.b || l.down.b))) return false;
+    if (b->n_going != b->n_seq && l.mixer == MD_MIXER_RETENTION) return false;
+  }
   return true;
 }
 
@@ -91,7 +94,7 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
       if (m->dtype == MD_DTYPE_BF16)
         part = std::max(part, std::max(md_gemm_grouped_most(l.gate_up, l.experts, most), md_gemm_grouped_most(l.down, l.experts, most)));
     } else if (l.ff > 0) {
-      if (m->dtype == MD_DTYPE_F32) gu = std::max(gu, M * l.gate_up.n_pad);
+      if (m->dtype == MD_DTYPE_F32 || l.gate_up.b) gu = std::max(gu, M * l.gate_up.n_pad);
       act = std::max(act, M * l.down.k_pad);
       partial(l.gate_up, false);
       partial(l.down, true);
@@ -301,7 +304,7 @@ struct Step {
   md_status to_residual(const void* a, int64_t lda, const md_linear& lin) {
     add = {};
     add.ld = m->width_pad;
-    const int sl = m->dtype == MD_DTYPE_BF16 ? md_gemm_partial_count(lin, b->n_rows) : 0;
+    const int sl = m->dtype == MD_DTYPE_BF16 && !lin.b ? md_gemm_partial_count(lin, b->n_rows) : 0;  // (slices carry no bias)
     if (sl > 0) {
       add.slices = sl;
       add.slice_stride = (int64_t)b->n_rows * lin.n_pad;
@@ -506,16 +509,16 @@ struct Step {
       g.out = (bf16_t*)w.act;
       g.ff_pad = l.ff_pad;
       MD_TRY(lm_step_silu(g, s));
-    } else if (m->dtype == MD_DTYPE_BF16 && (!dec || md_gemm_partial_count(l.gate_up, b->n_rows) == 1)) {
+    } else if (m->dtype == MD_DTYPE_F32 || l.gate_up.b) {
+      MD_TRY(linear(w.h, m->width_pad, l.gate_up, w.gu, l.gate_up.n_pad, b->n_rows));
+      MD_TRY(lm_silu_mul(m->dtype, w.gu, l.gate_up.n_pad, w.act, l.down.k_pad, b->n_rows, l.ff_pad, s));
+    } else if (!dec || md_gemm_partial_count(l.gate_up, b->n_rows) == 1) {
       MD_TRY(md_gemm_silu_bf16(w.h, m->width_pad, l.gate_up, w.act, l.down.k_pad, b->n_rows, s));
-    } else if (dec) {
+    } else {
       const int sl = md_gemm_partial_count(l.gate_up, b->n_rows);
       const int64_t ld = l.gate_up.n_pad, stride = (int64_t)b->n_rows * ld;
       MD_TRY(md_gemm_partial_rows(w.h, m->width_pad, l.gate_up, b->n_rows, sl, w.part, ld, stride, s));
       MD_TRY(lm_reduce_silu_mul(w.part, sl, ld, stride, w.act, l.down.k_pad, b->n_rows, l.ff_pad, s));
-    } else {
-      MD_TRY(linear(w.h, m->width_pad, l.gate_up, w.gu, l.gate_up.n_pad, b->n_rows));
-      MD_TRY(lm_silu_mul_f32(w.gu, l.gate_up.n_pad, w.act, l.down.k_pad, b->n_rows, l.ff_pad, s));
     }
     return finish(w.act, l.down.k_pad, l.down, few, l.mix2, nw, next);
   }
@@ -547,7 +550,7 @@ struct Step {
     add.src = w.y;
     if (m->dtype == MD_DTYPE_F32) {
       MD_TRY(lm_grouped_gemm_f32(w.h, m->width_pad, w.row_of, l.gate_up, l.experts, w.offsets, w.gu, ld, slots, chain, s));
-      MD_TRY(lm_silu_mul_f32(w.gu, ld, w.act, l.down.k_pad, slots, l.ff_pad, s));
+      MD_TRY(lm_silu_mul(m->dtype, w.gu, ld, w.act, l.down.k_pad, slots, l.ff_pad, s));
       return lm_grouped_gemm_f32(w.act, l.down.k_pad, nullptr, l.down, l.experts, w.offsets, w.y, m->width_pad, slots, chain, s);
     }
     MD_TRY(md_gemm_grouped_bf16(w.h, m->width_pad, w.row_of, l.gate_up, l.experts, w.offsets, w.act, l.down.k_pad, slots, true, true, s));

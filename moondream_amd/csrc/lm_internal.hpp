@@ -277,8 +277,8 @@ md_status lm_resid_norm(int dtype, float* x, int64_t ldx, const void* src, int64
 md_status lm_reduce_resid_norm(float* x, int64_t ldx, const float* part, int slices, int64_t ldp, int64_t slice_stride,
                                const md_rms_weight& w, float eps, int width, int width_pad, void* y, int64_t ldy, const int32_t* rows_idx,
                                bool write_x, int rows, hipStream_t s);
-// act = silu(gate) * up over [gate | up] rows
-md_status lm_silu_mul_f32(const void* gu, int64_t ldg, void* act, int64_t lda, int rows, int ff_pad, hipStream_t s);
+// act = silu(gate) * up over [gate | up] rows: fp32 products, and those with a bias
+md_status lm_silu_mul(int dtype, const void* gu, int64_t ldg, void* act, int64_t lda, int rows, int ff_pad, hipStream_t s);
 md_status lm_reduce_silu_mul(const float* part, int slices, int64_t ldp, int64_t slice_stride, void* act, int64_t lda, int rows, int ff_pad,
                              hipStream_t s);
 

@@ -83,17 +83,18 @@ md_status launch_resid(const ResidArgs& a, int rows, hipStream_t s) {
   return md_launch_status();
 }
 
-__global__ __launch_bounds__(256) void silu_mul_kernel(const float* __restrict__ gu, int64_t ldg, float* __restrict__ act, int64_t lda, int rows, int ff_pad) {
+template <typename T>
+__global__ __launch_bounds__(256) void silu_mul_kernel(const T* __restrict__ gu, int64_t ldg, T* __restrict__ act, int64_t lda, int rows, int ff_pad) {
   const int per_row = ff_pad / 4;
   const int64_t n = (int64_t)rows * per_row;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
     const int64_t row = i / per_row;
     const int c = (int)(i - row * per_row) * 4;
-    const float* g = gu + row * ldg + c;
+    const T* g = gu + row * ldg + c;
     const f32x4 z = ld4(g), u = ld4(g + ff_pad);
     f32x4 o;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = silu_f32(z[e]) * u[e];
+    for (int e = 0; e < 4; ++e) o[e] = silu_for<T>(z[e]) * u[e];
     st4(act + row * lda + c, o);
   }
 }
@@ -152,10 +153,13 @@ md_status lm_reduce_resid_norm(float* x, int64_t ldx, const float* part, int sli
   return launch_resid<bf16_t, 2>(a, rows, s);
 }
 
-md_status lm_silu_mul_f32(const void* gu, int64_t ldg, void* act, int64_t lda, int rows, int ff_pad, hipStream_t s) {
+md_status lm_silu_mul(int dtype, const void* gu, int64_t ldg, void* act, int64_t lda, int rows, int ff_pad, hipStream_t s) {
   const int64_t n = (int64_t)rows * (ff_pad / 4);
   const unsigned grid = (unsigned)((n + 255) / 256 < 8192 ? (n + 255) / 256 : 8192);
-  hipLaunchKernelGGL(silu_mul_kernel, dim3(grid), dim3(256), 0, s, (const float*)gu, ldg, (float*)act, lda, rows, ff_pad);
+  if (dtype == MD_DTYPE_F32)
+    hipLaunchKernelGGL(silu_mul_kernel<float>, dim3(grid), dim3(256), 0, s, (const float*)gu, ldg, (float*)act, lda, rows, ff_pad);
+  else
+    hipLaunchKernelGGL(silu_mul_kernel<bf16_t>, dim3(grid), dim3(256), 0, s, (const bf16_t*)gu, ldg, (bf16_t*)act, lda, rows, ff_pad);
   return md_launch_status();
 }
 

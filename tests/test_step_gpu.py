@@ -75,6 +75,29 @@ def test_misaligned_weights_are_refused(rows, which):
     m.step([(m.open_sequence(), U.tokens(3, 200, 9), [0])])
 
 
+@pytest.mark.parametrize("rows", [3, 40, 300])
+@pytest.mark.parametrize("which", ["out_proj", "gate_up", "down"])
+@pytest.mark.parametrize("cfg", [ONE, U.config([U.attention(4, 4, 32, 32, 64), U.attention(2, 2, 64, 64, 400)], width=328, vocab=200, ff=320)], ids=["streams", "plain"])
+def test_biases_count_at_every_number_of_rows(cfg, which, rows):
+    """The C structures allow a bias on every projection (the model folders have none there): bf16 beside fp32."""
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    out = {}
+    for dtype in (BF16, torch.float32):
+        m = LayeredLM(LayeredLMConfig.from_dict(cfg), U.weights(cfg, 3, 1.5), dtype=dtype, max_batch=2, max_context=320)
+        lin, ids = getattr(m.w.model.layers[0], which), U.tokens(rows, 200, rows)
+        for bias in (None, torch.linspace(-1.0, 1.0, lin.n_pad, device="cuda").to(BF16).to(dtype)):
+            if bias is not None:
+                bias[cfg["width"] if which != "gate_up" else lin.n_pad :] = 0  # (padded columns stay zero)
+                lin.b = bias.data_ptr()
+            s = m.open_sequence()
+            out[dtype, bias is not None] = m.step([(s, ids, range(rows))])
+            m.close_sequence(s)
+    moved = U.logit_error(out[torch.float32, True], out[torch.float32, False].double().cpu())
+    assert moved > 0.1 and U.logit_error(out[BF16, True], out[torch.float32, True].double().cpu()) < 0.25 * moved
+
+
 @pytest.mark.parametrize("rows", [5, 28])
 def test_residual_stream_behind_every_layer(rows):
     for cfg in (U.CONFIGS["shared"], TWO):
