@@ -1133,10 +1133,10 @@ namespace {
 // per_group: the expected rows of a group.  The four-wave tile from 64 on: it moves the fewest bytes per product, which bounds all of them,
 // though most of its rows are padding at first (a whole prefill through 32 experts of 2 x 1360 columns, 24 layers: 87 rows a group 8.29 -> 7.78 ms
 // against the 64 x 64 tile, 212 rows 11.8 -> 10.8 against 128 x 128, 612 rows 24.4 -> 21.5 and 1000 rows 35.3 -> 30.9 against an eight-wave
-// 256 x 256 tile; 50 rows: 7.15 either way).
+// 256 x 256 tile; 50 rows: 7.15 either way).  Not for gates that stay in fp32 (k.round_first unset): its epilogue rounds them.
 template <int EPI>
 md_status grouped_by_height(GemmK k, int per_group, hipStream_t stream) {
-  if (per_group >= 64 && k.n_pad >= 256 && md_gemm_w4_takes(k, EPI) && (uint64_t)k.groups * k.n_pad * k.ldw * 2 < (1ull << 32)) {
+  if (per_group >= 64 && k.n_pad >= 256 && (EPI != MD_EPI_SILU || k.round_first) && md_gemm_w4_takes(k, EPI) && (uint64_t)k.groups * k.n_pad * k.ldw * 2 < (1ull << 32)) {
     k.group_m = 4;
     return md_gemm_w4_launch_grouped(k, EPI, stream);
   }

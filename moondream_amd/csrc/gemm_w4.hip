@@ -599,7 +599,7 @@ __global__ __launch_bounds__(256) void gemm_w4_kernel(const GemmK p) {
       });
     };
     // MD_EPI_SILU: accumulator blocks 2 j and 2 j + 1 are gates and inputs of 16 columns, so a pass of 32 rows x 64 columns is a row pair of
-    // the wave's quarter; gates and inputs are rounded to bf16 before they meet (k.round_first is always set here)
+    // the wave's quarter; gates and inputs are rounded to bf16 before they meet (only launches with k.round_first come here)
     auto silu_epilogue = [&]() {
       const int lane_row = lane >> 3, lane_col = (lane & 7) * 8;
       const int c0 = (wn0 >> 1) + lane_col;
@@ -763,12 +763,13 @@ md_status md_gemm_w4_launch(const GemmK& k, int epi, hipStream_t stream) {
     case MD_EPI_GELU: return launch<MD_EPI_GELU>(k, stream);
     case MD_EPI_RESIDUAL: return launch<MD_EPI_RESIDUAL>(k, stream);
     case MD_EPI_QKV_ROPE: return launch<MD_EPI_QKV_ROPE>(k, stream);
-    case MD_EPI_SILU: return launch<MD_EPI_SILU>(k, stream);
+    case MD_EPI_SILU: return k.round_first ? launch<MD_EPI_SILU>(k, stream) : MD_ERR_UNSUPPORTED;
     default: return MD_ERR_INVALID_ARG;
   }
 }
 
 md_status md_gemm_w4_launch_grouped(const GemmK& k, int epi, hipStream_t stream) {
+  if (epi == MD_EPI_SILU && !k.round_first) return MD_ERR_UNSUPPORTED;
   if (k.K % 64 != 0 || k.M <= 0 || !k.offsets || k.groups <= 0 || k.bias) return MD_ERR_INVALID_ARG;
   // 32-bit byte offsets over all groups' matrices
   if (!md_gemm_w4_takes(k, epi) || (uint64_t)k.groups * (uint64_t)k.n_pad * (uint64_t)k.ldw * 2 >= (1ull << 32)) return MD_ERR_UNSUPPORTED;

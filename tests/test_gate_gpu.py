@@ -37,3 +37,16 @@ def test_experts(rows, experts, top, ff):
     e = U.logit_errors(got, want).sort().values
     # a router between nearly equal logits may choose another expert at single rows
     assert float(e[int(0.9 * (len(e) - 1))]) < 3e-2 and float(e.median()) < 1e-2
+
+
+def test_a_step_rounds_its_gates_alike_on_every_tile():
+    """Up to 128 rows gates stay in fp32 until they are multiplied; 64 rows per expert and one K slice (128 rows, 8 experts, 4 of them, 2752
+    columns) reach for another tile than 50 rows per expert do."""
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    cfg = U.stream_config([(mixer(), U.moe(8, 4, 1376))] * 2, width=320, vocab=120, streams=1, positions=64)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), U.weights(cfg, 3, 1.5), dtype=torch.bfloat16, max_batch=8, max_context=64)
+    ts = [U.tokens(n, cfg["vocab"], n) for n in (50, 49, 29)]
+    few, many = (m.step([(m.open_sequence(), t, range(len(t))) for t in part]) for part in (ts[:2], ts))
+    assert torch.equal(few, many[:99])
