@@ -769,24 +769,25 @@ class MoondreamModel(DeviceEngine):
 
     # PINNED staging for the uint8 crops (a pageable source makes the runtime bounce the copy through its own small pinned
     # buffers, synchronously: ~2x the time, and the host cannot queue the ViT launches behind it).  A small set of buffers
-    # rotates; a buffer is handed out again only after the copy that read it has completed (its event).
+    # rotates; a buffer is handed out again only after the copy that read it has completed (its event).  Sizes are powers of two and a
+    # larger buffer takes the place of a free smaller one, so that pictures of any sizes settle on as many buffers as are in use at once.
     def _pinned_crops(self, n_crops: int, crop_shape):
         shape = (int(n_crops),) + tuple(crop_shape)
         nbytes = int(np.prod(shape))
         ring = getattr(self, "_pinned", None)
         if ring is None:
             ring = self._pinned = {"bufs": [], "events": [], "busy": []}
-        pick = None
-        for i, (buf, busy) in enumerate(zip(ring["bufs"], ring["busy"])):
-            if not busy and buf.numel() >= nbytes:
-                pick = i
-                break
-        if pick is None:
+        free = [i for i, busy in enumerate(ring["busy"]) if not busy]
+        fits = [i for i in free if ring["bufs"][i].numel() >= nbytes]
+        if fits:
+            pick = min(fits, key=lambda i: ring["bufs"][i].numel())
+        else:
             with torch.inference_mode(False):
-                ring["bufs"].append(torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, pin_memory=True))
-            ring["events"].append(None)
-            ring["busy"].append(False)
-            pick = len(ring["bufs"]) - 1
+                buf = torch.empty(max(1 << (nbytes - 1).bit_length(), 1 << 20), dtype=torch.uint8, pin_memory=True)
+            done = [i for i in free if ring["events"][i] is None or ring["events"][i].query()]
+            pick = max(done, key=lambda i: ring["bufs"][i].numel()) if done else len(ring["bufs"])
+            for name, value in (("bufs", buf), ("events", None), ("busy", False)):
+                ring[name][pick : pick + 1] = [value]
         if ring["events"][pick] is not None:
             ring["events"][pick].synchronize()
             ring["events"][pick] = None

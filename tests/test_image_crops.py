@@ -178,3 +178,31 @@ def test_crop_count_and_out_buffer_match_the_allocating_form():
         out = np.full((n, 378, 378, 3), 7, dtype=np.uint8)
         got = overlap_crop_image(img, overlap_margin=4, max_crops=12, out=out)
         assert got["crops"] is out and np.array_equal(out, ref["crops"])
+
+
+class _Pinned:
+    """A MoondreamModel's staging alone, on ordinary memory."""
+
+    def __new__(cls, monkeypatch):
+        from moondream_amd.config import get_config
+        from moondream_amd.moondream import MoondreamModel
+
+        empty = torch.empty
+        monkeypatch.setattr(torch, "empty", lambda *a, pin_memory=False, **k: empty(*a, **k))
+        m = MoondreamModel.__new__(MoondreamModel)
+        m.config, m.vit_chunk_crops = get_config("tiny"), 26
+        return m
+
+
+def test_pinned_staging_settles_on_the_buffers_in_use(monkeypatch):
+    m, rng, most = _Pinned(monkeypatch), np.random.default_rng(0), 0
+    for i in range(300):  # two chunks under way at a time, of ever other sizes
+        a, b = (int(n) for n in rng.integers(1, 5_000_000, 2) + 10_000 * i)
+        most = max(most, a, b)
+        held = [m._pinned_crops(1, (n,)) for n in (a, b)]
+        assert held[0][1] != held[1][1] and [h.shape for h, _ in held] == [(1, a), (1, b)]
+        for _, token in held:
+            m._release_pinned(token)
+    sizes = [x.numel() for x in m._pinned["bufs"]]
+    assert len(sizes) == 2 and max(sizes) < 2 * most and m._pinned["busy"] == [False, False]
+
