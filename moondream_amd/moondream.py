@@ -651,25 +651,28 @@ class MoondreamModel(DeviceEngine):
             chunks.append((i0, i1, tot))
             i0 = i1
         staged, room = [], 1 << 30
-        for (c0, c1, tot) in chunks:  # all host work is queued up front; the GPU side follows chunk by chunk
-            plan = self._cut_plan(images[c0:c1], [t for _, t in counts[c0:c1]], min(room, 8 * tot * v.crop_size * v.crop_size * 3))
-            if plan is not None:
-                room -= plan.staged_bytes
-                host, token = self._pinned_crops(1, (plan.staged_bytes,))
-                _lib.check(self.lib.md_crops_plan(plan.images, plan.n, v.crop_size, plan.stride, host.ctypes.data, plan.staged_bytes), "md_crops_plan")
-                futs = []
-                for i, at in zip(range(c0, c1), plan.offsets):
-                    w, h = images[i].size
-                    futs.append(pool.submit(self._pixels_into, images[i], host[0, at : at + h * w * 3].reshape(h, w, 3), counts[i]))
-                staged.append((host, token, futs, plan))
-                continue
-            host, token = self._pinned_crops(tot, (v.crop_size, v.crop_size, 3))
-            futs, off = [], 0
-            for i in range(c0, c1):
-                n = counts[i][0]
-                futs.append(pool.submit(self._crop_into, images[i], host[off : off + n]))
-                off += n
-            staged.append((host, token, futs, None))
+        try:
+            for (c0, c1, tot) in chunks:  # all host work is queued up front; the GPU side follows chunk by chunk
+                plan = self._cut_plan(images[c0:c1], [t for _, t in counts[c0:c1]], min(room, 8 * tot * v.crop_size * v.crop_size * 3))
+                shape = (tot, v.crop_size, v.crop_size, 3) if plan is None else (1, plan.staged_bytes)
+                host, token = self._pinned_crops(shape[0], shape[1:])
+                futs: List[Any] = []
+                staged.append((host, token, futs, plan))  # (from here on whoever drains the list returns the buffer)
+                if plan is not None:
+                    room -= plan.staged_bytes
+                    _lib.check(self.lib.md_crops_plan(plan.images, plan.n, v.crop_size, plan.stride, host.ctypes.data, plan.staged_bytes), "md_crops_plan")
+                    for i, at in zip(range(c0, c1), plan.offsets):
+                        w, h = images[i].size
+                        futs.append(pool.submit(self._pixels_into, images[i], host[0, at : at + h * w * 3].reshape(h, w, 3), counts[i]))
+                    continue
+                off = 0
+                for i in range(c0, c1):
+                    n = counts[i][0]
+                    futs.append(pool.submit(self._crop_into, images[i], host[off : off + n]))
+                    off += n
+        except BaseException:
+            self._drain_staged((chunks, staged))
+            raise
         return chunks, staged
 
     def _cut_plan(self, images: Sequence[Image.Image], tilings, most: int):

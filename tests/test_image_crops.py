@@ -206,3 +206,21 @@ def test_pinned_staging_settles_on_the_buffers_in_use(monkeypatch):
     sizes = [x.numel() for x in m._pinned["bufs"]]
     assert len(sizes) == 2 and max(sizes) < 2 * most and m._pinned["busy"] == [False, False]
 
+
+def test_a_failed_plan_returns_its_buffers(monkeypatch):
+    import types
+
+    import pytest
+    from PIL import Image
+
+    from concurrent.futures import ThreadPoolExecutor
+    from moondream_amd import _lib, image_crops
+
+    monkeypatch.setattr(image_crops, "_pyvips", None)
+    m, real, calls = _Pinned(monkeypatch), _lib.load(), []
+    failing = lambda *a: calls.append(a) or (0 if len(calls) < 2 else 1)  # noqa: E731  (the second chunk's)
+    m.lib = types.SimpleNamespace(md_crops_staged_bytes=real.md_crops_staged_bytes, md_crops_plan=failing)
+    images = [Image.fromarray(np.zeros((700, 900, 3), np.uint8)) for _ in range(6)]
+    with ThreadPoolExecutor(2) as pool, pytest.raises(_lib.MoondreamHipError):
+        m._stage_crops(images, pool)
+    assert len(calls) == 2 and not any(m._pinned["busy"])
