@@ -1,5 +1,5 @@
 """fp32 products at the edges of their tiles: few rows, tiles with remainders, every count of K steps; one order of sums at every number of
-rows; prompts through retention layers, whose first tokens show any other order."""
+rows; prompts through retention layers, whose first tokens show any other order; grouped rows; scans of every state size."""
 import ctypes as C
 import os
 
@@ -8,8 +8,8 @@ import pytest
 import torch
 
 import lm_util as U
-
 from moondream_amd import _lib
+from oracle import layered_lm_oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -72,3 +72,37 @@ def test_prompts_through_retention_layers_keep_their_results(groups):
     fp32 rounding.  The results on record (made when every sum was one chain, token by token) stand, whatever else is in the step."""
     want = np.load(os.path.join(os.path.dirname(__file__), "golden", "retention_f32.npz"))["logits"]
     assert np.array_equal(retention_logits(groups).numpy(), want)
+
+
+def forward(cfg, lens, context=192):
+    """(logits of the prompts of one step and of a token behind each, the same in float64)"""
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    w = U.weights(cfg, 3)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=torch.float32, max_batch=8, max_context=context)
+    ts = [U.tokens(n + 1, cfg["vocab"], i) for i, n in enumerate(lens)]
+    slots = [m.open_sequence() for _ in ts]
+    got = [m.step([(s, t[:-1], range(len(t) - 1)) for s, t in zip(slots, ts)]), m.step([(s, t[-1:], [0]) for s, t in zip(slots, ts)])]
+    want = [O.forward(cfg, w, t) for t in ts]
+    return torch.cat(got), torch.cat([x[:-1] for x in want] + [x[-1:] for x in want])
+
+
+@pytest.mark.parametrize("rows,experts,top", [(9, 40, 1), (64, 1, 1), (65, 1, 1), (130, 2, 1), (131, 3, 2), (150, 70, 4)])
+def test_grouped_products(rows, experts, top):
+    """Empty groups, groups of one row, of whole tiles and of a row more, gathered rows; groups that begin inside a tile's rows."""
+    got, want = forward(U.stream_config([(U.ssm(1, 8, 8), U.moe(experts, top, 200))], width=320, vocab=64, streams=1, positions=160), [rows])
+    # a sum of k products in fp32 is off by up to sqrt(k) 2^-24 of its size, through four products in a row: 1e-6 at k = 320; twenty times that
+    assert U.logit_error(got, want) < 2e-5
+
+
+@pytest.mark.parametrize("dim", [20, 64, 100, 160, 224, 256])
+def test_retention_scans(dim):
+    got, want = forward(U.config([U.retention(2, dim, 40, rot=dim // 4 * 2)], width=64, vocab=64, ff=None, eps=1e-2), [1, 16, 17, 40])
+    assert U.logit_error(got, want) < 2e-5  # (the norm's eps keeps first tokens from enlarging it)
+
+
+@pytest.mark.parametrize("state", [16, 64, 100, 140, 256, 300, 512])
+def test_state_space_scans(state):
+    got, want = forward(U.stream_config([(U.ssm(2, 24, state), None)], width=64, vocab=64, streams=1, positions=64), [1, 8, 9, 33])
+    assert U.logit_error(got, want) < 2e-5

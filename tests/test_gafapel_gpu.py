@@ -234,12 +234,14 @@ def test_graph_replays_match_the_eager_steps():
         torch.cuda.synchronize()
 
 
-def test_grouped_tiles_of_the_bf16_product_agree():
-    """One model, steps of different heights: the 64, 128 and 256 row tiles of the grouped product give the same rows within rounding."""
-    cfg, w = _expert_model(2, 2, 256, width=256)
+@pytest.mark.parametrize("width,ff", [(256, 256), (192, 64)], ids=["four_wave_tile", "128_rows"])
+def test_grouped_tiles_of_the_bf16_product_agree(width, ff):
+    """One model, steps of different heights: the large tile of the grouped product (the four-wave one for 256 columns and more, 128 rows for
+    fewer) and the 64-row one give the same rows within rounding."""
+    cfg, w = _expert_model(2, 2, ff, width=width)
     t = U.tokens(1100, 64, 3)
     cfg["max_positions"] = 1200
-    w["pos"] = torch.zeros(1200, 256, dtype=BF16)
+    w["pos"] = torch.zeros(1200, width, dtype=BF16)
     m = load(cfg, w, BF16, max_batch=1)
     a, b, c = run(m, t, [1100]).double().cpu(), run(m, t, [200] * 5 + [100]).double().cpu(), run(m, t, [60] * 18 + [20]).double().cpu()
     assert U.logit_error(b, a) < 2e-2 and U.logit_error(c, a) < 2e-2

@@ -31,14 +31,21 @@ def test_rows_of_a_step(name):
     ts = [U.tokens(2, cfg["vocab"], i) for i in range(64)]
     want = torch.stack([O.forward(cfg, w, t) for t in ts])  # [64, 2, vocab]
     scale = (want - want.mean(-1, keepdim=True)).pow(2).mean().sqrt()
-    for n in (1, 2, 8, 9, 16, 17, 28, 29, 64):
+    # bf16 rounding through the layers, as in the other tests of whole models: 7e-2 at every row.  Routers, retention of first tokens and small
+    # norm groups enlarge it at single rows, and at the same rows whatever product runs: there, twice what the products of 64 rows show
+    limit = torch.full((2, 64), 7e-2, dtype=torch.float64)
+    enlarges = isinstance(name, str)
+    for n in (64, 1, 2, 8, 9, 16, 17, 28, 29):
         slots = [m.open_sequence() for _ in range(n)]
         for k in range(2):
             got = m.step([(s, [t[k]], [0]) for s, t in zip(slots, ts)]).double().cpu()
             d = got - want[:n, k]
-            e = ((d - d.mean(-1, keepdim=True)).pow(2).mean(-1).sqrt() / scale).sort().values
-            # bf16 rounding through the layers, as in the other tests of whole models: 7e-2; routers enlarge it at single rows
-            assert float(e[int(0.9 * (n - 1))]) < 7e-2 and float(e[-1]) < 1.0, (n, k, e[-4:])
+            e = (d - d.mean(-1, keepdim=True)).pow(2).mean(-1).sqrt() / scale
+            if n == 64 and enlarges:
+                top = e.sort().values
+                assert float(top[57]) < 7e-2 and float(top[-1]) < 1.0
+                limit[k] = torch.maximum(limit[k], 2 * e)
+            assert bool((e < limit[k, :n]).all()), (n, k, e - limit[k, :n])
         for s in slots:
             m.close_sequence(s)
     # both tokens of 14 sequences at once (28 rows), logits of some of them
@@ -46,18 +53,52 @@ def test_rows_of_a_step(name):
     places = [[1] if i % 3 == 0 else [1, 0] if i % 3 == 1 else [] for i in range(14)]
     got = m.step([(s, t, p) for s, t, p in zip(slots, ts, places)])
     ref = torch.cat([want[i][p] for i, p in enumerate(places) if p])
-    e = U.logit_errors(got, ref).sort().values
-    assert float(e[int(0.9 * (len(e) - 1))]) < 7e-2 and float(e[-1]) < 1.0
+    at_most = torch.cat([limit[p, i] for i, p in enumerate(places) if p])
+    assert bool((U.logit_errors(got, ref) < at_most).all())
     # more logits than rows
     t = U.tokens(9, cfg["vocab"], 5)
     got = m.step([(m.open_sequence(), t, [8, 0, 4] * 12)])
     e = U.logit_errors(got, O.forward(cfg, w, t)[[8, 0, 4] * 12]).sort().values
-    assert float(e[len(e) // 2]) < 7e-2 and float(e[-1]) < 1.0
+    assert float(e[len(e) // 2 if enlarges else -1]) < 7e-2 and float(e[-1]) < 1.0
     # no logits at all, then the state it left
     a, b = m.open_sequence(), m.open_sequence()
     assert m.step([(a, ts[0][:1], []), (b, ts[1][:1], [])]).shape[0] == 0
     got = m.step([(a, ts[0][1:], [0]), (b, ts[1][1:], [0])])
-    assert float(U.logit_errors(got, want[:2, 1]).max()) < 0.3
+    assert bool((U.logit_errors(got, want[:2, 1]) < limit[1, :2]).all())
+
+
+@pytest.mark.parametrize("heads,dim,vdim", [(40, 64, 64), (48, 96, 32), (64, 32, 32), (17, 128, 32), (40, 128, 32)], ids=str)
+@pytest.mark.parametrize("own", [True, False])
+def test_decode_attention_of_many_columns(heads, dim, vdim, own):
+    """A step's queries, keys and values in two and four pieces per thread (more than 2048 and 4096 columns), more than 32 heads, and a layer that
+    reads another one's keys; in two portions and then token by token."""
+    layers = [U.attention(heads, heads // 2 if heads % 2 == 0 else 1, dim, vdim, 40)]
+    if not own:
+        layers.append(dict(U.attention(heads, heads // 2 if heads % 2 == 0 else 1, dim, vdim, 33, taps=1, kv_from=0)))
+    cfg = U.config(layers, width=128, vocab=120, ff=None)
+    m, w, ts = build(cfg), U.weights(cfg, 3, 1.5), [U.tokens(n, 120, n) for n in (50, 31)]
+    want = [O.forward(cfg, w, t) for t in ts]
+    slots = [m.open_sequence() for _ in ts]
+    m.step([(s, t[:-12], []) for s, t in zip(slots, ts)])
+    for k in range(12, 0, -1):
+        got = m.step([(s, [t[-k]], [0]) for s, t in zip(slots, ts)])
+        assert float(U.logit_errors(got, torch.stack([x[-k] for x in want])).max()) < 7e-2, k
+
+
+@pytest.mark.parametrize("width", [2112, 4160])
+def test_rows_of_wide_models(width):
+    """More sums of squares per row than one pass of the step products takes (widths above 2048)."""
+    cfg = U.stream_config([(U.ssm(2, 32, 32), U.dense(128)), (U.latent(2, 32, 32, 64), None)], width=width, vocab=120, streams=2, positions=8)
+    m, w = build(cfg), U.weights(cfg, 3, 1.5)
+    ts = [U.tokens(2, 120, i) for i in range(28)]
+    want = torch.stack([O.forward(cfg, w, t) for t in ts])
+    for n in (1, 9, 17, 28):
+        slots = [m.open_sequence() for _ in range(n)]
+        for k in range(2):
+            got = m.step([(s, [t[k]], [0]) for s, t in zip(slots, ts)])
+            assert float(U.logit_errors(got, want[:n, k]).max()) < 7e-2, (n, k)
+        for s in slots:
+            m.close_sequence(s)
 
 
 @pytest.mark.parametrize("rows", [3, 40, 200])
