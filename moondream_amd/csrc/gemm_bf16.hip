@@ -822,8 +822,8 @@ int pick_tile(int M, int n_store, int K, int policy) {
     if (K >= 1024 && t128 <= 128) return 16;
     // ("small_m_rule": 0 = round 2's rule, 1 = the default below, n > 1 = that many tiles instead of 512 -- A/B)
     const int rule = knobs().small_m_rule;
-    //  * of these, where 256 x 128 tiles are one round of the CUs: a workgroup's loads through its CU bound all these configs (about
-    //    50 GB/s each), and 384 rows and columns per slice are fewer than two resident tiles' 512 (510 tiles, K 2048: 39.9 -> 33.0 us)
+    //  * of these, where 256 x 128 tiles are one round of the CUs: 384 rows and columns of operands per slice instead of two resident tiles'
+    //    512 (510 tiles, K 2048: 39.9 -> 33.0 us; every config here was seen to move about 50 GB/s through a CU, which is not explained yet)
     const long t256 = (long)((M + 255) / 256) * ((n_store + 127) / 128);
     if (rule == 1 && t128 > 256 && t128 <= 512 && t256 <= 256) return 1;
     if (rule != 0 && t128 <= (rule > 1 ? rule : 512)) return 2;

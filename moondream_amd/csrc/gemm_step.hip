@@ -20,9 +20,6 @@ namespace {
 
 constexpr int EPI_ROWS = 0, EPI_SILU = 1, EPI_RESID = 2;
 
-// Units (64 of K: two products) per load batch
-constexpr int batch_units(int mt) { return mt <= 2 ? 2 : 1; }
-
 // W waves, MT 16-row tiles.  A workgroup's columns: TN = 16, the matrix operand's rows; SiLU 8 gates and the 8 inputs beside them; or
 // TN = 8, for layers of so few columns that the tiles would not fill the chip evenly (2048 columns: 256 workgroups): the operand's upper 8
 // rows then hold the other 32 of a unit's 64 of K, so that one load is still 1 KB of weights.  It is multiplied with either half of the
@@ -32,7 +29,7 @@ template <int MT, int TN, int W, int EPI, int S>
 __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
   constexpr bool SPLIT = EPI != EPI_SILU && TN == 8, DIAG = MT == 0;
   static_assert(SPLIT || !DIAG, "");
-  constexpr int M16 = DIAG ? 1 : MT, U = batch_units(M16);
+  constexpr int M16 = DIAG ? 1 : MT, U = 2;  // (U: units, 64 of K, per load batch)
   constexpr int PW = SPLIT ? 1 : 2, PA = DIAG ? 1 : 2;  // operands per unit
   constexpr int C = SPLIT && !DIAG ? 2 : 1;             // accumulators per row tile
   auto row_of = [&](int m) { return EPI != EPI_RESID && S == 2 ? a.rows_idx[m] : m; };

@@ -209,7 +209,10 @@ struct LmRoute {
 
 // A product of a step of few rows and what follows it (gemm_step.hip).  Rows that a residual epilogue wrote carry no norm factor: it
 // comes from their sums of squares (sumsq; nullptr: the rows are complete).
-constexpr int LM_STEP_ROWS = 28;  // (32 rows: 1792 us a step against 1778 of the tile products on gafapel-dense, 23 rows: 1651 against 1752)
+// Up to how many rows they are ahead: a step of 24 layers against the one of tile products and row-wise launches, 24 / 28 / 32 rows: 0.92 / 0.95 / 0.98 of
+// its time with attention and retention (1732, 1802, 1855 us with 32 heads of 64; the same with 16 of 128), 0.97 / 1.00 / 1.03 with state space and
+// latent attention (1641, 1720, 1773 us; the same with 16 of 128); 17 rows 0.88 and 0.92, one row 0.72 and 0.74.
+constexpr int LM_STEP_ROWS = 28;
 struct LmStepGemm {
   const bf16_t* a;       // row m's columns 8 c .. 8 c + 7 at m * lda + c * chunk (plain rows: chunk 8)
   int64_t lda;

@@ -152,8 +152,8 @@ md_status conv(const LmSsm& a, hipStream_t s) {
 }
 
 // grid (n_seq, heads, vp / 16): 16 columns of the state, 16 neighbouring lanes per column, each owning rows 4 l .. + 3 of every 64.  Tokens are
-// staged 8 at a time and then run without a barrier: the recurrence is a chain, what counts is what lies on it (one sequence of 300 tokens, 32
-// heads of 64 x 64, fp32: 67 us, 342 us token by token).
+// staged 16 at a time (8 for states above 256) and then run without a barrier: the recurrence is a chain, what counts is what lies on it (one
+// sequence of 300 tokens, 32 heads of 64 x 64, fp32: 67 us, 342 us token by token).
 // Q: quads of state rows per thread, dp <= 64 Q (and for Q = 2 more than 64)
 template <typename T, int Q>
 __global__ __launch_bounds__(256) void ssm_scan_kernel(const LmSsm a) {
