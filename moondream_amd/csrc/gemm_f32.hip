@@ -2,11 +2,11 @@
 //
 //   gemm_f32_kernel        64 x 64 tiles (64 x 32 up to 128 of those), eight waves, K in steps of 64 through two LDS buffers: the next step's loads
 //                          are in registers under this step's products, one barrier per step.  Bound by the matrix cores (153 TFLOP/s in a large
-//                          library product) once every CU has tiles.  380 rows, 2048 columns, K 2048 and 5440 on average: 81 us, 192 tiles; with four
-//                          waves, one buffer and K in steps of 16: 157 us.  10880 columns of K 2048: 163 us, 104 TFLOP/s (171 us).
+//                          library product) once every CU has tiles.  380 rows, 2048 columns, K 2048 and 5440 on average: 81 us, 192 tiles; with
+//                          four waves, one buffer and K in steps of 16: 157 us.  10880 columns of K 2048: 161 us, 105 TFLOP/s (171 us).
 //   gemm_f32_rows_kernel   up to 32 rows, where the weights are a memory stream: a workgroup owns 16 columns and all of K, its eight waves load (three
-//                          stages ahead), one wave per 16 rows multiplies.  8 rows: a pass of 24 layers 3.2 ms, 14.1 through tiles; 30 rows 3.8 ms.  From 33 rows
-//                          on the tiles are ahead (64 rows: 5.6 ms).
+//                          stages ahead), one wave per 16 rows multiplies.  8 rows: a pass of 24 layers 3.2 ms, 14.1 through four-wave tiles; 30
+//                          rows: 3.8 ms.  64 rows through the tiles above: 5.6 ms.
 //   An element's sum has the same order in both, so a row's result does not depend on the rows beside it.  The order is the caller's:
 //     slabs: at most SLAB of K in one chain, the slabs added up.  A third of the rounding error of one chain (a pass of 24 layers against 64
 //            bits: 1.5e-6 -> 0.43e-6).
