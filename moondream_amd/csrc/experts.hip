@@ -3,7 +3,7 @@
 //   route_row_kernel    one workgroup per row: logits on the vector ALUs (any dtype), choice and weights; a decode step, fp32 models
 //   route_tile_kernel   sixteen rows per workgroup: logits on the matrix cores (bf16 operands, fp32 sums), choice and weights
 //   group_kernel        one workgroup per expert: its slots in row order, deterministic, no atomics
-// The products over the slots are gemm_bf16.hip's and gemm_f32.hip's.
+// The products over the slots are gemm_bf16.hip's and gemm_f32.hip's; those of few rows per expert are gemm_experts.hip's and need no group_kernel.
 //
 // Logits, softmax and weights are fp32.  A slot is one (row, chosen expert) pair; slots are numbered expert by expert.
 #include "gemm_internal.hpp"
@@ -206,6 +206,7 @@ md_status lm_route(int dtype, const LmRoute& a, hipStream_t s) {
     hipLaunchKernelGGL(fn, dim3((a.rows + 15) / 16), dim3(256), 0, s, a);
   }
   MD_TRY(md_launch_status());
+  if (!a.offsets) return MD_OK;
   hipLaunchKernelGGL(group_kernel, dim3(a.experts), dim3(1024), 0, s, a);
   return md_launch_status();
 }

@@ -8,7 +8,8 @@
 //   behind it sums: out / down -> residual add + norm; up to 128 rows also gate_up -> silu(gate) * up (otherwise the product's epilogue).
 // Few rows (LM_STEP_ROWS, bf16):  gemm_step.hip's products, which go on with the row-wise step themselves.
 // Experts:  router + choice | rows grouped by expert | grouped gate/up product with silu(gate) * up | grouped down product; the weighted sum
-//   of a row's experts is taken by the row-wise step that follows, as the sums of K-slice partials are.
+//   of a row's experts is taken by the row-wise step that follows, as the sums of K-slice partials are.  Few rows per expert: gemm_experts.hip's
+//   products, which take the choices as they are.
 // Residual streams:  the row-wise step between two sublayers mixes them (streams.hip); x is then [streams][rows][width_pad].
 #include "gemm_internal.hpp"
 #include "lm_internal.hpp"
@@ -525,14 +526,26 @@ struct Step {
 
   md_status expert_forward(const md_lm_layer& l) {
     const int rows = b->n_rows, slots = rows * l.top;
-    const LmRoute r = {w.h, rows, m->width_pad, l.experts, l.top, l.router.w, l.router_bias, w.chosen, w.route_weight, w.offsets, w.row_of, w.slot_of};
+    const bool step = dec && lm_expert_step_takes(rows, l.top, l.experts);
+    LmRoute r = {w.h, rows, m->width_pad, l.experts, l.top, l.router.w, l.router_bias, w.chosen, w.route_weight, w.offsets, w.row_of, w.slot_of};
+    if (step) r.offsets = r.row_of = r.slot_of = nullptr;
     MD_TRY(lm_route(m->dtype, r, s));
     const int64_t ld = l.gate_up.n_pad;
     add = {};
     add.ld = m->width_pad;
     add.top = l.top;
-    add.slot_of = w.slot_of;
+    add.slot_of = r.slot_of;
     add.weight = w.route_weight;
+    if (step) {
+      add.src = w.part;
+      add.slices = 1;
+      LmExpertGemm g = {(const bf16_t*)w.h, m->width_pad, rows, l.top, (const bf16_t*)l.gate_up.w, ld * l.gate_up.k_pad, l.gate_up.k_pad, l.experts,
+                        w.chosen, slots, l.ff_pad, w.act, l.down.k_pad};
+      MD_TRY(lm_expert_silu(g, s));
+      g = {(const bf16_t*)w.act, l.down.k_pad, slots, 1, (const bf16_t*)l.down.w, (int64_t)l.down.n_pad * l.down.k_pad, l.down.k_pad, l.experts,
+           w.chosen, slots, 0, w.part, m->width_pad};
+      return lm_expert_rows(g, l.down.n_pad, s);
+    }
     if (dec) {
       const int64_t stride = slots * ld;
       const int sl = md_gemm_grouped_slices(l.gate_up, l.experts, slots);

@@ -176,7 +176,7 @@ struct LmAddend {
   const void* src;       // nullptr: nothing pending
   int64_t ld, slice_stride;
   int slices, top;
-  const int32_t* slot_of;  // [rows][top]
+  const int32_t* slot_of;  // [rows][top]; nullptr: src is in the order of the choices
   const float* weight;     // [rows][top]
 };
 
@@ -204,7 +204,7 @@ struct LmRoute {
   int32_t* chosen;       // [rows][top]
   float* weight;         // [rows][top]
   // rows sorted by expert: slots offsets[e] .. offsets[e + 1] - 1 belong to expert e
-  int32_t *offsets, *row_of, *slot_of;  // [experts + 1], [rows * top], [rows][top]
+  int32_t *offsets, *row_of, *slot_of;  // [experts + 1], [rows * top], [rows][top]; nullptr: not wanted
 };
 
 // A product of a step of few rows and what follows it (gemm_step.hip).  Rows that a residual epilogue wrote carry no norm factor: it
@@ -240,6 +240,25 @@ struct LmStepGemm {
 md_status lm_step_rows(const LmStepGemm& a, int n, hipStream_t s);   // out = a w^T + bias
 md_status lm_step_silu(const LmStepGemm& a, hipStream_t s);          // out = silu(gate) * input
 md_status lm_step_resid(const LmStepGemm& a, hipStream_t s);         // streams += a w^T; out and sumsq_out for the next product
+
+// A product of the rows of a step with the matrices of the experts that they chose (gemm_experts.hip): choice i = k-th expert of row i / top
+constexpr int LM_EXPERT_CHOICES = 1024;
+struct LmExpertGemm {
+  const bf16_t* a;       // choice i reads row i / per
+  int64_t lda;
+  int a_rows, per;
+  const bf16_t* w;       // [expert][.][k]
+  int64_t expert_stride;
+  int k, experts;
+  const int32_t* chosen;  // [n]
+  int n;                 // choices
+  int ff_pad;            // SiLU gate: rows 0 .. of a matrix are the gates, ff_pad .. the inputs
+  void* out;             // [n][ldo], in the order of the choices
+  int64_t ldo;
+};
+bool lm_expert_step_takes(int rows, int top, int experts);
+md_status lm_expert_silu(const LmExpertGemm& a, hipStream_t s);          // out (bf16) = silu(gate) * input
+md_status lm_expert_rows(const LmExpertGemm& a, int n, hipStream_t s);   // out (fp32) = a w^T, n columns
 
 // dtype: MD_DTYPE_*
 md_status lm_embed_streams(const md_lm_model* m, const int32_t* tokens, const int32_t* row_pos, float* x, int64_t stride, int rows, hipStream_t s);

@@ -71,8 +71,14 @@ template <typename T>
 __device__ __forceinline__ f32x4 addend(const LmAddend& a, int row, int c) {
   if (a.top == 0) return a.slices == 0 ? ld4((const T*)a.src + (int64_t)row * a.ld + c) : slice_sum((const float*)a.src + (int64_t)row * a.ld + c, a.slices, a.slice_stride);
   f32x4 y = {0.f, 0.f, 0.f, 0.f};
-  const int32_t* slot = a.slot_of + (int64_t)row * a.top;
   const float* w = a.weight + (int64_t)row * a.top;
+  if (!a.slot_of) {
+    const float* src = (const float*)a.src + (int64_t)row * a.top * a.ld + c;
+#pragma unroll 4
+    for (int k = 0; k < a.top; ++k) y += w[k] * *(const f32x4*)(src + k * a.ld);
+    return y;
+  }
+  const int32_t* slot = a.slot_of + (int64_t)row * a.top;
   if (a.slices == 0) {
 #pragma unroll 4
     for (int k = 0; k < a.top; ++k) y += w[k] * ld4((const T*)a.src + (int64_t)slot[k] * a.ld + c);

@@ -50,3 +50,25 @@ def test_a_step_rounds_its_gates_alike_on_every_tile():
     ts = [U.tokens(n, cfg["vocab"], n) for n in (50, 49, 29)]
     few, many = (m.step([(m.open_sequence(), t, range(len(t))) for t in part]) for part in (ts[:2], ts))
     assert torch.equal(few, many[:99])
+
+
+@pytest.mark.parametrize("rows,experts,top,ff", [(1, 5, 2, 40), (3, 40, 7, 100), (8, 5, 3, 330), (9, 9, 1, 64), (16, 4, 2, 200), (17, 8, 4, 130), (40, 9, 2, 70),
+                                                 (41, 16, 4, 70), (128, 110, 8, 30), (120, 110, 9, 30)], ids=str)
+@pytest.mark.parametrize("alike", [False, True], ids=["spread", "one_choice"])
+def test_experts_of_a_step(rows, experts, top, ff, alike):
+    """Single tokens through the experts: a workgroup per choice and per expert, up to 8 and more than 16 choices of one expert, K of one unit, the most
+    choices that go by themselves and the first that are sorted."""
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    cfg = U.stream_config([(mixer(), U.moe(experts, top, ff))], width=320, vocab=120, streams=2, positions=64)
+    w = U.weights(cfg, 3, 1.5)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=torch.bfloat16, max_batch=128, max_context=64)
+    ts = [U.tokens(1, cfg["vocab"], 0 if alike else i) for i in range(rows)]
+    got = m.step([(m.open_sequence(), t, [0]) for t in ts])
+    want = torch.cat([O.forward(cfg, w, t) for t in ts[: 1 if alike else rows]]).expand(rows, -1)
+    e = U.logit_errors(got, want).sort().values
+    # (as in test_experts; a row alone is held to what its choice leaves)
+    assert float(e[int(0.9 * (len(e) - 1))]) < 3e-2 and float(e.median()) < 1e-2
+    if alike:
+        assert bool((got == got[:1]).all())
