@@ -6,32 +6,33 @@
 // mixture and the next norm.  The norm is split: the producer of a row stores  u * w  (bf16) and, per 8 columns, the sum of u^2; the
 // consumer multiplies its finished sums by  1 / sqrt(mean u^2 + eps), which is the same product with the row's factor taken out.
 //
-// Weights go from memory to the matrix operand directly (16 rows x 32 of K per wave and load, used once), and so do the activations: with
-// few rows they are a fraction of the weights' bytes per tile.  What one of these products makes for the next lies in the operand's order,
-// [column / 8][row][8], so that a load takes consecutive memory.  Two register buffers per wave keep two batches of loads in flight.
+// Weights go from memory to the matrix operand directly, used once, in whole cache lines (8 rows x 128 bytes per wave and load) with the
+// non-temporal policy: loads of 16 rows x 64 bytes, the operand's own shape, fetch half lines that are dropped before the other half is asked
+// for (4.9 TB/s of the 6.9 that a plain read reaches).  Activations are read directly too: with few rows they are a fraction of the weights'
+// bytes.  What one of these products makes for the next lies in the operand's order, [column / 8][row][8], so that a load takes consecutive memory.
+// Two register buffers per wave keep two batches of loads in flight.
 //
-// Measured, 2048 wide, 5440 feed-forward, one row (16 rows): 8192 columns 9.4 us (11.8), 33 MB; gates 11.8 us (15.6), 44 MB, 3.8 TB/s; the two
-// residual products 6.2 us (7.4) on average, 8 and 22 MB.  The tile products with K slices and their row-wise second launches took 12.8, 17.5
-// and 12.8 us.  A whole step of the 24-layer models: 1830 -> 1320 us (32 heads of 64), 1610 -> 1140 us (state space and latent attention).  About 4 us
-// of every launch are its start, the first loads and the sum over the waves.
+// Measured, 2048 wide, 5440 feed-forward, one row (16 rows, 28 rows): 8192 columns 9.0 us (9.5, 10.9), 33 MB; gates 10.9 us (11.5, 14.3), 44 MB; the two
+// residual products 4.4 and 7.0 us (5.0 and 8.3; 6.0 and 11.0), 8 and 22 MB; the head, 51200 columns, 36 us (40, 57), 210 MB.  With half lines: gates 12.2 us
+// (15.9), head 47 us.  The tile products with K slices and their row-wise second launches took 12.8, 17.5 and 12.8 us.  About 4 us of every launch
+// are its start, the first loads and the sum over the waves.
 #include "lm_internal.hpp"
 
 namespace {
 
 constexpr int EPI_ROWS = 0, EPI_SILU = 1, EPI_RESID = 2;
 
-// W waves, MT 16-row tiles.  A workgroup's columns: TN = 16, the matrix operand's rows; SiLU 8 gates and the 8 inputs beside them; or
-// TN = 8, for layers of so few columns that the tiles would not fill the chip evenly (2048 columns: 256 workgroups): the operand's upper 8
-// rows then hold the other 32 of a unit's 64 of K, so that one load is still 1 KB of weights.  It is multiplied with either half of the
-// activations, and the useful half of either product is kept.  MT = 0: up to 8 rows, whose two halves of K fit one operand as well.
+// W waves, MT 16-row tiles (0: up to 8 rows), U units of 64 of K per load batch.  A workgroup's columns are NX operands of 8; SiLU: 8 gates and the 8
+// inputs beside them.  A load is 8 rows x 128 bytes of weights, whole cache lines: the operand's upper 8 rows hold the other 32 of a unit's 64
+// of K.  It is multiplied with either half of the activations, and the useful half of either product is kept; up to 8 rows the two halves of
+// K of the activations fit one operand as well.  NX = 1: layers of so few columns that more would not fill the chip evenly.
 // S: streams of the residual epilogue (0: any count); otherwise 1: rows in order, 2: through rows_idx
-template <int MT, int TN, int W, int EPI, int S>
+template <int MT, int NX, int W, int U, int EPI, int S>
 __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
-  constexpr bool SPLIT = EPI != EPI_SILU && TN == 8, DIAG = MT == 0;
-  static_assert(SPLIT || !DIAG, "");
-  constexpr int M16 = DIAG ? 1 : MT, U = 2;  // (U: units, 64 of K, per load batch)
-  constexpr int PW = SPLIT ? 1 : 2, PA = DIAG ? 1 : 2;  // operands per unit
-  constexpr int C = SPLIT && !DIAG ? 2 : 1;             // accumulators per row tile
+  static_assert(EPI != EPI_SILU || NX == 2, "gates and inputs");
+  constexpr bool DIAG = MT == 0;
+  constexpr int M16 = DIAG ? 1 : MT, TN = EPI == EPI_SILU ? 8 : 8 * NX;
+  constexpr int PA = DIAG ? 1 : 2;  // operands of activations per unit, and accumulators per operand of weights
   auto row_of = [&](int m) { return EPI != EPI_RESID && S == 2 ? a.rows_idx[m] : m; };
   __shared__ f32x4 red[W][M16][64];
   __shared__ float row_scale[16 * M16];
@@ -53,18 +54,21 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
       }
   }
 
-  const int64_t n = EPI == EPI_SILU ? (int64_t)(r >> 3) * a.ff_pad + n0 + (r & 7) : n0 + (TN == 8 ? r & 7 : r);
-  const int kw = SPLIT ? 4 * (r >> 3) + g : g, ka = DIAG ? kw : g;  // 8-column piece of a unit that this lane takes
-  const bf16_t* wp = a.w + n * a.k + 8 * kw;
+  const int kw = 4 * (r >> 3) + g, ka = DIAG ? kw : g;  // 8-column piece of a unit that this lane takes
+  const bf16_t* wp[NX];
+#pragma unroll
+  for (int x = 0; x < NX; ++x) wp[x] = a.w + ((int64_t)x * (EPI == EPI_SILU ? a.ff_pad : 8) + n0 + (r & 7)) * a.k + 8 * kw;
   const bf16_t* ap[M16];
 #pragma unroll
   for (int i = 0; i < M16; ++i) ap[i] = a.a + (int64_t)row_of(min(16 * i + (DIAG ? r & 7 : r), a.rows - 1)) * a.lda + ka * a.chunk;
   const int units = a.k >> 6, lo = units * wave / W, hi = units * (wave + 1) / W;
-  f32x4 acc[C][M16];
+  f32x4 acc[NX][PA][M16];
 #pragma unroll
-  for (int h = 0; h < C; ++h)
+  for (int x = 0; x < NX; ++x)
 #pragma unroll
-    for (int i = 0; i < M16; ++i) acc[h][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int h = 0; h < PA; ++h)
+#pragma unroll
+      for (int i = 0; i < M16; ++i) acc[x][h][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // what the residual epilogue reads besides, under way before the weights
   constexpr int SM = EPI != EPI_RESID ? 1 : S > 0 ? S : MD_LM_MAX_STREAMS;
@@ -82,18 +86,18 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
       if (c + e < a.width) norm_w[e] = a.norm.w[(int64_t)(c + e) * a.norm.stride];
   }
 
-  u32x4 wf[2][PW * U], af[2][PA * U][M16];
+  u32x4 wf[2][U][NX], af[2][U][PA][M16];
   auto load = [&](auto buf, int u) {  // units u .. u + U - 1; past the end: the last one again, not used
     constexpr int B = decltype(buf)::value;
 #pragma unroll
     for (int q = 0; q < U; ++q) {
       const int k = min(u + q, hi - 1) * 64, kc = k / 8 * a.chunk;
 #pragma unroll
-      for (int h = 0; h < PW; ++h) wf[B][PW * q + h] = __builtin_nontemporal_load((const u32x4*)(wp + k + 32 * h));
+      for (int x = 0; x < NX; ++x) wf[B][q][x] = __builtin_nontemporal_load((const u32x4*)(wp[x] + k));
 #pragma unroll
       for (int h = 0; h < PA; ++h)
 #pragma unroll
-        for (int i = 0; i < M16; ++i) af[B][PA * q + h][i] = *(const u32x4*)(ap[i] + kc + 4 * h * a.chunk);
+        for (int i = 0; i < M16; ++i) af[B][q][h][i] = *(const u32x4*)(ap[i] + kc + 4 * h * a.chunk);
     }
   };
   auto multiply = [&](auto buf, int u) {
@@ -102,11 +106,13 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
     for (int q = 0; q < U; ++q)
       if (u + q < hi) {
 #pragma unroll
-        for (int h = 0; h < PA; ++h)
+        for (int x = 0; x < NX; ++x)
 #pragma unroll
-          for (int i = 0; i < M16; ++i)
-            acc[h % C][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(md_bf16x8v, wf[B][PW * q + h % PW]),
-                                                                    __builtin_bit_cast(md_bf16x8v, af[B][PA * q + h][i]), acc[h % C][i], 0, 0, 0);
+          for (int h = 0; h < PA; ++h)
+#pragma unroll
+            for (int i = 0; i < M16; ++i)
+              acc[x][h][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(md_bf16x8v, wf[B][q][x]), __builtin_bit_cast(md_bf16x8v, af[B][q][h][i]),
+                                                                     acc[x][h][i], 0, 0, 0);
       }
   };
   constexpr auto B0 = std::integral_constant<int, 0>{};
@@ -146,11 +152,20 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
   }
 #pragma unroll
   for (int i = 0; i < M16; ++i) {
-    f32x4 v = acc[0][i];
-    if (SPLIT) {  // columns 0 .. 7: lanes 0 .. 31 of the first half's product, 32 .. 63 of the other's; DIAG: rows 0 .. 7, and 8 .. 15
-      const int from = DIAG ? lane ^ 40 : lane ^ 32;
+    // an operand's 8 columns: lanes 0 .. 31 of the first half's product, 32 .. 63 of the other's; DIAG: rows 0 .. 7, and 8 .. 15.  The second
+    // operand's go to lanes 32 .. 63
+    f32x4 v;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] += __shfl(acc[C - 1][i][e], from, 64);
+    for (int e = 0; e < 4; ++e) {
+      if (NX == 1) {
+        v[e] = acc[0][0][i][e] + __shfl(acc[0][PA - 1][i][e], DIAG ? lane ^ 40 : lane ^ 32, 64);
+      } else if (DIAG) {
+        const float x = acc[0][0][i][e] + __shfl(acc[0][0][i][e], lane ^ 40, 64);
+        const float y = __shfl(acc[NX - 1][0][i][e], lane ^ 32, 64) + __shfl(acc[NX - 1][0][i][e], lane ^ 8, 64);
+        v[e] = g < 2 ? x : y;
+      } else {
+        v[e] = (g < 2 ? acc[0][0][i][e] : acc[NX - 1][PA - 1][i][e]) + __shfl(g < 2 ? acc[NX - 1][0][i][e] : acc[0][PA - 1][i][e], lane ^ 32, 64);
+      }
     }
     red[wave][i][lane] = v;
   }
@@ -205,25 +220,31 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
   }
 }
 
-template <int TN, int W, int EPI, int S>
+template <int MT, int NX, int W, int U, int EPI, int S>
 md_status launch(const LmStepGemm& a, int n, hipStream_t s) {
-  const dim3 grid(n / TN), block(64 * W);
-  if constexpr (EPI != EPI_SILU && TN == 8)
-    if (a.rows <= 8) {
-      hipLaunchKernelGGL((step_gemm_kernel<0, TN, W, EPI, S>), grid, block, 0, s, a);
-      return md_launch_status();
-    }
-  if (a.rows <= 16) hipLaunchKernelGGL((step_gemm_kernel<1, TN, W, EPI, S>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((step_gemm_kernel<2, TN, W, EPI, S>), grid, block, 0, s, a);
+  hipLaunchKernelGGL((step_gemm_kernel<MT, NX, W, U, EPI, S>), dim3(n / (EPI == EPI_SILU ? 8 : 8 * NX)), dim3(64 * W), 0, s, a);
   return md_launch_status();
 }
+template <int NX, int W, int U, int EPI, int S>
+md_status by_rows(const LmStepGemm& a, int n, hipStream_t s) {
+  return a.rows <= 8 ? launch<0, NX, W, U, EPI, S>(a, n, s) : a.rows <= 16 ? launch<1, NX, W, U, EPI, S>(a, n, s) : launch<2, NX, W, U, EPI, S>(a, n, s);
+}
 
-// 8 columns instead of 16 where that evens out few tiles and a unit is one load of either operand (6144 columns, 1 row: 8.5 us against
-// 9.7; 16 rows: 13.3 against 11.8; 51200 columns, 1 row: 50 against 41)
+// Columns and waves of a workgroup.  More than four workgroups of 16 columns per CU: two waves (51200 columns, 1 / 12 / 28 rows: 36 / 40 / 57 us; four waves
+// 36 / 41 / 58, eight 39 / 48 / 76).  Up to 8 rows, where a unit's activations are one load: 8 columns where that evens out few workgroups (6144
+// columns, 8 rows: 7.5 us against 8.0; 8192: 9.5 against 8.7), eight waves to share K otherwise.
 template <int S>
 md_status rows(const LmStepGemm& a, int n, hipStream_t s) {
   auto most = [&](int tn) { return (n / tn + 255) / 256 * tn; };  // columns that the fullest of the 256 CUs gets
-  return a.rows <= 8 && n <= 256 * 32 && most(8) < most(16) ? launch<8, 8, EPI_ROWS, S>(a, n, s) : launch<16, 8, EPI_ROWS, S>(a, n, s);
+  if (n > 256 * 64) return by_rows<2, 2, 1, EPI_ROWS, S>(a, n, s);
+  if (a.rows > 8) return by_rows<2, 4, 2, EPI_ROWS, S>(a, n, s);
+  return n <= 256 * 32 && most(8) < most(16) ? launch<0, 1, 4, 2, EPI_ROWS, S>(a, n, s) : launch<0, 2, 8, 1, EPI_ROWS, S>(a, n, s);
+}
+
+// Up to 8 rows four units per batch where K is long (5440: 6.8 us against 7.7; 2048: 4.4 either way)
+template <int S>
+md_status resid(const LmStepGemm& a, hipStream_t s) {
+  return a.rows <= 8 && a.k > 4096 ? launch<0, 1, 8, 4, EPI_RESID, S>(a, a.width_pad, s) : by_rows<1, 8, 2, EPI_RESID, S>(a, a.width_pad, s);
 }
 
 static_assert(LM_STEP_ROWS <= 32, "two row tiles");
@@ -241,15 +262,15 @@ md_status lm_step_rows(const LmStepGemm& a, int n, hipStream_t s) {
 
 md_status lm_step_silu(const LmStepGemm& a, hipStream_t s) {
   MD_CHECK_ARG(takes(a) && a.ff_pad % 64 == 0);
-  return launch<8, 4, EPI_SILU, 1>(a, a.ff_pad, s);
+  return by_rows<2, 2, 1, EPI_SILU, 1>(a, a.ff_pad, s);
 }
 
 md_status lm_step_resid(const LmStepGemm& a, hipStream_t s) {
   MD_CHECK_ARG(takes(a) && a.width_pad % 64 == 0 && a.streams >= 1 && a.streams <= MD_LM_MAX_STREAMS);
   switch (a.streams) {
-    case 1: return launch<8, 8, EPI_RESID, 1>(a, a.width_pad, s);
-    case 2: return launch<8, 8, EPI_RESID, 2>(a, a.width_pad, s);
-    case 4: return launch<8, 8, EPI_RESID, 4>(a, a.width_pad, s);
-    default: return launch<8, 8, EPI_RESID, 0>(a, a.width_pad, s);
+    case 1: return resid<1>(a, s);
+    case 2: return resid<2>(a, s);
+    case 4: return resid<4>(a, s);
+    default: return resid<0>(a, s);
   }
 }

@@ -40,9 +40,9 @@ struct LmWs {
 
 inline bool decode_regime(const md_lm_model* m, int rows) { return m->dtype == MD_DTYPE_BF16 && rows <= DECODE_ROWS; }
 
-// Most rows for which a product of gemm_step.hip is the faster one where nothing is saved behind it: the head (51200 columns; 1 row: 41-47 us
-// against 55 with its norm, 16 rows: 59 against 56, 32 rows: 85), and the first layer's projection.
-constexpr int STEP_PLAIN_ROWS = 8;
+// Most logits that gemm_step.hip's product makes of rows picked through an index (51200 columns; 1 row: 36 us against 50 of the tiles with the norm's
+// launch, 12 rows: 40 against 52, but 17 and 24 rows: 62 and 64 against 53 and 55).  Rows in order, as a decode step has them: 20 rows 52, 28 rows 58.
+constexpr int STEP_PICKED_ROWS = 16;
 
 // products that go on with the row-wise step behind them (gemm_step.hip)
 // (a router needs whole normed rows, which leaves nothing to go on with; and the first token's retention is its value times q . k, normed: only
@@ -287,7 +287,7 @@ struct Step {
 
   // a mixer's projection -> w.proj.  Few rows: K-slice partials and their sum in two launches, unless one slice fills the chip
   md_status project(const md_linear& lin) {
-    if (few && (sumsq || b->n_rows <= STEP_PLAIN_ROWS)) {
+    if (few) {
       LmStepGemm g = step_gemm(w.h, m->width_pad, lin, sumsq != nullptr);
       g.out = (bf16_t*)w.proj;
       g.ldo = lin.n_pad;
@@ -583,7 +583,7 @@ struct Step {
     const int64_t row_floats = (int64_t)b->n_rows * m->width_pad;
     if (own_row_steps(m)) MD_TRY(lm_embed_streams(m, b->tokens, b->row_pos, w.x, row_floats, b->n_rows, s));
     else MD_TRY(lm_embed(m->dtype, m->embed, m->width_pad, b->tokens, w.x, b->n_rows, m->vocab, s));
-    const bool few_logits = n_logits > 0 && n_logits <= STEP_PLAIN_ROWS;
+    const bool few_logits = n_logits > 0 && n_logits <= (logit_rows ? STEP_PICKED_ROWS : LM_STEP_ROWS);
     for (int i = 0; i < m->n_layers; ++i) {
       const md_lm_layer& l = m->layers[i];
       // what follows this layer: the next one's mixer, or the head

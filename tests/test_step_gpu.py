@@ -217,3 +217,26 @@ def test_state_space_prompts_that_fill_the_chip(lens):
     assert float(e[int(0.9 * len(e))]) < 7e-2 and float(e[-1]) < 1.0
     got = m.step([(s, t[-1:], [0]) for s, t in zip(slots, ts)])
     assert float(U.logit_errors(got, torch.cat([x[-1:] for x in want])).max()) < 7e-2
+
+
+def test_rows_of_many_columns():
+    """Step products of more than 16384 columns (the head), more than 8192 (an input projection) and of more than 4096 of K (the down product)."""
+    cfg = U.stream_config([(U.ssm(64, 64, 16), U.dense(4200))], width=128, vocab=16600, streams=2, positions=8)
+    m, w = build(cfg), U.weights(cfg, 3, 1.5)
+    ts = [U.tokens(2, cfg["vocab"], i) for i in range(28)]
+    want = torch.stack([O.forward(cfg, w, t) for t in ts])
+    for n in (1, 8, 9, 16, 17, 28):
+        slots = [m.open_sequence() for _ in range(n)]
+        for k in range(2):
+            got = m.step([(s, [t[k]], [0]) for s, t in zip(slots, ts)])
+            assert float(U.logit_errors(got, want[:n, k]).max()) < 7e-2, (n, k)
+        for s in slots:
+            m.close_sequence(s)
+        # rows in order, without an index: a decode step's logits
+        slots = [m.open_sequence() for _ in range(n)]
+        m.step([(s, t[:1], []) for s, t in zip(slots, ts)])
+        logits = m._decode_logits(n)
+        m._decode_lockstep(torch.tensor([t[1] for t in ts[:n]], dtype=torch.int32, device="cuda"), slots, 1)
+        assert float(U.logit_errors(logits[:n, : cfg["vocab"]], want[:n, 1]).max()) < 7e-2, n
+        for s in slots:
+            m.close_sequence(s)
