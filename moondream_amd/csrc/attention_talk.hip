@@ -509,6 +509,13 @@ __host__ __device__ constexpr TalkLds talk_lds(int hpad, int dp, int nw) {
   return l;
 }
 
+// Parts of a tile's keys: a tile's place among all tiles of a step (a sequence has at most len / 16 + 2), and what one part leaves
+constexpr int TALK_ROUNDS = 8, TALK_PARTS = 1536, TALK_LEAST = 3;  // parts of a step at most; 64 keys of a part at least
+__host__ __device__ inline int talk_rounds(int parts) { return parts > 1 ? 1 : TALK_ROUNDS; }
+inline int talk_longest(int span) { return (span + 31 + 63) / 64; }  // of 64 keys each; the first may begin before the chunk
+__device__ __forceinline__ int talk_slot(int row0, int seq, int tile) { return row0 / 16 + 2 * seq + tile; }
+__host__ __device__ inline int64_t talk_part_floats(int heads, int vp) { return (int64_t)heads * (16 * vp + 32); }
+
 // keeps the compiler from overlapping the phases of a tile: their register peaks would add up
 #define PHASE() __builtin_amdgcn_sched_barrier(0)
 
@@ -535,12 +542,27 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void attn_mfma_kernel(const LmAttn
   float* mss = (float*)(smem + L.ms);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, q = lane >> 4;
 
-  const int lin = xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
-  const int seq = lin / gridDim.x, tile = lin - seq * gridDim.x;
+  // which tile: every eighth one of a sequence to an XCD (its CUs share the sequence's keys and values in L2), longest first; whole tiles in eight rounds
+  // over the sequences, so that the last ones are short; parts one after the other.  Workgroups go to XCDs and their engines in turn, so neighbours have to
+  // be alike; a single sequence's parts begin at another engine each.  Equal sequences in eights: whole sequences to an XCD.
+  // (11 ragged prompts, 13250 tokens, 32 heads of 64: 699 us with a run of tiles per XCD, shortest first, 532 this way; 3 x 2048 tokens 544 and 330, 8 x 2048
+  // 817 and 743, 785 where XCDs share the sequences.  Persistent workgroups with a queue per XCD: 697, 460 and 1064, the loop around the tile costs
+  // registers.)
+  const int tiles8 = ((a.r.max_len + 30) / 16 + 7) >> 3, rounds = talk_rounds(a.n_split), per = (tiles8 + rounds - 1) / rounds, xcd = blockIdx.x & 7;
+  const int item = blockIdx.x >> 3, part = a.n_split > 1 ? item / (per * a.r.n_seq) : 0, at = item - part * per * a.r.n_seq;
+  const bool eights = a.n_split == 1 && a.r.n_seq % 8 == 0 && a.r.n_rows == a.r.n_seq * a.r.max_len;
+  const int seq = eights ? 8 * (item % (a.r.n_seq / 8)) + xcd : at / per % a.r.n_seq;
+  const int nth = eights ? item / (a.r.n_seq / 8) : (at / (per * a.r.n_seq) * per + (at + (a.r.n_seq == 1 ? part : 0)) % per) * 8 + xcd;
   const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, pos0 = a.r.seq_pos0[seq], slot = a.r.seq_slot[seq];
+  const int tile = (pos0 + len - 1) / 16 - pos0 / 16 - nth;
+  if (tile < 0) return;
   const int t0 = (pos0 / 16 + tile) * 16;
   const int lo = max(t0, pos0), hi = min(t0 + 15, pos0 + len - 1);  // positions of the tile's live queries
-  if (lo > hi) return;
+  // its keys, and this part of them
+  const int kfirst = (a.chunk > 0 ? lo / a.chunk * a.chunk : 0) & ~31;
+  const int kstart = kfirst + part * a.split_keys, klast = min(hi, kstart + a.split_keys - 1);
+  if (kstart > hi) return;
+  const bool whole = kfirst + a.split_keys > hi;
   const bf16_t* Kb = (const bf16_t*)a.k + (int64_t)slot * G * a.ctx * dp;
   const bf16_t* Vb = (const bf16_t*)a.v + (int64_t)slot * G * a.ctx * vp;
 
@@ -553,12 +575,12 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void attn_mfma_kernel(const LmAttn
       if (h < H) v = *(const u32x4*)((const bf16_t*)a.q + (row * H + h) * dp + ch * 8);
       *(u32x4*)(Qs + hn * (dp + 8) + ch * 8) = v;
     }
-    for (int h = tid; h < HP; h += NW * 64) {
-      float s = 0.f;
-      if (h < H)
-        for (int g = 0; g < H; ++g) s += a.mix[h * H + g] * a.slope[g];
-      mss[h] = s * kLog2e;
-    }
+    constexpr int LH = NW * 64 / HP;  // lanes per head
+    float s = 0.f;
+    for (int h = tid / LH, g = tid % LH; g < H; g += LH) s += h < H ? a.mix[h * H + g] * a.slope[g] : 0.f;
+#pragma unroll
+    for (int o = LH / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (tid % LH == 0) mss[tid / LH] = s * kLog2e;
   }
   // A operand of the mixture: row h = 16 mt + n, heads 8 q .. 8 q + 7 (HB 2) or 4 q .. 4 q + 3 (HB 1)
   bf16x8 tf[HB];
@@ -586,7 +608,7 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void attn_mfma_kernel(const LmAttn
 
   const float scale = a.scale * kLog2e;
   const int qpos = t0 + n, qfirst = a.chunk > 0 ? qpos / a.chunk * a.chunk : 0;
-  const int kstart = (a.chunk > 0 ? lo / a.chunk * a.chunk : 0) & ~31, hfirst = a.chunk > 0 ? hi / a.chunk * a.chunk : 0;
+  const int hfirst = a.chunk > 0 ? hi / a.chunk * a.chunk : 0;
 
   // Byte strides of a block of 32 keys / values and the reciprocal of the group size, made opaque once per tile: the heads' base addresses are
   // then computed where they are used (scalar) instead of being kept in registers across the whole loop.
@@ -613,7 +635,7 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void attn_mfma_kernel(const LmAttn
   };
 
   load_k(0, 0, kstart + 16 * wave);
-  for (int j0 = kstart; j0 <= hi; j0 += TK) {
+  for (int j0 = kstart; j0 <= klast; j0 += TK) {
     asm volatile("" : "+s"(kbs), "+s"(vbs), "+s"(inv_rep));
     const int jw = j0 + 16 * wave;
     const bool live = jw <= hi;
@@ -754,7 +776,7 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void attn_mfma_kernel(const LmAttn
       *(u32x4*)(dst + 8) = u32x4{pk[4], pk[5], pk[6], pk[7]};
     }
     __syncthreads();
-    if (j0 + TK <= hi) load_k(0, 0, jw + TK);
+    if (j0 + TK <= klast) load_k(0, 0, jw + TK);
 #pragma unroll
     for (int step = 0; step < NS; ++step) {
       if (step + PD < NS) load_v(step + PD, j0);
@@ -778,6 +800,15 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void attn_mfma_kernel(const LmAttn
 #pragma unroll
   for (int i = 0; i < HB * 4; ++i) mxs[(wave * HP + 16 * (i >> 2) + 4 * q + (i & 3)) * 16 + n] = l_run[i];
   __syncthreads();
+  // one of several parts: its sums as the lanes hold them, its maxima and weights
+  float* part_o = a.part + ((int64_t)talk_slot(row0, seq, tile) * a.n_split + part) * talk_part_floats(H, vp);
+  float* part_ml = part_o + H * 16 * vp;
+  if (!whole && wave == 0)
+#pragma unroll
+    for (int i = 0; i < HB * 4; ++i) {
+      const int h = 16 * (i >> 2) + 4 * q + (i & 3);
+      if (h < H) part_ml[h * 32 + n] = m_run[i];
+    }
 #pragma unroll
   for (int hh = 0; hh < HPW; ++hh) {
     const int h = wave * HPW + hh;
@@ -785,6 +816,12 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void attn_mfma_kernel(const LmAttn
     f32x4 l = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < NW; ++w) l += *(const f32x4*)(mxs + (w * HP + h) * 16 + 4 * q);
+    if (!whole) {
+      if (n == 0) *(f32x4*)(part_ml + h * 32 + 16 + 4 * q) = l;
+#pragma unroll
+      for (int t = 0; t < 2 * C; ++t) *(f32x4*)(part_o + ((h * 2 * C + t) * 64 + lane) * 4) = oacc[hh][t];
+      continue;
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int pos = t0 + 4 * q + r;
@@ -794,6 +831,47 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void attn_mfma_kernel(const LmAttn
 #pragma unroll
       for (int t = 0; t < 2 * C; ++t) dst[16 * t] = f2bf(oacc[hh][t][r] * inv);
     }
+  }
+}
+
+// sums the parts of a tile: grid (tiles, sequences, groups of 4 heads), a wave per head
+__global__ __launch_bounds__(256) void attn_parts_kernel(const LmAttn a) {
+  const int seq = blockIdx.y, h = blockIdx.z * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, n = lane & 15, q = lane >> 4;
+  const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, pos0 = a.r.seq_pos0[seq];
+  const int tile = blockIdx.x, t0 = (pos0 / 16 + tile) * 16, lo = max(t0, pos0), hi = min(t0 + 15, pos0 + len - 1);
+  const int kfirst = (a.chunk > 0 ? lo / a.chunk * a.chunk : 0) & ~31;
+  if (lo > hi || h >= a.heads || kfirst + a.split_keys > hi) return;
+  const int parts = (hi - kfirst) / a.split_keys + 1, pieces = a.vp / 16;
+  const int64_t stride = talk_part_floats(a.heads, a.vp);
+  const float* p = a.part + (int64_t)talk_slot(row0, seq, tile) * a.n_split * stride;
+  const float* ml = p + a.heads * 16 * a.vp + h * 32 + 4 * q;
+  f32x4 m = {-INFINITY, -INFINITY, -INFINITY, -INFINITY}, l = {0.f, 0.f, 0.f, 0.f}, o[8];
+  for (int k = 0; k < parts; ++k) {
+    const f32x4 mk = *(const f32x4*)(ml + k * stride);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) m[r] = fmaxf(m[r], mk[r]);
+  }
+#pragma unroll
+  for (int t = 0; t < 8; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int k = 0; k < parts; ++k) {
+    const f32x4 mk = *(const f32x4*)(ml + k * stride), lk = *(const f32x4*)(ml + k * stride + 16);
+    f32x4 w;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) w[r] = __builtin_amdgcn_exp2f(mk[r] - m[r]);
+    l += w * lk;
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+      if (t < pieces) o[t] += w * *(const f32x4*)(p + k * stride + ((h * pieces + t) * 64 + lane) * 4);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int pos = t0 + 4 * q + r;
+    if (pos < lo || pos > hi) continue;
+    const float inv = 1.0f / l[r];
+    bf16_t* dst = (bf16_t*)a.out + (int64_t)(row0 + pos - pos0) * a.ldo + h * a.vp + n;
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+      if (t < pieces) dst[16 * t] = f2bf(o[t][r] * inv);
   }
 }
 
@@ -837,11 +915,39 @@ TalkPick talk_pick(const LmAttn& a) {
 }  // namespace
 
 bool lm_attn_mfma_takes(const LmAttn& a) { return talk_pick(a).fn != nullptr; }
+// How many parts a tile's keys are cut into, and their length.  A tile of 64 keys takes 9.7 us and a workgroup 12 us besides, so a step of
+// fewer tiles than CUs lasts as long as its longest: 32 heads of 64, one prompt of 1000 tokens (63 tiles) 163 us, in six parts 63; 700 tokens 117 and 57, 350
+// 67 and 48, 200 as before; two prompts of 1500 tokens 246 and 162, five ragged ones (3900 tokens, 244 tiles) 227 and 200.  Up to 128 tiles the parts fill the
+// CUs once, up to 256 twice.  With more tiles the sums of the parts (132 KB each, written and read) cost more than they even out: 3 x 2048 tokens
+// 341 us whole, 368 in three parts.
+int lm_attn_mfma_parts(int n_rows, int n_seq, int span, int* split_keys) {
+  const int tiles = n_rows / 16 + n_seq, longest = talk_longest(span);
+  int keys = longest;
+  if (tiles <= 256) {
+    const double mean = longest - std::min<double>(n_rows / n_seq, span) / 128;
+    keys = std::max(TALK_LEAST, (int)(1.4 * tiles * mean / (tiles <= 128 ? 256 : 512)));
+    const int most = TALK_PARTS / (n_rows / 16 + 2 * n_seq);
+    if (most < 2) keys = longest;
+    else keys = std::max(keys, (longest + most - 1) / most);
+  }
+  if (keys + 1 >= longest) keys = longest;
+  *split_keys = 64 * keys;
+  return (longest + keys - 1) / keys;
+}
+size_t lm_attn_mfma_part_floats_most(int n_rows, int n_seq, int span, int heads, int vp) {
+  const int64_t parts = (talk_longest(span) + TALK_LEAST - 1) / TALK_LEAST, slots = n_rows / 16 + 2 * n_seq;
+  return parts > 1 ? (size_t)std::min<int64_t>(TALK_PARTS, slots * parts) * talk_part_floats(heads, vp) : 0;
+}
 md_status lm_attn_mfma(const LmAttn& a, hipStream_t s) {
   const TalkPick t = talk_pick(a);
   if (!t.fn) return MD_ERR_UNSUPPORTED;
   MD_TRY(md_ensure_dynamic_lds((const void*)t.fn, 160 * 1024));
-  hipLaunchKernelGGL(t.fn, dim3((a.r.max_len + 30) / 16, a.r.n_seq), dim3(t.waves * 64), t.lds, s, a);
+  const int tiles = (a.r.max_len + 30) / 16;
+  const int rounds = talk_rounds(a.n_split), items = 8 * rounds * (((tiles + 7) / 8 + rounds - 1) / rounds) * a.r.n_seq * a.n_split;
+  hipLaunchKernelGGL(t.fn, dim3(items), dim3(t.waves * 64), t.lds, s, a);
+  MD_TRY(md_launch_status());
+  if (a.n_split == 1) return MD_OK;
+  hipLaunchKernelGGL(attn_parts_kernel, dim3(tiles, a.r.n_seq, (a.heads + 3) / 4), dim3(256), 0, s, a);
   return md_launch_status();
 }
 

@@ -102,9 +102,10 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
     }
     if (l.mixer == MD_MIXER_ATTENTION) {
       q = std::max(q, (size_t)l.heads * l.dim_pad);
+      const int span = l.chunk > 0 ? std::min(l.chunk, max_ctx) : max_ctx;
+      if (max_len > 1 && m->dtype == MD_DTYPE_BF16) ap = std::max(ap, lm_attn_mfma_part_floats_most(rows, n_seq, span, l.heads, l.vdim_pad));
       if (max_len == 1) {
         int keys;
-        const int span = l.chunk > 0 ? std::min(l.chunk, max_ctx) : max_ctx;
         const int ns = lm_attn_decode_splits(n_seq, span, &keys);
         ap = std::max(ap, lm_attn_decode_part_floats(n_seq, ns, l.heads, l.vdim_pad));
       }
@@ -402,13 +403,17 @@ struct Step {
     a.q = w.q;
     a.out = w.att;
     a.ldo = l.out_proj.k_pad;
+    a.part = w.attn_part;
+    const int span = l.chunk > 0 ? std::min(l.chunk, b->max_ctx) : b->max_ctx;
     if (m->dtype == MD_DTYPE_BF16 && b->max_len == 1 && (g_lm_kernels & 2) && lm_attn_decode_takes(a)) {
-      a.part = w.attn_part;
-      a.n_split = lm_attn_decode_splits(b->n_seq, l.chunk > 0 ? std::min(l.chunk, b->max_ctx) : b->max_ctx, &a.split_keys);
+      a.n_split = lm_attn_decode_splits(b->n_seq, span, &a.split_keys);
       return lm_attn_decode(a, s);
     }
     MD_TRY(lm_attn_prep(m->dtype, a, s));
-    if (m->dtype == MD_DTYPE_BF16 && b->max_len > 1 && (g_lm_kernels & 1) && lm_attn_mfma_takes(a)) return lm_attn_mfma(a, s);
+    if (m->dtype == MD_DTYPE_BF16 && b->max_len > 1 && (g_lm_kernels & 1) && lm_attn_mfma_takes(a)) {
+      a.n_split = lm_attn_mfma_parts(b->n_rows, b->n_seq, span, &a.split_keys);
+      return lm_attn_mfma(a, s);
+    }
     return lm_attn_plain(m->dtype, a, s);
   }
 

@@ -383,3 +383,40 @@ def test_command_line(tmp_path, name):
     assert r.returncode == 0, r.stderr
     want = model(name, F32).batch_generate_ids([p, [3, 4]], max_tokens=5)
     assert [[int(x) for x in line.split()] for line in r.stdout.strip().splitlines()] == want
+
+
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(4, 4, 32, 32), (16, 4, 64, 64), (12, 12, 96, 128), (32, 32, 64, 64), (20, 5, 32, 64)], ids=str)
+@pytest.mark.parametrize("lens,chunk", [([260], 2000), ([700], 2000), ([620, 3, 250, 431], 2000), ([900], 333)], ids=str)
+def test_prompts_whose_tiles_are_cut_by_keys(heads, kv, dim, vdim, lens, chunk):
+    """Prefill attention of so few query tiles that their keys are divided between workgroups: first tiles whole and last ones in parts, ragged
+    sequences, chunks that begin inside a part, and a second portion behind odd positions."""
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    cfg = U.config([U.attention(heads, kv, dim, vdim, chunk)], width=96, vocab=120, ff=None)
+    w = U.weights(cfg, 3, 1.5)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=BF16, max_batch=4, max_context=1000)
+    ts = [U.tokens(n, 120, n) for n in lens]
+    want = [O.forward(cfg, w, t) for t in ts]
+    slots = [m.open_sequence() for _ in ts]
+    got = m.step([(s, t, range(len(t))) for s, t in zip(slots, ts)])
+    assert float(U.logit_errors(got, torch.cat(want)).max()) < 7e-2
+    s, cut = m.open_sequence(), lens[0] // 2 + 7
+    got = torch.cat([m.step([(s, ts[0][:cut], range(cut))]), m.step([(s, ts[0][cut:], range(lens[0] - cut))])])
+    assert float(U.logit_errors(got, want[0]).max()) < 7e-2
+
+
+@pytest.mark.parametrize("lens", [[530] * 8, [300] * 16, [530] * 7 + [10]], ids=["eight", "sixteen", "ragged"])
+def test_prompts_of_eight_sequences(lens):
+    """More query tiles than CUs, eight equal sequences (one to an XCD), sixteen, and eight that differ."""
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    cfg = U.config([U.attention(4, 2, 32, 64, 2000)], width=96, vocab=120, ff=None)
+    w = U.weights(cfg, 3, 1.5)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=BF16, max_batch=16, max_context=600)
+    ts = [U.tokens(n, 120, i % 3) for i, n in enumerate(lens)]
+    kept = {tuple(t): O.forward(cfg, w, t) for t in {tuple(t): t for t in ts}.values()}
+    want = [kept[tuple(t)] for t in ts]
+    got = m.step([(m.open_sequence(), t, range(len(t))) for t in ts])
+    assert float(U.logit_errors(got, torch.cat(want)).max()) < 7e-2
