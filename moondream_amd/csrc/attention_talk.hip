@@ -511,7 +511,8 @@ __host__ __device__ constexpr TalkLds talk_lds(int hpad, int dp, int nw) {
 
 // Parts of a tile's keys: a tile's place among all tiles of a step (a sequence has at most len / 16 + 2), and what one part leaves
 constexpr int TALK_ROUNDS = 8, TALK_PARTS = 1536, TALK_LEAST = 3;  // parts of a step at most; 64 keys of a part at least
-__host__ __device__ inline int talk_rounds(int parts) { return parts > 1 ? 1 : TALK_ROUNDS; }
+__host__ __device__ inline int talk_rounds(int tiles8, int parts) { return parts > 1 ? 1 : tiles8 < TALK_ROUNDS ? tiles8 : TALK_ROUNDS; }
+__host__ __device__ inline bool talk_few(int tiles, int parts) { return parts == 1 && tiles < 16; }  // short sequences: tile after tile
 inline int talk_longest(int span) { return (span + 31 + 63) / 64; }  // of 64 keys each; the first may begin before the chunk
 __device__ __forceinline__ int talk_slot(int row0, int seq, int tile) { return row0 / 16 + 2 * seq + tile; }
 __host__ __device__ inline int64_t talk_part_floats(int heads, int vp) { return (int64_t)heads * (16 * vp + 32); }
@@ -545,14 +546,16 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void attn_mfma_kernel(const LmAttn
   // which tile: every eighth one of a sequence to an XCD (its CUs share the sequence's keys and values in L2), longest first; whole tiles in eight rounds
   // over the sequences, so that the last ones are short; parts one after the other.  Workgroups go to XCDs and their engines in turn, so neighbours have to
   // be alike; a single sequence's parts begin at another engine each.  Equal sequences in eights: whole sequences to an XCD.
-  // (11 ragged prompts, 13250 tokens, 32 heads of 64: 699 us with a run of tiles per XCD, shortest first, 532 this way; 3 x 2048 tokens 544 and 330, 8 x 2048
-  // 817 and 743, 785 where XCDs share the sequences.  Persistent workgroups with a queue per XCD: 697, 460 and 1064, the loop around the tile costs
+  // (11 ragged prompts, 13250 tokens, 32 heads of 64: 699 us with a run of tiles per XCD, shortest first, 513 this way; 3 x 2048 tokens 544 and 330, 8 x 2048
+  // 817 and 691, 785 where XCDs share the sequences.  Persistent workgroups with a queue per XCD: 697, 460 and 1064, the loop around the tile costs
   // registers.)
-  const int tiles8 = ((a.r.max_len + 30) / 16 + 7) >> 3, rounds = talk_rounds(a.n_split), per = (tiles8 + rounds - 1) / rounds, xcd = blockIdx.x & 7;
-  const int item = blockIdx.x >> 3, part = a.n_split > 1 ? item / (per * a.r.n_seq) : 0, at = item - part * per * a.r.n_seq;
-  const bool eights = a.n_split == 1 && a.r.n_seq % 8 == 0 && a.r.n_rows == a.r.n_seq * a.r.max_len;
-  const int seq = eights ? 8 * (item % (a.r.n_seq / 8)) + xcd : at / per % a.r.n_seq;
-  const int nth = eights ? item / (a.r.n_seq / 8) : (at / (per * a.r.n_seq) * per + (at + (a.r.n_seq == 1 ? part : 0)) % per) * 8 + xcd;
+  const int tiles = (a.r.max_len + 30) / 16, tiles8 = (tiles + 7) >> 3, rounds = talk_rounds(tiles8, a.n_split), per = (tiles8 + rounds - 1) / rounds;
+  const int xcd = blockIdx.x & 7, item = blockIdx.x >> 3, part = a.n_split > 1 ? item / (per * a.r.n_seq) : 0, at = item - part * per * a.r.n_seq;
+  const bool few = talk_few(tiles, a.n_split), eights = a.n_split == 1 && a.r.n_seq % 8 == 0 && a.r.n_rows == a.r.n_seq * a.r.max_len;
+  const int seq = few ? blockIdx.x / tiles : eights ? 8 * (item % (a.r.n_seq / 8)) + xcd : at / per % a.r.n_seq;
+  const int nth = few      ? blockIdx.x % tiles
+                  : eights ? item / (a.r.n_seq / 8)
+                           : (at / (per * a.r.n_seq) * per + (at + (a.r.n_seq == 1 ? part : 0)) % per) * 8 + ((xcd + seq) & 7);
   const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, pos0 = a.r.seq_pos0[seq], slot = a.r.seq_slot[seq];
   const int tile = (pos0 + len - 1) / 16 - pos0 / 16 - nth;
   if (tile < 0) return;
@@ -943,7 +946,8 @@ md_status lm_attn_mfma(const LmAttn& a, hipStream_t s) {
   if (!t.fn) return MD_ERR_UNSUPPORTED;
   MD_TRY(md_ensure_dynamic_lds((const void*)t.fn, 160 * 1024));
   const int tiles = (a.r.max_len + 30) / 16;
-  const int rounds = talk_rounds(a.n_split), items = 8 * rounds * (((tiles + 7) / 8 + rounds - 1) / rounds) * a.r.n_seq * a.n_split;
+  const int tiles8 = (tiles + 7) / 8, rounds = talk_rounds(tiles8, a.n_split);
+  const int items = talk_few(tiles, a.n_split) ? tiles * a.r.n_seq : 8 * rounds * ((tiles8 + rounds - 1) / rounds) * a.r.n_seq * a.n_split;
   hipLaunchKernelGGL(t.fn, dim3(items), dim3(t.waves * 64), t.lds, s, a);
   MD_TRY(md_launch_status());
   if (a.n_split == 1) return MD_OK;
