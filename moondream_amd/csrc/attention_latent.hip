@@ -472,62 +472,67 @@ __global__ __launch_bounds__(64 * WK * WH * WR, 2) void latent_decode_kernel(con
   }
 }
 
-// grid (heads, sequences / SEQ): sum over the splits, then four threads per output column share the latent's columns.  SEQ 1: the waves
-// share the splits of one sequence; 4: a wave per sequence, and every weight that is read serves four
-constexpr int MAX_SPLITS = 64;
+// grid (heads, sequences / SEQ, columns / 32): sum over the splits, then eight threads per output column share the latent's columns.  SEQ 1: the
+// waves share the splits of one sequence; 4: a wave per sequence, and every weight that is read serves four.  What bounds it is the chain of
+// loads (weights of a head are 64 to 128 KB, sums as much): the weights are under way before the sums are looked up, and 32 columns per workgroup
+// put several on every CU, though they add up the splits each for itself.  20 sequences, 16 heads of 128, rank 512: 17.6 us with all columns of a
+// head in a workgroup and its weights behind the sums, 10.0 this way; 23 of 32 x 64: 10.0 and 8.2, one 9.7 and 7.1; 40 of 32 x 64, rank 256: 7.7 and 7.0.
+constexpr int MAX_SPLITS = 64, OUT_COLS = 32, MAX_RANK = 512;
 template <int SEQ>
 __global__ __launch_bounds__(256) void latent_out_kernel(const LmLatent a) {
   static_assert(SEQ == 1 || SEQ == 4, "");
   extern __shared__ __attribute__((aligned(16))) float zsm[];  // [4][rp]
   __shared__ float fs[4][MAX_SPLITS];
   const int h = blockIdx.x, s0 = blockIdx.y * SEQ, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, R = a.rp, n = a.n_split;
+  const int s = tid & 7, e = blockIdx.z * OUT_COLS + (tid >> 3);
+  const bf16_t* w = (const bf16_t*)a.up_kv.w + ((int64_t)a.heads * a.dp + h * a.vp + e) * R + 8 * s;
+  u32x4 wv[MAX_RANK / 64];
+#pragma unroll
+  for (int i = 0; i < MAX_RANK / 64; ++i) wv[i] = *(const u32x4*)(w + (64 * i < R ? 64 * i : 0));
   const int mine = SEQ == 1 ? s0 : min(s0 + wave, a.r.n_seq - 1);
   const int64_t base = ((int64_t)mine * a.heads + h) * n;
   const float* pm = a.part + (int64_t)a.r.n_seq * a.heads * n * R + base * 2;
   const float mk = lane < n ? pm[2 * lane] : -INFINITY, lk = lane < n ? pm[2 * lane + 1] : 0.f;
   const float m = wave_max(mk), f0 = lk == 0.f ? 0.f : __builtin_amdgcn_exp2f(mk - m), sum = wave_sum(f0 * lk);
+  const int live = 64 - __clzll((long long)__ballot(lk != 0.f));  // (an empty split wrote no sums; those behind the sequence's end are)
   fs[wave][lane] = f0 / sum;
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the wave's own row)
   for (int r = 4 * lane; r < R; r += 256) {
     f32x4 z = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 8
-    for (int k = SEQ == 1 ? wave : 0; k < n; k += SEQ == 1 ? 4 : 1) {
+    for (int k = SEQ == 1 ? wave : 0; k < live; k += SEQ == 1 ? 4 : 1) {
       const f32x4 v = *(const f32x4*)(a.part + (base + k) * R + r);
       const float f = fs[wave][k];
-      z += f != 0.f ? f * v : f32x4{0.f, 0.f, 0.f, 0.f};  // (an empty split wrote no sums)
+      z += f != 0.f ? f * v : f32x4{0.f, 0.f, 0.f, 0.f};
     }
     *(f32x4*)(zsm + wave * R + r) = z;
   }
   __syncthreads();
-  const int s = tid & 3;
-  for (int e = tid >> 2; e < a.vp; e += 64) {
-    const bf16_t* w = (const bf16_t*)a.up_kv.w + ((int64_t)a.heads * a.dp + h * a.vp + e) * R;
-    float o[SEQ];
+  float o[SEQ];
 #pragma unroll
-    for (int i = 0; i < SEQ; ++i) o[i] = 0.f;
-#pragma unroll 4
-    for (int r = 8 * s; r < R; r += 32) {
-      const u32x4 wv = *(const u32x4*)(w + r);
-      const f32x4 w0 = half8(wv, 0), w1 = half8(wv, 1);
+  for (int i = 0; i < SEQ; ++i) o[i] = 0.f;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const f32x4 t = w0 * *(const f32x4*)(zsm + k * R + r) + w1 * *(const f32x4*)(zsm + k * R + r + 4);
-        o[SEQ == 1 ? 0 : k] += (t[0] + t[1]) + (t[2] + t[3]);
-      }
+  for (int i = 0; i < MAX_RANK / 64; ++i) {
+    if (64 * i >= R) break;
+    const f32x4 w0 = half8(wv[i], 0), w1 = half8(wv[i], 1);
+    const float* z = zsm + 64 * i + 8 * s;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const f32x4 t = w0 * *(const f32x4*)(z + k * R) + w1 * *(const f32x4*)(z + k * R + 4);
+      o[SEQ == 1 ? 0 : k] += (t[0] + t[1]) + (t[2] + t[3]);
     }
-#pragma unroll
-    for (int i = 0; i < SEQ; ++i) {
-      o[i] += __shfl_xor(o[i], 1, 64);
-      o[i] += __shfl_xor(o[i], 2, 64);
-    }
-    float v = o[0];
-#pragma unroll
-    for (int i = 1; i < SEQ; ++i) v = s == i ? o[i] : v;  // thread s writes sequence s
-    if (s >= SEQ || s0 + s >= a.r.n_seq) continue;
-    const int64_t row = a.r.seq_row0[s0 + s];
-    if (a.col_g >= 0) v *= sigmoid_f32(bf2f(((const bf16_t*)a.proj)[row * a.ldp + a.col_g + h * a.vp + e]));
-    ((bf16_t*)a.out)[row * a.ldo + h * a.vp + e] = f2bf(v);
   }
+#pragma unroll
+  for (int i = 0; i < SEQ; ++i)
+#pragma unroll
+    for (int d = 1; d < 8; d <<= 1) o[i] += __shfl_xor(o[i], d, 64);
+  float v = o[0];
+#pragma unroll
+  for (int i = 1; i < SEQ; ++i) v = s == i ? o[i] : v;  // thread s writes sequence s
+  if (s >= SEQ || s0 + s >= a.r.n_seq) return;
+  const int64_t row = a.r.seq_row0[s0 + s];
+  if (a.col_g >= 0) v *= sigmoid_f32(bf2f(((const bf16_t*)a.proj)[row * a.ldp + a.col_g + h * a.vp + e]));
+  ((bf16_t*)a.out)[row * a.ldo + h * a.vp + e] = f2bf(v);
 }
 
 typedef void (*LatentKernel)(const LmLatent);
@@ -622,7 +627,7 @@ md_status lm_latent_decode(const LmLatent& a, hipStream_t s) {
   MD_TRY(md_launch_status());
   hipLaunchKernelGGL(k.attend, dim3(a.n_split, a.r.n_seq, (a.heads + 16 * k.head_tiles - 1) / (16 * k.head_tiles)), dim3(k.threads), k.lds, s, a);
   MD_TRY(md_launch_status());
-  if (a.r.n_seq >= 16) hipLaunchKernelGGL(latent_out_kernel<4>, dim3(a.heads, (a.r.n_seq + 3) / 4), dim3(256), 4 * a.rp * 4, s, a);
-  else hipLaunchKernelGGL(latent_out_kernel<1>, dim3(a.heads, a.r.n_seq), dim3(256), 4 * a.rp * 4, s, a);
+  if (a.r.n_seq >= 16) hipLaunchKernelGGL(latent_out_kernel<4>, dim3(a.heads, (a.r.n_seq + 3) / 4, a.vp / OUT_COLS), dim3(256), 4 * a.rp * 4, s, a);
+  else hipLaunchKernelGGL(latent_out_kernel<1>, dim3(a.heads, a.r.n_seq, a.vp / OUT_COLS), dim3(256), 4 * a.rp * 4, s, a);
   return md_launch_status();
 }
