@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256) void latent_plain_kernel(const LmLatent a) {
     for (int r = 0; r < R; r += 4) y += *(const f32x4*)(z + r) * ld4(w + r);
     float o = ((y[0] + y[1]) + (y[2] + y[3])) / l;
     if (a.col_g >= 0) o *= sigmoid_f32(ldf(proj + a.col_g + h * a.vp + e));
-    stf((T*)a.out + (int64_t)row * a.ldo + h * a.vp + e, o);
+    stf((T*)a.out + (int64_t)row * a.ldo + in_chunks(h * a.vp + e, a.out_chunk), o);
   }
 }
 
@@ -272,10 +272,10 @@ __global__ __launch_bounds__(256, 2) void latent_prefill_kernel(const LmLatent a
       }
       st4(ot + l31 * M::OS + e0, v);
     }
-  bf16_t* out = (bf16_t*)a.out + (int64_t)row0 * a.ldo + h * vp;
+  bf16_t* out = (bf16_t*)a.out + (int64_t)row0 * a.ldo;
   for (int i = lane; i < 32 * (vp / 8); i += 64) {  // (the wave's own tile: its LDS operations are in order)
     const int rr = i / (vp / 8), e = (i - rr * (vp / 8)) * 8;
-    if (w0 + rr < len) *(u32x4*)(out + (int64_t)(w0 + rr) * a.ldo + e) = *(const u32x4*)(ot + rr * M::OS + e);
+    if (w0 + rr < len) *(u32x4*)(out + (int64_t)(w0 + rr) * a.ldo + in_chunks(h * vp + e, a.out_chunk)) = *(const u32x4*)(ot + rr * M::OS + e);
   }
 }
 
@@ -532,7 +532,7 @@ __global__ __launch_bounds__(256) void latent_out_kernel(const LmLatent a) {
   if (s >= SEQ || s0 + s >= a.r.n_seq) return;
   const int64_t row = a.r.seq_row0[s0 + s];
   if (a.col_g >= 0) v *= sigmoid_f32(bf2f(((const bf16_t*)a.proj)[row * a.ldp + a.col_g + h * a.vp + e]));
-  ((bf16_t*)a.out)[row * a.ldo + h * a.vp + e] = f2bf(v);
+  ((bf16_t*)a.out)[row * a.ldo + in_chunks(h * a.vp + e, a.out_chunk)] = f2bf(v);
 }
 
 typedef void (*LatentKernel)(const LmLatent);

@@ -416,7 +416,7 @@ __global__ __launch_bounds__(256) void attn_plain_kernel(const LmAttn a) {
     }
     __syncthreads();
   }
-  for (int c = tid; c < H * vp; c += 256) stf((T*)a.out + (int64_t)row * a.ldo + c, acc[c] / ls[c / vp]);
+  for (int c = tid; c < H * vp; c += 256) stf((T*)a.out + (int64_t)row * a.ldo + in_chunks(c, a.out_chunk), acc[c] / ls[c / vp]);
 }
 
 template <typename T, int NI>
@@ -830,9 +830,9 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void attn_mfma_kernel(const LmAttn
       const int pos = t0 + 4 * q + r;
       if (pos < lo || pos > hi) continue;
       const float inv = 1.0f / l[r];
-      bf16_t* dst = (bf16_t*)a.out + (int64_t)(row0 + pos - pos0) * a.ldo + h * vp + n;
+      bf16_t* dst = (bf16_t*)a.out + (int64_t)(row0 + pos - pos0) * a.ldo + in_chunks(h * vp + n, a.out_chunk);
 #pragma unroll
-      for (int t = 0; t < 2 * C; ++t) dst[16 * t] = f2bf(oacc[hh][t][r] * inv);
+      for (int t = 0; t < 2 * C; ++t) dst[2 * t * a.out_chunk] = f2bf(oacc[hh][t][r] * inv);
     }
   }
 }
@@ -871,10 +871,10 @@ __global__ __launch_bounds__(256) void attn_parts_kernel(const LmAttn a) {
     const int pos = t0 + 4 * q + r;
     if (pos < lo || pos > hi) continue;
     const float inv = 1.0f / l[r];
-    bf16_t* dst = (bf16_t*)a.out + (int64_t)(row0 + pos - pos0) * a.ldo + h * a.vp + n;
+    bf16_t* dst = (bf16_t*)a.out + (int64_t)(row0 + pos - pos0) * a.ldo + in_chunks(h * a.vp + n, a.out_chunk);
 #pragma unroll
     for (int t = 0; t < 8; ++t)
-      if (t < pieces) dst[16 * t] = f2bf(o[t][r] * inv);
+      if (t < pieces) dst[2 * t * a.out_chunk] = f2bf(o[t][r] * inv);
   }
 }
 
@@ -1139,7 +1139,7 @@ __global__ __launch_bounds__(64 * NWD, 2) void attn_decode_kernel(const LmAttn a
       o += __shfl_xor(o, 16, 64);
       o += __shfl_xor(o, 32, 64);
       if (q4 != 0) continue;
-      if (a.n_split == 1) ((bf16_t*)a.out)[(int64_t)row * a.ldo + h * vp + 16 * t + n16] = f2bf(o * inv);
+      if (a.n_split == 1) ((bf16_t*)a.out)[(int64_t)row * a.ldo + in_chunks(h * vp + 16 * t + n16, a.out_chunk)] = f2bf(o * inv);
       else part[h * vp + 16 * t + n16] = o;
     }
   }
@@ -1178,7 +1178,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const LmAttn a) {
   __syncthreads();
   if (tid >= a.vp) return;
   for (int k = 1; k < groups; ++k) o += sums[k * a.vp + e];
-  ((bf16_t*)a.out)[(int64_t)a.r.seq_row0[seq] * a.ldo + h * a.vp + e] = f2bf(o / l);
+  ((bf16_t*)a.out)[(int64_t)a.r.seq_row0[seq] * a.ldo + in_chunks(h * a.vp + e, a.out_chunk)] = f2bf(o / l);
 }
 
 }  // namespace

@@ -9,27 +9,31 @@
 // Weights go from memory to the matrix operand directly, used once, in whole cache lines (8 rows x 128 bytes per wave and load) with the
 // non-temporal policy: loads of 16 rows x 64 bytes, the operand's own shape, fetch half lines that are dropped before the other half is asked
 // for (4.9 TB/s of the 6.9 that a plain read reaches).  Activations are read directly too: with few rows they are a fraction of the weights'
-// bytes.  What one of these products makes for the next lies in the operand's order, [column / 8][row][8], so that a load takes consecutive memory.
+// bytes.  What a product or a mixer makes for the next one lies in the operand's order, [column / 8][row][8], so that a load takes consecutive memory
+// (rows 4 KB apart meet on few channels: output projection of 40 rows 9.9 us against 7.6).
 // Two register buffers per wave keep two batches of loads in flight.
 //
-// Measured, 2048 wide, 5440 feed-forward, one row (16 rows, 28 rows): 8192 columns 9.0 us (9.5, 10.9), 33 MB; gates 10.9 us (11.5, 14.3), 44 MB; the two
-// residual products 4.4 and 7.0 us (5.0 and 8.3; 6.0 and 11.0), 8 and 22 MB; the head, 51200 columns, 36 us (40, 57), 210 MB.  With half lines: gates 12.2 us
-// (15.9), head 47 us.  The tile products with K slices and their row-wise second launches took 12.8, 17.5 and 12.8 us.  About 4 us of every launch
-// are its start, the first loads and the sum over the waves.
+// Measured, 2048 wide, 5440 feed-forward, one row (16 rows, 28, 40): 8192 columns 8.5 us (8.4, 9.8, 11.2), 33 MB; gates 10.1 us (10.9, 12.3, 13.8), 44 MB;
+// the two residual products 4.7 and 6.9 us (5.4 and 8.7; 6.3 and 11.0; 7.4 and 13.0), 8 and 22 MB; the head, 51200 columns, 36 us (39, 48, 56),
+// 210 MB.  The tile products at 40 rows: gates 16.2 us, the residual products and their row-wise launches 13.3 us each, 4352 columns in K slices 12.5 us (10.5).
+// About 4 us of every launch are its start, the first loads and the sum over the waves.
 #include "lm_internal.hpp"
+
+#include <algorithm>
 
 namespace {
 
 constexpr int EPI_ROWS = 0, EPI_SILU = 1, EPI_RESID = 2;
 
-// W waves, MT 16-row tiles (0: up to 8 rows), U units of 64 of K per load batch.  A workgroup's columns are NX operands of 8; SiLU: 8 gates and the 8
-// inputs beside them.  A load is 8 rows x 128 bytes of weights, whole cache lines: the operand's upper 8 rows hold the other 32 of a unit's 64
+// W waves, MT 16-row tiles (0: up to 8 rows; others: the residual product), U units of 64 of K per load batch.  A workgroup's columns are NX operands of 8;
+// SiLU: 8 gates and the 8 inputs beside them.  A load is 8 rows x 128 bytes of weights, whole cache lines: the operand's upper 8 rows hold the other 32 of a unit's 64
 // of K.  It is multiplied with either half of the activations, and the useful half of either product is kept; up to 8 rows the two halves of
 // K of the activations fit one operand as well.  NX = 1: layers of so few columns that more would not fill the chip evenly.
 // S: streams of the residual epilogue (0: any count); otherwise 1: rows in order, 2: through rows_idx
 template <int MT, int NX, int W, int U, int EPI, int S>
 __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
   static_assert(EPI != EPI_SILU || NX == 2, "gates and inputs");
+  static_assert(EPI == EPI_RESID || MT == 0, "step_gemm_tall_kernel's");
   constexpr bool DIAG = MT == 0;
   constexpr int M16 = DIAG ? 1 : MT, TN = EPI == EPI_SILU ? 8 : 8 * NX;
   constexpr int PA = DIAG ? 1 : 2;  // operands of activations per unit, and accumulators per operand of weights
@@ -82,8 +86,7 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
     for (int s = 0; s < SM; ++s)
       if (s < ns) old[s] = *(const f32x4*)(xr + s * a.stride);
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (c + e < a.width) norm_w[e] = a.norm.w[(int64_t)(c + e) * a.norm.stride];
+    for (int e = 0; e < 4; ++e) norm_w[e] = a.norm.w[(int64_t)min(c + e, a.width - 1) * a.norm.stride];  // (columns beyond hold zeros)
   }
 
   u32x4 wf[2][U][NX], af[2][U][PA][M16];
@@ -159,12 +162,10 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
     for (int e = 0; e < 4; ++e) {
       if (NX == 1) {
         v[e] = acc[0][0][i][e] + __shfl(acc[0][PA - 1][i][e], DIAG ? lane ^ 40 : lane ^ 32, 64);
-      } else if (DIAG) {
+      } else {
         const float x = acc[0][0][i][e] + __shfl(acc[0][0][i][e], lane ^ 40, 64);
         const float y = __shfl(acc[NX - 1][0][i][e], lane ^ 32, 64) + __shfl(acc[NX - 1][0][i][e], lane ^ 8, 64);
         v[e] = g < 2 ? x : y;
-      } else {
-        v[e] = (g < 2 ? acc[0][0][i][e] : acc[NX - 1][PA - 1][i][e]) + __shfl(g < 2 ? acc[NX - 1][0][i][e] : acc[0][PA - 1][i][e], lane ^ 32, 64);
       }
     }
     red[wave][i][lane] = v;
@@ -220,34 +221,210 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
   }
 }
 
-template <int MT, int NX, int W, int U, int EPI, int S>
-md_status launch(const LmStepGemm& a, int n, hipStream_t s) {
-  hipLaunchKernelGGL((step_gemm_kernel<MT, NX, W, U, EPI, S>), dim3(n / (EPI == EPI_SILU ? 8 : 8 * NX)), dim3(64 * W), 0, s, a);
-  return md_launch_status();
-}
-template <int NX, int W, int U, int EPI, int S>
-md_status by_rows(const LmStepGemm& a, int n, hipStream_t s) {
-  return a.rows <= 8 ? launch<0, NX, W, U, EPI, S>(a, n, s) : a.rows <= 16 ? launch<1, NX, W, U, EPI, S>(a, n, s) : launch<2, NX, W, U, EPI, S>(a, n, s);
+// Rows and gates of more than 8 rows, operands of 16 columns (SiLU: an odd NX of operands with 8 gates and the 8 inputs beside them, or pairs of 16 gates
+// and 16 inputs).  Two loads of 8 rows x 128 bytes make an operand of either half of a unit's 64 of K: the lanes of the upper rows take their
+// pieces in the other order, so that a choice between the two loads by lane is all it takes; the second half's columns come out turned by 8
+// and are turned back behind the sums.  Half the matrix instructions and two thirds of the registers of the kernel above, which pay for more columns per
+// workgroup: what bounds it beside the weights is that every workgroup reads all activations (28 rows, gates: 680 workgroups of 8 columns 14.7 us, 227
+// of 24 13.0).  The waves' parts of K are dealt in turn: with the same part first on every CU, loads meet on the same channels (227 of 24: 12.3 us).
+// Batches of D units; more in flight, in deeper rings or all at once, changed nothing.
+template <int MT, int NX, int W, int D, int EPI, int S>
+__global__ __launch_bounds__(64 * W) void step_gemm_tall_kernel(const LmStepGemm a) {
+  constexpr int TN = EPI == EPI_SILU ? 8 * NX : 16 * NX;  // columns of the result
+  auto row_of = [&](int m) { return S == 2 ? a.rows_idx[m] : m; };
+  __shared__ f32x4 red[W][NX * MT][64];
+  __shared__ float row_scale[16 * MT];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, g = lane >> 4, upper = r >> 3;
+  const int n0 = blockIdx.x * TN;
+
+  constexpr int RR = (16 * MT + 4 * W - 1) / (4 * W);  // sums of squares: 16 lanes per row, rounds of 4 W rows, under way before the products
+  f32x4 sq[RR][4];
+#pragma unroll
+  for (int i = 0; i < RR; ++i)
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      const int m = min(i * 4 * W + (tid >> 4), a.rows - 1), c = h * 64 + r * 4;
+      const float* p = a.sumsq ? a.sumsq + (int64_t)row_of(m) * a.sumsq_n + min(c, a.sumsq_n - 4) : (const float*)a.w;
+      sq[i][h] = *(const f32x4*)p;
+    }
+
+  // load h of an operand: its rows 8 h .., the piece of a unit that this lane takes
+  const bf16_t* wp[NX][2];
+#pragma unroll
+  for (int x = 0; x < NX; ++x)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      // (the last workgroup's columns may go beyond the last one)
+      const int64_t first = EPI != EPI_SILU ? min(n0 + 16 * x + 8 * h, a.n - 8)
+                            : NX & 1      ? (int64_t)h * a.ff_pad + min(n0 + 8 * x, a.n - 8)
+                                          : (int64_t)(x & 1) * a.ff_pad + min(n0 + 16 * (x >> 1) + 8 * h, a.n - 8);
+      wp[x][h] = a.w + (first + (r & 7)) * a.k + 8 * (4 * (upper ^ h) + g);
+    }
+  const bf16_t* ap[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) ap[i] = a.a + (int64_t)row_of(min(16 * i + r, a.rows - 1)) * a.lda + g * a.chunk;
+  const int units = a.k >> 6, part = (wave + (int)(blockIdx.x >> 3)) % W, lo = units * part / W, hi = units * (part + 1) / W;
+  f32x4 acc[NX][2][MT];
+#pragma unroll
+  for (int x = 0; x < NX; ++x)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < MT; ++i) acc[x][h][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  u32x4 wf[D][NX][2], af[D][2][MT];
+  auto load = [&](int b, int u) {
+    const int k = u * 64, kc = k / 8 * a.chunk;
+#pragma unroll
+    for (int x = 0; x < NX; ++x)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) wf[b][x][h] = __builtin_nontemporal_load((const u32x4*)(wp[x][h] + k));
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < MT; ++i) af[b][h][i] = *(const u32x4*)(ap[i] + kc + 4 * h * a.chunk);
+  };
+  auto multiply = [&](int b) {
+#pragma unroll
+    for (int x = 0; x < NX; ++x)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        u32x4 w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = upper ? wf[b][x][1 - h][e] : wf[b][x][h][e];
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+          acc[x][h][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(md_bf16x8v, w), __builtin_bit_cast(md_bf16x8v, af[b][h][i]), acc[x][h][i], 0, 0, 0);
+      }
+  };
+  const int last = max(hi - 1, 0);
+  auto load_batch = [&](int u) {  // past the end: the last one again, not used
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(d, min(u + d, last));
+  };
+  auto multiply_batch = [&](int u) {
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (u + d < hi) multiply(d);
+  };
+  load_batch(lo);
+  __builtin_amdgcn_sched_barrier(0);
+  float factor[RR];
+#pragma unroll
+  for (int i = 0; i < RR; ++i) {
+    f32x4 q = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+      if (h * 64 + r * 4 < a.sumsq_n) q += sq[i][h];
+    factor[i] = (q[0] + q[1]) + (q[2] + q[3]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  multiply_batch(lo);
+  for (int u = lo + D; u < hi; u += D) {
+    load_batch(u);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply_batch(u);
+  }
+#pragma unroll
+  for (int i = 0; i < RR; ++i) {
+    const int m = i * 4 * W + (tid >> 4);
+    if (a.sumsq)
+      for (int c = 256 + r * 4; c < a.sumsq_n; c += 64) {  // (widths above 2048)
+        const f32x4 q = *(const f32x4*)(a.sumsq + (int64_t)row_of(min(m, a.rows - 1)) * a.sumsq_n + c);
+        factor[i] += (q[0] + q[1]) + (q[2] + q[3]);
+      }
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) factor[i] += __shfl_xor(factor[i], o, 64);
+    if (r == 0 && m < 16 * MT) row_scale[m] = a.sumsq ? 1.0f / sqrtf(factor[i] / (float)a.width + a.eps) : 1.0f;
+  }
+#pragma unroll
+  for (int x = 0; x < NX; ++x)
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = acc[x][0][i][e] + __shfl(acc[x][1][i][e], lane ^ 32, 64);
+      red[part][x * MT + i][lane] = v;
+    }
+  __syncthreads();
+
+  // a lane holds four columns of one row: m = 16 i + (lane & 15), columns 4 (lane >> 4) .. of the operand's
+  auto total = [&](int t, int l) {
+    f32x4 v = red[0][t][l];
+#pragma unroll
+    for (int w = 1; w < W; ++w) v += red[w][t][l];
+    return v;
+  };
+  if (EPI == EPI_ROWS) {
+    for (int t = wave; t < NX * MT; t += W) {
+      const int m = 16 * (t % MT) + r, c = n0 + 16 * (t / MT) + 4 * g;
+      if (m >= a.rows || c >= a.n) continue;
+      f32x4 v = total(t, lane) * row_scale[m];
+      if (a.bias) v += ld4(a.bias + c);
+      st4(a.out + (int64_t)m * a.ldo + c, v);
+    }
+  } else {
+    constexpr int PAIRS = NX & 1 ? NX : NX / 2;
+    for (int t = wave; t < PAIRS * MT; t += W) {
+      const int x = t / MT, i = t % MT, m = 16 * i + r, c = n0 + (NX & 1 ? 8 : 16) * x + 4 * g;
+      if (m >= a.rows || c >= a.n || (NX & 1 && g >= 2)) continue;
+      const float s = row_scale[m];
+      const f32x4 z = total(NX & 1 ? t : 2 * x * MT + i, lane) * s, u = (NX & 1 ? total(t, lane + 32) : total((2 * x + 1) * MT + i, lane)) * s;
+      f32x4 y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = silu_fast(z[e]) * u[e];
+      st4(a.out + (c >> 3) * a.out_chunk + m * 8 + (c & 7), y);
+    }
+  }
 }
 
-// Columns and waves of a workgroup.  More than four workgroups of 16 columns per CU: two waves (51200 columns, 1 / 12 / 28 rows: 36 / 40 / 57 us; four waves
-// 36 / 41 / 58, eight 39 / 48 / 76).  Up to 8 rows, where a unit's activations are one load: 8 columns where that evens out few workgroups (6144
-// columns, 8 rows: 7.5 us against 8.0; 8192: 9.5 against 8.7), eight waves to share K otherwise.
+template <int MT, int NX, int W, int U, int EPI, int S>
+md_status launch(const LmStepGemm& a, hipStream_t s) {
+  hipLaunchKernelGGL((step_gemm_kernel<MT, NX, W, U, EPI, S>), dim3(a.n / (EPI == EPI_SILU ? 8 : 8 * NX)), dim3(64 * W), 0, s, a);
+  return md_launch_status();
+}
+template <int NX, int W, int EPI, int S>
+md_status tall(const LmStepGemm& a, hipStream_t s) {
+  constexpr int TN = EPI == EPI_SILU ? 8 * NX : 16 * NX;
+  const dim3 grid((a.n + TN - 1) / TN), block(64 * W);
+  if (a.rows <= 16) hipLaunchKernelGGL((step_gemm_tall_kernel<1, NX, W, 2, EPI, S>), grid, block, 0, s, a);
+  else if (a.rows <= 32) hipLaunchKernelGGL((step_gemm_tall_kernel<2, NX, W, 2, EPI, S>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((step_gemm_tall_kernel<3, NX, W, 2, EPI, S>), grid, block, 0, s, a);
+  return md_launch_status();
+}
+// As many operands per workgroup as leave the fullest of the 256 CUs with the fewest columns, the larger number where that is the same (40 rows, gates
+// of 5440: 1, 2, 3 operands 18.7, 18.2, 13.8 us; 8192 columns: 15.5, 11.2, 13.0; 4352: 14.2, 10.5, 12.5)
+template <int EPI, int S>
+md_status tall_by_columns(const LmStepGemm& a, hipStream_t s) {
+  auto most = [&](int nx) {
+    const int tn = (EPI == EPI_SILU ? 8 : 16) * nx;
+    return ((a.n + tn - 1) / tn + 255) / 256 * nx;
+  };
+  if (most(3) <= std::min(most(1), most(2))) return tall<3, 8, EPI, S>(a, s);
+  return most(2) <= most(1) ? tall<2, 8, EPI, S>(a, s) : tall<1, 8, EPI, S>(a, s);
+}
+
+// Columns and waves of a workgroup.  Up to 8 rows, where a unit's activations are one load: 8 columns where that evens out few workgroups (6144
+// columns, 8 rows: 7.5 us against 8.0; 8192: 9.5 against 8.7), eight waves to share K otherwise.  More than four workgroups of 16 columns per CU: fewer
+// waves (51200 columns, 1 row: two waves 36 us, eight 39; 28 / 40 rows: 32 columns to four waves 48 / 56 us, to eight 59 / 69).
 template <int S>
-md_status rows(const LmStepGemm& a, int n, hipStream_t s) {
-  auto most = [&](int tn) { return (n / tn + 255) / 256 * tn; };  // columns that the fullest of the 256 CUs gets
-  if (n > 256 * 64) return by_rows<2, 2, 1, EPI_ROWS, S>(a, n, s);
-  if (a.rows > 8) return by_rows<2, 4, 2, EPI_ROWS, S>(a, n, s);
-  return n <= 256 * 32 && most(8) < most(16) ? launch<0, 1, 4, 2, EPI_ROWS, S>(a, n, s) : launch<0, 2, 8, 1, EPI_ROWS, S>(a, n, s);
+md_status rows(const LmStepGemm& a, hipStream_t s) {
+  auto most = [&](int tn) { return (a.n / tn + 255) / 256 * tn; };  // columns that the fullest of the 256 CUs gets
+  const bool many = a.n > 256 * 64;
+  if (a.rows > 8) return many ? tall<2, 4, EPI_ROWS, S>(a, s) : tall_by_columns<EPI_ROWS, S>(a, s);
+  if (many) return launch<0, 2, 2, 1, EPI_ROWS, S>(a, s);
+  return a.n <= 256 * 32 && most(8) < most(16) ? launch<0, 1, 4, 2, EPI_ROWS, S>(a, s) : launch<0, 2, 8, 1, EPI_ROWS, S>(a, s);
 }
 
 // Up to 8 rows four units per batch where K is long (5440: 6.8 us against 7.7; 2048: 4.4 either way)
 template <int S>
 md_status resid(const LmStepGemm& a, hipStream_t s) {
-  return a.rows <= 8 && a.k > 4096 ? launch<0, 1, 8, 4, EPI_RESID, S>(a, a.width_pad, s) : by_rows<1, 8, 2, EPI_RESID, S>(a, a.width_pad, s);
+  if (a.rows <= 8) return a.k > 4096 ? launch<0, 1, 8, 4, EPI_RESID, S>(a, s) : launch<0, 1, 8, 2, EPI_RESID, S>(a, s);
+  return a.rows <= 16 ? launch<1, 1, 8, 2, EPI_RESID, S>(a, s) : a.rows <= 32 ? launch<2, 1, 8, 1, EPI_RESID, S>(a, s) : launch<3, 1, 8, 1, EPI_RESID, S>(a, s);
 }
 
-static_assert(LM_STEP_ROWS <= 32, "two row tiles");
+static_assert(LM_STEP_ROWS <= 48, "three row tiles");
 inline bool takes(const LmStepGemm& a) {
   return a.rows >= 1 && a.rows <= LM_STEP_ROWS && a.k >= 64 && a.k % 64 == 0 && a.lda % 8 == 0 && a.chunk % 8 == 0 &&
          (((uintptr_t)a.a | (uintptr_t)a.w | (uintptr_t)a.out) & 15) == 0;
@@ -255,18 +432,24 @@ inline bool takes(const LmStepGemm& a) {
 
 }  // namespace
 
-md_status lm_step_rows(const LmStepGemm& a, int n, hipStream_t s) {
-  MD_CHECK_ARG(takes(a) && n % 64 == 0 && a.ldo % 4 == 0);
-  return a.rows_idx ? rows<2>(a, n, s) : rows<1>(a, n, s);
+md_status lm_step_rows(const LmStepGemm& g, int n, hipStream_t s) {
+  MD_CHECK_ARG(takes(g) && n % 64 == 0 && g.ldo % 4 == 0);
+  LmStepGemm a = g;
+  a.n = n;
+  return a.rows_idx ? rows<2>(a, s) : rows<1>(a, s);
 }
 
-md_status lm_step_silu(const LmStepGemm& a, hipStream_t s) {
-  MD_CHECK_ARG(takes(a) && a.ff_pad % 64 == 0);
-  return by_rows<2, 2, 1, EPI_SILU, 1>(a, a.ff_pad, s);
+md_status lm_step_silu(const LmStepGemm& g, hipStream_t s) {
+  MD_CHECK_ARG(takes(g) && g.ff_pad % 64 == 0);
+  LmStepGemm a = g;
+  a.n = a.ff_pad;
+  return a.rows <= 8 ? launch<0, 2, 2, 1, EPI_SILU, 1>(a, s) : tall_by_columns<EPI_SILU, 1>(a, s);
 }
 
-md_status lm_step_resid(const LmStepGemm& a, hipStream_t s) {
-  MD_CHECK_ARG(takes(a) && a.width_pad % 64 == 0 && a.streams >= 1 && a.streams <= MD_LM_MAX_STREAMS);
+md_status lm_step_resid(const LmStepGemm& g, hipStream_t s) {
+  MD_CHECK_ARG(takes(g) && g.width_pad % 64 == 0 && g.streams >= 1 && g.streams <= MD_LM_MAX_STREAMS);
+  LmStepGemm a = g;
+  a.n = a.width_pad;
   switch (a.streams) {
     case 1: return resid<1>(a, s);
     case 2: return resid<2>(a, s);

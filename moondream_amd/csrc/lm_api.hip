@@ -40,10 +40,6 @@ struct LmWs {
 
 inline bool decode_regime(const md_lm_model* m, int rows) { return m->dtype == MD_DTYPE_BF16 && rows <= DECODE_ROWS; }
 
-// Most logits that gemm_step.hip's product makes of rows picked through an index (51200 columns; 1 row: 36 us against 50 of the tiles with the norm's
-// launch, 12 rows: 40 against 52, but 17 and 24 rows: 62 and 64 against 53 and 55).  Rows in order, as a decode step has them: 20 rows 52, 28 rows 58.
-constexpr int STEP_PICKED_ROWS = 16;
-
 // products that go on with the row-wise step behind them (gemm_step.hip)
 // (a router needs whole normed rows, which leaves nothing to go on with; and the first token's retention is its value times q . k, normed: only
 // the sign of q . k is left, so a rounding of the norm at another place turns it over where q . k is small.  A step in which any sequence may
@@ -402,7 +398,8 @@ struct Step {
     a.ctx = st->ctx;
     a.q = w.q;
     a.out = w.att;
-    a.ldo = l.out_proj.k_pad;
+    a.ldo = few ? 8 : l.out_proj.k_pad;
+    a.out_chunk = few ? 8 * b->n_rows : 8;
     a.part = w.attn_part;
     const int span = l.chunk > 0 ? std::min(l.chunk, b->max_ctx) : b->max_ctx;
     if (m->dtype == MD_DTYPE_BF16 && b->max_len == 1 && (g_lm_kernels & 2) && lm_attn_decode_takes(a)) {
@@ -430,7 +427,8 @@ struct Step {
     a.rot_dims = l.rot_dims;
     a.state = st->layers[i].ret;
     a.out = w.att;
-    a.ldo = l.out_proj.k_pad;
+    a.ldo = few ? 8 : l.out_proj.k_pad;
+    a.out_chunk = few ? 8 * b->n_rows : 8;
     a.qf = w.qf; a.kf = w.kf; a.of = w.of;
     a.chunk_state = w.chunk_state;
     a.n_chunk_max = (b->max_len + LM_RET_CHUNK - 1) / LM_RET_CHUNK;
@@ -456,7 +454,8 @@ struct Step {
     a.cache = st->layers[i].k;
     a.ctx = st->ctx;
     a.out = w.att;
-    a.ldo = l.out_proj.k_pad;
+    a.ldo = few ? 8 : l.out_proj.k_pad;
+    a.out_chunk = few ? 8 * b->n_rows : 8;
     a.ctx_rows = b->ctx_rows;
     a.seq_ctx0 = b->seq_ctx0;
     a.c_rows = w.c_rows; a.kv = w.kv; a.q_lat = w.q_lat; a.part = w.latent_part;
@@ -486,7 +485,8 @@ struct Step {
     a.conv_state = st->layers[i].conv;
     a.state = st->layers[i].ret;
     a.out = w.att;
-    a.ldo = l.out_proj.k_pad;
+    a.ldo = few ? 8 : l.out_proj.k_pad;
+    a.out_chunk = few ? 8 * b->n_rows : 8;
     a.u = w.conv_out; a.dt = w.dt; a.seg = w.seg; a.seg_decay = w.seg_decay;
     if (m->dtype == MD_DTYPE_BF16) {
       if (b->max_len == 1 && (g_lm_kernels & 2) && lm_ssm_decode_takes(a)) return lm_ssm_decode(a, s);
@@ -588,7 +588,7 @@ struct Step {
     const int64_t row_floats = (int64_t)b->n_rows * m->width_pad;
     if (own_row_steps(m)) MD_TRY(lm_embed_streams(m, b->tokens, b->row_pos, w.x, row_floats, b->n_rows, s));
     else MD_TRY(lm_embed(m->dtype, m->embed, m->width_pad, b->tokens, w.x, b->n_rows, m->vocab, s));
-    const bool few_logits = n_logits > 0 && n_logits <= (logit_rows ? STEP_PICKED_ROWS : LM_STEP_ROWS);
+    const bool few_logits = n_logits > 0 && n_logits <= LM_STEP_ROWS;
     for (int i = 0; i < m->n_layers; ++i) {
       const md_lm_layer& l = m->layers[i];
       // what follows this layer: the next one's mixer, or the head
@@ -600,11 +600,11 @@ struct Step {
       if (l.out_proj.k_pad != l.heads * l.vdim_pad) MD_TRY(zero_fill(w.att, (size_t)b->n_rows * l.out_proj.k_pad * esize(m), s));
       MD_TRY(mixer(i));
       if (l.ff > 0) {
-        MD_TRY(finish(w.att, l.out_proj.k_pad, l.out_proj, false, l.mix1, l.norm2, l.mix2));
+        MD_TRY(finish(w.att, l.out_proj.k_pad, l.out_proj, few, l.mix1, l.norm2, l.mix2));
         MD_TRY(input(l.norm2, l.mix2));
         MD_TRY(feed_forward(l, nw, next));
       } else {
-        MD_TRY(finish(w.att, l.out_proj.k_pad, l.out_proj, false, l.mix1, nw, next));
+        MD_TRY(finish(w.att, l.out_proj.k_pad, l.out_proj, few, l.mix1, nw, next));
       }
       if (layer_out) MD_TRY(tap(layer_out + i * row_floats));
     }

@@ -34,6 +34,10 @@ __device__ __forceinline__ void st8(float* p, f32x4 a, f32x4 b) {
   st4(p + 4, b);
 }
 
+// where column c lies in a row whose groups of 8 columns are `chunk` elements apart: 8 in plain rows, 8 * rows in the order of the matrix operand
+// that the products of few rows read (gemm_step.hip)
+__device__ __forceinline__ int in_chunks(int c, int chunk) { return (c >> 3) * chunk + (c & 7); }
+
 __device__ __forceinline__ float silu_f32(float z) { return z / (1.0f + expf(-z)); }
 template <typename T>
 __device__ __forceinline__ float silu_for(float z) {
@@ -103,8 +107,9 @@ struct LmAttn {
   void* conv_state;
   int ctx;
   void* q;         // [n_rows][heads * dp]: normed queries
-  void* out;       // [n_rows][ldo]
+  void* out;       // in_chunks(column, out_chunk) of rows ldo apart
   int64_t ldo;
+  int out_chunk;
   float* part;     // split keys: partial (m, l) and accumulators
   int n_split, split_keys;
 };
@@ -121,6 +126,7 @@ struct LmRet {
   float* state;    // [slots][heads][vp][dp]
   void* out;
   int64_t ldo;
+  int out_chunk;
   float *qf, *kf;  // plain kernels: rotated q and k, [n_rows][heads * dp]
   float* of;       // plain kernels: unnormed outputs, [n_rows][heads * vp]
   float* chunk_state;  // matrix-core prefill: state at the start of every chunk
@@ -141,6 +147,7 @@ struct LmLatent {
   int ctx;
   void* out;
   int64_t ldo;
+  int out_chunk;
   // prefill on the matrix cores: latent rows of every position of the step's sequences, packed by seq_ctx0, and what they expand to
   int ctx_rows;
   const int32_t* seq_ctx0;
@@ -163,6 +170,7 @@ struct LmSsm {
   float* state;          // [slots][heads][vp][dp]
   void* out;
   int64_t ldo;
+  int out_chunk;
   void* u;               // [n_rows][cw]: x | B | C behind the convolution and silu
   float* dt;             // [n_rows][heads], behind softplus
   float *seg, *seg_decay;  // matrix-core prefill in segments: [n_seq][n_seg][heads][vp][dp], [n_seq][n_seg][heads]
@@ -209,10 +217,10 @@ struct LmRoute {
 
 // A product of a step of few rows and what follows it (gemm_step.hip).  Rows that a residual epilogue wrote carry no norm factor: it
 // comes from their sums of squares (sumsq; nullptr: the rows are complete).
-// Up to how many rows they are ahead: a step of 24 layers against the one of tile products and row-wise launches, 24 / 28 / 32 rows: 0.92 / 0.95 / 0.98 of
-// its time with attention and retention (1732, 1802, 1855 us with 32 heads of 64; the same with 16 of 128), 0.97 / 1.00 / 1.03 with state space and
-// latent attention (1641, 1720, 1773 us; the same with 16 of 128); 17 rows 0.88 and 0.92, one row 0.72 and 0.74.
-constexpr int LM_STEP_ROWS = 28;
+// Up to how many rows they are ahead: a step of 24 layers against the one of tile products and row-wise launches, 20 / 28 / 32 / 40 / 48 rows: 0.81 / 0.81 /
+// 0.84 / 0.90 / 0.94 of its time with state space and latent attention (1301, 1409, 1469, 1614, 1729 us with 32 heads of 64; 0.81 to 0.92 with 16 of 128),
+// 0.84 / 0.83 / 0.81 / 0.86 / 0.89 with attention and retention (1431, 1531, 1593, 1734, 1857 us).  At 64 rows gates would take 18.2 us against 16.3.
+constexpr int LM_STEP_ROWS = 48;
 struct LmStepGemm {
   const bf16_t* a;       // row m's columns 8 c .. 8 c + 7 at m * lda + c * chunk (plain rows: chunk 8)
   int64_t lda;
@@ -228,7 +236,7 @@ struct LmStepGemm {
   int64_t ldo;
   int out_chunk;         // = 8 * rows
   const bf16_t* bias;
-  int ff_pad;            // SiLU gate: rows 0 .. of w are the gates, ff_pad .. the inputs
+  int n, ff_pad;         // columns of the result; SiLU gate: rows 0 .. of w are the gates, ff_pad .. the inputs
   // residual epilogue: streams, weights around this sublayer and of the next one (nullptr: plain sum), as in LmStreams
   float* x;
   int64_t stride;

@@ -129,8 +129,8 @@ __global__ __launch_bounds__(256) void ret_out_kernel(const LmRet a) {
     for (int d = lane; d < a.vp; d += 64) ss += o[d] * o[d];
     const float r = 1.0f / sqrtf(wave_sum(ss) / (float)a.vdim + a.eps);
     const T* g = (const T*)a.proj + (int64_t)row * a.ldp + a.col_g + h * a.vp;
-    T* dst = (T*)a.out + (int64_t)row * a.ldo + h * a.vp;
-    for (int d = lane; d < a.vp; d += 64) stf(dst + d, o[d] * r * silu_f32(ldf(g + d)));
+    T* dst = (T*)a.out + (int64_t)row * a.ldo;
+    for (int d = lane; d < a.vp; d += 64) stf(dst + in_chunks(h * a.vp + d, a.out_chunk), o[d] * r * silu_f32(ldf(g + d)));
   }
 }
 
@@ -393,11 +393,11 @@ __global__ __launch_bounds__(256) void ret_chunk_kernel(const LmRet a) {
     if (tt >= n) continue;
     const float rn = 1.0f / sqrtf(ss[e] / (float)a.vdim + a.eps);
     const bf16_t* g = base + (int64_t)tt * a.ldp + a.col_g + h * vp + 2 * C * r;
-    bf16_t* dst = (bf16_t*)a.out + (int64_t)(row0 + c * RC + tt) * a.ldo + h * vp + 2 * C * r;
+    bf16_t* dst = (bf16_t*)a.out + (int64_t)(row0 + c * RC + tt) * a.ldo;
 #pragma unroll
     for (int i = 0; i < C; ++i) {
       const uint32_t gg = *(const uint32_t*)(g + 2 * i);
-      *(uint32_t*)(dst + 2 * i) = pack_bf16x2(o[2 * i][e] * rn * silu_f32(lo_bf(gg)), o[2 * i + 1][e] * rn * silu_f32(hi_bf(gg)));
+      *(uint32_t*)(dst + in_chunks(h * vp + 2 * C * r + 2 * i, a.out_chunk)) = pack_bf16x2(o[2 * i][e] * rn * silu_f32(lo_bf(gg)), o[2 * i + 1][e] * rn * silu_f32(hi_bf(gg)));
     }
   }
 }
@@ -473,7 +473,7 @@ __global__ __launch_bounds__(256) void ret_decode_kernel(const LmRet a) {
   __syncthreads();
   const float o = tid < vp ? os[tid] : 0.f;
   const float ss = block_sum_256(o * o, red);
-  if (tid < vp) ((bf16_t*)a.out)[(int64_t)row * a.ldo + h * vp + tid] = f2bf(o / sqrtf(ss / (float)a.vdim + a.eps) * silu_f32(gate));
+  if (tid < vp) ((bf16_t*)a.out)[(int64_t)row * a.ldo + in_chunks(h * vp + tid, a.out_chunk)] = f2bf(o / sqrtf(ss / (float)a.vdim + a.eps) * silu_f32(gate));
 }
 template <int R>
 RetKernel ret_decode_by_width(int dp) {

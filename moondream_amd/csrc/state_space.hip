@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(const LmSsm a) {
       if (l == 0) os[t][col] = sum + skip * x;
     }
     __syncthreads();
-    if (col < n) stf((T*)a.out + (int64_t)(row0 + t0 + col) * a.ldo + h * vp + e0 + l, os[col][l] * silu_f32(zs[col][l]));
+    if (col < n) stf((T*)a.out + (int64_t)(row0 + t0 + col) * a.ldo + in_chunks(h * vp + e0 + l, a.out_chunk), os[col][l] * silu_f32(zs[col][l]));
   }
 #pragma unroll
   for (int i = 0; i < Q; ++i) {
@@ -255,10 +255,11 @@ __global__ __launch_bounds__(256) void ssm_norm_kernel(const LmSsm a) {
       const int f = k * gs + i, h = f / a.vdim;
       return h * a.vp + f - h * a.vdim;
     };
+    auto at = [&](int c) { return row + in_chunks(c, a.out_chunk); };
     const int first = (BLOCK ? threadIdx.x : lane) * V, step = (BLOCK ? 256 : 64) * V;
     float ss = 0.f;
     for (int i = first; i < gs; i += step) {
-      const T* p = row + column(i);
+      const T* p = at(column(i));
       if (V == 4) {
         const f32x4 v = ld4(p);
         ss += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
@@ -270,8 +271,8 @@ __global__ __launch_bounds__(256) void ssm_norm_kernel(const LmSsm a) {
     const float r = 1.0f / sqrtf(ss / (float)gs + a.eps);
     for (int i = first; i < gs; i += step) {
       const int c = column(i);
-      if (V == 4) st4(row + c, ld4(row + c) * r * *(const f32x4*)(a.out_norm + c));
-      else stf(row + c, ldf(row + c) * r * a.out_norm[c]);
+      if (V == 4) st4(at(c), ld4(at(c)) * r * *(const f32x4*)(a.out_norm + c));
+      else stf(at(c), ldf(at(c)) * r * a.out_norm[c]);
     }
   }
 }
@@ -458,14 +459,14 @@ __global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ssm_chunk_kernel(const
       if (t < n) {
         const int64_t row = row0 + t0 + t;
         const bf16_t* z = (const bf16_t*)a.proj + row * a.ldp + a.col_z + h * vp;
-        bf16_t* dst = (bf16_t*)a.out + row * a.ldo + h * vp;
+        bf16_t* dst = (bf16_t*)a.out + row * a.ldo;
 #pragma unroll
         for (int i = 0; i < PT; ++i) {
           const f32x4 x = ld4(X + t * XS + 16 * i + 4 * q), zz = ld4(z + 16 * i + 4 * q);
           f32x4 y = o[i] + skip * x;
 #pragma unroll
           for (int e = 0; e < 4; ++e) y[e] *= silu_fast(zz[e]);
-          st4(dst + 16 * i + 4 * q, y);
+          st4(dst + in_chunks(h * vp + 16 * i + 4 * q, a.out_chunk), y);
         }
       }
     }
@@ -622,7 +623,7 @@ __global__ __launch_bounds__(256) void ssm_decode_kernel(const LmSsm a) {
   }
   __syncthreads();
   for (int e = tid; e < vp; e += 256)
-    ((bf16_t*)a.out)[(int64_t)row * a.ldo + h * vp + e] = f2bf(out[e] * silu_f32(bf2f(p[a.col_z + h * vp + e])));
+    ((bf16_t*)a.out)[(int64_t)row * a.ldo + in_chunks(h * vp + e, a.out_chunk)] = f2bf(out[e] * silu_f32(bf2f(p[a.col_z + h * vp + e])));
 }
 
 template <int C>

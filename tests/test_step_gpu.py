@@ -101,6 +101,32 @@ def test_rows_of_wide_models(width):
             m.close_sequence(s)
 
 
+WIDE = [U.stream_config([(U.ssm(m, 32, 32), U.dense(ff)), (U.latent(4, 32, 32, 64), U.dense(96))], width=64, vocab=v, positions=8)
+        for m, ff, v in ((8, 2112, 120), (64, 2120, 200), (130, 4168, 120), (128, 6208, 16500))]
+
+
+@pytest.mark.parametrize("cfg", WIDE, ids=["gates", "pairs", "threes", "many"])
+def test_columns_of_a_workgroup(cfg):
+    """Products whose workgroups own one, two and three operands of columns, the last one fewer, at the edges of the row tiles."""
+    m, w = build(cfg), U.weights(cfg, 3, 1.5)
+    ts = [U.tokens(2, cfg["vocab"], i) for i in range(49)]
+    want = torch.stack([O.forward(cfg, w, t) for t in ts])
+    for n in (9, 16, 17, 32, 33, 48, 49):
+        slots = [m.open_sequence() for _ in range(n)]
+        for k in range(2):
+            got = m.step([(s, [t[k]], [0]) for s, t in zip(slots, ts)])
+            assert float(U.logit_errors(got, want[:n, k]).max()) < 7e-2, (n, k)
+        for s in slots:
+            m.close_sequence(s)
+    # a prompt and sequences that go on, logits of some rows in another order
+    t = U.tokens(7, cfg["vocab"], 77)
+    slots = [m.open_sequence() for _ in range(30)]
+    for k in range(2):
+        got = m.step([(s, [x[k]], [0]) for s, x in zip(slots, ts)] + ([(m.open_sequence(), t, [5, 0, 6])] if k else []))
+    assert float(U.logit_errors(got[:30], want[:30, 1]).max()) < 7e-2
+    assert float(U.logit_errors(got[30:], O.forward(cfg, w, t)[[5, 0, 6]]).max()) < 7e-2
+
+
 @pytest.mark.parametrize("rows", [3, 40, 200])
 @pytest.mark.parametrize("which", ["in_proj", "out_proj", "gate_up", "down", "head"])
 def test_misaligned_weights_are_refused(rows, which):
