@@ -121,7 +121,8 @@ __global__ __launch_bounds__(64 * W) void expert_gemm_kernel(const LmExpertGemm 
       const int64_t out = (int64_t)list[m] * a.ldo + n0 + 4 * g;
       if (EPI == EPI_SILU) {
         if (wave) continue;
-        const f32x4 z = total(0), u = total(1);
+        const float s = a.factor ? a.factor[list[m] / a.per] : 1.0f;
+        const f32x4 z = total(0) * s, u = total(1) * s;
         f32x4 y;
 #pragma unroll
         for (int e = 0; e < 4; ++e) y[e] = silu_fast(z[e]) * u[e];

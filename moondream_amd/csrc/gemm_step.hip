@@ -192,7 +192,7 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
     f32x4 y;
 #pragma unroll
     for (int e = 0; e < 4; ++e) y[e] = silu_fast(z[e]) * u[e];
-    st4(a.out + (c >> 3) * a.out_chunk + m * 8 + (c & 7), y);
+    st4(a.out + m * a.ldo + in_chunks(c, a.out_chunk), y);
   } else {
     const float *in_w = a.next, *out_w = a.prev ? a.prev + ns : nullptr, *mix = a.prev ? a.prev + 2 * ns : nullptr;
     const f32x4 y = total(lane);
@@ -215,7 +215,7 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
     float q = (u[0] * u[0] + u[1] * u[1]) + (u[2] * u[2] + u[3] * u[3]);
     q += __shfl_xor(q, 16, 64);  // (the two quarters of the 8 columns)
     if (live) {
-      st4(a.out + (c >> 3) * a.out_chunk + m * 8 + (c & 7), u * norm_w);
+      st4(a.out + m * a.ldo + in_chunks(c, a.out_chunk), u * norm_w);
       if (g == 0) a.sumsq_out[(int64_t)m * (a.width_pad / 8) + blockIdx.x] = q;
     }
   }
@@ -374,7 +374,7 @@ __global__ __launch_bounds__(64 * W) void step_gemm_tall_kernel(const LmStepGemm
       f32x4 y;
 #pragma unroll
       for (int e = 0; e < 4; ++e) y[e] = silu_fast(z[e]) * u[e];
-      st4(a.out + (c >> 3) * a.out_chunk + m * 8 + (c & 7), y);
+      st4(a.out + m * a.ldo + in_chunks(c, a.out_chunk), y);
     }
   }
 }

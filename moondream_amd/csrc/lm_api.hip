@@ -10,6 +10,7 @@
 // Experts:  router + choice | rows grouped by expert | grouped gate/up product with silu(gate) * up | grouped down product; the weighted sum
 //   of a row's experts is taken by the row-wise step that follows, as the sums of K-slice partials are.  Few rows per expert: gemm_experts.hip's
 //   products, which take the choices as they are.
+//   A step of few rows norms nothing whole there either: the router and the experts' first product take the rows' factors themselves.
 // Residual streams:  the row-wise step between two sublayers mixes them (streams.hip); x is then [streams][rows][width_pad].
 #include "gemm_internal.hpp"
 #include "lm_internal.hpp"
@@ -30,7 +31,7 @@ struct LmWs {
   char *h, *proj, *q, *att, *y, *gu, *act;
   float *part, *qf, *kf, *of, *chunk_state, *attn_part;
   char *c_rows, *kv, *q_lat, *conv_out;
-  float *latent_part, *dt, *seg, *seg_decay, *route_weight, *sumsq;
+  float *latent_part, *dt, *seg, *seg_decay, *route_weight, *sumsq, *row_factor;
   int32_t *chosen, *slot_of, *row_of, *offsets;
   void* splitk;
   size_t splitk_bytes;
@@ -41,14 +42,15 @@ struct LmWs {
 inline bool decode_regime(const md_lm_model* m, int rows) { return m->dtype == MD_DTYPE_BF16 && rows <= DECODE_ROWS; }
 
 // products that go on with the row-wise step behind them (gemm_step.hip)
-// (a router needs whole normed rows, which leaves nothing to go on with; and the first token's retention is its value times q . k, normed: only
+// (Experts: where their own products take the step.  The first token's retention is its value times q . k, normed: only
 // the sign of q . k is left, so a rounding of the norm at another place turns it over where q . k is small.  A step in which any sequence may
 // begin keeps the rounding of long prompts where a layer has retention: 12 tokens 1.78 ms, 1.29 this way.  Their sums and gates take no bias.)
 inline bool step_regime(const md_lm_model* m, const md_lm_batch* b) {
   if (m->dtype != MD_DTYPE_BF16 || b->n_rows > LM_STEP_ROWS) return false;
   for (int i = 0; i < m->n_layers; ++i) {
     const md_lm_layer& l = m->layers[i];
-    if (l.experts > 0 || l.out_proj.b || (l.ff > 0 && (l.gate_up.b || l.down.b))) return false;
+    if (l.experts > 0 && !lm_expert_step_takes(b->n_rows, l.top, l.experts)) return false;
+    if (l.out_proj.b || (l.ff > 0 && (l.gate_up.b || l.down.b))) return false;
     if (b->n_going != b->n_seq && l.mixer == MD_MIXER_RETENTION) return false;
   }
   return true;
@@ -167,6 +169,7 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
   w.row_of = (int32_t*)a.take(slots * 4);
   w.offsets = (int32_t*)a.take(slots ? (experts + 1) * 4 : 0);
   w.sumsq = (float*)a.take(m->dtype == MD_DTYPE_BF16 ? (size_t)std::min(rows, LM_STEP_ROWS) * (m->width_pad / 8) * 4 : 0);
+  w.row_factor = (float*)a.take(slots ? (size_t)std::min(rows, LM_STEP_ROWS) * 4 : 0);
   w.total = a.off;
   return w;
 }
@@ -253,6 +256,7 @@ struct Step {
     g.a = (const bf16_t*)a;
     g.lda = ordered ? 8 : lda;
     g.chunk = ordered ? 8 * b->n_rows : 8;
+    g.ldo = 8;
     g.out_chunk = 8 * b->n_rows;
     g.w = (const bf16_t*)lin.w;
     g.k = lin.k_pad;
@@ -314,11 +318,16 @@ struct Step {
   }
 
   // a sublayer's last projection.  Few rows: the residual stream(s) and the input of the next sublayer in the same launch
-  md_status finish(const void* a, int64_t lda, const md_linear& lin, bool ordered, const float* prev, const md_rms_weight& nw, const float* next) {
+  // (plain: rows for a router and experts)
+  md_status finish(const void* a, int64_t lda, const md_linear& lin, bool ordered, const float* prev, const md_rms_weight& nw, const float* next, bool plain = false) {
     mix = prev;
     if (!few) return to_residual(a, lda, lin);
     LmStepGemm g = step_gemm(a, lda, lin, ordered);
     g.out = (bf16_t*)w.h;
+    if (plain) {
+      g.ldo = m->width_pad;
+      g.out_chunk = 8;
+    }
     g.x = w.x;
     g.stride = (int64_t)b->n_rows * m->width_pad;
     g.streams = n_streams(m);
@@ -339,7 +348,28 @@ struct Step {
       return MD_OK;
     }
     sumsq = nullptr;
-    return add_norm(nw, w.h, next, nullptr, true, b->n_rows);
+    if (!few || (m->streams == 0 && add.top == 0)) return add_norm(nw, w.h, next, nullptr, true, b->n_rows);
+    LmStreams a = streams(nw, w.h, next);
+    a.out_chunk = 8 * b->n_rows;
+    a.sumsq_out = w.sumsq;
+    sumsq = w.sumsq;
+    add = {};
+    return lm_stream_split(a, b->n_rows, s);
+  }
+
+  LmStreams streams(const md_rms_weight& nw, void* y, const float* next) const {
+    LmStreams a = {};
+    a.x = w.x;
+    a.stride = (int64_t)b->n_rows * m->width_pad;
+    a.streams = n_streams(m);
+    a.add = add;
+    a.prev = mix;
+    a.next = next;
+    a.w = nw;
+    a.eps = m->eps;
+    a.width = m->width; a.width_pad = m->width_pad;
+    a.y = y;
+    return a;
   }
 
   // x += pending;  y = norm(x).  Streams: mixed with the weights around the pending sublayer, then u = their sum weighted for the next one
@@ -347,17 +377,7 @@ struct Step {
   md_status add_norm(const md_rms_weight& nw, void* y, const float* next, const int32_t* rows_idx, bool write_x, int rows, float* sum_out = nullptr) {
     md_status r;
     if (m->streams > 0 || add.top > 0) {
-      LmStreams a = {};
-      a.x = w.x;
-      a.stride = (int64_t)b->n_rows * m->width_pad;
-      a.streams = n_streams(m);
-      a.add = add;
-      a.prev = mix;
-      a.next = next;
-      a.w = nw;
-      a.eps = m->eps;
-      a.width = m->width; a.width_pad = m->width_pad;
-      a.y = y;
+      LmStreams a = streams(nw, y, next);
       a.sum_out = sum_out;
       a.rows_idx = rows_idx;
       a.write_x = write_x;
@@ -532,8 +552,18 @@ struct Step {
   md_status expert_forward(const md_lm_layer& l) {
     const int rows = b->n_rows, slots = rows * l.top;
     const bool step = dec && lm_expert_step_takes(rows, l.top, l.experts);
-    LmRoute r = {w.h, rows, m->width_pad, l.experts, l.top, l.router.w, l.router_bias, w.chosen, w.route_weight, w.offsets, w.row_of, w.slot_of};
-    if (step) r.offsets = r.row_of = r.slot_of = nullptr;
+    LmRoute r = {w.h, rows, m->width_pad, l.experts, l.top, l.router.w, l.router_bias, w.chosen, w.route_weight};
+    if (step) {
+      r.sumsq = sumsq;
+      r.sumsq_n = m->width_pad / 8;
+      r.width = m->width;
+      r.eps = m->eps;
+      r.factor = w.row_factor;
+    } else {
+      r.offsets = w.offsets;
+      r.row_of = w.row_of;
+      r.slot_of = w.slot_of;
+    }
     MD_TRY(lm_route(m->dtype, r, s));
     const int64_t ld = l.gate_up.n_pad;
     add = {};
@@ -545,10 +575,10 @@ struct Step {
       add.src = w.part;
       add.slices = 1;
       LmExpertGemm g = {(const bf16_t*)w.h, m->width_pad, rows, l.top, (const bf16_t*)l.gate_up.w, ld * l.gate_up.k_pad, l.gate_up.k_pad, l.experts,
-                        w.chosen, slots, l.ff_pad, w.act, l.down.k_pad};
+                        w.chosen, slots, l.ff_pad, sumsq ? w.row_factor : nullptr, w.act, l.down.k_pad};
       MD_TRY(lm_expert_silu(g, s));
       g = {(const bf16_t*)w.act, l.down.k_pad, slots, 1, (const bf16_t*)l.down.w, (int64_t)l.down.n_pad * l.down.k_pad, l.down.k_pad, l.experts,
-           w.chosen, slots, 0, w.part, m->width_pad};
+           w.chosen, slots, 0, nullptr, w.part, m->width_pad};
       return lm_expert_rows(g, l.down.n_pad, s);
     }
     if (dec) {
@@ -600,7 +630,7 @@ struct Step {
       if (l.out_proj.k_pad != l.heads * l.vdim_pad) MD_TRY(zero_fill(w.att, (size_t)b->n_rows * l.out_proj.k_pad * esize(m), s));
       MD_TRY(mixer(i));
       if (l.ff > 0) {
-        MD_TRY(finish(w.att, l.out_proj.k_pad, l.out_proj, few, l.mix1, l.norm2, l.mix2));
+        MD_TRY(finish(w.att, l.out_proj.k_pad, l.out_proj, few, l.mix1, l.norm2, l.mix2, l.experts > 0));
         MD_TRY(input(l.norm2, l.mix2));
         MD_TRY(feed_forward(l, nw, next));
       } else {

@@ -202,6 +202,9 @@ struct LmStreams {
   float* sum_out;        // optional: the weighted sum before the norm, fp32
   const int32_t* rows_idx;
   int write_x;
+  // lm_stream_split: y = the weighted sum times its norm weight, in chunks of columns; the rows' factors are left to who reads it, with these sums
+  int out_chunk;
+  float* sumsq_out;      // [rows][width_pad / 8]
 };
 
 struct LmRoute {
@@ -211,6 +214,11 @@ struct LmRoute {
   const float* bias;
   int32_t* chosen;       // [rows][top]
   float* weight;         // [rows][top]
+  // rows before their norm: sums of squares (LmStepGemm), and where to leave the rows' factors; nullptr: normed rows
+  const float* sumsq;
+  int sumsq_n, width;
+  float eps;
+  float* factor;         // [rows]
   // rows sorted by expert: slots offsets[e] .. offsets[e + 1] - 1 belong to expert e
   int32_t *offsets, *row_of, *slot_of;  // [experts + 1], [rows * top], [rows][top]; nullptr: not wanted
 };
@@ -232,9 +240,9 @@ struct LmStepGemm {
   int sumsq_n;
   float eps;
   int width;             // that the mean of squares is over
-  bf16_t* out;           // rows: [rows][ldo]; otherwise [columns / 8][rows][8], residual: the next sublayer's input times its norm weight
+  bf16_t* out;           // rows: [rows][ldo]; otherwise in_chunks(column, out_chunk) of rows ldo apart; residual: the next sublayer's input times its norm weight
   int64_t ldo;
-  int out_chunk;         // = 8 * rows
+  int out_chunk;
   const bf16_t* bias;
   int n, ff_pad;         // columns of the result; SiLU gate: rows 0 .. of w are the gates, ff_pad .. the inputs
   // residual epilogue: streams, weights around this sublayer and of the next one (nullptr: plain sum), as in LmStreams
@@ -261,6 +269,7 @@ struct LmExpertGemm {
   const int32_t* chosen;  // [n]
   int n;                 // choices
   int ff_pad;            // SiLU gate: rows 0 .. of a matrix are the gates, ff_pad .. the inputs
+  const float* factor;   // SiLU gate: of the rows of a, nullptr: ones
   void* out;             // [n][ldo], in the order of the choices
   int64_t ldo;
 };
@@ -271,6 +280,7 @@ md_status lm_expert_rows(const LmExpertGemm& a, int n, hipStream_t s);   // out 
 // dtype: MD_DTYPE_*
 md_status lm_embed_streams(const md_lm_model* m, const int32_t* tokens, const int32_t* row_pos, float* x, int64_t stride, int rows, hipStream_t s);
 md_status lm_stream_step(int dtype, const LmStreams& a, int rows, hipStream_t s);
+md_status lm_stream_split(const LmStreams& a, int rows, hipStream_t s);  // bf16
 
 md_status lm_latent_plain(int dtype, const LmLatent& a, hipStream_t s);  // any dtype and sizes
 bool lm_latent_mfma_takes(const LmLatent& a);

@@ -72,3 +72,28 @@ def test_experts_of_a_step(rows, experts, top, ff, alike):
     assert float(e[int(0.9 * (len(e) - 1))]) < 3e-2 and float(e.median()) < 1e-2
     if alike:
         assert bool((got == got[:1]).all())
+
+
+@pytest.mark.parametrize("streams,width", [(1, 320), (2, 2112), (4, 136), (5, 64)], ids=str)
+def test_experts_between_products_of_a_step(streams, width):
+    """Rows whose norm the router, the experts and the next projection finish: up to 48 rows, and the first that are normed whole; prompts beside tokens."""
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    cfg = U.stream_config([(U.ssm(2, 32, 32), U.moe(6, 1, 130)), (mixer(), U.dense(70)), (mixer(), U.moe(5, 1, 64))], width=width, vocab=120, streams=streams, positions=64)
+    w = U.weights(cfg, 3, 1.5)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=torch.bfloat16, max_batch=64, max_context=64)
+    ts = [U.tokens(3, cfg["vocab"], i) for i in range(49)]
+    want = torch.stack([O.forward(cfg, w, t) for t in ts])
+    for n in (1, 8, 9, 33, 48, 49):
+        slots = [m.open_sequence() for _ in range(n)]
+        got = [m.step([(s, t[k : k + 1], [0]) for s, t in zip(slots, ts)]) for k in range(2)]
+        for k in range(2):
+            e = U.logit_errors(got[k], want[:n, k]).sort().values
+            assert float(e[int(0.9 * (n - 1))]) < 7e-2 and float(e.median()) < 3e-2, (n, k, e)
+        if n == 8:  # the last token of each, beside a prompt
+            got = m.step([(s, t[2:], [0]) for s, t in zip(slots, ts)] + [(m.open_sequence(), ts[40], [2, 0])])
+            e = U.logit_errors(got, torch.cat([want[:8, 2], want[40, [2, 0]]])).sort().values
+            assert float(e[8]) < 7e-2 and float(e.median()) < 3e-2
+        for s in slots:
+            m.close_sequence(s)
