@@ -958,41 +958,42 @@ md_status lm_attn_mfma(const LmAttn& a, hipStream_t s) {
 // ---------------------------------------------------------------------------------------------------------------------------
 namespace {
 
-constexpr int DTK = 64;  // keys per tile of a decode workgroup: one per lane in the mixture and the softmax
-constexpr int NWD = 8;   // its waves
+constexpr int NWD = 8;  // waves of a decode workgroup
 
 struct DecodeLds {
   int q, raw, p, mix, stat, total;
 };
-__host__ __device__ inline DecodeLds decode_lds(int H, int dp) {
+__host__ __device__ inline DecodeLds decode_lds(int H, int dp, int tk) {
   const int hs = (H + 3) / 4 * 4;
   DecodeLds l;
   l.q = 0;
   l.raw = l.q + H * dp * 2;
-  l.p = l.raw + H * DTK * 4;
-  l.mix = l.p + hs * DTK * 4;
+  l.p = l.raw + H * tk * 4;
+  l.mix = l.p + hs * tk * 4;
   l.stat = l.mix + H * hs * 4;
   l.total = l.stat + 4 * hs * 4;
   return l;
 }
 
 // grid (splits, sequences).  Split s covers the keys base + s * split_keys ..., base = the chunk's first key rounded down to a block;
-// queries and the row's own key and value are attn_prep_kernel's.  HPW: output heads per wave, D: dp / 32, C: vp / 32.
+// queries and the row's own key and value are attn_prep_kernel's.  HPW: output heads per wave, D: dp / 32, C: vp / 32, TK: keys per tile.
 // Waves read many blocks before they use the first (no branch between loads): keys of a whole tile row by groups of heads, values of one
 // head at a time; blocks past the last key are read (finite spare positions) and masked.
-// Few keys: what counts is the chain of dependent loads, a batch of key heads and a value head after the other.  Eight waves (two share the
-// heads of 16 keys) halve it: 32 heads of 64, one sequence at 50 keys 13.3 us against 19.4 with four waves; many keys are the same either
-// way (64 sequences at 1500: 4.11 ms a step of the 24-layer model against 4.08).
-template <int HPW, int D, int C>
+// Few keys: what counts is the chain of dependent loads.  Splits of one block of 32 keys (up to 63 sequences in a graph) have tiles of their own: TK = 32 deals
+// the key heads to four pairs of waves and requests everything a wave reads, keys and values, before the queries are staged; the mixture's sum
+// over heads is shared by the halves of a wave.  32 heads of 64, one sequence at 100 keys: 13.0 us against 13.9 in tiles of 64 (a step of the 24-layer model 1104 against 1120, with
+// 16 heads of 128 1093 against 1119, 24 sequences at 1500 keys 2454 against 2529), which read a
+// block of values beyond the split and one key head batch after the other.
+template <int HPW, int D, int C, int TK>
 __global__ __launch_bounds__(64 * NWD, 2) void attn_decode_kernel(const LmAttn a) {
   extern __shared__ __attribute__((aligned(16))) char dsm[];
   const int H = a.heads, G = a.kv_heads, rep = H / G, dp = 32 * D, vp = 32 * C, hs = (H + 3) / 4 * 4;
-  const DecodeLds L = decode_lds(H, dp);
+  const DecodeLds L = decode_lds(H, dp, TK);
   bf16_t* qs = (bf16_t*)(dsm + L.q);
   float *raw = (float*)(dsm + L.raw), *ps = (float*)(dsm + L.p), *mixT = (float*)(dsm + L.mix);
   float *ms = (float*)(dsm + L.stat), *ls = ms + hs, *al = ls + hs, *sl = al + hs;
   const int split = blockIdx.x, seq = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n16 = lane & 15, q4 = lane >> 4;
-  const int row = a.r.seq_row0[seq], i = a.r.row_pos[row], slot = a.r.seq_slot[seq];
+  const int row = a.r.seq_row0[seq], i = a.r.seq_pos0[seq], slot = a.r.seq_slot[seq];
   const int first = a.chunk > 0 ? i / a.chunk * a.chunk : 0;
   const int k0 = (first & ~31) + split * a.split_keys, k1 = min(k0 + a.split_keys - 1, i);
   float* part = a.part + ((int64_t)seq * a.n_split + split) * (H * vp + 2 * H);
@@ -1003,18 +1004,6 @@ __global__ __launch_bounds__(64 * NWD, 2) void attn_decode_kernel(const LmAttn a
     }
     return;
   }
-  for (int c = tid * 8; c < H * dp; c += 512 * NWD) *(u32x4*)(qs + c) = *(const u32x4*)((const bf16_t*)a.q + (int64_t)row * H * dp + c);
-  for (int e = tid; e < H * hs; e += 64 * NWD) {  // transposed, heads padded to a multiple of four
-    const int h = e % hs, g = e / hs;
-    mixT[e] = h < H ? a.mix[h * H + g] : 0.f;
-  }
-  for (int h = tid; h < hs; h += 64 * NWD) {
-    ms[h] = -INFINITY;
-    ls[h] = 0.f;
-    sl[h] = h < H ? a.slope[h] : 0.f;
-  }
-  __syncthreads();
-
   const bf16_t* Kb = (const bf16_t*)a.k + (int64_t)slot * G * a.ctx * dp;
   const bf16_t* Vb = (const bf16_t*)a.v + (int64_t)slot * G * a.ctx * vp;
   float acc[HPW][2 * C];  // heads wave, wave + NWD, ..: coordinate 16 t + n16, the keys of this lane row
@@ -1023,79 +1012,117 @@ __global__ __launch_bounds__(64 * NWD, 2) void attn_decode_kernel(const LmAttn a
 #pragma unroll
     for (int t = 0; t < 2 * C; ++t) acc[u][t] = 0.f;
 
-  const int kwave = wave & 3, g_lo = (wave >> 2) * ((G + 1) / 2), g_hi = min(G, g_lo + (G + 1) / 2);
-  for (int j0 = k0; j0 <= k1; j0 += DTK) {
-    const int n = min(DTK, k1 + 1 - j0);
-    // waves w and w + 4: scores of keys 16 w .. 16 w + 15, half the key heads each, 16 query heads of one key head per matrix product
-    if (16 * kwave < n && g_lo < g_hi) {
-      constexpr int UG = D >= 3 ? 2 : 4;
-      const bf16_t* kw = Kb + key_block(j0 + 16 * kwave, 0, G, dp) + (kwave & 1) * (D * 512) + 8 * lane;
-      const float dist = (float)(i - (j0 + 16 * kwave + 4 * q4));
-      bf16x8 kf[2][UG][D];
-      auto load = [&](int buf, int g0) {
+  constexpr int KW = TK / 16, PARTS = NWD / KW;  // waves of a tile's keys, and of its key heads
+  const int kwave = wave % KW, heads_each = (G + PARTS - 1) / PARTS, g_lo = wave / KW * heads_each, g_hi = min(G, g_lo + heads_each);
+  constexpr bool AHEAD = TK == 32;  // values of all heads of the wave requested behind the first keys
+  constexpr int UG = D >= 3 ? 2 : 4, NB = TK / 32, VB = AHEAD && HPW * C <= 8 ? HPW : 2;
+  auto stage = [&] {
+    for (int c = tid * 8; c < H * dp; c += 512 * NWD) *(u32x4*)(qs + c) = *(const u32x4*)((const bf16_t*)a.q + (int64_t)row * H * dp + c);
+    for (int e = tid; e < H * hs; e += 64 * NWD) {  // transposed, heads padded to a multiple of four
+      const int h = e % hs, g = e / hs;
+      mixT[e] = h < H ? a.mix[h * H + g] : 0.f;
+    }
+    for (int h = tid; h < hs; h += 64 * NWD) {
+      ms[h] = -INFINITY;
+      ls[h] = 0.f;
+      sl[h] = h < H ? a.slope[h] : 0.f;
+    }
+    __syncthreads();
+  };
+  if (!AHEAD) stage();
+  for (int j0 = k0; j0 <= k1; j0 += TK) {
+    const int n = min(TK, k1 + 1 - j0);
+    // scores of keys 16 kwave .. 16 kwave + 15, this wave's key heads, 16 query heads of one key head per matrix product
+    const bf16_t* kw = Kb + key_block(j0 + 16 * kwave, 0, G, dp) + (kwave & 1) * (D * 512) + 8 * lane;
+    const float dist = (float)(i - (j0 + 16 * kwave + 4 * q4));
+    bf16x8 kf[2][UG][D];
+    auto load = [&](int buf, int g0) {
 #pragma unroll
-        for (int u = 0; u < UG; ++u)
+      for (int u = 0; u < UG; ++u)
 #pragma unroll
-          for (int d = 0; d < D; ++d) kf[buf][u][d] = *(const bf16x8*)(kw + min(g0 + u, g_hi - 1) * (32 * dp) + 512 * d);
-      };
-      auto scores = [&](int buf, int g0) {
+        for (int d = 0; d < D; ++d) kf[buf][u][d] = *(const bf16x8*)(kw + min(g0 + u, G - 1) * (32 * dp) + 512 * d);
+    };
+    auto scores = [&](int buf, int g0) {
 #pragma unroll
-        for (int u = 0; u < UG; ++u) {
-          const int g = min(g0 + u, g_hi - 1);
-          for (int r0 = 0; r0 < rep; r0 += 16) {
-            const int h = g * rep + min(r0 + n16, rep - 1);
-            f32x4 s = {0.f, 0.f, 0.f, 0.f};
+      for (int u = 0; u < UG; ++u) {
+        if (g0 + u >= g_hi) continue;
+        const int g = g0 + u;
+        for (int r0 = 0; r0 < rep; r0 += 16) {
+          const int h = g * rep + min(r0 + n16, rep - 1);
+          f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int d = 0; d < D; ++d)
-              s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(md_bf16x8v, kf[buf][u][d]),
-                                                          __builtin_bit_cast(md_bf16x8v, *(const bf16x8*)(qs + h * dp + 32 * d + 8 * q4)), s, 0, 0, 0);
-            if (r0 + n16 < rep) {
-              f32x4 o;
+          for (int d = 0; d < D; ++d)
+            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(md_bf16x8v, kf[buf][u][d]),
+                                                        __builtin_bit_cast(md_bf16x8v, *(const bf16x8*)(qs + h * dp + 32 * d + 8 * q4)), s, 0, 0, 0);
+          if (r0 + n16 < rep) {
+            f32x4 o;
 #pragma unroll
-              for (int e = 0; e < 4; ++e) o[e] = s[e] * a.scale - sl[h] * (dist - (float)e);
-              *(f32x4*)(raw + h * DTK + 16 * kwave + 4 * q4) = o;
-            }
+            for (int e = 0; e < 4; ++e) o[e] = s[e] * a.scale - sl[h] * (dist - (float)e);
+            *(f32x4*)(raw + h * TK + 16 * kwave + 4 * q4) = o;
           }
         }
-      };
-      load(0, g_lo);
-      for (int g0 = g_lo; g0 < g_hi; g0 += 2 * UG) {
-        load(1, g0 + UG);
-        scores(0, g0);
-        load(0, g0 + 2 * UG);  // (past the last head: clamped, unused)
-        scores(1, g0 + UG);
       }
-    }
-    constexpr int NB = DTK / 32;
-    u32x4 vf[2][NB][2 * C];
+    };
+    u32x4 vf[VB][NB][2 * C];
     auto load_v = [&](int u) {
       const bf16_t* vh = Vb + key_block(j0, min(wave + NWD * u, H - 1) / rep, G, vp) + 8 * lane;
 #pragma unroll
       for (int b = 0; b < NB; ++b)
 #pragma unroll
-        for (int t = 0; t < 2 * C; ++t) vf[u & 1][b][t] = *(const u32x4*)(vh + (int64_t)b * G * (32 * vp) + t * 512);
+        for (int t = 0; t < 2 * C; ++t) vf[u % VB][b][t] = *(const u32x4*)(vh + (int64_t)b * G * (32 * vp) + t * 512);
     };
-    load_v(0);  // under the mixture and the softmax
+    if (AHEAD) {
+      load(0, g_lo);
+      if (g_lo + UG < g_hi) load(1, g_lo + UG);
+#pragma unroll
+      for (int u = 0; u < VB; ++u) load_v(u);
+      __builtin_amdgcn_sched_barrier(0);
+      if (j0 == k0) stage();
+      for (int g0 = g_lo; g0 < g_hi; g0 += 2 * UG) {
+        scores(0, g0);
+        if (g0 + 2 * UG < g_hi) load(0, g0 + 2 * UG);
+        scores(1, g0 + UG);
+        if (g0 + 3 * UG < g_hi) load(1, g0 + 3 * UG);
+      }
+    } else {
+      if (16 * kwave < n && g_lo < g_hi) {
+        load(0, g_lo);
+        for (int g0 = g_lo; g0 < g_hi; g0 += 2 * UG) {
+          load(1, g0 + UG);
+          scores(0, g0);
+          load(0, g0 + 2 * UG);  // (past the last head: clamped, unused)
+          scores(1, g0 + UG);
+        }
+      }
+      load_v(0);  // under the mixture and the softmax
+    }
     __syncthreads();
     for (int h0 = 4 * wave; h0 < H; h0 += 4 * NWD) {
       f32x4 s = {0.f, 0.f, 0.f, 0.f};
+      const int key = lane % TK, half = (H + 1) / 2, m_lo = TK == 32 ? (lane >> 5) * half : 0, m_n = TK == 32 ? half : H;
 #pragma unroll 8
-      for (int g = 0; g < H; ++g) s += *(const f32x4*)(mixT + g * hs + h0) * raw[g * DTK + lane];
-      if (lane >= n || j0 + lane < first) s = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      for (int k = 0; k < m_n; ++k) {
+        const int g = m_lo + k;
+        if (TK == 64 || g < H) s += *(const f32x4*)(mixT + g * hs + h0) * raw[g * TK + key];
+      }
+      if (TK == 32)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] += __shfl_xor(s[e], 32, 64);
+      if (key >= n || j0 + key < first) s = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
       const f32x4 mo = *(const f32x4*)(ms + h0);
       f32x4 mn = s, p, sum;
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1)
+      for (int o = TK / 2; o > 0; o >>= 1)
 #pragma unroll
         for (int e = 0; e < 4; ++e) mn[e] = fmaxf(mn[e], __shfl_xor(mn[e], o, 64));
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         mn[e] = fmaxf(mn[e], mo[e]);
         p[e] = sum[e] = expf(s[e] - mn[e]);
-        ps[(h0 + e) * DTK + lane] = p[e];
+        ps[(h0 + e) * TK + key] = p[e];
       }
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1)
+      for (int o = TK / 2; o > 0; o >>= 1)
 #pragma unroll
         for (int e = 0; e < 4; ++e) sum[e] += __shfl_xor(sum[e], o, 64);
       if (lane == 0) {
@@ -1110,17 +1137,17 @@ __global__ __launch_bounds__(64 * NWD, 2) void attn_decode_kernel(const LmAttn a
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < HPW; ++u) {
-      if (u + 1 < HPW) load_v(u + 1);
+      if (VB == 2 ? u + 1 < HPW && (u > 0 || !AHEAD) : false) load_v(u + 1);
       const int h = min(wave + NWD * u, H - 1);
       const float f = al[h];
 #pragma unroll
       for (int t = 0; t < 2 * C; ++t) acc[u][t] *= f;
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
-        const f32x4 p0 = *(const f32x4*)(ps + h * DTK + 32 * b + 8 * q4), p1 = *(const f32x4*)(ps + h * DTK + 32 * b + 8 * q4 + 4);
+        const f32x4 p0 = *(const f32x4*)(ps + h * TK + 32 * b + 8 * q4), p1 = *(const f32x4*)(ps + h * TK + 32 * b + 8 * q4 + 4);
 #pragma unroll
         for (int t = 0; t < 2 * C; ++t) {
-          const u32x4 v = vf[u & 1][b][t];
+          const u32x4 v = vf[u % VB][b][t];
           acc[u][t] += p0[0] * lo_bf(v[0]) + p0[1] * hi_bf(v[0]) + p0[2] * lo_bf(v[1]) + p0[3] * hi_bf(v[1]) + p1[0] * lo_bf(v[2]) +
                        p1[1] * hi_bf(v[2]) + p1[2] * lo_bf(v[3]) + p1[3] * hi_bf(v[3]);
         }
@@ -1195,40 +1222,45 @@ int lm_attn_decode_splits(int n_seq, int span, int* split_keys) {
 size_t lm_attn_decode_part_floats(int n_seq, int n_split, int heads, int vp) { return n_split > 1 ? (size_t)n_seq * n_split * (heads * vp + 2 * heads) : 0; }
 
 namespace {
-template <int D, int C>
+template <int TK, int D, int C>
 TalkKernel decode_by_heads(int heads) {
-  return heads <= 8 ? attn_decode_kernel<1, D, C> : heads <= 16 ? attn_decode_kernel<2, D, C> : heads <= 32 ? attn_decode_kernel<4, D, C>
-         : heads <= 64 && D * C <= 4 ? attn_decode_kernel<8, D, C> : nullptr;
+  return heads <= 8 ? attn_decode_kernel<1, D, C, TK> : heads <= 16 ? attn_decode_kernel<2, D, C, TK> : heads <= 32 ? attn_decode_kernel<4, D, C, TK>
+         : heads <= 64 && D * C <= 4 ? attn_decode_kernel<8, D, C, TK> : nullptr;
 }
-template <int D>
+template <int TK, int D>
 TalkKernel decode_by_width(const LmAttn& a) {
   switch (a.vp / 32) {
-    case 1: return decode_by_heads<D, 1>(a.heads);
-    case 2: return decode_by_heads<D, 2>(a.heads);
-    case 3: return decode_by_heads<D, 3>(a.heads);
-    case 4: return decode_by_heads<D, 4>(a.heads);
+    case 1: return decode_by_heads<TK, D, 1>(a.heads);
+    case 2: return decode_by_heads<TK, D, 2>(a.heads);
+    case 3: return decode_by_heads<TK, D, 3>(a.heads);
+    case 4: return decode_by_heads<TK, D, 4>(a.heads);
     default: return nullptr;
   }
 }
-TalkKernel decode_pick(const LmAttn& a) {
-  if (decode_lds(a.heads, a.dp).total > 160 * 1024) return nullptr;
+template <int TK>
+TalkKernel decode_by_dim(const LmAttn& a) {
   switch (a.dp / 32) {
-    case 1: return decode_by_width<1>(a);
-    case 2: return decode_by_width<2>(a);
-    case 3: return decode_by_width<3>(a);
-    case 4: return decode_by_width<4>(a);
+    case 1: return decode_by_width<TK, 1>(a);
+    case 2: return decode_by_width<TK, 2>(a);
+    case 3: return decode_by_width<TK, 3>(a);
+    case 4: return decode_by_width<TK, 4>(a);
     default: return nullptr;
   }
+}
+TalkKernel decode_pick(const LmAttn& a, int tk) {
+  if (decode_lds(a.heads, a.dp, 64).total > 160 * 1024) return nullptr;
+  return tk == 32 ? decode_by_dim<32>(a) : decode_by_dim<64>(a);
 }
 }  // namespace
 
-bool lm_attn_decode_takes(const LmAttn& a) { return decode_pick(a) != nullptr; }
+bool lm_attn_decode_takes(const LmAttn& a) { return decode_pick(a, 64) != nullptr; }
 md_status lm_attn_decode(const LmAttn& a, hipStream_t s) {
-  const TalkKernel fn = decode_pick(a);
+  const int tk = a.split_keys == 32 ? 32 : 64;
+  const TalkKernel fn = decode_pick(a, tk);
   if (!fn) return MD_ERR_UNSUPPORTED;
   MD_TRY(md_ensure_dynamic_lds((const void*)fn, 160 * 1024));
   MD_TRY(lm_attn_prep(MD_DTYPE_BF16, a, s));
-  hipLaunchKernelGGL(fn, dim3(a.n_split, a.r.n_seq), dim3(64 * NWD), decode_lds(a.heads, a.dp).total, s, a);
+  hipLaunchKernelGGL(fn, dim3(a.n_split, a.r.n_seq), dim3(64 * NWD), decode_lds(a.heads, a.dp, tk).total, s, a);
   MD_TRY(md_launch_status());
   if (a.n_split == 1) return MD_OK;
   hipLaunchKernelGGL(attn_combine_kernel, dim3(a.heads, a.r.n_seq), dim3(256), 0, s, a);
