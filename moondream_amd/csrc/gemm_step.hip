@@ -81,6 +81,8 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
   const int ns = S > 0 ? S : a.streams;
   float* xr = EPI == EPI_RESID ? a.x + (int64_t)m * a.width_pad + c : nullptr;
   f32x4 old[SM], norm_w = {0.f, 0.f, 0.f, 0.f};
+  constexpr int HEADS = 8;  // sums of squares per lane under way with them
+  float head_sq[HEADS];
   if (EPI == EPI_RESID && live) {
 #pragma unroll
     for (int s = 0; s < SM; ++s)
@@ -88,6 +90,10 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) norm_w[e] = a.norm.w[(int64_t)min(c + e, a.width - 1) * a.norm.stride];  // (columns beyond hold zeros)
   }
+  const float* sq_row = EPI == EPI_RESID ? a.head_sumsq + (int64_t)min(m, a.rows - 1) * a.heads : nullptr;
+  if (EPI == EPI_RESID && a.head_sumsq && wave < M16)
+#pragma unroll
+    for (int j = 0; j < HEADS; ++j) head_sq[j] = sq_row[min(4 * j + g, a.heads - 1)];
 
   u32x4 wf[2][U][NX], af[2][U][PA][M16];
   auto load = [&](auto buf, int u) {  // units u .. u + U - 1; past the end: the last one again, not used
@@ -195,7 +201,17 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
     st4(a.out + m * a.ldo + in_chunks(c, a.out_chunk), y);
   } else {
     const float *in_w = a.next, *out_w = a.prev ? a.prev + ns : nullptr, *mix = a.prev ? a.prev + 2 * ns : nullptr;
-    const f32x4 y = total(lane);
+    f32x4 y = total(lane);
+    if (a.head_sumsq) {
+      float q = 0.f;
+#pragma unroll
+      for (int j = 0; j < HEADS; ++j)
+        if (4 * j + g < a.heads) q += head_sq[j];
+      for (int j = 4 * HEADS + g; j < a.heads; j += 4) q += sq_row[j];
+      q += __shfl_xor(q, 16, 64);
+      q += __shfl_xor(q, 32, 64);
+      y *= 1.0f / sqrtf(q / (float)a.normed + a.eps);
+    }
     f32x4 u = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < SM; ++t) {

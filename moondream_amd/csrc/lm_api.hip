@@ -31,7 +31,7 @@ struct LmWs {
   char *h, *proj, *q, *att, *y, *gu, *act;
   float *part, *qf, *kf, *of, *chunk_state, *attn_part;
   char *c_rows, *kv, *q_lat, *conv_out;
-  float *latent_part, *dt, *seg, *seg_decay, *route_weight, *sumsq, *row_factor;
+  float *latent_part, *dt, *seg, *seg_decay, *route_weight, *sumsq, *row_factor, *head_sumsq;
   int32_t *chosen, *slot_of, *row_of, *offsets;
   void* splitk;
   size_t splitk_bytes;
@@ -67,7 +67,7 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
   const size_t es = esize(m), M = rows;
   size_t in = 0, q = 0, att = 0, gu = 0, act = 0, qf = 0, of = 0, cs = 0, ap = 0, sk = 0, part = 0, y = M * m->width_pad;
   size_t c_rows = 0, kv = 0, q_lat = 0, lp = 0, conv = 0, dt = 0, seg = 0, segs = 0, slots = 0, experts = 0;
-  size_t sk_room = 0;
+  size_t sk_room = 0, ssm_heads = 0;
   auto splitk = [&](const md_linear& l, int n) {
     if (m->dtype != MD_DTYPE_BF16 || !l.w || n <= 0) return;
     sk = std::max(sk, md_gemm_workspace_bytes(&l, n, 1));
@@ -121,6 +121,7 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
     } else if (l.mixer == MD_MIXER_STATE_SPACE) {
       conv = std::max(conv, M * conv_columns(l));
       dt = std::max(dt, M * l.heads);
+      ssm_heads = std::max(ssm_heads, (size_t)l.heads);
       if (m->dtype == MD_DTYPE_BF16) {
         const size_t ns = lm_ssm_most_segments(n_seq, l.heads, max_len);
         segs = std::max(segs, ns * l.heads);
@@ -170,6 +171,7 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
   w.offsets = (int32_t*)a.take(slots ? (experts + 1) * 4 : 0);
   w.sumsq = (float*)a.take(m->dtype == MD_DTYPE_BF16 ? (size_t)std::min(rows, LM_STEP_ROWS) * (m->width_pad / 8) * 4 : 0);
   w.row_factor = (float*)a.take(slots ? (size_t)std::min(rows, LM_STEP_ROWS) * 4 : 0);
+  w.head_sumsq = (float*)a.take(conv && m->dtype == MD_DTYPE_BF16 ? (size_t)std::min(rows, LM_STEP_ROWS) * ssm_heads * 4 : 0);
   w.total = a.off;
   return w;
 }
@@ -248,6 +250,7 @@ struct Step {
   bool few = false;            // a step of few rows
   bool chain = false;          // fp32: the products' order of sums (gemm_f32.hip)
   bool ready = false;          // w.h holds the next sublayer's input already ...
+  const md_lm_layer* unnormed = nullptr;  // few rows: the state-space layer whose outputs lie before their norm in w.att
   const float* sumsq = nullptr;  // ... but for the factor that these give its rows, in the order of the matrix operand
 
   // ordered: the rows of `a` lie as another of these products left them
@@ -336,6 +339,12 @@ struct Step {
     g.next = next;
     g.norm = nw;
     g.sumsq_out = w.sumsq;
+    if (unnormed) {
+      g.head_sumsq = w.head_sumsq;
+      g.heads = unnormed->heads;
+      g.normed = unnormed->heads * unnormed->vdim;
+      unnormed = nullptr;
+    }
     sumsq = w.sumsq;
     ready = true;
     return lm_step_resid(g, s);
@@ -509,7 +518,13 @@ struct Step {
     a.out_chunk = few ? 8 * b->n_rows : 8;
     a.u = w.conv_out; a.dt = w.dt; a.seg = w.seg; a.seg_decay = w.seg_decay;
     if (m->dtype == MD_DTYPE_BF16) {
-      if (b->max_len == 1 && (g_lm_kernels & 2) && lm_ssm_decode_takes(a)) return lm_ssm_decode(a, s);
+      if (b->max_len == 1 && (g_lm_kernels & 2) && lm_ssm_decode_takes(a)) {
+        if (few && l.norm_groups == 1) {
+          a.sumsq = w.head_sumsq;
+          unnormed = &l;
+        }
+        return lm_ssm_decode(a, s);
+      }
       a.n_seg = lm_ssm_segments(b->n_seq, l.heads, b->max_len, &a.seg_chunks);
       if (b->max_len > 1 && (g_lm_kernels & 1) && lm_ssm_mfma_takes(a)) return lm_ssm_mfma(a, s);
     }
