@@ -981,9 +981,9 @@ __host__ __device__ inline DecodeLds decode_lds(int H, int dp, int tk) {
 // head at a time; blocks past the last key are read (finite spare positions) and masked.
 // Few keys: what counts is the chain of dependent loads.  Splits of one block of 32 keys (up to 63 sequences in a graph) have tiles of their own: TK = 32 deals
 // the key heads to four pairs of waves and requests everything a wave reads, keys and values, before the queries are staged; the mixture's sum
-// over heads is shared by the halves of a wave.  32 heads of 64, one sequence at 100 keys: 13.0 us against 13.9 in tiles of 64 (a step of the 24-layer model 1104 against 1120, with
-// 16 heads of 128 1093 against 1119, 24 sequences at 1500 keys 2454 against 2529), which read a
-// block of values beyond the split and one key head batch after the other.
+// over heads is shared by the halves of a wave.  32 heads of 64, one sequence at 100 keys: 13.0 us against 13.9 in tiles of 64, which read a block of
+// values beyond the split and one key head batch after the other (a step of the 24-layer model 1104 us against 1120, with 16 heads of 128 1093
+// against 1119, 24 sequences at 1500 keys 2454 against 2529).
 template <int HPW, int D, int C, int TK>
 __global__ __launch_bounds__(64 * NWD, 2) void attn_decode_kernel(const LmAttn a) {
   extern __shared__ __attribute__((aligned(16))) char dsm[];
