@@ -133,18 +133,20 @@ __global__ __launch_bounds__(512) void attn_prep_step_kernel(const LmAttn a) {
     y[i] = nw[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (c >= ncol) continue;
     constexpr int AT_ONCE = 4;  // the newest taps
+    // (a branch for each would wait for each: rows before the sequence's first are read from somewhere else and not used)
+    u32x2 raw[AT_ONCE];
     f32x4 u[AT_ONCE], w[AT_ONCE];
-    u[0] = ld4(proj + c);
-    w[0] = *(const f32x4*)(cw + (int64_t)(a.taps - 1) * a.conv_ld + c);
 #pragma unroll
-    for (int k = 1; k < AT_ONCE; ++k) {
-      u[k] = w[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (k < a.taps && pos - k >= 0) {
-        u[k] = ld4(ring + (int64_t)((pos - k) % a.taps) * a.conv_ld + c);
-        w[k] = *(const f32x4*)(cw + (int64_t)(a.taps - 1 - k) * a.conv_ld + c);
-      }
+    for (int k = 0; k < AT_ONCE; ++k) {
+      const bool in = k < a.taps && pos - k >= 0;
+      raw[k] = *(const u32x2*)(k > 0 && in ? ring + (int64_t)((pos - k) % a.taps) * a.conv_ld + c : proj + c);
+      w[k] = *(const f32x4*)(cw + (int64_t)(in ? a.taps - 1 - k : 0) * a.conv_ld + c);
     }
-    if (part < 2) nw[i] = *(const f32x4*)(norm + c);
+    nw[i] = *(const f32x4*)(part < 2 ? norm + c : cw + c);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < AT_ONCE; ++k)
+      u[k] = k < a.taps && pos - k >= 0 ? f32x4{lo_bf(raw[k][0]), hi_bf(raw[k][0]), lo_bf(raw[k][1]), hi_bf(raw[k][1])} : f32x4{0.f, 0.f, 0.f, 0.f};
     for (int k = AT_ONCE; k < a.taps && pos - k >= 0; ++k)
       y[i] += *(const f32x4*)(cw + (int64_t)(a.taps - 1 - k) * a.conv_ld + c) * ld4(ring + (int64_t)((pos - k) % a.taps) * a.conv_ld + c);
 #pragma unroll

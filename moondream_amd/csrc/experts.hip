@@ -63,12 +63,13 @@ __global__ __launch_bounds__(1024) void route_row_kernel(const LmRoute a) {
   constexpr int BATCH = 4;  // loads of a row in flight
   const int row = blockIdx.x, lane = threadIdx.x & 63;
   const T* h = (const T*)a.h + (int64_t)row * a.k_pad;
-  f32x4 sq = {0.f, 0.f, 0.f, 0.f};
-  if (a.sumsq)
-    for (int c = lane * 4; c < a.sumsq_n; c += 256) sq += *(const f32x4*)(a.sumsq + (int64_t)row * a.sumsq_n + c);
+  // (requested first and used last, without a branch)
+  const float* sumsq = a.sumsq + (int64_t)row * a.sumsq_n;
+  f32x4 sq = *(const f32x4*)(a.sumsq ? sumsq + min(lane * 4, a.sumsq_n - 4) : (const float*)a.router);
   for (int e = threadIdx.x >> 6; e < a.experts; e += 32) {
     const int e2 = min(e + 16, a.experts - 1);
     const T *w = (const T*)a.router + (int64_t)e * a.k_pad, *w2 = (const T*)a.router + (int64_t)e2 * a.k_pad;
+    const float bias = a.bias[e], bias2 = a.bias[e2];
     f32x4 s = {0.f, 0.f, 0.f, 0.f}, s2 = s;
     for (int k0 = lane * 8; k0 < a.k_pad; k0 += 512 * BATCH) {
       decltype(ld8(h)) x[BATCH], y[BATCH], y2[BATCH];
@@ -91,10 +92,15 @@ __global__ __launch_bounds__(1024) void route_row_kernel(const LmRoute a) {
       }
     }
     const float t = wave_sum(s[0] + s[1] + s[2] + s[3]), t2 = wave_sum(s2[0] + s2[1] + s2[2] + s2[3]);
-    const float factor = a.sumsq ? 1.0f / sqrtf(wave_sum((sq[0] + sq[1]) + (sq[2] + sq[3])) / (float)a.width + a.eps) : 1.0f;
+    float factor = 1.0f;
+    if (a.sumsq) {
+      f32x4 q = lane * 4 < a.sumsq_n ? sq : f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int c = 256 + lane * 4; c < a.sumsq_n; c += 256) q += *(const f32x4*)(sumsq + c);  // (widths above 2048)
+      factor = 1.0f / sqrtf(wave_sum((q[0] + q[1]) + (q[2] + q[3])) / (float)a.width + a.eps);
+    }
     if (lane == 0) {
-      z[e] = t * factor + a.bias[e];
-      if (e + 16 < a.experts) z[e2] = t2 * factor + a.bias[e2];
+      z[e] = t * factor + bias;
+      if (e + 16 < a.experts) z[e2] = t2 * factor + bias2;
       if (e == 0 && a.sumsq) a.factor[row] = factor;
     }
   }

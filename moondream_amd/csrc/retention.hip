@@ -431,7 +431,7 @@ __global__ __launch_bounds__(256) void ret_decode_kernel(const LmRet a) {
   __shared__ __attribute__((aligned(16))) float qs[256], ks[256], os[256];
   __shared__ float red[4];
   const int h = blockIdx.x, seq = blockIdx.y, tid = threadIdx.x, l = tid & 15, e0 = tid >> 4;
-  const int row = a.r.seq_row0[seq], pos = a.r.row_pos[row], dp = a.dp, vp = a.vp;
+  const int row = a.r.seq_row0[seq], pos = a.r.seq_pos0[seq], dp = a.dp, vp = a.vp;
   float* st = a.state + ((int64_t)a.r.seq_slot[seq] * a.heads + h) * vp * dp;
   const bf16_t* p = (const bf16_t*)a.proj + (int64_t)row * a.ldp;
   f32x4 S[R][E];

@@ -574,28 +574,32 @@ __global__ __launch_bounds__(256) void ssm_decode_kernel(const LmSsm a) {
 #pragma unroll
     for (int k = 0; k < E; ++k) {
       const int d = 64 * k + 4 * l;
-      S[i][k] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (pos > 0 && d < dp) S[i][k] = *(const f32x4*)(st + (int64_t)((tid >> 4) + 16 * i) * dp + d);
+      S[i][k] = *(const f32x4*)(st + (int64_t)((tid >> 4) + 16 * i) * dp + min(d, dp - 4));
     }
   const bf16_t* p = (const bf16_t*)a.proj + (int64_t)row * a.ldp;
   const int mine = h * vp + min(tid, vp - 1);  // the output that this thread writes in the end
   const bf16_t z = p[a.col_z + mine];
   const float norm_w = a.sumsq ? a.out_norm[mine] : 1.0f;
-  const float raw_dt = bf2f(p[a.col_dt + h]) + a.dt_bias[h];
+  const bf16_t dt_in = p[a.col_dt + h];
+  const float dt_bias = a.dt_bias[h], decay = a.decay[h], skip = a.skip[h];
   const bool shared_cols = h % (H / a.groups) == 0;  // the head of its group that also writes the ring's B and C columns
   bf16_t* ring = (bf16_t*)a.conv_state + (int64_t)slot * a.taps * cw;
   for (int i = tid * 4; i < vp + 2 * dp; i += 1024) {
     const int c = i < vp ? h * vp + i : i < vp + dp ? H * vp + g * dp + i - vp : H * vp + (a.groups + g) * dp + i - vp - dp;
     constexpr int AT_ONCE = 4;  // the newest taps: all their loads are requested before the first is used
+    // (a branch for each would wait for each: rows before the sequence's first are read from somewhere else and not used)
+    u32x2 raw[AT_ONCE];
     f32x4 x[AT_ONCE], w[AT_ONCE], y = *(const f32x4*)(a.conv_bias + c);
 #pragma unroll
     for (int k = 0; k < AT_ONCE; ++k) {
-      x[k] = w[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (k < a.taps && pos - k >= 0) {
-        x[k] = k == 0 ? ld4(p + a.col_x + c) : ld4(ring + (int64_t)((pos - k) % a.taps) * cw + c);
-        w[k] = *(const f32x4*)(a.conv + (int64_t)(a.taps - 1 - k) * cw + c);
-      }
+      const bool in = k < a.taps && pos - k >= 0;
+      raw[k] = *(const u32x2*)(k > 0 && in ? ring + (int64_t)((pos - k) % a.taps) * cw + c : p + a.col_x + c);
+      w[k] = *(const f32x4*)(a.conv + (int64_t)(in ? a.taps - 1 - k : 0) * cw + c);
     }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < AT_ONCE; ++k)
+      x[k] = k < a.taps && pos - k >= 0 ? f32x4{lo_bf(raw[k][0]), hi_bf(raw[k][0]), lo_bf(raw[k][1]), hi_bf(raw[k][1])} : f32x4{0.f, 0.f, 0.f, 0.f};
     for (int k = AT_ONCE; k < a.taps && pos - k >= 0; ++k) y += *(const f32x4*)(a.conv + (int64_t)(a.taps - 1 - k) * cw + c) * ld4(ring + (int64_t)((pos - k) % a.taps) * cw + c);
 #pragma unroll
     for (int k = AT_ONCE - 1; k >= 0; --k) y += w[k] * x[k];
@@ -604,7 +608,12 @@ __global__ __launch_bounds__(256) void ssm_decode_kernel(const LmSsm a) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) us[i + e] = bf2f(f2bf(silu_f32(y[e])));  // as a prefill stores it
   }
-  const float dt = softplus_f32(raw_dt), keep = expf(-a.decay[h] * dt), skip = a.skip[h];
+  const float dt = softplus_f32(bf2f(dt_in) + dt_bias), keep = expf(-decay * dt);
+#pragma unroll
+  for (int i = 0; i < 2 * C; ++i)
+#pragma unroll
+    for (int k = 0; k < E; ++k)
+      if (pos == 0 || 64 * k + 4 * l >= dp) S[i][k] = f32x4{0.f, 0.f, 0.f, 0.f};
   __syncthreads();
   float* out = us;  // (only the x part: every row's x is read by its own sixteen lanes before they write)
 #pragma unroll
