@@ -983,8 +983,8 @@ __host__ __device__ inline DecodeLds decode_lds(int H, int dp, int tk) {
 // head at a time; blocks past the last key are read (finite spare positions) and masked.
 // Few keys: what counts is the chain of dependent loads.  Splits of one block of 32 keys (up to 63 sequences in a graph) have tiles of their own: TK = 32 deals
 // the key heads to four pairs of waves and requests everything a wave reads, keys and values, before the queries are staged; the mixture's sum
-// over heads is shared by the halves of a wave.  32 heads of 64, one sequence at 100 keys: 13.0 us against 13.9 in tiles of 64, which read a block of
-// values beyond the split and one key head batch after the other (a step of the 24-layer model 1104 us against 1120, with 16 heads of 128 1093
+// over heads is shared by the halves of a wave.  32 heads of 64, one sequence at 100 keys: 11.8 us against 13.9 in tiles of 64, which read a block of
+// values beyond the split, one key head batch after the other, and waited for each of what is staged (with the waits 13.0: a step of the 24-layer model 1104 us against 1120, with 16 heads of 128 1093
 // against 1119, 24 sequences at 1500 keys 2454 against 2529).
 template <int HPW, int D, int C, int TK>
 __global__ __launch_bounds__(64 * NWD, 2) void attn_decode_kernel(const LmAttn a) {
@@ -1018,21 +1018,30 @@ __global__ __launch_bounds__(64 * NWD, 2) void attn_decode_kernel(const LmAttn a
   const int kwave = wave % KW, heads_each = (G + PARTS - 1) / PARTS, g_lo = wave / KW * heads_each, g_hi = min(G, g_lo + heads_each);
   constexpr bool AHEAD = TK == 32;  // values of all heads of the wave requested behind the first keys
   constexpr int UG = D >= 3 ? 2 : 4, NB = TK / 32, VB = AHEAD && HPW * C <= 8 ? HPW : 2;
+  // queries, the mixture (transposed, heads padded to a multiple of four) and slopes: the first round's loads go out before the keys', without a wait between
+  constexpr int MIX = 2, T = 64 * NWD;
+  auto mix_at = [&](int e) { return min(e % hs, H - 1) * H + min(e / hs, H - 1); };
+  const u32x4 q_in = *(const u32x4*)((const bf16_t*)a.q + (int64_t)row * H * dp + min(tid * 8, H * dp - 8));
+  float mix_in[MIX], slope_in = a.slope[min(tid, H - 1)];
+#pragma unroll
+  for (int k = 0; k < MIX; ++k) mix_in[k] = a.mix[mix_at(tid + T * k)];
+  __builtin_amdgcn_sched_barrier(0);
   auto stage = [&] {
-    for (int c = tid * 8; c < H * dp; c += 512 * NWD) *(u32x4*)(qs + c) = *(const u32x4*)((const bf16_t*)a.q + (int64_t)row * H * dp + c);
-    for (int e = tid; e < H * hs; e += 64 * NWD) {  // transposed, heads padded to a multiple of four
-      const int h = e % hs, g = e / hs;
-      mixT[e] = h < H ? a.mix[h * H + g] : 0.f;
-    }
-    for (int h = tid; h < hs; h += 64 * NWD) {
-      ms[h] = -INFINITY;
-      ls[h] = 0.f;
-      sl[h] = h < H ? a.slope[h] : 0.f;
+    if (tid * 8 < H * dp) *(u32x4*)(qs + tid * 8) = q_in;
+    for (int c = (tid + T) * 8; c < H * dp; c += T * 8) *(u32x4*)(qs + c) = *(const u32x4*)((const bf16_t*)a.q + (int64_t)row * H * dp + c);
+#pragma unroll
+    for (int k = 0; k < MIX; ++k)
+      if (tid + T * k < H * hs) mixT[tid + T * k] = (tid + T * k) % hs < H ? mix_in[k] : 0.f;
+    for (int e = tid + T * MIX; e < H * hs; e += T) mixT[e] = e % hs < H ? a.mix[mix_at(e)] : 0.f;
+    if (tid < hs) {  // (at most 64 heads)
+      ms[tid] = -INFINITY;
+      ls[tid] = 0.f;
+      sl[tid] = tid < H ? slope_in : 0.f;
     }
     __syncthreads();
   };
   if (!AHEAD) stage();
-  for (int j0 = k0; j0 <= k1; j0 += TK) {
+  for (int j0 = k0; j0 <= k1; j0 += TK) {  // (AHEAD: once)
     const int n = min(TK, k1 + 1 - j0);
     // scores of keys 16 kwave .. 16 kwave + 15, this wave's key heads, 16 query heads of one key head per matrix product
     const bf16_t* kw = Kb + key_block(j0 + 16 * kwave, 0, G, dp) + (kwave & 1) * (D * 512) + 8 * lane;
@@ -1079,7 +1088,7 @@ __global__ __launch_bounds__(64 * NWD, 2) void attn_decode_kernel(const LmAttn a
 #pragma unroll
       for (int u = 0; u < VB; ++u) load_v(u);
       __builtin_amdgcn_sched_barrier(0);
-      if (j0 == k0) stage();
+      stage();
       for (int g0 = g_lo; g0 < g_hi; g0 += 2 * UG) {
         scores(0, g0);
         if (g0 + 2 * UG < g_hi) load(0, g0 + 2 * UG);
@@ -1155,6 +1164,7 @@ __global__ __launch_bounds__(64 * NWD, 2) void attn_decode_kernel(const LmAttn a
         }
       }
     }
+    if (AHEAD) break;
     __syncthreads();
   }
 #pragma unroll
@@ -1179,30 +1189,59 @@ __global__ __launch_bounds__(64 * NWD, 2) void attn_decode_kernel(const LmAttn a
     }
 }
 
-// grid (heads, sequences)
+// grid (heads, sequences).  Few sequences: a chain of loads again, so a split's maximum and sum are read once and together, and the sums four splits
+// at a time up to the last that saw a key (n_split is what the longest sequence would need; up to 1024).
 __global__ __launch_bounds__(256) void attn_combine_kernel(const LmAttn a) {
-  __shared__ float ws[1024], sums[256], red[4];
+  __shared__ float ws[1024], sums[256], red[4], red_last[4];
   const int h = blockIdx.x, seq = blockIdx.y, tid = threadIdx.x, w = a.heads * a.vp, n = a.n_split;
   const int64_t stride = w + 2 * a.heads;
   const float* p = a.part + (int64_t)seq * n * stride;
-  float m = -INFINITY;
-  for (int s = tid; s < n; s += 256) m = fmaxf(m, p[s * stride + w + 2 * h]);
-  m = wave_max(m);
-  if ((tid & 63) == 0) red[tid >> 6] = m;
+  constexpr int R = 4;
+  md_f32x2 ml[R];
+#pragma unroll
+  for (int j = 0; j < R; ++j) ml[j] = *(const md_f32x2*)(p + min(tid + 256 * j, n - 1) * stride + w + 2 * h);
+  float m = -INFINITY, last = -1.f;
+#pragma unroll
+  for (int j = 0; j < R; ++j)
+    if (tid + 256 * j < n) {
+      m = fmaxf(m, ml[j][0]);
+      if (ml[j][1] != 0.f) last = (float)(tid + 256 * j);
+    }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    m = fmaxf(m, __shfl_xor(m, o, 64));
+    last = fmaxf(last, __shfl_xor(last, o, 64));
+  }
+  if ((tid & 63) == 0) {
+    red[tid >> 6] = m;
+    red_last[tid >> 6] = last;
+  }
   __syncthreads();
   m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  const int live = 1 + (int)fmaxf(fmaxf(red_last[0], red_last[1]), fmaxf(red_last[2], red_last[3]));
   float l = 0.f;
-  for (int s = tid; s < n; s += 256) {
-    const float ls = p[s * stride + w + 2 * h + 1], f = ls == 0.f ? 0.f : expf(p[s * stride + w + 2 * h] - m);
-    ws[s] = f;
-    l += ls * f;
-  }
-  l = block_sum_256(l, red);  // (its barriers also publish ws)
+#pragma unroll
+  for (int j = 0; j < R; ++j)
+    if (tid + 256 * j < n) {
+      const float ls = ml[j][1], f = ls == 0.f ? 0.f : expf(ml[j][0] - m);
+      ws[tid + 256 * j] = f;
+      l += ls * f;
+    }
+  __syncthreads();  // (red is read above and written below)
+  l = block_sum_256(l, red);
   const int groups = 256 / a.vp, e = tid % a.vp, g = tid / a.vp;
   float o = 0.f;
   if (g < groups)
-    for (int s = g; s < n; s += groups)
-      if (ws[s] != 0.f) o += ws[s] * p[s * stride + h * a.vp + e];  // an empty split wrote no sums
+    for (int s0 = g; s0 < live; s0 += groups * R) {
+      float v[R];
+#pragma unroll
+      for (int j = 0; j < R; ++j) v[j] = p[min(s0 + groups * j, live - 1) * stride + h * a.vp + e];
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        const int s = s0 + groups * j;
+        if (s < live && ws[s] != 0.f) o += ws[s] * v[j];  // an empty split wrote no sums
+      }
+    }
   sums[tid] = o;
   __syncthreads();
   if (tid >= a.vp) return;
