@@ -91,7 +91,7 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
     for (int e = 0; e < 4; ++e) norm_w[e] = a.norm.w[(int64_t)min(c + e, a.width - 1) * a.norm.stride];  // (columns beyond hold zeros)
   }
   const float* sq_row = EPI == EPI_RESID ? a.head_sumsq + (int64_t)min(m, a.rows - 1) * a.heads : nullptr;
-  if (EPI == EPI_RESID && a.head_sumsq && wave < M16)
+  if (EPI == EPI_RESID && a.head_sumsq && a.groups == 1 && wave < M16)
 #pragma unroll
     for (int j = 0; j < HEADS; ++j) head_sq[j] = sq_row[min(4 * j + g, a.heads - 1)];
 
@@ -159,6 +159,23 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
       if (r == 0 && m < 16 * M16) row_scale[m] = a.sumsq ? 1.0f / sqrtf(v / (float)a.width + a.eps) : 1.0f;
     }
   }
+  // norm groups: a wave's eighth of K lies in one of them.  Lane row g adds up the eighths 2 g and 2 g + 1 of the heads
+  float eighth[2] = {0.f, 0.f};
+  if (EPI == EPI_RESID && a.head_sumsq && a.groups > 1 && wave < M16) {
+    const int per = a.heads / 8;
+    float q[2][HEADS];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < HEADS; ++j) q[i][j] = sq_row[(2 * g + i) * per + min(j, per - 1)];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+      for (int j = 0; j < HEADS; ++j)
+        if (j < per) eighth[i] += q[i][j];
+      for (int j = HEADS; j < per; ++j) eighth[i] += sq_row[(2 * g + i) * per + j];
+    }
+  }
 #pragma unroll
   for (int i = 0; i < M16; ++i) {
     // an operand's 8 columns: lanes 0 .. 31 of the first half's product, 32 .. 63 of the other's; DIAG: rows 0 .. 7, and 8 .. 15.  The second
@@ -201,8 +218,25 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
     st4(a.out + m * a.ldo + in_chunks(c, a.out_chunk), y);
   } else {
     const float *in_w = a.next, *out_w = a.prev ? a.prev + ns : nullptr, *mix = a.prev ? a.prev + 2 * ns : nullptr;
-    f32x4 y = total(lane);
-    if (a.head_sumsq) {
+    static_assert(EPI != EPI_RESID || W == 8, "norm groups: eighths of K");
+    f32x4 y;
+    if (a.head_sumsq && a.groups > 1) {
+      float q[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) q[k] = __shfl(eighth[k & 1], (k >> 1) * 16 + r, 64);
+      if (a.groups <= 4)
+#pragma unroll
+        for (int k = 0; k < 8; k += 2) q[k] = q[k + 1] = q[k] + q[k + 1];
+      if (a.groups <= 2)
+#pragma unroll
+        for (int k = 0; k < 8; k += 4) q[k] = q[k + 1] = q[k + 2] = q[k + 3] = q[k] + q[k + 2];
+      y = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < W; ++w) y += red[w][wave][lane] * (1.0f / sqrtf(q[w & 7] / (float)a.normed + a.eps));
+    } else {
+      y = total(lane);
+    }
+    if (a.head_sumsq && a.groups == 1) {
       float q = 0.f;
 #pragma unroll
       for (int j = 0; j < HEADS; ++j)

@@ -342,7 +342,8 @@ struct Step {
     if (unnormed) {
       g.head_sumsq = w.head_sumsq;
       g.heads = unnormed->heads;
-      g.normed = unnormed->heads * unnormed->vdim;
+      g.groups = unnormed->norm_groups;
+      g.normed = unnormed->heads * unnormed->vdim / unnormed->norm_groups;
       unnormed = nullptr;
     }
     sumsq = w.sumsq;
@@ -519,7 +520,10 @@ struct Step {
     a.u = w.conv_out; a.dt = w.dt; a.seg = w.seg; a.seg_decay = w.seg_decay;
     if (m->dtype == MD_DTYPE_BF16) {
       if (b->max_len == 1 && (g_lm_kernels & 2) && lm_ssm_decode_takes(a)) {
-        if (few && l.norm_groups == 1) {
+        // (the product's waves take an eighth of K each)
+        const bool eighths = (l.norm_groups == 2 || l.norm_groups == 4 || l.norm_groups == 8) && l.heads % 8 == 0 && l.vdim == l.vdim_pad &&
+                             l.out_proj.k_pad == l.heads * l.vdim && l.out_proj.k_pad % 512 == 0;
+        if (few && (l.norm_groups == 1 || eighths)) {
           a.sumsq = w.head_sumsq;
           unnormed = &l;
         }

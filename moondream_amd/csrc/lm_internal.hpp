@@ -171,7 +171,7 @@ struct LmSsm {
   void* out;
   int64_t ldo;
   int out_chunk;
-  float* sumsq;          // decode, one norm group: [n_rows][heads], rows before their norm; nullptr: normed rows
+  float* sumsq;          // decode: [n_rows][heads], rows before their norm; nullptr: normed rows
   void* u;               // [n_rows][cw]: x | B | C behind the convolution and silu
   float* dt;             // [n_rows][heads], behind softplus
   float *seg, *seg_decay;  // matrix-core prefill in segments: [n_seq][n_seg][heads][vp][dp], [n_seq][n_seg][heads]
@@ -254,8 +254,9 @@ struct LmStepGemm {
   md_rms_weight norm;
   float* sumsq_out;      // [rows][width_pad / 8]
   // ... of rows of a before a norm over `normed` elements: [rows][heads] sums of squares; nullptr: complete rows
+  // groups (2, 4, 8) of as many heads each: heads % 8 == 0, k / 64 a multiple of 8 and all of it theirs
   const float* head_sumsq;
-  int heads, normed;
+  int heads, groups, normed;
 };
 md_status lm_step_rows(const LmStepGemm& a, int n, hipStream_t s);   // out = a w^T + bias
 md_status lm_step_silu(const LmStepGemm& a, hipStream_t s);          // out = silu(gate) * input

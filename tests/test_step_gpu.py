@@ -268,6 +268,30 @@ def test_rows_of_many_columns():
             m.close_sequence(s)
 
 
+@pytest.mark.parametrize("groups", [1, 2, 4, 8])
+@pytest.mark.parametrize("heads,vdim,state,width", [(16, 32, 32, 64), (40, 64, 16, 136), (88, 64, 16, 72)], ids=str)
+def test_state_space_norm_groups_of_a_step(heads, vdim, state, width, groups):
+    """The same with groups that are eighths, quarters and halves of the projection's K: more than eight heads to an eighth, and 49 rows, normed by a launch."""
+    cfg = U.stream_config([(U.ssm(heads, vdim, state, norm_groups=groups), U.dense(64)), (U.ssm(heads, vdim, state, norm_groups=groups), U.dense(96))],
+                          width=width, vocab=120, streams=2, positions=16)
+    m, w = build(cfg), U.weights(cfg, 3, 1.5)
+    ts = [U.tokens(3, cfg["vocab"], i) for i in range(49)]
+    want = torch.stack([O.forward(cfg, w, t) for t in ts])
+
+    def errors(n):
+        slots = [m.open_sequence() for _ in range(n)]
+        e = torch.stack([U.logit_errors(m.step([(s, [t[k]], [0]) for s, t in zip(slots, ts)]), want[:n, k]) for k in range(3)])
+        for s in slots:
+            m.close_sequence(s)
+        return e
+
+    whole = errors(49)
+    assert float(whole.median()) < 3e-2
+    for n in (1, 8, 9, 33, 48):  # (a bound on distributions, as below; groups of few heads enlarge single rows)
+        e, ref = errors(n).flatten().sort().values, whole[:, :n].flatten().sort().values
+        assert float(e.median()) < (1.5 if n >= 8 else 4) * float(ref.median()) and float(e[int(0.8 * len(e))]) < (2 if n >= 8 else 8) * float(ref[int(0.8 * len(ref))]), (n, e, ref)
+
+
 @pytest.mark.parametrize("heads,vdim,state,width", [(2, 32, 32, 64), (3, 20, 10, 72), (40, 32, 16, 136), (5, 100, 130, 320), (33, 72, 64, 64)], ids=str)
 def test_state_space_norm_of_a_step(heads, vdim, state, width):
     """Rows whose norm the output projection finishes: heads padded, more heads than a lane holds sums of, at the edges of the row tiles."""
