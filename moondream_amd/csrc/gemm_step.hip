@@ -467,6 +467,15 @@ md_status rows(const LmStepGemm& a, hipStream_t s) {
   return a.n <= 256 * 32 && most(8) < most(16) ? launch<0, 1, 4, 2, EPI_ROWS, S>(a, s) : launch<0, 2, 8, 1, EPI_ROWS, S>(a, s);
 }
 
+// Waves that share K, up to 8 rows.  Up to one workgroup of 8 columns per CU the chain of loads bounds it: eight (2048 wide, 256 / 2048 columns, 1 row: 5.4 /
+// 6.1 us, four 6.3 / 6.8, two 8.0 / 8.5; 4096 wide 7.8 / 8.9, two 13.6 / 15.3).  More: four (4096 wide, 10944 columns: 32 us, two 44, eight 34; 1024 wide, 5440
+// columns: 6.6, 6.8, 6.7), but two where the workgroups are many and a wave's half of K is of 8 to 16 units (2048 wide, 5440 / 8192 columns: 10.1 / 13.3
+// us, four 10.8 / 14.3; 2816 columns: 9.0 and 7.7).
+md_status gates(const LmStepGemm& a, hipStream_t s) {
+  if (a.n <= 256 * 8) return launch<0, 2, 8, 1, EPI_SILU, 1>(a, s);
+  return a.n > 2 * 256 * 8 && a.k > 1024 && a.k <= 2048 ? launch<0, 2, 2, 1, EPI_SILU, 1>(a, s) : launch<0, 2, 4, 1, EPI_SILU, 1>(a, s);
+}
+
 // Up to 8 rows four units per batch where K is long (5440: 6.8 us against 7.7; 2048: 4.4 either way)
 template <int S>
 md_status resid(const LmStepGemm& a, hipStream_t s) {
@@ -493,7 +502,7 @@ md_status lm_step_silu(const LmStepGemm& g, hipStream_t s) {
   MD_CHECK_ARG(takes(g) && g.ff_pad % 64 == 0);
   LmStepGemm a = g;
   a.n = a.ff_pad;
-  return a.rows <= 8 ? launch<0, 2, 2, 1, EPI_SILU, 1>(a, s) : tall_by_columns<EPI_SILU, 1>(a, s);
+  return a.rows <= 8 ? gates(a, s) : tall_by_columns<EPI_SILU, 1>(a, s);
 }
 
 md_status lm_step_resid(const LmStepGemm& g, hipStream_t s) {

@@ -101,6 +101,23 @@ def test_rows_of_wide_models(width):
             m.close_sequence(s)
 
 
+@pytest.mark.parametrize("width,ff", [(64, 40), (600, 2040), (320, 2112), (1032, 4160), (1000, 4160), (2112, 4160)], ids=str)
+def test_gates_of_up_to_eight_rows(width, ff):
+    """Gates whose K two, four and eight waves share: one unit of K for eight waves, the most columns of one workgroup per CU and the first of
+    more, and either side of the widths that two waves take."""
+    cfg = U.stream_config([(U.latent(2, 32, 32, 64), U.dense(ff))], width=width, vocab=120, streams=2, positions=8)
+    m, w = build(cfg), U.weights(cfg, 3, 1.5)
+    ts = [U.tokens(2, 120, i) for i in range(9)]
+    want = torch.stack([O.forward(cfg, w, t) for t in ts])
+    for n in (1, 8, 9):
+        slots = [m.open_sequence() for _ in range(n)]
+        for k in range(2):
+            got = m.step([(s, [t[k]], [0]) for s, t in zip(slots, ts)])
+            assert float(U.logit_errors(got, want[:n, k]).max()) < 7e-2, (n, k)
+        for s in slots:
+            m.close_sequence(s)
+
+
 WIDE = [U.stream_config([(U.ssm(m, 32, 32), U.dense(ff)), (U.latent(4, 32, 32, 64), U.dense(96))], width=64, vocab=v, positions=8)
         for m, ff, v in ((8, 2112, 120), (64, 2120, 200), (130, 4168, 120), (128, 6208, 16500))]
 
