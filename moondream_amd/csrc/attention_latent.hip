@@ -14,6 +14,8 @@
 // Scores, softmax and sums are fp32; q, c, the expanded keys / values, softmax weights and queries in the latent space enter matrix products as bf16.
 #include "lm_internal.hpp"
 
+#include <algorithm>
+
 namespace {
 
 constexpr float LOG2E = 1.4426950408889634f;
@@ -472,11 +474,11 @@ __global__ __launch_bounds__(64 * WK * WH * WR, 2) void latent_decode_kernel(con
   }
 }
 
-// grid (heads, sequences / SEQ, columns / 32): sum over the splits, then eight threads per output column share the latent's columns.  SEQ 1: the
-// waves share the splits of one sequence; 4: a wave per sequence, and every weight that is read serves four.  What bounds it is the chain of
-// loads (weights of a head are 64 to 128 KB, sums as much): the weights are under way before the sums are looked up, and 32 columns per workgroup
-// put several on every CU, though they add up the splits each for itself.  20 sequences, 16 heads of 128, rank 512: 17.6 us with all columns of a
-// head in a workgroup and its weights behind the sums, 10.0 this way; 23 of 32 x 64: 10.0 and 8.2, one 9.7 and 7.1; 40 of 32 x 64, rank 256: 7.7 and 7.0.
+// grid (heads, sequences / SEQ, parts of the columns): sum over the splits, then eight threads per output column share the latent's columns, 32 columns
+// after the other.  SEQ 1: the waves share the splits of one sequence; 4: a wave per sequence, and every weight that is read serves four.  What bounds it is
+// the chain of loads (weights of a head are 64 to 128 KB, sums as much): the weights are under way before the sums are looked up, and a head's columns go to
+// several workgroups, which add up the splits each for itself.  20 sequences, 16 heads of 128, rank 512: 17.6 us with all columns of a head in a workgroup and
+// its weights behind the sums, 10.0 with 32 columns per workgroup; 23 of 32 x 64: 10.0 and 8.2, one 9.7 and 7.1; 40 of 32 x 64, rank 256: 7.7 and 7.0.
 constexpr int MAX_SPLITS = 64, OUT_COLS = 32, MAX_RANK = 512;
 template <int SEQ>
 __global__ __launch_bounds__(256) void latent_out_kernel(const LmLatent a) {
@@ -484,11 +486,14 @@ __global__ __launch_bounds__(256) void latent_out_kernel(const LmLatent a) {
   extern __shared__ __attribute__((aligned(16))) float zsm[];  // [4][rp]
   __shared__ float fs[4][MAX_SPLITS];
   const int h = blockIdx.x, s0 = blockIdx.y * SEQ, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, R = a.rp, n = a.n_split;
-  const int s = tid & 7, e = blockIdx.z * OUT_COLS + (tid >> 3);
-  const bf16_t* w = (const bf16_t*)a.up_kv.w + ((int64_t)a.heads * a.dp + h * a.vp + e) * R + 8 * s;
+  const int s = tid & 7;
   u32x4 wv[MAX_RANK / 64];
+  auto load = [&](int e) {
+    const bf16_t* w = (const bf16_t*)a.up_kv.w + ((int64_t)a.heads * a.dp + h * a.vp + e) * R + 8 * s;
 #pragma unroll
-  for (int i = 0; i < MAX_RANK / 64; ++i) wv[i] = *(const u32x4*)(w + (64 * i < R ? 64 * i : 0));
+    for (int i = 0; i < MAX_RANK / 64; ++i) wv[i] = *(const u32x4*)(w + (64 * i < R ? 64 * i : 0));
+  };
+  load(blockIdx.z * OUT_COLS + (tid >> 3));
   const int mine = SEQ == 1 ? s0 : min(s0 + wave, a.r.n_seq - 1);
   const int64_t base = ((int64_t)mine * a.heads + h) * n;
   const float* pm = a.part + (int64_t)a.r.n_seq * a.heads * n * R + base * 2;
@@ -508,31 +513,43 @@ __global__ __launch_bounds__(256) void latent_out_kernel(const LmLatent a) {
     *(f32x4*)(zsm + wave * R + r) = z;
   }
   __syncthreads();
-  float o[SEQ];
+  for (int e0 = blockIdx.z * OUT_COLS; e0 < a.vp; e0 += gridDim.z * OUT_COLS) {
+    const int e = e0 + (tid >> 3);
+    float o[SEQ];
 #pragma unroll
-  for (int i = 0; i < SEQ; ++i) o[i] = 0.f;
+    for (int i = 0; i < SEQ; ++i) o[i] = 0.f;
 #pragma unroll
-  for (int i = 0; i < MAX_RANK / 64; ++i) {
-    if (64 * i >= R) break;
-    const f32x4 w0 = half8(wv[i], 0), w1 = half8(wv[i], 1);
-    const float* z = zsm + 64 * i + 8 * s;
+    for (int i = 0; i < MAX_RANK / 64; ++i) {
+      if (64 * i >= R) break;
+      const f32x4 w0 = half8(wv[i], 0), w1 = half8(wv[i], 1);
+      const float* z = zsm + 64 * i + 8 * s;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const f32x4 t = w0 * *(const f32x4*)(z + k * R) + w1 * *(const f32x4*)(z + k * R + 4);
-      o[SEQ == 1 ? 0 : k] += (t[0] + t[1]) + (t[2] + t[3]);
+      for (int k = 0; k < 4; ++k) {
+        const f32x4 t = w0 * *(const f32x4*)(z + k * R) + w1 * *(const f32x4*)(z + k * R + 4);
+        o[SEQ == 1 ? 0 : k] += (t[0] + t[1]) + (t[2] + t[3]);
+      }
     }
+    if (e0 + (int)gridDim.z * OUT_COLS < a.vp) load(e + gridDim.z * OUT_COLS);
+#pragma unroll
+    for (int i = 0; i < SEQ; ++i)
+#pragma unroll
+      for (int d = 1; d < 8; d <<= 1) o[i] += __shfl_xor(o[i], d, 64);
+    float v = o[0];
+#pragma unroll
+    for (int i = 1; i < SEQ; ++i) v = s == i ? o[i] : v;  // thread s writes sequence s
+    if (s >= SEQ || s0 + s >= a.r.n_seq) continue;
+    const int64_t row = a.r.seq_row0[s0 + s];
+    if (a.col_g >= 0) v *= sigmoid_f32(bf2f(((const bf16_t*)a.proj)[row * a.ldp + a.col_g + h * a.vp + e]));
+    ((bf16_t*)a.out)[row * a.ldo + in_chunks(h * a.vp + e, a.out_chunk)] = f2bf(v);
   }
-#pragma unroll
-  for (int i = 0; i < SEQ; ++i)
-#pragma unroll
-    for (int d = 1; d < 8; d <<= 1) o[i] += __shfl_xor(o[i], d, 64);
-  float v = o[0];
-#pragma unroll
-  for (int i = 1; i < SEQ; ++i) v = s == i ? o[i] : v;  // thread s writes sequence s
-  if (s >= SEQ || s0 + s >= a.r.n_seq) return;
-  const int64_t row = a.r.seq_row0[s0 + s];
-  if (a.col_g >= 0) v *= sigmoid_f32(bf2f(((const bf16_t*)a.proj)[row * a.ldp + a.col_g + h * a.vp + e]));
-  ((bf16_t*)a.out)[row * a.ldo + in_chunks(h * a.vp + e, a.out_chunk)] = f2bf(v);
+}
+
+// Parts of a head's columns: as many as give four workgroups per CU.  Beyond that adding up the splits again costs more than it hides.  A step of four layers of
+// this attention and little else, rank 512: 128 sequences, 128 heads of 128 (4096 workgroups) 659 us in one part, 698 in two, 778 in four; 16 of 128 (512) 294,
+// 281, 293; 64 sequences (256) 252, 235, 229.
+inline int out_parts(int workgroups, int tiles) {
+  const int most = std::max(1, std::min(tiles, 1024 / workgroups));
+  return (tiles + (tiles + most - 1) / most - 1) / ((tiles + most - 1) / most);
 }
 
 typedef void (*LatentKernel)(const LmLatent);
@@ -627,7 +644,8 @@ md_status lm_latent_decode(const LmLatent& a, hipStream_t s) {
   MD_TRY(md_launch_status());
   hipLaunchKernelGGL(k.attend, dim3(a.n_split, a.r.n_seq, (a.heads + 16 * k.head_tiles - 1) / (16 * k.head_tiles)), dim3(k.threads), k.lds, s, a);
   MD_TRY(md_launch_status());
-  if (a.r.n_seq >= 16) hipLaunchKernelGGL(latent_out_kernel<4>, dim3(a.heads, (a.r.n_seq + 3) / 4, a.vp / OUT_COLS), dim3(256), 4 * a.rp * 4, s, a);
-  else hipLaunchKernelGGL(latent_out_kernel<1>, dim3(a.heads, a.r.n_seq, a.vp / OUT_COLS), dim3(256), 4 * a.rp * 4, s, a);
+  const int seqs = a.r.n_seq >= 16 ? (a.r.n_seq + 3) / 4 : a.r.n_seq, z = out_parts(a.heads * seqs, a.vp / OUT_COLS);
+  if (a.r.n_seq >= 16) hipLaunchKernelGGL(latent_out_kernel<4>, dim3(a.heads, seqs, z), dim3(256), 4 * a.rp * 4, s, a);
+  else hipLaunchKernelGGL(latent_out_kernel<1>, dim3(a.heads, seqs, z), dim3(256), 4 * a.rp * 4, s, a);
   return md_launch_status();
 }

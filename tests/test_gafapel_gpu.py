@@ -80,6 +80,23 @@ def test_many_sequences_decode_together(dtype, count, heads, rank):
         assert U.logit_error(got[k], torch.stack([x[k] for x in want])) < TOL[dtype]
 
 
+@pytest.mark.parametrize("heads, vdim", [(40, 96), (72, 128), (9, 200)], ids=str)
+def test_columns_of_a_head_between_workgroups(heads, vdim):
+    """The last launch of a decode step's latent attention: a head's columns in one part, in as many as there are tiles, and in parts of which the
+    last has fewer tiles; one sequence per workgroup and four."""
+    cfg = U.stream_config([(U.latent(heads, 32, vdim, 100), None)], width=64, vocab=60, streams=2)
+    w = U.weights(cfg, 7)
+    m = load(cfg, w, BF16, max_batch=66, max_context=64)
+    ts = [U.tokens(3, 60, i) for i in range(66)]
+    want = torch.stack([O.forward(cfg, w, t) for t in ts])
+    for n in (1, 8, 12, 15, 16, 30, 66):
+        slots = [m.open_sequence() for _ in range(n)]
+        for k in range(3):
+            assert U.logit_error(m.step([(s, [t[k]], [0]) for s, t in zip(slots, ts)]), want[:n, k]) < TOL[BF16], (n, k)
+        for s in slots:
+            m.close_sequence(s)
+
+
 def _slow_state(heads, vdim, state):
     cfg = U.stream_config([(U.ssm(heads, vdim, state, conv=2), None)], width=64, vocab=50, streams=2)
     w = U.weights(cfg, 2)
