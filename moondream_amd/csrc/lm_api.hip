@@ -46,7 +46,7 @@ inline bool decode_regime(const md_lm_model* m, int rows) { return m->dtype == M
 // the sign of q . k is left, so a rounding of the norm at another place turns it over where q . k is small.  A step in which any sequence may
 // begin keeps the rounding of long prompts where a layer has retention: 12 tokens 1.78 ms, 1.29 this way.  Their sums and gates take no bias.)
 inline bool step_regime(const md_lm_model* m, const md_lm_batch* b) {
-  if (m->dtype != MD_DTYPE_BF16 || b->n_rows > LM_STEP_ROWS) return false;
+  if (m->dtype != MD_DTYPE_BF16 || b->n_rows > lm_step_most_rows(m->width_pad)) return false;
   for (int i = 0; i < m->n_layers; ++i) {
     const md_lm_layer& l = m->layers[i];
     if (l.experts > 0 && !lm_expert_step_takes(b->n_rows, l.top, l.experts)) return false;

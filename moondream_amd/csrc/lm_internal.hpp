@@ -226,10 +226,14 @@ struct LmRoute {
 
 // A product of a step of few rows and what follows it (gemm_step.hip).  Rows that a residual epilogue wrote carry no norm factor: it
 // comes from their sums of squares (sumsq; nullptr: the rows are complete).
-// Up to how many rows they are ahead: a step of 24 layers against the one of tile products and row-wise launches, 20 / 28 / 32 / 40 / 48 rows: 0.81 / 0.81 /
-// 0.84 / 0.90 / 0.94 of its time with state space and latent attention (1301, 1409, 1469, 1614, 1729 us with 32 heads of 64; 0.81 to 0.92 with 16 of 128),
-// 0.84 / 0.83 / 0.81 / 0.86 / 0.89 with attention and retention (1431, 1531, 1593, 1734, 1857 us).  At 64 rows gates would take 18.2 us against 16.3.
+// Up to how many rows they are ahead of the tile products and row-wise launches.  24 layers, 2048 wide, 20 / 28 / 32 / 40 / 48 rows: 0.81 / 0.81 / 0.84 / 0.90 /
+// 0.94 of a step's time with state space and latent attention (1301, 1409, 1469, 1614, 1729 us with 32 heads of 64; 0.81 to 0.92 with 16 of 128), 0.84 /
+// 0.83 / 0.81 / 0.86 / 0.89 with attention and retention (1431, 1531, 1593, 1734, 1857 us); at 64 rows gates would take 18.2 us against 16.3.  Every
+// workgroup reads all rows, so their share grows with the width, and from 2048 columns on there is more than one workgroup of the residual product per CU.
+// Four layers, 24 / 32 / 33 / 48 rows: 2560 wide 0.80 / 0.97 / 1.05 / 1.10, 3072 wide 0.80 / 0.96 / 1.01 / 1.10, 3584 wide 0.83 / 1.01 / 1.15 / 1.24, 4096
+// wide 0.75 / 0.92 / 1.00 / 1.08, 5120 wide 0.80 / 1.12 / 1.28 / 1.38.
 constexpr int LM_STEP_ROWS = 48;
+inline int lm_step_most_rows(int width_pad) { return width_pad <= 2048 ? LM_STEP_ROWS : width_pad <= 4096 ? 32 : 28; }
 struct LmStepGemm {
   const bf16_t* a;       // row m's columns 8 c .. 8 c + 7 at m * lda + c * chunk (plain rows: chunk 8)
   int64_t lda;

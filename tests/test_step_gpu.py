@@ -87,12 +87,12 @@ def test_decode_attention_of_many_columns(heads, dim, vdim, own):
 
 @pytest.mark.parametrize("width", [2112, 4160])
 def test_rows_of_wide_models(width):
-    """More sums of squares per row than one pass of the step products takes (widths above 2048)."""
+    """More sums of squares per row than one pass of the step products takes (widths above 2048), and the rows from which such widths take tiles."""
     cfg = U.stream_config([(U.ssm(2, 32, 32), U.dense(128)), (U.latent(2, 32, 32, 64), None)], width=width, vocab=120, streams=2, positions=8)
     m, w = build(cfg), U.weights(cfg, 3, 1.5)
-    ts = [U.tokens(2, 120, i) for i in range(28)]
+    ts = [U.tokens(2, 120, i) for i in range(49)]
     want = torch.stack([O.forward(cfg, w, t) for t in ts])
-    for n in (1, 9, 17, 28):
+    for n in (1, 9, 17, 28, 29, 32, 33, 49):
         slots = [m.open_sequence() for _ in range(n)]
         for k in range(2):
             got = m.step([(s, [t[k]], [0]) for s, t in zip(slots, ts)])
