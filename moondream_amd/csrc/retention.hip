@@ -423,10 +423,11 @@ RetKernel ret_chunk_pick(const LmRet& a) {
   }
 }
 
-// grid (heads, sequences).  Sixteen lanes per state row, sixteen rows at a time.  The state's bytes bound it where there are many sequences, the chain
-// of loads where there are few: everything that a thread reads is under way before the first use (R rows of up to 64 E columns per thread).  8
-// sequences, 16 heads of 128: 17.1 us with a row loaded after the other, 9.6 this way; 1 sequence, 32 heads of 64: 6.7 and 5.7; 64 of 32 x 64: 16.7 and 14.9.
-template <int R, int E>
+// grid (heads, sequences).  Sixteen lanes per state row, sixteen rows at a time, R rows of up to 64 E columns per thread.  Few sequences: the chain of loads
+// bounds it, and all of a head's rows are under way before the first use (ALL).  8 sequences, 16 heads of 128: 17.1 us with a row loaded after the other,
+// 9.6 this way; 1 sequence, 32 heads of 64: 6.7 and 5.7; 64 of 32 x 64: 16.7 and 14.9.  Many: the state's bytes, and more workgroups per CU hide more than
+// registers full of rows (128 sequences, 8 heads of 256: 122 us with all, 104 with a row after the other; 16 of 192: 141 and 114).
+template <int R, int E, bool ALL>
 __global__ __launch_bounds__(256) void ret_decode_kernel(const LmRet a) {
   __shared__ __attribute__((aligned(16))) float qs[256], ks[256], os[256];
   __shared__ float red[4];
@@ -436,15 +437,19 @@ __global__ __launch_bounds__(256) void ret_decode_kernel(const LmRet a) {
   const bf16_t* p = (const bf16_t*)a.proj + (int64_t)row * a.ldp;
   f32x4 S[R][E];
   float v[R];
+  auto load = [&](int e1) {
 #pragma unroll
-  for (int i = 0; i < R; ++i) {
+    for (int i = 0; i < R; ++i) {
+      const int e = e1 + e0 + 16 * i;
 #pragma unroll
-    for (int j = 0; j < E; ++j) {
-      S[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (pos > 0 && e0 + 16 * i < vp && 4 * l + 64 * j < dp) S[i][j] = *(const f32x4*)(st + (int64_t)(e0 + 16 * i) * dp + 4 * l + 64 * j);
+      for (int j = 0; j < E; ++j) {
+        S[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (pos > 0 && e < vp && 4 * l + 64 * j < dp) S[i][j] = *(const f32x4*)(st + (int64_t)e * dp + 4 * l + 64 * j);
+      }
+      v[i] = bf2f(p[a.col_v + h * vp + min(e, vp - 1)]);
     }
-    v[i] = bf2f(p[a.col_v + h * vp + min(e0 + 16 * i, vp - 1)]);
-  }
+  };
+  load(0);
   const float gate = bf2f(p[a.col_g + h * vp + min(tid, vp - 1)]), decay = a.decay[h];
   const float* cs = a.rope + (int64_t)pos * a.rot_dims;
   for (int d = tid; d < dp; d += 256) {
@@ -452,32 +457,44 @@ __global__ __launch_bounds__(256) void ret_decode_kernel(const LmRet a) {
     ks[d] = rotated(p + a.col_k + h * dp, d, a.rot_dims, cs) * a.scale;
   }
   __syncthreads();
+  for (int e1 = 0; e1 < vp; e1 += 16 * R) {
+    if (e1 > 0) load(e1);  // (ALL: once)
 #pragma unroll
-  for (int i = 0; i < R; ++i) {
-    const int e = e0 + 16 * i;
-    if (e >= vp) break;
-    float o = 0.f;
+    for (int i = 0; i < R; ++i) {
+      const int e = e1 + e0 + 16 * i;
+      if (e >= vp) break;
+      float o = 0.f;
 #pragma unroll
-    for (int j = 0; j < E; ++j) {
-      const int d = 4 * l + 64 * j;
-      if (d >= dp) continue;
-      const f32x4 k = *(const f32x4*)(ks + d), qv = *(const f32x4*)(qs + d);
-      const f32x4 s = decay * S[i][j] + k * v[i];
-      *(f32x4*)(st + (int64_t)e * dp + d) = s;
-      o += s[0] * qv[0] + s[1] * qv[1] + s[2] * qv[2] + s[3] * qv[3];
+      for (int j = 0; j < E; ++j) {
+        const int d = 4 * l + 64 * j;
+        if (d >= dp) continue;
+        const f32x4 k = *(const f32x4*)(ks + d), qv = *(const f32x4*)(qs + d);
+        const f32x4 s = decay * S[i][j] + k * v[i];
+        *(f32x4*)(st + (int64_t)e * dp + d) = s;
+        o += s[0] * qv[0] + s[1] * qv[1] + s[2] * qv[2] + s[3] * qv[3];
+      }
+#pragma unroll
+      for (int m = 1; m < 16; m <<= 1) o += __shfl_xor(o, m, 64);
+      if (l == 0) os[e] = o;
     }
-#pragma unroll
-    for (int m = 1; m < 16; m <<= 1) o += __shfl_xor(o, m, 64);
-    if (l == 0) os[e] = o;
+    if (ALL) break;
   }
   __syncthreads();
   const float o = tid < vp ? os[tid] : 0.f;
   const float ss = block_sum_256(o * o, red);
   if (tid < vp) ((bf16_t*)a.out)[(int64_t)row * a.ldo + in_chunks(h * vp + tid, a.out_chunk)] = f2bf(o / sqrtf(ss / (float)a.vdim + a.eps) * silu_f32(gate));
 }
-template <int R>
+template <int R, bool ALL>
 RetKernel ret_decode_by_width(int dp) {
-  return dp <= 64 ? ret_decode_kernel<R, 1> : dp <= 128 ? ret_decode_kernel<R, 2> : ret_decode_kernel<R, 4>;
+  return dp <= 64 ? ret_decode_kernel<R, 1, ALL> : dp <= 128 ? ret_decode_kernel<R, 2, ALL> : ret_decode_kernel<R, 4, ALL>;
+}
+// All rows at once as long as every workgroup's registers are on the chip at the same time, two rows after the other beyond.  A step of four layers of retention and
+// little else, all / two: 8 heads of 256, 32 sequences 187 / 220 us, 64 400 / 377; 16 of 128, 64 sequences 241 / 252, 96 354 / 338; 32 of 64, 64
+// sequences 188 / 188, 128 297 / 283; 16 of 192, 32 sequences 242 / 223.
+RetKernel ret_decode_pick(const LmRet& a) {
+  const int rows = a.vp <= 32 ? 2 : a.vp <= 64 ? 4 : a.vp <= 128 ? 8 : 16, columns = a.dp <= 64 ? 1 : a.dp <= 128 ? 2 : 4, workgroups = a.heads * a.r.n_seq;
+  if (workgroups > 2048 || workgroups * rows * columns > 256 * 64) return ret_decode_by_width<2, false>(a.dp);
+  return rows == 2 ? ret_decode_by_width<2, true>(a.dp) : rows == 4 ? ret_decode_by_width<4, true>(a.dp) : rows == 8 ? ret_decode_by_width<8, true>(a.dp) : ret_decode_by_width<16, true>(a.dp);
 }
 
 }  // namespace
@@ -498,7 +515,6 @@ md_status lm_ret_mfma(const LmRet& a, hipStream_t s) {
 
 bool lm_ret_decode_takes(const LmRet& a) { return a.dp <= 256 && a.vp <= 256; }
 md_status lm_ret_decode(const LmRet& a, hipStream_t s) {
-  const RetKernel fn = a.vp <= 32 ? ret_decode_by_width<2>(a.dp) : a.vp <= 64 ? ret_decode_by_width<4>(a.dp) : a.vp <= 128 ? ret_decode_by_width<8>(a.dp) : ret_decode_by_width<16>(a.dp);
-  hipLaunchKernelGGL(fn, dim3(a.heads, a.r.n_seq), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(ret_decode_pick(a), dim3(a.heads, a.r.n_seq), dim3(256), 0, s, a);
   return md_launch_status();
 }

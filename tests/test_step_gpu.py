@@ -242,6 +242,28 @@ def test_prompts_that_join_a_running_step_round_alike(lens, going):
     assert torch.equal(m.step(entries)[: sum(lens)], alone)
 
 
+@pytest.mark.parametrize("heads,dim,vdim,most", [(6, 250, 200, 42), (33, 100, 130, 15), (16, 128, 128, 64), (40, 60, 40, 51)], ids=str)
+def test_retention_of_many_sequences(heads, dim, vdim, most):
+    """Decode steps whose workgroups hold all rows of a head's state (the most sequences that do, and one), and one sequence more, in which they take two
+    after the other: rows and columns that are no multiple of what a pass takes."""
+    cfg = U.config([U.retention(heads, dim, vdim)], width=64, vocab=60, ff=None)
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    w = U.weights(cfg, 3, 1.5)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=BF16, max_batch=most + 1, max_context=64)
+    ts = [U.tokens(6, 60, i) for i in range(most + 1)]
+    want = torch.stack([O.forward(cfg, w, t) for t in ts])
+    for n in (1, most, most + 1):
+        slots = [m.open_sequence() for _ in range(n)]
+        m.step([(s, t[:3], []) for s, t in zip(slots, ts)])
+        for k in range(3, 6):
+            got = m.step([(s, [t[k]], [0]) for s, t in zip(slots, ts)])
+            assert float(U.logit_errors(got, want[:n, k]).max()) < 7e-2, (n, k)
+        for s in slots:
+            m.close_sequence(s)
+
+
 @pytest.mark.parametrize("lens", [[1100], [517, 3, 580]], ids=str)
 def test_state_space_prompts_that_fill_the_chip(lens):
     """Rows and columns enough for the convolution's 16 rows per thread (8224 columns), and a token behind each prompt, whose window is what
