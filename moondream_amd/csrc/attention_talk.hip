@@ -511,10 +511,18 @@ __host__ __device__ constexpr TalkLds talk_lds(int hpad, int dp, int nw) {
   return l;
 }
 
+// Order of a step's tiles, as workgroups go to XCDs and their engines in turn (so neighbours have to be alike) and an XCD's CUs share keys and values in L2:
+//   ROUNDS  every eighth tile of a sequence to an XCD, in eight rounds over the sequences, so that the last tiles are short
+//   WHOLE   whole sequences to an XCD, tile by tile
+//   ACROSS  the last tile of every sequence, then the ones before it, so turned that any sequence's go evenly to the 32 engines
+// Longest first in each.  32 heads of 64: 11 ragged prompts, 13250 tokens, 699 us with a run of tiles per XCD, shortest first, 513 in ROUNDS; 3 x 2048 tokens 544 and
+// 330; 8 x 2048 817, 785 and 691 WHOLE (launches of one after the other; 814 WHOLE in a whole pass, 915 with a run per XCD).  Persistent workgroups with a
+// queue per XCD: 697, 460 and 1064, the loop around the tile costs registers.
+enum { TALK_ROUNDS, TALK_WHOLE, TALK_ACROSS };
+
 // Parts of a tile's keys: a tile's place among all tiles of a step (a sequence has at most len / 16 + 2), and what one part leaves
-constexpr int TALK_ROUNDS = 8, TALK_PARTS = 1536, TALK_LEAST = 3;  // parts of a step at most; 64 keys of a part at least
-__host__ __device__ inline int talk_rounds(int tiles8, int parts) { return parts > 1 ? 1 : tiles8 < TALK_ROUNDS ? tiles8 : TALK_ROUNDS; }
-__host__ __device__ inline bool talk_few(int tiles, int parts) { return parts == 1 && tiles < 16; }  // short sequences: tile after tile
+constexpr int TALK_TURNS = 8, TALK_PARTS = 1536, TALK_LEAST = 3;  // parts of a step at most; 64 keys of a part at least
+__host__ __device__ inline int talk_turns(int tiles8, int parts) { return parts > 1 ? 1 : tiles8 < TALK_TURNS ? tiles8 : TALK_TURNS; }
 inline int talk_longest(int span) { return (span + 31 + 63) / 64; }  // of 64 keys each; the first may begin before the chunk
 __device__ __forceinline__ int talk_slot(int row0, int seq, int tile) { return row0 / 16 + 2 * seq + tile; }
 __host__ __device__ inline int64_t talk_part_floats(int heads, int vp) { return (int64_t)heads * (16 * vp + 32); }
@@ -545,19 +553,26 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void attn_mfma_kernel(const LmAttn
   float* mss = (float*)(smem + L.ms);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, q = lane >> 4;
 
-  // which tile: every eighth one of a sequence to an XCD (its CUs share the sequence's keys and values in L2), longest first; whole tiles in eight rounds
-  // over the sequences, so that the last ones are short; parts one after the other.  Workgroups go to XCDs and their engines in turn, so neighbours have to
-  // be alike; a single sequence's parts begin at another engine each.  Equal sequences in eights: whole sequences to an XCD.
-  // (11 ragged prompts, 13250 tokens, 32 heads of 64: 699 us with a run of tiles per XCD, shortest first, 513 this way; 3 x 2048 tokens 544 and 330, 8 x 2048
-  // 817 and 691, 785 where XCDs share the sequences.  Persistent workgroups with a queue per XCD: 697, 460 and 1064, the loop around the tile costs
-  // registers.)
-  const int tiles = (a.r.max_len + 30) / 16, tiles8 = (tiles + 7) >> 3, rounds = talk_rounds(tiles8, a.n_split), per = (tiles8 + rounds - 1) / rounds;
-  const int xcd = blockIdx.x & 7, item = blockIdx.x >> 3, part = a.n_split > 1 ? item / (per * a.r.n_seq) : 0, at = item - part * per * a.r.n_seq;
-  const bool few = talk_few(tiles, a.n_split), eights = a.n_split == 1 && a.r.n_seq % 8 == 0 && a.r.n_rows == a.r.n_seq * a.r.max_len;
-  const int seq = few ? blockIdx.x / tiles : eights ? 8 * (item % (a.r.n_seq / 8)) + xcd : at / per % a.r.n_seq;
-  const int nth = few      ? blockIdx.x % tiles
-                  : eights ? item / (a.r.n_seq / 8)
-                           : (at / (per * a.r.n_seq) * per + (at + (a.r.n_seq == 1 ? part : 0)) % per) * 8 + ((xcd + seq) & 7);
+  // which tile, counted from the sequence's last, and which part of its keys
+  const int tiles = (a.r.max_len + 30) / 16, N = a.r.n_seq, xcd = blockIdx.x & 7, item = blockIdx.x >> 3;
+  int seq, nth, part = 0;
+  if (a.order == TALK_ACROSS) {
+    const int rank = blockIdx.x / N;
+    part = rank / tiles;
+    nth = rank - part * tiles;
+    seq = (blockIdx.x + (N - nth * min(N & -N, 32) / 32 % N)) % N;  // (a step of N workgroups meets 32 / gcd(N, 32) engines)
+  } else if (a.order == TALK_WHOLE) {
+    const int each = (N + 7) >> 3;
+    nth = item / each;
+    seq = 8 * (item - nth * each) + xcd;
+    if (seq >= N) return;
+  } else {
+    const int tiles8 = (tiles + 7) >> 3, turns = talk_turns(tiles8, a.n_split), per = (tiles8 + turns - 1) / turns;
+    part = a.n_split > 1 ? item / (per * N) : 0;
+    const int at = item - part * per * N;
+    seq = at / per % N;
+    nth = (at / (per * N) * per + (at + (N == 1 ? part : 0)) % per) * 8 + ((xcd + seq) & 7);  // (a single sequence's parts begin at another engine each)
+  }
   const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, pos0 = a.r.seq_pos0[seq], slot = a.r.seq_slot[seq];
   const int tile = (pos0 + len - 1) / 16 - pos0 / 16 - nth;
   if (tile < 0) return;
@@ -943,13 +958,25 @@ size_t lm_attn_mfma_part_floats_most(int n_rows, int n_seq, int span, int heads,
   const int64_t parts = (talk_longest(span) + TALK_LEAST - 1) / TALK_LEAST, slots = n_rows / 16 + 2 * n_seq;
   return parts > 1 ? (size_t)std::min<int64_t>(TALK_PARTS, slots * parts) * talk_part_floats(heads, vp) : 0;
 }
-md_status lm_attn_mfma(const LmAttn& a, hipStream_t s) {
-  const TalkPick t = talk_pick(a);
+// WHOLE where the fullest XCD has at most a tenth more than the mean: two layers, 15 x 1000 tokens 2336 us in ROUNDS and 2117, 7 x 2000 + 1999 2978 and
+// 2834, 32 x 100 520 and 505.  Otherwise ACROSS for fewer than 16 tiles, which leave most XCDs or engines idle in ROUNDS, and for parts of several sequences: 63
+// single tokens beside a prompt of 40, 1900 keys, 1117 and 619 us, 39 beside 1500 tokens, 1000 keys, 937 and 750, 20 x 200 648 and 612 (one sequence after
+// the other).
+static int talk_order(const LmRows& r, int n_split) {
+  const int64_t fullest = (int64_t)((r.n_seq + 7) / 8) * 8 * r.max_len;
+  if (n_split == 1 && 10 * fullest <= 11 * (int64_t)r.n_rows) return TALK_WHOLE;
+  return (r.max_len + 30) / 16 < 16 || (n_split > 1 && r.n_seq > 1) ? TALK_ACROSS : TALK_ROUNDS;
+}
+md_status lm_attn_mfma(const LmAttn& args, hipStream_t s) {
+  const TalkPick t = talk_pick(args);
   if (!t.fn) return MD_ERR_UNSUPPORTED;
   MD_TRY(md_ensure_dynamic_lds((const void*)t.fn, 160 * 1024));
-  const int tiles = (a.r.max_len + 30) / 16;
-  const int tiles8 = (tiles + 7) / 8, rounds = talk_rounds(tiles8, a.n_split);
-  const int items = talk_few(tiles, a.n_split) ? tiles * a.r.n_seq : 8 * rounds * ((tiles8 + rounds - 1) / rounds) * a.r.n_seq * a.n_split;
+  LmAttn a = args;
+  a.order = talk_order(a.r, a.n_split);
+  const int tiles = (a.r.max_len + 30) / 16, tiles8 = (tiles + 7) / 8, turns = talk_turns(tiles8, a.n_split);
+  const int items = a.order == TALK_ACROSS  ? tiles * a.r.n_seq * a.n_split
+                    : a.order == TALK_WHOLE ? 8 * ((a.r.n_seq + 7) / 8) * tiles
+                                            : 8 * turns * ((tiles8 + turns - 1) / turns) * a.r.n_seq * a.n_split;
   hipLaunchKernelGGL(t.fn, dim3(items), dim3(t.waves * 64), t.lds, s, a);
   MD_TRY(md_launch_status());
   if (a.n_split == 1) return MD_OK;

@@ -112,6 +112,7 @@ struct LmAttn {
   int out_chunk;
   float* part;     // split keys: partial (m, l) and accumulators
   int n_split, split_keys;
+  int order;       // of the tiles of a matrix-core prefill (attention_talk.hip)
 };
 
 struct LmRet {

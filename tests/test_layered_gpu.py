@@ -406,9 +406,11 @@ def test_prompts_whose_tiles_are_cut_by_keys(heads, kv, dim, vdim, lens, chunk):
     assert float(U.logit_errors(got, want[0]).max()) < 7e-2
 
 
-@pytest.mark.parametrize("lens", [[530] * 8, [300] * 16, [530] * 7 + [10]], ids=["eight", "sixteen", "ragged"])
+@pytest.mark.parametrize("lens", [[530] * 8, [300] * 16, [530] * 7 + [10], [530] * 7 + [500], [300] * 15, [300] * 13, [90] * 16],
+                         ids=["eight", "sixteen", "ragged", "nearly", "fifteen", "thirteen", "short"])
 def test_prompts_of_eight_sequences(lens):
-    """More query tiles than CUs, eight equal sequences (one to an XCD), sixteen, and eight that differ."""
+    """More query tiles than CUs: eight equal sequences (one to an XCD), sixteen, eight that differ, little and much, a last eight of seven, thirteen;
+    short ones."""
     from moondream_amd.config import LayeredLMConfig
     from moondream_amd.layered_lm import LayeredLM
 
@@ -420,3 +422,27 @@ def test_prompts_of_eight_sequences(lens):
     want = [kept[tuple(t)] for t in ts]
     got = m.step([(m.open_sequence(), t, range(len(t))) for t in ts])
     assert float(U.logit_errors(got, torch.cat(want)).max()) < 7e-2
+
+
+@pytest.mark.parametrize("running,before,prompt", [(1, 300, 200), (3, 400, 290), (7, 20, 250), (15, 150, 40), (20, 300, 3), (31, 50, 330)], ids=str)
+def test_prompts_beside_single_tokens(running, before, prompt):
+    """Sequences of one query tile beside one of many, keys in parts and whole: every tile of every sequence."""
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    cfg = U.config([U.attention(4, 2, 32, 64, 2000)], width=96, vocab=120, ff=None)
+    w = U.weights(cfg, 3, 1.5)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=BF16, max_batch=running + 1, max_context=640)
+    ts = [U.tokens(before + 9 * (i % 4) + 1, 120, i % 5) for i in range(running)] + [U.tokens(prompt, 120, 77)]
+    kept = {tuple(t): O.forward(cfg, w, t) for t in {tuple(t): t for t in ts}.values()}
+    want = [kept[tuple(t)] for t in ts]
+    for at in (running, 0, running // 2):  # the prompt's place
+        slots = [m.open_sequence() for _ in ts]
+        m.step([(s, t[:-1], []) for s, t in zip(slots[:running], ts)])
+        entries = [(s, t[-1:], [0]) for s, t in zip(slots[:running], ts)]
+        ref = [x[-1:] for x in want[:running]]
+        entries.insert(at, (slots[running], ts[running], range(prompt)))
+        ref.insert(at, want[running])
+        assert float(U.logit_errors(m.step(entries), torch.cat(ref)).max()) < 7e-2
+        for s in slots:
+            m.close_sequence(s)
