@@ -520,7 +520,8 @@ __host__ __device__ constexpr TalkLds talk_lds(int hpad, int dp, int nw) {
 // queue per XCD: 697, 460 and 1064, the loop around the tile costs registers.
 enum { TALK_ROUNDS, TALK_WHOLE, TALK_ACROSS };
 
-// Parts of a tile's keys: a tile's place among all tiles of a step (a sequence has at most len / 16 + 2), and what one part leaves
+// Parts of a tile's keys: a tile's place among all tiles of a step (a sequence has at most len / 16 + 2), and what one part leaves.  Their room is the most that any
+// step up to the workspace's size can want, since a workspace of the largest serves all: at most 208 MB with 32 heads of 64 (1536 times 135 KB).
 constexpr int TALK_TURNS = 8, TALK_PARTS = 1536, TALK_LEAST = 3;  // parts of a step at most; 64 keys of a part at least
 __host__ __device__ inline int talk_turns(int tiles8, int parts) { return parts > 1 ? 1 : tiles8 < TALK_TURNS ? tiles8 : TALK_TURNS; }
 inline int talk_longest(int span) { return (span + 31 + 63) / 64; }  // of 64 keys each; the first may begin before the chunk
@@ -939,18 +940,28 @@ bool lm_attn_mfma_takes(const LmAttn& a) { return talk_pick(a).fn != nullptr; }
 // fewer tiles than CUs lasts as long as its longest: 32 heads of 64, one prompt of 1000 tokens (63 tiles) 163 us, in six parts 63; 700 tokens 117 and 57, 350
 // 67 and 48, 200 as before; two prompts of 1500 tokens 246 and 162, five ragged ones (3900 tokens, 244 tiles) 227 and 200.  Up to 128 tiles the parts fill the
 // CUs once, up to 256 twice.  With more tiles the sums of the parts (132 KB each, written and read) cost more than they even out: 3 x 2048 tokens
-// 341 us whole, 368 in three parts.
-int lm_attn_mfma_parts(int n_rows, int n_seq, int span, int* split_keys) {
-  const int tiles = n_rows / 16 + n_seq, longest = talk_longest(span);
+// 341 us whole, 368 in three parts.  So they do where nearly every CU has a tile and all are alike short, so the expected times are compared: two layers,
+// 12 x 300 tokens 594 us whole and 597 in parts, 6 x 600 677 and 692, 16 x 240 564 and 596, 10 x 400 674 (not cut).
+int lm_attn_mfma_parts(const LmRows& r, int ctx_rows, int span, int heads, int vp, int* split_keys) {
+  const int tiles = r.n_rows / 16 + r.n_seq, longest = talk_longest(span);
   int keys = longest;
   if (tiles <= 256) {
-    const double mean = longest - std::min<double>(n_rows / n_seq, span) / 128;
+    const double mean = longest - std::min<double>(r.n_rows / r.n_seq, span) / 128;
     keys = std::max(TALK_LEAST, (int)(1.4 * tiles * mean / (tiles <= 128 ? 256 : 512)));
-    const int most = TALK_PARTS / (n_rows / 16 + 2 * n_seq);
+    const int most = TALK_PARTS / (r.n_rows / 16 + 2 * r.n_seq);
     if (most < 2) keys = longest;
     else keys = std::max(keys, (longest + most - 1) / most);
   }
-  if (keys + 1 >= longest) keys = longest;
+  if (keys + 1 < longest) {
+    double mean = (ctx_rows - 0.5 * r.n_rows) / r.n_seq;  // keys of a tile
+    if (span < r.max_ctx) mean = std::min(mean, 0.5 * span);
+    mean /= 64;
+    const double most = 12 + 9.7 * keys, parts = tiles * (mean / keys + 0.5);
+    const double compute = parts <= 256 ? most : std::max(most, (12 * parts + 9.7 * tiles * mean) / 256 + most / 2);
+    if (compute + 5 + parts * talk_part_floats(heads, vp) * 4 / 2e6 >= 12 + 9.7 * longest) keys = longest;  // (sums: 1 MB in 0.5 us)
+  } else {
+    keys = longest;
+  }
   *split_keys = 64 * keys;
   return (longest + keys - 1) / keys;
 }
@@ -960,7 +971,7 @@ size_t lm_attn_mfma_part_floats_most(int n_rows, int n_seq, int span, int heads,
 }
 // WHOLE where the fullest XCD has at most a tenth more than the mean: two layers, 15 x 1000 tokens 2336 us in ROUNDS and 2117, 7 x 2000 + 1999 2978 and
 // 2834, 32 x 100 520 and 505.  Otherwise ACROSS for fewer than 16 tiles, which leave most XCDs or engines idle in ROUNDS, and for parts of several sequences: 63
-// single tokens beside a prompt of 40, 1900 keys, 1117 and 619 us, 39 beside 1500 tokens, 1000 keys, 937 and 750, 20 x 200 648 and 612 (one sequence after
+// single tokens beside a prompt of 40, 1900 keys, 1117 and 619 us, 39 beside 1500 tokens, 1000 keys, 937 and 713, 20 x 200 648 and 606 (one sequence after
 // the other).
 static int talk_order(const LmRows& r, int n_split) {
   const int64_t fullest = (int64_t)((r.n_seq + 7) / 8) * 8 * r.max_len;

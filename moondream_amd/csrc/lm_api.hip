@@ -438,7 +438,7 @@ struct Step {
     }
     MD_TRY(lm_attn_prep(m->dtype, a, s));
     if (m->dtype == MD_DTYPE_BF16 && b->max_len > 1 && (g_lm_kernels & 1) && lm_attn_mfma_takes(a)) {
-      a.n_split = lm_attn_mfma_parts(b->n_rows, b->n_seq, span, &a.split_keys);
+      a.n_split = lm_attn_mfma_parts(a.r, b->ctx_rows, span, l.heads, l.vdim_pad, &a.split_keys);
       return lm_attn_mfma(a, s);
     }
     return lm_attn_plain(m->dtype, a, s);

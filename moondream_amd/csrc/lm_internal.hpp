@@ -339,7 +339,7 @@ md_status lm_reduce_rows(const float* part, int slices, int64_t ldp, int64_t sli
 md_status lm_attn_prep(int dtype, const LmAttn& a, hipStream_t s);      // convolution, norms, cache rows, convolution state
 md_status lm_attn_plain(int dtype, const LmAttn& a, hipStream_t s);     // one workgroup per query row, any dtype
 bool lm_attn_mfma_takes(const LmAttn& a);
-int lm_attn_mfma_parts(int n_rows, int n_seq, int span, int* split_keys);
+int lm_attn_mfma_parts(const LmRows& r, int ctx_rows, int span, int heads, int vp, int* split_keys);
 size_t lm_attn_mfma_part_floats_most(int n_rows, int n_seq, int span, int heads, int vp);  // floats that the parts of steps up to that size take at most
 md_status lm_attn_mfma(const LmAttn& a, hipStream_t s);                 // bf16 prefill on the matrix cores
 int lm_attn_decode_splits(int n_seq, int max_keys, int* split_keys);
