@@ -507,6 +507,8 @@ md_status lm_step_silu(const LmStepGemm& g, hipStream_t s) {
 
 md_status lm_step_resid(const LmStepGemm& g, hipStream_t s) {
   MD_CHECK_ARG(takes(g) && g.width_pad % 64 == 0 && g.streams >= 1 && g.streams <= MD_LM_MAX_STREAMS);
+  // (norm groups: a wave's part of K is an eighth, and lies in one of them)
+  MD_CHECK_ARG(!g.head_sumsq || (g.heads >= 1 && g.normed > 0 && (g.groups == 1 || ((g.groups == 2 || g.groups == 4 || g.groups == 8) && g.heads % 8 == 0 && g.k % 512 == 0))));
   LmStepGemm a = g;
   a.n = a.width_pad;
   switch (a.streams) {

@@ -289,7 +289,8 @@ struct Step {
     return md_gemm_bf16(&g, s);
   }
 
-  // a mixer's projection -> w.proj.  Few rows: K-slice partials and their sum in two launches, unless one slice fills the chip
+  // a mixer's projection -> w.proj.  Few rows: one product of whole columns; up to 128 and short prompts: K-slice partials and their sum in two launches, unless one
+  // slice fills the chip
   md_status project(const md_linear& lin) {
     if (few) {
       LmStepGemm g = step_gemm(w.h, m->width_pad, lin, sumsq != nullptr);
