@@ -67,9 +67,9 @@ def test_experts_of_a_step(rows, experts, top, ff, alike):
     ts = [U.tokens(1, cfg["vocab"], 0 if alike else i) for i in range(rows)]
     got = m.step([(m.open_sequence(), t, [0]) for t in ts])
     want = torch.cat([O.forward(cfg, w, t) for t in ts[: 1 if alike else rows]]).expand(rows, -1)
-    e = U.logit_errors(got, want).sort().values
-    # (as in test_experts; a row alone is held to what its choice leaves)
-    assert float(e[int(0.9 * (len(e) - 1))]) < 3e-2 and float(e.median()) < 1e-2
+    e = U.logit_errors(got, want)
+    # (every row: no choice is so near with these weights that rounding turns it over)
+    assert float(e.max()) < 3e-2 and float(e.median()) < 1e-2
     if alike:
         assert bool((got == got[:1]).all())
 
@@ -89,11 +89,11 @@ def test_experts_between_products_of_a_step(streams, width):
         slots = [m.open_sequence() for _ in range(n)]
         got = [m.step([(s, t[k : k + 1], [0]) for s, t in zip(slots, ts)]) for k in range(2)]
         for k in range(2):
-            e = U.logit_errors(got[k], want[:n, k]).sort().values
-            assert float(e[int(0.9 * (n - 1))]) < 7e-2 and float(e.median()) < 3e-2, (n, k, e)
+            e = U.logit_errors(got[k], want[:n, k])
+            assert float(e.max()) < 7e-2 and float(e.median()) < 3e-2, (n, k, e)
         if n == 8:  # the last token of each, beside a prompt
             got = m.step([(s, t[2:], [0]) for s, t in zip(slots, ts)] + [(m.open_sequence(), ts[40], [2, 0])])
-            e = U.logit_errors(got, torch.cat([want[:8, 2], want[40, [2, 0]]])).sort().values
-            assert float(e[8]) < 7e-2 and float(e.median()) < 3e-2
+            e = U.logit_errors(got, torch.cat([want[:8, 2], want[40, [2, 0]]]))
+            assert float(e.max()) < 7e-2 and float(e.median()) < 3e-2
         for s in slots:
             m.close_sequence(s)

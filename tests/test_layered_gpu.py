@@ -446,3 +446,45 @@ def test_prompts_beside_single_tokens(running, before, prompt):
         assert float(U.logit_errors(m.step(entries), torch.cat(ref)).max()) < 7e-2
         for s in slots:
             m.close_sequence(s)
+
+
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(4, 4, 32, 32), (20, 5, 32, 64), (3, 1, 96, 128), (40, 40, 32, 32)], ids=str)
+@pytest.mark.parametrize("count,ctx,chunk", [(128, 1100, 4000), (130, 2060, 4000), (128, 2060, 1700), (256, 1600, 4000)], ids=["a_tile", "two_tiles", "chunks", "five_blocks"])
+def test_many_sequences_of_a_long_context(heads, kv, dim, vdim, count, ctx, chunk):
+    """Decode attention whose splits are two, three and four blocks of 32 keys: a tile of 64 keys, two tiles of which the last is half of one, and splits that
+    end within a tile, at a chunk's first key and before the split; every row."""
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    cfg = U.config([U.attention(heads, kv, dim, vdim, chunk)], width=96, vocab=120, ff=None)
+    w = U.weights(cfg, 3, 1.5)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=BF16, max_batch=count, max_context=ctx)
+    text = U.tokens(ctx, 120, 5)
+    lens = [ctx, 1050, 700, 129, 97, 96, 65, 64, 33] + [1 + (7 * i) % 50 for i in range(count - 9)]  # (with the token of the step)
+    ref = O.forward(cfg, w, text)  # (causal: a shorter text's logits are among them)
+    slots = [m.open_sequence() for _ in lens]
+    m.step([(s, text[: n - 1], []) for s, n in zip(slots, lens) if n > 1])
+    got = m.step([(s, text[n - 1 : n], [0]) for s, n in zip(slots, lens)])
+    e = U.logit_errors(got, ref[[n - 1 for n in lens]])
+    assert float(e.max()) < 7e-2, e
+
+
+def test_captured_steps_of_many_sequences():
+    """64 sequences in a graph with a context of 2048: splits of 64 keys; tokens and the last step's logits against the oracle."""
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    cfg = U.config([U.attention(6, 2, 32, 64, 4000)], width=96, vocab=120, ff=None)
+    w = U.weights(cfg, 3, 1.5)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=BF16, max_batch=64, max_context=2048)
+    m.compile()
+    ts = [U.tokens(3 + (11 * i) % 60 if i else 200, 120, i) for i in range(64)]
+    for _ in range(2):  # (the second time the graph is replayed at once)
+        slots = [m.open_sequence() for _ in ts]
+        m.step([(s, t[:-1], []) for s, t in zip(slots, ts)])
+        logits = m._decode_logits(64)
+        hist = m._decode_lockstep(torch.tensor([t[-1] for t in ts], dtype=torch.int32, device="cuda"), slots, 6).t().tolist()
+        want = torch.stack([O.forward(cfg, w, t[:-1] + h[:-1])[-1] for t, h in zip(ts, hist)])
+        assert float(U.logit_errors(logits[:64, :120], want).max()) < 7e-2
+        for s in slots:
+            m.close_sequence(s)
