@@ -516,7 +516,7 @@ __host__ __device__ constexpr TalkLds talk_lds(int hpad, int dp, int nw) {
 //   WHOLE   whole sequences to an XCD, tile by tile
 //   ACROSS  the last tile of every sequence, then the ones before it, so turned that any sequence's go evenly to the 32 engines
 // Longest first in each.  32 heads of 64: 11 ragged prompts, 13250 tokens, 699 us with a run of tiles per XCD, shortest first, 513 in ROUNDS; 3 x 2048 tokens 544 and
-// 330; 8 x 2048 817, 785 and 691 WHOLE (launches of one after the other; 814 WHOLE in a whole pass, 915 with a run per XCD).  Persistent workgroups with a
+// 330; 8 x 2048 817, 785 and 691 WHOLE (launches of one after the other; in a whole pass 915 with a run per XCD, 798 WHOLE).  Persistent workgroups with a
 // queue per XCD: 697, 460 and 1064, the loop around the tile costs registers.
 enum { TALK_ROUNDS, TALK_WHOLE, TALK_ACROSS };
 
