@@ -29,7 +29,7 @@ inline size_t esize(const md_lm_model* m) { return m->dtype == MD_DTYPE_F32 ? 4 
 struct LmWs {
   float* x;
   char *h, *proj, *q, *att, *y, *gu, *act;
-  float *part, *qf, *kf, *of, *chunk_state, *attn_part;
+  float *part, *qf, *kf, *of, *ret_seg, *attn_part;
   char *c_rows, *kv, *q_lat, *conv_out;
   float *latent_part, *dt, *seg, *seg_decay, *route_weight, *sumsq, *row_factor, *head_sumsq;
   int32_t *chosen, *slot_of, *row_of, *offsets;
@@ -65,7 +65,7 @@ inline int conv_columns(const md_lm_layer& l) { return l.heads * l.vdim_pad + 2 
 LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base) {
   const int rows = b->n_rows, n_seq = b->n_seq, max_len = b->max_len, max_ctx = b->max_ctx;
   const size_t es = esize(m), M = rows;
-  size_t in = 0, q = 0, att = 0, gu = 0, act = 0, qf = 0, of = 0, cs = 0, ap = 0, sk = 0, part = 0, y = M * m->width_pad;
+  size_t in = 0, q = 0, att = 0, gu = 0, act = 0, qf = 0, of = 0, rs = 0, ap = 0, sk = 0, part = 0, y = M * m->width_pad;
   size_t c_rows = 0, kv = 0, q_lat = 0, lp = 0, conv = 0, dt = 0, seg = 0, segs = 0, slots = 0, experts = 0;
   size_t sk_room = 0, ssm_heads = 0;
   auto splitk = [&](const md_linear& l, int n) {
@@ -130,7 +130,7 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
     } else {
       qf = std::max(qf, (size_t)l.heads * l.dim_pad);
       of = std::max(of, (size_t)l.heads * l.vdim_pad);
-      cs = std::max(cs, (size_t)l.heads * l.dim_pad * l.vdim_pad);
+      rs = std::max(rs, (size_t)lm_ret_most_segments(n_seq, l.heads, l.dim_pad, l.vdim_pad, max_len) * l.heads * l.dim_pad * l.vdim_pad);
     }
   }
   splitk(m->head, n_logits);
@@ -149,13 +149,12 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
   w.splitk = a.take(sk_room);
   w.splitk_bytes = sk;
   w.attn_part = (float*)a.take(ap * 4);
-  // the plain retention kernels' rotated rows and the matrix-core kernels' chunk states are never live together
-  const size_t plain = M * (2 * qf + of), chunks = (size_t)n_seq * ((max_len + LM_RET_CHUNK - 1) / LM_RET_CHUNK) * cs;
-  float* r = (float*)a.take(std::max(plain, chunks) * 4);
+  // the plain retention kernels' rotated rows and the matrix-core kernels' segment states are never live together
+  float* r = (float*)a.take(std::max(M * (2 * qf + of), rs) * 4);
   w.qf = r;
   w.kf = r + M * qf;
   w.of = r + 2 * M * qf;
-  w.chunk_state = r;
+  w.ret_seg = r;
   w.c_rows = (char*)a.take(c_rows * es);
   w.kv = (char*)a.take(kv * es);
   w.q_lat = (char*)a.take(q_lat * es);
@@ -461,8 +460,8 @@ struct Step {
     a.ldo = few ? 8 : l.out_proj.k_pad;
     a.out_chunk = few ? 8 * b->n_rows : 8;
     a.qf = w.qf; a.kf = w.kf; a.of = w.of;
-    a.chunk_state = w.chunk_state;
-    a.n_chunk_max = (b->max_len + LM_RET_CHUNK - 1) / LM_RET_CHUNK;
+    a.seg = w.ret_seg;
+    a.n_seg = lm_ret_segments(b->n_seq, l.heads, l.dim_pad, l.vdim_pad, b->max_len, &a.seg_chunks);
     if (m->dtype == MD_DTYPE_BF16) {
       if (b->max_len == 1 && (g_lm_kernels & 2) && lm_ret_decode_takes(a)) return lm_ret_decode(a, s);
       if (b->max_len > 1 && (g_lm_kernels & 1) && lm_ret_mfma_takes(a)) return lm_ret_mfma(a, s);

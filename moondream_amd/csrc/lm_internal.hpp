@@ -130,8 +130,8 @@ struct LmRet {
   int out_chunk;
   float *qf, *kf;  // plain kernels: rotated q and k, [n_rows][heads * dp]
   float* of;       // plain kernels: unnormed outputs, [n_rows][heads * vp]
-  float* chunk_state;  // matrix-core prefill: state at the start of every chunk
-  int n_chunk_max;
+  float* seg;      // matrix-core prefill in more segments than one: what each adds to the state, then the state each starts from
+  int n_seg, seg_chunks;  // segments per sequence, their length in chunks
 };
 
 struct LmLatent {
@@ -349,6 +349,8 @@ md_status lm_attn_decode(const LmAttn& a, hipStream_t s);               // bf16 
 
 md_status lm_ret_plain(int dtype, const LmRet& a, hipStream_t s);
 constexpr int LM_RET_CHUNK = 64;
+int lm_ret_segments(int n_seq, int heads, int dp, int vp, int max_len, int* chunks);  // as lm_ssm_segments
+int lm_ret_most_segments(int n_seq, int heads, int dp, int vp, int max_len);
 bool lm_ret_mfma_takes(const LmRet& a);
 md_status lm_ret_mfma(const LmRet& a, hipStream_t s);                   // bf16 prefill, chunked on the matrix cores
 bool lm_ret_decode_takes(const LmRet& a);

@@ -4,15 +4,17 @@
 //
 // Plain kernels (any dtype, fp32 on the vector ALUs): rotation, token-by-token recurrence, output norm and gate.
 //
-// bf16 prefill on the matrix cores, in chunks of 64 tokens:
-//   ret_increment_kernel  per (sequence, head, chunk): what the chunk adds to the state, sum_t decay^(n-1-t) v_t k_t^T
-//   ret_states_kernel     running over the chunks: the state at the start of each, and the slot's state at the end
-//   ret_chunk_kernel      per (sequence, head, chunk): decay^(t+1) S^T q_t + sum_{s<=t} decay^(t-s) (q_t . k_s) v_s, output norm, gate
+// bf16 prefill on the matrix cores, in chunks of 64 tokens, the chunks of a segment one after the other with the state in registers:
+//   ret_run_kernel        per (sequence, head, segment): decay^(t+1) S^T q_t + sum_{s<=t} decay^(t-s) (q_t . k_s) v_s, output norm, gate, and the chunk's
+//                         sum_t decay^(n-1-t) v_t k_t^T onto the state
+//   INC, ret_segments_kernel  where more segments than one fill the chip: what each adds to the state, and the states they start from
 // Everything behind the projections counts as fp32: rotated q and k, decay-weighted products and states enter a product as the sum of
 // two bf16 (16 mantissa bits; hi hi + hi lo + lo hi), the values are the projection's own bf16.
 //
 // bf16 decode step: ret_decode_kernel, one workgroup per (sequence, head): rotation, state update, output, norm and gate in one launch.
 #include "lm_internal.hpp"
+
+#include <algorithm>
 
 namespace {
 
@@ -152,28 +154,6 @@ md_status lm_ret_plain(int dtype, const LmRet& a, hipStream_t s) { return dtype 
 
 namespace {
 
-// eight consecutive elements (d0 a multiple of 8) of a head's rotated row
-__device__ __forceinline__ void rotated8(const bf16_t* h, int d0, int rot_dims, const float* cs, float (&o)[8]) {
-  const u32x4 own = *(const u32x4*)(h + d0);
-  const int half = rot_dims >> 1;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) o[e] = (e & 1) ? hi_bf(own[e >> 1]) : lo_bf(own[e >> 1]);
-  if (d0 >= rot_dims) return;
-  if ((half & 7) == 0) {
-    const bool low = d0 < half;
-    const u32x4 other = *(const u32x4*)(h + (low ? d0 + half : d0 - half));
-    const float* c = cs + 2 * (low ? d0 : d0 - half);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float p = (e & 1) ? hi_bf(other[e >> 1]) : lo_bf(other[e >> 1]);
-      const float sn = c[2 * e + 1];
-      o[e] = o[e] * c[2 * e] + (low ? -p : p) * sn;
-    }
-  } else {
-    for (int e = 0; e < 8; ++e) o[e] = rotated(h, d0 + e, rot_dims, cs);
-  }
-}
-
 __device__ __forceinline__ float pow_int(float log2_decay, int n) { return n == 0 ? 1.0f : __builtin_amdgcn_exp2f(log2_decay * (float)n); }
 
 __device__ __forceinline__ void split8(const float (&v)[8], u32x4& hi, u32x4& lo) {
@@ -190,236 +170,358 @@ __device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x
 
 constexpr int RC = LM_RET_CHUNK;
 
-// grid (chunks, heads, sequences)
-__global__ __launch_bounds__(256) void ret_increment_kernel(const LmRet a) {
-  extern __shared__ __attribute__((aligned(16))) bf16_t rsm[];
-  constexpr int TS = RC + 8;
-  const int c = blockIdx.x, h = blockIdx.y, seq = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, dp = a.dp, vp = a.vp;
-  const int n = min(RC, len - c * RC);
-  if (n <= 0) return;
-  bf16_t *Kh = rsm, *Kl = Kh + dp * TS, *Vt = Kl + dp * TS;  // [d][t], [d][t], [e][t]
-  const float ld = log2f(a.decay[h]);
-  const bf16_t* base = (const bf16_t*)a.proj + (int64_t)(row0 + c * RC) * a.ldp;
-  for (int i = tid; i < RC * (dp >> 3); i += 256) {
-    const int t = i & (RC - 1), d0 = (i / RC) * 8;
-    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (t < n) {
-      const int pos = a.r.seq_pos0[seq] + c * RC + t;
-      rotated8(base + (int64_t)t * a.ldp + a.col_k + h * dp, d0, a.rot_dims, a.rope + (int64_t)pos * a.rot_dims, v);
-      const float w = a.scale * pow_int(ld, n - 1 - t);
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+// Eight tokens of one column per lane from a row-major LDS tile: lane row q gets tokens t0 + 4 q .. + 3 and t0 + 16 + 4 q .. + 3 of column c0 + lane % 16
+__device__ __forceinline__ u32x4 read_columns(const bf16_t* tile, int stride, int t0, int c0, int lane) {
+  const bf16_t* p = tile + (t0 + 4 * (lane >> 4) + ((lane & 15) >> 2)) * stride + c0 + 4 * (lane & 3);
+  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
+  const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(p + 16 * stride));
+  const u32x2 lo = __builtin_bit_cast(u32x2, a), hi = __builtin_bit_cast(u32x2, b);
+  return u32x4{lo[0], lo[1], hi[0], hi[1]};
+}
+// orders this wave's LDS accesses before against those behind, also between lanes (a wave's are carried out in order)
+__device__ __forceinline__ void wave_lds_order() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Two pieces of eight coordinates of a head's row: unit j < rot_dims / 16 the pieces j and j + rot_dims / 16, which turn into each other, with one load
+// of the angles; units behind them two pieces that do not turn.  rot_dims not a multiple of 16: pieces 2 j and 2 j + 1, element by element.
+struct RetUnit {
+  int d[2];
+  bool turns, whole;
+};
+__device__ __forceinline__ RetUnit ret_unit(int j, int rot_dims) {
+  const bool whole = (rot_dims & 15) == 0;
+  const int hp = whole ? rot_dims >> 4 : 0;
+  const bool turns = whole && j < hp;
+  return RetUnit{{8 * (turns ? j : 2 * j), 8 * (turns ? j + hp : 2 * j + 1)}, turns, whole};
+}
+// row: the head's row in memory (only read where pieces turn element by element).  ALL: all of a row turns
+template <bool ALL>
+__device__ __forceinline__ void ret_turn(const RetUnit& u, const u32x4& a, const u32x4& b, const f32x4 (&cs)[4], const bf16_t* row, int rot_dims, const float* angles,
+                                         float (&x)[8], float (&y)[8]) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] *= w;
-    }
-    u32x4 hi, lo;
-    split8(v, hi, lo);
-#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float p = (e & 1) ? hi_bf(a[e >> 1]) : lo_bf(a[e >> 1]), q = (e & 1) ? hi_bf(b[e >> 1]) : lo_bf(b[e >> 1]);
+    const float c = cs[e >> 1][2 * (e & 1)], s = cs[e >> 1][2 * (e & 1) + 1];
+    x[e] = ALL || u.turns ? p * c + -q * s : p;
+    y[e] = ALL || u.turns ? q * c + p * s : q;
+  }
+  if (!ALL && !u.whole)
     for (int e = 0; e < 8; ++e) {
-      Kh[(d0 + e) * TS + t] = (bf16_t)(hi[e >> 1] >> (16 * (e & 1)));
-      Kl[(d0 + e) * TS + t] = (bf16_t)(lo[e >> 1] >> (16 * (e & 1)));
+      x[e] = rotated(row, u.d[0] + e, rot_dims, angles);
+      y[e] = rotated(row, u.d[1] + e, rot_dims, angles);
     }
-  }
-  for (int i = tid; i < RC * (vp >> 3); i += 256) {
-    const int t = i & (RC - 1), e0 = (i / RC) * 8;
-    u32x4 v = {0u, 0u, 0u, 0u};
-    if (t < n) v = *(const u32x4*)(base + (int64_t)t * a.ldp + a.col_v + h * vp + e0);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) Vt[(e0 + e) * TS + t] = (bf16_t)(v[e >> 1] >> (16 * (e & 1)));
-  }
-  __syncthreads();
-  float* dst = a.chunk_state + (((int64_t)seq * a.n_chunk_max + c) * a.heads + h) * vp * dp;
-  const int r = lane & 15, q = lane >> 4, nd = dp >> 4, tiles = (vp >> 4) * nd;
-  for (int tile = wave; tile < tiles; tile += 4) {
-    const int te = tile / nd, td = tile - te * nd;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < RC; s += 32) {
-      const u32x4 v = *(const u32x4*)(Vt + (16 * te + r) * TS + s + 8 * q);
-      acc = mfma(v, *(const u32x4*)(Kh + (16 * td + r) * TS + s + 8 * q), acc);
-      acc = mfma(v, *(const u32x4*)(Kl + (16 * td + r) * TS + s + 8 * q), acc);
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) dst[(int64_t)(16 * te + 4 * q + e) * dp + 16 * td + r] = acc[e];
-  }
 }
 
-// grid (heads * vp * dp / 2048, sequences): a thread owns eight consecutive state elements.  In: the chunks' increments; out, in their
-// place: the state at the start of each chunk as [8 bf16 high parts | 8 bf16 low parts].
-__global__ __launch_bounds__(256) void ret_states_kernel(const LmRet a) {
-  const int seq = blockIdx.y, per_head = a.vp * a.dp;
-  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8, n_el = (int64_t)a.heads * per_head;
-  if (i >= n_el) return;
-  const int h = (int)(i / per_head), len = a.r.seq_row0[seq + 1] - a.r.seq_row0[seq], nc = (len + RC - 1) / RC;
-  const float ld = log2f(a.decay[h]), full = pow_int(ld, RC);
-  float* st = a.state + (int64_t)a.r.seq_slot[seq] * n_el + i;
-  float* p = a.chunk_state + (int64_t)seq * a.n_chunk_max * n_el + i;
-  float S[8];
-  const bool cont = a.r.seq_pos0[seq] > 0;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) S[e] = cont ? st[e] : 0.f;
-  constexpr int U = 4;  // chunks in flight
-  for (int c0 = 0; c0 < nc; c0 += U) {
-    f32x4 inc[U][2];
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (c0 + u < nc) {
-        inc[u][0] = *(const f32x4*)(p + (c0 + u) * n_el);
-        inc[u][1] = *(const f32x4*)(p + (c0 + u) * n_el + 4);
-      }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (c0 + u < nc) {
-        u32x4 hi, lo;
-        split8(S, hi, lo);
-        *(u32x4*)(p + (c0 + u) * n_el) = hi;
-        *(u32x4*)(p + (c0 + u) * n_el + 4) = lo;
-        const int n = min(RC, len - (c0 + u) * RC);
-        const float f = n == RC ? full : pow_int(ld, n);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) S[e] = f * S[e] + inc[u][e >> 2][e & 3];
-      }
-  }
-#pragma unroll
-  for (int e = 0; e < 8; ++e) st[e] = S[e];
-}
-
-// grid (chunks, heads, sequences), four waves of 16 tokens.  D: dp / 32, C: vp / 32; column n of output tile t is coordinate 2 C n + t.
-template <int D, int C>
-__global__ __launch_bounds__(256) void ret_chunk_kernel(const LmRet a) {
-  constexpr int dp = 32 * D, vp = 32 * C, KS = dp + 8, VS = RC + 4;
-  __shared__ __attribute__((aligned(16))) bf16_t Kh[RC * KS], Kl[RC * KS], Vt[vp * VS];
-  const int c = blockIdx.x, h = blockIdx.y, seq = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, q = lane >> 4;
-  const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0;
-  const int n = min(RC, len - c * RC);
-  if (n <= 0) return;
-  const int p0 = a.r.seq_pos0[seq] + c * RC;
+// Prefill.  grid (heads, segments, sequences), four waves; a workgroup walks the chunks of a segment with the head's state in registers, a wave owns 16
+// tokens of the outputs and C * D 16 x 16 tiles of the state.  The next chunk's rows are under way while one is worked on.  All memory is read and
+// written by pieces of 16 bytes that follow one another, four lanes to 64 bytes at least, and reordered in LDS: a load whose lanes each take another row costs
+// four times that (what bounded the form before this, a workgroup per chunk with the state at its start from memory).  A wave's gates lie over its own queries, which it
+// has in registers by then, and its outputs over its gates.
+// 8 x 2048 tokens, 32 heads of 64: 113 us, 43 and 8 for the increments and states of two segments each, against 196 + 100 + 49 (increments of all chunks, their
+// states and outputs); bytes 65 us.  What is left is about 800 vector instructions per wave and chunk, and LDS.
+// INC: only what the segment adds to the state.  D: dp / 32, C: vp / 32
+template <int D, int C, bool INC>
+__global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ret_run_kernel(const LmRet a) {
+  constexpr int dp = 32 * D, vp = 32 * C, QS = (2 * dp > vp ? 2 * dp : vp) + 8, KS = dp + 8, VS = vp + 8, NT = C * D, PT = 2 * C;
+  constexpr int PER = C == 3 ? 3 : C == 4 ? 2 : 1;  // a wave's state tiles i and i + PER have the same 16 columns of v
+  constexpr int UNITS = dp / 16, NU = (RC * UNITS + 255) / 256;
+  extern __shared__ __attribute__((aligned(16))) bf16_t rsm[];
+  bf16_t *Kh = rsm, *Kl = Kh + RC * KS, *V = Kl + RC * KS, *Q = V + RC * VS, *Sh = Q + RC * QS, *Sl = Sh + vp * KS;  // Q: [token][high | low]
+  __shared__ float ws[RC], later[2 * RC];  // decay^(n-1-t) of the tokens; [63 - age]: decay^age, 0 of an age below 0
+  const int h = blockIdx.x, sg = blockIdx.y, seq = blockIdx.z, tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, first = sg * a.seg_chunks * RC, last = min(first + a.seg_chunks * RC, len);
+  if (first >= last) return;
+  const bool final = last == len;
+  if (INC && final) return;  // nobody starts behind the last segment
+  const int pos0 = a.r.seq_pos0[seq];
   const float ld = log2f(a.decay[h]);
-  const bf16_t* base = (const bf16_t*)a.proj + (int64_t)(row0 + c * RC) * a.ldp;
-  for (int i = tid; i < RC * (dp >> 3); i += 256) {
-    const int t = i / (dp >> 3), d0 = (i - t * (dp >> 3)) * 8;
-    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (t < n) {
-      rotated8(base + (int64_t)t * a.ldp + a.col_k + h * dp, d0, a.rot_dims, a.rope + (int64_t)(p0 + t) * a.rot_dims, v);
+  const bf16_t* proj = (const bf16_t*)a.proj + (int64_t)row0 * a.ldp;
+  const int cq = a.col_q + h * dp, ck = a.col_k + h * dp, cv = a.col_v + h * vp, cg = a.col_g + h * vp;
+  const bool all_turns = a.rot_dims == dp;
+
+  f32x4 S[NT];
+  float* slot = a.state + ((int64_t)a.r.seq_slot[seq] * a.heads + h) * vp * dp;
+  float* seg = a.seg + (((int64_t)seq * a.n_seg + sg) * a.heads + h) * vp * dp;
+  const float* from = INC ? nullptr : a.n_seg > 1 ? seg : pos0 > 0 ? slot : nullptr;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] *= a.scale;
-    }
-    u32x4 hi, lo;
-    split8(v, hi, lo);
-    *(u32x4*)(Kh + t * KS + d0) = hi;
-    *(u32x4*)(Kl + t * KS + d0) = lo;
+  for (int i = 0; i < NT; ++i) {
+    const int tile = wave + 4 * i, pt = tile % PT, nt = tile / PT;
+    S[i] = from ? *(const f32x4*)(from + (16 * pt + r) * dp + 16 * nt + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  for (int i = tid; i < RC * (vp >> 3); i += 256) {
-    const int t = i & (RC - 1), e0 = (i / RC) * 8;
-    u32x4 v = {0u, 0u, 0u, 0u};
-    if (t < n) v = *(const u32x4*)(base + (int64_t)t * a.ldp + a.col_v + h * vp + e0);
+
+  u32x4 qr[NU][2], kr[NU][2], vr[C], gr[C];
+  f32x4 cs[NU][4];
+  constexpr u32x4 none = {0u, 0u, 0u, 0u};
+  if (!INC && tid < 2 * RC) later[tid] = tid <= RC - 1 ? pow_int(ld, RC - 1 - tid) : 0.f;  // [63 - age]
+  auto load = [&](int t0) {  // rows past the end: the last one again
+    const int n = min(RC, last - t0);
+    const bf16_t* rows = proj + (int64_t)t0 * a.ldp;
+    const float* angles = a.rope + (int64_t)(pos0 + t0) * a.rot_dims;
+    auto piece = [&](int t, int c) { return *(const u32x4*)(rows + ((uint32_t)min(t, n - 1) * (uint32_t)a.ldp + (uint32_t)c)); };
 #pragma unroll
-    for (int e = 0; e < 8; ++e) Vt[(e0 + e) * VS + t] = (bf16_t)(v[e >> 1] >> (16 * (e & 1)));
-  }
-  const int t = 16 * wave + r, tq = min(t, n - 1);  // this lane's query (rows past the chunk's end replay its last one)
-  u32x4 qh[D], ql[D];
+    for (int i = 0; i < NU; ++i) {
+      const int u = tid + 256 * i, t = u / UNITS;
+      const RetUnit at = ret_unit(u % UNITS, a.rot_dims);
 #pragma unroll
-  for (int s = 0; s < D; ++s) {
-    float v[8];
-    rotated8(base + (int64_t)tq * a.ldp + a.col_q + h * dp, 32 * s + 8 * q, a.rot_dims, a.rope + (int64_t)(p0 + tq) * a.rot_dims, v);
-    split8(v, qh[s], ql[s]);
-  }
-  __syncthreads();
-  if (16 * wave >= n) return;
-  f32x4 o[2 * C];
-#pragma unroll
-  for (int i = 0; i < 2 * C; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  if (p0 > 0) {
-    const float* S = a.chunk_state + (((int64_t)seq * a.n_chunk_max + c) * a.heads + h) * vp * dp;
-#pragma unroll
-    for (int s = 0; s < D; ++s)
-#pragma unroll
-      for (int i = 0; i < 2 * C; ++i) {
-        const float* sp = S + (2 * C * r + i) * dp + 32 * s + 8 * q;
-        const u32x4 sh = *(const u32x4*)sp, sl = *(const u32x4*)(sp + 4);
-        o[i] = mfma(qh[s], sh, o[i]);
-        o[i] = mfma(qh[s], sl, o[i]);
-        o[i] = mfma(ql[s], sh, o[i]);
+      for (int k = 0; k < 2; ++k) {
+        if (!INC) qr[i][k] = piece(t, cq + at.d[k]);
+        kr[i][k] = piece(t, ck + at.d[k]);
       }
-    f32x4 w;
+      if (a.rot_dims > 0) {
+        const uint32_t from = (uint32_t)min(t, n - 1) * (uint32_t)a.rot_dims + (at.turns ? 2 * at.d[0] : 0);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) w[e] = pow_int(ld, 16 * wave + 4 * q + e + 1);
-#pragma unroll
-    for (int i = 0; i < 2 * C; ++i) o[i] *= w;
-  }
-#pragma unroll
-  for (int b = 0; b < RC / 32; ++b) {
-    if (2 * b > wave) continue;
-    float p[8];  // token slots (block 2 b, 4 q + j) and (block 2 b + 1, 4 q + j) of the products' contraction
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const int sb = 2 * b + half;
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-      if (sb <= wave) {
-#pragma unroll
-        for (int s = 0; s < D; ++s) {
-          const u32x4 kh = *(const u32x4*)(Kh + (16 * sb + r) * KS + 32 * s + 8 * q), kl = *(const u32x4*)(Kl + (16 * sb + r) * KS + 32 * s + 8 * q);
-          acc = mfma(kh, qh[s], acc);
-          acc = mfma(kh, ql[s], acc);
-          acc = mfma(kl, qh[s], acc);
-        }
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int d = t - (16 * sb + 4 * q + e);
-        p[4 * half + e] = (sb <= wave && d >= 0) ? acc[e] * pow_int(ld, d) : 0.f;
+        for (int k = 0; k < 4; ++k) cs[i][k] = at.whole ? *(const f32x4*)(angles + (from + 4 * k)) : f32x4{0.f, 0.f, 0.f, 0.f};
       }
     }
-    u32x4 ph, pl;
-    split8(p, ph, pl);
-#pragma unroll
-    for (int i = 0; i < 2 * C; ++i) {
-      const bf16_t* vr = Vt + (2 * C * r + i) * VS + 32 * b + 4 * q;
-      const u32x2 v0 = *(const u32x2*)vr, v1 = *(const u32x2*)(vr + 16);
-      const u32x4 v = {v0[0], v0[1], v1[0], v1[1]};
-      o[i] = mfma(ph, v, o[i]);
-      o[i] = mfma(pl, v, o[i]);
-    }
-  }
-  f32x4 ss = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < 2 * C; ++i) ss += o[i] * o[i];
-#pragma unroll
-  for (int m = 1; m < 16; m <<= 1)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) ss[e] += __shfl_xor(ss[e], m, 64);
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int tt = 16 * wave + 4 * q + e;
-    if (tt >= n) continue;
-    const float rn = 1.0f / sqrtf(ss[e] / (float)a.vdim + a.eps);
-    const bf16_t* g = base + (int64_t)tt * a.ldp + a.col_g + h * vp + 2 * C * r;
-    bf16_t* dst = (bf16_t*)a.out + (int64_t)(row0 + c * RC + tt) * a.ldo;
 #pragma unroll
     for (int i = 0; i < C; ++i) {
-      const uint32_t gg = *(const uint32_t*)(g + 2 * i);
-      *(uint32_t*)(dst + in_chunks(h * vp + 2 * C * r + 2 * i, a.out_chunk)) = pack_bf16x2(o[2 * i][e] * rn * silu_f32(lo_bf(gg)), o[2 * i + 1][e] * rn * silu_f32(hi_bf(gg)));
+      const int p = tid + 256 * i;
+      vr[i] = piece(p / (vp / 8), cv + p % (vp / 8) * 8);
     }
+    if (!INC)
+#pragma unroll
+      for (int i = 0; i < C; ++i) {  // the wave's own tokens
+        const int p = lane + 64 * i;
+        gr[i] = piece(16 * wave + p / (vp / 8), cg + p % (vp / 8) * 8);
+      }
+  };
+  load(first);
+  const int t = 16 * wave + r;  // this lane's query
+  const float et = pow_int(ld, t + 1);
+
+  for (int t0 = first; t0 < last; t0 += RC) {
+    const int n = min(RC, last - t0);
+    const bool stated = from || t0 > first;
+    __syncthreads();  // the previous chunk's tiles have been read
+    auto stage = [&](auto all) {
+      constexpr bool ALL = decltype(all)::value;
+#pragma unroll
+      for (int i = 0; i < NU; ++i) {
+        const int u = tid + 256 * i, tu = u / UNITS;
+        if (RC * UNITS % 256 != 0 && u >= RC * UNITS) break;
+        const RetUnit at = ret_unit(u % UNITS, a.rot_dims);
+        const int tl = min(tu, n - 1);
+        const bf16_t* row = proj + (int64_t)(t0 + tl) * a.ldp;
+        const float* angles = a.rope + (int64_t)(pos0 + t0 + tl) * a.rot_dims;
+        float x[2][8];
+        u32x4 hi, lo;
+        if (!INC) {
+          ret_turn<ALL>(at, qr[i][0], qr[i][1], cs[i], row + cq, a.rot_dims, angles, x[0], x[1]);
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            split8(x[k], hi, lo);
+            *(u32x4*)(Q + tu * QS + at.d[k]) = hi;
+            *(u32x4*)(Q + tu * QS + dp + at.d[k]) = lo;
+          }
+        }
+        ret_turn<ALL>(at, kr[i][0], kr[i][1], cs[i], row + ck, a.rot_dims, angles, x[0], x[1]);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) x[k][e] *= a.scale;
+          split8(x[k], hi, lo);
+          if (n < RC && tu >= n) hi = lo = none;
+          *(u32x4*)(Kh + tu * KS + at.d[k]) = hi;
+          *(u32x4*)(Kl + tu * KS + at.d[k]) = lo;
+        }
+      }
+    };
+    if (all_turns) stage(std::true_type{});
+    else stage(std::false_type{});
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      const int p = tid + 256 * i, tv = p / (vp / 8);
+      *(u32x4*)(V + tv * VS + p % (vp / 8) * 8) = n < RC && tv >= n ? none : vr[i];
+    }
+    if (!INC && stated)
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        const int tile = wave + 4 * i, pt = tile % PT, nt = tile / PT, at = (16 * pt + r) * KS + 16 * nt + 4 * q;
+        const u32x2 hi = {pack_bf16x2(S[i][0], S[i][1]), pack_bf16x2(S[i][2], S[i][3])};
+        *(u32x2*)(Sh + at) = hi;
+        *(u32x2*)(Sl + at) = u32x2{pack_bf16x2(S[i][0] - lo_bf(hi[0]), S[i][1] - hi_bf(hi[0])), pack_bf16x2(S[i][2] - lo_bf(hi[1]), S[i][3] - hi_bf(hi[1]))};
+      }
+    if (tid < RC) ws[tid] = tid < n ? pow_int(ld, n - 1 - tid) : 0.f;
+    u32x4 gc[C];
+    if (!INC)
+#pragma unroll
+      for (int i = 0; i < C; ++i) gc[i] = gr[i];
+    __syncthreads();
+    if (t0 + RC < last) load(t0 + RC);
+
+    if (!INC && 16 * wave < n) {
+      bf16_t* G = Q + 16 * wave * QS;  // the wave's own rows
+      u32x4 qh[D], ql[D];
+#pragma unroll
+      for (int s = 0; s < D; ++s) {
+        qh[s] = *(const u32x4*)(G + r * QS + 32 * s + 8 * q);
+        ql[s] = *(const u32x4*)(G + r * QS + dp + 32 * s + 8 * q);
+      }
+      wave_lds_order();
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        const int p = lane + 64 * i;
+        *(u32x4*)(G + p / (vp / 8) * QS + p % (vp / 8) * 8) = gc[i];
+      }
+      wave_lds_order();
+      f32x4 o[PT];
+#pragma unroll
+      for (int i = 0; i < PT; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (stated) {
+#pragma unroll
+        for (int s = 0; s < D; ++s)
+#pragma unroll
+          for (int i = 0; i < PT; ++i) {
+            const u32x4 sh = *(const u32x4*)(Sh + (16 * i + r) * KS + 32 * s + 8 * q), sl = *(const u32x4*)(Sl + (16 * i + r) * KS + 32 * s + 8 * q);
+            o[i] = mfma(sh, qh[s], o[i]);
+            o[i] = mfma(sl, qh[s], o[i]);
+            o[i] = mfma(sh, ql[s], o[i]);
+          }
+#pragma unroll
+        for (int i = 0; i < PT; ++i) o[i] *= et;
+      }
+#pragma unroll
+      for (int b = 0; b < RC / 32; ++b) {
+        if (2 * b > wave) continue;
+        float p[8];  // tokens 32 b + 4 q + j and 32 b + 16 + 4 q + j: the order of read_columns
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          const int sb = 2 * b + half;
+          f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+          if (sb <= wave) {
+#pragma unroll
+            for (int s = 0; s < D; ++s) {
+              const u32x4 kh = *(const u32x4*)(Kh + (16 * sb + r) * KS + 32 * s + 8 * q), kl = *(const u32x4*)(Kl + (16 * sb + r) * KS + 32 * s + 8 * q);
+              acc = mfma(kh, qh[s], acc);
+              acc = mfma(kh, ql[s], acc);
+              acc = mfma(kl, qh[s], acc);
+            }
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) p[4 * half + e] = later[RC - 1 - t + 16 * sb + 4 * q + e];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) p[4 * half + e] = p[4 * half + e] != 0.f ? acc[e] * p[4 * half + e] : 0.f;
+        }
+        u32x4 ph, pl;
+        split8(p, ph, pl);
+#pragma unroll
+        for (int i = 0; i < PT; ++i) {
+          const u32x4 v = read_columns(V, VS, 32 * b, 16 * i, lane);
+          o[i] = mfma(v, ph, o[i]);
+          o[i] = mfma(v, pl, o[i]);
+        }
+      }
+      f32x4 sq = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < PT; ++i) sq += o[i] * o[i];
+      float ss = (sq[0] + sq[1]) + (sq[2] + sq[3]);
+      ss += __shfl_xor(ss, 16, 64);
+      ss += __shfl_xor(ss, 32, 64);
+      const float rn = 1.0f / sqrtf(ss / (float)a.vdim + a.eps);
+#pragma unroll
+      for (int i = 0; i < PT; ++i) {
+        bf16_t* at = G + r * QS + 16 * i + 4 * q;
+        f32x4 y = ld4(at);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = o[i][e] * rn * silu_fast(y[e]);
+        st4(at, y);
+      }
+      wave_lds_order();
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        const int p = lane + 64 * i, tg = p / (vp / 8), d = p % (vp / 8) * 8;
+        if (16 * wave + tg < n)
+          *(u32x4*)((bf16_t*)a.out + (int64_t)(row0 + t0 + 16 * wave + tg) * a.ldo + in_chunks(h * vp + d, a.out_chunk)) = *(const u32x4*)(G + tg * QS + d);
+      }
+    }
+
+    const float keep = pow_int(ld, n);
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int pt = (wave + 4 * j) % PT;
+      u32x4 vh[RC / 32], vl[RC / 32];
+#pragma unroll
+      for (int k = 0; k < RC / 32; ++k) {
+        const u32x4 x = read_columns(V, VS, 32 * k, 16 * pt, lane);
+        const f32x4 w0 = *(const f32x4*)(ws + 32 * k + 4 * q), w1 = *(const f32x4*)(ws + 32 * k + 16 + 4 * q);
+        const float v[8] = {lo_bf(x[0]) * w0[0], hi_bf(x[0]) * w0[1], lo_bf(x[1]) * w0[2], hi_bf(x[1]) * w0[3],
+                            lo_bf(x[2]) * w1[0], hi_bf(x[2]) * w1[1], lo_bf(x[3]) * w1[2], hi_bf(x[3]) * w1[3]};
+        split8(v, vh[k], vl[k]);
+      }
+#pragma unroll
+      for (int i = j; i < NT; i += PER) {
+        const int nt = (wave + 4 * i) / PT;
+        S[i] *= keep;
+#pragma unroll
+        for (int k = 0; k < RC / 32; ++k) {
+          const u32x4 kh = read_columns(Kh, KS, 32 * k, 16 * nt, lane), kl = read_columns(Kl, KS, 32 * k, 16 * nt, lane);
+          S[i] = mfma(kh, vh[k], S[i]);
+          S[i] = mfma(kh, vl[k], S[i]);
+          S[i] = mfma(kl, vh[k], S[i]);
+        }
+      }
+    }
+  }
+  float* to = INC ? seg : final ? slot : nullptr;
+  if (to)
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const int tile = wave + 4 * i, pt = tile % PT, nt = tile / PT;
+      *(f32x4*)(to + (16 * pt + r) * dp + 16 * nt + 4 * q) = S[i];
+    }
+}
+
+// grid (heads * vp * dp / 1024, sequences): what the segments add -> the states they start from
+__global__ __launch_bounds__(256) void ret_segments_kernel(const LmRet a) {
+  const int seq = blockIdx.y, per_head = a.vp * a.dp;
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4, n_el = (int64_t)a.heads * per_head;
+  if (i >= n_el) return;
+  const int h = (int)(i / per_head), len = a.r.seq_row0[seq + 1] - a.r.seq_row0[seq], n = (len + a.seg_chunks * RC - 1) / (a.seg_chunks * RC);
+  const float keep = pow_int(log2f(a.decay[h]), a.seg_chunks * RC);
+  f32x4 S = {0.f, 0.f, 0.f, 0.f};
+  if (a.r.seq_pos0[seq] > 0) S = *(const f32x4*)(a.state + (int64_t)a.r.seq_slot[seq] * n_el + i);
+  for (int sg = 0; sg < n; ++sg) {
+    float* p = a.seg + ((int64_t)seq * a.n_seg + sg) * n_el + i;
+    f32x4 inc = {0.f, 0.f, 0.f, 0.f};
+    if (sg + 1 < n) inc = *(const f32x4*)p;
+    *(f32x4*)p = S;
+    S = keep * S + inc;
   }
 }
 
 typedef void (*RetKernel)(const LmRet);
+struct RetPick {
+  RetKernel run, inc;
+  int lds;
+};
+template <int D, int C>
+RetPick ret_run_of() {
+  constexpr int dp = 32 * D, vp = 32 * C, QS = (2 * dp > vp ? 2 * dp : vp) + 8;
+  return RetPick{ret_run_kernel<D, C, false>, ret_run_kernel<D, C, true>, (RC * (2 * (dp + 8) + vp + 8 + QS) + 2 * vp * (dp + 8)) * 2};
+}
 template <int D>
-RetKernel ret_chunk_by_width(int c) {
+RetPick ret_run_by_width(int c) {
   switch (c) {
-    case 1: return ret_chunk_kernel<D, 1>;
-    case 2: return ret_chunk_kernel<D, 2>;
-    case 3: return ret_chunk_kernel<D, 3>;
-    case 4: return ret_chunk_kernel<D, 4>;
-    default: return nullptr;
+    case 1: return ret_run_of<D, 1>();
+    case 2: return ret_run_of<D, 2>();
+    case 3: return ret_run_of<D, 3>();
+    case 4: return ret_run_of<D, 4>();
+    default: return RetPick{nullptr, nullptr, 0};
   }
 }
-RetKernel ret_chunk_pick(const LmRet& a) {
+RetPick ret_run_pick(const LmRet& a) {
+  const RetPick none = {nullptr, nullptr, 0};
+  if ((a.col_q | a.col_k | a.col_v | a.col_g | a.ldp | a.ldo | a.out_chunk) % 8 != 0) return none;  // pieces of eight
   switch (a.dp / 32) {
-    case 1: return ret_chunk_by_width<1>(a.vp / 32);
-    case 2: return ret_chunk_by_width<2>(a.vp / 32);
-    case 3: return ret_chunk_by_width<3>(a.vp / 32);
-    case 4: return ret_chunk_by_width<4>(a.vp / 32);
-    default: return nullptr;
+    case 1: return ret_run_by_width<1>(a.vp / 32);
+    case 2: return ret_run_by_width<2>(a.vp / 32);
+    case 3: return ret_run_by_width<3>(a.vp / 32);
+    case 4: return ret_run_by_width<4>(a.vp / 32);
+    default: return none;
   }
 }
 
@@ -499,17 +601,33 @@ RetKernel ret_decode_pick(const LmRet& a) {
 
 }  // namespace
 
-bool lm_ret_mfma_takes(const LmRet& a) { return ret_chunk_pick(a) != nullptr; }
+// Segments: as many as keep to the workgroups that a CU holds, two, or one of the largest heads (ret_run_kernel's registers).  The increments cost half of the
+// outputs, and they and the states two launches, about two chunks.  Eight layers of little else: 32 heads of 64, 700 tokens, up to 512 workgroups 620 us, 256 702; 8 x 2048
+// tokens 4255 and 4448; 16 heads of 128: 800 and 748, 5369 and 5214.
+inline int ret_room(int dp, int vp) { return dp * vp > 9 * 1024 ? 256 : 512; }
+int lm_ret_segments(int n_seq, int heads, int dp, int vp, int max_len, int* chunks) {
+  const int n = (max_len + RC - 1) / RC, segs = ret_room(dp, vp) / (n_seq * heads), per = segs > 1 ? (n + segs - 1) / segs : n;
+  *chunks = 3 * per + 4 < 2 * n ? per : n;
+  return (n + *chunks - 1) / *chunks;
+}
+int lm_ret_most_segments(int n_seq, int heads, int dp, int vp, int max_len) {
+  const int64_t n = (max_len + RC - 1) / RC;
+  return n > 1 ? (int)std::min(n_seq * n, (int64_t)(ret_room(dp, vp) / heads)) : 0;
+}
+bool lm_ret_mfma_takes(const LmRet& a) { return ret_run_pick(a).run != nullptr; }
 md_status lm_ret_mfma(const LmRet& a, hipStream_t s) {
-  const RetKernel fn = ret_chunk_pick(a);
-  if (!fn) return MD_ERR_UNSUPPORTED;
-  const dim3 grid(a.n_chunk_max, a.heads, a.r.n_seq);
-  const int lds = (2 * a.dp + a.vp) * (RC + 8) * 2;
-  hipLaunchKernelGGL(ret_increment_kernel, grid, dim3(256), lds, s, a);
-  MD_TRY(md_launch_status());
-  hipLaunchKernelGGL(ret_states_kernel, dim3((a.heads * a.vp * a.dp + 2047) / 2048, a.r.n_seq), dim3(256), 0, s, a);
-  MD_TRY(md_launch_status());
-  hipLaunchKernelGGL(fn, grid, dim3(256), 0, s, a);
+  const RetPick k = ret_run_pick(a);
+  if (!k.run) return MD_ERR_UNSUPPORTED;
+  const dim3 grid(a.heads, a.n_seg, a.r.n_seq);
+  MD_TRY(md_ensure_dynamic_lds((const void*)k.run, k.lds));
+  if (a.n_seg > 1) {
+    MD_TRY(md_ensure_dynamic_lds((const void*)k.inc, k.lds));
+    hipLaunchKernelGGL(k.inc, grid, dim3(256), k.lds, s, a);
+    MD_TRY(md_launch_status());
+    hipLaunchKernelGGL(ret_segments_kernel, dim3((a.heads * a.vp * a.dp + 1023) / 1024, a.r.n_seq), dim3(256), 0, s, a);
+    MD_TRY(md_launch_status());
+  }
+  hipLaunchKernelGGL(k.run, grid, dim3(256), k.lds, s, a);
   return md_launch_status();
 }
 
