@@ -38,6 +38,22 @@ __device__ __forceinline__ void st8(float* p, f32x4 a, f32x4 b) {
 // that the products of few rows read (gemm_step.hip)
 __device__ __forceinline__ int in_chunks(int c, int chunk) { return (c >> 3) * chunk + (c & 7); }
 
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+// Eight tokens of one column per lane from a row-major LDS tile: lane row q (lane / 16) gets tokens t0 + 4 q .. + 3 and t0 + 16 + 4 q .. + 3 of
+// column c0 + lane % 16 (in a 16-lane group, lane i points at four columns of token i / 4 and receives four tokens of column i % 16).
+__device__ __forceinline__ u32x4 read_columns(const bf16_t* tile, int stride, int t0, int c0, int lane) {
+  const bf16_t* p = tile + (t0 + 4 * (lane >> 4) + ((lane & 15) >> 2)) * stride + c0 + 4 * (lane & 3);
+  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
+  const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(p + 16 * stride));
+  const u32x2 lo = __builtin_bit_cast(u32x2, a), hi = __builtin_bit_cast(u32x2, b);
+  return u32x4{lo[0], lo[1], hi[0], hi[1]};
+}
+// orders a wave's LDS accesses before against those behind, also between its lanes (they are carried out in order)
+__device__ __forceinline__ void wave_lds_order() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+}
+
 __device__ __forceinline__ float silu_f32(float z) { return z / (1.0f + expf(-z)); }
 template <typename T>
 __device__ __forceinline__ float silu_for(float z) {

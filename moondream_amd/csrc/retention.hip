@@ -170,21 +170,6 @@ __device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x
 
 constexpr int RC = LM_RET_CHUNK;
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-// Eight tokens of one column per lane from a row-major LDS tile: lane row q gets tokens t0 + 4 q .. + 3 and t0 + 16 + 4 q .. + 3 of column c0 + lane % 16
-__device__ __forceinline__ u32x4 read_columns(const bf16_t* tile, int stride, int t0, int c0, int lane) {
-  const bf16_t* p = tile + (t0 + 4 * (lane >> 4) + ((lane & 15) >> 2)) * stride + c0 + 4 * (lane & 3);
-  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
-  const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(p + 16 * stride));
-  const u32x2 lo = __builtin_bit_cast(u32x2, a), hi = __builtin_bit_cast(u32x2, b);
-  return u32x4{lo[0], lo[1], hi[0], hi[1]};
-}
-// orders this wave's LDS accesses before against those behind, also between lanes (a wave's are carried out in order)
-__device__ __forceinline__ void wave_lds_order() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_wave_barrier();
-}
-
 // Two pieces of eight coordinates of a head's row: unit j < rot_dims / 16 the pieces j and j + rot_dims / 16, which turn into each other, with one load
 // of the angles; units behind them two pieces that do not turn.  rot_dims not a multiple of 16: pieces 2 j and 2 j + 1, element by element.
 struct RetUnit {

@@ -18,6 +18,9 @@
 // state enter a product as the sum of two bf16 (16 mantissa bits).  Operands that need consecutive tokens per lane come from row-major LDS
 // tiles through the transposing LDS read.  When sequences x heads do not fill the chip, a sequence is cut into segments: a first launch of
 // the same kernel makes what every segment adds to the state (INC), ssm_segments_kernel the states they start from.
+// What bounds a chunk is the chain through it (load, LDS, products, LDS; 4.2 us of 64 x 64 x 128).  C, the gates and the outputs go through LDS too, so that
+// memory is read and written by whole pieces in a row, not by a piece of another row per lane: 5 ragged sequences, 4900 tokens, 64 heads of 64 x 128, 106 -> 102 us, 700
+// tokens of 16 x 128 x 128 in segments 17.7 -> 16.0 and 8.8 -> 8.1.
 #include "lm_internal.hpp"
 
 namespace {
@@ -300,16 +303,6 @@ md_status plain(const LmSsm& a, hipStream_t s) {
 // ---------------------------------------------------------------------------------------------------------------------------
 constexpr float LOG2E = 1.4426950408889634f;
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-// Eight tokens of one column per lane from a row-major LDS tile: lane row q (lane / 16) gets tokens t0 + 4 q .. + 3 and t0 + 16 + 4 q .. + 3 of
-// column c0 + lane % 16 (in a 16-lane group, lane i points at four columns of token i / 4 and receives four tokens of column i % 16).
-__device__ __forceinline__ u32x4 read_columns(const bf16_t* tile, int stride, int t0, int c0, int lane) {
-  const bf16_t* p = tile + (t0 + 4 * (lane >> 4) + ((lane & 15) >> 2)) * stride + c0 + 4 * (lane & 3);
-  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
-  const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(p + 16 * stride));
-  const u32x2 lo = __builtin_bit_cast(u32x2, a), hi = __builtin_bit_cast(u32x2, b);
-  return u32x4{lo[0], lo[1], hi[0], hi[1]};
-}
 __device__ __forceinline__ md_bf16x8v op(const u32x4& v) { return __builtin_bit_cast(md_bf16x8v, v); }
 __device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x4& c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(op(a), op(b), c, 0, 0, 0); }
 __device__ __forceinline__ void split8(const float (&v)[8], u32x4& hi, u32x4& lo) {
@@ -326,10 +319,10 @@ constexpr int L = LM_SSM_CHUNK;
 // D: dp / 32, C: vp / 32
 template <int D, int C, bool INC>
 __global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ssm_chunk_kernel(const LmSsm a) {
-  constexpr int dp = 32 * D, vp = 32 * C, XS = vp + 8, BS = dp + 8, NT = C * D, PT = 2 * C;
+  constexpr int dp = 32 * D, vp = 32 * C, XS = vp + 8, BS = dp + 8, QS = (dp > vp ? dp : vp) + 8, NT = C * D, PT = 2 * C;
   constexpr int PER = C == 3 ? 3 : C == 4 ? 2 : 1;  // a wave's state tiles i and i + PER have the same 16 columns of x
   extern __shared__ __attribute__((aligned(16))) bf16_t sm[];
-  bf16_t *X = sm, *B = X + L * XS, *Sh = B + L * BS, *Sl = Sh + vp * BS;
+  bf16_t *X = sm, *B = X + L * XS, *Sh = B + L * BS, *Sl = Sh + vp * BS, *Q = Sl + vp * BS;  // Q: C of the chunk, then a wave's gates and outputs over its own rows
   __shared__ float cum[L], dts[L], ws[L];
   const int h = blockIdx.x, sg = blockIdx.y, seq = blockIdx.z, tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -352,7 +345,7 @@ __global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ssm_chunk_kernel(const
     S[i] = from ? *(const f32x4*)(from + (16 * pt + r) * dp + 16 * nt + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  u32x4 xr[C], br[D], qn[D], qc[D];
+  u32x4 xr[C], br[D], qr[D], zr[C];
   float dt_r = 0.f;
   auto load = [&](int t0) {
     const int n = min(L, last - t0);
@@ -367,9 +360,16 @@ __global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ssm_chunk_kernel(const
       br[i] = t < n ? *(const u32x4*)(u + (int64_t)(t0 + t) * cw + cb + d) : u32x4{0u, 0u, 0u, 0u};
     }
     if (!INC) {
-      const int t = min(16 * wave + r, n - 1);  // rows past the end replay the last one, and are not stored
 #pragma unroll
-      for (int s = 0; s < D; ++s) qn[s] = *(const u32x4*)(u + (int64_t)(t0 + t) * cw + cc + 32 * s + 8 * q);
+      for (int i = 0; i < D; ++i) {
+        const int piece = tid + 256 * i, t = piece / (dp / 8), d = (piece - t * (dp / 8)) * 8;
+        qr[i] = t < n ? *(const u32x4*)(u + (int64_t)(t0 + t) * cw + cc + d) : u32x4{0u, 0u, 0u, 0u};
+      }
+#pragma unroll
+      for (int i = 0; i < C; ++i) {  // gates: the wave's own tokens
+        const int piece = lane + 64 * i, t = 16 * wave + piece / (vp / 8), d = piece % (vp / 8) * 8;
+        zr[i] = t < n ? *(const u32x4*)((const bf16_t*)a.proj + (int64_t)(row0 + t0 + t) * a.ldp + a.col_z + h * vp + d) : u32x4{0u, 0u, 0u, 0u};
+      }
     }
     if (tid < L) dt_r = tid < n ? a.dt[(int64_t)(row0 + t0 + tid) * H + h] : 0.f;
   };
@@ -398,8 +398,15 @@ __global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ssm_chunk_kernel(const
         *(u32x2*)(Sl + at) = u32x2{pack_bf16x2(S[i][0] - lo_bf(hi[0]), S[i][1] - hi_bf(hi[0])), pack_bf16x2(S[i][2] - lo_bf(hi[1]), S[i][3] - hi_bf(hi[1]))};
       }
 #pragma unroll
-      for (int s = 0; s < D; ++s) qc[s] = qn[s];
+      for (int i = 0; i < D; ++i) {
+        const int piece = tid + 256 * i, t = piece / (dp / 8), d = (piece - t * (dp / 8)) * 8;
+        *(u32x4*)(Q + t * QS + d) = qr[i];
+      }
     }
+    u32x4 zc[C];
+    if (!INC)
+#pragma unroll
+      for (int i = 0; i < C; ++i) zc[i] = zr[i];
     if (tid < L) {
       float c = rate * dt_r;
 #pragma unroll
@@ -418,6 +425,17 @@ __global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ssm_chunk_kernel(const
     if (!INC && 16 * wave < n) {
       const int t = 16 * wave + r;
       const float ct = cum[t];
+      bf16_t* G = Q + 16 * wave * QS;
+      u32x4 qc[D];
+#pragma unroll
+      for (int s = 0; s < D; ++s) qc[s] = *(const u32x4*)(G + r * QS + 32 * s + 8 * q);
+      wave_lds_order();
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        const int piece = lane + 64 * i;
+        *(u32x4*)(G + piece / (vp / 8) * QS + piece % (vp / 8) * 8) = zc[i];
+      }
+      wave_lds_order();
       f32x4 o[PT];
 #pragma unroll
       for (int i = 0; i < PT; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -456,18 +474,21 @@ __global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ssm_chunk_kernel(const
           o[i] = mfma(x, pl, o[i]);
         }
       }
-      if (t < n) {
-        const int64_t row = row0 + t0 + t;
-        const bf16_t* z = (const bf16_t*)a.proj + row * a.ldp + a.col_z + h * vp;
-        bf16_t* dst = (bf16_t*)a.out + row * a.ldo;
 #pragma unroll
-        for (int i = 0; i < PT; ++i) {
-          const f32x4 x = ld4(X + t * XS + 16 * i + 4 * q), zz = ld4(z + 16 * i + 4 * q);
-          f32x4 y = o[i] + skip * x;
+      for (int i = 0; i < PT; ++i) {
+        bf16_t* at = G + r * QS + 16 * i + 4 * q;
+        const f32x4 x = ld4(X + t * XS + 16 * i + 4 * q), zz = ld4(at);
+        f32x4 y = o[i] + skip * x;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) y[e] *= silu_fast(zz[e]);
-          st4(dst + in_chunks(h * vp + 16 * i + 4 * q, a.out_chunk), y);
-        }
+        for (int e = 0; e < 4; ++e) y[e] *= silu_fast(zz[e]);
+        st4(at, y);
+      }
+      wave_lds_order();
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        const int piece = lane + 64 * i, tz = piece / (vp / 8), d = piece % (vp / 8) * 8;
+        if (16 * wave + tz < n)
+          *(u32x4*)((bf16_t*)a.out + (int64_t)(row0 + t0 + 16 * wave + tz) * a.ldo + in_chunks(h * vp + d, a.out_chunk)) = *(const u32x4*)(G + tz * QS + d);
       }
     }
 
@@ -536,7 +557,7 @@ struct ChunkPick {
 };
 template <int D, int C>
 ChunkPick chunk_of() {
-  return ChunkPick{ssm_chunk_kernel<D, C, false>, ssm_chunk_kernel<D, C, true>, (L * (32 * C + 8) + (L + 64 * C) * (32 * D + 8)) * 2};
+  return ChunkPick{ssm_chunk_kernel<D, C, false>, ssm_chunk_kernel<D, C, true>, (L * (32 * C + 8) + (L + 64 * C) * (32 * D + 8) + L * (32 * (D > C ? D : C) + 8)) * 2};
 }
 template <int D>
 ChunkPick chunk_by_width(int c) {
