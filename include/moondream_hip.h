@@ -108,12 +108,12 @@ typedef struct {
 
 /* Tile choice of a launch with more than 64 rows -- a PER-CALL property (ABI 5; up to ABI 4 a process-wide tuning key):
  *   MD_TILE_BY_SHAPE  the config that is fastest for (m, n, k): small launches (one image: 730 / 1458 rows) take the
- *                     64x64 / 128x128 / 256x128 configs (32x32x16 MFMAs), large ones the four-wave 256x256 kernel
+ *                     64x64 / 128x128 / 256x128 configs (32x32x16 or 16x16x32 MFMAs), large ones the four-wave 256x256 kernel
  *                     (16x16x32 MFMAs).  The two families sum K in different associations: equal to fp32 rounding of the
- *                     accumulator, not bitwise -- so a row's bits can depend on how many rows travel with it.
- *   MD_TILE_PINNED    the tile config is a function of the layer (n, k) alone, never of m: every launch of more than 64
- *                     rows takes the 256x256 kernel, so a sequence gets the same bits alone and in any batch.  That
- *                     kernel addresses a launch with 32-bit byte offsets (m * lda * 2 < 4 GiB, (m + 256) * ldc * 2 <
+ *                     accumulator, not always bitwise -- so a row's bits can depend on how many rows travel with it.
+ *   MD_TILE_PINNED    the products and their order are a function of the layer (n, k) alone, never of m: every launch of more
+ *                     than 64 rows takes the 256x256 kernel, or smaller tiles of the same bits where that leaves CUs without
+ *                     work, so a sequence gets the same bits alone and in any batch.  The 256x256 kernel addresses a launch with 32-bit byte offsets (m * lda * 2 < 4 GiB, (m + 256) * ldc * 2 <
  *                     0xfffff000: ~150 000 rows of the 2B fused qkv|fc1 layer); a larger launch is cut into row blocks
  *                     of the same kernel (same bits), and one that cannot be cut -- a broadcast residual
  *                     (res_row_mod != 0), the RoPE epilogue -- returns MD_ERR_UNSUPPORTED instead of changing family.

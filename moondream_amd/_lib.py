@@ -16,12 +16,12 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 REPO = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB_PATH = os.path.join(HERE, "libmoondream_hip.so")
-SOURCES = ["gemm_bf16.hip", "gemm_w4.hip", "gemm_fp8w.hip", "gemm_f8.hip", "quant_f8.hip", "attention_f8kv.hip", "decode_b1.hip", "attention.hip",
+SOURCES = ["gemm_bf16.hip", "gemm_w4.hip", "gemm_mid.hip", "gemm_fp8w.hip", "gemm_f8.hip", "quant_f8.hip", "attention_f8kv.hip", "decode_b1.hip", "attention.hip",
            "elementwise.hip", "image_crops.hip", "sampling_region.hip", "api.hip", "abi.hip", "lm_ops.hip", "gemm_step.hip", "gemm_f32.hip", "attention_talk.hip", "retention.hip",
            "attention_latent.hip", "state_space.hip", "experts.hip", "gemm_experts.hip", "streams.hip", "lm_api.hip"]
 # the part of the library that the layered language models use: a checkout that serves only such a model compiles no more
 LM_LIB_PATH = os.path.join(HERE, "libmoondream_lm.so")
-LM_SOURCES = ["gemm_bf16.hip", "gemm_w4.hip", "elementwise.hip", "sampling_region.hip", "abi.hip", "lm_ops.hip", "gemm_step.hip", "gemm_f32.hip", "attention_talk.hip",
+LM_SOURCES = ["gemm_bf16.hip", "gemm_w4.hip", "gemm_mid.hip", "elementwise.hip", "sampling_region.hip", "abi.hip", "lm_ops.hip", "gemm_step.hip", "gemm_f32.hip", "attention_talk.hip",
               "retention.hip", "attention_latent.hip", "state_space.hip", "experts.hip", "gemm_experts.hip", "streams.hip", "lm_api.hip"]
 HEADERS = ["md_common.hpp", "gemm_internal.hpp", "stage_common.hpp", "lm_internal.hpp"]
 

@@ -756,6 +756,8 @@ md_status launch_epi(const GemmK& k, int tile, hipStream_t stream) {
     // weight panel per 128 rows instead of one per 64.  Same K order per output element as 16.
     case 21: return k.slices > 1 ? launch_cfg<128, 64, 4, 1, EPI, true, 4, 64, 0, 2>(k, stream)
                                  : launch_cfg<128, 64, 4, 1, EPI, false, 4, 64, 0, 2>(k, stream);
+    case 22: return md_gemm_mid_launch(k, EPI, 256, stream);  // 256 x 128 and 128 x 128, operands of two slices in registers (gemm_mid.hip)
+    case 23: return md_gemm_mid_launch(k, EPI, 128, stream);
     // up to one tile per CU: a ring of four instead of a second resident workgroup (216 tiles, K 2048: 32.8 -> 19.5 us)
     default:
       return (long)((k.M + 127) / 128) * ((k.n_store + 127) / 128) <= 256 ? launch_cfg<128, 128, 2, 2, EPI, false, 4>(k, stream)
@@ -789,60 +791,58 @@ int decode_slices(int n_store, int k_pad) {
   return s;
 }
 
-// Tile choice: every CU works through ceil(tiles / 256) tiles, a tile costs its area
-// over the config's measured efficiency (256x256 alternating schedule = 1; 256x128
-// ~0.78; 128x128 ~0.62 -- profiles/r01_gemm_alternating_sweep*.txt).  A function of the shape
-// (M, N, K) only, so a given layer always runs the same kernel -- and every config
-// accumulates K in the same order (sequential 16-wide MFMA steps), so results do
-// not depend on it.
+// Tile choice: every CU works through ceil(tiles / 256) tiles, a tile costs its area over the config's measured rate.  256 x 256 = 1; 256 x 128 0.82; 128 x 128
+// 0.61 (K 2048, rounds of tiles: 47, 28.5 and 19.3 us each; 2940 rows, 2048 columns, K 2048 / 8192: 43 / 169 us, 29 / 102, 38 / 116; 2322 rows, K 4352, 1152 columns
+// 94, 48, 34; 4900 rows, 2048 columns 51, 55, 58; 8000 rows, 4352 columns 138, 150, 168).  A function of the shape
+// (M, N, K) only, so a given layer always runs the same kernel.  small: the config for 128 x 128
+int by_rounds(int M, int n_store, int small) {
+  const int bm[3] = {256, 256, 128}, bn[3] = {256, 128, 128}, tile[3] = {20, 22, small};
+  const double rate[3] = {1.0, 0.82, 0.61};
+  int best = 2;
+  double best_cost = 1e300;
+  for (int c = 0; c < 3; ++c) {
+    const long tiles = (long)((M + bm[c] - 1) / bm[c]) * ((n_store + bn[c] - 1) / bn[c]);
+    const double cost = (double)((tiles + 255) / 256) * bm[c] * bn[c] / rate[c];
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = c;
+    }
+  }
+  return tile[best];
+}
 int pick_tile(int M, int n_store, int K, int policy) {
   if (knobs().tile >= 0) return knobs().tile;  // experiments / tests: force a tile config
-  // MD_TILE_PINNED (md_gemm_args.tile_policy, per call): the config is a function of the layer, never of the row count --
-  // the 256x256 kernel (16x16x32 MFMAs; the small-shape configs below multiply with 32x32x16: equal to fp32 rounding, not
-  // bitwise), so that a sequence gets the same bits alone and in a batch
-  if (policy == MD_TILE_PINNED && M > 64) return knobs().w4 ? 20 : 11;
+  // MD_TILE_PINNED (md_gemm_args.tile_policy, per call): the products and their order are a function of the layer, never of the row count -- 16x16x32
+  // MFMAs with K in order (the small-shape configs below multiply with 32x32x16: equal to fp32 rounding, not always bitwise), so that a
+  // sequence gets the same bits alone and in a batch: the 256 x 256 kernel, or where its tiles leave CUs without work the smaller tiles of gemm_mid.hip
+  if (policy == MD_TILE_PINNED && M > 64) return knobs().w4 ? by_rounds(M, n_store, 23) : 11;
   // MD_TILE_DECODE_TALL: 65 .. 128 rows of a decode step -- the 128 x 64 weight-streaming tile (21), except for the widest layers
   // (lm_head: 800 column panels keep every CU busy with the 128 x 128 two-stage config, measured 57 vs 73 us); every config
   // involved multiplies with 32x32x16 in the same K order as the 64-row decode configs
   if (policy == MD_TILE_DECODE_TALL && M > 64 && M <= 128 && n_store < 16384) return 21;
-  // Single-image regime (1458 ViT rows / 735 decoder rows; every config named here multiplies with 32x32x16 in the same K
-  // order: the choice never changes a bit).
+  // Single-image regime (1458 ViT rows / 735 decoder rows; every config named here sums K in the same order, as 32x32x16 or (22, 23) 16x16x32 products).
   //  * at most 128 tiles of 128 x 128 and a long K (proj / fc2 of both towers): half the chip is idle whatever the tile and the
   //    launch runs at the latency of its K loop -- the 64 x 64 tiles with the 4-deep ring and DMA helper waves (the decode-regime
   //    config) quadruple the workgroups (tools/sweep_gemm_b1.py, round 2: text fc2 at 730 rows 81 -> 61 us, ViT fc2 50 -> 30 us).
-  //    Round 5 re-swept it: a 128 x 128 tile on a four-stage ring wins the back-to-back sweep (text fc2 63.7 -> 52.0 us) and LOSES
-  //    inside a caption, where the layer's weights come from HBM and 96 workgroups pull them through 96 CUs (ViT proj / fc2 23.7 ->
-  //    24.9 us, text 42.0 -> 42.5 us per launch: profiles/r05_b1_tile_config_sweep.txt) -- the 64 x 64 config stays.
   //  * up to 512 tiles of 128 x 128 (ViT qkv / fc1, projector fc1): the two-stage 128 x 128 config keeps TWO workgroups per CU, so
   //    all of them are resident at once; the cost model below counts one workgroup per CU and preferred 256 x 128.  Inside a
   //    caption: ViT qkv 25.9 -> 21.5 us, fc1 29.2 -> 24.9 us per launch (round 5).  Wider layers (the decoder's fused qkv|fc1: 672
   //    such tiles) stay with the cost model, i.e. the four-wave kernel.
   if (M > 64) {
     const long t128 = (long)((M + 127) / 128) * ((n_store + 127) / 128);
-    if (K >= 1024 && t128 <= 128) return 16;
+    //    From about 90 tiles of 128 x 128 on they beat the 64 x 64 ones (700 rows, 2048 columns, K 2048 / 5440 / 8192: 17.6 / 43 / 57 us against 18.1 / 46 / 64; 300 rows
+    //    16.9 / 40 / 55 and 13.8 / 31 / 45).
+    if (K >= 1024 && t128 <= 128) return t128 > 90 ? 23 : 16;
     // ("small_m_rule": 0 = round 2's rule, 1 = the default below, n > 1 = that many tiles instead of 512 -- A/B)
     const int rule = knobs().small_m_rule;
-    //  * of these, where 256 x 128 tiles are one round of the CUs: 384 rows and columns of operands per slice instead of two resident tiles'
-    //    512 (510 tiles, K 2048: 39.9 -> 33.0 us; every config here was seen to move about 50 GB/s through a CU, which is not explained yet)
+    //  * of these, where 256 x 128 tiles are one round of the CUs (700 rows, 10880 columns, K 2048: 47 us as 128 x 128, 40 as 256 x 128, 35 with the operands of two
+    //    slices in registers)
     const long t256 = (long)((M + 255) / 256) * ((n_store + 127) / 128);
-    if (rule == 1 && t128 > 256 && t128 <= 512 && t256 <= 256) return 1;
+    if (rule == 1 && t128 > 256 && t128 <= 512 && t256 <= 256) return 22;
     if (rule != 0 && t128 <= (rule > 1 ? rule : 512)) return 2;
   }
-  const int bm[3] = {256, 256, 128}, bn[3] = {256, 128, 128};
-  const double eff[3] = {1.0, 0.70, 0.55};
-  int best = 2;
-  double best_cost = 1e300;
-  for (int c = 0; c < 3; ++c) {
-    const long tiles = (long)((M + bm[c] - 1) / bm[c]) * ((n_store + bn[c] - 1) / bn[c]);
-    const long per_cu = (tiles + 255) / 256;
-    const double cost = (double)per_cu * bm[c] * bn[c] / eff[c];
-    if (cost < best_cost) {
-      best_cost = cost;
-      best = c;
-    }
-  }
-  if (best == 0) best = knobs().w4 ? 20 : 11;
-  return best;
+  const int best = by_rounds(M, n_store, 2);
+  return best == 20 && !knobs().w4 ? 11 : best;
 }
 
 }  // namespace
@@ -895,6 +895,8 @@ md_status gemm_dispatch(const md_gemm_args* a, void* stream, const md_rope_fuse*
   k.slabs = nullptr;
   k.tickets = nullptr;
   const bool forced = knobs().tile >= 0;
+  // (the RoPE epilogue is the four-wave kernel's; what it refuses or takes in blocks of rows does not depend on the tile that the rows would have had)
+  if (a->tile_policy == MD_TILE_PINNED && (tile == 22 || tile == 23) && !(knobs().tile >= 0) && (rf != nullptr || !md_gemm_w4_takes(k, a->epilogue))) tile = 20;
   if (tile == 20 && !md_gemm_w4_takes(k, a->epilogue)) {
     if (a->tile_policy != MD_TILE_PINNED) {
       tile = 11;
@@ -1090,7 +1092,7 @@ md_status md_gemm_partial_rows(const void* a, int64_t lda, const md_linear& lin,
   ProfScope prof;
   if (prof.begin(2.0 * (double)lin.n * (double)lin.k, s) != MD_OK) return MD_ERR_LAUNCH;
   const int cfg = decode_cfg();
-  const md_status st = m > 128 ? launch_cfg<128, 128, 2, 2, MD_EPI_BIAS, true, 4>(k, s)
+  const md_status st = m > 128 ? md_gemm_mid_partial(k, s)
                        : m > 64 ? launch_cfg<128, 64, 4, 1, MD_EPI_BIAS, true, 4, 64, 0, 2>(k, s)
                        : (cfg == 17 || cfg == 18) ? launch_cfg<64, 64, 2, 2, MD_EPI_BIAS, true, 4, 64, 0, 2>(k, s)
                        : (cfg == 16 || cfg == 19) ? launch_cfg<64, 64, 2, 1, MD_EPI_BIAS, true, 4, 64, 0, 2>(k, s)
@@ -1174,7 +1176,8 @@ md_status md_gemm_silu_bf16(const void* a, int64_t lda, const md_linear& lin, vo
     case 11: return launch_cfg<256, 256, 2, 4, MD_EPI_SILU, false, 4, 32, 2>(k, s);
     case 21: return launch_cfg<128, 64, 4, 1, MD_EPI_SILU, false, 4, 64, 0, 2>(k, s);
     case 16: return launch_cfg<64, 64, 2, 1, MD_EPI_SILU, false, 4, 64, 0, 2>(k, s);
-    case 1: return launch_cfg<256, 128, 4, 2, MD_EPI_SILU, false, 3>(k, s);
+    case 22: return md_gemm_mid_launch(k, MD_EPI_SILU, 256, s);
+    case 23: return md_gemm_mid_launch(k, MD_EPI_SILU, 128, s);
     default:
       return (long)((rows + 127) / 128) * ((k.n_store + 127) / 128) <= 256 ? launch_cfg<128, 128, 2, 2, MD_EPI_SILU, false, 4>(k, s)
                                                                          : launch_cfg<128, 128, 2, 2, MD_EPI_SILU>(k, s);

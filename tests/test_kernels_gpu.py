@@ -119,6 +119,28 @@ def test_gemm_tile_configs_agree_bitwise(lib, force_tile):
         assert torch.equal(gemm(lib, a, lin), first), f"tile 20 rep {rep}"
 
 
+@pytest.mark.parametrize("k,n", [(64, 64), (128, 1000), (192, 304), (256, 2048), (320, 136), (1152, 1152), (2100, 520)], ids=str)
+def test_smaller_tiles_have_the_bits_of_the_four_wave_kernel(lib, force_tile, k, n):
+    """256 x 128 (22) and 128 x 128 (23) tiles with the operands of two slices in registers: rings that are not filled, tiles with one live row and one dead, columns
+    behind the last tile's, every epilogue; a residual that several row blocks share."""
+    w, b = randn(n, k, scale=1 / math.sqrt(k), seed=72), randn(n, scale=0.1, seed=73)
+    lin = PackedLinear(w, b, "cuda")
+    pos = randn(65, n, seed=75)
+    for m in (65, 127, 128, 129, 256, 257, 300, 641):
+        a, r = pad_k(randn(m, k, seed=m), lin.k_pad), randn(m, n, seed=m + 1)
+        for kw in (dict(), dict(epi=_lib.MD_EPI_GELU), dict(epi=_lib.MD_EPI_RESIDUAL, r=r), dict(epi=_lib.MD_EPI_RESIDUAL, r=pos, res_row_mod=65)):
+            got = {}
+            for tile in (11 if kw.get("res_row_mod") else 20, 22, 23):  # (the four-wave kernel takes no residual of fewer rows than a tile has)
+                force_tile(tile)
+                got[tile] = gemm(lib, a, lin, **kw)
+            want, g22, g23 = got.values()
+            assert torch.equal(g22, g23), (m, kw.keys())
+            if kw.get("res_row_mod"):
+                compare(f"{m} x {n} residual", g22, want, 3e-4, 2e-2)
+            else:
+                assert torch.equal(g22, want), (m, kw.keys())
+
+
 def test_tile_policy_is_a_per_call_field(lib, force_tile):
     """ABI 5: md_gemm_args.tile_policy.  MD_TILE_PINNED makes the tile config of a > 64-row launch a function of the layer alone --
     the 256 x 256 kernel whatever the row count -- so a row gets the same bits in a 100-row and in a 5000-row launch; MD_TILE_BY_SHAPE
