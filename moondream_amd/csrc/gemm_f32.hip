@@ -1,9 +1,7 @@
 // Matrix products in fp32:  C[m][n] = sum_k A[m][k] W[n][k] + b[n],  K and N multiples of 64 (v_mfma_f32_16x16x4_f32).
 //
-//   gemm_f32_kernel        64 x 64 tiles (64 x 32 up to 128 of those), eight waves, K in steps of 64 through two LDS buffers: the next step's loads
-//                          are in registers under this step's products, one barrier per step.  Bound by the matrix cores (153 TFLOP/s in a large
-//                          library product) once every CU has tiles.  380 rows, 2048 columns, K 2048 and 5440 on average: 81 us, 192 tiles; with
-//                          four waves, one buffer and K in steps of 16: 157 us.  10880 columns of K 2048: 161 us, 105 TFLOP/s (171 us).
+//   gemm_f32_kernel        tiles of 64 x 64 or 48 x 64, 64 x 32 up to 128 of those; one barrier per step of 64.  Bound by the matrix cores (153 TFLOP/s in a
+//                          large library product) once every CU has tiles.
 //   gemm_f32_rows_kernel   up to 32 rows, where the weights are a memory stream: a workgroup owns 16 columns and all of K, its eight waves load (three
 //                          stages ahead), one wave per 16 rows multiplies.  8 rows: a pass of 24 layers 3.2 ms, 14.1 through four-wave tiles; 30
 //                          rows: 3.8 ms.  64 rows through the tiles above: 5.6 ms.
@@ -17,6 +15,8 @@
 //   grouped: a tile's rows are slots of one group, gathered through row_of (gemm_internal.hpp)
 #include "gemm_internal.hpp"
 #include "lm_internal.hpp"
+
+#include <type_traits>
 
 namespace {
 
@@ -36,81 +36,123 @@ struct F32Args {
   int chain;
 };
 
-// BN: columns.  A wave has 32 x 16 of a 64 x 64 tile, 16 x 16 of a 64 x 32 tile
-template <bool GRP, int BN>
-__global__ __launch_bounds__(512) void gemm_f32_kernel(const F32Args p) {
-  constexpr int NI = BN / 32;  // 16-row blocks per wave, f32x4 of the weight tile per thread
-  __shared__ __attribute__((aligned(16))) float As[2][64 * LS], Ws[2][BN * LS];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int m0 = blockIdx.y * 64, m_end = p.m, group = 0;
+// WM x WN waves, each MI x NI blocks of 16 x 16: tiles of 16 MI WM x 16 NI WN.  K in steps of 64 through two LDS buffers, the step after the next in
+// registers.  What bounds it beside the products is the LDS port (reads of 4 bytes, two lanes to a bank: 58 % busy with 32 x 16 per wave), so a wave has 32 x 32 or 48 x 16,
+// and reads its operands NB products ahead, not all at once behind the barrier.  380 rows, K 2048: 10880 columns 188 -> 167 us (32 x 16 per wave, four
+// products ahead -> two); two k side by side for one read of 8 bytes: 171 and 167.  48 rows where they even out the CUs: 2048 columns 46 -> 39, K 5440 118 -> 99.
+template <bool GRP, int WM, int MI, int WN, int NI, int NB>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(const F32Args p) {
+  constexpr int BM = 16 * MI * WM, BN = 16 * WN * NI, NT = 64 * WM * WN, NA = (BM * 16 + NT - 1) / NT, NW = BN * 16 / NT + (BN * 16 % NT != 0);
+  __shared__ __attribute__((aligned(16))) float As[2][BM * LS], Ws[2][BN * LS];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int m0 = blockIdx.y * BM, m_end = p.m, group = 0;
   if constexpr (GRP)
-    if (!grouped_tile(p.offsets, p.groups, 64, blockIdx.y, group, m0, m_end)) return;
-  constexpr int WM = 4 / NI;  // waves along the rows
-  const int n0 = blockIdx.x * BN, wm = (wave & (WM - 1)) * 16 * NI, wn = wave / WM * 16;
-  const int lr = tid >> 4, lc = (tid & 15) * 4;  // f32x4 of the operand tiles: rows lr and lr + 32
-  const float *ap[2], *wp[NI];
+    if (!grouped_tile(p.offsets, p.groups, BM, blockIdx.y, group, m0, m_end)) return;
+  const int n0 = blockIdx.x * BN, wm = wave % WM * 16 * MI, wn = wave / WM * 16 * NI;
+  // f32x4 tid + NT j of the operand tiles, 16 to a row: bytes within the tile (32 bits beside a uniform base), or of gathered rows
+  typedef typename std::conditional<GRP, uint64_t, uint32_t>::type Offset;
+  Offset ao[NA];
+  uint32_t wo[NW];
+  auto row_of = [&](int j) { return (tid + NT * j) >> 4; };
+  const int lc = (tid & 15) * 4;
+  const float *ab = p.a + (GRP ? 0 : (int64_t)m0 * p.lda), *wb = p.w + ((int64_t)group * p.n_pad + n0) * p.k;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    int64_t row = min(m0 + lr + 32 * j, m_end - 1);
+  for (int j = 0; j < NA; ++j) {
+    int64_t row = min(m0 + row_of(j), m_end - 1);
     if constexpr (GRP)
       if (p.row_of) row = p.row_of[row];
-    ap[j] = p.a + row * p.lda + lc;
+    ao[j] = (Offset)(((row - (GRP ? 0 : m0)) * p.lda + lc) * 4);
   }
 #pragma unroll
-  for (int j = 0; j < NI; ++j) wp[j] = p.w + ((int64_t)group * p.n_pad + n0 + lr + 32 * j) * p.k + lc;
-  f32x4 av[2], wv[NI], acc[NI], sum[NI];
+  for (int j = 0; j < NW; ++j) wo[j] = ((uint32_t)min(row_of(j), BN - 1) * (uint32_t)p.k + lc) * 4;
+  f32x4 av[2][NA], wv[2][NW], acc[MI][NI], sum[MI][NI];
 #pragma unroll
-  for (int i = 0; i < NI; ++i) acc[i] = sum[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j) acc[i][j] = sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int r = lane & 15, kq = lane >> 4;
-  auto load = [&](int k0) {
+  auto load = [&](auto set_c, int k0) {  // past the end: the last step again, not used
+    constexpr int S = decltype(set_c)::value;
+    const int k = min(k0, p.k - BK);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) av[j] = *(const f32x4*)(ap[j] + k0);
+    for (int j = 0; j < NA; ++j) av[S][j] = *(const f32x4*)((const char*)(ab + k) + ao[j]);
 #pragma unroll
-    for (int j = 0; j < NI; ++j) wv[j] = *(const f32x4*)(wp[j] + k0);
+    for (int j = 0; j < NW; ++j) wv[S][j] = *(const f32x4*)((const char*)(wb + k) + wo[j]);
   };
-  auto store = [&](int buf) {
+  auto store = [&](auto set_c, int buf) {
+    constexpr int S = decltype(set_c)::value;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) *(f32x4*)(As[buf] + (lr + 32 * j) * LS + lc) = av[j];
+    for (int j = 0; j < NA; ++j)
+      if (NA * NT == BM * 16 || row_of(j) < BM) *(f32x4*)(As[buf] + row_of(j) * LS + lc) = av[S][j];
 #pragma unroll
-    for (int j = 0; j < NI; ++j) *(f32x4*)(Ws[buf] + (lr + 32 * j) * LS + lc) = wv[j];
+    for (int j = 0; j < NW; ++j)
+      if (NW * NT == BN * 16 || row_of(j) < BN) *(f32x4*)(Ws[buf] + row_of(j) * LS + lc) = wv[S][j];
   };
-  load(0);
-  store(0);
-  __syncthreads();
-  for (int k0 = 0, buf = 0; k0 < p.k; k0 += BK, buf ^= 1) {
-    const bool more = k0 + BK < p.k;  // (uniform)
-    if (more) load(k0 + BK);
-    const float *as = As[buf] + (wm + r) * LS + kq, *ws = Ws[buf] + (wn + r) * LS + kq;
-    float a[BK / 4][NI], w[BK / 4];
+  float a[2][NB][MI], w[2][NB][NI];
+  auto read = [&](int set, int buf, int batch) {
+    const float *as = As[buf] + (wm + r) * LS + kq + 4 * NB * batch, *ws = Ws[buf] + (wn + r) * LS + kq + 4 * NB * batch;
 #pragma unroll
-    for (int s = 0; s < BK / 4; ++s) {
+    for (int s = 0; s < NB; ++s) {
 #pragma unroll
-      for (int i = 0; i < NI; ++i) a[s][i] = as[16 * i * LS + 4 * s];
-      w[s] = ws[4 * s];
+      for (int i = 0; i < MI; ++i) a[set][s][i] = as[16 * i * LS + 4 * s];
+#pragma unroll
+      for (int j = 0; j < NI; ++j) w[set][s][j] = ws[16 * j * LS + 4 * s];
     }
+  };
+  constexpr auto S0 = std::integral_constant<int, 0>{};
+  constexpr auto S1 = std::integral_constant<int, 1>{};
+  load(S0, 0);
+  load(S1, BK);
+  store(S0, 0);
+  __syncthreads();
+  // buffer B holds step k0; the registers of the other set the next one
+  auto step = [&](auto buf_c, int k0) {
+    constexpr int B = decltype(buf_c)::value;
+    constexpr auto OTHER = std::integral_constant<int, 1 - B>{};
+    const bool more = k0 + BK < p.k;  // (uniform)
+    read(0, B, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    load(buf_c, k0 + 2 * BK);
 #pragma unroll
-    for (int s = 0; s < BK / 4; ++s)
+    for (int b = 0; b < BK / 4 / NB; ++b) {
+      if (b + 1 < BK / 4 / NB) read((b + 1) & 1, B, b + 1);
+      if (b == 1 && more) store(OTHER, 1 - B);  // (read last before the previous barrier)
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < NI; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][i], w[s], acc[i], 0, 0, 0);
+      for (int s = 0; s < NB; ++s)
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[b & 1][s][i], w[b & 1][s][j], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     if (!more || (!p.chain && (k0 & (SLAB - 1)) == SLAB - BK)) {
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        sum[i] += acc[i];
-        acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+          sum[i][j] += acc[i][j];
+          acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
     }
-    if (more) store(buf ^ 1);  // (read last before the previous barrier)
     __syncthreads();
+  };
+  for (int k0 = 0; k0 < p.k; k0 += 2 * BK) {
+    step(S0, k0);
+    if (k0 + BK < p.k) step(S1, k0 + BK);
   }
-  const int n = n0 + wn + r;
-  const float b = p.bias ? p.bias[n] : 0.f;
 #pragma unroll
-  for (int i = 0; i < NI; ++i)
+  for (int j = 0; j < NI; ++j) {
+    const int n = n0 + wn + 16 * j + r;
+    const float b = p.bias ? p.bias[n] : 0.f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int m = m0 + wm + 16 * i + 4 * kq + e;
-      if (m < m_end) p.c[(int64_t)m * p.ldc + n] = sum[i][e] + b;
-    }
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int m = m0 + wm + 16 * i + 4 * kq + e;
+        if (m < m_end) p.c[(int64_t)m * p.ldc + n] = sum[i][j][e] + b;
+      }
+  }
 }
 
 // MT 16-row tiles; RK of K per stage, two of them in LDS, AHEAD more in registers.  What bounds a workgroup is the chain of dependent products (22 ns
@@ -203,8 +245,12 @@ md_status lm_gemm_f32(const void* a, int64_t lda, const md_linear& lin, void* c,
     else hipLaunchKernelGGL(gemm_f32_rows_kernel<2>, grid, block, 0, s, p);
   } else {
     const int rows = (m + 63) / 64;
-    if (rows * (lin.n_pad / 64) <= 128) hipLaunchKernelGGL((gemm_f32_kernel<false, 32>), dim3(lin.n_pad / 32, rows), dim3(512), 0, s, p);
-    else hipLaunchKernelGGL((gemm_f32_kernel<false, 64>), dim3(lin.n_pad / 64, rows), dim3(512), 0, s, p);
+    // rows that the fullest of the 256 CUs gets: tiles of 48 rows where they even that out (a row of theirs takes 5 % longer; 380 rows, 6144 columns 100 us against 120, 51200: 25
+    // tiles of 48 or 19 of 64 on the fullest CU, 1042 and 930)
+    const int cols = lin.n_pad / 64, by64 = (rows * cols + 255) / 256 * 64, by48 = ((m + 47) / 48 * cols + 255) / 256 * 48;
+    if (rows * cols <= 128) hipLaunchKernelGGL((gemm_f32_kernel<false, 4, 1, 2, 1, 4>), dim3(lin.n_pad / 32, rows), dim3(512), 0, s, p);
+    else if (by48 * 22 < by64 * 21) hipLaunchKernelGGL((gemm_f32_kernel<false, 1, 3, 4, 1, 4>), dim3(cols, (m + 47) / 48), dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((gemm_f32_kernel<false, 2, 2, 2, 2, 2>), dim3(cols, rows), dim3(256), 0, s, p);
   }
   return md_launch_status();
 }
@@ -217,6 +263,6 @@ extern "C" md_status md_gemm_f32(const void* a, int64_t lda, const md_linear* li
 md_status lm_grouped_gemm_f32(const void* a, int64_t lda, const int32_t* row_of, const md_linear& lin, int experts, const int32_t* offsets, void* c,
                               int64_t ldc, int slots, bool chain, hipStream_t s) {
   const F32Args p = {(const float*)a, lda, (const float*)lin.w, nullptr, (float*)c, ldc, slots, lin.k_pad, lin.n_pad, row_of, offsets, experts, chain};
-  hipLaunchKernelGGL((gemm_f32_kernel<true, 64>), dim3(lin.n_pad / 64, grouped_tiles(slots, experts, 64)), dim3(512), 0, s, p);
+  hipLaunchKernelGGL((gemm_f32_kernel<true, 2, 2, 2, 2, 2>), dim3(lin.n_pad / 64, grouped_tiles(slots, experts, 64)), dim3(256), 0, s, p);
   return md_launch_status();
 }

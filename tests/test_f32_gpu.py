@@ -88,6 +88,31 @@ def forward(cfg, lens, context=192):
     return torch.cat(got), torch.cat([x[:-1] for x in want] + [x[-1:] for x in want])
 
 
+@pytest.mark.parametrize("m,n,k", [(380, 2048, 192), (385, 2048, 64), (129, 4224, 128), (145, 2880, 448), (65, 8256, 64), (449, 2048, 320)], ids=str)
+def test_tiles_of_48_and_64_rows(m, n, k):
+    """Tiles of 48 rows where they even out the CUs (380, 129, 145 rows), of 64 elsewhere, last tiles of one row and of all but one, K of one step: the bits of the kernel
+    that takes up to 32 rows, row by row, and fp32 rounding from 64 bits."""
+    import ctypes as C
+
+    from moondream_amd import _lib
+
+    lib, g = _lib.load(), torch.Generator(device="cuda").manual_seed(m)
+    a, w, b = (torch.randn(*s, device="cuda", generator=g) for s in ((m, k), (n, k), (n,)))
+    lin = _lib.MdLinear(w.data_ptr(), b.data_ptr(), n, k, n, k)
+
+    def product(rows):
+        c = torch.full((rows.shape[0] + 1, n), float("nan"), device="cuda")
+        _lib.check(lib.md_gemm_f32(rows.data_ptr(), k, C.byref(lin), c.data_ptr(), n, rows.shape[0], torch.cuda.current_stream().cuda_stream))
+        assert bool(c[-1].isnan().all())
+        return c[:-1]
+
+    got = product(a)
+    assert torch.equal(got, torch.cat([product(x) for x in a.split(32)]))
+    want = a.double() @ w.double().t() + b.double()
+    # a chain of at most 128 products and k / 128 sums of them: half an ulp each, added up as a walk
+    assert float((got - want).pow(2).mean().sqrt()) < 2.0 ** -24 * k ** 0.5 * (min(k, 128) + k / 128) ** 0.5
+
+
 @pytest.mark.parametrize("rows,experts,top", [(9, 40, 1), (64, 1, 1), (65, 1, 1), (130, 2, 1), (131, 3, 2), (150, 70, 4)])
 def test_grouped_products(rows, experts, top):
     """Empty groups, groups of one row, of whole tiles and of a row more, gathered rows; groups that begin inside a tile's rows."""
