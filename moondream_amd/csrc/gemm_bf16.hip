@@ -793,17 +793,20 @@ int decode_slices(int n_store, int k_pad) {
 
 // Tile choice: every CU works through ceil(tiles / 256) tiles, a tile costs its area over the config's measured rate.  256 x 256 = 1; 256 x 128 0.82; 128 x 128
 // 0.61 (K 2048, rounds of tiles: 47, 28.5 and 19.3 us each; 2940 rows, 2048 columns, K 2048 / 8192: 43 / 169 us, 29 / 102, 38 / 116; 2322 rows, K 4352, 1152 columns
-// 94, 48, 34; 4900 rows, 2048 columns 51, 55, 58; 8000 rows, 4352 columns 138, 150, 168).  A function of the shape
+// 94, 48, 34; 4900 rows, 2048 columns 51, 55, 58; 8000 rows, 4352 columns 138, 150, 168).  Smaller tiles have to promise a sixth at least: by three rounds for
+// two they lose, since the 256 x 256 kernel's last round runs faster the fewer CUs it has work for (K 2048, 4900 rows, 4608 columns 83 us against 88, 4096 columns
+// 82 : 84; 2940 rows, 6144 columns 81 : 82, 8192 columns 83 : 89).  A function of the shape
 // (M, N, K) only, so a given layer always runs the same kernel.  small: the config for 128 x 128
 int by_rounds(int M, int n_store, int small) {
   const int bm[3] = {256, 256, 128}, bn[3] = {256, 128, 128}, tile[3] = {20, 22, small};
   const double rate[3] = {1.0, 0.82, 0.61};
-  int best = 2;
-  double best_cost = 1e300;
+  int best = 0;
+  double best_cost = 0;
   for (int c = 0; c < 3; ++c) {
     const long tiles = (long)((M + bm[c] - 1) / bm[c]) * ((n_store + bn[c] - 1) / bn[c]);
     const double cost = (double)((tiles + 255) / 256) * bm[c] * bn[c] / rate[c];
-    if (cost < best_cost) {
+    if (c == 0) best_cost = cost * 0.85;  // what the smaller ones have to beat
+    else if (cost < best_cost) {
       best_cost = cost;
       best = c;
     }
