@@ -127,22 +127,28 @@ __device__ __forceinline__ md_bf16x8v op(const u32x4& v) { return __builtin_bit_
 // registers meanwhile.  S^T = K Q^T (32x32x16), so a lane holds one query and 16 of every 32 keys: maximum and sum stay in the lane but for
 // one exchange, and the weights go from the accumulators straight into the second operand of O^T += V^T P^T; the order of the keys that this
 // implies is the one in which the transposing LDS reads fetch V.  D: dp / 32, C: vp / 32
+// KG: groups of four waves that take the tiles of keys in turn; the second's sums go to the first through LDS.  What bounds a workgroup is the chain through its tiles
+// (2 us each with one wave on a SIMD, where LDS and the address unit are half idle; 2.6 for two tiles with two), so two groups where each CU has one workgroup.
+// Whole passes of 8 layers, one group and two: 16 heads of 128, one prompt of 700 tokens 771 and 757 us (28 and 24 a launch), 1000 890 : 837, 2000 1293 : 1179; 4 heads
+// of 64, 1000 757 : 702, 3 x 2000 1512 : 1407.  Not for up to three tiles (7 x 100, 16 heads 684 : 690, 4 heads 556 : 590) and not past a workgroup per CU (32 heads,
+// 2000 1222 : 1266).  Two groups of two waves and blocks of 64 queries: as one group or slower, each tile's loads and LDS writes serve half as many queries.
 constexpr int value_stride(int vp) { return vp == 32 ? 32 : vp == 128 ? 160 : 96; }  // four rows of 64 bytes fall on different banks
-template <int D, int C>
+template <int D, int C, int KG>
 struct PrefillLds {
   static constexpr int KS = 32 * D + 8, VS = value_stride(32 * C), buffer = 64 * (KS + VS), OS = 32 * C + 8;
-  static constexpr int bytes = 2 * (2 * buffer > 4 * 32 * OS ? 2 * buffer : 4 * 32 * OS);
+  static constexpr int tiles = 2 * KG * buffer, outputs = 4 * 32 * OS, sums = KG > 1 ? 2 * 256 * (16 * C + 2) : 0;  // (fp32: two elements)
+  static constexpr int bytes = 2 * (tiles > outputs + sums ? tiles : outputs + sums);
 };
-template <int D, int C>
-__global__ __launch_bounds__(256, 2) void latent_prefill_kernel(const LmLatent a, int n_qblk) {
-  using M = PrefillLds<D, C>;
+template <int D, int C, int KG>
+__global__ __launch_bounds__(256 * KG, 2 / KG) void latent_prefill_kernel(const LmLatent a, int n_qblk) {
+  using M = PrefillLds<D, C, KG>;
   constexpr int dp = 32 * D, vp = 32 * C, KS = M::KS, VS = M::VS;
   extern __shared__ __attribute__((aligned(16))) bf16_t psm[];
   // all query blocks of a (sequence, head) on one XCD, whose L2 then holds its keys and values; the longest first
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, bh = (slot / n_qblk) * 8 + xcd;
   if (bh >= a.r.n_seq * a.heads) return;
-  const int seq = bh / a.heads, h = bh - seq * a.heads, tid = threadIdx.x, lane = tid & 63, hi = lane >> 5, l31 = lane & 31;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int seq = bh / a.heads, h = bh - seq * a.heads, tid = threadIdx.x & 255, lane = tid & 63, hi = lane >> 5, l31 = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
   const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, pos0 = a.r.seq_pos0[seq];
   const int q0 = (n_qblk - 1 - slot % n_qblk) * 128;
   if (q0 >= len) return;
@@ -190,17 +196,20 @@ __global__ __launch_bounds__(256, 2) void latent_prefill_kernel(const LmLatent a
       *(u32x4*)(V + j * VS + d) = vr[i];
     }
   };
-  load(0);
-  store(psm);
-  if (64 < kv_end) load(64);
+  constexpr int STEP = 64 * KG;
+  const int first = 64 * kg;  // (tiles past the end replay its last row, and are not used)
+  bf16_t* tiles = psm + 2 * kg * M::buffer;
+  load(first);
+  store(tiles);
+  if (first + STEP < kv_end) load(first + STEP);
   const int i16 = lane & 15, v_lane = (4 * hi + (i16 >> 2)) * VS + 16 * ((lane >> 4) & 1) + 4 * (i16 & 3);
   int buf = 0;
-  for (int j0 = 0; j0 < kv_end; j0 += 64, buf ^= 1) {
+  for (int j0 = first; j0 - first < kv_end; j0 += STEP, buf ^= 1) {
     __syncthreads();  // this tile is in LDS, and nobody reads the other buffer any more
-    const bf16_t *K = psm + buf * M::buffer, *V = K + 64 * KS;
-    if (j0 + 64 < kv_end) {
-      store(psm + (buf ^ 1) * M::buffer);
-      if (j0 + 128 < kv_end) load(j0 + 128);
+    const bf16_t *K = tiles + buf * M::buffer, *V = K + 64 * KS;
+    if (j0 + STEP < kv_end) {
+      store(tiles + (buf ^ 1) * M::buffer);
+      if (j0 + 2 * STEP < kv_end) load(j0 + 2 * STEP);
     }
     if (j0 > w_hi || w0 >= len) continue;  // (wave-uniform) no key of this tile is visible to the wave
     f32x16 s[2];
@@ -226,7 +235,7 @@ __global__ __launch_bounds__(256, 2) void latent_prefill_kernel(const LmLatent a
       for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[sub][e]);
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * sc;  // (a negative scale turns the order round: the bound below still holds for sc > 0 only)
     if (__any(mx - m > 6.0f)) {  // rescale only when a weight could exceed 2^6; the first tile always holds key 0, visible to all
-      const float mn = fmaxf(m, mx), f = __builtin_amdgcn_exp2f(m - mn);
+      const float mn = fmaxf(m, mx), f = KG > 1 && mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
       m = mn;
       l *= f;
 #pragma unroll
@@ -234,6 +243,7 @@ __global__ __launch_bounds__(256, 2) void latent_prefill_kernel(const LmLatent a
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[c][e] *= f;
     }
+    const float ref = KG > 1 && m == -INFINITY ? 0.f : m;  // (a second group's query may have seen no key yet)
     u32x4 p[2][2];
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub)
@@ -241,7 +251,7 @@ __global__ __launch_bounds__(256, 2) void latent_prefill_kernel(const LmLatent a
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float p0 = __builtin_amdgcn_exp2f(fmaf(s[sub][8 * u + 2 * e], sc, -m)), p1 = __builtin_amdgcn_exp2f(fmaf(s[sub][8 * u + 2 * e + 1], sc, -m));
+          const float p0 = __builtin_amdgcn_exp2f(fmaf(s[sub][8 * u + 2 * e], sc, -ref)), p1 = __builtin_amdgcn_exp2f(fmaf(s[sub][8 * u + 2 * e + 1], sc, -ref));
           l += p0 + p1;
           p[sub][u][e] = pack_bf16x2(p0, p1);
         }
@@ -256,9 +266,25 @@ __global__ __launch_bounds__(256, 2) void latent_prefill_kernel(const LmLatent a
           o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op(u32x4{v0[0], v0[1], v1[0], v1[1]}), op(p[sub][u]), o[c], 0, 0, 0);
         }
   }
-  const float inv = 1.0f / (l + __shfl_xor(l, 32, 64));
   __syncthreads();
+  if constexpr (KG > 1) {
+    float* sums = (float*)(psm + M::outputs) + tid;
+    constexpr int N = 16 * C;
+    if (kg) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) sums[256 * i] = o[i >> 4][i & 15];
+      sums[256 * N] = m;
+      sums[256 * (N + 1)] = l;
+    }
+    __syncthreads();
+    if (kg) return;
+    const float m1 = sums[256 * N], mn = fmaxf(m, m1), f0 = __builtin_amdgcn_exp2f(m - mn), f1 = __builtin_amdgcn_exp2f(m1 - mn);  // (m: key 0's group)
+    l = l * f0 + sums[256 * (N + 1)] * f1;
+#pragma unroll
+    for (int i = 0; i < N; ++i) o[i >> 4][i & 15] = o[i >> 4][i & 15] * f0 + sums[256 * i] * f1;
+  }
   if (w0 >= len) return;
+  const float inv = 1.0f / (l + __shfl_xor(l, 32, 64));
   const bf16_t* grow = (const bf16_t*)a.proj + (int64_t)(row0 + t) * a.ldp + a.col_g + h * vp;
   bf16_t* ot = psm + wave * 32 * M::OS;
 #pragma unroll
@@ -283,27 +309,31 @@ __global__ __launch_bounds__(256, 2) void latent_prefill_kernel(const LmLatent a
 
 typedef void (*PrefillKernel)(const LmLatent, int);
 struct PrefillPick {
-  PrefillKernel fn;
-  int lds;
+  PrefillKernel fn[2];  // one and two groups
+  int lds[2];
 };
+template <int D, int C>
+PrefillPick prefill_of() {
+  return {{latent_prefill_kernel<D, C, 1>, latent_prefill_kernel<D, C, 2>}, {PrefillLds<D, C, 1>::bytes, PrefillLds<D, C, 2>::bytes}};
+}
 template <int D>
 PrefillPick prefill_by_width(int c) {
   switch (c) {
-    case 1: return {latent_prefill_kernel<D, 1>, PrefillLds<D, 1>::bytes};
-    case 2: return {latent_prefill_kernel<D, 2>, PrefillLds<D, 2>::bytes};
-    case 3: return {latent_prefill_kernel<D, 3>, PrefillLds<D, 3>::bytes};
-    case 4: return {latent_prefill_kernel<D, 4>, PrefillLds<D, 4>::bytes};
-    default: return {nullptr, 0};
+    case 1: return prefill_of<D, 1>();
+    case 2: return prefill_of<D, 2>();
+    case 3: return prefill_of<D, 3>();
+    case 4: return prefill_of<D, 4>();
+    default: return {};
   }
 }
 PrefillPick prefill_pick(const LmLatent& a) {
-  if (!(a.scale > 0.f)) return {nullptr, 0};
+  if (!(a.scale > 0.f)) return {};
   switch (a.dp / 32) {
     case 1: return prefill_by_width<1>(a.vp / 32);
     case 2: return prefill_by_width<2>(a.vp / 32);
     case 3: return prefill_by_width<3>(a.vp / 32);
     case 4: return prefill_by_width<4>(a.vp / 32);
-    default: return {nullptr, 0};
+    default: return {};
   }
 }
 
@@ -615,13 +645,14 @@ md_status lm_latent_plain(int dtype, const LmLatent& a, hipStream_t s) {
   return md_launch_status();
 }
 
-bool lm_latent_mfma_takes(const LmLatent& a) { return prefill_pick(a).fn != nullptr; }
+bool lm_latent_mfma_takes(const LmLatent& a) { return prefill_pick(a).fn[0] != nullptr; }
 md_status lm_latent_mfma(const LmLatent& a, hipStream_t s) {
   const PrefillPick k = prefill_pick(a);
-  if (!k.fn) return MD_ERR_UNSUPPORTED;
-  MD_TRY(md_ensure_dynamic_lds((const void*)k.fn, k.lds));
+  if (!k.fn[0]) return MD_ERR_UNSUPPORTED;
   const int n_qblk = (a.r.max_len + 127) / 128, n_bh = a.r.n_seq * a.heads;
-  hipLaunchKernelGGL(k.fn, dim3((n_bh + 7) / 8 * 8 * n_qblk), dim3(256), k.lds, s, a, n_qblk);
+  const int two = a.r.max_ctx > 192 && n_bh * n_qblk <= 256;  // a workgroup per CU, and tiles for both groups
+  MD_TRY(md_ensure_dynamic_lds((const void*)k.fn[two], k.lds[two]));
+  hipLaunchKernelGGL(k.fn[two], dim3((n_bh + 7) / 8 * 8 * n_qblk), dim3(two ? 512 : 256), k.lds[two], s, a, n_qblk);
   return md_launch_status();
 }
 

@@ -295,6 +295,31 @@ def test_retention_prompts(heads, dim, vdim, rot):
                 m.close_sequence(s)
 
 
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 64, 64), (3, 128, 128), (2, 96, 32), (1, 32, 128), (40, 64, 96)], ids=str)
+def test_latent_prompts(heads, dim, vdim):
+    """Prompts at the edges of a tile of 64 keys and of a block of 128 queries, short ones beside long ones (tiles that one group of waves has not got), few heads and more
+    than a workgroup per compute unit; then cut, the second part on the context of the first."""
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    cfg = U.stream_config([(U.latent(heads, dim, vdim, 64), None)], width=64, vocab=60, positions=512)
+    w = U.weights(cfg, 3, 1.5)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=BF16, max_batch=8, max_context=512)
+    for lens in ([193], [2, 64, 65, 128, 256], [257, 1, 129], [450, 63], [320, 321, 450]):
+        ts = [U.tokens(n, 60, n) for n in lens]
+        want = [O.forward(cfg, w, t) for t in ts]
+        for cut in (0, 1, 64, 190):
+            slots = [m.open_sequence() for _ in ts]
+            ks = [min(cut, n - 1) for n in lens]
+            if cut:
+                m.step([(s, t[:k], []) for s, t, k in zip(slots, ts, ks) if k])
+            got = m.step([(s, t[k:], range(n - k)) for s, t, k, n in zip(slots, ts, ks, lens)])
+            e = U.logit_errors(got, torch.cat([x[k:] for x, k in zip(want, ks)]))
+            assert float(e.max()) < 7e-2, (lens, cut, e.sort().values[-4:])  # bf16 through a layer, as in the tests of whole models
+            for s in slots:
+                m.close_sequence(s)
+
+
 @pytest.mark.parametrize("lens", [[1100], [517, 3, 580]], ids=str)
 def test_state_space_prompts_that_fill_the_chip(lens):
     """Rows and columns enough for the convolution's 16 rows per thread (8224 columns), and a token behind each prompt, whose window is what
