@@ -6,17 +6,19 @@
 // mixture and the next norm.  The norm is split: the producer of a row stores  u * w  (bf16) and, per 8 columns, the sum of u^2; the
 // consumer multiplies its finished sums by  1 / sqrt(mean u^2 + eps), which is the same product with the row's factor taken out.
 //
-// Weights go from memory to the matrix operand directly, used once, in whole cache lines (8 rows x 128 bytes per wave and load) with the
+// Weights are used once and come in whole cache lines (8 rows x 128 bytes per wave and load) with the
 // non-temporal policy: loads of 16 rows x 64 bytes, the operand's own shape, fetch half lines that are dropped before the other half is asked
-// for (4.9 TB/s of the 6.9 that a plain read reaches).  Activations are read directly too: with few rows they are a fraction of the weights'
-// bytes.  What a product or a mixer makes for the next one lies in the operand's order, [column / 8][row][8], so that a load takes consecutive memory
+// for (4.9 TB/s of the 6.9 that a plain read reaches).  They go through LDS, a ring of each wave's own without a barrier (see load_weights), but for layers
+// of up to 8 rows and few columns, where what counts is the way from the first load to the sum (2048 wide, 2048 columns 5.2 us, through LDS 5.3; 4096 wide 7.0 and
+// 7.3).  Activations are read directly: with few rows they are a fraction of the weights' bytes.  What a product or a mixer makes for the next one lies in the operand's order, [column / 8][row][8], so that a load takes consecutive memory
 // (rows 4 KB apart meet on few channels: output projection of 40 rows 9.9 us against 7.6).
-// Two register buffers per wave keep two batches of loads in flight.
 //
-// Measured, 2048 wide, 5440 feed-forward, one row (16 rows, 28, 40): 8192 columns 8.5 us (8.4, 9.8, 11.2), 33 MB; gates 10.1 us (10.9, 12.3, 13.8), 44 MB;
-// the two residual products 4.7 and 6.9 us (5.4 and 8.7; 6.3 and 11.0; 7.4 and 13.0), 8 and 22 MB; the head, 51200 columns, 36 us (39, 48, 56),
-// 210 MB.  The tile products at 40 rows: gates 16.2 us, the residual products and their row-wise launches 13.3 us each, 4352 columns in K slices 12.5 us (10.5).
-// About 4 us of every launch are its start, the first loads and the sum over the waves.
+// Measured, 2048 wide, 5440 feed-forward, one stream, one row (16 rows, 28, 40): 8192 columns 8.4 us (7.9, 9.0, 10.5), 33 MB; gates 10.0 us (10.1, 11.2, 12.4), 44 MB;
+// the two residual products 4.4 and 6.7 us (4.9 and 8.2; 5.8 and 10.1; 6.5 and 11.9), 8 and 22 MB; the head, 51200 columns, 34 us (36, 41, 46),
+// 210 MB.  With the weights loaded in the operand's shape: 8.5 us (8.3, 9.8, 11.2), 10.1 (10.8, 12.2, 13.9), 6.6 (8.5, 10.4, 12.3), 36 (39, 48, 57).  The tile products
+// at 40 rows: gates 16.2 us, the residual products and their row-wise launches 13.3 us each, 4352 columns in K slices 12.5 us (9.4).
+// About 4 us of every launch are its start, the first loads and the sum over the waves; at 40 rows the activations, which every workgroup reads, are as many bytes
+// as the weights.
 #include "lm_internal.hpp"
 
 #include <algorithm>
@@ -25,7 +27,45 @@ namespace {
 
 constexpr int EPI_ROWS = 0, EPI_SILU = 1, EPI_RESID = 2;
 
-// W waves, MT 16-row tiles (0: up to 8 rows; others: the residual product), U units of 64 of K per load batch.  A workgroup's columns are NX operands of 8;
+// Weights through LDS: a wave's load of 8 rows x 128 bytes puts piece p of row r at 128 r + 16 (p ^ r) of a kilobyte of its own, from which operands are
+// read without bank conflicts.  A load into registers in the operand's shape has its neighbouring lanes in different rows, which costs the address unit 80 cycles per
+// KB, and 8 lanes to a row 38; into LDS 20.
+__device__ __forceinline__ uint32_t lds_address(char* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)p; }
+__device__ __forceinline__ void load_weights(const bf16_t* w, char* dst) {  // (2: non-temporal)
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)w, (__attribute__((address_space(3))) void*)dst, 16, 0, 2);
+}
+// One operand, or the two of a unit of 16 columns, for each x: in assembly, as the compiler would wait for all loads into LDS that are under way
+template <int NX>
+__device__ __forceinline__ void read_weights(uint32_t p, u32x4 (&w)[NX]) {
+  static_assert(NX <= 2, "operands");
+  if constexpr (NX == 1) asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(w[0]) : "v"(p) : "memory");
+  else asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:1024\n\ts_waitcnt lgkmcnt(0)" : "=&v"(w[0]), "=&v"(w[1]) : "v"(p) : "memory");
+}
+template <int NX>
+__device__ __forceinline__ void read_weights(uint32_t p, u32x4 (&w)[NX][2]) {
+  const uint32_t q = p ^ 64;  // the other 32 of a unit's 64 of K
+  if constexpr (NX == 1) {
+    asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)" : "=&v"(w[0][0]), "=&v"(w[0][1]) : "v"(p), "v"(q) : "memory");
+  } else {
+    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %4 offset:2048\n\tds_read_b128 %3, %5 offset:2048\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(w[0][0]), "=&v"(w[0][1]), "=&v"(w[1][0]), "=&v"(w[1][1]) : "v"(p), "v"(q) : "memory");
+    if constexpr (NX == 3)
+      asm volatile("ds_read_b128 %0, %2 offset:4096\n\tds_read_b128 %1, %3 offset:4096\n\ts_waitcnt lgkmcnt(0)" : "=&v"(w[2][0]), "=&v"(w[2][1]) : "v"(p), "v"(q) : "memory");
+    if constexpr (NX == 4)
+      asm volatile("ds_read_b128 %0, %4 offset:4096\n\tds_read_b128 %1, %5 offset:4096\n\tds_read_b128 %2, %4 offset:6144\n\tds_read_b128 %3, %5 offset:6144\n\ts_waitcnt lgkmcnt(0)"
+                   : "=&v"(w[2][0]), "=&v"(w[2][1]), "=&v"(w[3][0]), "=&v"(w[3][1]) : "v"(p), "v"(q) : "memory");
+  }
+}
+// Waits until a unit's P loads have arrived, with those of `left` more, D at most, under way behind it
+template <int D, int P>
+__device__ __forceinline__ void wait_units(int left) {
+  static_assert(D * P < 64, "vmcnt has six bits");
+  if constexpr (D == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  else if (left >= D) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(D * P) : "memory");
+  else wait_units<D - 1, P>(left);
+}
+
+// W waves, MT 16-row tiles (0: up to 8 rows; others: the residual product), U units of 64 of K under way (in registers: two batches of U).  A workgroup's columns are NX operands of 8;
 // SiLU: 8 gates and the 8 inputs beside them.  A load is 8 rows x 128 bytes of weights, whole cache lines: the operand's upper 8 rows hold the other 32 of a unit's 64
 // of K.  It is multiplied with either half of the activations, and the useful half of either product is kept; up to 8 rows the two halves of
 // K of the activations fit one operand as well.  NX = 1: layers of so few columns that more would not fill the chip evenly.
@@ -38,7 +78,9 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
   constexpr int M16 = DIAG ? 1 : MT, TN = EPI == EPI_SILU ? 8 : 8 * NX;
   constexpr int PA = DIAG ? 1 : 2;  // operands of activations per unit, and accumulators per operand of weights
   auto row_of = [&](int m) { return EPI != EPI_RESID && S == 2 ? a.rows_idx[m] : m; };
+  constexpr bool LDS = NX > 1 || !DIAG;  // weights through LDS
   __shared__ f32x4 red[W][M16][64];
+  __shared__ __attribute__((aligned(128))) char ring[W][LDS ? U * NX * 1024 : 16];
   __shared__ float row_scale[16 * M16];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
@@ -61,7 +103,10 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
   const int kw = 4 * (r >> 3) + g, ka = DIAG ? kw : g;  // 8-column piece of a unit that this lane takes
   const bf16_t* wp[NX];
 #pragma unroll
-  for (int x = 0; x < NX; ++x) wp[x] = a.w + ((int64_t)x * (EPI == EPI_SILU ? a.ff_pad : 8) + n0 + (r & 7)) * a.k + 8 * kw;
+  for (int x = 0; x < NX; ++x) {
+    const int64_t first = (int64_t)x * (EPI == EPI_SILU ? a.ff_pad : 8) + n0;
+    wp[x] = a.w + (LDS ? (first + (lane >> 3)) * a.k + 8 * ((lane & 7) ^ (lane >> 3)) : (first + (r & 7)) * a.k + 8 * kw);
+  }
   const bf16_t* ap[M16];
 #pragma unroll
   for (int i = 0; i < M16; ++i) ap[i] = a.a + (int64_t)row_of(min(16 * i + (DIAG ? r & 7 : r), a.rows - 1)) * a.lda + ka * a.chunk;
@@ -95,54 +140,95 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
 #pragma unroll
     for (int j = 0; j < HEADS; ++j) head_sq[j] = sq_row[min(4 * j + g, a.heads - 1)];
 
-  u32x4 wf[2][U][NX], af[2][U][PA][M16];
-  auto load = [&](auto buf, int u) {  // units u .. u + U - 1; past the end: the last one again, not used
-    constexpr int B = decltype(buf)::value;
+  if constexpr (LDS) {
+    char* mine = ring[wave];
+    const uint32_t rd = lds_address(mine) + (r & 7) * 128 + (kw ^ (r & 7)) * 16;
+    u32x4 af[U][PA][M16];
+    constexpr int P = NX + PA * M16;
+    auto load = [&](int b, int u) {
+      const int k = u * 64, kc = k / 8 * a.chunk;
 #pragma unroll
-    for (int q = 0; q < U; ++q) {
-      const int k = min(u + q, hi - 1) * 64, kc = k / 8 * a.chunk;
-#pragma unroll
-      for (int x = 0; x < NX; ++x) wf[B][q][x] = __builtin_nontemporal_load((const u32x4*)(wp[x] + k));
+      for (int x = 0; x < NX; ++x) load_weights(wp[x] + k, mine + (b * NX + x) * 1024);
 #pragma unroll
       for (int h = 0; h < PA; ++h)
 #pragma unroll
-        for (int i = 0; i < M16; ++i) af[B][q][h][i] = *(const u32x4*)(ap[i] + kc + 4 * h * a.chunk);
+        for (int i = 0; i < M16; ++i) af[b][h][i] = *(const u32x4*)(ap[i] + kc + 4 * h * a.chunk);
+      asm volatile("" ::: "memory");  // (the waits count: a unit's loads stay together)
+    };
+    auto multiply = [&](int b) {
+      u32x4 w[NX];
+      read_weights<NX>(rd + b * NX * 1024, w);
+#pragma unroll
+      for (int x = 0; x < NX; ++x)
+#pragma unroll
+        for (int h = 0; h < PA; ++h)
+#pragma unroll
+          for (int i = 0; i < M16; ++i)
+            acc[x][h][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(md_bf16x8v, w[x]), __builtin_bit_cast(md_bf16x8v, af[b][h][i]), acc[x][h][i], 0, 0, 0);
+    };
+#pragma unroll
+    for (int d = 0; d < U; ++d)
+      if (lo + d < hi) load(d, lo + d);
+    for (int u = lo; u < hi; u += U) {
+#pragma unroll
+      for (int d = 0; d < U; ++d) {
+        const int left = hi - 1 - (u + d);
+        if (left < 0) break;
+        wait_units<U - 1, P>(left);
+        multiply(d);
+        if (left >= U) load(d, u + d + U);
+      }
     }
-  };
-  auto multiply = [&](auto buf, int u) {
-    constexpr int B = decltype(buf)::value;
+  } else {
+    u32x4 wf[2][U][NX], af[2][U][PA][M16];
+    auto load = [&](auto buf, int u) {  // units u .. u + U - 1; past the end: the last one again, not used
+      constexpr int B = decltype(buf)::value;
 #pragma unroll
-    for (int q = 0; q < U; ++q)
-      if (u + q < hi) {
+      for (int q = 0; q < U; ++q) {
+        const int k = min(u + q, hi - 1) * 64, kc = k / 8 * a.chunk;
 #pragma unroll
-        for (int x = 0; x < NX; ++x)
+        for (int x = 0; x < NX; ++x) wf[B][q][x] = __builtin_nontemporal_load((const u32x4*)(wp[x] + k));
 #pragma unroll
-          for (int h = 0; h < PA; ++h)
+        for (int h = 0; h < PA; ++h)
 #pragma unroll
-            for (int i = 0; i < M16; ++i)
-              acc[x][h][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(md_bf16x8v, wf[B][q][x]), __builtin_bit_cast(md_bf16x8v, af[B][q][h][i]),
-                                                                     acc[x][h][i], 0, 0, 0);
+          for (int i = 0; i < M16; ++i) af[B][q][h][i] = *(const u32x4*)(ap[i] + kc + 4 * h * a.chunk);
       }
-  };
-  constexpr auto B0 = std::integral_constant<int, 0>{};
-  constexpr auto B1 = std::integral_constant<int, 1>{};
-  if (lo < hi) {
-    load(B0, lo);
-    for (int u = lo;;) {
-      if (u + U >= hi) {
+    };
+    auto multiply = [&](auto buf, int u) {
+      constexpr int B = decltype(buf)::value;
+#pragma unroll
+      for (int q = 0; q < U; ++q)
+        if (u + q < hi) {
+#pragma unroll
+          for (int x = 0; x < NX; ++x)
+#pragma unroll
+            for (int h = 0; h < PA; ++h)
+#pragma unroll
+              for (int i = 0; i < M16; ++i)
+                acc[x][h][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(md_bf16x8v, wf[B][q][x]), __builtin_bit_cast(md_bf16x8v, af[B][q][h][i]),
+                                                                       acc[x][h][i], 0, 0, 0);
+        }
+    };
+    constexpr auto B0 = std::integral_constant<int, 0>{};
+    constexpr auto B1 = std::integral_constant<int, 1>{};
+    if (lo < hi) {
+      load(B0, lo);
+      for (int u = lo;;) {
+        if (u + U >= hi) {
+          multiply(B0, u);
+          break;
+        }
+        load(B1, u + U);
         multiply(B0, u);
-        break;
-      }
-      load(B1, u + U);
-      multiply(B0, u);
-      u += U;
-      if (u + U >= hi) {
+        u += U;
+        if (u + U >= hi) {
+          multiply(B1, u);
+          break;
+        }
+        load(B0, u + U);
         multiply(B1, u);
-        break;
+        u += U;
       }
-      load(B0, u + U);
-      multiply(B1, u);
-      u += U;
     }
   }
   if (EPI != EPI_RESID) {
@@ -272,17 +358,17 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
 }
 
 // Rows and gates of more than 8 rows, operands of 16 columns (SiLU: an odd NX of operands with 8 gates and the 8 inputs beside them, or pairs of 16 gates
-// and 16 inputs).  Two loads of 8 rows x 128 bytes make an operand of either half of a unit's 64 of K: the lanes of the upper rows take their
-// pieces in the other order, so that a choice between the two loads by lane is all it takes; the second half's columns come out turned by 8
-// and are turned back behind the sums.  Half the matrix instructions and two thirds of the registers of the kernel above, which pay for more columns per
+// and 16 inputs).  Two loads of 8 rows x 128 bytes make the operands of both halves of a unit's 64 of K.
+// Half the matrix instructions of the kernel above, and more columns per
 // workgroup: what bounds it beside the weights is that every workgroup reads all activations (28 rows, gates: 680 workgroups of 8 columns 14.7 us, 227
-// of 24 13.0).  The waves' parts of K are dealt in turn: with the same part first on every CU, loads meet on the same channels (227 of 24: 12.3 us).
-// Batches of D units; more in flight, in deeper rings or all at once, changed nothing.
+// of 24 13.0).  The waves' parts of K are dealt in turn: with the same part first on every CU, loads meet on the same channels (227 of 24: 12.3 us; through LDS
+// 11.2).  D units under way: three and four changed nothing but for NX = 3 (28 rows, 10304 columns 11.0 and 10.8 us).
 template <int MT, int NX, int W, int D, int EPI, int S>
 __global__ __launch_bounds__(64 * W) void step_gemm_tall_kernel(const LmStepGemm a) {
   constexpr int TN = EPI == EPI_SILU ? 8 * NX : 16 * NX;  // columns of the result
   auto row_of = [&](int m) { return S == 2 ? a.rows_idx[m] : m; };
-  __shared__ f32x4 red[W][NX * MT][64];
+  constexpr int STAGE = NX * 2048, RING = D * STAGE > NX * MT * 1024 ? D * STAGE : NX * MT * 1024;
+  __shared__ __attribute__((aligned(128))) char ring[W][RING];
   __shared__ float row_scale[16 * MT];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4, upper = r >> 3;
@@ -309,8 +395,10 @@ __global__ __launch_bounds__(64 * W) void step_gemm_tall_kernel(const LmStepGemm
       const int64_t first = EPI != EPI_SILU ? min(n0 + 16 * x + 8 * h, a.n - 8)
                             : NX & 1      ? (int64_t)h * a.ff_pad + min(n0 + 8 * x, a.n - 8)
                                           : (int64_t)(x & 1) * a.ff_pad + min(n0 + 16 * (x >> 1) + 8 * h, a.n - 8);
-      wp[x][h] = a.w + (first + (r & 7)) * a.k + 8 * (4 * (upper ^ h) + g);
+      wp[x][h] = a.w + (first + (lane >> 3)) * a.k + 8 * ((lane & 7) ^ (lane >> 3));
     }
+  char* mine = ring[wave];
+  const uint32_t rd = lds_address(mine) + upper * 1024 + (r & 7) * 128 + (g ^ (r & 7)) * 16;
   const bf16_t* ap[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) ap[i] = a.a + (int64_t)row_of(min(16 * i + r, a.rows - 1)) * a.lda + g * a.chunk;
@@ -323,42 +411,34 @@ __global__ __launch_bounds__(64 * W) void step_gemm_tall_kernel(const LmStepGemm
 #pragma unroll
       for (int i = 0; i < MT; ++i) acc[x][h][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  u32x4 wf[D][NX][2], af[D][2][MT];
+  u32x4 af[D][2][MT];
+  constexpr int P = 2 * NX + 2 * MT;
   auto load = [&](int b, int u) {
     const int k = u * 64, kc = k / 8 * a.chunk;
 #pragma unroll
     for (int x = 0; x < NX; ++x)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) wf[b][x][h] = __builtin_nontemporal_load((const u32x4*)(wp[x][h] + k));
+      for (int h = 0; h < 2; ++h) load_weights(wp[x][h] + k, mine + b * STAGE + x * 2048 + h * 1024);
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < MT; ++i) af[b][h][i] = *(const u32x4*)(ap[i] + kc + 4 * h * a.chunk);
+    asm volatile("" ::: "memory");  // (the waits count: a unit's loads stay together)
   };
   auto multiply = [&](int b) {
+    u32x4 w[NX][2];
+    read_weights<NX>(rd + b * STAGE, w);
 #pragma unroll
     for (int x = 0; x < NX; ++x)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        u32x4 w;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) w[e] = upper ? wf[b][x][1 - h][e] : wf[b][x][h][e];
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int i = 0; i < MT; ++i)
-          acc[x][h][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(md_bf16x8v, w), __builtin_bit_cast(md_bf16x8v, af[b][h][i]), acc[x][h][i], 0, 0, 0);
-      }
+          acc[x][h][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(md_bf16x8v, w[x][h]), __builtin_bit_cast(md_bf16x8v, af[b][h][i]), acc[x][h][i], 0, 0, 0);
   };
-  const int last = max(hi - 1, 0);
-  auto load_batch = [&](int u) {  // past the end: the last one again, not used
 #pragma unroll
-    for (int d = 0; d < D; ++d) load(d, min(u + d, last));
-  };
-  auto multiply_batch = [&](int u) {
-#pragma unroll
-    for (int d = 0; d < D; ++d)
-      if (u + d < hi) multiply(d);
-  };
-  load_batch(lo);
+  for (int d = 0; d < D; ++d)
+    if (lo + d < hi) load(d, lo + d);
   __builtin_amdgcn_sched_barrier(0);
   float factor[RR];
 #pragma unroll
@@ -370,11 +450,15 @@ __global__ __launch_bounds__(64 * W) void step_gemm_tall_kernel(const LmStepGemm
     factor[i] = (q[0] + q[1]) + (q[2] + q[3]);
   }
   __builtin_amdgcn_sched_barrier(0);
-  multiply_batch(lo);
-  for (int u = lo + D; u < hi; u += D) {
-    load_batch(u);
-    __builtin_amdgcn_sched_barrier(0);
-    multiply_batch(u);
+  for (int u = lo; u < hi; u += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int left = hi - 1 - (u + d);
+      if (left < 0) break;
+      wait_units<D - 1, P>(left);
+      multiply(d);
+      if (left >= D) load(d, u + d + D);
+    }
   }
 #pragma unroll
   for (int i = 0; i < RR; ++i) {
@@ -391,19 +475,15 @@ __global__ __launch_bounds__(64 * W) void step_gemm_tall_kernel(const LmStepGemm
 #pragma unroll
   for (int x = 0; x < NX; ++x)
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      f32x4 v;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = acc[x][0][i][e] + __shfl(acc[x][1][i][e], lane ^ 32, 64);
-      red[part][x * MT + i][lane] = v;
-    }
+    for (int i = 0; i < MT; ++i) ((f32x4*)mine)[(x * MT + i) * 64 + lane] = acc[x][0][i] + acc[x][1][i];  // (its own ring, read to the end)
   __syncthreads();
 
   // a lane holds four columns of one row: m = 16 i + (lane & 15), columns 4 (lane >> 4) .. of the operand's
   auto total = [&](int t, int l) {
-    f32x4 v = red[0][t][l];
+    auto of = [&](int p) { return ((const f32x4*)ring[(p + 8 * W - (int)(blockIdx.x >> 3) % W) % W])[t * 64 + l]; };  // part p's wave
+    f32x4 v = of(0);
 #pragma unroll
-    for (int w = 1; w < W; ++w) v += red[w][t][l];
+    for (int w = 1; w < W; ++w) v += of(w);
     return v;
   };
   if (EPI == EPI_ROWS) {
@@ -434,17 +514,18 @@ md_status launch(const LmStepGemm& a, hipStream_t s) {
   hipLaunchKernelGGL((step_gemm_kernel<MT, NX, W, U, EPI, S>), dim3(a.n / (EPI == EPI_SILU ? 8 : 8 * NX)), dim3(64 * W), 0, s, a);
   return md_launch_status();
 }
-template <int NX, int W, int EPI, int S>
-md_status tall(const LmStepGemm& a, hipStream_t s) {
+template <int MT, int NX, int W, int EPI, int S>
+md_status tall_rows(const LmStepGemm& a, hipStream_t s) {
   constexpr int TN = EPI == EPI_SILU ? 8 * NX : 16 * NX;
-  const dim3 grid((a.n + TN - 1) / TN), block(64 * W);
-  if (a.rows <= 16) hipLaunchKernelGGL((step_gemm_tall_kernel<1, NX, W, 2, EPI, S>), grid, block, 0, s, a);
-  else if (a.rows <= 32) hipLaunchKernelGGL((step_gemm_tall_kernel<2, NX, W, 2, EPI, S>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((step_gemm_tall_kernel<3, NX, W, 2, EPI, S>), grid, block, 0, s, a);
+  hipLaunchKernelGGL((step_gemm_tall_kernel<MT, NX, W, NX == 3 ? 3 : 2, EPI, S>), dim3((a.n + TN - 1) / TN), dim3(64 * W), 0, s, a);
   return md_launch_status();
 }
-// As many operands per workgroup as leave the fullest of the 256 CUs with the fewest columns, the larger number where that is the same (40 rows, gates
-// of 5440: 1, 2, 3 operands 18.7, 18.2, 13.8 us; 8192 columns: 15.5, 11.2, 13.0; 4352: 14.2, 10.5, 12.5)
+template <int NX, int W, int EPI, int S>
+md_status tall(const LmStepGemm& a, hipStream_t s) {
+  return a.rows <= 16 ? tall_rows<1, NX, W, EPI, S>(a, s) : a.rows <= 32 ? tall_rows<2, NX, W, EPI, S>(a, s) : tall_rows<3, NX, W, EPI, S>(a, s);
+}
+// As many operands per workgroup as leave the fullest of the 256 CUs with the fewest columns, the larger number where that is the same (40 rows,
+// 10304 columns: 1, 2, 3 operands 21.5, 17.8, 12.0 us; 8192: 15.4, 10.4, 11.5; 4352: 14.2, 9.5, 10.8)
 template <int EPI, int S>
 md_status tall_by_columns(const LmStepGemm& a, hipStream_t s) {
   auto most = [&](int nx) {
@@ -456,31 +537,33 @@ md_status tall_by_columns(const LmStepGemm& a, hipStream_t s) {
 }
 
 // Columns and waves of a workgroup.  Up to 8 rows, where a unit's activations are one load: 8 columns where that evens out few workgroups (6144
-// columns, 8 rows: 7.5 us against 8.0; 8192: 9.5 against 8.7), eight waves to share K otherwise.  More than four workgroups of 16 columns per CU: fewer
-// waves (51200 columns, 1 row: two waves 36 us, eight 39; 28 / 40 rows: 32 columns to four waves 48 / 56 us, to eight 59 / 69).
+// columns, 8 rows: 7.4 us against 7.9; 8192: 9.4 against 8.5), eight waves to share K otherwise.  More than four workgroups of 16 columns per CU: fewer
+// waves (51200 columns, 1 row: two waves 34.6 us, eight 37.0), and from 17 rows on more columns, whose activations are read less often (16 / 28 / 40 rows: 32 columns to
+// four waves 36.6 / 43 / 50 us, 64 columns 38.4 / 41 / 46, 64 to eight waves 43 / 47 / 51).
 template <int S>
 md_status rows(const LmStepGemm& a, hipStream_t s) {
   auto most = [&](int tn) { return (a.n / tn + 255) / 256 * tn; };  // columns that the fullest of the 256 CUs gets
   const bool many = a.n > 256 * 64;
-  if (a.rows > 8) return many ? tall<2, 4, EPI_ROWS, S>(a, s) : tall_by_columns<EPI_ROWS, S>(a, s);
-  if (many) return launch<0, 2, 2, 1, EPI_ROWS, S>(a, s);
-  return a.n <= 256 * 32 && most(8) < most(16) ? launch<0, 1, 4, 2, EPI_ROWS, S>(a, s) : launch<0, 2, 8, 1, EPI_ROWS, S>(a, s);
+  if (a.rows > 8) return !many ? tall_by_columns<EPI_ROWS, S>(a, s) : a.rows <= 16 ? tall<2, 4, EPI_ROWS, S>(a, s) : tall<4, 4, EPI_ROWS, S>(a, s);
+  if (many) return launch<0, 2, 2, 2, EPI_ROWS, S>(a, s);
+  return a.n <= 256 * 32 && most(8) < most(16) ? launch<0, 1, 4, 2, EPI_ROWS, S>(a, s) : launch<0, 2, 8, 2, EPI_ROWS, S>(a, s);
 }
 
-// Waves that share K, up to 8 rows.  Up to one workgroup of 8 columns per CU the chain of loads bounds it: eight (2048 wide, 256 / 2048 columns, 1 row: 5.4 /
-// 6.1 us, four 6.3 / 6.8, two 8.0 / 8.5; 4096 wide 7.8 / 8.9, two 13.6 / 15.3).  More: four (4096 wide, 10944 columns: 32 us, two 44, eight 34; 1024 wide, 5440
-// columns: 6.6, 6.8, 6.7), but two where the workgroups are many and a wave's half of K is of 8 to 16 units (2048 wide, 5440 / 8192 columns: 10.1 / 13.3
-// us, four 10.8 / 14.3; 2816 columns: 9.0 and 7.7).
+// Waves that share K, up to 8 rows.  Up to one workgroup of 8 columns per CU the chain of loads bounds it: eight (2048 wide, 256 / 2048 columns, 1 row: 5.2 /
+// 6.0 us, four 6.2 / 6.8, two 8.2 / 8.5; 4096 wide 6.9 / 8.7, two 13.9 / 15.6).  More: four (4096 wide, 10944 columns: 31 us, two 40, eight 32; 1024 wide, 5440
+// columns: 6.3, 6.9, 6.5), but two where the workgroups are many and a wave's half of K is of 8 to 16 units (2048 wide, 5440 / 8192 columns: 10.2 / 12.7
+// us, four 10.1 / 13.6; 2816 columns: 9.1 and 7.3).  Four units under way: nothing but for two waves (5440 columns 10.1, 8192 13.0).
 md_status gates(const LmStepGemm& a, hipStream_t s) {
-  if (a.n <= 256 * 8) return launch<0, 2, 8, 1, EPI_SILU, 1>(a, s);
-  return a.n > 2 * 256 * 8 && a.k > 1024 && a.k <= 2048 ? launch<0, 2, 2, 1, EPI_SILU, 1>(a, s) : launch<0, 2, 4, 1, EPI_SILU, 1>(a, s);
+  if (a.n <= 256 * 8) return launch<0, 2, 8, 2, EPI_SILU, 1>(a, s);
+  return a.n > 2 * 256 * 8 && a.k > 1024 && a.k <= 2048 ? launch<0, 2, 2, 2, EPI_SILU, 1>(a, s) : launch<0, 2, 4, 2, EPI_SILU, 1>(a, s);
 }
 
 // Up to 8 rows four units per batch where K is long (5440: 6.8 us against 7.7; 2048: 4.4 either way)
 template <int S>
 md_status resid(const LmStepGemm& a, hipStream_t s) {
+  // (more rows: two units under way, three row tiles have the registers for one: 5440 wide, 40 rows 11.9 us, two 12.2, three 12.1; 16 rows 9.6 and 8.2)
   if (a.rows <= 8) return a.k > 4096 ? launch<0, 1, 8, 4, EPI_RESID, S>(a, s) : launch<0, 1, 8, 2, EPI_RESID, S>(a, s);
-  return a.rows <= 16 ? launch<1, 1, 8, 2, EPI_RESID, S>(a, s) : a.rows <= 32 ? launch<2, 1, 8, 1, EPI_RESID, S>(a, s) : launch<3, 1, 8, 1, EPI_RESID, S>(a, s);
+  return a.rows <= 16 ? launch<1, 1, 8, 2, EPI_RESID, S>(a, s) : a.rows <= 32 ? launch<2, 1, 8, 2, EPI_RESID, S>(a, s) : launch<3, 1, 8, 1, EPI_RESID, S>(a, s);
 }
 
 static_assert(LM_STEP_ROWS <= 48, "three row tiles");

@@ -148,6 +148,23 @@ def test_columns_of_a_workgroup(cfg):
     assert float(U.logit_errors(got[30:], O.forward(cfg, w, t)[[5, 0, 6]]).max()) < 7e-2
 
 
+@pytest.mark.parametrize("width,vdim,ff,vocab", [(64, 32, 64, 16500), (1000, 96, 330, 120), (1560, 32, 3080, 120), (2100, 130, 2080, 16500)], ids=str)
+def test_weights_through_lds(width, vdim, ff, vocab):
+    """Waves with no unit of K, with one, with as many as are under way and one more or less, in workgroups of one operand of columns to four, and gates, and residual
+    products, at the edges of the row tiles: the ring of each wave comes round, ends early and is not used at all."""
+    cfg = U.stream_config([(U.latent(4, 32, vdim, 64), U.dense(ff))], width=width, vocab=vocab, streams=2, positions=8)
+    m, w = build(cfg), U.weights(cfg, 3, 1.5)
+    ts = [U.tokens(2, vocab, i) for i in range(48)]
+    want = torch.stack([O.forward(cfg, w, t) for t in ts])
+    for n in (1, 8, 9, 16, 17, 32, 33, 48):
+        slots = [m.open_sequence() for _ in range(n)]
+        for k in range(2):
+            got = m.step([(s, [t[k]], [0]) for s, t in zip(slots, ts)])
+            assert float(U.logit_errors(got, want[:n, k]).max()) < 7e-2, (n, k)
+        for s in slots:
+            m.close_sequence(s)
+
+
 @pytest.mark.parametrize("rows", [3, 40, 200])
 @pytest.mark.parametrize("which", ["in_proj", "out_proj", "gate_up", "down", "head"])
 def test_misaligned_weights_are_refused(rows, which):
