@@ -23,7 +23,7 @@ SOURCES = ["gemm_bf16.hip", "gemm_w4.hip", "gemm_mid.hip", "gemm_fp8w.hip", "gem
 LM_LIB_PATH = os.path.join(HERE, "libmoondream_lm.so")
 LM_SOURCES = ["gemm_bf16.hip", "gemm_w4.hip", "gemm_mid.hip", "elementwise.hip", "sampling_region.hip", "abi.hip", "lm_ops.hip", "gemm_step.hip", "gemm_f32.hip", "attention_talk.hip",
               "retention.hip", "attention_latent.hip", "state_space.hip", "experts.hip", "gemm_experts.hip", "streams.hip", "lm_api.hip"]
-HEADERS = ["md_common.hpp", "gemm_internal.hpp", "stage_common.hpp", "lm_internal.hpp"]
+HEADERS = ["md_common.hpp", "gemm_internal.hpp", "stage_common.hpp", "lm_internal.hpp", "step_weights.hpp"]
 
 MD_OK = 0
 ABI_VERSION = 5  # include/moondream_hip.h MD_ABI_VERSION

@@ -5,26 +5,28 @@
 // the expert's rows itself, by ballots over the step's choices, so the choices need no sorting and no launch for it; results stay in the
 // order of the choices.
 //
-// A weight load is 8 rows x 128 bytes, whole cache lines, non-temporal, and goes to the matrix operand directly: the operand's upper 8 rows
-// then hold the other 32 of a unit's 64 of K.  It is multiplied with either half of the activations and the useful half of either
+// A weight load is 8 rows x 128 bytes, whole cache lines, non-temporal, through LDS: the operand's upper 8 rows
+// hold the other 32 of a unit's 64 of K.  It is multiplied with either half of the activations and the useful half of either
 // product kept; up to 8 rows of activations, the two halves of K fit one operand as well.  16 rows x 64 bytes per load, the operand's
 // own shape, fetches half lines: 4.95 TB/s with the non-temporal policy, which drops a line before its other half is asked for, 5.66 without,
 // against 6.4 (a plain read of the same bytes: 6.9).  Activations of rows that do not exist are not fetched (a buffer load out of range gives zeros).
 //
 // Measured, 32 experts, 4 per row, 2 x 1360 and 1360 columns of 2048, against tiles of 64 rows and the launch that sorts the choices (4.6 us):
-// 23 rows 77 -> 55 us (358 MB) and 42 -> 30 us (179 MB).  Two waves with one unit each on its way besides the one multiplied: four waves 58 and 36 us,
-// two units 54 and 33, one wave 68 and 30.
-#include "lm_internal.hpp"
+// 23 rows 77 -> 53.7 us (358 MB) and 42 -> 29.4 us (179 MB), 6.7 and 6.1 TB/s; weights loaded in the operand's shape, two units on their way, 54.7 and 30.4.  Three units
+// on their way: one 57.0 and 31.3, two 53.5 and 30.1, four 53.8 and 30.3.  Twice the columns per workgroup: 56.8 and 30.2.
+#include "step_weights.hpp"
 
 namespace {
 
 constexpr int EPI_ROWS = 0, EPI_SILU = 1;
 constexpr int W = 2;  // waves
+constexpr int D = 3;  // units of 64 of K under way
 
 // A workgroup's 16 columns, two operands of 8: columns 0 .. 7 and 8 .. 15; SiLU: 8 gates and the 8 inputs beside them
 template <int EPI>
 __global__ __launch_bounds__(64 * W) void expert_gemm_kernel(const LmExpertGemm a) {
   __shared__ f32x4 red[W][2][64];
+  __shared__ __attribute__((aligned(128))) char ring[W][D * 2048];
   __shared__ uint16_t lists[W][LM_EXPERT_CHOICES];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
@@ -47,8 +49,10 @@ __global__ __launch_bounds__(64 * W) void expert_gemm_kernel(const LmExpertGemm 
   if (count == 0 || (by_choice && list[0] != blockIdx.y)) return;  // (the same in every wave) nobody's, or an earlier choice's
 
   const int kw = 4 * (r >> 3) + g;  // 8-column piece of a unit, 64 of K, that this lane takes
-  const bf16_t* w0 = a.w + expert * a.expert_stride + (int64_t)(n0 + (r & 7)) * a.k + 8 * kw;
+  const bf16_t* w0 = a.w + expert * a.expert_stride + (int64_t)(n0 + (lane >> 3)) * a.k + 8 * ((lane & 7) ^ (lane >> 3));
   const bf16_t* w1 = w0 + (int64_t)(EPI == EPI_SILU ? a.ff_pad : 8) * a.k;
+  char* mine = ring[wave];
+  const uint32_t rd = lds_address(mine) + (r & 7) * 128 + (kw ^ (r & 7)) * 16;
   const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc((void*)a.a, 0, (int)(a.a_rows * a.lda * 2), 0x00020000);
   const int units = a.k >> 6, lo = units * wave / W, hi = units * (wave + 1) / W;
 
@@ -63,39 +67,34 @@ __global__ __launch_bounds__(64 * W) void expert_gemm_kernel(const LmExpertGemm 
       for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int h = 0; h < PA; ++h) acc[i][h] = f32x4{0.f, 0.f, 0.f, 0.f};
-      u32x4 wf[2][2], af[2][PA];
-      auto load = [&](auto buf, int u) {
-        constexpr int B = decltype(buf)::value;
-        wf[B][0] = __builtin_nontemporal_load((const u32x4*)(w0 + u * 64));
-        wf[B][1] = __builtin_nontemporal_load((const u32x4*)(w1 + u * 64));
+      u32x4 af[D][PA];
+      auto load = [&](int b, int u) {
+        load_weights(w0 + u * 64, mine + b * 2048);
+        load_weights(w1 + u * 64, mine + b * 2048 + 1024);
 #pragma unroll
-        for (int h = 0; h < PA; ++h) af[B][h] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rows, at + 128u * u + 64u * h, 0, 0));
+        for (int h = 0; h < PA; ++h) af[b][h] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rows, at + 128u * u + 64u * h, 0, 0));
+        asm volatile("" ::: "memory");  // (the waits count: a unit's loads stay together)
       };
-      auto multiply = [&](auto buf) {
-        constexpr int B = decltype(buf)::value;
+      auto multiply = [&](int b) {
+        u32x4 w[2];
+        read_weights<2>(rd + b * 2048, w);
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
           for (int h = 0; h < PA; ++h)
-            acc[i][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(md_bf16x8v, wf[B][i]), __builtin_bit_cast(md_bf16x8v, af[B][h]), acc[i][h], 0, 0, 0);
+            acc[i][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(md_bf16x8v, w[i]), __builtin_bit_cast(md_bf16x8v, af[b][h]), acc[i][h], 0, 0, 0);
       };
-      constexpr auto B0 = std::integral_constant<int, 0>{};
-      constexpr auto B1 = std::integral_constant<int, 1>{};
-      if (lo < hi) {
-        load(B0, lo);
-        for (int u = lo;; u += 2) {
-          if (u + 1 >= hi) {
-            multiply(B0);
-            break;
-          }
-          load(B1, u + 1);
-          multiply(B0);
-          if (u + 2 >= hi) {
-            multiply(B1);
-            break;
-          }
-          load(B0, u + 2);
-          multiply(B1);
+#pragma unroll
+      for (int d = 0; d < D; ++d)
+        if (lo + d < hi) load(d, lo + d);
+      for (int u = lo; u < hi; u += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+          const int left = hi - 1 - (u + d);
+          if (left < 0) break;
+          wait_units<D - 1, 2 + PA>(left);
+          multiply(d);
+          if (left >= D) load(d, u + d + D);
         }
       }
       if (r0 > 0) __syncthreads();  // (the sums before these were read)

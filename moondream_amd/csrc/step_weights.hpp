@@ -1,0 +1,45 @@
+// How the products of few rows read their weights (gemm_step.hip, gemm_experts.hip).
+#pragma once
+#include "lm_internal.hpp"
+
+namespace {
+
+// Weights through LDS: a wave's load of 8 rows x 128 bytes puts piece p of row r at 128 r + 16 (p ^ r) of a kilobyte of its own, from which operands are
+// read without bank conflicts.  A load into registers in the operand's shape has its neighbouring lanes in different rows, which costs the address unit 80 cycles per
+// KB, and 8 lanes to a row 38; into LDS 20.
+__device__ __forceinline__ uint32_t lds_address(char* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)p; }
+__device__ __forceinline__ void load_weights(const bf16_t* w, char* dst) {  // (2: non-temporal)
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)w, (__attribute__((address_space(3))) void*)dst, 16, 0, 2);
+}
+// One operand, or the two of a unit of 16 columns, for each x: in assembly, as the compiler would wait for all loads into LDS that are under way
+template <int NX>
+__device__ __forceinline__ void read_weights(uint32_t p, u32x4 (&w)[NX]) {
+  static_assert(NX == 1 || NX == 2, "operands");
+  if constexpr (NX == 1) asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(w[0]) : "v"(p) : "memory");
+  else asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:1024\n\ts_waitcnt lgkmcnt(0)" : "=&v"(w[0]), "=&v"(w[1]) : "v"(p) : "memory");
+}
+template <int NX>
+__device__ __forceinline__ void read_weights(uint32_t p, u32x4 (&w)[NX][2]) {
+  const uint32_t q = p ^ 64;  // the other 32 of a unit's 64 of K
+  if constexpr (NX == 1) {
+    asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)" : "=&v"(w[0][0]), "=&v"(w[0][1]) : "v"(p), "v"(q) : "memory");
+  } else {
+    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %4 offset:2048\n\tds_read_b128 %3, %5 offset:2048\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(w[0][0]), "=&v"(w[0][1]), "=&v"(w[1][0]), "=&v"(w[1][1]) : "v"(p), "v"(q) : "memory");
+    if constexpr (NX == 3)
+      asm volatile("ds_read_b128 %0, %2 offset:4096\n\tds_read_b128 %1, %3 offset:4096\n\ts_waitcnt lgkmcnt(0)" : "=&v"(w[2][0]), "=&v"(w[2][1]) : "v"(p), "v"(q) : "memory");
+    if constexpr (NX == 4)
+      asm volatile("ds_read_b128 %0, %4 offset:4096\n\tds_read_b128 %1, %5 offset:4096\n\tds_read_b128 %2, %4 offset:6144\n\tds_read_b128 %3, %5 offset:6144\n\ts_waitcnt lgkmcnt(0)"
+                   : "=&v"(w[2][0]), "=&v"(w[2][1]), "=&v"(w[3][0]), "=&v"(w[3][1]) : "v"(p), "v"(q) : "memory");
+  }
+}
+// Waits until a unit's P loads have arrived, with those of `left` more, D at most, under way behind it
+template <int D, int P>
+__device__ __forceinline__ void wait_units(int left) {
+  static_assert(D * P < 64, "vmcnt has six bits");
+  if constexpr (D == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  else if (left >= D) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(D * P) : "memory");
+  else wait_units<D - 1, P>(left);
+}
+
+}  // namespace

@@ -188,6 +188,16 @@ def test_experts(dtype, shape):
         assert float(e.sort().values[-9 if dtype == BF16 else -1]) < TOL[dtype]
 
 
+@pytest.mark.parametrize("width,ff", [(64, 64), (192, 320), (448, 384), (640, 512)], ids=str)
+def test_weights_of_experts_through_lds(width, ff):
+    """Waves with no unit of 64 of K, with as many as are under way and one more or less, for up to eight rows of an expert and for several passes of 16."""
+    cfg, w = _expert_model(4, 2, ff, width=width)
+    t = U.tokens(60, 64, 6)
+    want, m = O.forward(cfg, w, t), load(cfg, w, BF16)
+    for cuts in ([20] * 3, [1] * 10 + [5] * 10):
+        assert float(U.logit_errors(run(m, t, cuts), want).sort().values[-2]) < TOL[BF16]  # (a row whose choice is close may choose otherwise in bf16)
+
+
 @dtypes
 def test_one_expert_takes_every_row(dtype):
     """The other experts have no rows at all."""
