@@ -514,6 +514,8 @@ RetPick ret_run_pick(const LmRet& a) {
 // bounds it, and all of a head's rows are under way before the first use (ALL).  8 sequences, 16 heads of 128: 17.1 us with a row loaded after the other,
 // 9.6 this way; 1 sequence, 32 heads of 64: 6.7 and 5.7; 64 of 32 x 64: 16.7 and 14.9.  Many: the state's bytes, and more workgroups per CU hide more than
 // registers full of rows (128 sequences, 8 heads of 256: 122 us with all, 104 with a row after the other; 16 of 192: 141 and 114).
+// The state is read and written once a step, past the caches (non-temporal): 32 heads of 64, 16 / 32 / 64 sequences 6.8 / 9.5 / 16.3 -> 6.2 / 8.0 / 14.1 us, 16 of 128
+// 9.8 / 17.4 / 28.6 -> 8.9 / 13.4 / 24.2, 96 23.1 -> 22.1 and 40.2 -> 39.8; one sequence 5.1 and 5.2.
 template <int R, int E, bool ALL>
 __global__ __launch_bounds__(256) void ret_decode_kernel(const LmRet a) {
   __shared__ __attribute__((aligned(16))) float qs[256], ks[256], os[256];
@@ -531,7 +533,7 @@ __global__ __launch_bounds__(256) void ret_decode_kernel(const LmRet a) {
 #pragma unroll
       for (int j = 0; j < E; ++j) {
         S[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (pos > 0 && e < vp && 4 * l + 64 * j < dp) S[i][j] = *(const f32x4*)(st + (int64_t)e * dp + 4 * l + 64 * j);
+        if (pos > 0 && e < vp && 4 * l + 64 * j < dp) S[i][j] = __builtin_nontemporal_load((const f32x4*)(st + (int64_t)e * dp + 4 * l + 64 * j));
       }
       v[i] = bf2f(p[a.col_v + h * vp + min(e, vp - 1)]);
     }
@@ -557,7 +559,7 @@ __global__ __launch_bounds__(256) void ret_decode_kernel(const LmRet a) {
         if (d >= dp) continue;
         const f32x4 k = *(const f32x4*)(ks + d), qv = *(const f32x4*)(qs + d);
         const f32x4 s = decay * S[i][j] + k * v[i];
-        *(f32x4*)(st + (int64_t)e * dp + d) = s;
+        __builtin_nontemporal_store(s, (f32x4*)(st + (int64_t)e * dp + d));
         o += s[0] * qv[0] + s[1] * qv[1] + s[2] * qv[2] + s[3] * qv[3];
       }
 #pragma unroll

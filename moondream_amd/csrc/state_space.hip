@@ -580,6 +580,9 @@ ChunkPick chunk_pick(const LmSsm& a) {
 }
 
 // grid (heads, sequences).  Sixteen lanes per state row, sixteen rows at a time; the state is requested before anything else.
+// The state's bytes bound it from about eight sequences on.  It is read and written once a step, past the caches (non-temporal, both): 40 sequences, 32 heads of 64 x 64,
+// 12.2 -> 9.9 us (42 MB); 23, 64 of 64 x 128, 25.0 -> 20.2 us (96 MB, 4.8 TB/s); 8 of these 10.8 -> 8.9; one 6.3 and 6.4; 32 of 64 x 64, one 5.7 and 5.8.
+// Either alone: stores 12.1 and 24.2 us, loads 11.8 and 23.0.
 // C: vp / 32, E: passes of 64 state columns.  a.sumsq: rows are left before their norm, times its weights, with every head's sum of squares: the
 // product behind takes the rows' factors, and there is no launch of one workgroup per row (4.8 us) between them.
 template <int C, int E>
@@ -595,7 +598,7 @@ __global__ __launch_bounds__(256) void ssm_decode_kernel(const LmSsm a) {
 #pragma unroll
     for (int k = 0; k < E; ++k) {
       const int d = 64 * k + 4 * l;
-      S[i][k] = *(const f32x4*)(st + (int64_t)((tid >> 4) + 16 * i) * dp + min(d, dp - 4));
+      S[i][k] = __builtin_nontemporal_load((const f32x4*)(st + (int64_t)((tid >> 4) + 16 * i) * dp + min(d, dp - 4)));
     }
   const bf16_t* p = (const bf16_t*)a.proj + (int64_t)row * a.ldp;
   const int mine = h * vp + min(tid, vp - 1);  // the output that this thread writes in the end
@@ -648,7 +651,7 @@ __global__ __launch_bounds__(256) void ssm_decode_kernel(const LmSsm a) {
       if (d < dp) {
         const f32x4 b = *(const f32x4*)(us + vp + d), c = *(const f32x4*)(us + vp + dp + d);
         const f32x4 s = keep * S[i][k] + b * in;
-        *(f32x4*)(st + (int64_t)e * dp + d) = s;
+        __builtin_nontemporal_store(s, (f32x4*)(st + (int64_t)e * dp + d));
         o += s[0] * c[0] + s[1] * c[1] + s[2] * c[2] + s[3] * c[3];
       }
     }
