@@ -16,6 +16,9 @@
 // half of every 128-wide K step (two 1 KiB weight loads per step).  Two activation paths, chosen by the row count:
 //   RESIDENT (m <= 8, the few-sequence decode step): the whole activation slice [m][K slice] is put into LDS once; the
 //     loop is then a pure weight stream -- no barrier, 8 steps (16 KiB) of weight loads in flight per wave.
+//     Each weight is used once a step: non-temporal loads (1 / 5 / 8 rows, launches in a graph, e4m3: 14336 columns of K 2048 9.6 / 10.0 / 10.3 -> 8.6 / 9.2 /
+//     9.2 us, 51200 columns 25.1 / 25.8 / 26.0 -> 23.5 / 24.2 / 24.6, the pair 8.7 / 9.5 / 9.4 -> 8.5 / 8.9 / 9.0; 4-bit 13.5 -> 12.9, 30.1 -> 29.5, 11.4 -> 10.9).
+//     The ring keeps plain ones (2048 columns of K 2048, 16 / 64 rows 8.1 / 11.2 us, non-temporal 9.0 / 12.4).
 //   RING (m <= 64): the bf16 activation chunk [rows][128] of every step goes through a 3-stage LDS ring (row stride
 //     272 B: conflict-free ds_read_b128), one barrier per step; activation and weight loads of a step are issued
 //     together, 4 steps ahead (loads return in order: a wait for an activation chunk must not imply a wait for younger
@@ -141,11 +144,12 @@ __device__ __forceinline__ void fp8w_body(const Fp8K& p, char* smem) {
   const u32x4 zero4 = {0u, 0u, 0u, 0u};
   auto load_w = [&](int i, u32x4 (&dst)[2]) {
     const int ic = min(i, nsteps - 1);
+    auto weights = [&](int at) { return RESIDENT ? __builtin_nontemporal_load(wp + at) : wp[at]; };
     if constexpr (FMT == 0) {
-      dst[0] = wp[(4 * ic) * 64];
-      dst[1] = wp[(4 * ic + 1) * 64];
+      dst[0] = weights((4 * ic) * 64);
+      dst[1] = weights((4 * ic + 1) * 64);
     } else {
-      dst[0] = wp[(2 * ic) * 64];
+      dst[0] = weights((2 * ic) * 64);
       const u32x2 qp = qpp[(int64_t)ic * p.n_pad];  // a dead step's slot is replaced by zeros below: scale 0 makes its weights 0
       u32x4 t4 = {0u, 0u, 0u, 0u};
       t4.x = qp.x;  // scale
