@@ -130,7 +130,7 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
     } else {
       qf = std::max(qf, (size_t)l.heads * l.dim_pad);
       of = std::max(of, (size_t)l.heads * l.vdim_pad);
-      rs = std::max(rs, (size_t)lm_ret_most_segments(n_seq, l.heads, l.dim_pad, l.vdim_pad, max_len) * l.heads * l.dim_pad * l.vdim_pad);
+      if (m->dtype == MD_DTYPE_BF16) rs = std::max(rs, (size_t)lm_ret_most_states(n_seq, l.heads, l.dim_pad, l.vdim_pad, max_len) * l.heads * l.dim_pad * l.vdim_pad);
     }
   }
   splitk(m->head, n_logits);

@@ -146,7 +146,7 @@ struct LmRet {
   int out_chunk;
   float *qf, *kf;  // plain kernels: rotated q and k, [n_rows][heads * dp]
   float* of;       // plain kernels: unnormed outputs, [n_rows][heads * vp]
-  float* seg;      // matrix-core prefill in more segments than one: what each adds to the state, then the state each starts from
+  float* seg;      // matrix-core prefill in more segments than one: increments of chunks, states that segments start from (retention.hip)
   int n_seg, seg_chunks;  // segments per sequence, their length in chunks
 };
 
@@ -366,7 +366,7 @@ md_status lm_attn_decode(const LmAttn& a, hipStream_t s);               // bf16 
 md_status lm_ret_plain(int dtype, const LmRet& a, hipStream_t s);
 constexpr int LM_RET_CHUNK = 64;
 int lm_ret_segments(int n_seq, int heads, int dp, int vp, int max_len, int* chunks);  // as lm_ssm_segments
-int lm_ret_most_segments(int n_seq, int heads, int dp, int vp, int max_len);
+int lm_ret_most_states(int n_seq, int heads, int dp, int vp, int max_len);  // that any step of up to so many sequences and tokens keeps in memory
 bool lm_ret_mfma_takes(const LmRet& a);
 md_status lm_ret_mfma(const LmRet& a, hipStream_t s);                   // bf16 prefill, chunked on the matrix cores
 bool lm_ret_decode_takes(const LmRet& a);

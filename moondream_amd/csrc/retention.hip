@@ -7,7 +7,7 @@
 // bf16 prefill on the matrix cores, in chunks of 64 tokens, the chunks of a segment one after the other with the state in registers:
 //   ret_run_kernel        per (sequence, head, segment): decay^(t+1) S^T q_t + sum_{s<=t} decay^(t-s) (q_t . k_s) v_s, output norm, gate, and the chunk's
 //                         sum_t decay^(n-1-t) v_t k_t^T onto the state
-//   INC, ret_segments_kernel  where more segments than one fill the chip: what each adds to the state, and the states they start from
+//   ret_increment_kernel, ret_segments_kernel  where more segments than one fill the chip: what the chunks add to the state, and the states that segments start from
 // Everything behind the projections counts as fp32: rotated q and k, decay-weighted products and states enter a product as the sum of
 // two bf16 (16 mantissa bits; hi hi + hi lo + lo hi), the values are the projection's own bf16.
 //
@@ -170,6 +170,17 @@ __device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x
 
 constexpr int RC = LM_RET_CHUNK;
 
+// chunks of a sequence before its last segment
+__device__ __forceinline__ int ret_chunks_ahead(const LmRet& a, int len) {
+  const int per = a.seg_chunks * RC;
+  return ((len + per - 1) / per - 1) * a.seg_chunks;
+}
+// Memory of a step in more segments than one, per sequence: the state that it starts from, then what each chunk before the last segment adds to it.  The
+// last chunk's place before a segment becomes the state which that segment starts from: place k * seg_chunks of segment k.
+__device__ __forceinline__ float* ret_seg_state(const LmRet& a, int seq, int place, int h) {
+  return a.seg + (((int64_t)seq * ((a.n_seg - 1) * a.seg_chunks + 1) + place) * a.heads + h) * a.vp * a.dp;
+}
+
 // Two pieces of eight coordinates of a head's row: unit j < rot_dims / 16 the pieces j and j + rot_dims / 16, which turn into each other, with one load
 // of the angles; units behind them two pieces that do not turn.  rot_dims not a multiple of 16: pieces 2 j and 2 j + 1, element by element.
 struct RetUnit {
@@ -182,6 +193,16 @@ __device__ __forceinline__ RetUnit ret_unit(int j, int rot_dims) {
   const bool turns = whole && j < hp;
   return RetUnit{{8 * (turns ? j : 2 * j), 8 * (turns ? j + hp : 2 * j + 1)}, turns, whole};
 }
+// the angles of a unit of row t
+__device__ __forceinline__ void ret_angles(const RetUnit& u, const float* angles, int t, int rot_dims, f32x4 (&cs)[4]) {
+  if (rot_dims <= 0) return;
+  const uint32_t from = (uint32_t)t * (uint32_t)rot_dims + (u.turns ? 2 * u.d[0] : 0);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) cs[k] = u.whole ? *(const f32x4*)(angles + (from + 4 * k)) : f32x4{0.f, 0.f, 0.f, 0.f};
+}
+// own * c + other * s.  Which of the two products is rounded by itself is written out, so that a prompt's bits do not hang on the compiler's choice: the first, but
+// for the first of eight coordinates, as recorded results have it.
+__device__ __forceinline__ float turned(int e, float own, float other, float c, float s) { return e == 0 ? fmaf(own, c, other * s) : fmaf(other, s, own * c); }
 // row: the head's row in memory (only read where pieces turn element by element).  ALL: all of a row turns
 template <bool ALL>
 __device__ __forceinline__ void ret_turn(const RetUnit& u, const u32x4& a, const u32x4& b, const f32x4 (&cs)[4], const bf16_t* row, int rot_dims, const float* angles,
@@ -190,8 +211,8 @@ __device__ __forceinline__ void ret_turn(const RetUnit& u, const u32x4& a, const
   for (int e = 0; e < 8; ++e) {
     const float p = (e & 1) ? hi_bf(a[e >> 1]) : lo_bf(a[e >> 1]), q = (e & 1) ? hi_bf(b[e >> 1]) : lo_bf(b[e >> 1]);
     const float c = cs[e >> 1][2 * (e & 1)], s = cs[e >> 1][2 * (e & 1) + 1];
-    x[e] = ALL || u.turns ? p * c + -q * s : p;
-    y[e] = ALL || u.turns ? q * c + p * s : q;
+    x[e] = ALL || u.turns ? turned(e, p, -q, c, s) : p;
+    y[e] = ALL || u.turns ? turned(e, q, p, c, s) : q;
   }
   if (!ALL && !u.whole)
     for (int e = 0; e < 8; ++e) {
@@ -200,28 +221,90 @@ __device__ __forceinline__ void ret_turn(const RetUnit& u, const u32x4& a, const
     }
 }
 
+// y = x * w, rounded: what is left of it behind the high parts is not taken from the product itself, so that a key has the same bits in every kernel
+__device__ __forceinline__ void scaled8(const float (&x)[8], float w, float (&y)[8]) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    y[e] = x[e] * w;
+    asm("" : "+v"(y[e]));
+  }
+}
+
+// The LDS of a workgroup, in elements: keys and values by token, queries [high | low], the state, and the keys with their weights, high and low parts each but for the
+// values.  The weighted keys take the place of the keys, two barriers more per chunk, where a workgroup of their own size would not fit a CU, or not twice.
+template <int D, int C>
+struct RetLds {
+  static constexpr int dp = 32 * D, vp = 32 * C, KS = dp + 8, VS = vp + 8, QS = (2 * dp > vp ? 2 * dp : vp) + 8;
+  static constexpr int joint = 2 * (RC * (2 * KS + VS + QS) + 2 * vp * KS), own = joint + 4 * RC * KS;
+  static constexpr bool apart = own <= 81920 || (joint > 81920 && own <= 163840);
+  static constexpr int bytes = apart ? own : joint, increment = 2 * RC * (2 * KS + VS);
+};
+// Tile p of 16 columns of v: row or column n of it in a product is column v_column(p, n).  A lane of the outputs then has 8 C columns in a row.
+template <int C>
+__device__ __forceinline__ int v_column(int p, int n) { return 8 * C * (n >> 2) + 4 * p + (n & 3); }
+// ... in LDS tile after tile: a piece of 8 columns lies in two
+template <int C>
+__device__ __forceinline__ void put_values(bf16_t* row, int piece, const u32x4& v) {
+  bf16_t* at = row + 32 * (piece % C) + 4 * (piece / C);
+  *(u32x2*)at = u32x2{v[0], v[1]};
+  *(u32x2*)(at + 16) = u32x2{v[2], v[3]};
+}
+// as read_columns, lane row q with tokens t0 + 8 q .. + 7
+__device__ __forceinline__ u32x4 read_tokens(const bf16_t* tile, int stride, int t0, int c0, int lane) {
+  const bf16_t* p = tile + (t0 + 8 * (lane >> 4) + ((lane & 15) >> 2)) * stride + c0 + 4 * (lane & 3);
+  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
+  const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(p + 4 * stride));
+  const u32x2 lo = __builtin_bit_cast(u32x2, a), hi = __builtin_bit_cast(u32x2, b);
+  return u32x4{lo[0], lo[1], hi[0], hi[1]};
+}
+// sum_t w_t v_t k_t^T of a chunk for each of a wave's C * D tiles of the state: use(tile, sums)
+template <int D, int C, class F>
+__device__ __forceinline__ void ret_increments(const bf16_t* V, const bf16_t* Wh, const bf16_t* Wl, int wave, int lane, F&& use) {
+  using M = RetLds<D, C>;
+  constexpr int PT = 2 * C, PER = C == 3 ? 3 : C == 4 ? 2 : 1;  // a wave's tiles i and i + PER have the same 16 columns of v
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    u32x4 v[RC / 32];
+#pragma unroll
+    for (int k = 0; k < RC / 32; ++k) v[k] = read_tokens(V, M::VS, 32 * k, 16 * ((wave + 4 * j) % PT), lane);
+#pragma unroll
+    for (int i = j; i < C * D; i += PER) {
+      const int nt = (wave + 4 * i) / PT;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < RC / 32; ++k) {
+        acc = mfma(read_tokens(Wh, M::KS, 32 * k, 16 * nt, lane), v[k], acc);
+        acc = mfma(read_tokens(Wl, M::KS, 32 * k, 16 * nt, lane), v[k], acc);
+      }
+      use(i, acc);
+    }
+  }
+}
+
 // Prefill.  grid (heads, segments, sequences), four waves; a workgroup walks the chunks of a segment with the head's state in registers, a wave owns 16
 // tokens of the outputs and C * D 16 x 16 tiles of the state.  The next chunk's rows are under way while one is worked on.  All memory is read and
 // written by pieces of 16 bytes that follow one another, four lanes to 64 bytes at least, and reordered in LDS: a load whose lanes each take another row costs
 // four times that (what bounded the form before this, a workgroup per chunk with the state at its start from memory).  A wave's gates lie over its own queries, which it
 // has in registers by then, and its outputs over its gates.
-// 8 x 2048 tokens, 32 heads of 64: 113 us, 43 and 8 for the increments and states of two segments each, against 196 + 100 + 49 (increments of all chunks, their
-// states and outputs); bytes 65 us.  What is left is about 800 vector instructions per wave and chunk, and LDS.
-// INC: only what the segment adds to the state.  D: dp / 32, C: vp / 32
-template <int D, int C, bool INC>
-__global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ret_run_kernel(const LmRet a) {
-  constexpr int dp = 32 * D, vp = 32 * C, QS = (2 * dp > vp ? 2 * dp : vp) + 8, KS = dp + 8, VS = vp + 8, NT = C * D, PT = 2 * C;
-  constexpr int PER = C == 3 ? 3 : C == 4 ? 2 : 1;  // a wave's state tiles i and i + PER have the same 16 columns of v
+// The state goes from chunk to chunk as decay^n S + increment, the increment summed by itself, whatever the segments: a sequence has the same bits alone and beside others.
+// The keys take the weights in fp32, before they become two parts; the values' own bits enter.  (Weights on the values, rounded as two parts again: states 4.4e-6 from 64 bits,
+// 2.5e-6 this way; 1500 tokens.)
+// 8 x 2048 tokens, all launches: 32 heads of 64 169 us, 16 of 128 279; a workgroup per chunk with states in memory 318 and 504; bytes 65.  One prompt of 700: 24 and 35, 33 and 51.  What
+// bounds a chunk is vector instructions (about 1000 per wave; 16 gates per lane in full precision are 300 of them) and LDS.
+// D: dp / 32, C: vp / 32
+template <int D, int C>
+__global__ __launch_bounds__(256, (RetLds<D, C>::bytes <= 81920 ? 2 : 1)) void ret_run_kernel(const LmRet a) {
+  using M = RetLds<D, C>;
+  constexpr int dp = M::dp, vp = M::vp, QS = M::QS, KS = M::KS, VS = M::VS, NT = C * D, PT = 2 * C;
   constexpr int UNITS = dp / 16, NU = (RC * UNITS + 255) / 256;
   extern __shared__ __attribute__((aligned(16))) bf16_t rsm[];
-  bf16_t *Kh = rsm, *Kl = Kh + RC * KS, *V = Kl + RC * KS, *Q = V + RC * VS, *Sh = Q + RC * QS, *Sl = Sh + vp * KS;  // Q: [token][high | low]
-  __shared__ float ws[RC], later[2 * RC];  // decay^(n-1-t) of the tokens; [63 - age]: decay^age, 0 of an age below 0
+  bf16_t *Kh = rsm, *Kl = Kh + RC * KS, *V = Kl + RC * KS, *Q = V + RC * VS, *Sh = Q + RC * QS, *Sl = Sh + vp * KS;
+  bf16_t *Wh = M::apart ? Sl + vp * KS : Kh, *Wl = Wh + RC * KS;
   const int h = blockIdx.x, sg = blockIdx.y, seq = blockIdx.z, tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, first = sg * a.seg_chunks * RC, last = min(first + a.seg_chunks * RC, len);
   if (first >= last) return;
   const bool final = last == len;
-  if (INC && final) return;  // nobody starts behind the last segment
   const int pos0 = a.r.seq_pos0[seq];
   const float ld = log2f(a.decay[h]);
   const bf16_t* proj = (const bf16_t*)a.proj + (int64_t)row0 * a.ldp;
@@ -230,18 +313,16 @@ __global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ret_run_kernel(const L
 
   f32x4 S[NT];
   float* slot = a.state + ((int64_t)a.r.seq_slot[seq] * a.heads + h) * vp * dp;
-  float* seg = a.seg + (((int64_t)seq * a.n_seg + sg) * a.heads + h) * vp * dp;
-  const float* from = INC ? nullptr : a.n_seg > 1 ? seg : pos0 > 0 ? slot : nullptr;
+  const float* from = pos0 + first == 0 ? nullptr : a.n_seg > 1 ? ret_seg_state(a, seq, sg * a.seg_chunks, h) : slot;
 #pragma unroll
   for (int i = 0; i < NT; ++i) {
     const int tile = wave + 4 * i, pt = tile % PT, nt = tile / PT;
-    S[i] = from ? *(const f32x4*)(from + (16 * pt + r) * dp + 16 * nt + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
+    S[i] = from ? *(const f32x4*)(from + v_column<C>(pt, r) * dp + 16 * nt + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
   u32x4 qr[NU][2], kr[NU][2], vr[C], gr[C];
   f32x4 cs[NU][4];
   constexpr u32x4 none = {0u, 0u, 0u, 0u};
-  if (!INC && tid < 2 * RC) later[tid] = tid <= RC - 1 ? pow_int(ld, RC - 1 - tid) : 0.f;  // [63 - age]
   auto load = [&](int t0) {  // rows past the end: the last one again
     const int n = min(RC, last - t0);
     const bf16_t* rows = proj + (int64_t)t0 * a.ldp;
@@ -253,26 +334,21 @@ __global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ret_run_kernel(const L
       const RetUnit at = ret_unit(u % UNITS, a.rot_dims);
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
-        if (!INC) qr[i][k] = piece(t, cq + at.d[k]);
+        qr[i][k] = piece(t, cq + at.d[k]);
         kr[i][k] = piece(t, ck + at.d[k]);
       }
-      if (a.rot_dims > 0) {
-        const uint32_t from = (uint32_t)min(t, n - 1) * (uint32_t)a.rot_dims + (at.turns ? 2 * at.d[0] : 0);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) cs[i][k] = at.whole ? *(const f32x4*)(angles + (from + 4 * k)) : f32x4{0.f, 0.f, 0.f, 0.f};
-      }
+      ret_angles(at, angles, min(t, n - 1), a.rot_dims, cs[i]);
     }
 #pragma unroll
     for (int i = 0; i < C; ++i) {
       const int p = tid + 256 * i;
       vr[i] = piece(p / (vp / 8), cv + p % (vp / 8) * 8);
     }
-    if (!INC)
 #pragma unroll
-      for (int i = 0; i < C; ++i) {  // the wave's own tokens
-        const int p = lane + 64 * i;
-        gr[i] = piece(16 * wave + p / (vp / 8), cg + p % (vp / 8) * 8);
-      }
+    for (int i = 0; i < C; ++i) {  // the wave's own tokens
+      const int p = lane + 64 * i;
+      gr[i] = piece(16 * wave + p / (vp / 8), cg + p % (vp / 8) * 8);
+    }
   };
   load(first);
   const int t = 16 * wave + r;  // this lane's query
@@ -280,7 +356,8 @@ __global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ret_run_kernel(const L
 
   for (int t0 = first; t0 < last; t0 += RC) {
     const int n = min(RC, last - t0);
-    const bool stated = from || t0 > first;
+    const bool stated = from || t0 > first, on = final || t0 + RC < last;  // on: somebody needs the state behind this chunk
+    u32x4 wh[NU][2], wl[NU][2];
     __syncthreads();  // the previous chunk's tiles have been read
     auto stage = [&](auto all) {
       constexpr bool ALL = decltype(all)::value;
@@ -294,24 +371,31 @@ __global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ret_run_kernel(const L
         const float* angles = a.rope + (int64_t)(pos0 + t0 + tl) * a.rot_dims;
         float x[2][8];
         u32x4 hi, lo;
-        if (!INC) {
-          ret_turn<ALL>(at, qr[i][0], qr[i][1], cs[i], row + cq, a.rot_dims, angles, x[0], x[1]);
-#pragma unroll
-          for (int k = 0; k < 2; ++k) {
-            split8(x[k], hi, lo);
-            *(u32x4*)(Q + tu * QS + at.d[k]) = hi;
-            *(u32x4*)(Q + tu * QS + dp + at.d[k]) = lo;
-          }
-        }
-        ret_turn<ALL>(at, kr[i][0], kr[i][1], cs[i], row + ck, a.rot_dims, angles, x[0], x[1]);
+        ret_turn<ALL>(at, qr[i][0], qr[i][1], cs[i], row + cq, a.rot_dims, angles, x[0], x[1]);
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) x[k][e] *= a.scale;
           split8(x[k], hi, lo);
-          if (n < RC && tu >= n) hi = lo = none;
-          *(u32x4*)(Kh + tu * KS + at.d[k]) = hi;
-          *(u32x4*)(Kl + tu * KS + at.d[k]) = lo;
+          *(u32x4*)(Q + tu * QS + at.d[k]) = hi;
+          *(u32x4*)(Q + tu * QS + dp + at.d[k]) = lo;
+        }
+        ret_turn<ALL>(at, kr[i][0], kr[i][1], cs[i], row + ck, a.rot_dims, angles, x[0], x[1]);
+        const float w = a.scale * pow_int(ld, n - 1 - tl);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          float y[8];
+          scaled8(x[k], a.scale, y);
+          split8(y, hi, lo);
+          const bool dead = n < RC && tu >= n;
+          *(u32x4*)(Kh + tu * KS + at.d[k]) = dead ? none : hi;
+          *(u32x4*)(Kl + tu * KS + at.d[k]) = dead ? none : lo;
+          if (!on) continue;
+          scaled8(x[k], w, y);
+          split8(y, wh[i][k], wl[i][k]);
+          if (dead) wh[i][k] = wl[i][k] = none;
+          if (M::apart) {
+            *(u32x4*)(Wh + tu * KS + at.d[k]) = wh[i][k];
+            *(u32x4*)(Wl + tu * KS + at.d[k]) = wl[i][k];
+          }
         }
       }
     };
@@ -320,9 +404,9 @@ __global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ret_run_kernel(const L
 #pragma unroll
     for (int i = 0; i < C; ++i) {
       const int p = tid + 256 * i, tv = p / (vp / 8);
-      *(u32x4*)(V + tv * VS + p % (vp / 8) * 8) = n < RC && tv >= n ? none : vr[i];
+      put_values<C>(V + tv * VS, p % (vp / 8), n < RC && tv >= n ? none : vr[i]);
     }
-    if (!INC && stated)
+    if (stated)
 #pragma unroll
       for (int i = 0; i < NT; ++i) {
         const int tile = wave + 4 * i, pt = tile % PT, nt = tile / PT, at = (16 * pt + r) * KS + 16 * nt + 4 * q;
@@ -330,15 +414,13 @@ __global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ret_run_kernel(const L
         *(u32x2*)(Sh + at) = hi;
         *(u32x2*)(Sl + at) = u32x2{pack_bf16x2(S[i][0] - lo_bf(hi[0]), S[i][1] - hi_bf(hi[0])), pack_bf16x2(S[i][2] - lo_bf(hi[1]), S[i][3] - hi_bf(hi[1]))};
       }
-    if (tid < RC) ws[tid] = tid < n ? pow_int(ld, n - 1 - tid) : 0.f;
     u32x4 gc[C];
-    if (!INC)
 #pragma unroll
-      for (int i = 0; i < C; ++i) gc[i] = gr[i];
+    for (int i = 0; i < C; ++i) gc[i] = gr[i];
     __syncthreads();
     if (t0 + RC < last) load(t0 + RC);
 
-    if (!INC && 16 * wave < n) {
+    if (16 * wave < n) {
       bf16_t* G = Q + 16 * wave * QS;  // the wave's own rows
       u32x4 qh[D], ql[D];
 #pragma unroll
@@ -369,6 +451,8 @@ __global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ret_run_kernel(const L
 #pragma unroll
         for (int i = 0; i < PT; ++i) o[i] *= et;
       }
+      int age0 = t - 4 * q;
+      asm volatile("" : "+v"(age0));  // (powers made here: 16 registers less than in front of the loop)
 #pragma unroll
       for (int b = 0; b < RC / 32; ++b) {
         if (2 * b > wave) continue;
@@ -387,9 +471,10 @@ __global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ret_run_kernel(const L
             }
           }
 #pragma unroll
-          for (int e = 0; e < 4; ++e) p[4 * half + e] = later[RC - 1 - t + 16 * sb + 4 * q + e];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) p[4 * half + e] = p[4 * half + e] != 0.f ? acc[e] * p[4 * half + e] : 0.f;
+          for (int e = 0; e < 4; ++e) {
+            const int age = age0 - 16 * sb - e;
+            p[4 * half + e] = sb <= wave && age >= 0 ? acc[e] * pow_int(ld, age) : 0.f;
+          }
         }
         u32x4 ph, pl;
         split8(p, ph, pl);
@@ -400,20 +485,31 @@ __global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ret_run_kernel(const L
           o[i] = mfma(v, pl, o[i]);
         }
       }
-      f32x4 sq = {0.f, 0.f, 0.f, 0.f};
+      // the lane's columns 8 C q ..: four sums of 2 C in a row, then over the quarters (written out, as the rotation)
+      float sq[4];
 #pragma unroll
-      for (int i = 0; i < PT; ++i) sq += o[i] * o[i];
+      for (int k = 0; k < 4; ++k) {
+        auto at = [&](int d) { return o[(PT * k + d) >> 2][(PT * k + d) & 3]; };
+        sq[k] = fmaf(at(0), at(0), at(1) * at(1));
+#pragma unroll
+        for (int d = 2; d < PT; ++d) sq[k] = fmaf(at(d), at(d), sq[k]);
+      }
       float ss = (sq[0] + sq[1]) + (sq[2] + sq[3]);
       ss += __shfl_xor(ss, 16, 64);
       ss += __shfl_xor(ss, 32, 64);
       const float rn = 1.0f / sqrtf(ss / (float)a.vdim + a.eps);
 #pragma unroll
-      for (int i = 0; i < PT; ++i) {
-        bf16_t* at = G + r * QS + 16 * i + 4 * q;
-        f32x4 y = ld4(at);
+      for (int i = 0; i < C; ++i) {
+        bf16_t* at = G + r * QS + 8 * C * q + 8 * i;
+        const u32x4 g = *(const u32x4*)at;
+        u32x4 y;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) y[e] = o[i][e] * rn * silu_fast(y[e]);
-        st4(at, y);
+        for (int e = 0; e < 4; ++e) {
+          const f32x4& x = o[2 * i + (e >> 1)];
+          const int c = 2 * (e & 1);
+          y[e] = pack_bf16x2(x[c] * rn * silu_f32(lo_bf(g[e])), x[c + 1] * rn * silu_f32(hi_bf(g[e])));
+        }
+        *(u32x4*)at = y;
       }
       wave_lds_order();
 #pragma unroll
@@ -423,70 +519,124 @@ __global__ __launch_bounds__(256, C * D > 9 ? 1 : 2) void ret_run_kernel(const L
           *(u32x4*)((bf16_t*)a.out + (int64_t)(row0 + t0 + 16 * wave + tg) * a.ldo + in_chunks(h * vp + d, a.out_chunk)) = *(const u32x4*)(G + tg * QS + d);
       }
     }
-
-    const float keep = pow_int(ld, n);
+    if (!on) break;
+    if (!M::apart) {
+      __syncthreads();  // the keys have been read
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
-      const int pt = (wave + 4 * j) % PT;
-      u32x4 vh[RC / 32], vl[RC / 32];
+      for (int i = 0; i < NU; ++i) {
+        const int u = tid + 256 * i, tu = u / UNITS;
+        if (RC * UNITS % 256 != 0 && u >= RC * UNITS) break;
+        const RetUnit at = ret_unit(u % UNITS, a.rot_dims);
 #pragma unroll
-      for (int k = 0; k < RC / 32; ++k) {
-        const u32x4 x = read_columns(V, VS, 32 * k, 16 * pt, lane);
-        const f32x4 w0 = *(const f32x4*)(ws + 32 * k + 4 * q), w1 = *(const f32x4*)(ws + 32 * k + 16 + 4 * q);
-        const float v[8] = {lo_bf(x[0]) * w0[0], hi_bf(x[0]) * w0[1], lo_bf(x[1]) * w0[2], hi_bf(x[1]) * w0[3],
-                            lo_bf(x[2]) * w1[0], hi_bf(x[2]) * w1[1], lo_bf(x[3]) * w1[2], hi_bf(x[3]) * w1[3]};
-        split8(v, vh[k], vl[k]);
-      }
-#pragma unroll
-      for (int i = j; i < NT; i += PER) {
-        const int nt = (wave + 4 * i) / PT;
-        S[i] *= keep;
-#pragma unroll
-        for (int k = 0; k < RC / 32; ++k) {
-          const u32x4 kh = read_columns(Kh, KS, 32 * k, 16 * nt, lane), kl = read_columns(Kl, KS, 32 * k, 16 * nt, lane);
-          S[i] = mfma(kh, vh[k], S[i]);
-          S[i] = mfma(kh, vl[k], S[i]);
-          S[i] = mfma(kl, vh[k], S[i]);
+        for (int k = 0; k < 2; ++k) {
+          *(u32x4*)(Wh + tu * KS + at.d[k]) = wh[i][k];
+          *(u32x4*)(Wl + tu * KS + at.d[k]) = wl[i][k];
         }
       }
+      __syncthreads();
     }
+    const float keep = pow_int(ld, n);
+    ret_increments<D, C>(V, Wh, Wl, wave, lane, [&](int i, const f32x4& inc) { S[i] = S[i] * keep + inc; });
   }
-  float* to = INC ? seg : final ? slot : nullptr;
-  if (to)
+  if (final)
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
       const int tile = wave + 4 * i, pt = tile % PT, nt = tile / PT;
-      *(f32x4*)(to + (16 * pt + r) * dp + 16 * nt + 4 * q) = S[i];
+      *(f32x4*)(slot + v_column<C>(pt, r) * dp + 16 * nt + 4 * q) = S[i];
     }
 }
 
-// grid (heads * vp * dp / 1024, sequences): what the segments add -> the states they start from
+// grid (heads, chunks, sequences): what each chunk before the last segment adds to the state
+template <int D, int C>
+__global__ __launch_bounds__(256) void ret_increment_kernel(const LmRet a) {
+  using M = RetLds<D, C>;
+  constexpr int dp = M::dp, vp = M::vp, KS = M::KS, VS = M::VS, PT = 2 * C, UNITS = dp / 16, NU = (RC * UNITS + 255) / 256;
+  extern __shared__ __attribute__((aligned(16))) bf16_t rsm[];
+  bf16_t *Wh = rsm, *Wl = Wh + RC * KS, *V = Wl + RC * KS;
+  const int h = blockIdx.x, c = blockIdx.y, seq = blockIdx.z, tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0;
+  if (c >= ret_chunks_ahead(a, len)) return;  // (all of them whole)
+  const float ld = log2f(a.decay[h]);
+  const bf16_t* rows = (const bf16_t*)a.proj + (int64_t)(row0 + c * RC) * a.ldp;
+  const float* angles = a.rope + (int64_t)(a.r.seq_pos0[seq] + c * RC) * a.rot_dims;
+  const int ck = a.col_k + h * dp, cv = a.col_v + h * vp;
+  auto piece = [&](int t, int col) { return *(const u32x4*)(rows + ((uint32_t)t * (uint32_t)a.ldp + (uint32_t)col)); };
+  u32x4 vr[C];
+#pragma unroll
+  for (int i = 0; i < C; ++i) {
+    const int p = tid + 256 * i;
+    vr[i] = piece(p / (vp / 8), cv + p % (vp / 8) * 8);
+  }
+#pragma unroll
+  for (int i = 0; i < NU; ++i) {
+    const int u = tid + 256 * i, t = u / UNITS;
+    if (RC * UNITS % 256 != 0 && u >= RC * UNITS) break;
+    const RetUnit at = ret_unit(u % UNITS, a.rot_dims);
+    f32x4 cs[4];
+    ret_angles(at, angles, t, a.rot_dims, cs);
+    float x[2][8];
+    ret_turn<false>(at, piece(t, ck + at.d[0]), piece(t, ck + at.d[1]), cs, rows + (int64_t)t * a.ldp + ck, a.rot_dims, angles + (int64_t)t * a.rot_dims, x[0], x[1]);
+    const float w = a.scale * pow_int(ld, RC - 1 - t);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      float y[8];
+      u32x4 hi, lo;
+      scaled8(x[k], w, y);
+      split8(y, hi, lo);
+      *(u32x4*)(Wh + t * KS + at.d[k]) = hi;
+      *(u32x4*)(Wl + t * KS + at.d[k]) = lo;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < C; ++i) {
+    const int p = tid + 256 * i;
+    put_values<C>(V + p / (vp / 8) * VS, p % (vp / 8), vr[i]);
+  }
+  __syncthreads();
+  float* to = ret_seg_state(a, seq, c + 1, h);
+  ret_increments<D, C>(V, Wh, Wl, wave, lane, [&](int i, const f32x4& inc) {
+    const int tile = wave + 4 * i, pt = tile % PT, nt = tile / PT;
+    *(f32x4*)(to + v_column<C>(pt, r) * dp + 16 * nt + 4 * q) = inc;
+  });
+}
+
+// grid (heads * vp * dp / 1024, sequences): the states that the segments start from, chunk by chunk as within a segment
 __global__ __launch_bounds__(256) void ret_segments_kernel(const LmRet a) {
   const int seq = blockIdx.y, per_head = a.vp * a.dp;
   const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4, n_el = (int64_t)a.heads * per_head;
   if (i >= n_el) return;
-  const int h = (int)(i / per_head), len = a.r.seq_row0[seq + 1] - a.r.seq_row0[seq], n = (len + a.seg_chunks * RC - 1) / (a.seg_chunks * RC);
-  const float keep = pow_int(log2f(a.decay[h]), a.seg_chunks * RC);
+  const int h = (int)(i / per_head), n = ret_chunks_ahead(a, a.r.seq_row0[seq + 1] - a.r.seq_row0[seq]);
+  const float keep = pow_int(log2f(a.decay[h]), RC);
   f32x4 S = {0.f, 0.f, 0.f, 0.f};
   if (a.r.seq_pos0[seq] > 0) S = *(const f32x4*)(a.state + (int64_t)a.r.seq_slot[seq] * n_el + i);
-  for (int sg = 0; sg < n; ++sg) {
-    float* p = a.seg + ((int64_t)seq * a.n_seg + sg) * n_el + i;
-    f32x4 inc = {0.f, 0.f, 0.f, 0.f};
-    if (sg + 1 < n) inc = *(const f32x4*)p;
-    *(f32x4*)p = S;
-    S = keep * S + inc;
+  float* p = ret_seg_state(a, seq, 0, 0) + i;
+  *(f32x4*)p = S;
+  constexpr int U = 4;  // chunks in flight
+  for (int c0 = 0; c0 < n; c0 += U) {
+    f32x4 inc[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (c0 + u < n) inc[u] = *(const f32x4*)(p + (c0 + u + 1) * n_el);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (c0 + u < n) {
+        S = S * keep + inc[u];
+        if ((c0 + u + 1) % a.seg_chunks == 0) *(f32x4*)(p + (c0 + u + 1) * n_el) = S;  // in the place of what is in it now
+      }
   }
 }
 
 typedef void (*RetKernel)(const LmRet);
 struct RetPick {
   RetKernel run, inc;
-  int lds;
+  int lds, inc_lds;
 };
 template <int D, int C>
 RetPick ret_run_of() {
-  constexpr int dp = 32 * D, vp = 32 * C, QS = (2 * dp > vp ? 2 * dp : vp) + 8;
-  return RetPick{ret_run_kernel<D, C, false>, ret_run_kernel<D, C, true>, (RC * (2 * (dp + 8) + vp + 8 + QS) + 2 * vp * (dp + 8)) * 2};
+  using M = RetLds<D, C>;
+  static_assert(M::bytes <= 163840, "LDS");
+  return RetPick{ret_run_kernel<D, C>, ret_increment_kernel<D, C>, M::bytes, M::increment};
 }
 template <int D>
 RetPick ret_run_by_width(int c) {
@@ -495,11 +645,11 @@ RetPick ret_run_by_width(int c) {
     case 2: return ret_run_of<D, 2>();
     case 3: return ret_run_of<D, 3>();
     case 4: return ret_run_of<D, 4>();
-    default: return RetPick{nullptr, nullptr, 0};
+    default: return RetPick{nullptr, nullptr, 0, 0};
   }
 }
 RetPick ret_run_pick(const LmRet& a) {
-  const RetPick none = {nullptr, nullptr, 0};
+  const RetPick none = {nullptr, nullptr, 0, 0};
   if ((a.col_q | a.col_k | a.col_v | a.col_g | a.ldp | a.ldo | a.out_chunk) % 8 != 0) return none;  // pieces of eight
   switch (a.dp / 32) {
     case 1: return ret_run_by_width<1>(a.vp / 32);
@@ -597,9 +747,9 @@ int lm_ret_segments(int n_seq, int heads, int dp, int vp, int max_len, int* chun
   *chunks = 3 * per + 4 < 2 * n ? per : n;
   return (n + *chunks - 1) / *chunks;
 }
-int lm_ret_most_segments(int n_seq, int heads, int dp, int vp, int max_len) {
-  const int64_t n = (max_len + RC - 1) / RC;
-  return n > 1 ? (int)std::min(n_seq * n, (int64_t)(ret_room(dp, vp) / heads)) : 0;
+int lm_ret_most_states(int n_seq, int heads, int dp, int vp, int max_len) {
+  const int n = (max_len + RC - 1) / RC;
+  return n > 1 && dp <= 128 && vp <= 128 ? std::min(n_seq, ret_room(dp, vp) / (2 * heads)) * n : 0;  // (more sequences: no segments)
 }
 bool lm_ret_mfma_takes(const LmRet& a) { return ret_run_pick(a).run != nullptr; }
 md_status lm_ret_mfma(const LmRet& a, hipStream_t s) {
@@ -608,8 +758,8 @@ md_status lm_ret_mfma(const LmRet& a, hipStream_t s) {
   const dim3 grid(a.heads, a.n_seg, a.r.n_seq);
   MD_TRY(md_ensure_dynamic_lds((const void*)k.run, k.lds));
   if (a.n_seg > 1) {
-    MD_TRY(md_ensure_dynamic_lds((const void*)k.inc, k.lds));
-    hipLaunchKernelGGL(k.inc, grid, dim3(256), k.lds, s, a);
+    MD_TRY(md_ensure_dynamic_lds((const void*)k.inc, k.inc_lds));
+    hipLaunchKernelGGL(k.inc, dim3(a.heads, (a.n_seg - 1) * a.seg_chunks, a.r.n_seq), dim3(256), k.inc_lds, s, a);
     MD_TRY(md_launch_status());
     hipLaunchKernelGGL(ret_segments_kernel, dim3((a.heads * a.vp * a.dp + 1023) / 1024, a.r.n_seq), dim3(256), 0, s, a);
     MD_TRY(md_launch_status());
