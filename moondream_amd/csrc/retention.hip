@@ -238,6 +238,7 @@ struct RetLds {
   static constexpr int joint = 2 * (RC * (2 * KS + VS + QS) + 2 * vp * KS), own = joint + 4 * RC * KS;
   static constexpr bool apart = own <= 81920 || (joint > 81920 && own <= 163840);
   static constexpr int bytes = apart ? own : joint, increment = 2 * RC * (2 * KS + VS);
+  static constexpr int resident = C * D == 1 ? 3 : bytes <= 81920 ? 2 : 1;  // workgroups on a CU: by LDS, and the registers of the smallest heads
 };
 // Tile p of 16 columns of v: row or column n of it in a product is column v_column(p, n).  A lane of the outputs then has 8 C columns in a row.
 template <int C>
@@ -293,7 +294,7 @@ __device__ __forceinline__ void ret_increments(const bf16_t* V, const bf16_t* Wh
 // bounds a chunk is vector instructions (about 1000 per wave; 16 gates per lane in full precision are 300 of them) and LDS.
 // D: dp / 32, C: vp / 32
 template <int D, int C>
-__global__ __launch_bounds__(256, (RetLds<D, C>::bytes <= 81920 ? 2 : 1)) void ret_run_kernel(const LmRet a) {
+__global__ __launch_bounds__(256, (RetLds<D, C>::resident)) void ret_run_kernel(const LmRet a) {
   using M = RetLds<D, C>;
   constexpr int dp = M::dp, vp = M::vp, QS = M::QS, KS = M::KS, VS = M::VS, NT = C * D, PT = 2 * C;
   constexpr int UNITS = dp / 16, NU = (RC * UNITS + 255) / 256;
@@ -630,13 +631,13 @@ __global__ __launch_bounds__(256) void ret_segments_kernel(const LmRet a) {
 typedef void (*RetKernel)(const LmRet);
 struct RetPick {
   RetKernel run, inc;
-  int lds, inc_lds;
+  int lds, inc_lds, resident;
 };
 template <int D, int C>
 RetPick ret_run_of() {
   using M = RetLds<D, C>;
   static_assert(M::bytes <= 163840, "LDS");
-  return RetPick{ret_run_kernel<D, C>, ret_increment_kernel<D, C>, M::bytes, M::increment};
+  return RetPick{ret_run_kernel<D, C>, ret_increment_kernel<D, C>, M::bytes, M::increment, M::resident};
 }
 template <int D>
 RetPick ret_run_by_width(int c) {
@@ -645,19 +646,21 @@ RetPick ret_run_by_width(int c) {
     case 2: return ret_run_of<D, 2>();
     case 3: return ret_run_of<D, 3>();
     case 4: return ret_run_of<D, 4>();
-    default: return RetPick{nullptr, nullptr, 0, 0};
+    default: return RetPick{};
+  }
+}
+RetPick ret_run_by_widths(int dp, int vp) {
+  switch (dp / 32) {
+    case 1: return ret_run_by_width<1>(vp / 32);
+    case 2: return ret_run_by_width<2>(vp / 32);
+    case 3: return ret_run_by_width<3>(vp / 32);
+    case 4: return ret_run_by_width<4>(vp / 32);
+    default: return RetPick{};
   }
 }
 RetPick ret_run_pick(const LmRet& a) {
-  const RetPick none = {nullptr, nullptr, 0, 0};
-  if ((a.col_q | a.col_k | a.col_v | a.col_g | a.ldp | a.ldo | a.out_chunk) % 8 != 0) return none;  // pieces of eight
-  switch (a.dp / 32) {
-    case 1: return ret_run_by_width<1>(a.vp / 32);
-    case 2: return ret_run_by_width<2>(a.vp / 32);
-    case 3: return ret_run_by_width<3>(a.vp / 32);
-    case 4: return ret_run_by_width<4>(a.vp / 32);
-    default: return none;
-  }
+  if ((a.col_q | a.col_k | a.col_v | a.col_g | a.ldp | a.ldo | a.out_chunk) % 8 != 0) return RetPick{};  // pieces of eight
+  return ret_run_by_widths(a.dp, a.vp);
 }
 
 // grid (heads, sequences).  Sixteen lanes per state row, sixteen rows at a time, R rows of up to 64 E columns per thread.  Few sequences: the chain of loads
@@ -738,18 +741,19 @@ RetKernel ret_decode_pick(const LmRet& a) {
 
 }  // namespace
 
-// Segments: as many as keep to the workgroups that a CU holds, two, or one of the largest heads (ret_run_kernel's registers).  The increments cost half of the
-// outputs, and they and the states two launches, about two chunks.  Eight layers of little else: 32 heads of 64, 700 tokens, up to 512 workgroups 620 us, 256 702; 8 x 2048
-// tokens 4255 and 4448; 16 heads of 128: 800 and 748, 5369 and 5214.
-inline int ret_room(int dp, int vp) { return dp * vp > 9 * 1024 ? 256 : 512; }
+// Segments: as many as keep to the workgroups that the CUs hold by their LDS (64 x 64: two, larger heads mostly one).  The increments cost about half of the outputs, and
+// they and the states two launches, about two chunks.  us with 1, 2, .. segments: 32 heads of 64 x 64, one prompt of 130 tokens 17.4, 19.1, 14.9; 700 11 segments 23.8, 6 24.9;
+// 3 x 2048 5 79.0, 8 80.7; 8 x 2048 184, 168, 200 (3).  16 of 64 x 128, 16 segments of 2000 38.8 and 32 41.1; 3 x 700 4 41.6, 6 49.3; 8 x 500 66.8, 52.7, 58.9 (4); 8 x 2048 259,
+// 175, 191 (4).  16 of 96 x 96, 8 x 2048 286, 202, 224 (4).
+inline int ret_room(int dp, int vp) { return 256 * ret_run_by_widths(dp, vp).resident; }
 int lm_ret_segments(int n_seq, int heads, int dp, int vp, int max_len, int* chunks) {
   const int n = (max_len + RC - 1) / RC, segs = ret_room(dp, vp) / (n_seq * heads), per = segs > 1 ? (n + segs - 1) / segs : n;
-  *chunks = 3 * per + 4 < 2 * n ? per : n;
+  *chunks = 3 * per + 3 <= 2 * n ? per : n;
   return (n + *chunks - 1) / *chunks;
 }
 int lm_ret_most_states(int n_seq, int heads, int dp, int vp, int max_len) {
   const int n = (max_len + RC - 1) / RC;
-  return n > 1 && dp <= 128 && vp <= 128 ? std::min(n_seq, ret_room(dp, vp) / (2 * heads)) * n : 0;  // (more sequences: no segments)
+  return n > 1 ? std::min(n_seq, ret_room(dp, vp) / (2 * heads)) * n : 0;  // (more sequences: no segments)
 }
 bool lm_ret_mfma_takes(const LmRet& a) { return ret_run_pick(a).run != nullptr; }
 md_status lm_ret_mfma(const LmRet& a, hipStream_t s) {

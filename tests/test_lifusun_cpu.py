@@ -190,3 +190,21 @@ def test_every_planted_mistake_shows(fault):
     name = U.SHOWS[fault]
     good, bad = U.oracle_logits(name, [61]), U.oracle_logits(name, [61], fault=fault)
     assert U.logit_error(bad[0], good[0]) > 2e-3
+
+
+@pytest.mark.parametrize("dim,vdim,resident", [(32, 32, 3), (32, 128, 2), (64, 64, 2), (64, 96, 2), (64, 128, 1), (96, 96, 1), (128, 32, 1), (128, 64, 1), (128, 128, 1), (160, 64, 0)])
+def test_segments_of_retention_prompts(dim, vdim, resident):
+    """As many as are resident by the kernel's LDS on 256 compute units, none of them empty, within the states that the largest step reserves."""
+    lib = _lib.load()
+    segments, most = lib._Z15lm_ret_segmentsiiiiiPi, lib._Z18lm_ret_most_statesiiiii  # (internal: lm_internal.hpp)
+    for heads in (1, 3, 16, 40, 300):
+        for n_seq in (1, 2, 7, 64):
+            for n in (2, 64, 65, 130, 200, 500, 700, 2048, 100000):
+                per = ctypes.c_int()
+                segs, chunks = segments(n_seq, heads, dim, vdim, n, ctypes.byref(per)), -(-n // 64)
+                assert (segs - 1) * per.value < chunks <= segs * per.value
+                if segs > 1:
+                    assert segs * n_seq * heads <= 256 * resident
+                    assert all(n_seq * ((segs - 1) * per.value + 1) <= most(s, heads, dim, vdim, m) for s in (n_seq, 64) for m in (n, 100000))
+                elif resident * 256 >= 4 * n_seq * heads:
+                    assert chunks < 4
