@@ -823,23 +823,25 @@ int pick_tile(int M, int n_store, int K, int policy) {
   // (lm_head: 800 column panels keep every CU busy with the 128 x 128 two-stage config, measured 57 vs 73 us); every config
   // involved multiplies with 32x32x16 in the same K order as the 64-row decode configs
   if (policy == MD_TILE_DECODE_TALL && M > 64 && M <= 128 && n_store < 16384) return 21;
-  // Single-image regime (1458 ViT rows / 735 decoder rows; every config named here sums K in the same order, as 32x32x16 or (22, 23) 16x16x32 products).
+  // Single-image regime (1458 ViT rows / 735 decoder rows; every config named here sums K in the same order, as 32x32x16 or (22) 16x16x32 products).
   //  * at most 128 tiles of 128 x 128 and a long K (proj / fc2 of both towers): half the chip is idle whatever the tile and the
   //    launch runs at the latency of its K loop -- the 64 x 64 tiles with the 4-deep ring and DMA helper waves (the decode-regime
-  //    config) quadruple the workgroups (tools/sweep_gemm_b1.py, round 2: text fc2 at 730 rows 81 -> 61 us, ViT fc2 50 -> 30 us).
+  //    config) quadruple the workgroups (tools/sweep_gemm_b1.py: text fc2 at 730 rows 81 -> 61 us, ViT fc2 50 -> 30 us).
+  //    128 x 128 tiles with a four-stage ring win back-to-back sweeps of 91 to 128 tiles (text fc2 63.7 -> 52.0 us, with operands of two slices in registers 64 -> 57) and LOSE
+  //    inside a caption, where the layer's weights come from HBM and 96 or 108 workgroups pull them through as many CUs (ViT proj / fc2 23.7 -> 24.9 us, text 42.0 -> 42.5 us
+  //    per launch: profiles/r05_b1_tile_config_sweep.txt; the other form 25.1 -> 26.3 beside a four-wave kernel of the same 58 us, a caption 0.1 ms).  Prompts of 150 to 380 tokens
+  //    of the layered models: 0.99 to 1.01 of each other.  A decode step of 65 .. 128 rows and 16384 columns takes this config too: the bits of the 64-row configs.
   //  * up to 512 tiles of 128 x 128 (ViT qkv / fc1, projector fc1): the two-stage 128 x 128 config keeps TWO workgroups per CU, so
   //    all of them are resident at once; the cost model below counts one workgroup per CU and preferred 256 x 128.  Inside a
-  //    caption: ViT qkv 25.9 -> 21.5 us, fc1 29.2 -> 24.9 us per launch (round 5).  Wider layers (the decoder's fused qkv|fc1: 672
+  //    caption: ViT qkv 25.9 -> 21.5 us, fc1 29.2 -> 24.9 us per launch.  Wider layers (the decoder's fused qkv|fc1: 672
   //    such tiles) stay with the cost model, i.e. the four-wave kernel.
   if (M > 64) {
     const long t128 = (long)((M + 127) / 128) * ((n_store + 127) / 128);
-    //    From about 90 tiles of 128 x 128 on they beat the 64 x 64 ones (700 rows, 2048 columns, K 2048 / 5440 / 8192: 17.6 / 43 / 57 us against 18.1 / 46 / 64; 300 rows
-    //    16.9 / 40 / 55 and 13.8 / 31 / 45).
-    if (K >= 1024 && t128 <= 128) return t128 > 90 ? 23 : 16;
+    if (K >= 1024 && t128 <= 128) return 16;
     // ("small_m_rule": 0 = round 2's rule, 1 = the default below, n > 1 = that many tiles instead of 512 -- A/B)
     const int rule = knobs().small_m_rule;
     //  * of these, where 256 x 128 tiles are one round of the CUs (700 rows, 10880 columns, K 2048: 47 us as 128 x 128, 40 as 256 x 128, 35 with the operands of two
-    //    slices in registers)
+    //    slices in registers; inside a caption, beside a four-wave kernel of 58 us, the ViT's qkv 20.2 -> 19.2 and fc1 23.6 -> 22.5)
     const long t256 = (long)((M + 255) / 256) * ((n_store + 127) / 128);
     if (rule == 1 && t128 > 256 && t128 <= 512 && t256 <= 256) return 22;
     if (rule != 0 && t128 <= (rule > 1 ? rule : 512)) return 2;

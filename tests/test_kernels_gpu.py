@@ -141,6 +141,20 @@ def test_smaller_tiles_have_the_bits_of_the_four_wave_kernel(lib, force_tile, k,
                 assert torch.equal(g22, want), (m, kw.keys())
 
 
+@pytest.mark.parametrize("n,k", [(16320, 1088), (16384, 1024), (16384, 1152), (16448, 2048)], ids=str)
+def test_decode_steps_of_many_columns_round_as_the_64_row_regime(lib, n, k):
+    """MD_TILE_DECODE_TALL on both sides of 16384 columns, where a launch of 65 .. 128 rows leaves the weight-streaming tile: the bits of its rows in launches of 64.
+    The second half of K takes the first half's products away again, in another order, so that what is left is the rounding of every partial sum."""
+    order = torch.randperm(k // 2, generator=torch.Generator().manual_seed(7)).cuda()
+    a, w = randn(128, k, seed=81), randn(n, k, seed=82)
+    a[:, k // 2:], w[:, k // 2:] = a[:, : k // 2][:, order], -w[:, : k // 2][:, order]
+    lin = PackedLinear(w, torch.zeros(n, dtype=BF16), "cuda")
+    a = pad_k(a, lin.k_pad)
+    want = torch.cat([gemm(lib, x.contiguous(), lin) for x in a.split(64)])
+    for m in (65, 100, 128):
+        assert torch.equal(gemm(lib, a[:m].contiguous(), lin, tile_policy=_lib.MD_TILE_DECODE_TALL), want[:m]), m
+
+
 def test_tile_policy_is_a_per_call_field(lib, force_tile):
     """ABI 5: md_gemm_args.tile_policy.  MD_TILE_PINNED makes the tile config of a > 64-row launch a function of the layer alone --
     the 256 x 256 kernel whatever the row count -- so a row gets the same bits in a 100-row and in a 5000-row launch; MD_TILE_BY_SHAPE
