@@ -305,9 +305,9 @@ def test_retention_prompts(heads, dim, vdim, rot):
             if cut:
                 m.step([(s, t[:k], []) for s, t, k in zip(slots, ts, ks) if k])
             got = m.step([(s, t[k:], range(n - k)) for s, t, k, n in zip(slots, ts, ks, lens)])
-            e = U.logit_errors(got, torch.cat([x[k:] for x, k in zip(want, ks)])).sort().values
-            # bf16 through a layer: 7e-2, as in the tests of whole models; first tokens hang on the sign of q . k, one in a hundred rows may turn
-            assert float(e[-1 - len(e) // 100 - (cut == 0) * len(ts)]) < 7e-2, (lens, cut, e[-8:])
+            e = U.logit_errors(got, torch.cat([x[k:] for x, k in zip(want, ks)]))
+            # bf16 through a layer: 7e-2 at every row, as in the tests of whole models (first tokens hang on q . k, which is nowhere small enough here to turn its sign)
+            assert float(e.max()) < 7e-2, (lens, cut, e.sort().values[-8:])
             for s in slots:
                 m.close_sequence(s)
 
