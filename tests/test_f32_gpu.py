@@ -88,10 +88,14 @@ def forward(cfg, lens, context=192):
     return torch.cat(got), torch.cat([x[:-1] for x in want] + [x[-1:] for x in want])
 
 
-@pytest.mark.parametrize("m,n,k", [(380, 2048, 192), (385, 2048, 64), (129, 4224, 128), (145, 2880, 448), (65, 8256, 64), (449, 2048, 320)], ids=str)
+@pytest.mark.parametrize("m,n,k", [(380, 2048, 192), (385, 2048, 64), (129, 4224, 128), (145, 2880, 448), (65, 8256, 64), (449, 2048, 320),
+                                   (383, 2048, 384), (95, 8256, 192), (447, 2048, 256), (511, 2048, 1024)], ids=str)
 def test_tiles_of_48_and_64_rows(m, n, k):
-    """Tiles of 48 rows where they even out the CUs (380, 129, 145 rows), of 64 elsewhere, last tiles of one row and of all but one, K of one step: the bits of the kernel
-    that takes up to 32 rows, row by row, and fp32 rounding from 64 bits."""
+    """Tiles of 48 rows where they even out the CUs (380, 129, 145, 65, 383 and 95 rows: last tiles of 44, 33, 1, 17 and 47), of 64 elsewhere (385, 449, 447 and 511: of 1
+    and 63); K of one step of 64, of odd and even numbers of them, and of several sums of 128: the bits of the kernel that takes up to 32 rows, row by row, and fp32
+    rounding from 64 bits."""
+    rows, cols = -(-m // 64), n // 64  # (the rule beside lm_gemm_f32)
+    assert rows * cols > 128 and (-(-(-(-m // 48) * cols) // 256) * 48 * 22 < -(-rows * cols // 256) * 64 * 21) == (m in (380, 129, 145, 65, 383, 95))
     import ctypes as C
 
     from moondream_amd import _lib
