@@ -113,10 +113,11 @@ typedef struct {
  *                     accumulator, not always bitwise -- so a row's bits can depend on how many rows travel with it.
  *   MD_TILE_PINNED    the products and their order are a function of the layer (n, k) alone, never of m: every launch of more
  *                     than 64 rows takes the 256x256 kernel, or smaller tiles of the same bits where that leaves CUs without
- *                     work, so a sequence gets the same bits alone and in any batch.  The 256x256 kernel addresses a launch with 32-bit byte offsets (m * lda * 2 < 4 GiB, (m + 256) * ldc * 2 <
- *                     0xfffff000: ~150 000 rows of the 2B fused qkv|fc1 layer); a larger launch is cut into row blocks
- *                     of the same kernel (same bits), and one that cannot be cut -- a broadcast residual
- *                     (res_row_mod != 0), the RoPE epilogue -- returns MD_ERR_UNSUPPORTED instead of changing family.
+ *                     work, so a sequence gets the same bits alone and in any batch.  The 256x256 kernel addresses a launch
+ *                     with 32-bit byte offsets (m * lda * 2 < 4 GiB, (m + 256) * ldc * 2 < 0xfffff000: ~150 000 rows of the
+ *                     2B fused qkv|fc1 layer); a larger launch is cut into row blocks (same bits), and one that cannot be
+ *                     cut -- a broadcast residual (res_row_mod != 0), the RoPE epilogue -- returns MD_ERR_UNSUPPORTED
+ *                     instead of changing family.
  *   MD_TILE_DECODE_TALL  (round 6; set by md_decode_step / md_text_forward themselves for a decode step of 65 .. 128 sequences, accepted
  *                     from a caller of md_gemm_bf16 too) a launch of 65 .. 128 rows is a WEIGHT STREAM like the <= 64-row regime: one
  *                     128 x 64 tile per weight panel (four compute waves + two DMA waves), the same K order per output element as
@@ -245,15 +246,16 @@ md_status md_amax_bf16(const void* x, int64_t ldx, int32_t rows, int32_t cols, f
  * knobs at run time (the same knobs are read once from MD_GEMM_* / MD_DECODE_* environment
  * variables at first use).  PROCESS-WIDE and not thread-safe: for sweeps and A/B tests only; nothing that decides the
  * bits of a product call lives here (that is md_gemm_args.tile_policy, per call).  The complete key list:
- *   "tile"          -1 = automatic; 20 = four-wave 256x256, 11 / 15 = the eight-wave 256x256 baselines, 1 = 256x128,
- *                   2 = 128x128, 16 / 10 / 3 = decode-regime configs (forces the config for every launch)
+ *   "tile"          -1 = automatic; 20 = four-wave 256x256, 22 / 23 = 256x128 and 128x128 of the same bits, 2 = 128x128,
+ *                   16 / 10 / 3 = decode-regime configs (forces the config for every launch); 11 / 15 = the
+ *                   eight-wave 256x256 baselines, 1 = 256x128 of their family, never chosen by itself
  *   "small_m_rule"  tile rule of MD_TILE_BY_SHAPE launches: 1 (default) = round 5's (the 128x128 config for up to 512 tiles
  *                   of 128x128), 0 = round 2's (the cost model above 128 such tiles), n > 1 = n tiles instead of 512; same
  *                   bits either way
  *   "w4"            0: the eight-wave 256x256 kernels wherever the four-wave one would be picked (also under
  *                   MD_TILE_PINNED)
  *   "persist"       0: eight-wave kernels without their persistent tile loop
- *   "group_m"       row panels per tile-order group (0 = by shape)
+ *   "group_m"       row panels per tile-order group (0 = by shape; tiles 22 and 23 keep their own order)
  *   "decode_nt"     1: decode-regime weights streamed non-temporally
  *   "decode_cfg"    16 (default) / 10 / 3: decode-regime tile config
  *   "decode_slices" K slices per decode-regime tile (0 = by shape)

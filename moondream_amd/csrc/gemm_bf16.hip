@@ -721,7 +721,7 @@ template <int EPI>
 md_status launch_epi(const GemmK& k, int tile, hipStream_t stream) {
   switch (tile) {
     case 20: return md_gemm_w4_launch(k, EPI, stream);                              // 256x256, four waves (gemm_w4.hip)
-    case 1: return launch_cfg<256, 128, 4, 2, EPI, false, 3>(k, stream);
+    case 1: return launch_cfg<256, 128, 4, 2, EPI, false, 3>(k, stream);  // only forced ("tile"): 22 is faster wherever it was chosen
     case 3: return k.slices > 1 ? launch_cfg<64, 128, 1, 2, EPI, true, DEC_STAGES>(k, stream)
                                 : launch_cfg<64, 128, 1, 2, EPI, false, DEC_STAGES>(k, stream);
     // decode regime, 64x64 tiles: twice the tiles of 64x128 -> the wide fused layer needs no
@@ -1181,6 +1181,7 @@ md_status md_gemm_silu_bf16(const void* a, int64_t lda, const md_linear& lin, vo
     case 11: return launch_cfg<256, 256, 2, 4, MD_EPI_SILU, false, 4, 32, 2>(k, s);
     case 21: return launch_cfg<128, 64, 4, 1, MD_EPI_SILU, false, 4, 64, 0, 2>(k, s);
     case 16: return launch_cfg<64, 64, 2, 1, MD_EPI_SILU, false, 4, 64, 0, 2>(k, s);
+    case 1: return launch_cfg<256, 128, 4, 2, MD_EPI_SILU, false, 3>(k, s);  // only forced
     case 22: return md_gemm_mid_launch(k, MD_EPI_SILU, 256, s);
     case 23: return md_gemm_mid_launch(k, MD_EPI_SILU, 128, s);
     default:

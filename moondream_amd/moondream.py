@@ -322,9 +322,9 @@ class MoondreamModel(DeviceEngine):
     def _select_kernels(self, n_sequences: int):
         """The library's tile choice by row count would give a lone image (730 / 1458 rows) the small-shape tile configs and a
         batch the four-wave kernel, whose 16x16x32 MFMAs sum K in another association.  Every call is therefore made with the
-        tile config PINNED to the layer shape (``tile_policy = MD_TILE_PINNED`` in THIS model's ``md_vit_model`` /
-        ``md_text_model`` structs, read by the library per call: ABI 5; no process-wide state, so two models or threads in
-        one process do not affect each other's bits) -- so that ``batch_generate_ids(B)[i] == batch_generate_ids([x_i])``
+        products PINNED to the layer shape -- that kernel, or smaller tiles of its bits where it would leave compute units
+        without work -- (``tile_policy = MD_TILE_PINNED`` in THIS model's ``md_vit_model`` / ``md_text_model`` structs, read by
+        the library per call: ABI 5; no process-wide state, so two models or threads in one process do not affect each other's bits) -- so that ``batch_generate_ids(B)[i] == batch_generate_ids([x_i])``
         holds bit for bit in the DEFAULT mode as long as the lone sequence runs on the batched kernels -- except the
         documented latency path: ONE sequence with ``single_sequence_kernel`` on (small-shape tiles at prefill, the persistent
         kernel at decode).  Called by every public entry point that can launch a GEMM of more than 64 rows."""

@@ -156,9 +156,9 @@ def test_decode_steps_of_many_columns_round_as_the_64_row_regime(lib, n, k):
 
 
 def test_tile_policy_is_a_per_call_field(lib, force_tile):
-    """ABI 5: md_gemm_args.tile_policy.  MD_TILE_PINNED makes the tile config of a > 64-row launch a function of the layer alone --
-    the 256 x 256 kernel whatever the row count -- so a row gets the same bits in a 100-row and in a 5000-row launch; MD_TILE_BY_SHAPE
-    lets small launches take the small-shape configs (another MFMA shape: equal to fp32 rounding, not bitwise).  The policy travels
+    """ABI 5: md_gemm_args.tile_policy.  MD_TILE_PINNED makes the products of a > 64-row launch and their order a function of the layer alone --
+    the 256 x 256 kernel, or smaller tiles of its bits (100 rows: 128 x 128; 2940: 256 x 128) -- so a row gets the same bits in a 100-row and in a
+    5000-row launch; MD_TILE_BY_SHAPE lets small launches take the small-shape configs (another MFMA shape: equal to fp32 rounding, not bitwise).  The policy travels
     with the call: two interleaved callers with different policies do not affect each other, the "w4" A/B knob is honoured under the
     pin, launches of <= 64 rows ignore it, and an unknown value is refused."""
     k, n = 2048, 2048
@@ -168,13 +168,14 @@ def test_tile_policy_is_a_per_call_field(lib, force_tile):
     small = big[:100].contiguous()
     pinned_big = gemm(lib, big, lin, tile_policy=_lib.MD_TILE_PINNED)
     force_tile(20)
-    assert torch.equal(gemm(lib, big, lin), pinned_big)           # the pin IS the four-wave kernel
+    assert torch.equal(gemm(lib, big, lin), pinned_big)           # the pin at 5000 rows IS the four-wave kernel
     force_tile(-1)
     for rep in range(3):  # interleaved callers
         p_small = gemm(lib, small, lin, tile_policy=_lib.MD_TILE_PINNED)
         s_small = gemm(lib, small, lin, tile_policy=_lib.MD_TILE_BY_SHAPE)
         assert torch.equal(p_small, pinned_big[:100])             # same bits alone and in the big launch
         compare("by-shape vs pinned", s_small, p_small, 3e-4, 2e-2)
+    assert torch.equal(gemm(lib, big[:2940].contiguous(), lin, tile_policy=_lib.MD_TILE_PINNED), pinned_big[:2940])
     _lib.check(lib.md_gemm_set_tuning(b"w4", 0))
     try:
         eight = gemm(lib, small, lin, tile_policy=_lib.MD_TILE_PINNED)
