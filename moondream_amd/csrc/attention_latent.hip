@@ -132,6 +132,8 @@ __device__ __forceinline__ md_bf16x8v op(const u32x4& v) { return __builtin_bit_
 // Whole passes of 8 layers, one group and two: 16 heads of 128, one prompt of 700 tokens 771 and 757 us (28 and 24 a launch), 1000 890 : 837, 2000 1293 : 1179; 4 heads
 // of 64, 1000 757 : 702, 3 x 2000 1512 : 1407.  Not for up to three tiles (7 x 100, 16 heads 684 : 690, 4 heads 556 : 590) and not past a workgroup per CU (32 heads,
 // 2000 1222 : 1266).  Two groups of two waves and blocks of 64 queries: as one group or slower, each tile's loads and LDS writes serve half as many queries.
+// The rule counts the workgroups and keys of the step, so a prompt's rounding hangs on the prompts beside it.  Against 64 bits, one group and two: 16 heads of 128, 700 tokens 2.03e-3
+// and 2.00e-3 (sharp scores 1.89e-3, 1.80e-3), 4 of 64, 2000 tokens 2.08e-3 and 2.05e-3 (1.97e-3, 1.88e-3): weights are bf16, either way.
 constexpr int value_stride(int vp) { return vp == 32 ? 32 : vp == 128 ? 160 : 96; }  // four rows of 64 bytes fall on different banks
 template <int D, int C, int KG>
 struct PrefillLds {
