@@ -121,7 +121,6 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ u32x2 read_tr(const bf16_t* p) {  // lane i of a 16-lane group: four rows of column i % 16 (see read_columns)
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p));
 }
-__device__ __forceinline__ md_bf16x8v op(const u32x4& v) { return __builtin_bit_cast(md_bf16x8v, v); }
 
 // Four waves of 32 queries of one (sequence, head); keys and values stream through LDS in tiles of 64, two buffers, the next tile's loads in
 // registers meanwhile.  S^T = K Q^T (32x32x16), so a lane holds one query and 16 of every 32 keys: maximum and sum stay in the lane but for

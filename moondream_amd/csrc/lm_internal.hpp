@@ -85,6 +85,16 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 __device__ __forceinline__ float block_sum_256(float v, float* red) { return block_sum<4>(v, red); }
 
 typedef __bf16 md_bf16x8v __attribute__((ext_vector_type(8)));  // what the gfx950 MFMA builtins take
+__device__ __forceinline__ md_bf16x8v op(const u32x4& v) { return __builtin_bit_cast(md_bf16x8v, v); }
+__device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x4& c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(op(a), op(b), c, 0, 0, 0); }
+// fp32 as the sum of two bf16 (16 mantissa bits)
+__device__ __forceinline__ void split8(const float (&v)[8], u32x4& hi, u32x4& lo) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    hi[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
+    lo[i] = pack_bf16x2(v[2 * i] - lo_bf(hi[i]), v[2 * i + 1] - hi_bf(hi[i]));
+  }
+}
 
 // ---- cache layout: keys and values in the order the matrix instructions take them -------------------------------------------
 // A slot is a run of blocks of 32 positions, each holding all heads one after the other (a workgroup that reads all heads of a tile

@@ -156,18 +156,6 @@ namespace {
 
 __device__ __forceinline__ float pow_int(float log2_decay, int n) { return n == 0 ? 1.0f : __builtin_amdgcn_exp2f(log2_decay * (float)n); }
 
-__device__ __forceinline__ void split8(const float (&v)[8], u32x4& hi, u32x4& lo) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    hi[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
-    lo[i] = pack_bf16x2(v[2 * i] - lo_bf(hi[i]), v[2 * i + 1] - hi_bf(hi[i]));
-  }
-}
-__device__ __forceinline__ md_bf16x8v as_op(const u32x4& v) { return __builtin_bit_cast(md_bf16x8v, v); }
-__device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x4& c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_op(a), as_op(b), c, 0, 0, 0);
-}
-
 constexpr int RC = LM_RET_CHUNK;
 
 // chunks of a sequence before its last segment

@@ -303,16 +303,6 @@ md_status plain(const LmSsm& a, hipStream_t s) {
 // ---------------------------------------------------------------------------------------------------------------------------
 constexpr float LOG2E = 1.4426950408889634f;
 
-__device__ __forceinline__ md_bf16x8v op(const u32x4& v) { return __builtin_bit_cast(md_bf16x8v, v); }
-__device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x4& c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(op(a), op(b), c, 0, 0, 0); }
-__device__ __forceinline__ void split8(const float (&v)[8], u32x4& hi, u32x4& lo) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    hi[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
-    lo[i] = pack_bf16x2(v[2 * i] - lo_bf(hi[i]), v[2 * i + 1] - hi_bf(hi[i]));
-  }
-}
-
 constexpr int L = LM_SSM_CHUNK;
 
 // grid (heads, segments, sequences), four waves; a wave owns 16 tokens of the outputs and C * D 16 x 16 tiles of the state.
