@@ -635,7 +635,7 @@ md_status md_lm_head(const md_text_model* m, const void* hidden, int32_t batch, 
  * moondream.py:183-192 -> text.py:128-160, at batch 1).  x_in / hidden: bf16 [dim]; kv: the sequence's slot
  * (k / v pointing at its batch entry); sync_state: >= 16 KiB of device memory owned by the caller, ZERO before first
  * use and written by nothing else (barrier counters carry over from launch to launch; word 704 is raised if a
- * barrier ever timed out).  fp32 matrix-vector products and per-slice softmax maxima: the same tolerance against the
+ * wait ever timed out); the workspace may hold anything.  fp32 matrix-vector products and per-slice softmax maxima: the same tolerance against the
  * reference as the batched kernels, not bit-identical to them.  Needs the fused qkv|fc1 packing and n_kv_heads ==
  * n_heads, head_dim 64. */
 size_t md_decode_b1_workspace_bytes(const md_text_model* m);

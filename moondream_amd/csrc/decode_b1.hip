@@ -19,6 +19,15 @@
 // Activations that cross workgroups (x, qkv|fc1 row, attention partials) move through global memory with agent-scope
 // atomic loads / stores (L2-bypassing: the 8 XCDs have private L2s), so the barriers need no cache write-back.
 //
+// Rows are their own flags: the residual stream and the fused row are words of two values and the block they belong to, and who needs them reads until
+// they are there.  The one barrier of a block is the one between attention partials and their combination, whose wait lies behind the fc2 rows.  Between
+// phase A and B a workgroup waits for its head's q, k and v only, which are the first rows that every workgroup makes, and for the rest of the row behind
+// its attention.  2B, one token at 760 keys, blocks only: 699 us with three barriers a block, 657 so (13.8 us of a block's 27 are its 101 MB at
+// the rate of a large read; the rest is latency: two round trips per hand-over, and stragglers of phase A, 12 us where the median wave takes 9).
+// Tried beside it and slower: non-temporal weights (+1 %), rings of two chunks (+7 %) or four rows (+14 %), row pairs dealt by tickets between
+// workgroups (+2 to 5 %), attention in four waves while the others go on with fc1 (+1 %) or in four further waves (+7 %): under a saturated memory every
+// hand-over takes 2 to 3 us instead of one.
+//
 // Numerics: fp32 dot products in a different association than the MFMA kernels (lane-strided partial sums + a wave
 // butterfly), softmax with per-slice maxima (flash-decoding) -- within the same tolerance of the reference as the
 // batched path, not bit-identical to it.  Weights: the SAME packed row-major bf16 matrices as every other kernel.
@@ -47,17 +56,17 @@ struct B1Args {
   int64_t layer_stride;
   const int32_t* pos;
   const bf16_t* x_first;  // the first block's input (nullptr: row token[0] of wte)
-  bf16_t* x[2];           // residual stream between blocks, ping-pong
-  bf16_t* x_last;         // the last block's output (nullptr: x[n_layers & 1])
+  uint64_t* x[2];         // residual stream between blocks, ping-pong: tagged pairs, [dim / 2]
+  bf16_t* x_last;         // the last block's output where no head follows
   // whole decode step (lm_w != nullptr): embedding lookup in front, final layer norm + lm_head + greedy choice behind
   const int32_t* token;
   const bf16_t *wte, *post_ln_w, *post_ln_b, *lm_w, *lm_b;
   int ld_lm, vocab, suppress;
   bf16_t* logits;
   int32_t *next, *pos_out;
-  bf16_t* act;       // [qkv_w + ff]: the fused linear's output row
+  uint64_t* act;     // the fused linear's output row: tagged pairs, [(qkv_w + ff) / 2]
   float* part;       // [n_heads][B1_SLICES][B1_PART]
-  unsigned* sync;    // [0] epoch, [64 (1 + xcd)] per-XCD arrivals, [64 * 9] top-level arrivals, [64 * 10] flag, [64 * 11] error
+  unsigned* sync;    // see GridBarrier
   float eps, scale_log2;
 };
 
@@ -79,6 +88,16 @@ __device__ __forceinline__ u32x4 ld_coh128(__amdgpu_buffer_rsrc_t r, int byte_of
 __device__ __forceinline__ void st_coh32(void* p, uint32_t v) {
   __hip_atomic_store((uint32_t*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ void st_coh64(void* p, uint64_t v) {
+  __hip_atomic_store((uint64_t*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Rows that cross workgroups without a barrier: two bf16 values and, in the upper half of the same 8-byte word, the block they belong to.  Who needs
+// a row reads it until every tag is the block's.  Against a barrier that saves the acknowledgement of the stores, the flag and the wait for those
+// whose rows are not needed.
+__device__ __forceinline__ void st_pair(uint64_t* p, uint32_t pair, unsigned tag) { st_coh64(p, (uint64_t)tag << 32 | pair); }
+// two words
+__device__ __forceinline__ bool is_block(const u32x4& v, unsigned tag) { return v[1] == tag && v[3] == tag; }
 
 // Grid barrier without atomics: workgroup b publishes the barrier's number in ITS word of a flag array once its stores
 // are acknowledged; everybody polls the whole array (one 4-byte coherent load per lane, gridDim / 64 waves) until every
@@ -119,6 +138,17 @@ struct GridBarrier {
       }
     }
     __syncthreads();
+  }
+  // repeats look(), a load of tagged words and the check of their tags, until it holds for all active lanes
+  template <class F>
+  __device__ __forceinline__ void until(F look) {
+    for (unsigned spins = 0; !__all(look()); ++spins) {
+      if (spins > B1_SPIN_LIMIT) {
+        __hip_atomic_store(sync + 64 * 11, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
   }
 };
 
@@ -220,11 +250,12 @@ __global__ __launch_bounds__(64 * NWV) void decode_b1_kernel(const B1Args p) {
   __shared__ float sc[B1_MAX_KEYS];
   __shared__ float head_m[64 * B1_SLICES], head_l[64 * B1_SLICES];  // phase C: slice statistics of every head
   __shared__ __attribute__((aligned(16))) bf16_t newrow[3][64];      // phase B: rotated q, rotated k, v of the new token
+  __shared__ uint32_t rawrow[3][32];                                 // ... and before the rotation, in pairs
   __shared__ float fc2_part[B1_MAX_Q][2][2];                         // fc2 dot products: [pair of the workgroup][K half][row]
   __shared__ float proj_part[NWV / 2][2][2];
   __shared__ int best_i[NWV];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   constexpr int NT = 64 * NWV;
   GridBarrier bar{p.sync, ld_coh32(p.sync)};
   // measurement hook: with word 768 of the sync state non-zero, workgroup 0 stamps the 100 MHz real-time counter at
@@ -292,16 +323,33 @@ __global__ __launch_bounds__(64 * NWV) void decode_b1_kernel(const B1Args p) {
     }
   };
   prime_first(npw_a, p.layer[0].w1, p.ld1);
+  // the workspace may hold anything: this workgroup's words of the residual stream get a tag that no block of this launch has.  (The fused row's
+  // are written by the first block, behind which every workgroup waits for all others.)
+  for (int q = tid; q < npw_c; q += NT) {
+    const int pc = blockIdx.x + gridDim.x * q;
+    st_pair(p.x[0] + pc, 0u, bar.base);
+    st_pair(p.x[1] + pc, 0u, bar.base);
+  }
 
-  // layer norm of the residual stream (every workgroup, redundantly) -> lds_row
-  auto layer_norm_to_lds = [&](const bf16_t* xsrc, const bf16_t* lnw, const bf16_t* lnb) {
+  // layer norm of the residual stream (every workgroup, redundantly) -> lds_row; tag: of the block that left it (the launch's epoch: the first block's plain input)
+  auto layer_norm_to_lds = [&](const void* xsrc, unsigned tag, const bf16_t* lnw, const bf16_t* lnb) {
     float v[8];
     float sum = 0.f;
     const int nch = D >> 3;
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = 0.f;
     if (tid < nch) {
-      const u32x4 q = ld_coh128(coh_rsrc(xsrc), tid * 16);
+      u32x4 q;
+      const __amdgpu_buffer_rsrc_t r_x = coh_rsrc(xsrc);
+      if (tag == bar.base) {
+        q = ld_coh128(r_x, tid * 16);
+      } else {
+        bar.until([&] {
+          const u32x4 lo = ld_coh128(r_x, tid * 32), hi = ld_coh128(r_x, tid * 32 + 16);
+          q = u32x4{lo[0], lo[2], hi[0], hi[2]};
+          return is_block(lo, tag) && is_block(hi, tag);
+        });
+      }
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         v[2 * e] = lo_bf(q[e]);
@@ -350,14 +398,15 @@ __global__ __launch_bounds__(64 * NWV) void decode_b1_kernel(const B1Args p) {
   };
   const int n_items = p.n_heads * B1_SLICES;
 
-  const bf16_t* xc = p.x_first;
-  if (!xc) xc = p.wte + (int64_t)min(max(p.token[0], 0), p.vocab - 1) * D;
+  const bf16_t* x_plain = p.x_first;
+  if (!x_plain) x_plain = p.wte + (int64_t)min(max(p.token[0], 0), p.vocab - 1) * D;
   for (int l = 0; l < p.n_layers; ++l) {
     const B1Layer& w = p.layer[l];
-    bf16_t* xn = (l + 1 == p.n_layers && p.x_last) ? p.x_last : p.x[(l + 1) & 1];
+    const unsigned tag = bar.base + 1 + l;  // (the launch's barriers number more than its blocks: the next one's tags are others)
+    const uint64_t* xc = p.x[l & 1];
 
     // ================= phase A: layer norm + fused [qkv | fc1] rows ===================================================
-    layer_norm_to_lds(xc, w.ln_w, w.ln_b);
+    layer_norm_to_lds(l == 0 ? (const void*)x_plain : (const void*)xc, tag - 1, w.ln_w, w.ln_b);
     run_rows(npw_a, w.w1, p.ld1, w.b1, [&](int pp, float d0, float d1, uint32_t bw) {
       if (lane == 0) {
         uint32_t o = pack_bf16x2(d0 + lo_bf(bw), d1 + hi_bf(bw));  // F.linear's rounding point
@@ -365,11 +414,11 @@ __global__ __launch_bounds__(64 * NWV) void decode_b1_kernel(const B1Args p) {
           const md_f32x2 gl = gelu_tanh_f32x2(md_f32x2{lo_bf(o), hi_bf(o)});
           o = pack_bf16x2(gl[0], gl[1]);
         }
-        st_coh32(p.act + 2 * pp, o);
+        st_pair(p.act + pp, o, tag);
       }
     });
     stamp();
-    bar.arrive();
+    if (l == 0) bar.arrive();
     u32x4 kq[KPT], vq[KPT];
     if ((int)blockIdx.x < n_items) {
       load_kv(l, blockIdx.x, kq, vq);
@@ -377,22 +426,21 @@ __global__ __launch_bounds__(64 * NWV) void decode_b1_kernel(const B1Args p) {
 #pragma unroll
       for (int i = 0; i < KPT; ++i) kq[i] = vq[i] = u32x4{0u, 0u, 0u, 0u};
     }
-    bar.wait();
+    if (l == 0) bar.wait();  // (from here on no word holds a tag of this launch that was not written by it)
     stamp();
 
     // ================= phase B: attention partials, one (head, key slice) per workgroup; then the fc2 rows ============
     // gelu(fc1) -> LDS for the fc2 rows: requested now, parked in LDS after the attention slice (the latency of these
     // loads runs under it)
-    constexpr int NFQ = B1_MAX_FF / 8 / NT > 0 ? B1_MAX_FF / 8 / NT : 1;
+    constexpr int NFQ = B1_MAX_FF / 4 / NT > 0 ? B1_MAX_FF / 4 / NT : 1;
     u32x4 ffq[NFQ];
-    {
-      const __amdgpu_buffer_rsrc_t r_ff = coh_rsrc(p.act + QW);
+    const __amdgpu_buffer_rsrc_t r_ff = coh_rsrc(p.act + (QW >> 1));
+    auto load_ff = [&](int i) {
+      const int ch = tid + NT * i;
+      ffq[i] = ld_coh128(r_ff, (ch < (FF >> 2) ? ch : 0) * 16);
+    };
 #pragma unroll
-      for (int i = 0; i < NFQ; ++i) {
-        const int ch = tid + NT * i;
-        ffq[i] = ld_coh128(r_ff, (ch < (FF >> 3) ? ch : 0) * 16);
-      }
-    }
+    for (int i = 0; i < NFQ; ++i) load_ff(i);
     for (int idx = blockIdx.x; idx < n_items; idx += gridDim.x) {
       const int h = idx / B1_SLICES, sl = idx % B1_SLICES;
       const int j0 = sl * chunk, j1 = min(L, j0 + chunk);
@@ -405,17 +453,23 @@ __global__ __launch_bounds__(64 * NWV) void decode_b1_kernel(const B1Args p) {
         continue;
       }
       if (idx != (int)blockIdx.x) load_kv(l, idx, kq, vq);
+      if (tid < 96) {  // this head's rows of the fused product, which were the first ones that their workgroups made
+        const uint64_t* from = p.act + ((tid >> 5) * p.n_heads + h) * 32 + (tid & 31);
+        uint64_t v;
+        bar.until([&] {
+          v = ld_coh64(from);
+          return (unsigned)(v >> 32) == tag;
+        });
+        rawrow[tid >> 5][tid & 31] = (uint32_t)v;
+      }
+      __syncthreads();
       // rotated q (every slice needs it) and, for the slice that holds the new position, rotated k and v (rope.py:20-48)
       {
         const int hr = p.rot >> 1;
-        auto act_at = [&](int col) -> float {  // one bf16 of the fused row, through a coherent 4-byte load
-          const uint32_t wv = ld_coh32(p.act + (col & ~1));
-          return (col & 1) ? hi_bf(wv) : lo_bf(wv);
-        };
+        auto raw_at = [&](int which, int i) -> float { return (i & 1) ? hi_bf(rawrow[which][i >> 1]) : lo_bf(rawrow[which][i >> 1]); };
         if (tid < 2 * hr) {
           const int which = tid / hr, j = tid % hr;
-          const int base = (which ? (p.n_heads + h) : h) * 64;
-          const float re = act_at(base + j), im = act_at(base + hr + j);
+          const float re = raw_at(which, j), im = raw_at(which, hr + j);
           const float cs = p.freqs[((int64_t)pos * hr + j) * 2], sn = p.freqs[((int64_t)pos * hr + j) * 2 + 1];
           float o_re, o_im;
           md_rope_pair(re, im, cs, sn, o_re, o_im);
@@ -423,9 +477,9 @@ __global__ __launch_bounds__(64 * NWV) void decode_b1_kernel(const B1Args p) {
           newrow[which][2 * j + 1] = f2bf(o_im);
         } else if (tid >= 64 && tid < 64 + 2 * (64 - p.rot)) {
           const int t2 = tid - 64, which = t2 / (64 - p.rot), i = p.rot + t2 % (64 - p.rot);
-          newrow[which][i] = f2bf(act_at((which ? (p.n_heads + h) : h) * 64 + i));
+          newrow[which][i] = f2bf(raw_at(which, i));
         } else if (tid >= 192 && tid < 256) {
-          newrow[2][tid - 192] = f2bf(act_at((2 * p.n_heads + h) * 64 + tid - 192));
+          newrow[2][tid - 192] = f2bf(raw_at(2, tid - 192));
         }
       }
       __syncthreads();
@@ -504,10 +558,16 @@ __global__ __launch_bounds__(64 * NWV) void decode_b1_kernel(const B1Args p) {
 #pragma unroll
     for (int i = 0; i < NFQ; ++i) {
       const int ch = tid + NT * i;
-      if (ch < (FF >> 3)) *(u32x4*)(lds_ff + 16 * ch) = ffq[i];
+      if (!__all(is_block(ffq[i], tag)))
+        bar.until([&] {
+          load_ff(i);
+          return is_block(ffq[i], tag);
+        });
+      if (ch < (FF >> 2)) *(uint2*)(lds_ff + 8 * ch) = uint2{ffq[i][0], ffq[i][2]};
     }
     stamp();
     bar.arrive();  // (also publishes lds_ff to every wave)
+    auto residual = [&](int pc) { return l == 0 ? ld_coh32(x_plain + 2 * pc) : (uint32_t)ld_coh64(xc + pc); };  // (every tag of it has been seen)
     // fc2 needs gelu(fc1), not the attention: its rows stream while the barrier collects the attention partials
     const bf16_t *prow[2], *frow[2];
     int kp = 0, kf = 0;
@@ -551,7 +611,7 @@ __global__ __launch_bounds__(64 * NWV) void decode_b1_kernel(const B1Args p) {
     uint32_t xo0 = 0, bpw0 = 0, b2w0 = 0;
     if (tid < PPP && tid < npw_c) {
       const int pc = blockIdx.x + gridDim.x * tid;
-      xo0 = ld_coh32(xc + 2 * pc);
+      xo0 = residual(pc);
       bpw0 = *(const uint32_t*)(w.bp + 2 * pc);
       b2w0 = *(const uint32_t*)(w.b2 + 2 * pc);
     }
@@ -618,32 +678,27 @@ __global__ __launch_bounds__(64 * NWV) void decode_b1_kernel(const B1Args p) {
           const float dp0 = proj_part[tid][0][0] + proj_part[tid][1][0], dp1 = proj_part[tid][0][1] + proj_part[tid][1][1];
           const float df0 = fc2_part[q0 + tid][0][0] + fc2_part[q0 + tid][1][0];
           const float df1 = fc2_part[q0 + tid][0][1] + fc2_part[q0 + tid][1][1];
-          const uint32_t xo = q0 == 0 ? xo0 : ld_coh32(xc + 2 * pc);
+          const uint32_t xo = q0 == 0 ? xo0 : residual(pc);
           const uint32_t bpw = q0 == 0 ? bpw0 : *(const uint32_t*)(w.bp + 2 * pc), b2w = q0 == 0 ? b2w0 : *(const uint32_t*)(w.b2 + 2 * pc);
           const uint32_t t1 = pack_bf16x2(dp0 + lo_bf(bpw), dp1 + hi_bf(bpw));
           const uint32_t x1 = pack_bf16x2(lo_bf(xo) + lo_bf(t1), hi_bf(xo) + hi_bf(t1));
           const uint32_t t2 = pack_bf16x2(df0 + lo_bf(b2w), df1 + hi_bf(b2w));
-          st_coh32(xn + 2 * pc, pack_bf16x2(lo_bf(x1) + lo_bf(t2), hi_bf(x1) + hi_bf(t2)));
+          const uint32_t x2 = pack_bf16x2(lo_bf(x1) + lo_bf(t2), hi_bf(x1) + hi_bf(t2));
+          if (l + 1 == p.n_layers && !p.lm_w) *(uint32_t*)(p.x_last + 2 * pc) = x2;
+          else st_pair(p.x[(l + 1) & 1] + pc, x2, tag);
         }
         __syncthreads();
       }
     }
     stamp();
-    const bool more = l + 1 < p.n_layers;
-    if (more || p.lm_w) {
-      bar.arrive();
-      // the next phase's first weight rows go out while the barrier collects arrivals
-      if (more) prime_first(npw_a, p.layer[l + 1].w1, p.ld1);
-      else prime_first(npw_d, p.lm_w, p.ld_lm);
-      bar.wait();
-    }
-    stamp();
-    xc = xn;
+    // the next phase's first weight rows go out while the residual stream's pairs are on their way
+    if (l + 1 < p.n_layers) prime_first(npw_a, p.layer[l + 1].w1, p.ld1);
+    else if (p.lm_w) prime_first(npw_d, p.lm_w, p.ld_lm);
   }
 
   // ================= phase D (whole decode step): final layer norm, lm_head rows, argmax ==============================
   if (p.lm_w) {
-    layer_norm_to_lds(xc, p.post_ln_w, p.post_ln_b);
+    layer_norm_to_lds(p.x[p.n_layers & 1], bar.base + p.n_layers, p.post_ln_w, p.post_ln_b);
     float best = -INFINITY;
     int bi = 0x7fffffff;
     run_rows(npw_d, p.lm_w, p.ld_lm, p.lm_b, [&](int pp, float d0, float d1, uint32_t bw) {
@@ -722,7 +777,7 @@ __global__ __launch_bounds__(64 * NWV) void decode_b1_kernel(const B1Args p) {
 extern "C" size_t md_decode_b1_workspace_bytes(const md_text_model* m) {
   if (!m || !m->blocks) return 0;
   const size_t dim = m->dim, ffp = m->blocks[0].fc1.n_pad;
-  return 2 * ((dim * 2 + 255) / 256 * 256) + ((3 * dim + ffp) * 2 + 255) / 256 * 256 +
+  return 2 * ((dim * 4 + 255) / 256 * 256) + ((3 * dim + ffp) * 4 + 255) / 256 * 256 +
          ((size_t)m->n_heads * B1_SLICES * B1_PART * 4 + 255) / 256 * 256;
 }
 
@@ -755,10 +810,10 @@ md_status b1_fill(const md_text_model* m, const md_kv_cache* kv, const int32_t* 
   a.layer_stride = kv->layer_stride;
   a.pos = pos;
   char* ws = (char*)workspace;
-  const size_t xb = ((size_t)m->dim * 2 + 255) / 256 * 256, ab = ((size_t)(3 * m->dim + b0.fc1.n_pad) * 2 + 255) / 256 * 256;
-  a.x[0] = (bf16_t*)ws;
-  a.x[1] = (bf16_t*)(ws + xb);
-  a.act = (bf16_t*)(ws + 2 * xb);
+  const size_t xb = ((size_t)m->dim * 4 + 255) / 256 * 256, ab = ((size_t)(3 * m->dim + b0.fc1.n_pad) * 4 + 255) / 256 * 256;
+  a.x[0] = (uint64_t*)ws;
+  a.x[1] = (uint64_t*)(ws + xb);
+  a.act = (uint64_t*)(ws + 2 * xb);
   a.part = (float*)(ws + 2 * xb + ab);
   a.sync = (unsigned*)sync_state;
   a.eps = 1e-5f;
@@ -847,11 +902,11 @@ extern "C" md_status md_decode_b1_layers(const md_text_model* m, const void* x_i
   MD_TRY(b1_fill(m, kv, pos, workspace, sync_state, a));
   a.x_first = (const bf16_t*)x_in;
   // (x_in == hidden is allowed: with one block the in-place update would race, so only then go through the workspace)
-  a.x_last = (m->n_layers > 1 || x_in != hidden) ? (bf16_t*)hidden : nullptr;
+  const bool copy = m->n_layers == 1 && x_in == hidden;
+  a.x_last = copy ? (bf16_t*)a.x[1] : (bf16_t*)hidden;  // (with one block nothing else uses it)
   hipStream_t s = (hipStream_t)stream;
   MD_TRY(b1_launch(m, a, s));
-  if (!a.x_last && hipMemcpyAsync(hidden, a.x[m->n_layers & 1], (size_t)m->dim * 2, hipMemcpyDeviceToDevice, s) != hipSuccess)
-    return MD_ERR_LAUNCH;
+  if (copy && hipMemcpyAsync(hidden, a.x_last, (size_t)m->dim * 2, hipMemcpyDeviceToDevice, s) != hipSuccess) return MD_ERR_LAUNCH;
   return MD_OK;
 }
 

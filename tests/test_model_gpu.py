@@ -949,6 +949,49 @@ def test_single_sequence_kernel_tracks_batched_kernels(tiny):
         model.single_sequence_kernel = True
 
 
+@pytest.mark.parametrize("dim, heads, ff, layers", [(128, 2, 64, 3), (256, 4, 704, 1), (1024, 16, 4096, 3), (2048, 32, 1024, 2)])
+def test_single_sequence_kernel_at_its_edges(dim, heads, ff, layers):
+    """Fewer row pairs than workgroups, one block, odd numbers of pairs per wave, a (head, slice) for every workgroup; a workspace that
+    holds words with the tags of the blocks to come.  Against the batched kernels at one row, three tokens in a row."""
+    import ctypes as C
+    import math
+    from dataclasses import replace
+
+    from moondream_amd.moondream import IdTokenizer, MoondreamModel
+
+    cfg = get_config("tiny")
+    cfg = replace(cfg, text=replace(cfg.text, dim=dim, n_heads=heads, n_kv_heads=heads, ff_dim=ff, n_layers=layers),
+                  vision=replace(cfg.vision, proj_out_dim=dim), region=replace(cfg.region, dim=dim))
+    model = MoondreamModel(cfg, synth.synthetic_state_dict(cfg, seed=3, device="cuda"), device="cuda", tokenizer=IdTokenizer())
+    model.use_graphs = False
+    enc = model.encode_image(synth.synthetic_image(5, 1))
+    prompt = list(cfg.tokenizer.templates["caption"]["normal"])
+    logits, rows = [], []
+    for flag in (False, True):
+        model.single_sequence_kernel = flag
+        model.load_encoded_image(enc)
+        _, _, pos = model._prefill_prompts([prompt], enc.pos, 0)
+        steps = []
+        for k, token in enumerate((17, 400, 401)):
+            if flag:
+                ws = model._workspace(model.lib.md_decode_step_b1_workspace_bytes(C.byref(model.w.text)), 2)
+                ws = ws[: ws.numel() // 8 * 8].view(torch.int32)
+                epoch = 0 if model._b1_sync is None else int(model._b1_sync[0])
+                with torch.inference_mode():
+                    ws.copy_(epoch + 1 + torch.arange(ws.numel(), device="cuda", dtype=torch.int32) // 2 % (layers + 1))
+            model._decode_greedy(torch.tensor([token], dtype=torch.int32, device="cuda"), pos + k, 1, cfg.tokenizer.answer_id, 0, None)
+            assert model._b1_used is flag
+            steps.append(model._logits_buf[0].float().clone())
+        logits.append(torch.stack(steps))
+        rows.append(torch.stack([kv[:, 0, :, pos : pos + 3].float() for kv in (model._kv_k, model._kv_v)]))
+    assert int(model._b1_sync[64 * 11]) == 0, "a wait timed out"
+    # bf16 through up to three blocks: a rounding of 2^-8 in each of some six places a block, which add up as their squares do
+    bound = 2.0 ** -8 * math.sqrt(6 * layers)
+    for got, want in ((logits[1], logits[0]), (rows[1], rows[0])):
+        rel = float((got - want).norm() / want.norm())
+        assert rel <= bound, (rel, bound)
+
+
 def fp8_decode_report(model, images, prompts, ids_bf16, ref_margins, label):
     """Run the same generation with FP8 decode weights; the first decode step's logits (identical image prefix in the
     KV cache, identical input token) must stay within tolerance of the bf16 logits, and token streams may only leave the bf16 stream at
