@@ -9,7 +9,8 @@
 //   conv_state_kernel    the last projections of every sequence of the step -> its slot (row p % taps of the slot's ring)
 //   attn_plain_kernel    one workgroup per query row, fp32 on the vector ALUs: any dtype, any head size
 //   attn_mfma_kernel     bf16 prefill on the matrix cores: 16 queries x all heads per workgroup
-//   attn_decode_kernel   bf16 decode step: split-key attention behind attn_prep_kernel (made in every split, the convolution and norms
+//   attn_heads_*         bf16 decode step with one key head per query head: see there
+//   attn_decode_kernel   any other bf16 decode step: split-key attention behind attn_prep_kernel (made in every split, the convolution and norms
 //                        would be its longest chain of dependent loads)
 //   attn_combine_kernel  ... and the sum over the splits
 //
@@ -1021,7 +1022,7 @@ __host__ __device__ inline DecodeLds decode_lds(int H, int dp, int tk) {
 // head at a time; blocks past the last key are read (finite spare positions) and masked.
 // Few keys: what counts is the chain of dependent loads.  Splits of one block of 32 keys (up to 63 sequences in a graph) have tiles of their own: TK = 32 deals
 // the key heads to four pairs of waves and requests everything a wave reads, keys and values, before the queries are staged; the mixture's sum
-// over heads is shared by the halves of a wave.  32 heads of 64, one sequence at 100 keys: 11.8 us against 13.9 in tiles of 64, which read a block of
+// over heads is shared by the halves of a wave.  32 heads of 64 (which attn_heads_* take since), one sequence at 100 keys: 11.8 us against 13.9 in tiles of 64, which read a block of
 // values beyond the split, one key head batch after the other, and waited for each of what is staged (with the waits 13.0: a step of the 24-layer model 1104 us against 1120, with 16 heads of 128 1093
 // against 1119, 24 sequences at 1500 keys 2454 against 2529).
 template <int HPW, int D, int C, int TK>
@@ -1343,5 +1344,299 @@ md_status lm_attn_decode(const LmAttn& a, hipStream_t s) {
   MD_TRY(md_launch_status());
   if (a.n_split == 1) return MD_OK;
   hipLaunchKernelGGL(attn_combine_kernel, dim3(a.heads, a.r.n_seq), dim3(256), 0, s, a);
+  return md_launch_status();
+}
+
+// ---------------------------------------------------------------------------------------------------------------------------
+// A decode step in two launches instead of three, where a layer's own keys and values have one head per query head.  Few sequences are bound by chains of dependent
+// loads in a few workgroups, so all that can be is done beside another chain, and heads as well as keys go to different workgroups.
+//   attn_heads_scores_kernel  (256 columns of heads, 128 keys, sequence): convolution of its queries, their scores with the cached keys, heads unmixed; the
+//                             workgroup of the new position also makes its key, its value (-> cache) and the convolution state.  The norms' factors are taken out of
+//                             the products: every workgroup leaves the sums of squares of its columns
+//   attn_heads_mix_kernel     (head, 256 keys, sequence): mixture, softmax, weighted values; the last of a head's workgroups adds up their parts
+// The score of a head and key is one float, so the mixture's all-to-all costs 4 bytes, read by every head, beside the 4 dim of keys and values, read
+// once.  How many keys there are is known on the device only (a captured step sees any number): workgroups beyond the last key leave at once.
+// 32 heads of 64, one sequence at 100 keys: 6.6 and 5.8 us a layer against 5.1, 11.9 and 4.7; a step of two such layers and two of retention, before and now: 1 / 8
+// sequences at 100 keys 217 / 232 -> 200 / 217 us, 8 at 1500 269 -> 250, 32 at 100 / 500 / 1500 286 / 367 / 508 -> 274 / 314 / 420, 64 at 500 / 1500 642 / 706 -> 494 / 696, 128
+// at 20 / 1500 528 / 1131 -> 523 / 1090; 16 heads of 128 within 1 % of the same.  64 heads read 256 bytes of scores per key and head: 64 of 64, 40 sequences at 500 keys
+// 648 -> 585, but 64 at 1200 1068 -> 1177, hence the limit of many_heads.  Keys and values past the caches: 64 at 1200 2 to 3 % faster, 40 at 100 2 % slower.
+namespace {
+
+constexpr int HEADS_COLS = 256, HEADS_KEYS = 128, HEADS_SPAN = 256;
+
+struct HeadsPart {  // places in a.part, in floats
+  int keys;       // room for the keys of a sequence
+  int64_t raw, khat, sq, part, ticket, total;
+};
+__host__ __device__ inline HeadsPart heads_part(int n_seq, int span, int H, int dp, int vp) {
+  HeadsPart f;
+  const int splits = (span + 31 + HEADS_SPAN - 1) / HEADS_SPAN, groups = H * dp / HEADS_COLS;
+  f.keys = splits * HEADS_SPAN;
+  f.raw = 0;
+  f.khat = f.raw + (int64_t)n_seq * H * f.keys;
+  f.sq = f.khat + (int64_t)n_seq * H * dp;
+  f.part = f.sq + (int64_t)n_seq * 2 * groups;
+  f.ticket = f.part + (int64_t)n_seq * H * splits * (vp + 2);
+  f.total = f.ticket + (int64_t)n_seq * H;
+  return f;
+}
+
+template <int D>
+__global__ __launch_bounds__(256) void attn_heads_scores_kernel(const LmAttn a, const HeadsPart f) {
+  constexpr int dp = 32 * D, HG = HEADS_COLS / dp, TILES = HEADS_KEYS / 16 / 4;  // heads of a workgroup, key tiles of a wave
+  __shared__ __attribute__((aligned(16))) bf16_t qs[HEADS_COLS];
+  __shared__ float ks[HEADS_COLS], red[4];
+  const int H = a.heads, groups = H / HG, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n16 = lane & 15, q4 = lane >> 4;
+  const int seq = blockIdx.y, group = blockIdx.x % groups, split = blockIdx.x / groups;
+  const int row = a.r.seq_row0[seq], i = a.r.seq_pos0[seq], slot = a.r.seq_slot[seq];
+  const int base = (a.chunk > 0 ? i / a.chunk * a.chunk : 0) & ~31, k0 = base + split * HEADS_KEYS;
+  if (k0 > i) return;
+  const bool own = i < k0 + HEADS_KEYS;  // the new position's workgroup
+
+  // column c of a projection, convolved: the newest taps are requested together (rows before the sequence's first are read from somewhere else and not used)
+  const int c = group * HEADS_COLS + tid;
+  constexpr int TAPS = 4;
+  struct Column {
+    bf16_t u[TAPS];
+    float w[TAPS], norm;
+  };
+  const bf16_t* ring = (const bf16_t*)a.conv_state + (int64_t)slot * a.taps * a.conv_ld;
+  auto request = [&](int col0, const float* norm) {
+    Column x;
+    const int col = col0 + c;
+    const bf16_t* proj = (const bf16_t*)a.proj + (int64_t)row * a.ldp + col;
+#pragma unroll
+    for (int k = 0; k < TAPS; ++k) {
+      const bool in = k < a.taps && i - k >= 0;
+      x.u[k] = *(k > 0 && in ? ring + (int64_t)((i - k) % a.taps) * a.conv_ld + col : proj);
+      x.w[k] = a.conv[(int64_t)(in ? a.taps - 1 - k : 0) * a.conv_ld + col];
+    }
+    x.norm = norm ? norm[c] : 1.f;
+    return x;
+  };
+  auto convolve = [&](const Column& x) {
+    float y = 0.f;
+#pragma unroll
+    for (int k = TAPS - 1; k >= 0; --k)
+      if (k < a.taps && i - k >= 0) y += x.w[k] * bf2f(x.u[k]);
+    return y;
+  };
+  Column q = request(a.col_q, a.q_norm), kx, vx;
+  if (own) {
+    kx = request(a.col_k, a.k_norm);
+    vx = request(a.col_v, nullptr);
+  }
+  const bf16_t* Kb = (const bf16_t*)a.k + (int64_t)slot * H * a.ctx * dp;
+  u32x4 kf[TILES][HG][D];
+#pragma unroll
+  for (int t = 0; t < TILES; ++t) {
+    const int j = k0 + 16 * (wave + 4 * t);
+    if (j > i) continue;
+    const bf16_t* kw = Kb + key_block(j, group * HG, H, dp) + ((j >> 4) & 1) * (D * 512) + 8 * lane;
+#pragma unroll
+    for (int h = 0; h < HG; ++h)
+#pragma unroll
+      for (int d = 0; d < D; ++d) kf[t][h][d] = *(const u32x4*)(kw + h * (32 * dp) + 512 * d);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  const float y = convolve(q);
+  qs[tid] = f2bf(y * q.norm);
+  float* sq = a.part + f.sq + (int64_t)seq * 2 * groups + group;
+  if (own) {
+    const float k = convolve(kx), v = convolve(vx);
+    const float qq = block_sum_256(y * y, red), kk = block_sum_256(k * k, red);
+    if (tid == 0) {
+      sq[0] = qq;
+      sq[groups] = kk;
+    }
+    ks[tid] = k * kx.norm;
+    a.part[f.khat + (int64_t)seq * H * dp + c] = k * kx.norm;
+    float r = 1.0f;
+    if (a.value_norm) {
+      float s = v * v;
+#pragma unroll
+      for (int o = (dp < 64 ? dp : 64) / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+      if (dp == 128) {
+        __syncthreads();
+        if (lane == 0) red[wave] = s;
+        __syncthreads();
+        s = red[wave] + red[wave ^ 1];
+      }
+      r = 1.0f / sqrtf(s / (float)a.vdim + a.eps);
+    }
+    const int g = c / dp, e = c % dp;
+    ((bf16_t*)a.v)[(int64_t)slot * a.ctx * H * dp + value_index(i, g, e, H, dp)] = f2bf(v * r);
+    if (a.taps > 1) {
+      bf16_t* to = (bf16_t*)a.conv_state + ((int64_t)slot * a.taps + i % a.taps) * a.conv_ld + c;
+      to[a.col_q] = q.u[0];
+      to[a.col_k] = kx.u[0];
+      to[a.col_v] = vx.u[0];
+    }
+    if (tid < HG) ((unsigned*)(a.part + f.ticket))[seq * H + group * HG + tid] = 0u;
+  }
+  __syncthreads();
+  float* raw = a.part + f.raw + ((int64_t)seq * H + group * HG) * f.keys + (k0 - base);  // [head][key]
+#pragma unroll
+  for (int t = 0; t < TILES; ++t) {
+    const int at = 16 * (wave + 4 * t);
+    if (k0 + at > i) continue;
+    f32x4 mine = {0.f, 0.f, 0.f, 0.f};  // lane n16 keeps head n16's (the product's columns are all the same query)
+#pragma unroll
+    for (int h = 0; h < HG; ++h) {
+      f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int d = 0; d < D; ++d) s = mfma(kf[t][h][d], *(const u32x4*)(qs + h * dp + 32 * d + 8 * q4), s);
+      if (n16 == h) mine = s;
+    }
+    if (n16 >= HG) continue;
+    float* to = raw + (int64_t)n16 * f.keys + at + 4 * q4;
+    const int left = i - (k0 + at + 4 * q4);  // keys of these four before the new one
+    if (left >= 4) {
+      *(f32x4*)to = mine * a.scale;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (e < left) to[e] = mine[e] * a.scale;
+    }
+  }
+  if (!own) return;
+  for (int h = wave; h < HG; h += 4) {  // the new key's scores
+    float s = 0.f;
+    for (int d = lane; d < dp; d += 64) s += bf2f(qs[h * dp + d]) * ks[h * dp + d];
+    s = wave_sum(s);
+    if (lane == 0) raw[(int64_t)h * f.keys + i - k0] = s * a.scale;
+  }
+}
+
+template <int C>
+__global__ __launch_bounds__(256) void attn_heads_mix_kernel(const LmAttn a, const HeadsPart f) {
+  constexpr int vp = 32 * C, BLOCKS = HEADS_SPAN / 32 / 4;  // blocks of 32 keys of a wave
+  __shared__ __attribute__((aligned(16))) float ps[HEADS_SPAN], sums[4][vp], red[4];
+  __shared__ unsigned order;
+  const int H = a.heads, dp = vp, groups = H * dp / HEADS_COLS, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n16 = lane & 15,
+            q4 = lane >> 4;
+  const int seq = blockIdx.y, h = blockIdx.x % H, split = blockIdx.x / H;
+  const int row = a.r.seq_row0[seq], i = a.r.seq_pos0[seq], slot = a.r.seq_slot[seq];
+  const int first = a.chunk > 0 ? i / a.chunk * a.chunk : 0, base = first & ~31, k0 = base + split * HEADS_SPAN;
+  if (k0 > i) return;
+  const int live = (i - base) / HEADS_SPAN + 1;
+  const bf16_t* Vb = (const bf16_t*)a.v + (int64_t)slot * H * a.ctx * vp;
+  const float* sq = a.part + f.sq + (int64_t)seq * 2 * groups;
+  const float qq_in = lane < groups ? sq[lane] : 0.f, kk_in = lane < groups ? sq[groups + lane] : 0.f;
+  const float slope_in = lane < H ? a.mix[h * H + lane] * a.slope[lane] : 0.f;
+  const float* raw = a.part + f.raw + (int64_t)seq * H * f.keys + split * HEADS_SPAN + tid;
+  const float* mix = a.mix + h * H;
+  float s = 0.f;
+  u32x4 vf[BLOCKS][2 * C];
+  constexpr int AT_ONCE = 32;
+  float x[AT_ONCE];
+#pragma unroll
+  for (int g = 0; g < AT_ONCE; ++g) x[g] = raw[(int64_t)min(g, H - 1) * f.keys];  // (keys beyond the last: whatever is there, masked)
+#pragma unroll
+  for (int b = 0; b < BLOCKS; ++b) {
+    const int j = k0 + 32 * (wave + 4 * b);
+    const bf16_t* vh = Vb + key_block(min(j, i), h, H, vp) + 8 * lane;
+#pragma unroll
+    for (int t = 0; t < 2 * C; ++t) vf[b][t] = *(const u32x4*)(vh + t * 512);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int g = 0; g < AT_ONCE; ++g)
+    if (g < H) s += mix[g] * x[g];
+  for (int g = AT_ONCE; g < H; ++g) s += mix[g] * raw[(int64_t)g * f.keys];
+  const float qq = wave_sum(qq_in), kk = wave_sum(kk_in), slope = wave_sum(slope_in);
+  const float rq = 1.0f / sqrtf(qq / (float)(H * a.dim) + a.eps), rk = 1.0f / sqrtf(kk / (float)(H * a.dim) + a.eps);
+  const int j = k0 + tid;
+  s = s * (j == i ? rq * rk : rq) - slope * (float)(i - j);
+  if (j > i || j < first) s = -INFINITY;
+  float m = wave_max(s);
+  if (lane == 0) red[wave] = m;
+  __syncthreads();
+  m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  const float p = expf(s - m);
+  ps[tid] = p;
+  const float l = block_sum_256(p, red);  // (its barriers also publish ps)
+  float acc[2 * C];
+#pragma unroll
+  for (int t = 0; t < 2 * C; ++t) acc[t] = 0.f;
+#pragma unroll
+  for (int b = 0; b < BLOCKS; ++b) {
+    const int at = 32 * (wave + 4 * b);
+    if (k0 + at > i) continue;
+    const f32x4 p0 = *(const f32x4*)(ps + at + 8 * q4), p1 = *(const f32x4*)(ps + at + 8 * q4 + 4);
+#pragma unroll
+    for (int t = 0; t < 2 * C; ++t) {
+      const u32x4 v = vf[b][t];
+      acc[t] += p0[0] * lo_bf(v[0]) + p0[1] * hi_bf(v[0]) + p0[2] * lo_bf(v[1]) + p0[3] * hi_bf(v[1]) + p1[0] * lo_bf(v[2]) + p1[1] * hi_bf(v[2]) +
+                p1[2] * lo_bf(v[3]) + p1[3] * hi_bf(v[3]);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < 2 * C; ++t) {
+    acc[t] += __shfl_xor(acc[t], 16, 64);
+    acc[t] += __shfl_xor(acc[t], 32, 64);
+    if (q4 == 0) sums[wave][16 * t + n16] = acc[t];
+  }
+  __syncthreads();
+  if (i < k0 + HEADS_SPAN && tid < dp)  // the new key, with its norm's factor
+    ((bf16_t*)a.k)[(int64_t)slot * a.ctx * H * dp + key_index(i, h, tid, H, dp)] = f2bf(a.part[f.khat + (int64_t)seq * H * dp + h * dp + tid] * rk);
+  float o = 0.f;
+  if (tid < vp) o = (sums[0][tid] + sums[1][tid]) + (sums[2][tid] + sums[3][tid]);
+  bf16_t* out = (bf16_t*)a.out + (int64_t)row * a.ldo;
+  if (live == 1) {
+    if (tid < vp) out[in_chunks(h * vp + tid, a.out_chunk)] = f2bf(o / l);
+    return;
+  }
+  // several parts: stores and loads past the private L2s, the last to arrive adds up
+  auto leave = [](float* to, float v) { __hip_atomic_store(to, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  auto fetch = [](const float* from) { return __hip_atomic_load(from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  const int splits = f.keys / HEADS_SPAN;
+  float* part = a.part + f.part + ((int64_t)seq * H + h) * splits * (vp + 2);
+  if (tid < vp) leave(part + split * (vp + 2) + tid, o);
+  if (tid == 0) {
+    leave(part + split * (vp + 2) + vp, m);
+    leave(part + split * (vp + 2) + vp + 1, l);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0) order = __hip_atomic_fetch_add((unsigned*)(a.part + f.ticket) + seq * H + h, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (order != (unsigned)live - 1 || tid >= vp) return;
+  float M = -INFINITY, L = 0.f, O = 0.f;
+  for (int k = 0; k < live; ++k) M = fmaxf(M, fetch(part + k * (vp + 2) + vp));
+#pragma unroll 4
+  for (int k = 0; k < live; ++k) {
+    const float w = expf(fetch(part + k * (vp + 2) + vp) - M);
+    L += w * fetch(part + k * (vp + 2) + vp + 1);
+    O += w * fetch(part + k * (vp + 2) + tid);
+  }
+  out[in_chunks(h * vp + tid, a.out_chunk)] = f2bf(O / L);
+}
+
+// (heads that divide 256 columns)
+bool heads_takes(int H, int G, int dp, int vp, int taps, bool own_kv) {
+  return own_kv && H == G && dp == vp && (dp == 32 || dp == 64 || dp == 128) && H * dp % HEADS_COLS == 0 && H <= 64 && taps <= 4;
+}
+
+}  // namespace
+
+size_t lm_attn_heads_floats(int n_seq, int span, int H, int G, int dp, int vp, int taps, bool own_kv) {
+  return heads_takes(H, G, dp, vp, taps, own_kv) ? (size_t)heads_part(n_seq, span, H, dp, vp).total : 0;
+}
+bool lm_attn_heads_takes(const LmAttn& a) {
+  if (!heads_takes(a.heads, a.kv_heads, a.dp, a.vp, a.taps, a.own_kv)) return false;
+  const bool many_heads = a.heads > 32 && a.r.n_seq > 40;
+  return !many_heads || !lm_attn_decode_takes(a);
+}
+md_status lm_attn_heads(const LmAttn& a, int span, hipStream_t s) {
+  if (!lm_attn_heads_takes(a)) return MD_ERR_UNSUPPORTED;
+  const HeadsPart f = heads_part(a.r.n_seq, span, a.heads, a.dp, a.vp);
+  const int groups = a.heads * a.dp / HEADS_COLS;
+  auto scores = a.dp == 32 ? attn_heads_scores_kernel<1> : a.dp == 64 ? attn_heads_scores_kernel<2> : attn_heads_scores_kernel<4>;
+  auto mix = a.dp == 32 ? attn_heads_mix_kernel<1> : a.dp == 64 ? attn_heads_mix_kernel<2> : attn_heads_mix_kernel<4>;
+  hipLaunchKernelGGL(scores, dim3(groups * ((span + 31 + HEADS_KEYS - 1) / HEADS_KEYS), a.r.n_seq), dim3(256), 0, s, a, f);
+  MD_TRY(md_launch_status());
+  hipLaunchKernelGGL(mix, dim3(a.heads * (f.keys / HEADS_SPAN), a.r.n_seq), dim3(256), 0, s, a, f);
   return md_launch_status();
 }

@@ -106,6 +106,7 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
         int keys;
         const int ns = lm_attn_decode_splits(n_seq, span, &keys);
         ap = std::max(ap, lm_attn_decode_part_floats(n_seq, ns, l.heads, l.vdim_pad));
+        ap = std::max(ap, lm_attn_heads_floats(n_seq, span, l.heads, l.kv_heads, l.dim_pad, l.vdim_pad, l.taps, l.kv_layer == i));
       }
     } else if (l.mixer == MD_MIXER_LATENT) {
       if (m->dtype != MD_DTYPE_BF16) continue;
@@ -432,6 +433,7 @@ struct Step {
     a.out_chunk = few ? 8 * b->n_rows : 8;
     a.part = w.attn_part;
     const int span = l.chunk > 0 ? std::min(l.chunk, b->max_ctx) : b->max_ctx;
+    if (m->dtype == MD_DTYPE_BF16 && b->max_len == 1 && (g_lm_kernels & 2) && lm_attn_heads_takes(a)) return lm_attn_heads(a, span, s);
     if (m->dtype == MD_DTYPE_BF16 && b->max_len == 1 && (g_lm_kernels & 2) && lm_attn_decode_takes(a)) {
       a.n_split = lm_attn_decode_splits(b->n_seq, span, &a.split_keys);
       return lm_attn_decode(a, s);

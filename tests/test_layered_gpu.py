@@ -469,6 +469,30 @@ def test_many_sequences_of_a_long_context(heads, kv, dim, vdim, count, ctx, chun
     assert float(e.max()) < 7e-2, e
 
 
+@pytest.mark.parametrize("heads,dim,taps", [(8, 30, 1), (4, 64, 4), (2, 128, 2), (64, 32, 3), (12, 60, 3), (64, 100, 4)], ids=str)
+@pytest.mark.parametrize("chunk", [4000, 300])
+def test_decode_of_heads_with_keys_of_their_own(heads, dim, taps, chunk):
+    """Scores and mixture in two launches: the first tokens (fewer than the convolution's taps), last keys at the edges of tiles of 16, of a
+    workgroup's 128 and 256, sums of one, two and three workgroups; two steps, the second of which reads what the first one wrote."""
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    cfg = U.config([U.attention(heads, heads, dim, dim, chunk, taps=taps)], width=96, vocab=120, ff=None)
+    w = U.weights(cfg, 3, 1.5)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=BF16, max_batch=64, max_context=640)
+    text = U.tokens(620, 120, 5)
+    ref = O.forward(cfg, w, text)  # (causal: a shorter text's logits are among them)
+    for lens in ([1, 2, 16, 17, 128, 129, 255, 256, 257, 299, 300, 301, 512, 513, 618], [4], [1 + (37 * i) % 600 for i in range(50)]):
+        slots = [m.open_sequence() for _ in lens]
+        m.step([(s, text[: n - 1], []) for s, n in zip(slots, lens) if n > 1])
+        for k in range(2):
+            got = m.step([(s, text[n - 1 + k : n + k], [0]) for s, n in zip(slots, lens)])
+            e = U.logit_errors(got, ref[[n - 1 + k for n in lens]])
+            assert float(e.max()) < 7e-2, (lens, k, e)
+        for s in slots:
+            m.close_sequence(s)
+
+
 def test_captured_steps_of_many_sequences():
     """64 sequences in a graph with a context of 2048: splits of 64 keys; tokens and the last step's logits against the oracle."""
     from moondream_amd.config import LayeredLMConfig
