@@ -831,7 +831,8 @@ md_status md_argmax_f32(const void* logits, int64_t ld, int32_t batch, int32_t v
 md_status md_gemm_f32(const void* a, int64_t lda, const md_linear* lin, void* c, int64_t ldc, int32_t m, void* stream);
 
 /* Test hook: bit 0 = run the matrix-core attention / retention kernels of a bf16 prefill, bit 1 = the split-key decode
- * attention; cleared bits take the plain kernels (which fp32 models always take).  Default 3.  Process-wide. */
+ * attention; cleared bits take the plain kernels (which fp32 models always take); bit 2 set = the kernels of long prompts for
+ * attention of any.  Default 3.  Process-wide. */
 void md_lm_set_kernels(int32_t mask);
 
 #ifdef __cplusplus

@@ -28,6 +28,9 @@
 // The cache holds keys and values in operand order, so every load of either is 1 KiB of consecutive memory per wave.
 #include "lm_internal.hpp"
 
+#include <algorithm>
+#include <type_traits>
+
 namespace {
 
 // ---------------------------------------------------------------------------------------------------------------------------
@@ -182,13 +185,14 @@ __device__ __forceinline__ void store8(float* p, const float (&v)[8]) {
 }
 
 // grid (blocks of 8 positions, sequences, q | k | v); a block starts at a multiple of 8, so its values fill whole operand rows of the
-// cache.  A thread owns columns 4 tid .. of every 1024 (NI of them), all 8 rows in registers.  TAPS: taps of the convolution when they are
+// cache.  A thread owns columns 4 tid .., all 8 rows in registers (as many threads as that takes: 2048 columns, 40 / 900 / 14000 tokens 9.2 / 13.5 / 93 us, 256 threads with
+// eight columns each 12.2 / 15.9 / 101).  TAPS: taps of the convolution when they are
 // few (every projected row is then read once), 0: any number.
-template <typename T, int NI, int TAPS>
-__global__ __launch_bounds__(256) void attn_prep_block_kernel(const LmAttn a) {
-  extern __shared__ __attribute__((aligned(16))) float hs[];  // values: [8][NI * 256] sums of squares of four columns, then [8][kv_heads];
+template <typename T, int TAPS, int NT>
+__global__ __launch_bounds__(NT) void attn_prep_block_kernel(const LmAttn a) {
+  extern __shared__ __attribute__((aligned(16))) float hs[];  // values: [8][NT] sums of squares of four columns, then [8][kv_heads];
                                                               // bf16: then the finished cache rows, in the cache's order
-  __shared__ float red[4][8];
+  __shared__ float red[NT / 64][8];
   const int seq = blockIdx.y, part = blockIdx.z, tid = threadIdx.x;
   const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, pos0 = a.r.seq_pos0[seq], slot = a.r.seq_slot[seq];
   const int t0 = (pos0 / 8 + blockIdx.x) * 8, lo = max(t0, pos0), hi = min(t0 + 7, pos0 + len - 1);
@@ -196,20 +200,19 @@ __global__ __launch_bounds__(256) void attn_prep_block_kernel(const LmAttn a) {
   const int nh = part == 0 ? a.heads : a.kv_heads, hp = part == 2 ? a.vp : a.dp, ncol = nh * hp;
   const bool all = lo == t0 && hi == t0 + 7;
   constexpr bool STAGE = sizeof(T) == 2;  // whole blocks of 8 positions leave through LDS: 16-byte pieces in the order of the cache
-  bf16_t* stage = (bf16_t*)(hs + 8 * NI * 256 + 8 * a.kv_heads);
+  bf16_t* stage = (bf16_t*)(hs + 8 * NT + 8 * a.kv_heads);
   const int col0 = part == 0 ? a.col_q : part == 1 ? a.col_k : a.col_v;
   const T* proj = (const T*)a.proj + (int64_t)(row0 - pos0) * a.ldp + col0;  // + position * ldp
   const T* ring = (const T*)a.conv_state + (int64_t)slot * a.taps * a.conv_ld + col0;
-  f32x4 y[8][NI];
+  f32x4 y[8];
   float ss[8];
+  const int c = 4 * tid;
 #pragma unroll
-  for (int r = 0; r < 8; ++r) ss[r] = 0.f;
-#pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const int c = 4 * tid + 1024 * i;
-#pragma unroll
-    for (int r = 0; r < 8; ++r) y[r][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (c >= ncol) continue;
+  for (int r = 0; r < 8; ++r) {
+    ss[r] = 0.f;
+    y[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  if (c < ncol) {
     auto input = [&](int p) { return p >= pos0 ? ld4(proj + (int64_t)p * a.ldp + c) : ld4(ring + (int64_t)(p % a.taps) * a.conv_ld + c); };
     if constexpr (TAPS > 0) {
       f32x4 w[TAPS];
@@ -226,7 +229,7 @@ __global__ __launch_bounds__(256) void attn_prep_block_kernel(const LmAttn a) {
         if (t0 - TAPS + 1 + k < 0) u[k] = f32x4{0.f, 0.f, 0.f, 0.f};  // before the sequence
 #pragma unroll
         for (int r = 0; r < 8; ++r)
-          if (k - r >= 0 && k - r < TAPS) y[r][i] += w[k - r] * u[k];
+          if (k - r >= 0 && k - r < TAPS) y[r] += w[k - r] * u[k];
       }
     } else
     for (int j = 0; j < a.taps; ++j) {
@@ -235,14 +238,14 @@ __global__ __launch_bounds__(256) void attn_prep_block_kernel(const LmAttn a) {
       for (int r = 0; r < 8; ++r) {
         const int p = t0 + r - a.taps + 1 + j;
         if (t0 + r < lo || t0 + r > hi || p < 0) continue;
-        y[r][i] += w * input(p);
+        y[r] += w * input(p);
       }
     }
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-      const float s = y[r][i][0] * y[r][i][0] + y[r][i][1] * y[r][i][1] + y[r][i][2] * y[r][i][2] + y[r][i][3] * y[r][i][3];
-      if (part < 2) ss[r] += s;
-      else hs[r * (NI * 256) + tid + 256 * i] = s;
+      const float s = y[r][0] * y[r][0] + y[r][1] * y[r][1] + y[r][2] * y[r][2] + y[r][3] * y[r][3];
+      if (part < 2) ss[r] = s;
+      else hs[r * NT + tid] = s;
     }
   }
   if (part < 2) {
@@ -256,47 +259,43 @@ __global__ __launch_bounds__(256) void attn_prep_block_kernel(const LmAttn a) {
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
       if (t0 + r < lo || t0 + r > hi) continue;
-      const float f = 1.0f / sqrtf((red[0][r] + red[1][r] + red[2][r] + red[3][r]) / (float)(nh * a.dim) + a.eps);
+      float total = 0.f;
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int c = 4 * tid + 1024 * i;
-        if (c >= ncol) continue;
-        const f32x4 o = y[r][i] * f * *(const f32x4*)(w + c);
-        if (part == 0) st4((T*)a.q + (int64_t)(row0 + t0 + r - pos0) * ncol + c, o);
-        else if (STAGE && all) st4(stage + (c >> 3) * 64 + r * 8 + (c & 7), o);
-        else store_key4<T>(a, slot, t0 + r, c, o);
-      }
+      for (int w = 0; w < NT / 64; ++w) total += red[w][r];
+      const float f = 1.0f / sqrtf(total / (float)(nh * a.dim) + a.eps);
+      if (c >= ncol) continue;
+      const f32x4 o = y[r] * f * *(const f32x4*)(w + c);
+      if (part == 0) st4((T*)a.q + (int64_t)(row0 + t0 + r - pos0) * ncol + c, o);
+      else if (STAGE && all) st4(stage + (c >> 3) * 64 + r * 8 + (c & 7), o);
+      else store_key4<T>(a, slot, t0 + r, c, o);
     }
     if (STAGE && all && part == 1) {
       __syncthreads();
       bf16_t* dst = (bf16_t*)a.k + (int64_t)slot * a.ctx * nh * hp;
-      for (int k = tid; k < ncol; k += 256) {  // piece k: eight coordinates of position t0 + k % 8
+      for (int k = tid; k < ncol; k += NT) {  // piece k: eight coordinates of position t0 + k % 8
         const int c = (k >> 3) * 8, g = c / hp;
         *(u32x4*)(dst + key_index(t0 + (k & 7), g, c - g * hp, nh, hp)) = *(const u32x4*)(stage + k * 8);
       }
     }
     return;
   }
-  float* rn = hs + 8 * NI * 256;
+  float* rn = hs + 8 * NT;
   __syncthreads();
-  for (int k = tid; k < 8 * nh; k += 256) {
+  for (int k = tid; k < 8 * nh; k += NT) {
     const int r = k / nh, g = k - r * nh, m = hp / 4;
     float s = 0.f;
-    for (int e = 0; e < m; ++e) s += hs[r * (NI * 256) + g * m + e];
+    for (int e = 0; e < m; ++e) s += hs[r * NT + g * m + e];
     rn[k] = a.value_norm ? 1.0f / sqrtf(s / (float)a.vdim + a.eps) : 1.0f;
   }
   __syncthreads();
-#pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const int c = 4 * tid + 1024 * i;
-    if (c >= ncol) continue;
+  if (c < ncol) {
     const int g = c / hp, e0 = c - g * hp;
     T* dst = (T*)a.v + (int64_t)slot * a.ctx * nh * hp;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       float v[8];
 #pragma unroll
-      for (int r = 0; r < 8; ++r) v[r] = y[r][i][e] * rn[r * nh + g];
+      for (int r = 0; r < 8; ++r) v[r] = y[r][e] * rn[r * nh + g];
       if (STAGE && all) {
         store8(stage + (c + e) * 8, v);
       } else if (all) {
@@ -311,7 +310,7 @@ __global__ __launch_bounds__(256) void attn_prep_block_kernel(const LmAttn a) {
   if (STAGE && all) {
     __syncthreads();
     bf16_t* dst = (bf16_t*)a.v + (int64_t)slot * a.ctx * nh * hp;
-    for (int c = tid; c < ncol; c += 256) {
+    for (int c = tid; c < ncol; c += NT) {
       const int g = c / hp;
       *(u32x4*)(dst + value_index(t0, g, c - g * hp, nh, hp)) = *(const u32x4*)(stage + c * 8);
     }
@@ -422,19 +421,19 @@ __global__ __launch_bounds__(256) void attn_plain_kernel(const LmAttn a) {
   for (int c = tid; c < H * vp; c += 256) stf((T*)a.out + (int64_t)row * a.ldo + in_chunks(c, a.out_chunk), acc[c] / ls[c / vp]);
 }
 
-template <typename T, int NI>
+template <typename T, int NT>
 void (*prep_block_pick(int taps))(const LmAttn) {
   switch (taps) {
-    case 1: return attn_prep_block_kernel<T, NI, 1>;
-    case 2: return attn_prep_block_kernel<T, NI, 2>;
-    case 3: return attn_prep_block_kernel<T, NI, 3>;
-    case 4: return attn_prep_block_kernel<T, NI, 4>;
-    default: return attn_prep_block_kernel<T, NI, 0>;
+    case 1: return attn_prep_block_kernel<T, 1, NT>;
+    case 2: return attn_prep_block_kernel<T, 2, NT>;
+    case 3: return attn_prep_block_kernel<T, 3, NT>;
+    case 4: return attn_prep_block_kernel<T, 4, NT>;
+    default: return attn_prep_block_kernel<T, 0, NT>;
   }
 }
 
 template <typename T>
-md_status prep(const LmAttn& a, hipStream_t s) {
+md_status prep(const LmAttn& a, bool state, hipStream_t s) {
   const int mx = a.heads * a.dp > a.kv_heads * a.vp ? a.heads * a.dp : a.kv_heads * a.vp;
   const int lds = mx * 4;
   const bool step = a.r.max_len == 1;
@@ -444,19 +443,19 @@ md_status prep(const LmAttn& a, hipStream_t s) {
     auto sf = mc <= 2048 ? attn_prep_step_kernel<1> : mc <= 4096 ? attn_prep_step_kernel<2> : attn_prep_step_kernel<4>;
     hipLaunchKernelGGL(sf, dim3(a.r.n_rows, a.own_kv ? 3 : 1), dim3(512), a.own_kv ? a.kv_heads * a.vp * 4 : 0, s, a);
   } else if (!step && mc <= 4096) {
-    auto bf = mc <= 1024 ? prep_block_pick<T, 1>(a.taps) : mc <= 2048 ? prep_block_pick<T, 2>(a.taps) : prep_block_pick<T, 4>(a.taps);
-    const int ni = mc <= 1024 ? 1 : mc <= 2048 ? 2 : 4;
+    auto bf = mc <= 1024 ? prep_block_pick<T, 256>(a.taps) : mc <= 2048 ? prep_block_pick<T, 512>(a.taps) : prep_block_pick<T, 1024>(a.taps);
+    const int nt = mc <= 1024 ? 256 : mc <= 2048 ? 512 : 1024;
     const int kvc = a.kv_heads * (a.dp > a.vp ? a.dp : a.vp);
-    const int block_lds = (8 * ni * 256 + 8 * a.kv_heads) * 4 + (sizeof(T) == 2 && a.own_kv ? kvc * 16 : 0);
+    const int block_lds = (8 * nt + 8 * a.kv_heads) * 4 + (sizeof(T) == 2 && a.own_kv ? kvc * 16 : 0);
     MD_TRY(md_ensure_dynamic_lds((const void*)bf, 150 * 1024));
-    hipLaunchKernelGGL(bf, dim3((a.r.max_len + 14) / 8, a.r.n_seq, a.own_kv ? 3 : 1), dim3(256), block_lds, s, a);
+    hipLaunchKernelGGL(bf, dim3((a.r.max_len + 14) / 8, a.r.n_seq, a.own_kv ? 3 : 1), dim3(nt), block_lds, s, a);
   } else {
     if (lds > 150 * 1024) return MD_ERR_UNSUPPORTED;
     MD_TRY(md_ensure_dynamic_lds((const void*)fn, 150 * 1024));
     hipLaunchKernelGGL(fn, dim3(a.r.n_rows, a.own_kv ? 3 : 1), dim3(256), lds, s, a);
   }
   MD_TRY(md_launch_status());
-  if (step || a.taps == 1) return MD_OK;
+  if (step || a.taps == 1 || !state) return MD_OK;
   hipLaunchKernelGGL(conv_state_kernel<T>, dim3(a.r.n_seq), dim3(256), 0, s, a, a.conv_ld);
   return md_launch_status();
 }
@@ -472,7 +471,7 @@ md_status plain(const LmAttn& a, hipStream_t s) {
 
 }  // namespace
 
-md_status lm_attn_prep(int dtype, const LmAttn& a, hipStream_t s) { return dtype == MD_DTYPE_F32 ? prep<float>(a, s) : prep<bf16_t>(a, s); }
+md_status lm_attn_prep(int dtype, const LmAttn& a, hipStream_t s) { return dtype == MD_DTYPE_F32 ? prep<float>(a, true, s) : prep<bf16_t>(a, true, s); }
 md_status lm_attn_plain(int dtype, const LmAttn& a, hipStream_t s) { return dtype == MD_DTYPE_F32 ? plain<float>(a, s) : plain<bf16_t>(a, s); }
 
 // ---------------------------------------------------------------------------------------------------------------------------
@@ -993,6 +992,295 @@ md_status lm_attn_mfma(const LmAttn& args, hipStream_t s) {
   MD_TRY(md_launch_status());
   if (a.n_split == 1) return MD_OK;
   hipLaunchKernelGGL(attn_parts_kernel, dim3(tiles, a.r.n_seq, (a.heads + 3) / 4), dim3(256), 0, s, a);
+  return md_launch_status();
+}
+
+// ---------------------------------------------------------------------------------------------------------------------------
+// Prompts of up to some thousand tokens: attn_mfma_kernel has few tiles then, and each is a long chain.  The mixed scores of all pairs fit the caches (4 bytes of a head
+// and pair), so they go through memory:
+//   attn_pairs_scores_kernel  (32 keys, 16 queries, sequence): a wave's share of the heads, their scores to LDS in the order of the mixture's operand (two bf16 for
+//                             a float), mixture, scale, distance and mask; the scores leave in the order of the other kernel's operand.  One workgroup row
+//                             more keeps the convolution's state
+//   attn_pairs_out_kernel     (head, 16 queries, sequence): softmax over all keys, weighted values; a wave has every NW-th block of 32 keys, whose scores are loaded
+//                             before the first is used, and the waves' sums meet in LDS
+// 32 heads of 64, one prompt of 40 / 250 tokens: 10 and 4 / 5 us a layer, against 28 / 53 us (parts of keys and their sum) and 6 for the state.  Whole prompts through
+// 24 layers (12 of attention), before and now, with attn_prep_block_kernel's share: 40 / 250 / 550 / 900 tokens 2.06 / 3.15 / 3.75 / 4.82 -> 1.78 / 2.58 / 3.33 / 4.53 ms; 4 x 50 / 200 / 500
+// 2.72 / 4.60 / 7.97 -> 2.44 / 4.15 / 7.83.  Scores of 48 million floats (12 x 300 tokens) took 11.64 for 11.51 ms: hence PAIRS_FLOATS.
+namespace {
+
+typedef void (*TalkKernelBlocks)(const LmAttn, int);
+constexpr int PAIRS_BLOCKS = 4, PAIRS_MOST = 8 * PAIRS_BLOCKS;  // blocks of 32 keys: of a wave, and of a tile
+
+// (a tile's first block may begin before the chunk, and its last query may be one of the next chunk)
+__host__ __device__ inline int pairs_blocks(int span) { return (span - 1 + 15 + 31) / 32 + 1; }
+__host__ __device__ inline int64_t pairs_at(int64_t slot, int h, int kb, int H, int blocks) { return ((slot * H + h) * blocks + kb) * 512; }
+
+template <int HB, int D>
+__global__ __launch_bounds__(256) void attn_pairs_scores_kernel(const LmAttn a, int blocks) {
+  constexpr int HP = 16 * HB, HW = HP / 4, dp = 32 * D, W = HW / 2;  // heads of a wave, dwords of them in an operand
+  typedef typename std::conditional<HB == 2, u32x4, u32x2>::type Op;
+  __shared__ Op b_lds[32][2][4][16];  // [key][high | low part][wave][query]
+  __shared__ float mss[HP];
+  const int H = a.heads, G = a.kv_heads, rep = H / G, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, q = lane >> 4;
+  const int kb = blockIdx.x, tile = blockIdx.y, seq = blockIdx.z;
+  const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, pos0 = a.r.seq_pos0[seq], slot = a.r.seq_slot[seq];
+  if (tile == (int)gridDim.y - 1) {  // conv_state_kernel's work
+    bf16_t* ring = (bf16_t*)a.conv_state + (int64_t)slot * a.taps * a.conv_ld;
+    const int keep = min(len, a.taps - 1), pieces = a.conv_ld / 4, n_pieces = keep * pieces, step = gridDim.x * 256;
+    constexpr int AT_ONCE = 8;
+    for (int p0 = kb * 256 + tid; p0 < n_pieces; p0 += AT_ONCE * step) {
+      u32x2 v[AT_ONCE];
+#pragma unroll
+      for (int k = 0; k < AT_ONCE; ++k) {
+        const int p = min(p0 + k * step, n_pieces - 1), t = len - keep + p / pieces;
+        v[k] = *(const u32x2*)((const bf16_t*)a.proj + (int64_t)(row0 + t) * a.ldp + p % pieces * 4);
+      }
+#pragma unroll
+      for (int k = 0; k < AT_ONCE; ++k) {
+        const int p = p0 + k * step, t = len - keep + p / pieces;
+        if (p < n_pieces) *(u32x2*)(ring + (int64_t)((pos0 + t) % a.taps) * a.conv_ld + p % pieces * 4) = v[k];
+      }
+    }
+    return;
+  }
+  const int t0 = (pos0 / 16 + tile) * 16, lo = max(t0, pos0), hi = min(t0 + 15, pos0 + len - 1);  // positions of the live queries
+  const int j0 = ((a.chunk > 0 ? lo / a.chunk * a.chunk : 0) & ~31) + 32 * kb;
+  if (lo > hi || j0 > hi) return;
+  const bf16_t* qrow = (const bf16_t*)a.q + (int64_t)(row0 + min(max(t0 + n, lo), hi) - pos0) * H * dp + 8 * q;  // (rows outside replay a live one)
+  const bf16_t* Kb = (const bf16_t*)a.k + (int64_t)slot * G * a.ctx * dp + 8 * lane;
+  // everything that the wave reads is requested before the first product (the second 16 keys where the first ones' registers get free)
+  constexpr int LH = 256 / HP;  // lanes per head of the slopes' mixture
+  float tm[HB][8], slope_in = 0.f;  // A operand of the mixture, as in attn_mfma_kernel
+#pragma unroll
+  for (int mt = 0; mt < HB; ++mt)
+#pragma unroll
+    for (int j = 0; j < (HB == 2 ? 8 : 4); ++j) tm[mt][j] = a.mix[min(16 * mt + n, H - 1) * H + min(HB == 2 ? 8 * q + j : 4 * q + j, H - 1)];
+  u32x4 qf[HW][D], kf[HW][D];
+  auto keys = [&](int x, int mt) {  // (heads beyond the last: their mixture's weights are zero)
+    const bf16_t* kh = Kb + key_block(j0, min(HW * wave + x, H - 1) / rep, G, dp);
+#pragma unroll
+    for (int d = 0; d < D; ++d) kf[x][d] = *(const u32x4*)(kh + (mt * D + d) * 512);
+  };
+#pragma unroll
+  for (int x = 0; x < HW; ++x) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) qf[x][d] = *(const u32x4*)(qrow + min(HW * wave + x, H - 1) * dp + 32 * d);
+    keys(x, 0);
+  }
+#pragma unroll
+  for (int k = 0; k < HP / LH; ++k) {
+    const int h = tid / LH, g = tid % LH + LH * k;
+    const float w = a.mix[min(h, H - 1) * H + min(g, H - 1)] * a.slope[min(g, H - 1)];
+    slope_in += h < H && g < H ? w : 0.f;
+  }
+  PHASE();
+  f32x4 acc[HW][2];
+#pragma unroll
+  for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+    for (int x = 0; x < HW; ++x) {
+      acc[x][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int d = 0; d < D; ++d) acc[x][mt] = mfma(kf[x][d], qf[x][d], acc[x][mt]);
+      if (mt == 0) keys(x, 1);
+      PHASE();
+    }
+#pragma unroll
+  for (int o = LH / 2; o > 0; o >>= 1) slope_in += __shfl_xor(slope_in, o, 64);
+  if (tid % LH == 0) mss[tid / LH] = slope_in * kLog2e;
+  bf16x8 tf[HB];
+#pragma unroll
+  for (int mt = 0; mt < HB; ++mt)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) tf[mt][j] = (16 * mt + n < H && (HB == 2 ? 8 * q + j : 4 * q + j) < H && (HB == 2 || j < 4)) ? (short)f2bf(tm[mt][j]) : (short)0;
+#pragma unroll
+  for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      Op high, low;
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        const float x = acc[2 * w][mt][e], y = acc[2 * w + 1][mt][e];
+        high[w] = pack_bf16x2(x, y);
+        low[w] = pack_bf16x2(x - lo_bf(high[w]), y - hi_bf(high[w]));
+      }
+      const int key = 16 * mt + 4 * q + e;
+      b_lds[key][0][wave][n] = high;
+      b_lds[key][1][wave][n] = low;
+    }
+  __syncthreads();
+  // keys 8 wave ..: heads 16 mt + 4 q + r of query n
+  const float scale = a.scale * kLog2e;
+  const int qpos = t0 + n, qfirst = a.chunk > 0 ? qpos / a.chunk * a.chunk : 0;
+  float ms[HB][4];
+#pragma unroll
+  for (int mt = 0; mt < HB; ++mt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) ms[mt][r] = mss[16 * mt + 4 * q + r];
+  float* out = a.part + pairs_at(talk_slot(row0, seq, tile), 0, kb, H, blocks) + (wave * 16 + n) * 4;
+#pragma unroll
+  for (int kg = 0; kg < 2; ++kg) {
+    f32x4 st[4][HB];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int part = 1; part >= 0; --part) {  // low parts, then high parts on top
+        const Op b = b_lds[8 * wave + 4 * kg + k][part][q][n];
+#pragma unroll
+        for (int mt = 0; mt < HB; ++mt) {
+          const f32x4 z = part ? f32x4{0.f, 0.f, 0.f, 0.f} : st[k][mt];
+          if constexpr (HB == 2) {
+            st[k][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(md_bf16x8v, tf[mt]), __builtin_bit_cast(md_bf16x8v, b), z, 0, 0, 0);
+          } else {
+            const bf16x4 t = {tf[mt][0], tf[mt][1], tf[mt][2], tf[mt][3]};
+            st[k][mt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(t, __builtin_bit_cast(bf16x4, b), z, 0, 0, 0);
+          }
+        }
+      }
+#pragma unroll
+    for (int mt = 0; mt < HB; ++mt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int h = 16 * mt + 4 * q + r;
+        f32x4 o;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int j = j0 + 8 * wave + 4 * kg + k;
+          o[k] = j > qpos || j < qfirst ? -INFINITY : st[k][mt][r] * scale - ms[mt][r] * (float)(qpos - j);
+        }
+        if (h < H) *(f32x4*)(out + (int64_t)h * blocks * 512 + kg * 256) = o;
+      }
+  }
+}
+
+template <int NW, int C>
+__global__ __launch_bounds__(64 * NW) void attn_pairs_out_kernel(const LmAttn a, int blocks) {
+  constexpr int vp = 32 * C, NB = PAIRS_BLOCKS;
+  __shared__ __attribute__((aligned(16))) float o_lds[NW][16][vp + 4], m_lds[NW][16], l_lds[NW][16];
+  const int H = a.heads, G = a.kv_heads, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, q = lane >> 4;
+  const int h = blockIdx.x, tile = blockIdx.y, seq = blockIdx.z;
+  const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, pos0 = a.r.seq_pos0[seq], slot = a.r.seq_slot[seq];
+  const int t0 = (pos0 / 16 + tile) * 16, lo = max(t0, pos0), hi = min(t0 + 15, pos0 + len - 1);
+  if (lo > hi) return;
+  const int kfirst = (a.chunk > 0 ? lo / a.chunk * a.chunk : 0) & ~31, nkb = (hi - kfirst) / 32 + 1;
+  const float* in = a.part + pairs_at(talk_slot(row0, seq, tile), h, 0, H, blocks) + 4 * lane;
+  const bf16_t* Vb = (const bf16_t*)a.v + (int64_t)slot * G * a.ctx * vp + key_block(kfirst, h / (H / G), G, vp) + 8 * lane;
+  const int64_t vstep = (int64_t)G * 32 * vp;
+  f32x4 s[NB][2];  // keys 8 q + 4 i .. of query n
+  u32x4 vf[NB][2 * C];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const int kb = wave + NW * b;
+    s[b][0] = s[b][1] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    if (kb >= nkb) continue;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) s[b][i] = *(const f32x4*)(in + (int64_t)kb * 512 + i * 256);
+#pragma unroll
+    for (int t = 0; t < 2 * C; ++t) vf[b][t] = *(const u32x4*)(Vb + kb * vstep + t * 512);
+  }
+  float m = -INFINITY;
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m = fmaxf(m, fmaxf(s[b][0][e], s[b][1][e]));
+  m = fmaxf(m, __shfl_xor(m, 16, 64));
+  m = fmaxf(m, __shfl_xor(m, 32, 64));
+  const float ref = m == -INFINITY ? 0.f : m;
+  f32x4 o[2 * C];
+#pragma unroll
+  for (int t = 0; t < 2 * C; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float l = 0.f;
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    if (wave + NW * b >= nkb) continue;
+    u32x4 p;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float p0 = __builtin_amdgcn_exp2f(s[b][i][2 * e] - ref), p1 = __builtin_amdgcn_exp2f(s[b][i][2 * e + 1] - ref);
+        l += p0 + p1;
+        p[2 * i + e] = pack_bf16x2(p0, p1);
+      }
+#pragma unroll
+    for (int t = 0; t < 2 * C; ++t) o[t] = mfma(p, vf[b][t], o[t]);
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (q == 0) {
+    m_lds[wave][n] = m;
+    l_lds[wave][n] = l;
+  }
+#pragma unroll
+  for (int t = 0; t < 2 * C; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o_lds[wave][4 * q + r][16 * t + n] = o[t][r];
+  __syncthreads();
+  for (int at = tid; at < 16 * vp / 8; at += 64 * NW) {  // eight coordinates of a query
+    const int row = at / (vp / 8), e0 = at % (vp / 8) * 8, pos = t0 + row;
+    if (pos < lo || pos > hi) continue;
+    float M = -INFINITY, L = 0.f, v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, m_lds[w][row]);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float f = __builtin_amdgcn_exp2f(m_lds[w][row] - M);
+      L += f * l_lds[w][row];
+      const f32x4 x = *(const f32x4*)(&o_lds[w][row][e0]), y = *(const f32x4*)(&o_lds[w][row][e0 + 4]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] += f * x[e];
+        v[4 + e] += f * y[e];
+      }
+    }
+    const float inv = 1.0f / L;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] *= inv;
+    store8((bf16_t*)a.out + (int64_t)(row0 + pos - pos0) * a.ldo + in_chunks(h * vp + e0, a.out_chunk), v);
+  }
+}
+
+constexpr int64_t PAIRS_FLOATS = 40 << 20;  // most scores of a step
+int64_t pairs_floats(int n_rows, int n_seq, int span, int H) { return (int64_t)(n_rows / 16 + 2 * n_seq) * H * std::min(pairs_blocks(span), PAIRS_MOST) * 512; }
+bool pairs_form(int H, int dp, int vp) { return H <= 32 && dp <= 128 && vp <= 128 && (H <= 16 || dp <= 64); }
+
+template <int HB>
+TalkKernelBlocks pairs_scores_pick(int dp) {
+  switch (dp / 32) {
+    case 1: return attn_pairs_scores_kernel<HB, 1>;
+    case 2: return attn_pairs_scores_kernel<HB, 2>;
+    case 3: return attn_pairs_scores_kernel<HB, 3>;
+    default: return attn_pairs_scores_kernel<HB, 4>;
+  }
+}
+template <int NW>
+TalkKernelBlocks pairs_out_pick(int vp) {
+  switch (vp / 32) {
+    case 1: return attn_pairs_out_kernel<NW, 1>;
+    case 2: return attn_pairs_out_kernel<NW, 2>;
+    case 3: return attn_pairs_out_kernel<NW, 3>;
+    default: return attn_pairs_out_kernel<NW, 4>;
+  }
+}
+
+}  // namespace
+
+size_t lm_attn_pairs_floats_most(int n_rows, int n_seq, int span, int H, int dp, int vp) {
+  return pairs_form(H, dp, vp) ? (size_t)std::min(PAIRS_FLOATS, pairs_floats(n_rows, n_seq, span, H)) : 0;
+}
+bool lm_attn_pairs_takes(const LmAttn& a, int span) {
+  return pairs_form(a.heads, a.dp, a.vp) && pairs_blocks(span) <= PAIRS_MOST && pairs_floats(a.r.n_rows, a.r.n_seq, span, a.heads) <= PAIRS_FLOATS;
+}
+md_status lm_attn_pairs(const LmAttn& a, int span, hipStream_t s) {
+  if (!lm_attn_pairs_takes(a, span)) return MD_ERR_UNSUPPORTED;
+  MD_TRY(prep<bf16_t>(a, false, s));
+  const int blocks = pairs_blocks(span), tiles = (a.r.max_len + 30) / 16;
+  const auto scores = a.heads <= 16 ? pairs_scores_pick<1>(a.dp) : pairs_scores_pick<2>(a.dp);
+  const auto out = blocks <= 2 * PAIRS_BLOCKS ? pairs_out_pick<2>(a.vp) : blocks <= 4 * PAIRS_BLOCKS ? pairs_out_pick<4>(a.vp) : pairs_out_pick<8>(a.vp);
+  const int waves = blocks <= 2 * PAIRS_BLOCKS ? 2 : blocks <= 4 * PAIRS_BLOCKS ? 4 : 8;
+  hipLaunchKernelGGL(scores, dim3(blocks, tiles + 1, a.r.n_seq), dim3(256), 0, s, a, blocks);
+  MD_TRY(md_launch_status());
+  hipLaunchKernelGGL(out, dim3(a.heads, tiles, a.r.n_seq), dim3(64 * waves), 0, s, a, blocks);
   return md_launch_status();
 }
 

@@ -101,7 +101,8 @@ LmWs layout(const md_lm_model* m, const md_lm_batch* b, int n_logits, void* base
     if (l.mixer == MD_MIXER_ATTENTION) {
       q = std::max(q, (size_t)l.heads * l.dim_pad);
       const int span = l.chunk > 0 ? std::min(l.chunk, max_ctx) : max_ctx;
-      if (max_len > 1 && m->dtype == MD_DTYPE_BF16) ap = std::max(ap, lm_attn_mfma_part_floats_most(rows, n_seq, span, l.heads, l.vdim_pad));
+      if (max_len > 1 && m->dtype == MD_DTYPE_BF16)
+        ap = std::max({ap, lm_attn_mfma_part_floats_most(rows, n_seq, span, l.heads, l.vdim_pad), lm_attn_pairs_floats_most(rows, n_seq, span, l.heads, l.dim_pad, l.vdim_pad)});
       if (max_len == 1) {
         int keys;
         const int ns = lm_attn_decode_splits(n_seq, span, &keys);
@@ -438,6 +439,7 @@ struct Step {
       a.n_split = lm_attn_decode_splits(b->n_seq, span, &a.split_keys);
       return lm_attn_decode(a, s);
     }
+    if (m->dtype == MD_DTYPE_BF16 && b->max_len > 1 && (g_lm_kernels & 5) == 1 && lm_attn_pairs_takes(a, span)) return lm_attn_pairs(a, span, s);
     MD_TRY(lm_attn_prep(m->dtype, a, s));
     if (m->dtype == MD_DTYPE_BF16 && b->max_len > 1 && (g_lm_kernels & 1) && lm_attn_mfma_takes(a)) {
       a.n_split = lm_attn_mfma_parts(a.r, b->ctx_rows, span, l.heads, l.vdim_pad, &a.split_keys);

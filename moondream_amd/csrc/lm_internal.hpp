@@ -364,6 +364,10 @@ md_status lm_reduce_rows(const float* part, int slices, int64_t ldp, int64_t sli
 
 md_status lm_attn_prep(int dtype, const LmAttn& a, hipStream_t s);      // convolution, norms, cache rows, convolution state
 md_status lm_attn_plain(int dtype, const LmAttn& a, hipStream_t s);     // one workgroup per query row, any dtype
+// bf16 prompts of a few hundred tokens, scores through memory: lm_attn_prep and the rest (span: most keys of a query)
+bool lm_attn_pairs_takes(const LmAttn& a, int span);
+size_t lm_attn_pairs_floats_most(int n_rows, int n_seq, int span, int heads, int dp, int vp);  // of steps up to that size
+md_status lm_attn_pairs(const LmAttn& a, int span, hipStream_t s);
 bool lm_attn_mfma_takes(const LmAttn& a);
 int lm_attn_mfma_parts(const LmRows& r, int ctx_rows, int span, int heads, int vp, int* split_keys);
 size_t lm_attn_mfma_part_floats_most(int n_rows, int n_seq, int span, int heads, int vp);  // floats that the parts of steps up to that size take at most

@@ -406,6 +406,50 @@ def test_prompts_whose_tiles_are_cut_by_keys(heads, kv, dim, vdim, lens, chunk):
     assert float(U.logit_errors(got, want[0]).max()) < 7e-2
 
 
+@pytest.mark.parametrize("heads,kv,dim,vdim,chunk", [(3, 1, 128, 96, 33), (17, 17, 64, 128, 2000), (32, 8, 30, 128, 45), (16, 16, 128, 128, 77), (1, 1, 32, 32, 2000), (30, 10, 64, 20, 300)], ids=str)
+def test_prompts_whose_scores_go_through_memory(heads, kv, dim, vdim, chunk):
+    """Heads that fill no wave's share, tiles whose queries lie in two chunks, blocks of 32 keys that begin before one, last keys at the edges of blocks and of a wave's
+    share of them, one to eight waves; the second portion's convolution reads what the first one kept."""
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    cfg = U.config([U.attention(heads, kv, dim, vdim, chunk)], width=96, vocab=120, ff=None)
+    w = U.weights(cfg, 3, 1.5)
+    text = U.tokens(900, 120, 9)
+    ref = O.forward(cfg, w, text)  # (causal: a shorter text's logits are among them)
+    for most, lens in ((900, [900]), (480, [2, 31, 32, 33, 64, 65, 255, 256, 257, 480]), (130, [5, 130])):
+        m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=BF16, max_batch=12, max_context=most)
+        for cut in (0, 17):
+            slots = [m.open_sequence() for _ in lens]
+            if cut:
+                m.step([(s, text[:cut], []) for s, n in zip(slots, lens) if n > cut])
+            got = m.step([(s, text[cut * (n > cut) : n], range(n - cut * (n > cut))) for s, n in zip(slots, lens)])
+            want = torch.cat([ref[cut * (n > cut) : n] for n in lens])
+            assert float(U.logit_errors(got, want).max()) < 7e-2, (lens, cut)
+            for s in slots:
+                m.close_sequence(s)
+
+
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(4, 4, 32, 32), (12, 12, 96, 128), (32, 32, 64, 64)], ids=str)
+@pytest.mark.parametrize("lens,chunk", [([260], 2000), ([700], 2000), ([620, 3, 250, 431], 2000), ([900], 333), ([300] * 13, 2000), ([530] * 8, 2000)], ids=str)
+def test_prompts_whose_scores_stay_on_the_cu(heads, kv, dim, vdim, lens, chunk):
+    """The kernels of longer prompts at the sizes that the others take: keys in parts, whole tiles in each of their orders."""
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    cfg = U.config([U.attention(heads, kv, dim, vdim, chunk)], width=96, vocab=120, ff=None)
+    w = U.weights(cfg, 3, 1.5)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=BF16, max_batch=16, max_context=1000)
+    text = U.tokens(max(lens), 120, 9)
+    ref = O.forward(cfg, w, text)
+    m.lib.md_lm_set_kernels(5)
+    try:
+        got = m.step([(m.open_sequence(), text[:n], range(n)) for n in lens])
+    finally:
+        m.lib.md_lm_set_kernels(3)
+    assert float(U.logit_errors(got, torch.cat([ref[:n] for n in lens])).max()) < 7e-2
+
+
 @pytest.mark.parametrize("lens", [[530] * 8, [300] * 16, [530] * 7 + [10], [530] * 7 + [500], [300] * 15, [300] * 13, [90] * 16],
                          ids=["eight", "sixteen", "ragged", "nearly", "fifteen", "thirteen", "short"])
 def test_prompts_of_eight_sequences(lens):
