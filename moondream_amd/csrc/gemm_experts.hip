@@ -49,8 +49,9 @@ __global__ __launch_bounds__(64 * W) void expert_gemm_kernel(const LmExpertGemm 
   if (count == 0 || (by_choice && list[0] != blockIdx.y)) return;  // (the same in every wave) nobody's, or an earlier choice's
 
   const int kw = 4 * (r >> 3) + g;  // 8-column piece of a unit, 64 of K, that this lane takes
-  const bf16_t* w0 = a.w + expert * a.expert_stride + (int64_t)(n0 + (lane >> 3)) * a.k + 8 * ((lane & 7) ^ (lane >> 3));
-  const bf16_t* w1 = w0 + (int64_t)(EPI == EPI_SILU ? a.ff_pad : 8) * a.k;
+  const bf16_t* w0 = a.w + expert * a.expert_stride + (int64_t)n0 * a.k;
+  const __amdgpu_buffer_rsrc_t w_rows[2] = {weight_rows(w0), weight_rows(w0 + (int64_t)(EPI == EPI_SILU ? a.ff_pad : 8) * a.k)};
+  const uint32_t w_at = weight_at(lane, a.k);
   char* mine = ring[wave];
   const uint32_t rd = lds_address(mine) + (r & 7) * 128 + (kw ^ (r & 7)) * 16;
   const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc((void*)a.a, 0, (int)(a.a_rows * a.lda * 2), 0x00020000);
@@ -69,8 +70,8 @@ __global__ __launch_bounds__(64 * W) void expert_gemm_kernel(const LmExpertGemm 
         for (int h = 0; h < PA; ++h) acc[i][h] = f32x4{0.f, 0.f, 0.f, 0.f};
       u32x4 af[D][PA];
       auto load = [&](int b, int u) {
-        load_weights(w0 + u * 64, mine + b * 2048);
-        load_weights(w1 + u * 64, mine + b * 2048 + 1024);
+        load_weights(w_rows[0], w_at, 128u * u, mine + b * 2048);
+        load_weights(w_rows[1], w_at, 128u * u, mine + b * 2048 + 1024);
 #pragma unroll
         for (int h = 0; h < PA; ++h) af[b][h] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rows, at + 128u * u + 64u * h, 0, 0));
         asm volatile("" ::: "memory");  // (the waits count: a unit's loads stay together)
@@ -84,19 +85,7 @@ __global__ __launch_bounds__(64 * W) void expert_gemm_kernel(const LmExpertGemm 
           for (int h = 0; h < PA; ++h)
             acc[i][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(md_bf16x8v, w[i]), __builtin_bit_cast(md_bf16x8v, af[b][h]), acc[i][h], 0, 0, 0);
       };
-#pragma unroll
-      for (int d = 0; d < D; ++d)
-        if (lo + d < hi) load(d, lo + d);
-      for (int u = lo; u < hi; u += D) {
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-          const int left = hi - 1 - (u + d);
-          if (left < 0) break;
-          wait_units<D - 1, 2 + PA>(left);
-          multiply(d);
-          if (left >= D) load(d, u + d + D);
-        }
-      }
+      stream_units<D, 2 + PA>(lo, hi, load, multiply, [] {});
       if (r0 > 0) __syncthreads();  // (the sums before these were read)
       // 8 columns: lanes 0 .. 31 of the first half's product, 32 .. 63 of the other's; up to 8 choices: rows 0 .. 7, and 8 .. 15
 #pragma unroll

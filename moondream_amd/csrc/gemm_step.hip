@@ -13,10 +13,14 @@
 // 7.3).  Activations are read directly: with few rows they are a fraction of the weights' bytes.  What a product or a mixer makes for the next one lies in the operand's order, [column / 8][row][8], so that a load takes consecutive memory
 // (rows 4 KB apart meet on few channels: output projection of 40 rows 9.9 us against 7.6).
 //
-// Measured, 2048 wide, 5440 feed-forward, one stream, one row (16 rows, 28, 40): 8192 columns 8.4 us (7.9, 9.0, 10.5), 33 MB; gates 10.0 us (10.1, 11.2, 12.4), 44 MB;
-// the two residual products 4.4 and 6.7 us (4.9 and 8.2; 5.8 and 10.1; 6.5 and 11.9), 8 and 22 MB; the head, 51200 columns, 34 us (36, 41, 46),
+// Units of K are under way without a gap in between (stream_units): while the weights' loads into LDS were global ones, every use of loaded activations waited for
+// all loads, once in a ring's length.  1 / 8 / 16 / 28 / 40 rows, before and since: gates 10.3 -> 9.7, 10.3 -> 9.9, 10.4 -> 10.0, 11.2 -> 10.9, 12.5 -> 12.2 us; 8192 columns, 40 rows
+// 10.5 -> 10.1, 4352 9.5 -> 9.0.  The residual products are bound by the activations and did not change; the head is not peeled.
+//
+// Measured, 2048 wide, 5440 feed-forward, one stream, one row (16 rows, 28, 40): 8192 columns 8.6 us (8.0, 8.8, 10.1), 33 MB; gates 9.7 us (10.0, 10.9, 12.2), 44 MB;
+// the two residual products 4.5 and 6.7 us (4.9 and 8.2; 5.7 and 10.0; 6.5 and 11.9), 8 and 22 MB; the head, 51200 columns, 35 us (36, 41, 45),
 // 210 MB.  With the weights loaded in the operand's shape: 8.5 us (8.3, 9.8, 11.2), 10.1 (10.8, 12.2, 13.9), 6.6 (8.5, 10.4, 12.3), 36 (39, 48, 57).  The tile products
-// at 40 rows: gates 16.2 us, the residual products and their row-wise launches 13.3 us each, 4352 columns in K slices 12.5 us (9.4).
+// at 40 rows: gates 16.2 us, the residual products and their row-wise launches 13.3 us each, 4352 columns in K slices 12.5 us (9.0).
 // About 4 us of every launch are its start, the first loads and the sum over the waves; at 40 rows the activations, which every workgroup reads, are as many bytes
 // as the weights.
 #include "lm_internal.hpp"
@@ -64,12 +68,7 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
   }
 
   const int kw = 4 * (r >> 3) + g, ka = DIAG ? kw : g;  // 8-column piece of a unit that this lane takes
-  const bf16_t* wp[NX];
-#pragma unroll
-  for (int x = 0; x < NX; ++x) {
-    const int64_t first = (int64_t)x * (EPI == EPI_SILU ? a.ff_pad : 8) + n0;
-    wp[x] = a.w + (LDS ? (first + (lane >> 3)) * a.k + 8 * ((lane & 7) ^ (lane >> 3)) : (first + (r & 7)) * a.k + 8 * kw);
-  }
+  auto w_row = [&](int x) { return (int64_t)x * (EPI == EPI_SILU ? a.ff_pad : 8) + n0; };
   const bf16_t* ap[M16];
 #pragma unroll
   for (int i = 0; i < M16; ++i) ap[i] = a.a + (int64_t)row_of(min(16 * i + (DIAG ? r & 7 : r), a.rows - 1)) * a.lda + ka * a.chunk;
@@ -105,13 +104,16 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
 
   if constexpr (LDS) {
     char* mine = ring[wave];
-    const uint32_t rd = lds_address(mine) + (r & 7) * 128 + (kw ^ (r & 7)) * 16;
+    const uint32_t rd = lds_address(mine) + (r & 7) * 128 + (kw ^ (r & 7)) * 16, at = weight_at(lane, a.k);
+    __amdgpu_buffer_rsrc_t w_rows[NX];
+#pragma unroll
+    for (int x = 0; x < NX; ++x) w_rows[x] = weight_rows(a.w + w_row(x) * a.k);
     u32x4 af[U][PA][M16];
     constexpr int P = NX + PA * M16;
     auto load = [&](int b, int u) {
       const int k = u * 64, kc = k / 8 * a.chunk;
 #pragma unroll
-      for (int x = 0; x < NX; ++x) load_weights(wp[x] + k, mine + (b * NX + x) * 1024);
+      for (int x = 0; x < NX; ++x) load_weights(w_rows[x], at, 2u * k, mine + (b * NX + x) * 1024);
 #pragma unroll
       for (int h = 0; h < PA; ++h)
 #pragma unroll
@@ -129,20 +131,11 @@ __global__ __launch_bounds__(64 * W) void step_gemm_kernel(const LmStepGemm a) {
           for (int i = 0; i < M16; ++i)
             acc[x][h][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(md_bf16x8v, w[x]), __builtin_bit_cast(md_bf16x8v, af[b][h][i]), acc[x][h][i], 0, 0, 0);
     };
-#pragma unroll
-    for (int d = 0; d < U; ++d)
-      if (lo + d < hi) load(d, lo + d);
-    for (int u = lo; u < hi; u += U) {
-#pragma unroll
-      for (int d = 0; d < U; ++d) {
-        const int left = hi - 1 - (u + d);
-        if (left < 0) break;
-        wait_units<U - 1, P>(left);
-        multiply(d);
-        if (left >= U) load(d, u + d + U);
-      }
-    }
+    stream_units<U, P, !(W == 2 && EPI == EPI_ROWS)>(lo, hi, load, multiply, [] {});
   } else {
+    const bf16_t* wp[NX];
+#pragma unroll
+    for (int x = 0; x < NX; ++x) wp[x] = a.w + (w_row(x) + (r & 7)) * a.k + 8 * kw;
     u32x4 wf[2][U][NX], af[2][U][PA][M16];
     auto load = [&](auto buf, int u) {  // units u .. u + U - 1; past the end: the last one again, not used
       constexpr int B = decltype(buf)::value;
@@ -349,7 +342,7 @@ __global__ __launch_bounds__(64 * W) void step_gemm_tall_kernel(const LmStepGemm
     }
 
   // load h of an operand: its rows 8 h .., the piece of a unit that this lane takes
-  const bf16_t* wp[NX][2];
+  __amdgpu_buffer_rsrc_t w_rows[NX][2];
 #pragma unroll
   for (int x = 0; x < NX; ++x)
 #pragma unroll
@@ -358,9 +351,10 @@ __global__ __launch_bounds__(64 * W) void step_gemm_tall_kernel(const LmStepGemm
       const int64_t first = EPI != EPI_SILU ? min(n0 + 16 * x + 8 * h, a.n - 8)
                             : NX & 1      ? (int64_t)h * a.ff_pad + min(n0 + 8 * x, a.n - 8)
                                           : (int64_t)(x & 1) * a.ff_pad + min(n0 + 16 * (x >> 1) + 8 * h, a.n - 8);
-      wp[x][h] = a.w + (first + (lane >> 3)) * a.k + 8 * ((lane & 7) ^ (lane >> 3));
+      w_rows[x][h] = weight_rows(a.w + first * a.k);
     }
   char* mine = ring[wave];
+  const uint32_t at = weight_at(lane, a.k);
   const uint32_t rd = lds_address(mine) + upper * 1024 + (r & 7) * 128 + (g ^ (r & 7)) * 16;
   const bf16_t* ap[MT];
 #pragma unroll
@@ -381,7 +375,7 @@ __global__ __launch_bounds__(64 * W) void step_gemm_tall_kernel(const LmStepGemm
 #pragma unroll
     for (int x = 0; x < NX; ++x)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) load_weights(wp[x][h] + k, mine + b * STAGE + x * 2048 + h * 1024);
+      for (int h = 0; h < 2; ++h) load_weights(w_rows[x][h], at, 2u * k, mine + b * STAGE + x * 2048 + h * 1024);
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -399,30 +393,19 @@ __global__ __launch_bounds__(64 * W) void step_gemm_tall_kernel(const LmStepGemm
         for (int i = 0; i < MT; ++i)
           acc[x][h][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(md_bf16x8v, w[x][h]), __builtin_bit_cast(md_bf16x8v, af[b][h][i]), acc[x][h][i], 0, 0, 0);
   };
-#pragma unroll
-  for (int d = 0; d < D; ++d)
-    if (lo + d < hi) load(d, lo + d);
-  __builtin_amdgcn_sched_barrier(0);
   float factor[RR];
+  stream_units<D, P, !(NX == 4 && MT == 3)>(lo, hi, load, multiply, [&] {
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int i = 0; i < RR; ++i) {
-    f32x4 q = {0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < RR; ++i) {
+      f32x4 q = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int h = 0; h < 4; ++h)
-      if (h * 64 + r * 4 < a.sumsq_n) q += sq[i][h];
-    factor[i] = (q[0] + q[1]) + (q[2] + q[3]);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  for (int u = lo; u < hi; u += D) {
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const int left = hi - 1 - (u + d);
-      if (left < 0) break;
-      wait_units<D - 1, P>(left);
-      multiply(d);
-      if (left >= D) load(d, u + d + D);
+      for (int h = 0; h < 4; ++h)
+        if (h * 64 + r * 4 < a.sumsq_n) q += sq[i][h];
+      factor[i] = (q[0] + q[1]) + (q[2] + q[3]);
     }
-  }
+    __builtin_amdgcn_sched_barrier(0);
+  });
 #pragma unroll
   for (int i = 0; i < RR; ++i) {
     const int m = i * 4 * W + (tid >> 4);

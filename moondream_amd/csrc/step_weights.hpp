@@ -8,8 +8,12 @@ namespace {
 // read without bank conflicts.  A load into registers in the operand's shape has its neighbouring lanes in different rows, which costs the address unit 80 cycles per
 // KB, and 8 lanes to a row 38; into LDS 20.
 __device__ __forceinline__ uint32_t lds_address(char* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)p; }
-__device__ __forceinline__ void load_weights(const bf16_t* w, char* dst) {  // (2: non-temporal)
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)w, (__attribute__((address_space(3))) void*)dst, 16, 0, 2);
+// As buffer loads: beside a flat or global load into LDS, which counts as one of either memory, the compiler lets a use of ANY loaded register wait for all
+// loads under way, and every ring ran empty once in its length (see stream_units).  rows: of 8 or more rows of k from here on (base uniform); at: a lane's place in 8 of them
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t weight_rows(const bf16_t* base) { return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)0xffffffff, 0x00020000); }
+__device__ __forceinline__ uint32_t weight_at(int lane, int k) { return 2u * ((uint32_t)(lane >> 3) * (uint32_t)k + 8u * (uint32_t)((lane & 7) ^ (lane >> 3))); }
+__device__ __forceinline__ void load_weights(__amdgpu_buffer_rsrc_t rows, uint32_t at, uint32_t offset, char* dst) {  // (2: non-temporal)
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (__attribute__((address_space(3))) void*)dst, 16, at, offset, 0, 2);
 }
 // One operand, or the two of a unit of 16 columns, for each x: in assembly, as the compiler would wait for all loads into LDS that are under way
 template <int NX>
@@ -40,6 +44,68 @@ __device__ __forceinline__ void wait_units(int left) {
   if constexpr (D == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   else if (left >= D) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(D * P) : "memory");
   else wait_units<D - 1, P>(left);
+}
+
+// The units lo .. hi - 1 of a wave, D under way: load(b, u) requests unit u (P loads, always) into buffer b, multiply(b) uses it; between() runs behind the
+// first requests.  PEELED: the loads of the loop stand under no condition.  The compiler counts loads into registers by itself; where one may not have been
+// issued it waits as if it had not, and the ring runs short once in its length.  It costs registers and instructions, so not where workgroups are many and short.
+template <int D, int P, bool PEELED = true, class Load, class Multiply, class Between>
+__device__ __forceinline__ void stream_units(int lo, int hi, Load load, Multiply multiply, Between between) {
+  if constexpr (!PEELED) {
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (lo + d < hi) load(d, lo + d);
+    between();
+    for (int u = lo; u < hi; u += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        const int left = hi - 1 - (u + d);
+        if (left < 0) break;
+        wait_units<D - 1, P>(left);
+        multiply(d);
+        if (left >= D) load(d, u + d + D);
+      }
+    }
+  } else if (hi - lo >= D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(d, lo + d);
+    between();
+    int u = lo;
+    for (; u + 2 * D <= hi; u += D)
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        wait_units<D - 1, P>(D - 1);
+        multiply(d);
+        load(d, u + D + d);
+      }
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int left = hi - 1 - (u + d);
+      wait_units<D - 1, P>(left);
+      multiply(d);
+      if (left >= D) load(d, u + D + d);
+    }
+    u += D;
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d) {
+      const int left = hi - 1 - (u + d);
+      if (left < 0) break;
+      wait_units<D - 1, P>(left);
+      multiply(d);
+    }
+  } else {
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d)
+      if (lo + d < hi) load(d, lo + d);
+    between();
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d) {
+      const int left = hi - 1 - (lo + d);
+      if (left < 0) break;
+      wait_units<D - 1, P>(left);
+      multiply(d);
+    }
+  }
 }
 
 }  // namespace

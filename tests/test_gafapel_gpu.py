@@ -198,6 +198,12 @@ def test_weights_of_experts_through_lds(width, ff):
         assert float(U.logit_errors(run(m, t, cuts), want).sort().values[-2]) < TOL[BF16]  # (a row whose choice is close may choose otherwise in bf16)
 
 
+@pytest.mark.parametrize("width,ff", [(832, 704), (896, 1024)], ids=str)
+def test_units_of_an_experts_wave_past_two_rings(width, ff):
+    """Two waves' parts of K of 6 and 7, 5 and 6, 7, and 8 units of 64, three under way: every number of units behind the loop whose loads stand under no condition."""
+    test_weights_of_experts_through_lds(width, ff)
+
+
 @dtypes
 def test_one_expert_takes_every_row(dtype):
     """The other experts have no rows at all."""

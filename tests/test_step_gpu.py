@@ -165,6 +165,13 @@ def test_weights_through_lds(width, vdim, ff, vocab):
             m.close_sequence(s)
 
 
+@pytest.mark.parametrize("width", [1088, 2624, 3648], ids=str)
+def test_units_of_a_wave_past_two_rings(width):
+    """Eight waves' parts of K of 2 and 3, 5 and 6, 7 and 8 units, two waves' of 8 and 9 (two or three units under way): the loop whose loads stand under no
+    condition runs not at all, once, and more often, and leaves every number of units to the code behind it."""
+    test_weights_through_lds(width, 32, width - 8, 120)
+
+
 @pytest.mark.parametrize("rows", [3, 40, 200])
 @pytest.mark.parametrize("which", ["in_proj", "out_proj", "gate_up", "down", "head"])
 def test_misaligned_weights_are_refused(rows, which):
