@@ -7,7 +7,7 @@
 //   attn_prep_step_kernel   the same for a decode step (one row per sequence), up to 8192 columns, in registers
 //   attn_prep_block_kernel  the same for 8 positions per workgroup (prefill, up to 4096 columns)
 //   conv_state_kernel    the last projections of every sequence of the step -> its slot (row p % taps of the slot's ring)
-//   attn_plain_kernel    one workgroup per query row, fp32 on the vector ALUs: any dtype, any head size
+//   attn_plain_kernel    one workgroup per query row or two, fp32 on the vector ALUs: any dtype, any head size
 //   attn_mfma_kernel     bf16 prefill on the matrix cores: 16 queries x all heads per workgroup
 //   attn_heads_*         bf16 decode step with one key head per query head: see there
 //   attn_decode_kernel   any other bf16 decode step: split-key attention behind attn_prep_kernel (made in every split, the convolution and norms
@@ -332,62 +332,76 @@ __global__ __launch_bounds__(256) void conv_state_kernel(const LmAttn a, int nco
 // ---------------------------------------------------------------------------------------------------------------------------
 constexpr int PLAIN_TK = 64;
 
-// Its cost is the keys' and values' way through L2, once per row: eight elements of a key, or of eight keys, per load (380 rows of 190 keys, 16
-// heads of 128, fp32: 93 us, 560 us with one at a time).  Sums run over coordinates and keys in order, one chain each.
-template <typename T>
-__global__ __launch_bounds__(256) void attn_plain_kernel(const LmAttn a) {
-  extern __shared__ __attribute__((aligned(16))) float sm[];
+// A row's tiles are a chain of loads, mixture, softmax and loads again: eight waves per row (380 rows of 190 keys, 16 heads of 128, fp32: four waves 93 us, 560 us with
+// one element per load; eight or sixteen 60).  NR rows that follow one another in a sequence (and, with chunks, begin at the same key): a key or value is read once for all of them.  Sums run over
+// coordinates and keys in order, one chain each: the same bits whatever NR and NT.
+inline int plain_lds(const LmAttn& a, int nr) { return nr * (a.heads * (a.dp + a.vp) + 2 * a.heads * PLAIN_TK + 3 * a.heads) * 4; }
+template <typename T, int NT, int NR>
+__device__ __forceinline__ void attn_plain_rows(const LmAttn& a, int row, float* sm) {
   const int H = a.heads, G = a.kv_heads, dp = a.dp, vp = a.vp, rep = H / G;
-  float* qs = sm;                      // [H][dp]
-  float* acc = qs + H * dp;            // [H][vp]
-  float* raw = acc + H * vp;           // [H][TK]
-  float* mixed = raw + H * PLAIN_TK;   // [H][TK]
-  float* ms = mixed + H * PLAIN_TK;    // [H] running maximum
-  float* ls = ms + H;                  // [H] running sum
-  float* al = ls + H;                  // [H] rescale of this tile
-  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  float* qs = sm;                           // [NR][H][dp]
+  float* acc = qs + NR * H * dp;            // [NR][H][vp]
+  float* raw = acc + NR * H * vp;           // [NR][H][TK]
+  float* mixed = raw + NR * H * PLAIN_TK;   // [NR][H][TK]
+  float* ms = mixed + NR * H * PLAIN_TK;    // [NR][H] running maximum
+  float* ls = ms + NR * H;                  // [NR][H] running sum
+  float* al = ls + NR * H;                  // [NR][H] rescale of this tile
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int seq = a.r.row_seq[row], i = a.r.row_pos[row], slot = a.r.seq_slot[seq];
   const T* kb = (const T*)a.k + (int64_t)slot * G * a.ctx * dp;
   const T* vb = (const T*)a.v + (int64_t)slot * G * a.ctx * vp;
-  for (int c = tid; c < H * dp; c += 256) qs[c] = ldf((const T*)a.q + (int64_t)row * H * dp + c);
-  for (int c = tid; c < H * vp; c += 256) acc[c] = 0.f;
-  for (int h = tid; h < H; h += 256) {
+  for (int c = tid; c < NR * H * dp; c += NT) qs[c] = ldf((const T*)a.q + (int64_t)row * H * dp + c);
+  for (int c = tid; c < NR * H * vp; c += NT) acc[c] = 0.f;
+  for (int h = tid; h < NR * H; h += NT) {
     ms[h] = -INFINITY;
     ls[h] = 0.f;
   }
   __syncthreads();
   const int first = a.chunk > 0 ? i / a.chunk * a.chunk : 0;
-  for (int j0 = first; j0 <= i; j0 += PLAIN_TK) {
-    const int n = min(PLAIN_TK, i + 1 - j0);
-    for (int e = tid; e < H * PLAIN_TK; e += 256) {
+  for (int j0 = first; j0 < i + NR; j0 += PLAIN_TK) {
+    int n[NR];  // keys of this tile that a row sees
+#pragma unroll
+    for (int r = 0; r < NR; ++r) n[r] = max(0, min(PLAIN_TK, i + r + 1 - j0));
+    for (int e = tid; e < H * PLAIN_TK; e += NT) {
       const int g = e / PLAIN_TK, jj = e - g * PLAIN_TK;
-      if (jj >= n) continue;
-      float s = 0.f;
+      if (jj >= n[NR - 1]) continue;
+      float s[NR];
+#pragma unroll
+      for (int r = 0; r < NR; ++r) s[r] = 0.f;
 #pragma unroll 4
       for (int d = 0; d < dp; d += 8) {  // (coordinates behind the head's are zeros)
         const auto k = ld8(kb + key_index(j0 + jj, g / rep, d, G, dp));
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
-          const f32x4 kv = half8(k, hf), qv = *(const f32x4*)(qs + g * dp + d + 4 * hf);
+          const f32x4 kv = half8(k, hf);
 #pragma unroll
-          for (int t = 0; t < 4; ++t) s = __builtin_fmaf(qv[t], kv[t], s);
+          for (int r = 0; r < NR; ++r) {
+            const f32x4 qv = *(const f32x4*)(qs + (r * H + g) * dp + d + 4 * hf);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) s[r] = __builtin_fmaf(qv[t], kv[t], s[r]);
+          }
         }
       }
-      raw[e] = __builtin_fmaf(a.scale, s, -(a.slope[g] * (float)(i - (j0 + jj))));
+#pragma unroll
+      for (int r = 0; r < NR; ++r) raw[r * H * PLAIN_TK + e] = __builtin_fmaf(a.scale, s[r], -(a.slope[g] * (float)(i + r - (j0 + jj))));
     }
     __syncthreads();
-    for (int e = tid; e < H * PLAIN_TK; e += 256) {
-      const int h = e / PLAIN_TK, jj = e - h * PLAIN_TK;
+    for (int e = tid; e < NR * H * PLAIN_TK; e += NT) {
+      const int r = e / (H * PLAIN_TK), h = e / PLAIN_TK - r * H, jj = e % PLAIN_TK;
       float s = -INFINITY;
-      if (jj < n) {
+      if (jj < min(PLAIN_TK, i + r + 1 - j0)) {
         s = 0.f;
 #pragma unroll 4
-        for (int g = 0; g < H; ++g) s += a.mix[h * H + g] * raw[g * PLAIN_TK + jj];
+        for (int g = 0; g < H; ++g) s += a.mix[h * H + g] * raw[(r * H + g) * PLAIN_TK + jj];
       }
       mixed[e] = s;
     }
     __syncthreads();
-    for (int h = wave; h < H; h += 4) {
+    for (int h = wave; h < NR * H; h += NT / 64) {
+      if (j0 > i + h / H) {  // (uniform) no key of this tile
+        if (lane == 0) al[h] = 1.f;
+        continue;
+      }
       const float s = mixed[h * PLAIN_TK + lane];
       const float mo = ms[h], mn = fmaxf(mo, wave_max(s));
       const float p = expf(s - mn), f = expf(mo - mn);
@@ -400,25 +414,54 @@ __global__ __launch_bounds__(256) void attn_plain_kernel(const LmAttn a) {
       }
     }
     __syncthreads();
-    for (int c = tid; c < H * vp; c += 256) {
+    for (int c = tid; c < H * vp; c += NT) {
       const int h = c / vp, d = c - h * vp;
       const float* p = mixed + h * PLAIN_TK;
-      float o = acc[c] * al[h];
-      auto one = [&](int jj) { o = __builtin_fmaf(p[jj], ldf(vb + value_index(j0 + jj, h / rep, d, G, vp)), o); };
-      const int lo = min(-j0 & 7, n), hi = lo + ((n - lo) & ~7);  // the values of a row of eight keys lie together
+      float o[NR];
+#pragma unroll
+      for (int r = 0; r < NR; ++r) o[r] = acc[r * H * vp + c] * al[r * H + h];
+      auto one = [&](int jj) {
+        const float v = ldf(vb + value_index(j0 + jj, h / rep, d, G, vp));
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+          if (jj < n[r]) o[r] = __builtin_fmaf(p[r * H * PLAIN_TK + jj], v, o[r]);
+      };
+      const int lo = min(-j0 & 7, n[0]), hi = lo + ((n[0] - lo) & ~7);  // the values of a row of eight keys lie together
       for (int jj = 0; jj < lo; ++jj) one(jj);
 #pragma unroll 4
       for (int jj = lo; jj < hi; jj += 8) {
         const auto v = ld8(vb + value_index(j0 + jj, h / rep, d, G, vp));
 #pragma unroll
-        for (int t = 0; t < 8; ++t) o = __builtin_fmaf(p[jj + t], half8(v, t / 4)[t & 3], o);
+        for (int t = 0; t < 8; ++t)
+#pragma unroll
+          for (int r = 0; r < NR; ++r) o[r] = __builtin_fmaf(p[r * H * PLAIN_TK + jj + t], half8(v, t / 4)[t & 3], o[r]);
       }
-      for (int jj = hi; jj < n; ++jj) one(jj);
-      acc[c] = o;
+      for (int jj = hi; jj < n[NR - 1]; ++jj) one(jj);
+#pragma unroll
+      for (int r = 0; r < NR; ++r) acc[r * H * vp + c] = o[r];
     }
     __syncthreads();
   }
-  for (int c = tid; c < H * vp; c += 256) stf((T*)a.out + (int64_t)row * a.ldo + in_chunks(c, a.out_chunk), acc[c] / ls[c / vp]);
+  for (int c = tid; c < NR * H * vp; c += NT) {
+    const int r = c / (H * vp), cc = c - r * H * vp;
+    stf((T*)a.out + (int64_t)(row + r) * a.ldo + in_chunks(cc, a.out_chunk), acc[c] / ls[r * H + cc / vp]);
+  }
+}
+template <typename T, int NT, int NR>
+__global__ __launch_bounds__(NT) void attn_plain_kernel(const LmAttn a) {
+  extern __shared__ __attribute__((aligned(16))) float sm[];
+  const int row = blockIdx.x * NR, end = min(row + NR, a.r.n_rows);
+  if constexpr (NR > 1) {  // all of one sequence, from the same key on?
+    const int last = end - 1, i = a.r.row_pos[row];
+    if (end - row == NR && a.r.row_seq[row] == a.r.row_seq[last] && (a.chunk <= 0 || i / a.chunk == (i + NR - 1) / a.chunk)) {
+      attn_plain_rows<T, NT, NR>(a, row, sm);
+      return;
+    }
+  }
+  for (int r = row; r < end; ++r) {
+    attn_plain_rows<T, NT, 1>(a, r, sm);
+    __syncthreads();
+  }
 }
 
 template <typename T, int NT>
@@ -462,10 +505,13 @@ md_status prep(const LmAttn& a, bool state, hipStream_t s) {
 
 template <typename T>
 md_status plain(const LmAttn& a, hipStream_t s) {
-  const int lds = (a.heads * (a.dp + a.vp) + 2 * a.heads * PLAIN_TK + 3 * a.heads) * 4;
-  if (lds > 160 * 1024) return MD_ERR_UNSUPPORTED;
-  MD_TRY(md_ensure_dynamic_lds((const void*)attn_plain_kernel<T>, 160 * 1024));
-  hipLaunchKernelGGL(attn_plain_kernel<T>, dim3(a.r.n_rows), dim3(256), lds, s, a);
+  if (plain_lds(a, 1) > 160 * 1024) return MD_ERR_UNSUPPORTED;
+  // Pairs of rows where that still leaves a workgroup per CU: up to there the chain of a row's tiles bounds it, beyond the reads do (24 layers, 12 of attention, 16 heads of
+  // 128, one row and two per workgroup: 380 tokens 12.4 and 12.8 ms, 1000 31.5 and 30.5, 3 x 833 71.4 and 68.5)
+  const int nr = a.r.n_rows > 512 && a.r.n_rows >= 8 * a.r.n_seq && plain_lds(a, 2) <= 160 * 1024 ? 2 : 1, lds = plain_lds(a, nr);
+  const auto fn = nr == 2 ? attn_plain_kernel<T, 512, 2> : attn_plain_kernel<T, 512, 1>;
+  MD_TRY(md_ensure_dynamic_lds((const void*)fn, 160 * 1024));
+  hipLaunchKernelGGL(fn, dim3((a.r.n_rows + nr - 1) / nr), dim3(512), lds, s, a);
   return md_launch_status();
 }
 
