@@ -88,3 +88,20 @@ def test_a_model_with_graphs_is_no_cycle(monkeypatch):
     with engine.no_collection():
         del e
         assert gone() is None
+
+
+def test_layers_of_a_cache_as_one_tensor():
+    """What ``encode_image`` hands out is taken as one tensor, in every other form layer by layer."""
+    import torch
+
+    from moondream_amd.moondream import _layers_as_one
+
+    whole = torch.randn(4, 1, 3, 5, 8)
+    views = list(whole.unbind(0))
+    assert torch.equal(_layers_as_one(views, 4), whole)
+    part = [t[:, :, 1:4] for t in views]  # rows left out, strides kept
+    assert torch.equal(_layers_as_one(part, 4), whole[:, :, :, 1:4])
+    assert torch.equal(_layers_as_one(list(whole.transpose(0, 2).contiguous().transpose(0, 2).unbind(0)), 4), whole)
+    for other in ([t.clone() for t in views], views[::-1], views[:3], [views[0]] * 4, views[:3] + [views[3][:, :, :4]], views[:3] + [views[3].clone()],
+                  views[:3] + [views[3].double()], [views[k] for k in (0, 2, 1, 3)], [t[0] for t in views], [t.transpose(1, 2) if i == 2 else t for i, t in enumerate(views)]):
+        assert _layers_as_one(other, 4) is None

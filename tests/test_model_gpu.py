@@ -89,6 +89,24 @@ def test_encode_image_kv_matches_reference(tiny):
         compare(f"v{li}", v[0, :, ::rs], bits_to_bf16(g[f"img0.cap.v{li}"]), 1.5e-2)
 
 
+def test_encoded_images_load_alike_in_any_form(tiny):
+    """The caches as they come, as tensors of their own, and from host memory: the same rows in the slot, and none behind them."""
+    g, cfg, sd, model = tiny
+    enc = model.encode_image(golden_image(g, 0))
+    for caches in (enc.caches, [(k.clone(), v.clone()) for k, v in enc.caches], [(k.cpu(), v) for k, v in enc.caches]):
+        model._ensure_batch(2)
+        with torch.inference_mode():
+            model._kv_k.fill_(3.0)
+            model._kv_v.fill_(5.0)
+        model.load_encoded_image(type(enc)(pos=enc.pos, caches=caches), 1)
+        for l, (k, v) in enumerate(enc.caches):
+            assert torch.equal(model._kv_k[l, 1:2, :, : enc.pos], k) and torch.equal(model._kv_v[l, 1:2, :, : enc.pos], v)
+        assert bool((model._kv_k[:, 0] == 3.0).all()) and bool((model._kv_k[:, 1, :, enc.pos :] == 3.0).all()) and bool((model._kv_v[:, 1, :, enc.pos :] == 5.0).all())
+    with torch.inference_mode():
+        model._kv_k.zero_()
+        model._kv_v.zero_()
+
+
 @pytest.mark.parametrize("idx", [0, 1, 2])
 def test_greedy_token_ids_bit_exact_vs_reference(tiny, idx):
     g, cfg, sd, model = tiny
