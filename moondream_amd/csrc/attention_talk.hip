@@ -333,7 +333,7 @@ __global__ __launch_bounds__(256) void conv_state_kernel(const LmAttn a, int nco
 constexpr int PLAIN_TK = 64;
 
 // A row's tiles are a chain of loads, mixture, softmax and loads again: eight waves per row (380 rows of 190 keys, 16 heads of 128, fp32: four waves 93 us, 560 us with
-// one element per load; eight or sixteen 60).  NR rows that follow one another in a sequence (and, with chunks, begin at the same key): a key or value is read once for all of them.  Sums run over
+// one element per load; eight or sixteen 65).  NR rows that follow one another in a sequence (and, with chunks, begin at the same key): a key or value is read once for all of them.  Sums run over
 // coordinates and keys in order, one chain each: the same bits whatever NR and NT.
 inline int plain_lds(const LmAttn& a, int nr) { return nr * (a.heads * (a.dp + a.vp) + 2 * a.heads * PLAIN_TK + 3 * a.heads) * 4; }
 template <typename T, int NT, int NR>

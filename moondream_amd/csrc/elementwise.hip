@@ -341,50 +341,71 @@ __device__ __forceinline__ void load_logits8(const float* p, float (&v)[8]) {
 }
 
 // greedy argmax, ties -> lowest index; optionally bumps pos[b].  Rows hold round_up(vocab, 8) readable logits.
+// One row per workgroup, in a chain that the next step waits for: a batch of loads is requested at once and its logits compared by value alone (a thread's
+// indices rise).  51200 logits, one row 9.3 -> 6.7 us, 40 rows 9.9 -> 7.4.
 template <typename T>
 __global__ __launch_bounds__(1024) void argmax_kernel(const T* __restrict__ logits, int64_t ld,
                                                      int vocab, int suppress, int32_t* __restrict__ next,
                                                      int32_t* __restrict__ pos_inc) {
+  constexpr int NONE = 0x7fffffff, AHEAD = sizeof(T) == 2 ? 8 : 4;
   __shared__ float sv[16];
   __shared__ int si[16];
-  const int b = blockIdx.x;
+  const int b = blockIdx.x, chunks = (vocab + 7) >> 3;
   const T* lr = logits + (int64_t)b * ld;
   float best = -INFINITY;
-  int bi = 0x7fffffff;
-  // 16 waves per row: the single-sequence decode step waits on this kernel's dependent-load chain
-  for (int ch = threadIdx.x; ch < ((vocab + 7) >> 3); ch += 1024) {
-    float lv[8];
-    load_logits8(lr + ch * 8, lv);
+  int bi = NONE;
+  auto logits8 = [&](int ch, float (&lv)[8]) {
+    load_logits8(lr + min(ch, chunks - 1) * 8, lv);
+  };
+  auto mask = [&](int ch, float (&lv)[8]) {
+    if (ch == suppress >> 3 || ch * 8 + 8 > vocab)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int idx = ch * 8 + e;
-      const float v = (idx == suppress || idx >= vocab) ? -INFINITY : lv[e];
-      if (v > best || (v == best && idx < bi)) {
-        best = v;
-        bi = idx;
-      }
+      for (int e = 0; e < 8; ++e)
+        if (ch * 8 + e == suppress || ch * 8 + e >= vocab) lv[e] = -INFINITY;
+  };
+  for (int c0 = threadIdx.x; c0 < chunks; c0 += 1024 * AHEAD) {
+    float lv[AHEAD][8];
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) logits8(c0 + 1024 * k, lv[k]);
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) {
+      mask(c0 + 1024 * k, lv[k]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (lv[k][e] > best) {
+          best = lv[k][e];
+          bi = (c0 + 1024 * k) * 8 + e;
+        }
     }
   }
+  if (bi == NONE)  // nothing above -inf: the first one that is not NaN
+    for (int ch = threadIdx.x; ch < chunks && bi == NONE; ch += 1024) {
+      float lv[8];
+      logits8(ch, lv);
+      mask(ch, lv);
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(best, o, 64);
-    const int oi = __shfl_xor(bi, o, 64);
+      for (int e = 7; e >= 0; --e)
+        if (lv[e] == best) bi = ch * 8 + e;
+    }
+  auto take = [&](float ov, int oi) {
     if (ov > best || (ov == best && oi < bi)) {
       best = ov;
       bi = oi;
     }
-  }
+  };
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) take(__shfl_xor(best, o, 64), __shfl_xor(bi, o, 64));
   if ((threadIdx.x & 63) == 0) {
     sv[threadIdx.x >> 6] = best;
     si[threadIdx.x >> 6] = bi;
   }
   __syncthreads();
+  if (threadIdx.x >= 64) return;
+  best = sv[threadIdx.x & 15];
+  bi = si[threadIdx.x & 15];
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) take(__shfl_xor(best, o, 64), __shfl_xor(bi, o, 64));
   if (threadIdx.x == 0) {
-    for (int w = 1; w < 16; ++w)
-      if (sv[w] > best || (sv[w] == best && si[w] < bi)) {
-        best = sv[w];
-        bi = si[w];
-      }
     // an all-NaN row selects nothing: fall back to id 0 rather than an out-of-range id that the
     // next md_embed_tokens would use as a table index
     next[b] = (bi >= vocab) ? 0 : bi;

@@ -990,6 +990,37 @@ def test_embed_and_argmax(lib):
     assert int(nxt[3]) == int(torch.argmax(ref[3]))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, BF16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("vocab", [1, 7, 8, 63, 8192, 8201, 32768, 65535, 65536, 65545, 140000])
+def test_argmax_at_the_edges_of_its_batches(lib, vocab, dtype):
+    """The largest logit at the first and last place of a thread's batch of loads and of the row, ties across threads and batches, a suppressed largest, padding above
+    everything, rows of -inf, of NaN, and of NaN but for some -inf."""
+    ld, n = (vocab + 7) // 8 * 8, 10
+    x = (torch.randn(n, ld, generator=torch.Generator().manual_seed(vocab)) * 2).to(dtype)
+    x[:, vocab:] = 99
+    places = sorted({p for p in (0, 5, vocab - 1, vocab // 2, 8191, 8192, 32767, 65528, 65536) if p < vocab})
+    for i, p in enumerate(places[:5]):
+        x[i, p] = 50
+    x[5, places] = 50  # ties: the lowest
+    x[6, :vocab] = float("-inf")
+    x[7, :vocab] = float("nan")
+    x[8, :vocab] = float("nan")
+    x[8, places[len(places) // 2 :]] = float("-inf")
+    x[9, places[0]], x[9, places[-1]] = 60, 55
+    for skip in (-1, places[0], vocab - 1):
+        want = []
+        for row in x[:, :vocab].float():
+            row = row.clone()
+            if skip >= 0:
+                row[skip] = float("-inf")
+            live = ~row.isnan()
+            want.append(int((row == row[live].max()).nonzero()[0]) if bool(live.any()) else 0)
+        nxt = torch.full((n,), -1, dtype=torch.int32, device="cuda")
+        d = x.cuda()
+        _lib.check((lib.md_argmax_f32 if dtype == torch.float32 else lib.md_argmax_bf16)(d.data_ptr(), ld, n, vocab, skip, nxt.data_ptr(), stream()))
+        assert nxt.tolist() == want, skip
+
+
 @pytest.mark.parametrize("th,tw", [(1, 1), (2, 3), (3, 4), (4, 1)])
 def test_stitch_pool_concat(lib, th, tw):
     from oracle import moondream_oracle as O
