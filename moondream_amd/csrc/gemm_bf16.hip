@@ -1141,8 +1141,18 @@ namespace {
 // though most of its rows are padding at first (a whole prefill through 32 experts of 2 x 1360 columns, 24 layers: 87 rows a group 8.29 -> 7.78 ms
 // against the 64 x 64 tile, 212 rows 11.8 -> 10.8 against 128 x 128, 612 rows 24.4 -> 21.5 and 1000 rows 35.3 -> 30.9 against an eight-wave
 // 256 x 256 tile; 50 rows: 7.15 either way).  Not for gates that stay in fp32 (k.round_first unset): its epilogue rounds them.
+// Tiles of 128 x 128 with operands of two slices in registers (gemm_mid.hip) from 28 rows on (32 experts of 2048, weights from memory, us, 64 x 64 / 128 x 128: 32
+// rows, 2816 / 5504 / 1408 columns 100 / 88, 186 / 159, 58 / 56, the products back 50 / 41, 94 / 76, 29 / 24; 50 rows 115 / 88 and 63 / 42; 22 rows 90 / 86, but 1408
+// columns 50 / 56).  From 64 on where a group's rows are one tile and their rounds of the CUs, priced as in by_rounds, cost 0.7 of the four-wave tile's at most (65 and 100
+// rows, 2816 columns: 107 / 91 and 109 / 94; where they promise 0.82, 2048 / 5504 / 1408 columns: 43 / 43, 168 / 175, 54 / 58), or those of 256 x 128 0.92 (137 / 175 rows,
+// 2816 columns, 352 four-wave tiles in two rounds: 133 / 107, 138 / 119; 217 rows, a pass of 24 layers 10.77 / 10.84 ms; 237 rows, some groups two tiles: 140 / 154).
 template <int EPI>
 md_status grouped_by_height(GemmK k, int per_group, hipStream_t stream) {
+  auto rounds = [&](int bn) { return (double)(((long)k.groups * ((k.n_store + bn - 1) / bn) + 255) / 256); };
+  const double by_four = rounds(256) * 256 * 256;
+  // (104, 200: one tile, with the spread of rows that choose at random)
+  if (per_group >= 28 && (per_group < 64 || (per_group <= 104 && rounds(128) * 128 * 128 / 0.61 <= 0.7 * by_four))) return md_gemm_mid_launch_grouped(k, EPI, 128, stream);
+  if (per_group >= 64 && per_group <= 200 && rounds(128) * 256 * 128 / 0.82 <= 0.92 * by_four) return md_gemm_mid_launch_grouped(k, EPI, 256, stream);
   if (per_group >= 64 && k.n_pad >= 256 && (EPI != MD_EPI_SILU || k.round_first) && md_gemm_w4_takes(k, EPI) && (uint64_t)k.groups * k.n_pad * k.ldw * 2 < (1ull << 32)) {
     k.group_m = 4;
     return md_gemm_w4_launch_grouped(k, EPI, stream);

@@ -131,6 +131,7 @@ md_status md_gemm_w4_launch_grouped(const GemmK& k, int epi, hipStream_t stream)
 bool md_gemm_w4_takes(const GemmK& k, int epi);  // shape limits of the four-wave kernel for this launch
 // gemm_mid.hip: tiles of bm (256 or 128) x 128, and fp32 sums of k.slices slices of K by 128 x 128 (k.partial); the bits of the four-wave kernel
 md_status md_gemm_mid_launch(const GemmK& k, int epi, int bm, hipStream_t stream);
+md_status md_gemm_mid_launch_grouped(const GemmK& k, int epi, int bm, hipStream_t stream);  // k.offsets: bias-free rows or MD_EPI_SILU
 md_status md_gemm_mid_partial(const GemmK& k, hipStream_t stream);
 void md_gemm_w4_set_grid(int v);     // persistent workgroups per launch of the four-wave kernel (0 = one per CU)
 void md_gemm_w4_set_debug(int half, uint32_t v);  // measurement builds: device buffer for in-kernel stamps

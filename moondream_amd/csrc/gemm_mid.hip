@@ -42,7 +42,8 @@ __device__ __forceinline__ void lds_read(bf16x8& dst, uint32_t addr) {
 }
 
 // PART: fp32 sums of a slice of K -> p.partial.  EPI as in gemm_bf16.hip; SiLU: a wave's 64 columns are 32 gates and their inputs
-template <int BM, int BN, int WM, int WN, int S, int EPI, bool PART>
+// GRP: a grouped product (GemmK.offsets): a tile's rows are slots of one group, gathered through row_of, its matrix is that group's
+template <int BM, int BN, int WM, int WN, int S, int EPI, bool PART, bool GRP>
 __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_mid_kernel(const GemmK p) {
   constexpr int NT = WM * WN * 64, TM = BM / WM, TN = BN / WN, MI = TM / 16, NI = TN / 16;
   constexpr int A_BYTES = BM * 128, STAGE = (BM + BN) * 128;
@@ -53,10 +54,20 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_mid_kernel(const GemmK p
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave / WN, wn = wave % WN;
 
   // slices of K apart, then a run of tiles per XCD, group_m row panels of a column panel after the other
-  const int tiles = p.tiles_m * p.tiles_n, L0 = xcd_remap(blockIdx.x, tiles * p.slices);
+  const int tiles = (GRP ? grouped_total(p.offsets, p.groups, BM) : p.tiles_m) * p.tiles_n;
+  if (GRP && (int)blockIdx.x >= tiles) return;  // (a grouped launch knows an upper bound)
+  const int L0 = xcd_remap(blockIdx.x, tiles * p.slices);
   const int slice = PART ? L0 / tiles : 0, L = PART ? L0 - slice * tiles : L0;
-  const int per_group = p.group_m * p.tiles_n, first_m = L / per_group * p.group_m, gsz = min(p.tiles_m - first_m, p.group_m);
-  const int tm = first_m + L % per_group % gsz, tn = L % per_group / gsz, m0 = tm * BM, n0 = tn * BN;
+  int m0, n0, m_end = p.M, group = 0;  // m_end: rows from there on belong to another group, or to nobody
+  if constexpr (GRP) {
+    // a row panel's columns after one another: few panels share weights, all of a panel's tiles its rows
+    if (!grouped_tile(p.offsets, p.groups, BM, L / p.tiles_n, group, m0, m_end)) return;
+    n0 = L % p.tiles_n * BN;
+  } else {
+    const int per_group = p.group_m * p.tiles_n, first_m = L / per_group * p.group_m, gsz = min(p.tiles_m - first_m, p.group_m);
+    m0 = (first_m + L % per_group % gsz) * BM;
+    n0 = L % per_group / gsz * BN;
+  }
 
   int nk = p.K / BK, k0 = 0;
   if constexpr (PART) {
@@ -68,7 +79,9 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_mid_kernel(const GemmK p
 #pragma unroll
   for (int j = 0; j < NA; ++j) {
     const int at = j * NT + tid, row = at >> 3, c = (at & 7) ^ ((row >> 1) & 7);
-    a_src[j] = (const char*)(p.A + (int64_t)min(m0 + row, p.M - 1) * p.lda + k0 * BK + c * 8);
+    int a_row = min(m0 + row, m_end - 1);
+    if (GRP && p.row_of) a_row = p.row_of[a_row];
+    a_src[j] = (const char*)(p.A + (int64_t)a_row * p.lda + k0 * BK + c * 8);
   }
 #pragma unroll
   for (int j = 0; j < NB; ++j) {
@@ -78,7 +91,7 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_mid_kernel(const GemmK p
       const int v = n0 + row, half = p.n_pad >> 1;
       n = min((v >> 6) * 32 + (v & 31), half - 1) + ((v & 32) ? half : 0);
     }
-    b_src[j] = (const char*)(p.W + (int64_t)n * p.ldw + k0 * BK + c * 8);
+    b_src[j] = (const char*)(p.W + (GRP ? group * p.group_stride : 0) + (int64_t)n * p.ldw + k0 * BK + c * 8);
   }
   auto issue = [&](auto piece_c, int stage) {
     constexpr int X = decltype(piece_c)::value;
@@ -131,6 +144,7 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_mid_kernel(const GemmK p
   wait_lds();
   __builtin_amdgcn_sched_barrier(0);
 
+  const bool live = m0 + wm * TM < m_end;
   // slice t: its operands are in f[t & 1].  STEADY: slice t + S exists
   auto step = [&](int t, auto buf_c, auto steady_c) {
     constexpr int B = decltype(buf_c)::value;
@@ -140,6 +154,10 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_mid_kernel(const GemmK p
     barrier();  // ... everybody's part of it; and everybody has read slice t
     const bool more = STEADY || t + 1 < nk, refill = STEADY || t + S < nk;
     const int stage = t % S;
+    if (GRP && !live) {  // (wave-uniform) only padding: this wave's share of the copies
+      if (refill) static_for<0, P>([&](auto y) { issue(y, stage); });
+      return;
+    }
     const uint32_t st1 = (uint32_t)((t + 1) % S) * STAGE;
     static_for<0, MULS>([&](auto x_c) {
       constexpr int X = decltype(x_c)::value, H = X / (MI * NI), I = X / NI % MI, J = X % NI;
@@ -188,7 +206,7 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_mid_kernel(const GemmK p
       for (int q = 0; q < 8; ++q) {
         const int row = 4 * q + g, m = mw + 32 * b + row, n = nw + 4 * r;
         const f32x4 v = *(const f32x4*)(own + row * LD + 4 * r);
-        if (m < p.M && n < p.n_store) *(f32x4*)(dst + (int64_t)m * p.partial_ld + n) = v;
+        if (m < m_end && n < p.n_store) *(f32x4*)(dst + (int64_t)m * p.partial_ld + n) = v;
       }
     }
     return;
@@ -216,7 +234,7 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_mid_kernel(const GemmK p
         const int idx = q * 64 + lane, row = idx >> 2, ch = idx & 3;
         const u32x4 v = *(const u32x4*)(own + row * 64 + ((ch ^ ((row >> 1) & 3)) * 16));
         const int m = mw + 32 * b + row, n = (nw >> 1) + ch * 8;
-        if (m < p.M && n < (p.n_store >> 1)) *(u32x4*)(p.C + (int64_t)m * p.ldc + n) = v;
+        if (m < m_end && n < (p.n_store >> 1)) *(u32x4*)(p.C + (int64_t)m * p.ldc + n) = v;
       }
     }
     return;
@@ -238,7 +256,7 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_mid_kernel(const GemmK p
       for (int q = 0; q < 4; ++q) {
         const int m = mw + 32 * b + 8 * q + (lane >> 3), n = nw + (lane & 7) * 8;
         res[b][q] = u32x4{0u, 0u, 0u, 0u};
-        if (m < p.M && n < p.n_store) res[b][q] = *(const u32x4*)(p.R + (int64_t)(p.res_row_mod ? m % p.res_row_mod : m) * p.ldr + n);
+        if (m < m_end && n < p.n_store) res[b][q] = *(const u32x4*)(p.R + (int64_t)(p.res_row_mod ? m % p.res_row_mod : m) * p.ldr + n);
       }
 #pragma unroll
   for (int b = 0; b < MI / 2; ++b) {
@@ -254,7 +272,7 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_mid_kernel(const GemmK p
     for (int q = 0; q < 4; ++q) {
       const int row = 8 * q + (lane >> 3), ch = lane & 7, m = mw + 32 * b + row, n = nw + ch * 8;
       u32x4 v = *(const u32x4*)(own + row * 128 + ((ch ^ (row & 7)) * 16));
-      if (m >= p.M || n >= p.n_store) continue;
+      if (m >= m_end || n >= p.n_store) continue;
       if constexpr (EPI == MD_EPI_GELU) {
         if (n >= p.gelu_from)
 #pragma unroll
@@ -283,13 +301,13 @@ inline int mid_group(int tiles_m, int tiles_n, int slices, int bm, int bn) {
   return best;
 }
 
-template <int BM, int BN, int WM, int WN, int S, int EPI, bool PART>
+template <int BM, int BN, int WM, int WN, int S, int EPI, bool PART, bool GRP = false>
 md_status launch(GemmK k, hipStream_t s) {
   constexpr int lds = S * (BM + BN) * 128;
   static_assert(lds <= 163840 && lds >= WM * WN * 32 * 68 * 4, "LDS");
-  const auto fn = gemm_mid_kernel<BM, BN, WM, WN, S, EPI, PART>;
+  const auto fn = gemm_mid_kernel<BM, BN, WM, WN, S, EPI, PART, GRP>;
   MD_TRY(md_ensure_dynamic_lds((const void*)fn, lds));
-  k.tiles_m = (k.M + BM - 1) / BM;
+  k.tiles_m = GRP ? grouped_tiles(k.M, k.groups, BM) : (k.M + BM - 1) / BM;
   k.tiles_n = (k.n_store + BN - 1) / BN;
   if (!PART) k.slices = 1;
   k.group_m = mid_group(k.tiles_m, k.tiles_n, k.slices, BM, BN);
@@ -314,5 +332,10 @@ md_status md_gemm_mid_launch(const GemmK& k, int epi, int bm, hipStream_t s) {
     case MD_EPI_SILU: return by_height<MD_EPI_SILU>(k, bm, s);
     default: return MD_ERR_UNSUPPORTED;
   }
+}
+md_status md_gemm_mid_launch_grouped(const GemmK& k, int epi, int bm, hipStream_t s) {
+  if (epi == MD_EPI_SILU) return bm == 256 ? launch<256, 128, 4, 2, 3, MD_EPI_SILU, false, true>(k, s) : launch<128, 128, 2, 2, 4, MD_EPI_SILU, false, true>(k, s);
+  if (epi == MD_EPI_BIAS) return bm == 256 ? launch<256, 128, 4, 2, 3, MD_EPI_BIAS, false, true>(k, s) : launch<128, 128, 2, 2, 4, MD_EPI_BIAS, false, true>(k, s);
+  return MD_ERR_UNSUPPORTED;
 }
 md_status md_gemm_mid_partial(const GemmK& k, hipStream_t s) { return launch<128, 128, 2, 2, 4, MD_EPI_BIAS, true>(k, s); }
