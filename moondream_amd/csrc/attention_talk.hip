@@ -185,14 +185,14 @@ __device__ __forceinline__ void store8(float* p, const float (&v)[8]) {
 }
 
 // grid (blocks of 8 positions, sequences, q | k | v); a block starts at a multiple of 8, so its values fill whole operand rows of the
-// cache.  A thread owns columns 4 tid .., all 8 rows in registers (as many threads as that takes: 2048 columns, 40 / 900 / 14000 tokens 9.2 / 13.5 / 93 us, 256 threads with
-// eight columns each 12.2 / 15.9 / 101).  TAPS: taps of the convolution when they are
+// cache.  A thread owns columns 4 tid .., all 8 rows in registers (as many threads as that takes: 2048 columns, 40 / 900 / 14000 tokens 8.4 / 12.3 / 85 us, 256 threads with
+// eight columns each 10.1 / 13.4 / 96; 4096 columns 10.2 / 24.5 / 225, with sixteen each 16.1 / 31.3 / 315).  The norms' sums run in one order whatever the threads.  TAPS: taps of the convolution when they are
 // few (every projected row is then read once), 0: any number.
 template <typename T, int TAPS, int NT>
 __global__ __launch_bounds__(NT) void attn_prep_block_kernel(const LmAttn a) {
-  extern __shared__ __attribute__((aligned(16))) float hs[];  // values: [8][NT] sums of squares of four columns, then [8][kv_heads];
+  extern __shared__ __attribute__((aligned(16))) float hs[];  // [8][NT] sums of squares of four columns; values: then [8][kv_heads];
                                                               // bf16: then the finished cache rows, in the cache's order
-  __shared__ float red[NT / 64][8];
+  __shared__ float red[8][4];
   const int seq = blockIdx.y, part = blockIdx.z, tid = threadIdx.x;
   const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, pos0 = a.r.seq_pos0[seq], slot = a.r.seq_slot[seq];
   const int t0 = (pos0 / 8 + blockIdx.x) * 8, lo = max(t0, pos0), hi = min(t0 + 7, pos0 + len - 1);
@@ -205,13 +205,9 @@ __global__ __launch_bounds__(NT) void attn_prep_block_kernel(const LmAttn a) {
   const T* proj = (const T*)a.proj + (int64_t)(row0 - pos0) * a.ldp + col0;  // + position * ldp
   const T* ring = (const T*)a.conv_state + (int64_t)slot * a.taps * a.conv_ld + col0;
   f32x4 y[8];
-  float ss[8];
   const int c = 4 * tid;
 #pragma unroll
-  for (int r = 0; r < 8; ++r) {
-    ss[r] = 0.f;
-    y[r] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+  for (int r = 0; r < 8; ++r) y[r] = f32x4{0.f, 0.f, 0.f, 0.f};
   if (c < ncol) {
     auto input = [&](int p) { return p >= pos0 ? ld4(proj + (int64_t)p * a.ldp + c) : ld4(ring + (int64_t)(p % a.taps) * a.conv_ld + c); };
     if constexpr (TAPS > 0) {
@@ -241,28 +237,28 @@ __global__ __launch_bounds__(NT) void attn_prep_block_kernel(const LmAttn a) {
         y[r] += w * input(p);
       }
     }
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const float s = y[r][0] * y[r][0] + y[r][1] * y[r][1] + y[r][2] * y[r][2] + y[r][3] * y[r][3];
-      if (part < 2) ss[r] = s;
-      else hs[r * NT + tid] = s;
-    }
   }
+#pragma unroll
+  for (int r = 0; r < 8; ++r) hs[r * NT + tid] = y[r][0] * y[r][0] + y[r][1] * y[r][1] + y[r][2] * y[r][2] + y[r][3] * y[r][3];
+  __syncthreads();
   if (part < 2) {
+    // a row's sum in norm_row's order, whatever NT: 256 lanes take every 256th column group, then a butterfly per 64 lanes, then the four
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) ss[r] = wave_sum(ss[r]);
-    if ((tid & 63) == 0)
+    for (int k = wave; k < 32; k += NT / 64) {
+      const float* from = hs + (k >> 2) * NT + (k & 3) * 64 + (tid & 63);
+      float s = 0.f;
 #pragma unroll
-      for (int r = 0; r < 8; ++r) red[tid >> 6][r] = ss[r];
+      for (int i = 0; i < NT / 256; ++i) s += from[256 * i];
+      s = wave_sum(s);
+      if ((tid & 63) == 0) red[k >> 2][k & 3] = s;
+    }
     __syncthreads();
     const float* w = part == 0 ? a.q_norm : a.k_norm;
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
       if (t0 + r < lo || t0 + r > hi) continue;
-      float total = 0.f;
-#pragma unroll
-      for (int w = 0; w < NT / 64; ++w) total += red[w][r];
-      const float f = 1.0f / sqrtf(total / (float)(nh * a.dim) + a.eps);
+      const float f = 1.0f / sqrtf((red[r][0] + red[r][1] + red[r][2] + red[r][3]) / (float)(nh * a.dim) + a.eps);
       if (c >= ncol) continue;
       const f32x4 o = y[r] * f * *(const f32x4*)(w + c);
       if (part == 0) st4((T*)a.q + (int64_t)(row0 + t0 + r - pos0) * ncol + c, o);
@@ -280,7 +276,6 @@ __global__ __launch_bounds__(NT) void attn_prep_block_kernel(const LmAttn a) {
     return;
   }
   float* rn = hs + 8 * NT;
-  __syncthreads();
   for (int k = tid; k < 8 * nh; k += NT) {
     const int r = k / nh, g = k - r * nh, m = hp / 4;
     float s = 0.f;

@@ -406,6 +406,24 @@ def test_prompts_whose_tiles_are_cut_by_keys(heads, kv, dim, vdim, lens, chunk):
     assert float(U.logit_errors(got, want[0]).max()) < 7e-2
 
 
+@pytest.mark.parametrize("heads,dim", [(4, 32), (16, 64), (17, 64), (32, 64), (33, 64), (32, 128)], ids=str)
+def test_norms_of_prompts_sum_in_one_order(heads, dim):
+    """Keys in the cache after a whole prompt (eight positions per workgroup, 256 to 1024 threads) are those of its tokens one at a time (a row per
+    workgroup, 256 threads), bit for bit: fp32, where the products in front have one order of sums whatever their rows."""
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    cfg = U.config([U.attention(heads, heads, dim, dim, 2000)], width=64, vocab=60, ff=None)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), U.weights(cfg, 3, 1.5), dtype=F32, max_batch=2, max_context=64)
+    text = U.tokens(43, 60, 1)
+    whole, single = m.open_sequence(), m.open_sequence()
+    m.step([(whole, text, [])])
+    for t in text:
+        m.step([(single, [t], [])])
+    keys = m.state._slabs[0]["k"]
+    assert bool(keys[whole].any()) and torch.equal(keys[whole], keys[single])
+
+
 @pytest.mark.parametrize("heads,kv,dim,vdim,chunk", [(3, 1, 20, 40, 2000), (4, 4, 32, 32, 33), (20, 5, 32, 24, 64), (40, 40, 128, 128, 300)], ids=str)
 def test_fp32_rows_in_pairs(heads, kv, dim, vdim, chunk):
     """More than 512 rows in fp32: pairs of rows in one workgroup, pairs that two sequences or two chunks share, a last row without a second one, a second row with a tile
