@@ -1039,10 +1039,10 @@ md_status lm_attn_mfma(const LmAttn& args, hipStream_t s) {
 // ---------------------------------------------------------------------------------------------------------------------------
 // Prompts of up to some thousand tokens: attn_mfma_kernel has few tiles then, and each is a long chain.  The mixed scores of all pairs fit the caches (4 bytes of a head
 // and pair), so they go through memory:
-//   attn_pairs_scores_kernel  (32 keys, 16 queries, sequence): a wave's share of the heads, their scores to LDS in the order of the mixture's operand (two bf16 for
+//   attn_pairs_scores_kernel  (32 keys, 16 queries): a wave's share of the heads, their scores to LDS in the order of the mixture's operand (two bf16 for
 //                             a float), mixture, scale, distance and mask; the scores leave in the order of the other kernel's operand.  One workgroup row
 //                             more keeps the convolution's state
-//   attn_pairs_out_kernel     (head, 16 queries, sequence): softmax over all keys, weighted values; a wave has every NW-th block of 32 keys, whose scores are loaded
+//   attn_pairs_out_kernel     (head, 16 queries): softmax over all keys, weighted values; a wave has every NW-th block of 32 keys, whose scores are loaded
 //                             before the first is used, and the waves' sums meet in LDS
 // 32 heads of 64, one prompt of 40 / 250 tokens: 10 and 4 / 5 us a layer, against 28 / 53 us (parts of keys and their sum) and 6 for the state.  Whole prompts through
 // 24 layers (12 of attention), before and now, with attn_prep_block_kernel's share: 40 / 250 / 550 / 900 tokens 2.06 / 3.15 / 3.75 / 4.82 -> 1.78 / 2.58 / 3.33 / 4.53 ms; 4 x 50 / 200 / 500
@@ -1056,6 +1056,25 @@ constexpr int PAIRS_BLOCKS = 4, PAIRS_MOST = 8 * PAIRS_BLOCKS;  // blocks of 32 
 __host__ __device__ inline int pairs_blocks(int span) { return (span - 1 + 15 + 31) / 32 + 1; }
 __host__ __device__ inline int64_t pairs_at(int64_t slot, int h, int kb, int H, int blocks) { return ((slot * H + h) * blocks + kb) * 512; }
 
+// The sequence whose tile has this slot (talk_slot), and which of its tiles that is.  Workgroups are launched for slots, of which a sequence of one token has two, and not for
+// as many tiles as the longest of the sequences has: steps of ten layers, 4 heads of 64, 60 running sequences of 850 keys beside a prompt of 900 1.40 -> 0.94 ms (58 empty tiles
+// a running sequence, each in 30 blocks of keys; attn_mfma_kernel 1.13), 8 heads 1.57 -> 1.12 (1.30); even batches as before
+__device__ __forceinline__ int pairs_seq(const LmRows& r, int slot, int& tile) {
+  int seq = 0;
+  if (r.n_seq > 1) {
+    const int lane = threadIdx.x & 63;
+    seq = -1;
+    for (int s0 = 0; s0 < r.n_seq; s0 += 64) {
+      const int n = __popcll(__ballot(s0 + lane < r.n_seq && talk_slot(r.seq_row0[min(s0 + lane, r.n_seq - 1)], s0 + lane, 0) <= slot));
+      seq += n;
+      if (n < 64) break;
+    }
+  }
+  tile = slot - talk_slot(r.seq_row0[seq], seq, 0);
+  return seq;
+}
+inline int pairs_slots(const LmRows& r) { return r.n_rows / 16 + 2 * r.n_seq; }
+
 template <int HB, int D>
 __global__ __launch_bounds__(256) void attn_pairs_scores_kernel(const LmAttn a, int blocks) {
   constexpr int HP = 16 * HB, HW = HP / 4, dp = 32 * D, W = HW / 2;  // heads of a wave, dwords of them in an operand
@@ -1063,9 +1082,11 @@ __global__ __launch_bounds__(256) void attn_pairs_scores_kernel(const LmAttn a, 
   __shared__ Op b_lds[32][2][4][16];  // [key][high | low part][wave][query]
   __shared__ float mss[HP];
   const int H = a.heads, G = a.kv_heads, rep = H / G, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, q = lane >> 4;
-  const int kb = blockIdx.x, tile = blockIdx.y, seq = blockIdx.z;
+  const int kb = blockIdx.x, keeps = (int)blockIdx.y - ((int)gridDim.y - a.r.n_seq);  // >= 0: the sequence whose state is kept
+  int tile = 0;
+  const int seq = keeps >= 0 ? keeps : pairs_seq(a.r, blockIdx.y, tile);
   const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, pos0 = a.r.seq_pos0[seq], slot = a.r.seq_slot[seq];
-  if (tile == (int)gridDim.y - 1) {  // conv_state_kernel's work
+  if (keeps >= 0) {  // conv_state_kernel's work
     bf16_t* ring = (bf16_t*)a.conv_state + (int64_t)slot * a.taps * a.conv_ld;
     const int keep = min(len, a.taps - 1), pieces = a.conv_ld / 4, n_pieces = keep * pieces, step = gridDim.x * 256;
     constexpr int AT_ONCE = 8;
@@ -1199,7 +1220,9 @@ __global__ __launch_bounds__(64 * NW) void attn_pairs_out_kernel(const LmAttn a,
   constexpr int vp = 32 * C, NB = PAIRS_BLOCKS;
   __shared__ __attribute__((aligned(16))) float o_lds[NW][16][vp + 4], m_lds[NW][16], l_lds[NW][16];
   const int H = a.heads, G = a.kv_heads, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, q = lane >> 4;
-  const int h = blockIdx.x, tile = blockIdx.y, seq = blockIdx.z;
+  const int h = blockIdx.x;
+  int tile;
+  const int seq = pairs_seq(a.r, blockIdx.y, tile);
   const int row0 = a.r.seq_row0[seq], len = a.r.seq_row0[seq + 1] - row0, pos0 = a.r.seq_pos0[seq], slot = a.r.seq_slot[seq];
   const int t0 = (pos0 / 16 + tile) * 16, lo = max(t0, pos0), hi = min(t0 + 15, pos0 + len - 1);
   if (lo > hi) return;
@@ -1315,13 +1338,13 @@ bool lm_attn_pairs_takes(const LmAttn& a, int span) {
 md_status lm_attn_pairs(const LmAttn& a, int span, hipStream_t s) {
   if (!lm_attn_pairs_takes(a, span)) return MD_ERR_UNSUPPORTED;
   MD_TRY(prep<bf16_t>(a, false, s));
-  const int blocks = pairs_blocks(span), tiles = (a.r.max_len + 30) / 16;
+  const int blocks = pairs_blocks(span), slots = pairs_slots(a.r);
   const auto scores = a.heads <= 16 ? pairs_scores_pick<1>(a.dp) : pairs_scores_pick<2>(a.dp);
   const auto out = blocks <= 2 * PAIRS_BLOCKS ? pairs_out_pick<2>(a.vp) : blocks <= 4 * PAIRS_BLOCKS ? pairs_out_pick<4>(a.vp) : pairs_out_pick<8>(a.vp);
   const int waves = blocks <= 2 * PAIRS_BLOCKS ? 2 : blocks <= 4 * PAIRS_BLOCKS ? 4 : 8;
-  hipLaunchKernelGGL(scores, dim3(blocks, tiles + 1, a.r.n_seq), dim3(256), 0, s, a, blocks);
+  hipLaunchKernelGGL(scores, dim3(blocks, slots + a.r.n_seq), dim3(256), 0, s, a, blocks);
   MD_TRY(md_launch_status());
-  hipLaunchKernelGGL(out, dim3(a.heads, tiles, a.r.n_seq), dim3(64 * waves), 0, s, a, blocks);
+  hipLaunchKernelGGL(out, dim3(a.heads, slots), dim3(64 * waves), 0, s, a, blocks);
   return md_launch_status();
 }
 

@@ -466,6 +466,30 @@ def test_prompts_whose_scores_go_through_memory(heads, kv, dim, vdim, chunk):
                 m.close_sequence(s)
 
 
+@pytest.mark.parametrize("count", [1, 63, 64, 65, 130])
+def test_scores_of_prompts_beside_many_running_sequences(count):
+    """Tiles found by their slots among fewer sequences than a wave has lanes, as many, one more and twice as many: single tokens and prompts of several tiles in
+    one step, at positions of every remainder; a second step reads the convolution's state that the first one kept."""
+    from moondream_amd.config import LayeredLMConfig
+    from moondream_amd.layered_lm import LayeredLM
+
+    cfg = U.config([U.attention(4, 2, 32, 32, 2000)], width=96, vocab=120, ff=None)
+    w = U.weights(cfg, 3, 1.5)
+    text = U.tokens(210, 120, 9)
+    ref = O.forward(cfg, w, text)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=BF16, max_batch=count, max_context=256)
+    at = [(29 * i) % 90 for i in range(count)]
+    slots = [m.open_sequence() for _ in at]
+    if any(at):
+        m.step([(s, text[:n], []) for s, n in zip(slots, at) if n])
+    for k in range(2):
+        new = [(1 if i % 5 else 33 + i % 20) for i in range(count)]
+        got = m.step([(s, text[a : a + n], range(n)) for s, a, n in zip(slots, at, new)])
+        want = torch.cat([ref[a : a + n] for a, n in zip(at, new)])
+        assert float(U.logit_errors(got, want).max()) < 7e-2, k
+        at = [a + n for a, n in zip(at, new)]
+
+
 @pytest.mark.parametrize("heads,kv,dim,vdim", [(4, 4, 32, 32), (12, 12, 96, 128), (32, 32, 64, 64)], ids=str)
 @pytest.mark.parametrize("lens,chunk", [([260], 2000), ([700], 2000), ([620, 3, 250, 431], 2000), ([900], 333), ([300] * 13, 2000), ([530] * 8, 2000)], ids=str)
 def test_prompts_whose_scores_stay_on_the_cu(heads, kv, dim, vdim, lens, chunk):
