@@ -1710,8 +1710,7 @@ md_status lm_attn_decode(const LmAttn& a, hipStream_t s) {
 // once.  How many keys there are is known on the device only (a captured step sees any number): workgroups beyond the last key leave at once.
 // 32 heads of 64, one sequence at 100 keys: 6.6 and 5.8 us a layer against 5.1, 11.9 and 4.7; a step of two such layers and two of retention, before and now: 1 / 8
 // sequences at 100 keys 217 / 232 -> 200 / 217 us, 8 at 1500 269 -> 250, 32 at 100 / 500 / 1500 286 / 367 / 508 -> 274 / 314 / 420, 64 at 500 / 1500 642 / 706 -> 494 / 696, 128
-// at 20 / 1500 528 / 1131 -> 523 / 1090; 16 heads of 128 within 1 % of the same.  64 heads read 256 bytes of scores per key and head: 64 of 64, 40 sequences at 500 keys
-// 648 -> 585, but 64 at 1200 1068 -> 1177, hence the limit of many_heads.  Keys and values past the caches: 64 at 1200 2 to 3 % faster, 40 at 100 2 % slower.
+// at 20 / 1500 528 / 1131 -> 523 / 1090; 16 heads of 128 within 1 % of the same.
 namespace {
 
 constexpr int HEADS_COLS = 256, HEADS_KEYS = 128, HEADS_SPAN = 256;
@@ -1976,13 +1975,20 @@ bool heads_takes(int H, int G, int dp, int vp, int taps, bool own_kv) {
 size_t lm_attn_heads_floats(int n_seq, int span, int H, int G, int dp, int vp, int taps, bool own_kv) {
   return heads_takes(H, G, dp, vp, taps, own_kv) ? (size_t)heads_part(n_seq, span, H, dp, vp).total : 0;
 }
-bool lm_attn_heads_takes(const LmAttn& a) {
+// Where the three launches of attn_decode_kernel are the better ones (steps of attention layers alone, ms, three launches / two).  Its workgroups read a head's scores from LDS, these from memory, H times for
+// every key, which counts against the 4 dim of keys and values from H = dim on: 64 heads of 64, 40 sequences at 200 / 500 / 1000 keys 0.90 / 0.73, 1.20 / 1.19, 1.79 / 1.97, 24 at 500 / 1000
+// 0.86 / 0.80, 1.18 / 1.25; 64 of 32, where the others are slower, 40 at 1500 1.91 / 1.79, 64 2.78 / 2.90; 32 of 32, 24 / 64 at 1000 0.477 / 0.477, 0.87 / 0.89.  The fewest keys of more than
+// 40 sequences: 64 of 64 at 30 0.72 / 0.79, 48 of 64 0.635 / 0.587.  One or two groups of columns, from where parts of a head are added up: 24 layers of 4 of 64, one sequence at 200 / 500 /
+// 1500 0.501 / 0.503, 0.508 / 0.546, 0.54 / 0.60, 40 at 500 0.78 / 0.75; 16 of 32, 24 / 40 at 1500 0.96 / 1.04, 1.23 / 1.32; but 4 of 128, 8 at 1000 0.69 / 0.66.
+bool lm_attn_heads_takes(const LmAttn& a, int span) {
   if (!heads_takes(a.heads, a.kv_heads, a.dp, a.vp, a.taps, a.own_kv)) return false;
-  const bool many_heads = a.heads > 32 && a.r.n_seq > 40;
-  return !many_heads || !lm_attn_decode_takes(a);
+  const int64_t H = a.heads, dp = a.dp, n_seq = a.r.n_seq;
+  const bool scores = H >= dp && n_seq * span * dp * dp > 20480 * H * H, many = H > 48 && n_seq > 40;
+  const bool few = H * dp <= 512 && dp < 128 && span > HEADS_SPAN && n_seq * dp <= 1280;
+  return !(scores || many || few) || !lm_attn_decode_takes(a);
 }
 md_status lm_attn_heads(const LmAttn& a, int span, hipStream_t s) {
-  if (!lm_attn_heads_takes(a)) return MD_ERR_UNSUPPORTED;
+  if (!heads_takes(a.heads, a.kv_heads, a.dp, a.vp, a.taps, a.own_kv)) return MD_ERR_UNSUPPORTED;
   const HeadsPart f = heads_part(a.r.n_seq, span, a.heads, a.dp, a.vp);
   const int groups = a.heads * a.dp / HEADS_COLS;
   auto scores = a.dp == 32 ? attn_heads_scores_kernel<1> : a.dp == 64 ? attn_heads_scores_kernel<2> : attn_heads_scores_kernel<4>;

@@ -434,7 +434,7 @@ struct Step {
     a.out_chunk = few ? 8 * b->n_rows : 8;
     a.part = w.attn_part;
     const int span = l.chunk > 0 ? std::min(l.chunk, b->max_ctx) : b->max_ctx;
-    if (m->dtype == MD_DTYPE_BF16 && b->max_len == 1 && (g_lm_kernels & 2) && lm_attn_heads_takes(a)) return lm_attn_heads(a, span, s);
+    if (m->dtype == MD_DTYPE_BF16 && b->max_len == 1 && (g_lm_kernels & 2) && lm_attn_heads_takes(a, span)) return lm_attn_heads(a, span, s);
     if (m->dtype == MD_DTYPE_BF16 && b->max_len == 1 && (g_lm_kernels & 2) && lm_attn_decode_takes(a)) {
       a.n_split = lm_attn_decode_splits(b->n_seq, span, &a.split_keys);
       return lm_attn_decode(a, s);

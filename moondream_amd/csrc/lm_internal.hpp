@@ -377,7 +377,7 @@ size_t lm_attn_decode_part_floats(int n_seq, int n_split, int heads, int vp);
 bool lm_attn_decode_takes(const LmAttn& a);
 md_status lm_attn_decode(const LmAttn& a, hipStream_t s);               // bf16 decode step: prep + split-key attention + combine
 // ... of heads with keys of their own, in two launches (span: most keys of a query)
-bool lm_attn_heads_takes(const LmAttn& a);
+bool lm_attn_heads_takes(const LmAttn& a, int span);
 size_t lm_attn_heads_floats(int n_seq, int span, int heads, int kv_heads, int dp, int vp, int taps, bool own_kv);
 md_status lm_attn_heads(const LmAttn& a, int span, hipStream_t s);
 
