@@ -96,7 +96,7 @@ __device__ __forceinline__ void st_coh64(void* p, uint64_t v) {
 // a row reads it until every tag is the block's.  Against a barrier that saves the acknowledgement of the stores, the flag and the wait for those
 // whose rows are not needed.
 __device__ __forceinline__ void st_pair(uint64_t* p, uint32_t pair, unsigned tag) { st_coh64(p, (uint64_t)tag << 32 | pair); }
-// two words
+// two words (each written whole by st_pair and read whole: an aligned 8-byte half of a 16-byte load is one access, so that a tag never comes with an older value)
 __device__ __forceinline__ bool is_block(const u32x4& v, unsigned tag) { return v[1] == tag && v[3] == tag; }
 
 // Grid barrier without atomics: workgroup b publishes the barrier's number in ITS word of a flag array once its stores
@@ -143,6 +143,7 @@ struct GridBarrier {
   template <class F>
   __device__ __forceinline__ void until(F look) {
     for (unsigned spins = 0; !__all(look()); ++spins) {
+      asm volatile("" ::: "memory");  // ld_coh128 is an ordinary load to the compiler: the next look reads again
       if (spins > B1_SPIN_LIMIT) {
         __hip_atomic_store(sync + 64 * 11, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         break;
