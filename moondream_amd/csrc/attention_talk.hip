@@ -1310,12 +1310,10 @@ bool pairs_form(int H, int dp, int vp) { return H <= 32 && dp <= 128 && vp <= 12
 
 template <int HB>
 TalkKernelBlocks pairs_scores_pick(int dp) {
-  switch (dp / 32) {
-    case 1: return attn_pairs_scores_kernel<HB, 1>;
-    case 2: return attn_pairs_scores_kernel<HB, 2>;
-    case 3: return attn_pairs_scores_kernel<HB, 3>;
-    default: return attn_pairs_scores_kernel<HB, 4>;
-  }
+  if (dp == 32) return attn_pairs_scores_kernel<HB, 1>;
+  if constexpr (HB == 1)  // (pairs_form: more than 16 heads up to 64 wide)
+    if (dp > 64) return dp == 96 ? attn_pairs_scores_kernel<1, 3> : attn_pairs_scores_kernel<1, 4>;
+  return attn_pairs_scores_kernel<HB, 2>;
 }
 template <int NW>
 TalkKernelBlocks pairs_out_pick(int vp) {
