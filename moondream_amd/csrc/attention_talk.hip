@@ -1331,7 +1331,8 @@ size_t lm_attn_pairs_floats_most(int n_rows, int n_seq, int span, int H, int dp,
   return pairs_form(H, dp, vp) ? (size_t)std::min(PAIRS_FLOATS, pairs_floats(n_rows, n_seq, span, H)) : 0;
 }
 bool lm_attn_pairs_takes(const LmAttn& a, int span) {
-  return pairs_form(a.heads, a.dp, a.vp) && pairs_blocks(span) <= PAIRS_MOST && pairs_floats(a.r.n_rows, a.r.n_seq, span, a.heads) <= PAIRS_FLOATS;
+  return pairs_form(a.heads, a.dp, a.vp) && pairs_blocks(span) <= PAIRS_MOST && pairs_floats(a.r.n_rows, a.r.n_seq, span, a.heads) <= PAIRS_FLOATS &&
+         pairs_slots(a.r) + a.r.n_seq <= 65535;  // (a grid's height; few keys of one head or two would allow more)
 }
 md_status lm_attn_pairs(const LmAttn& a, int span, hipStream_t s) {
   if (!lm_attn_pairs_takes(a, span)) return MD_ERR_UNSUPPORTED;
