@@ -294,3 +294,34 @@ def test_grouped_tiles_of_a_few_dozen_rows(width, ff, tokens):
     assert float(U.logit_errors(got, O.forward(cfg, w, t)).max()) < TOL[BF16]
     # both are within the oracle's 7e-2, so within twice that of one another: a token whose eight experts nearly cancel is 0.037 apart (257 tokens)
     assert U.logit_error(got, few) < 2 * TOL[BF16]
+
+
+@pytest.mark.parametrize("width,ff,tokens", [(64, 64, 112), (320, 320, 200), (192, 128, 257), (576, 576, 280), (1152, 1152, 560)], ids=str)
+@pytest.mark.parametrize("copied", [True, False], ids=["gates_seen", "products_seen"])
+def test_grouped_tiles_column_by_column(width, ff, tokens, copied):
+    """Every number that the experts add to the residual stream against 64 bits, at the tiles of 128 x 128 and (560 tokens) 256 x 128: with ``copied`` the second product hands
+    the gated columns on as they are, so that a wrong column of one expert shows whole, in either product."""
+    cfg, w = _expert_model(32, 8, ff, width=width)
+    cfg["max_positions"] = 600
+    w["pos"] = torch.zeros(600, width, dtype=BF16)
+    for k in range(32):
+        if copied:
+            w[f"l0.mlp.e{k}.down"] = torch.eye(width, ff).to(BF16)
+    t, got, before = U.tokens(tokens, 64, 3), [], []
+    m = load(cfg, w, BF16, max_batch=1, max_context=600)
+    m.step([(m.open_sequence(), t, [])], layer_out=got)
+    O.forward(dict(cfg, layers=[dict(layer, mlp=None) for layer in cfg["layers"]]), w, t, layers_out=before)
+    d = {n: x.double().cuda() for n, x in w.items()}
+    streams = before[0][None].cuda()
+    h = (O.rms_norm(O.stream_input(streams, d["l0.hc2.in"]), cfg["norm"]["eps"]) * d["l0.norm2"]).to(BF16).double()  # (what the experts read is bf16)
+    z = h @ d["l0.mlp.router"].T + d["l0.mlp.router.b"]
+    top = z.topk(8, -1)
+    share = torch.zeros_like(z).scatter(-1, top.indices, torch.softmax(top.values, -1))
+    parts = torch.stack([share[:, k : k + 1] * O.gated_mlp(d, f"l0.mlp.e{k}.", h) for k in range(32)])
+    want = O.stream_update(streams, d["l0.hc2.mix"], d["l0.hc2.out"], parts.sum(0)).sum(0)
+    # Roundings to bf16 of up to 2^-9 each: what the experts read (seen by gate and input), gated values, results: 2^-7 of a value if all add up, and of a row's values for one
+    # that its terms nearly cancel in; twice that for the largest of half a million, and twice again where a sum of such terms follows.  One expert's wrong column is a tenth of a
+    # row's values and more.
+    size = parts.abs().sum(0)
+    far = float(((got[0][0].double() - want).abs() / (size + size.pow(2).mean(-1, keepdim=True).sqrt()) / d["l0.hc2.out"].abs()).max())
+    assert far < (2.0 ** -6 if copied else 2.0 ** -5), far
