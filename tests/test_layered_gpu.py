@@ -129,9 +129,9 @@ def test_slots_are_used_again(name, dtype):
 
 @pytest.mark.parametrize("name", sorted(U.CONFIGS))
 def test_kernel_families_agree(name):
-    """The plain kernels and the matrix-core / decode kernels on the same bf16 model."""
+    """The plain kernels and the matrix-core / decode kernels on the same bf16 model, prompts' attention by size and as for long ones."""
     ts, out = toks(name), []
-    for mask in (0, 1, 2, 3):
+    for mask in (0, 1, 2, 3, 5, 7):
         m = model(name, BF16)
         m.lib.md_lm_set_kernels(mask)
         slots = [m.open_sequence() for _ in ts]
@@ -385,9 +385,20 @@ def test_command_line(tmp_path, name):
     assert [[int(x) for x in line.split()] for line in r.stdout.strip().splitlines()] == want
 
 
+@pytest.fixture(params=[3, 7], ids=["by_size", "as_for_long_ones"])
+def prompt_attention(request):
+    """Attention over prompts by the kernels that their size chooses, and by those of long prompts."""
+    from moondream_amd import _lib
+
+    lib = _lib.load()
+    lib.md_lm_set_kernels(request.param)
+    yield
+    lib.md_lm_set_kernels(3)
+
+
 @pytest.mark.parametrize("heads,kv,dim,vdim", [(4, 4, 32, 32), (16, 4, 64, 64), (12, 12, 96, 128), (32, 32, 64, 64), (20, 5, 32, 64)], ids=str)
 @pytest.mark.parametrize("lens,chunk", [([260], 2000), ([700], 2000), ([620, 3, 250, 431], 2000), ([900], 333)], ids=str)
-def test_prompts_whose_tiles_are_cut_by_keys(heads, kv, dim, vdim, lens, chunk):
+def test_prompts_whose_tiles_are_cut_by_keys(heads, kv, dim, vdim, lens, chunk, prompt_attention):
     """Prefill attention of so few query tiles that their keys are divided between workgroups: first tiles whole and last ones in parts, ragged
     sequences, chunks that begin inside a part, and a second portion behind odd positions."""
     from moondream_amd.config import LayeredLMConfig
@@ -424,7 +435,7 @@ def test_norms_of_prompts_sum_in_one_order(heads, dim):
     assert bool(keys[whole].any()) and torch.equal(keys[whole], keys[single])
 
 
-@pytest.mark.parametrize("heads,kv,dim,vdim,chunk", [(3, 1, 20, 40, 2000), (4, 4, 32, 32, 33), (20, 5, 32, 24, 64), (40, 40, 128, 128, 300)], ids=str)
+@pytest.mark.parametrize("heads,kv,dim,vdim,chunk", [(3, 1, 20, 40, 2000), (4, 4, 32, 32, 33), (20, 5, 32, 24, 64), (40, 40, 128, 128, 300), (64, 64, 128, 128, 300)], ids=str)
 def test_fp32_rows_in_pairs(heads, kv, dim, vdim, chunk):
     """More than 512 rows in fp32: pairs of rows in one workgroup, pairs that two sequences or two chunks share, a last row without a second one, a second row with a tile
     of its own, heads whose pairs do not fit LDS; the same logits as those rows alone, up to the order in which a product's sums run."""
@@ -512,7 +523,7 @@ def test_prompts_whose_scores_stay_on_the_cu(heads, kv, dim, vdim, lens, chunk):
 
 @pytest.mark.parametrize("lens", [[530] * 8, [300] * 16, [530] * 7 + [10], [530] * 7 + [500], [300] * 15, [300] * 13, [90] * 16],
                          ids=["eight", "sixteen", "ragged", "nearly", "fifteen", "thirteen", "short"])
-def test_prompts_of_eight_sequences(lens):
+def test_prompts_of_eight_sequences(lens, prompt_attention):
     """More query tiles than CUs: eight equal sequences (one to an XCD), sixteen, eight that differ, little and much, a last eight of seven, thirteen;
     short ones."""
     from moondream_amd.config import LayeredLMConfig
@@ -529,7 +540,7 @@ def test_prompts_of_eight_sequences(lens):
 
 
 @pytest.mark.parametrize("running,before,prompt", [(1, 300, 200), (3, 400, 290), (7, 20, 250), (15, 150, 40), (20, 300, 3), (31, 50, 330)], ids=str)
-def test_prompts_beside_single_tokens(running, before, prompt):
+def test_prompts_beside_single_tokens(running, before, prompt, prompt_attention):
     """Sequences of one query tile beside one of many, keys in parts and whole: every tile of every sequence."""
     from moondream_amd.config import LayeredLMConfig
     from moondream_amd.layered_lm import LayeredLM
@@ -573,7 +584,7 @@ def test_many_sequences_of_a_long_context(heads, kv, dim, vdim, count, ctx, chun
     assert float(e.max()) < 7e-2, e
 
 
-@pytest.mark.parametrize("heads,dim,taps", [(8, 30, 1), (4, 64, 4), (2, 128, 2), (64, 32, 3), (12, 60, 3), (64, 100, 4)], ids=str)
+@pytest.mark.parametrize("heads,dim,taps", [(8, 30, 1), (4, 64, 4), (2, 128, 2), (64, 32, 3), (12, 60, 3), (64, 100, 4), (48, 64, 3), (64, 64, 3)], ids=str)
 @pytest.mark.parametrize("chunk", [4000, 300])
 def test_decode_of_heads_with_keys_of_their_own(heads, dim, taps, chunk):
     """Scores and mixture in two launches: the first tokens (fewer than the convolution's taps), last keys at the edges of tiles of 16, of a
