@@ -586,6 +586,12 @@ md_status md_attention_decode_rope_f8(const void* qkv, int64_t ld, void* o, int6
 md_status md_kv_quantize_f8(const md_kv_cache* kv, int32_t n_layers, int32_t batch, int32_t n_heads, const int32_t* pos0,
                             int32_t pos_fixed, int32_t n_pos, void* stream);
 
+/* The first n_pos rows of every layer's K and V of the slot that kv->k / kv->v point at, between the slabs and tensors of their own (an image's
+ * snapshot: encode_image, load_encoded_image; moondream.py:259-268, 620-623): k, v: host arrays of n_layers device addresses, each of a
+ * contiguous bf16 [n_heads][n_pos][head_dim], 16-byte aligned; to_cache: into the slabs, else out of them. */
+md_status md_kv_copy(const md_kv_cache* kv, int32_t n_layers, int32_t n_heads, int32_t head_dim, int32_t n_pos, void* const* k, void* const* v,
+                     int32_t to_cache, void* stream);
+
 size_t md_text_workspace_bytes(const md_text_model* m, int32_t batch, int32_t q_len);
 
 /* text_decoder over a block of q_len new tokens per sequence (reference:

@@ -637,3 +637,63 @@ extern "C" md_status md_stitch_pool_concat(const void* feats, void* out, int64_t
   return md_stitch_pool_batched(feats, out, ld_out, 0, 1, dim, grid, margin, tiles_h, tiles_w,
                                 (hipStream_t)stream);
 }
+
+// ---------------------------------------------------------------------------
+// An image's rows of all layers, K and V, between the slabs and tensors of their own: one launch where a copy per tensor is 48 of 4.5 us.
+// Memory-bound; four pieces of 16 bytes per thread under way.
+// ---------------------------------------------------------------------------
+namespace {
+
+constexpr int KV_COPY_LAYERS = 64, KV_COPY_PIECES = 4;
+struct KvTensors {
+  void *k[KV_COPY_LAYERS], *v[KV_COPY_LAYERS];
+};
+
+template <bool TO_CACHE>
+__global__ __launch_bounds__(256) void kv_copy_kernel(bf16_t* k, bf16_t* v, int64_t layer_stride, int64_t head_stride,
+                                                      const KvTensors t, int row_pieces, int n_pieces) {
+  const int layer = blockIdx.y >> 1;
+  bf16_t* slab = ((blockIdx.y & 1) ? v : k) + layer * layer_stride;
+  u32x4* own = (u32x4*)((blockIdx.y & 1) ? t.v[layer] : t.k[layer]);
+  u32x4 x[KV_COPY_PIECES];
+  const int first = blockIdx.x * (256 * KV_COPY_PIECES) + threadIdx.x;
+  auto in_slab = [&](int at) { return (u32x4*)(slab + at / row_pieces * head_stride) + at % row_pieces; };  // row_pieces: of a head's rows
+#pragma unroll
+  for (int i = 0; i < KV_COPY_PIECES; ++i) {
+    const int at = min(first + 256 * i, n_pieces - 1);
+    x[i] = TO_CACHE ? own[at] : *in_slab(at);
+  }
+#pragma unroll
+  for (int i = 0; i < KV_COPY_PIECES; ++i) {
+    const int at = first + 256 * i;
+    if (at >= n_pieces) continue;
+    if (TO_CACHE) *in_slab(at) = x[i];
+    else own[at] = x[i];
+  }
+}
+
+}  // namespace
+
+extern "C" md_status md_kv_copy(const md_kv_cache* kv, int32_t n_layers, int32_t n_heads, int32_t head_dim, int32_t n_pos, void* const* k, void* const* v,
+                                int32_t to_cache, void* stream) {
+  MD_CHECK_ARG(kv && kv->k && kv->v && k && v && n_layers > 0 && n_heads > 0 && head_dim > 0 && head_dim % 8 == 0 && n_pos >= 0 && n_pos <= kv->ctx);
+  MD_CHECK_ARG((((uintptr_t)kv->k | (uintptr_t)kv->v) & 15) == 0 && kv->layer_stride % 8 == 0);
+  if (n_pos == 0) return MD_OK;
+  const int64_t pieces = (int64_t)n_heads * n_pos * head_dim / 8, head_stride = (int64_t)kv->ctx * head_dim;
+  MD_CHECK_ARG(pieces < (1 << 30));
+  for (int l = 0; l < n_layers; ++l) MD_CHECK_ARG(k[l] && v[l] && (((uintptr_t)k[l] | (uintptr_t)v[l]) & 15) == 0);
+  for (int l0 = 0; l0 < n_layers; l0 += KV_COPY_LAYERS) {
+    KvTensors t = {};
+    const int n = std::min(n_layers - l0, KV_COPY_LAYERS);
+    for (int l = 0; l < n; ++l) {
+      t.k[l] = k[l0 + l];
+      t.v[l] = v[l0 + l];
+    }
+    constexpr int PER = 256 * KV_COPY_PIECES;
+    hipLaunchKernelGGL(to_cache ? kv_copy_kernel<true> : kv_copy_kernel<false>, dim3((unsigned)((pieces + PER - 1) / PER), 2 * n), dim3(256), 0, (hipStream_t)stream,
+                       (bf16_t*)kv->k + l0 * kv->layer_stride, (bf16_t*)kv->v + l0 * kv->layer_stride, kv->layer_stride, head_stride, t,
+                       n_pos * (head_dim / 8), (int)pieces);
+    MD_TRY(md_launch_status());
+  }
+  return MD_OK;
+}

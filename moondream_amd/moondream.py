@@ -44,7 +44,7 @@ SpatialRefs = List[Union[Tuple[float, float], Tuple[float, float, float, float]]
 
 
 def _layers_as_one(parts: Sequence[torch.Tensor], layers: int) -> Optional[torch.Tensor]:
-    """[layers, ...] over tensors of one shape that lie at equal distances in one storage, as ``encode_image`` makes them (None: others)."""
+    """[layers, ...] over tensors of one shape that lie at equal distances in one storage, as host copies of stacked caches do (None: others)."""
     first = parts[0] if len(parts) == layers and layers > 1 else None
     if first is None or first.dim() != 4:
         return None
@@ -868,22 +868,41 @@ class MoondreamModel(DeviceEngine):
         with torch.inference_mode():
             self._ensure_batch(1)
             pos = self._prefill_images(self._run_vision_encoder(image)[None], 0, lora)
-            # one copy for all layers' keys, one for their values (a copy per layer: 0.1 ms each way, and as much again of the host's time)
-            caches = list(zip(self._kv_k[:, 0:1, :, :pos, :].clone().unbind(0), self._kv_v[:, 0:1, :, :pos, :].clone().unbind(0)))
+            # tensors of their own, filled by one launch (a copy per layer: 0.1 ms each way, and as much again of the host's time)
+            t = self.config.text
+            new = lambda: torch.empty(1, t.n_kv_heads, pos, t.head_dim, dtype=BF16, device=self._device)  # noqa: E731
+            caches = [(new(), new()) for _ in range(t.n_layers)]
+            self._copy_layers(caches, 0, False)
         return EncodedImage(pos=pos, caches=caches)
+
+    def _copy_layers(self, caches: Sequence[Tuple[torch.Tensor, torch.Tensor]], slot: int, to_cache: bool) -> bool:
+        """The rows of all layers between the slot and ``caches`` in one launch; False where these are not what the kernel takes (contiguous
+        bf16 tensors of one shape on the slabs' device)."""
+        t, device = self.config.text, self._kv_k.device
+        if len(caches) != t.n_layers or caches[0][0].dim() != 4:
+            return False
+        shape = (1, t.n_kv_heads, caches[0][0].shape[2], t.head_dim)
+        if shape[2] > t.max_context:
+            return False
+        if any(x.dtype != BF16 or x.device != device or x.shape != shape or not x.is_contiguous() or x.data_ptr() % 16 for c in caches for x in c):
+            return False
+        kv, at = self._kv_struct(slot), [(C.c_void_p * t.n_layers)(*(c[i].data_ptr() for c in caches)) for i in (0, 1)]
+        _lib.check(self.lib.md_kv_copy(C.byref(kv), t.n_layers, t.n_kv_heads, t.head_dim, shape[2], at[0], at[1], int(to_cache), self._stream()), "md_kv_copy")
+        return True
 
     def load_encoded_image(self, encoded_image: EncodedImage, slot: int = 0):
         """reference: moondream.py:620-623."""
         self._ensure_batch(slot + 1)
         with torch.inference_mode():
-            ks, vs = (_layers_as_one([c[i] for c in encoded_image.caches], self.config.text.n_layers) for i in (0, 1))
-            if ks is not None and vs is not None:
-                self._kv_k[:, slot : slot + 1, :, : ks.size(3), :] = ks
-                self._kv_v[:, slot : slot + 1, :, : vs.size(3), :] = vs
-            else:
-                for l, (k, v) in enumerate(encoded_image.caches):
-                    self._kv_k[l, slot : slot + 1, :, : k.size(2), :] = k
-                    self._kv_v[l, slot : slot + 1, :, : v.size(2), :] = v
+            if not self._copy_layers(encoded_image.caches, slot, True):
+                ks, vs = (_layers_as_one([c[i] for c in encoded_image.caches], self.config.text.n_layers) for i in (0, 1))
+                if ks is not None and vs is not None:
+                    self._kv_k[:, slot : slot + 1, :, : ks.size(3), :] = ks
+                    self._kv_v[:, slot : slot + 1, :, : vs.size(3), :] = vs
+                else:
+                    for l, (k, v) in enumerate(encoded_image.caches):
+                        self._kv_k[l, slot : slot + 1, :, : k.size(2), :] = k
+                        self._kv_v[l, slot : slot + 1, :, : v.size(2), :] = v
             if self._kv8_scales is not None:  # fp8 mode: rebuild the e4m3 copy of the rows just loaded
                 kv = self._kv_struct(slot)
                 t = self.config.text

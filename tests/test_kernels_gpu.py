@@ -1301,3 +1301,26 @@ def test_decode_attention_over_e4m3_kv_cache(lib):
         pr = torch.exp(s - s.amax(dim=1, keepdim=True))
         want = (torch.einsum("hn,hnd->hd", pr.to(BF16).float(), vd) / pr.sum(dim=1, keepdim=True)).to(BF16)
         compare(f"decode attention over the e4m3 cache, len {n}", o[bi].view(h, hd), want, 6e-3, 4e-2)
+
+
+@pytest.mark.parametrize("layers,heads,hd,n_pos", [(1, 1, 64, 1), (2, 3, 64, 43), (24, 4, 64, 128), (64, 2, 8, 5), (65, 2, 64, 9), (130, 1, 16, 17)], ids=str)
+def test_kv_copy(lib, layers, heads, hd, n_pos):
+    """Rows of all layers out of the slabs and into them: more layers than a launch takes, first and last pieces of a workgroup's, nothing behind the rows or in other slots."""
+    ctx, slots = 128, 3
+    slab = [randn(layers, slots, heads, ctx, hd, seed=90 + i) for i in (0, 1)]
+    kv = _lib.MdKvCache(slab[0][:, 1].data_ptr(), slab[1][:, 1].data_ptr(), slots * heads * ctx * hd, heads * ctx * hd, ctx)
+    own = [[torch.empty(heads, n_pos, hd, dtype=BF16, device="cuda") for _ in range(layers)] for _ in (0, 1)]
+    at = [(C.c_void_p * layers)(*(t.data_ptr() for t in x)) for x in own]
+    _lib.check(lib.md_kv_copy(C.byref(kv), layers, heads, hd, n_pos, at[0], at[1], 0, stream()))
+    for x, y in zip(own, slab):
+        assert torch.equal(torch.stack(x), y[:, 1, :, :n_pos])
+    want = [x.clone() for x in slab]
+    for i in (0, 1):
+        for l, t in enumerate(own[i]):
+            t.add_(1)
+            want[i][l, 1, :, :n_pos] = t
+    _lib.check(lib.md_kv_copy(C.byref(kv), layers, heads, hd, n_pos, at[0], at[1], 1, stream()))
+    assert torch.equal(slab[0], want[0]) and torch.equal(slab[1], want[1])
+    bad = (C.c_void_p * layers)(*(t.data_ptr() + 2 for t in own[0]))
+    for args in ((0, heads, hd, n_pos, at[0]), (layers, heads, 12, n_pos, at[0]), (layers, heads, hd, ctx + 1, at[0]), (layers, heads, hd, n_pos, bad)):
+        assert lib.md_kv_copy(C.byref(kv), *args[:4], args[4], at[1], 0, stream()) == 1

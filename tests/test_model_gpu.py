@@ -107,6 +107,42 @@ def test_encoded_images_load_alike_in_any_form(tiny):
         model._kv_v.zero_()
 
 
+def test_encoded_images_hold_their_own_bytes(tiny):
+    """One layer's tensor keeps and saves its own rows, not those of all layers; an image is pickled at its size; and caches of any other layout load as before."""
+    import pickle
+
+    g, cfg, sd, model = tiny
+    enc = model.encode_image(golden_image(g, 0))
+    own = [x for c in enc.caches for x in c]
+    size = sum(x.numel() * x.element_size() for x in own)
+    assert all(x.is_contiguous() and x.untyped_storage().nbytes() == x.numel() * x.element_size() for x in own)
+    assert size <= len(pickle.dumps(enc)) < size + 1000 * len(own)
+
+    def stacked(f):
+        ks, vs = (f(torch.stack([c[i] for c in enc.caches])).unbind(0) for i in (0, 1))
+        return list(zip(ks, vs))
+
+    ragged = [(k[:, :, : enc.pos - l], v[:, :, : enc.pos - l]) for l, (k, v) in enumerate(enc.caches)]
+    for caches in (stacked(lambda x: x), stacked(lambda x: x.cpu()), stacked(lambda x: x.float()), stacked(lambda x: x.transpose(2, 3).contiguous().transpose(2, 3)),
+                   stacked(lambda x: x[:, :, :, :5]), stacked(lambda x: x[:, :, :, :0]), ragged, [(k, v[:, :, :7]) for k, v in enc.caches],
+                   [tuple(torch.cat([x.flatten().new_zeros(1), x.flatten()])[1:].view(x.shape) for x in c) for c in enc.caches], enc.caches[:1],
+                   [(k[:, :1], v[:, :1]) for k, v in enc.caches]):
+        model._ensure_batch(2)
+        want = []
+        with torch.inference_mode():
+            for slab in (model._kv_k, model._kv_v):
+                slab.copy_(torch.arange(slab.shape[3], device="cuda").view(1, 1, 1, -1, 1) % 97)
+                want.append(slab.clone())
+            for l, c in enumerate(caches):
+                for i in (0, 1):
+                    want[i][l, 1:2, :, : c[i].size(2)] = c[i]
+        model.load_encoded_image(type(enc)(pos=enc.pos, caches=caches), 1)
+        assert torch.equal(model._kv_k, want[0]) and torch.equal(model._kv_v, want[1])
+    with torch.inference_mode():
+        model._kv_k.zero_()
+        model._kv_v.zero_()
+
+
 @pytest.mark.parametrize("idx", [0, 1, 2])
 def test_greedy_token_ids_bit_exact_vs_reference(tiny, idx):
     g, cfg, sd, model = tiny
