@@ -1037,7 +1037,7 @@ md_status lm_attn_mfma(const LmAttn& args, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
-// Prompts of up to some thousand tokens: attn_mfma_kernel has few tiles then, and each is a long chain.  The mixed scores of all pairs fit the caches (4 bytes of a head
+// Prompts of up to 978 keys (PAIRS_MOST blocks of 32) and 40 million scores: attn_mfma_kernel has few tiles then, and each is a long chain.  The mixed scores of all pairs fit the caches (4 bytes of a head
 // and pair), so they go through memory:
 //   attn_pairs_scores_kernel  (32 keys, 16 queries): a wave's share of the heads, their scores to LDS in the order of the mixture's operand (two bf16 for
 //                             a float), mixture, scale, distance and mask; the scores leave in the order of the other kernel's operand.  One workgroup row

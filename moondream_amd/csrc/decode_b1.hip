@@ -1,7 +1,7 @@
 // Single-sequence decode step as ONE persistent kernel (gfx950): all decoder blocks of one token -- layer norm, the fused
 // qkv|fc1 linear with GELU, RoPE + KV-slab write, attention over the slab, proj and fc2 with both residual adds -- run
-// inside one launch of one workgroup per CU, separated by grid barriers instead of kernel boundaries (reference: the
-// body of _decode_one_tok, moondream.py:183-192 -> text.py:128-160, at batch 1).
+// inside one launch of one workgroup per CU; phases wait for the rows they read, and once a block at a grid barrier, instead of at kernel
+// boundaries (reference: the body of _decode_one_tok, moondream.py:183-192 -> text.py:128-160, at batch 1).
 //
 // Why: at one sequence a decoder block is ~100 MB of weights (17 us at 6 TB/s) but four launches at ~4.5 us each
 // (profiles/r02 B = 1 trace); a grid barrier with one counter per XCD costs 2.0 us (profiles/r02_grid_barrier_probe.txt).

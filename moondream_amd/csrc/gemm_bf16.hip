@@ -1146,6 +1146,9 @@ namespace {
 // columns 50 / 56).  From 64 on where a group's rows are one tile and their rounds of the CUs, priced as in by_rounds, cost 0.7 of the four-wave tile's at most (65 and 100
 // rows, 2816 columns: 107 / 91 and 109 / 94; where they promise 0.82, 2048 / 5504 / 1408 columns: 43 / 43, 168 / 175, 54 / 58), or those of 256 x 128 0.92 (137 / 175 rows,
 // 2816 columns, 352 four-wave tiles in two rounds: 133 / 107, 138 / 119; 217 rows, a pass of 24 layers 10.77 / 10.84 ms; 237 rows, some groups two tiles: 140 / 154).
+// The rule sees the mean only.  Experts that are chosen unequally, 24 layers of 32, 30 / 37 / 52 / 65 / 100 / 137 / 175 rows on average, ms without and with these tiles: a router's bias spread over +-1.5
+// 6.24 / 6.49 / 7.20 / 7.51 / 9.07 / 9.71 / 10.38 and 5.84 / 5.95 / 6.48 / 6.93 / 8.72 / 9.74 / 10.47; over +-3, where most rows go to a few experts, 5.95 / 6.19 / 6.96 / 6.04 / 7.87 / 8.59 / 9.94 and
+// 5.04 / 5.18 / 5.83 / 6.13 / 7.41 / 8.17 / 9.94: up to 1.6 % slower in three of fourteen, up to 20 % faster in ten.
 template <int EPI>
 md_status grouped_by_height(GemmK k, int per_group, hipStream_t stream) {
   auto rounds = [&](int bn) { return (double)(((long)k.groups * ((k.n_store + bn - 1) / bn) + 255) / 256); };

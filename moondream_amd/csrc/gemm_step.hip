@@ -14,8 +14,9 @@
 // (rows 4 KB apart meet on few channels: output projection of 40 rows 9.9 us against 7.6).
 //
 // Units of K are under way without a gap in between (stream_units): while the weights' loads into LDS were global ones, every use of loaded activations waited for
-// all loads, once in a ring's length.  1 / 8 / 16 / 28 / 40 rows, before and since: gates 10.3 -> 9.7, 10.3 -> 9.9, 10.4 -> 10.0, 11.2 -> 10.9, 12.5 -> 12.2 us; 8192 columns, 40 rows
-// 10.5 -> 10.1, 4352 9.5 -> 9.0.  The residual products are bound by the activations and did not change; the head is not peeled.
+// all loads, once in a ring's length.  In a model's decode steps, before and since, in turn: gates of up to 8 / 16 / 32 / 40 rows 11.3 -> 10.7, 10.9 -> 10.5, 12.2 -> 11.3, 13.1 -> 12.7 us; 8192
+// columns 9.5 -> 9.2, 8.2 either way, 9.4 -> 9.1, 10.7 -> 10.2; 6144 columns of up to 8 and 16 rows 8.2 and 7.5 either way, 32 / 40 rows 9.4 -> 9.0, 10.6 -> 10.1.  The residual products are bound by
+// the activations and did not change.
 //
 // Measured, 2048 wide, 5440 feed-forward, one stream, one row (16 rows, 28, 40): 8192 columns 8.6 us (8.0, 8.8, 10.1), 33 MB; gates 9.7 us (10.0, 10.9, 12.2), 44 MB;
 // the two residual products 4.5 and 6.7 us (4.9 and 8.2; 5.7 and 10.0; 6.5 and 11.9), 8 and 22 MB; the head, 51200 columns, 35 us (36, 41, 45),

@@ -364,7 +364,7 @@ md_status lm_reduce_rows(const float* part, int slices, int64_t ldp, int64_t sli
 
 md_status lm_attn_prep(int dtype, const LmAttn& a, hipStream_t s);      // convolution, norms, cache rows, convolution state
 md_status lm_attn_plain(int dtype, const LmAttn& a, hipStream_t s);     // one workgroup per query row, any dtype
-// bf16 prompts of a few hundred tokens, scores through memory: lm_attn_prep and the rest (span: most keys of a query)
+// bf16 prompts of up to 978 keys and 40 million scores, scores through memory: lm_attn_prep and the rest (span: most keys of a query)
 bool lm_attn_pairs_takes(const LmAttn& a, int span);
 size_t lm_attn_pairs_floats_most(int n_rows, int n_seq, int span, int heads, int dp, int vp);  // of steps up to that size
 md_status lm_attn_pairs(const LmAttn& a, int span, hipStream_t s);
