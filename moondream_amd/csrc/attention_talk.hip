@@ -1305,6 +1305,8 @@ __global__ __launch_bounds__(64 * NW) void attn_pairs_out_kernel(const LmAttn a,
 }
 
 constexpr int64_t PAIRS_FLOATS = 40 << 20;  // most scores of a step
+// Slots, and half as many sequences at most, are a grid's height.  A slot has two blocks of a head's scores at least (pairs_blocks), which bounds them
+static_assert(PAIRS_FLOATS / (2 * 512) * 3 / 2 <= 65535, "grid height");
 int64_t pairs_floats(int n_rows, int n_seq, int span, int H) { return (int64_t)(n_rows / 16 + 2 * n_seq) * H * std::min(pairs_blocks(span), PAIRS_MOST) * 512; }
 bool pairs_form(int H, int dp, int vp) { return H <= 32 && dp <= 128 && vp <= 128 && (H <= 16 || dp <= 64); }
 
@@ -1331,8 +1333,7 @@ size_t lm_attn_pairs_floats_most(int n_rows, int n_seq, int span, int H, int dp,
   return pairs_form(H, dp, vp) ? (size_t)std::min(PAIRS_FLOATS, pairs_floats(n_rows, n_seq, span, H)) : 0;
 }
 bool lm_attn_pairs_takes(const LmAttn& a, int span) {
-  return pairs_form(a.heads, a.dp, a.vp) && pairs_blocks(span) <= PAIRS_MOST && pairs_floats(a.r.n_rows, a.r.n_seq, span, a.heads) <= PAIRS_FLOATS &&
-         pairs_slots(a.r) + a.r.n_seq <= 65535;  // (a grid's height; few keys of one head or two would allow more)
+  return pairs_form(a.heads, a.dp, a.vp) && pairs_blocks(span) <= PAIRS_MOST && pairs_floats(a.r.n_rows, a.r.n_seq, span, a.heads) <= PAIRS_FLOATS;
 }
 md_status lm_attn_pairs(const LmAttn& a, int span, hipStream_t s) {
   if (!lm_attn_pairs_takes(a, span)) return MD_ERR_UNSUPPORTED;
