@@ -327,9 +327,9 @@ __global__ __launch_bounds__(256) void conv_state_kernel(const LmAttn a, int nco
 // ---------------------------------------------------------------------------------------------------------------------------
 constexpr int PLAIN_TK = 64;
 
-// A row's tiles are a chain of loads, mixture, softmax and loads again: eight waves per row (380 rows of 190 keys, 16 heads of 128, fp32: four waves 93 us, 560 us with
-// one element per load; eight or sixteen 65).  NR rows that follow one another in a sequence (and, with chunks, begin at the same key): a key or value is read once for all of them.  Sums run over
-// coordinates and keys in order, one chain each: the same bits whatever NR and NT.
+// A row's tiles are a chain of loads, mixture, softmax and loads again, which waves shorten (380 rows of 190 keys, 16 heads of 128, fp32: four waves 93 us, 560 us with one element per load; eight or
+// sixteen 65).  NR rows that follow one another in a sequence (and, with chunks, begin at the same key): a key or value is read once for all of them.  Sums run over coordinates and keys in order, one
+// chain each: the same bits whatever NR and NT.
 inline int plain_lds(const LmAttn& a, int nr) { return nr * (a.heads * (a.dp + a.vp) + 2 * a.heads * PLAIN_TK + 3 * a.heads) * 4; }
 template <typename T, int NT, int NR>
 __device__ __forceinline__ void attn_plain_rows(const LmAttn& a, int row, float* sm) {
@@ -382,7 +382,7 @@ __device__ __forceinline__ void attn_plain_rows(const LmAttn& a, int row, float*
     }
     __syncthreads();
     for (int e = tid; e < NR * H * PLAIN_TK; e += NT) {
-      const int r = e / (H * PLAIN_TK), h = e / PLAIN_TK - r * H, jj = e % PLAIN_TK;
+      const int r = NR == 1 ? 0 : e / (H * PLAIN_TK), h = e / PLAIN_TK - r * H, jj = e % PLAIN_TK;
       float s = -INFINITY;
       if (jj < min(PLAIN_TK, i + r + 1 - j0)) {
         s = 0.f;
@@ -393,7 +393,7 @@ __device__ __forceinline__ void attn_plain_rows(const LmAttn& a, int row, float*
     }
     __syncthreads();
     for (int h = wave; h < NR * H; h += NT / 64) {
-      if (j0 > i + h / H) {  // (uniform) no key of this tile
+      if (NR > 1 && j0 > i + h / H) {  // (uniform) no key of this tile
         if (lane == 0) al[h] = 1.f;
         continue;
       }
@@ -438,24 +438,25 @@ __device__ __forceinline__ void attn_plain_rows(const LmAttn& a, int row, float*
     __syncthreads();
   }
   for (int c = tid; c < NR * H * vp; c += NT) {
-    const int r = c / (H * vp), cc = c - r * H * vp;
+    const int r = NR == 1 ? 0 : c / (H * vp), cc = c - r * H * vp;
     stf((T*)a.out + (int64_t)(row + r) * a.ldo + in_chunks(cc, a.out_chunk), acc[c] / ls[r * H + cc / vp]);
   }
 }
 template <typename T, int NT, int NR>
 __global__ __launch_bounds__(NT) void attn_plain_kernel(const LmAttn a) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
-  const int row = blockIdx.x * NR, end = min(row + NR, a.r.n_rows);
-  if constexpr (NR > 1) {  // all of one sequence, from the same key on?
-    const int last = end - 1, i = a.r.row_pos[row];
-    if (end - row == NR && a.r.row_seq[row] == a.r.row_seq[last] && (a.chunk <= 0 || i / a.chunk == (i + NR - 1) / a.chunk)) {
+  if constexpr (NR == 1) {
+    attn_plain_rows<T, NT, 1>(a, blockIdx.x, sm);
+  } else {
+    const int row = blockIdx.x * NR, end = min(row + NR, a.r.n_rows), last = end - 1, i = a.r.row_pos[row];
+    if (end - row == NR && a.r.row_seq[row] == a.r.row_seq[last] && (a.chunk <= 0 || i / a.chunk == (i + NR - 1) / a.chunk)) {  // all of one sequence, from the same key on
       attn_plain_rows<T, NT, NR>(a, row, sm);
       return;
     }
-  }
-  for (int r = row; r < end; ++r) {
-    attn_plain_rows<T, NT, 1>(a, r, sm);
-    __syncthreads();
+    for (int r = row; r < end; ++r) {
+      attn_plain_rows<T, NT, 1>(a, r, sm);
+      __syncthreads();
+    }
   }
 }
 
@@ -498,15 +499,35 @@ md_status prep(const LmAttn& a, bool state, hipStream_t s) {
   return md_launch_status();
 }
 
+// Eight waves where rows are so few that their chains bound it, four where CUs hold more rows than the keys' way needs, pairs of rows where that way does (ms of 12 layers, four waves / eight / pairs).
+// 16 heads of 128, fp32: one prompt of 300 / 700 / 900 tokens 2.32 / 1.79 / 2.35, 4.26 / 4.13 / 4.40, 5.70 / 6.47 / 5.40, 8 x 1000 61.8 / 50.9 / 34.4; 30 x 20, whose chains are short, 1.69 / 1.66 / 1.63.
+// 8 of 64: 300 / 1000 tokens 0.99 / 0.86 / 1.02, 2.21 / 2.19 / 2.30, 8 x 1000 11.1 / 12.0 / 10.0; 12 of 64: 800 tokens 2.38 / 2.43 / 2.81, 8 x 1000 16.1 / 17.7 / 15.1; 9 of 32: 5 x 500 2.61 / 2.71 / 2.74.  Up
+// to four heads leave half of eight waves idle: 4 of 32, 900 tokens 1.05 / 1.35 / 1.61; 2 of 64, 8 x 1000 5.04 / 7.12 / 6.57.  Where two workgroups with pairs do not fit a CU's LDS, pairs pay only if keys and
+// values outweigh the mixture: 40 of 128, 900 tokens / 3 x 900 19.6 / 17.6 / 19.5, 53.3 / 59.8 / 46.2; 64 of 64 21.4 / 16.0 / 20.9, 49.9 / 41.1 / 47.5; 48 of 64, 3 x 900 31.6 / 27.9 / 33.9.  bf16 halves
+// that way: 40 of 64, 3 x 900 18.1 / 15.8 / 19.2, 64 of 64 42.2 / 27.9 / 34.4.
+struct PlainShape {
+  int threads, rows;  // of a workgroup
+};
+PlainShape plain_shape(const LmAttn& a, bool f32) {
+  const int H = a.heads, rows = a.r.n_rows, cols = H * (a.dp + a.vp);
+  if (H <= 4) return {256, 1};
+  if (!f32 || rows < 8 * a.r.n_seq || plain_lds(a, 2) > 160 * 1024) return {512, 1};
+  const bool many = rows >= 2048;
+  if (plain_lds(a, 2) > 80 * 1024) return {512, many && a.kv_heads * (a.dp + a.vp) >= 5 * H * H ? 2 : 1};
+  if (rows <= 512 || (rows <= 768 && a.r.max_ctx > PLAIN_TK)) return {512, 1};
+  const bool pairs = many ? cols >= 1536 || (cols >= 1024 && H % 8 == 0) : cols >= 4096;
+  return pairs ? PlainShape{512, 2} : PlainShape{256, 1};
+}
+
 template <typename T>
 md_status plain(const LmAttn& a, hipStream_t s) {
   if (plain_lds(a, 1) > 160 * 1024) return MD_ERR_UNSUPPORTED;
-  // Pairs of rows where that still leaves a workgroup per CU: up to there the chain of a row's tiles bounds it, beyond the reads do (24 layers, 12 of attention, 16 heads of
-  // 128, one row and two per workgroup: 380 tokens 12.4 and 12.8 ms, 1000 31.5 and 30.5, 3 x 833 71.4 and 68.5)
-  const int nr = a.r.n_rows > 512 && a.r.n_rows >= 8 * a.r.n_seq && plain_lds(a, 2) <= 160 * 1024 ? 2 : 1, lds = plain_lds(a, nr);
-  const auto fn = nr == 2 ? attn_plain_kernel<T, 512, 2> : attn_plain_kernel<T, 512, 1>;
+  const PlainShape shape = plain_shape(a, sizeof(T) == 4);
+  auto fn = shape.threads == 256 ? attn_plain_kernel<T, 256, 1> : attn_plain_kernel<T, 512, 1>;
+  if constexpr (sizeof(T) == 4)
+    if (shape.rows == 2) fn = attn_plain_kernel<T, 512, 2>;
   MD_TRY(md_ensure_dynamic_lds((const void*)fn, 160 * 1024));
-  hipLaunchKernelGGL(fn, dim3((a.r.n_rows + nr - 1) / nr), dim3(512), lds, s, a);
+  hipLaunchKernelGGL(fn, dim3((a.r.n_rows + shape.rows - 1) / shape.rows), dim3(shape.threads), plain_lds(a, shape.rows), s, a);
   return md_launch_status();
 }
 

@@ -435,21 +435,22 @@ def test_norms_of_prompts_sum_in_one_order(heads, dim):
     assert bool(keys[whole].any()) and torch.equal(keys[whole], keys[single])
 
 
-@pytest.mark.parametrize("heads,kv,dim,vdim,chunk", [(3, 1, 20, 40, 2000), (4, 4, 32, 32, 33), (20, 5, 32, 24, 64), (40, 40, 128, 128, 300), (64, 64, 128, 128, 300)], ids=str)
-def test_fp32_rows_in_pairs(heads, kv, dim, vdim, chunk):
-    """More than 512 rows in fp32: pairs of rows in one workgroup, pairs that two sequences or two chunks share, a last row without a second one, a second row with a tile
-    of its own, heads whose pairs do not fit LDS; the same logits as those rows alone, up to the order in which a product's sums run."""
+@pytest.mark.parametrize("copies", [1, 4])
+@pytest.mark.parametrize("heads,kv,dim,vdim,chunk", [(3, 1, 20, 40, 2000), (4, 4, 32, 32, 33), (20, 5, 32, 24, 64), (24, 8, 64, 30, 33), (16, 16, 32, 32, 2000), (40, 40, 128, 128, 300), (64, 64, 128, 128, 300)], ids=str)
+def test_fp32_rows_in_pairs(heads, kv, dim, vdim, chunk, copies):
+    """561 rows in fp32, one at a time, and 2244: pairs of rows in one workgroup (16, 24 and 40 heads), pairs that two sequences or two chunks share, a last row without a second one, a
+    second row with a tile of its own, heads whose pairs do not fit LDS; the same logits as those rows alone, up to the order in which a product's sums run."""
     from moondream_amd.config import LayeredLMConfig
     from moondream_amd.layered_lm import LayeredLM
 
     cfg = U.config([U.attention(heads, kv, dim, vdim, chunk)], width=64, vocab=60, ff=None)
     w = U.weights(cfg, 3, 1.5)
-    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=F32, max_batch=8, max_context=600)
+    m = LayeredLM(LayeredLMConfig.from_dict(cfg), w, dtype=F32, max_batch=24, max_context=600)
     ts = [U.tokens(n, 60, n) for n in (301, 64, 1, 130, 65)]
-    slots = [m.open_sequence() for _ in ts]
-    got = m.step([(s, t, range(len(t))) for s, t in zip(slots, ts)])
+    slots = [m.open_sequence() for _ in range(copies * len(ts))]
+    got = m.step([(s, t, range(len(t))) for s, t in zip(slots, copies * ts)])
     alone = torch.cat([m.step([(m.open_sequence(), t, range(len(t)))]) for t in ts[:3]])
-    assert float(U.logit_errors(got, torch.cat([O.forward(cfg, w, t) for t in ts])).max()) < TOL[F32]
+    assert float(U.logit_errors(got, torch.cat(copies * [O.forward(cfg, w, t) for t in ts])).max()) < TOL[F32]
     assert float(U.logit_errors(got[: len(alone)], alone.double().cpu()).max()) < TOL[F32]
 
 
