@@ -238,20 +238,34 @@ __global__ __launch_bounds__(NT) void attn_prep_block_kernel(const LmAttn a) {
       }
     }
   }
+  float ss[8];
 #pragma unroll
-  for (int r = 0; r < 8; ++r) hs[r * NT + tid] = y[r][0] * y[r][0] + y[r][1] * y[r][1] + y[r][2] * y[r][2] + y[r][3] * y[r][3];
-  __syncthreads();
+  for (int r = 0; r < 8; ++r) ss[r] = y[r][0] * y[r][0] + y[r][1] * y[r][1] + y[r][2] * y[r][2] + y[r][3] * y[r][3];
+  if (NT > 256 || part == 2) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) hs[r * NT + tid] = ss[r];
+    __syncthreads();
+  }
   if (part < 2) {
-    // a row's sum in norm_row's order, whatever NT: 256 lanes take every 256th column group, then a butterfly per 64 lanes, then the four
+    // a row's sum in norm_row's order, whatever NT: 256 lanes take every 256th column group, then a butterfly per 64 lanes, then the four.  (256 threads: what they hold.  Through LDS as
+    // the others, 512 columns, 2400 / 7500 tokens 9.5 / 16.6 us take 10.9 / 18.9.)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if constexpr (NT == 256) {
 #pragma unroll
-    for (int k = wave; k < 32; k += NT / 64) {
-      const float* from = hs + (k >> 2) * NT + (k & 3) * 64 + (tid & 63);
-      float s = 0.f;
+      for (int r = 0; r < 8; ++r) ss[r] = wave_sum(ss[r]);
+      if ((tid & 63) == 0)
 #pragma unroll
-      for (int i = 0; i < NT / 256; ++i) s += from[256 * i];
-      s = wave_sum(s);
-      if ((tid & 63) == 0) red[k >> 2][k & 3] = s;
+        for (int r = 0; r < 8; ++r) red[r][wave] = ss[r];
+    } else {
+#pragma unroll
+      for (int k = wave; k < 32; k += NT / 64) {
+        const float* from = hs + (k >> 2) * NT + (k & 3) * 64 + (tid & 63);
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < NT / 256; ++i) s += from[256 * i];
+        s = wave_sum(s);
+        if ((tid & 63) == 0) red[k >> 2][k & 3] = s;
+      }
     }
     __syncthreads();
     const float* w = part == 0 ? a.q_norm : a.k_norm;
