@@ -1072,7 +1072,7 @@ md_status lm_attn_mfma(const LmAttn& args, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
-// Prompts of up to 978 keys (PAIRS_MOST blocks of 32) and 40 million scores: attn_mfma_kernel has few tiles then, and each is a long chain.  The mixed scores of all pairs fit the caches (4 bytes of a head
+// Prompts of up to 978 keys (PAIRS_MOST blocks of 32; see lm_attn_pairs_takes) and 40 million scores: attn_mfma_kernel has few tiles then, and each is a long chain.  The mixed scores of all pairs fit the caches (4 bytes of a head
 // and pair), so they go through memory:
 //   attn_pairs_scores_kernel  (32 keys, 16 queries): a wave's share of the heads, their scores to LDS in the order of the mixture's operand (two bf16 for
 //                             a float), mixture, scale, distance and mask; the scores leave in the order of the other kernel's operand.  One workgroup row
@@ -1367,8 +1367,13 @@ TalkKernelBlocks pairs_out_pick(int vp) {
 size_t lm_attn_pairs_floats_most(int n_rows, int n_seq, int span, int H, int dp, int vp) {
   return pairs_form(H, dp, vp) ? (size_t)std::min(PAIRS_FLOATS, pairs_floats(n_rows, n_seq, span, H)) : 0;
 }
+// ... and of 60 million scores (keys wider than 64: 40) with the heads that fill up the products' 16 or 32, which cost as much: 12 layers, 8 x 940 tokens, 4 heads of 64 2.42 -> 2.58 ms against
+// attn_mfma_kernel, of 128 2.76 -> 3.35, one head of 128 2.56 -> 2.90; 24 x 300, 4 of 128 2.18 -> 2.27; but 4 x 940, 4 of 64 1.70 -> 1.52.  All heads at 30 blocks at most, 914 keys: one prompt of 800 / 950 tokens, 32
+// heads of 64 on 8 of keys 1.33 -> 1.19 / 1.38 -> 1.41, 32 of 32 1.11 -> 1.01 / 1.20 -> 1.28; 20 of 64 still 1.29 -> 1.22.
 bool lm_attn_pairs_takes(const LmAttn& a, int span) {
-  return pairs_form(a.heads, a.dp, a.vp) && pairs_blocks(span) <= PAIRS_MOST && pairs_floats(a.r.n_rows, a.r.n_seq, span, a.heads) <= PAIRS_FLOATS;
+  if (!pairs_form(a.heads, a.dp, a.vp) || pairs_blocks(span) > (a.heads > 24 ? 30 : PAIRS_MOST)) return false;
+  auto floats = [&](int heads) { return pairs_floats(a.r.n_rows, a.r.n_seq, span, heads); };
+  return floats(a.heads) <= PAIRS_FLOATS && floats(a.heads <= 16 ? 16 : 32) <= (a.dp > 64 ? 40 << 20 : 60 << 20);
 }
 md_status lm_attn_pairs(const LmAttn& a, int span, hipStream_t s) {
   if (!lm_attn_pairs_takes(a, span)) return MD_ERR_UNSUPPORTED;
