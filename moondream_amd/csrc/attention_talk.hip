@@ -2019,12 +2019,15 @@ size_t lm_attn_heads_floats(int n_seq, int span, int H, int G, int dp, int vp, i
 // every key, which counts against the 4 dim of keys and values from H = dim on: 64 heads of 64, 40 sequences at 200 / 500 / 1000 keys 0.90 / 0.73, 1.20 / 1.19, 1.79 / 1.97, 24 at 500 / 1000
 // 0.86 / 0.80, 1.18 / 1.25; 64 of 32, where the others are slower, 40 at 1500 1.91 / 1.79, 64 2.78 / 2.90; 32 of 32, 24 / 64 at 1000 0.477 / 0.477, 0.87 / 0.89.  The fewest keys of more than
 // 40 sequences: 64 of 64 at 30 0.72 / 0.79, 48 of 64 0.635 / 0.587.  One or two groups of columns, from where parts of a head are added up: 24 layers of 4 of 64, one sequence at 200 / 500 /
-// 1500 0.501 / 0.503, 0.508 / 0.546, 0.54 / 0.60, 40 at 500 0.78 / 0.75; 16 of 32, 24 / 40 at 1500 0.96 / 1.04, 1.23 / 1.32; but 4 of 128, 8 at 1000 0.69 / 0.66.
+// 1500 0.501 / 0.503, 0.508 / 0.546, 0.54 / 0.60, 40 at 500 0.78 / 0.75; 16 of 32, 24 / 40 at 1500 0.96 / 1.04, 1.23 / 1.32; but 4 of 128, 8 at 1000 0.69 / 0.66.  Twelve layers: 16 of 32, 64 / 128 at
+// 1800 1.03 / 1.10, 1.66 / 1.85, where 4 of 64 take 0.93 / 0.75, 1.30 / 1.10; 48 of 64, 128 at 800 / 1000 / 1800 4.96 / 4.73, 4.73 / 5.29, 7.73 / 9.05, 64 at 1800 5.13 / 4.80; 40 of 64, 128 at 1800
+// 6.90 / 6.96.  A second workgroup for a few keys of each of many heads: 64 of 32, 20 at 220 / 300 / 420 0.67 / 0.59, 0.69 / 0.75, 0.96 / 0.78; 64 of 64, 40 at 300 1.36 / 1.44.
 bool lm_attn_heads_takes(const LmAttn& a, int span) {
   if (!heads_takes(a.heads, a.kv_heads, a.dp, a.vp, a.taps, a.own_kv)) return false;
   const int64_t H = a.heads, dp = a.dp, n_seq = a.r.n_seq;
-  const bool scores = H >= dp && n_seq * span * dp * dp > 20480 * H * H, many = H > 48 && n_seq > 40;
-  const bool few = H * dp <= 512 && dp < 128 && span > HEADS_SPAN && n_seq * dp <= 1280;
+  const bool scores = (H >= dp && n_seq * span * dp * dp > 20480 * H * H) || (4 * H >= 3 * dp && n_seq * span > 120000);
+  const bool many = H > 48 && (n_seq > 40 || (n_seq >= 16 && span > HEADS_SPAN && 2 * span <= 3 * HEADS_SPAN));
+  const bool few = H * dp <= 512 && span > HEADS_SPAN && (dp == 32 || (dp == 64 && n_seq <= 20));
   return !(scores || many || few) || !lm_attn_decode_takes(a);
 }
 md_status lm_attn_heads(const LmAttn& a, int span, hipStream_t s) {
