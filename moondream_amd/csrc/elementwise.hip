@@ -341,13 +341,14 @@ __device__ __forceinline__ void load_logits8(const float* p, float (&v)[8]) {
 }
 
 // greedy argmax, ties -> lowest index; optionally bumps pos[b].  Rows hold round_up(vocab, 8) readable logits.
-// One row per workgroup, in a chain that the next step waits for: a batch of loads is requested at once and its logits compared by value alone (a thread's
-// indices rise).  51200 logits, one row 9.3 -> 6.7 us, 40 rows 9.9 -> 7.4.
+// One row per workgroup, in a chain that the next step waits for: two loads are requested at once and their logits compared by value alone (a thread's
+// indices rise).  51200 bf16 logits, 1 / 40 / 512 rows 8.7 -> 5.0, 9.0 -> 5.4, 14.3 -> 10.8 us; 8192, 1 / 512 rows 4.6 -> 4.5, 6.0 -> 5.5; 262144, 1 row 30 -> 13.8.  Eight at once, mostly past the end of
+// short rows: 6.1, 6.5, 17.4; 7.1, 14.7; 14.4.
 template <typename T>
 __global__ __launch_bounds__(1024) void argmax_kernel(const T* __restrict__ logits, int64_t ld,
                                                      int vocab, int suppress, int32_t* __restrict__ next,
                                                      int32_t* __restrict__ pos_inc) {
-  constexpr int NONE = 0x7fffffff, AHEAD = sizeof(T) == 2 ? 8 : 4;
+  constexpr int NONE = 0x7fffffff, AHEAD = 2;
   __shared__ float sv[16];
   __shared__ int si[16];
   const int b = blockIdx.x, chunks = (vocab + 7) >> 3;
